@@ -1,0 +1,125 @@
+"""Paged attention of prompt rows at the edges of its tiles, pages and key
+parts, against fp64 on the CPU. Results are bf16, off by up to 2^-9 of
+themselves. The weights that meet 128-wide values are rounded to bf16 as well:
+2^-9 of the weighted sum of |v|; twice both is allowed (the weights' sum is not
+rounded the same way). 64-wide heads keep 32-bit weights: 2^-18 for their
+exponentials, whose arguments are rounded products of up to 2^5."""
+import math
+
+import pytest
+import torch
+
+from xllm_service_amd import ops
+
+pytestmark = pytest.mark.gpu
+PAGE = 16
+
+
+def make(lens, ctx, kv_heads, per, dim, seed, spare=3):
+    """bf16 queries behind a wider row, caches over scattered pages, and the
+    lengths, on the CPU."""
+    g = torch.Generator().manual_seed(seed)
+    need = [-(-(n + c) // PAGE) for n, c in zip(lens, ctx)]
+    order = torch.randperm(sum(need) + spare, generator=g).to(torch.int32)
+    table = torch.zeros(len(lens), max(need), dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = order[at:at + n]
+        at += n
+    pool = (sum(need) + spare, kv_heads, PAGE, dim)
+    k, v = (torch.randn(pool, generator=g).to(torch.bfloat16)
+            for _ in range(2))
+    heads = kv_heads * per
+    rows = torch.randn(sum(lens), (heads + 2) * dim, generator=g)
+    return rows.to(torch.bfloat16), k, v, table
+
+
+def want(q, k, v, table, lens, ctx, scale):
+    """(result, weighted sum of |v|) in fp64; q [T, heads, dim]."""
+    heads, dim = q.shape[1:]
+    per = heads // k.shape[1]
+    out, big, at = [], [], 0
+    for s, (n, c) in enumerate(zip(lens, ctx)):
+        pages = table[s, :-(-(n + c) // PAGE)].long()
+        kk, vv = (x[pages].transpose(1, 2).reshape(-1, k.shape[1], dim)[:n + c]
+                  .double().repeat_interleave(per, 1) for x in (k, v))
+        z = torch.einsum("thd,lhd->htl", q[at:at + n].double(), kk) * scale
+        late = torch.arange(n + c)[None] > c + torch.arange(n)[:, None]
+        p = torch.softmax(z.masked_fill(late, -math.inf), -1)
+        out.append(torch.einsum("htl,lhd->thd", p, vv))
+        big.append(torch.einsum("htl,lhd->thd", p, vv.abs()))
+        at += n
+    return torch.cat(out), torch.cat(big)
+
+
+def check(got, ref, big):
+    off = (got.double().cpu() - ref).abs()
+    assert torch.isfinite(got).all()
+    weights = 2.0 ** (-8 if got.shape[-1] == 128 else -18)
+    over = off - weights * big - 2.0 ** -8 * ref.abs() - 1e-6
+    assert over.max() <= 0, f"off by {off.max():.3g}, over by {over.max():.3g}"
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("lens,ctx,kv_heads,per", [
+    ([1, 31, 32, 33], [0, 15, 16, 17], 3, 1),       # waves and pages
+    ([63, 64, 65], [0, 1, 63], 2, 2),               # key tiles
+    ([127, 128, 129, 1], [0, 0, 5, 64], 1, 1),      # row tiles
+    ([18, 19, 37], [47, 300, 0], 4, 7),             # heads that share keys
+    ([3, 1, 9], [2100, 1033, 4500], 2, 4),          # keys split over parts
+    ([1], [9000], 1, 8),                            # over 64 tiles of one page
+    ([1] * 70 + [5], [3] * 70 + [40], 2, 3),        # more than 64 sequences
+])
+def test_prefill_edges(dim, lens, ctx, kv_heads, per):
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(lens) + dim)
+    heads, scale = kv_heads * per, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)))
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)])
+    dev = [t.cuda() for t in (k, v, table, cu.int(), sl.int())]
+    qd = rows.cuda()[:, :heads * dim].unflatten(-1, (heads, dim))
+    # the result goes into rows of a wider tensor; what is beside them stays
+    wide = torch.full((sum(lens), (heads + 1) * dim), 7.0,
+                      dtype=torch.bfloat16, device="cuda")
+    out = wide[:, :heads * dim].unflatten(-1, (heads, dim))
+    for sign in (1.0, -1.0):
+        got = ops.paged_attn_prefill(qd, *dev, sign * scale, out=out)
+        check(got, *want(q, k, v, table, lens, ctx, sign * scale))
+    assert (wide[:, heads * dim:] == 7.0).all()
+
+
+def test_prefill_standout_scores():
+    """Scores far apart: the running maximum moves within and across tiles."""
+    lens, ctx = [40], [150]
+    rows, k, v, table = make(lens, ctx, 1, 2, 128, 5)
+    k[table[0, 4], 0, 3] *= 30.0
+    k[table[0, 9], 0, 15] *= 60.0
+    q = rows[:, :256].unflatten(-1, (2, 128))
+    got = ops.paged_attn_prefill(
+        q.contiguous().cuda(), k.cuda(), v.cuda(), table.cuda(),
+        torch.tensor([0, 40], dtype=torch.int32, device="cuda"),
+        torch.tensor([190], dtype=torch.int32, device="cuda"), 0.3)
+    check(got, *want(q, k, v, table, lens, ctx, 0.3))
+
+
+def test_prefill_needs_no_host():
+    """No list of tiles, no wait: the call can be captured, and a replay
+    follows the lengths on the device."""
+    rows, k, v, table = make([40, 24], [20, 0], 2, 2, 128, 9)
+    q = rows[:, :512].unflatten(-1, (4, 128)).contiguous()
+    dev = [t.cuda() for t in (q, k, v, table)]
+    cu = torch.tensor([0, 40, 64], dtype=torch.int32, device="cuda")
+    sl = torch.tensor([60, 24], dtype=torch.int32, device="cuda")
+    out = torch.empty_like(dev[0])
+    ops.paged_attn_prefill(*dev, cu, sl, 0.1, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.paged_attn_prefill(*dev, cu, sl, 0.1, out=out)
+    for lens, ctx in (([40, 24], [20, 0]), ([30, 34], [10, 14])):
+        cu.copy_(torch.tensor([0, lens[0], 64]))
+        sl.copy_(torch.tensor([n + c for n, c in zip(lens, ctx)]))
+        out.fill_(3.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        check(out, *want(q, k, v, table, lens, ctx, 0.1))

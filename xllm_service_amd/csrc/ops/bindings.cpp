@@ -39,11 +39,12 @@ void launch_paged_attn_decode(unsigned short*, const unsigned short*,
                               int, int, int, int, int, long, long,
                               hipStream_t);
 int paged_attn_decode_partitions(int, int);
-void launch_paged_attn_prefill(unsigned short*, const unsigned short*,
+int paged_attn_prefill_parts(long, int, int, int, int);
+void launch_paged_attn_prefill(unsigned short*, float*, float*,
                                const unsigned short*, const unsigned short*,
-                               const int*, const int*, const int*, const int*,
-                               const int*, int, float, int, int, int, long,
-                               long, hipStream_t);
+                               const unsigned short*, const int*, const int*,
+                               const int*, long, int, float, int, int, int,
+                               int, long, long, int, hipStream_t);
 void launch_greedy_sample(long*, const unsigned short*, int, int, hipStream_t);
 void launch_mfma_gemm(unsigned short*, const unsigned short*,
                       const unsigned short*, const unsigned short*, int, int,
@@ -242,24 +243,39 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
 void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
                         torch::Tensor k_cache, torch::Tensor v_cache,
                         torch::Tensor block_tables, torch::Tensor cu_q,
-                        torch::Tensor seq_lens, torch::Tensor tile_seq,
-                        torch::Tensor tile_q0, double scale) {
+                        torch::Tensor seq_lens, double scale) {
   CHECK_BF16_ROWVIEW(out); CHECK_BF16_ROWVIEW(q);
   CHECK_BF16_CUDA(k_cache); CHECK_BF16_CUDA(v_cache);
-  for (auto* t : {&block_tables, &cu_q, &seq_lens, &tile_seq, &tile_q0}) {
+  for (auto* t : {&block_tables, &cu_q, &seq_lens}) {
     TORCH_CHECK(t->dtype() == torch::kInt && t->is_cuda() && t->is_contiguous());
   }
+  const long tokens = q.size(0);
   const int n_qheads = q.size(1);
   const int D = q.size(2);
   const int n_kv = k_cache.size(1);
-  TORCH_CHECK(D == 128, "prefill kernel requires head_dim == 128");
+  const int n_seqs = cu_q.size(0) - 1;
+  TORCH_CHECK(D == 128 || D == 64, "prefill kernel: head_dim 64 or 128");
   TORCH_CHECK(k_cache.size(2) == 16, "block_size must be 16");
+  TORCH_CHECK(k_cache.size(3) == D && v_cache.sizes() == k_cache.sizes() &&
+              n_qheads % n_kv == 0 && out.sizes() == q.sizes() &&
+              seq_lens.size(0) >= n_seqs && block_tables.size(0) >= n_seqs,
+              "prefill kernel: shapes do not match");
+  const int n_part = xllm::paged_attn_prefill_parts(
+      tokens, n_seqs, n_qheads / n_kv, n_kv, block_tables.size(1));
+  torch::Tensor ws;            // [tokens * heads][parts][D + 2], fp32
+  float *ws_o = nullptr, *ws_ml = nullptr;
+  if (n_part > 1) {
+    const long n = tokens * n_qheads * n_part;
+    ws = torch::empty({n * (D + 2)}, q.options().dtype(torch::kFloat));
+    ws_o = ws.data_ptr<float>();
+    ws_ml = ws_o + n * D;
+  }
   xllm::launch_paged_attn_prefill(
-      u16(out), u16c(q), u16c(k_cache), u16c(v_cache),
+      u16(out), ws_o, ws_ml, u16c(q), u16c(k_cache), u16c(v_cache),
       block_tables.data_ptr<int>(), cu_q.data_ptr<int>(),
-      seq_lens.data_ptr<int>(), tile_seq.data_ptr<int>(),
-      tile_q0.data_ptr<int>(), tile_seq.size(0), (float)scale, n_qheads, n_kv,
-      block_tables.size(1), q.stride(0), out.stride(0), cur_stream());
+      seq_lens.data_ptr<int>(), tokens, n_seqs, (float)scale, n_qheads, n_kv,
+      D, block_tables.size(1), q.stride(0), out.stride(0), n_part,
+      cur_stream());
 }
 
 torch::Tensor greedy_sample(torch::Tensor logits) {

@@ -4,26 +4,50 @@
 // cache (chunked prefill and prefix-cache hits share this one code path:
 // new tokens' K/V are scattered into the cache first, then this runs).
 //
-// v3 structure (v2 at 4 waves x 32 q rows allocated 247 VGPR + 76 AGPR =
-// 1 wave/SIMD — zero latency hiding, 111 TF; v1 was the guide's "2-phase
-// stall" shape at ~76 TF):
-//   * workgroup = 512 threads = 8 waves; one workgroup per
-//     (128-row q tile, q_head); each wave owns 16 q rows (1 MFMA m-tile),
-//     halving per-wave register state -> 2 waves/SIMD occupancy with the
-//     same K/V staging amortization (128 q rows per staged tile)
-//   * KV tile = 64 keys (4 cache blocks) staged cooperatively:
-//     K row-major [64][128+8] (padded against the 16-way ds_read_b128
-//     conflict), V into two tr16 images so P·V B-fragments come from
-//     ds_read_b64_tr_b16 (see paged_attn_decode.hip for the image math)
-//   * per wave and KV tile: 16 QK^T MFMAs -> online softmax (row stats
-//     reduced over the 16 lanes holding a row's columns) -> P via LDS ->
-//     16 P·V MFMAs
+// The G query heads of a key/value head attend to the same keys, so the
+// (query, head) pairs of a sequence are rows of one matrix, row = query * G +
+// head in group. A workgroup (4 waves) owns 128 rows of one key/value head, a
+// wave 32; two workgroups share a CU. Short chunks fill their tiles better
+// that way (93 queries x 7 heads: 6 tiles, not 7 x 1) and a workgroup's rows
+// span few positions, so little of a tile on the diagonal is masked.
 //
-// MFMA fragment layout assumptions (verified on hardware by
-// tests/test_gpu_ops.py::test_mfma_fragment_layout):
-//   A: lane l holds A[l&15][(l>>4)*8 + j], j=0..7  (8 contiguous bf16)
-//   B: lane l holds B[(l>>4)*8 + j][l&15]
-//   C: lane l holds C[(l>>4)*4 + r][l&15], r=0..3
+// Per tile of 64 keys:
+//   S^T[key][row] = K Q^T        32x32x16 products, A = K rows from LDS, B = Q
+//                                in registers for the whole kernel
+//   online softmax               a lane holds 32 of the tile's scores of ONE
+//                                row and its partner lane (l ^ 32) the others:
+//                                a row maximum is a chain of v_max and one lane
+//                                swap, the sums meet once, at the very end
+//   O^T[d][row] += V^T P^T       A = V^T by hardware transpose reads, B = the
+//                                lane's own weights, rounded to bf16: no trip
+//                                through LDS
+// The C layout of S^T hands lane half h the rows 8i + 4h + r; feeding key
+// 16(i>>1) + 8h + 4(i&1) + r as A row 8i + 4h + r makes those the keys
+// 16t + 8h + 0..7 that the B operand of step t wants of that lane.
+//
+// K and V tiles go from memory straight to LDS (no registers, no ds_write),
+// double-buffered with one barrier per tile. The loads place 16 B per lane in
+// lane order, so rows cannot be padded; the 16 B chunks of a row are permuted
+// by its key instead (on the side of the memory address), which makes both
+// the row reads of K and the transpose reads of V free of bank conflicts.
+//
+// Few row tiles over a long context leave most of the chip idle: then the
+// keys are split over n_part workgroups and a second kernel merges the fp32
+// partial results.
+//
+// Bound by the matrix pipe and the vector unit in turn: a tile costs a wave
+// 32 products (about 1000 cycles) and about as many cycles of exponentials,
+// maxima and conversions, which the second wave of the SIMD overlaps; LDS
+// reads feed 32 rows each and stay just below the pipe's rate. Measured, 4
+// prompts of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads: 371 us,
+// 873 TFLOP/s (a large bf16 matrix product: 1466); one head and 16 rows per
+// wave on 16x16x32 products, P through LDS: 1209 us. 3 chunks of 93-261 tokens
+// over 0.5-1.8 k, 28 heads, with the key split: 31 us, without a list of tiles
+// made on the host; before: 110 us and 48 us of copies and waiting. 8 prompts
+// of 109-438 tokens, 12 heads of 64: 11 us, an eager loop before: 14 ms.
+//
+// Fragments (lane l, h = l >> 5) of v_mfma_f32_32x32x16_bf16:
+//   A[l&31][h*8 + j], B[h*8 + j][l&31], C[8*(r>>2) + 4h + (r&3)][l&31]
 //
 // Parity: reference engine's paged-attention prefill.
 #include "common.h"
@@ -32,289 +56,431 @@ namespace xllm {
 
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
-typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
+typedef __attribute__((ext_vector_type(2))) __bf16 bfx2;
+typedef __attribute__((ext_vector_type(2))) float fx2;
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
 
-#define PF_QW 16           // q rows per wave (1 m-tile)
-#define PF_WGQ 128         // q rows per workgroup (8 waves)
-#define PF_KBLK 64         // keys per KV tile (4 cache blocks)
-#define PF_D 128           // head_dim (required)
-#define PF_KPAD 8          // pad elements per K row
-#define PF_PPAD 8          // pad elements per P row
+#define PF_ROWS 128        // rows per workgroup
+#define PF_KT 64           // keys per tile
 #define PF_BS 16           // cache block size
 
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
-void paged_attn_prefill_kernel(
+typedef __attribute__((address_space(3))) unsigned short lds_u16;
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
+typedef __attribute__((address_space(3))) void lds_void;
+typedef const __attribute__((address_space(1))) void glb_void;
+
+// larger of a lane's and its partner's (l ^ 32) value
+XLLM_DEV float pair_max(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+XLLM_DEV float pair_sum(float v) {
+  const unsigned u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+XLLM_DEV unsigned pack_bf16(float a, float b) {
+  const fx2 f = {a, b};
+  const bfx2 x = __builtin_convertvector(f, bfx2);
+  return __builtin_bit_cast(unsigned, x);
+}
+
+// Row tile `b` of the batch -> sequence and tile within it; later tiles of a
+// sequence (more keys) come first. False: past the last one. One wave looks
+// 64 sequences over at a time.
+XLLM_DEV bool pf_locate(int b, const int* cu_q, int n_seqs, int G, int lane,
+                        int* s, int* lt) {
+  int acc = 0;
+  for (int base = 0; base < n_seqs; base += 64) {
+    const int i = base + lane;
+    int nt = 0;
+    if (i < n_seqs)
+      nt = ((cu_q[i + 1] - cu_q[i]) * G + PF_ROWS - 1) / PF_ROWS;
+    int sum = nt;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(sum, off, 64);
+      if (lane >= off) sum += up;
+    }
+    const unsigned long long hit = __ballot(b < acc + sum);
+    if (hit != 0) {
+      const int first = __ffsll(hit) - 1;
+      *s = __builtin_amdgcn_readfirstlane(base + first);
+      *lt = __builtin_amdgcn_readfirstlane(acc + __shfl(sum, first, 64) - 1 -
+                                           b);
+      return true;
+    }
+    acc += __shfl(sum, 63, 64);
+  }
+  return false;
+}
+
+// TERMS: bf16 terms a softmax weight is split into. One rounds it to bf16;
+// three (8 + 8 + 8 mantissa bits) hold all of its 32-bit value, each with a
+// product of its own into the same fp32 sums.
+template <int D, int TERMS>
+__global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
     unsigned short* __restrict__ out,        // [total_q, n_qheads, D] bf16
+    float* __restrict__ ws_o,                // [total_q*n_qheads][n_part][D]
+    float* __restrict__ ws_ml,               // [total_q*n_qheads][n_part][2]
     const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
     const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
     const unsigned short* __restrict__ v_cache,
     const int* __restrict__ block_tables,    // [num_seqs, max_blocks]
     const int* __restrict__ cu_q,            // [num_seqs+1] query offsets
     const int* __restrict__ seq_lens,        // [num_seqs] total key len
-    const int* __restrict__ tile_seq,        // [total_tiles] tile -> seq
-    const int* __restrict__ tile_q0,         // [total_tiles] tile -> local q0
-    const float scale,
-    const int n_qheads, const int n_kv_heads, const int max_blocks_per_seq,
-    const long q_stride, const long out_stride) {
-  const int tile = blockIdx.x;
-  const int qh = blockIdx.y;
-  const int kvh = qh / (n_qheads / n_kv_heads);
-  const int seq = tile_seq[tile];
-  const int q0 = tile_q0[tile];
+    const int n_seqs, const float scale, const int G, const int n_kv,
+    const int max_blocks, const long q_stride, const long out_stride,
+    const int n_part) {
+  constexpr int KS = D / 16;                 // k steps of a score product
+  constexpr int DT = D / 32;                 // 32-wide tiles of the head
+  constexpr int CPR = D / 8;                 // 16 B chunks of a row
+  constexpr int RPI = 64 / CPR;              // rows one load instruction fills
+  constexpr int NI = 16 / RPI;               // ... instructions per page
+  constexpr int TILE = PF_KT * D;            // elements of a K or V tile
+  __shared__ __attribute__((aligned(1024))) unsigned short kv_lds[4 * TILE];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, c32 = lane & 31;
+
+  const int kvh = blockIdx.x % n_kv;
+  const int part = (blockIdx.x / n_kv) % n_part;
+  int seq, lt;
+  if (!pf_locate(blockIdx.x / (n_kv * n_part), cu_q, n_seqs, G, lane, &seq,
+                 &lt))
+    return;
   const int q_start = cu_q[seq];
   const int q_len = cu_q[seq + 1] - q_start;
   const int seq_len = seq_lens[seq];
   const int ctx = seq_len - q_len;
+  const int rows = q_len * G;
+  const int n_qheads = n_kv * G;
 
-  const int wid = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int frow = lane & 15;
-  const int fcol8 = (lane >> 4) * 8;
-  const int crow4 = (lane >> 4) * 4;
+  const int row0 = lt * PF_ROWS;
+  const int kmax = ctx + (min(row0 + PF_ROWS, rows) - 1) / G + 1;
+  const int n_tiles = (kmax + PF_KT - 1) / PF_KT;
+  // parts of at least four tiles; the rest of them stay empty
+  const int parts = min(n_part, (n_tiles + 3) / 4);
+  const int tpp = parts > 0 ? (n_tiles + parts - 1) / parts : 0;
+  const int t_begin = part * tpp;
+  const int t_end = min(n_tiles, t_begin + tpp);
 
-  const int wq0 = q0 + wid * PF_QW;
-  const int wq_rows = min(PF_QW, q_len - wq0);
-  const bool wave_active = wq_rows > 0;
-  const int wave_kmax = wave_active ? (ctx + wq0 + wq_rows) : 0;
-  const int wg_q_end = min(q0 + PF_WGQ, q_len);
-  const int wg_kmax = ctx + wg_q_end;
+  // ---- this lane's row -----------------------------------------------------
+  const int wrow0 = row0 + wid * 32;
+  const bool wave_on = wrow0 < rows;
+  const int rho = wrow0 + c32;
+  const bool row_ok = rho < rows;
+  const int qi = rho / G;
+  const int head = kvh * G + rho - qi * G;
+  const int limit = row_ok ? ctx + qi + 1 : 0;   // keys this row sees
+  const int wmin = ctx + wrow0 / G + 1;          // fewest of a row in the wave
+  const int wmax = ctx + (min(wrow0 + 32, rows) - 1) / G + 1;
 
-  // v4: SINGLE-buffered K/V staging (52 KB total) + registers capped at
-  // 128 so TWO 8-wave workgroups co-reside per CU. That costs a second
-  // barrier per tile, but with 2 WGs the other workgroup's MFMAs cover
-  // every barrier/stage stall — the round-1 single-WG profile parked 45%
-  // of wave-cycles at SQ_WAIT with nothing to switch to.
-  __shared__ unsigned short k_lds[PF_KBLK][PF_D + PF_KPAD];
-  __shared__ unsigned short v_img[2][4096];     // tr16 image per 32-key half
-  __shared__ unsigned short p_lds[8][PF_QW][PF_KBLK + PF_PPAD];
-
-  // ---- Q fragment: one m-tile, lane row frow -------------------------------
-  bf16x8 qf[4];
-  {
-    const int qrow = wq0 + frow;
-    if (wave_active && qrow < q_len) {
-      const long qoff = (long)(q_start + qrow) * q_stride + (long)qh * PF_D;
+  // weights are 2^(c (s - m)); a negative scale turns the queries' signs
+  const short flip = scale < 0.0f ? (short)0x8000 : (short)0;
+  const float c = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
+  bf16x8 qf[KS];
 #pragma unroll
-      for (int ks = 0; ks < 4; ks++)
-        qf[ks] = *reinterpret_cast<const bf16x8*>(q + qoff + ks * 32 + fcol8);
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++) qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
+  for (int ks = 0; ks < KS; ks++) {
+    qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (row_ok)
+      qf[ks] = *reinterpret_cast<const bf16x8*>(
+          q + (long)(q_start + qi) * q_stride + (long)head * D + ks * 16 +
+          h * 8);
+    qf[ks] ^= flip;
   }
 
-  float m_r[4], l_r[4];
-  f32x4 o_acc[8];
+  f32x16 o_acc[DT];
 #pragma unroll
-  for (int r = 0; r < 4; r++) { m_r[r] = -INFINITY; l_r[r] = 0.0f; }
+  for (int i = 0; i < DT; i++)
 #pragma unroll
-  for (int n = 0; n < 8; n++) o_acc[n] = f32x4{0, 0, 0, 0};
+    for (int r = 0; r < 16; r++) o_acc[i][r] = 0.0f;
+  float m = -INFINITY, l = 0.0f;
 
-  const int* btab = block_tables + (long)seq * max_blocks_per_seq;
-  const long head_stride = (long)PF_BS * PF_D;
-
-  // ---- T14 async-stage split (guide Guideline 15): the next tile's global
-  // loads issue BEFORE this tile's compute; the LDS write lands after the
-  // read barrier. Each of the 512 threads owns 2 fixed 8-element strips
-  // of the 64x128 tile (threadIdx*8 + it*4096).
-  ushort8_t stg_k[2], stg_v[2];
-  const int sidx0 = threadIdx.x * 8;
-
-  auto stage_load = [&](int kv0) {
+  // ---- staging: a wave moves the tile's page `wid` ---------------------------
+  const int* btab = block_tables + (long)seq * max_blocks;
+  const int last_blk = (seq_len - 1) / PF_BS;
+  const int last_row = (seq_len - 1) % PF_BS;
+  const int srow = lane / CPR, spos = lane % CPR;
+  // byte offset in a page of what this lane moves: row r of the page, its
+  // chunk permuted by the row's key
+  auto off_of = [&](int r, int key, bool val) {
+    const int x = val ? (D == 128 ? (key & 3) << 2 : ((key >> 1) & 1) << 2)
+                      : (D == 128 ? key & 15 : (key >> 1) & 7);
+    return (unsigned)(r * (2 * D) + ((spos ^ x) << 4));
+  };
+  unsigned koff[NI], voff[NI];
 #pragma unroll
-    for (int it = 0; it < 2; it++) {
-      const int idx = sidx0 + it * 4096;
-      const int kt = idx / PF_D;
-      const int d = idx % PF_D;
-      const int tok = kv0 + kt;
-      // clamp (not branch) the address: an in-loop conditional around each
-      // load makes hipcc branch + drain per element (guide traps 4(c))
-      const int tok_c = tok < seq_len ? tok : seq_len - 1;
-      const long base =
-          ((long)btab[tok_c / PF_BS] * n_kv_heads + kvh) * head_stride +
-          (long)(tok_c % PF_BS) * PF_D + d;
-      stg_k[it] = *reinterpret_cast<const ushort8_t*>(k_cache + base);
-      stg_v[it] = *reinterpret_cast<const ushort8_t*>(v_cache + base);
+  for (int i = 0; i < NI; i++) {
+    const int r = i * RPI + srow;
+    koff[i] = off_of(r, r, false);
+    voff[i] = off_of(r, r, true);
+  }
+  // ids of this wave's pages of 64 tiles from tile tb on, one per lane: a
+  // scalar load per tile would make every wait for LDS a wait for it too
+  int tb = t_begin;
+  auto pages_from = [&](int t) {
+    return btab[min(t * (PF_KT / PF_BS) + wid + lane * (PF_KT / PF_BS),
+                    last_blk)];
+  };
+  auto put = [&](const char* kp, const char* vp, unsigned ko, unsigned vo,
+                 unsigned short* dst) {
+    __builtin_amdgcn_global_load_lds((glb_void*)(kp + ko), (lds_void*)dst, 16,
+                                     0, 0);
+    __builtin_amdgcn_global_load_lds((glb_void*)(vp + vo),
+                                     (lds_void*)(dst + TILE), 16, 0, 0);
+  };
+  auto stage = [&](int t, int page, int buf) {
+    const int pg = t * (PF_KT / PF_BS) + wid;
+    const long base = ((long)page * n_kv + kvh) * (PF_BS * D * 2);
+    const char* kp = reinterpret_cast<const char*>(k_cache) + base;
+    const char* vp = reinterpret_cast<const char*>(v_cache) + base;
+    unsigned short* dst = kv_lds + buf * 2 * TILE + wid * 16 * D;
+    if (pg < last_blk) {
+#pragma unroll
+      for (int i = 0; i < NI; i++)
+        put(kp, vp, koff[i], voff[i], dst + i * RPI * D);
+      return;
+    }
+    // rows past the last key repeat it: masked below, and finite
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int r = i * RPI + srow;
+      const int rr = pg > last_blk ? last_row : min(r, last_row);
+      put(kp, vp, off_of(rr, r, false), off_of(rr, r, true), dst + i * RPI * D);
     }
   };
 
-  auto stage_write = [&](int kv0) {
-#pragma unroll
-    for (int it = 0; it < 2; it++) {
-      const int idx = sidx0 + it * 4096;
-      const int kt = idx / PF_D;
-      const int d = idx % PF_D;
-      ushort8_t kvv = stg_k[it], vvv = stg_v[it];
-      if (kv0 + kt >= seq_len) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) { kvv.x[j] = 0; vvv.x[j] = 0; }
-      }
-      *reinterpret_cast<ushort8_t*>(&k_lds[kt][d]) = kvv;
-      const int k32 = kt & 31;
-      const int koff =
-          ((k32 >> 2) & 1) * 256 + (k32 >> 3) * 64 + (k32 & 3) * 16;
-      *reinterpret_cast<ushort8_t*>(
-          &v_img[kt >> 5][(d >> 4) * 512 + koff + (d & 15)]) = vvv;
-    }
-  };
+  // ---- LDS addresses (elements) --------------------------------------------
+  // K row of A row m = lane & 31, chunk 2 ks + h
+  const int km = ((c32 >> 4) << 4) | (((c32 >> 2) & 1) << 3) |
+                 (((c32 >> 3) & 1) << 2) | (c32 & 3);
+  const int kbase =
+      km * D + ((h ^ (D == 128 ? (km & 15) : ((km >> 1) & 7))) << 3);
+  // V: rows 16t + 8h + (i >> 2) (+4), columns dt*32 + dhalf*16 + (i & 3)*4
+  const int vi = lane & 15, dh = (lane >> 4) & 1;
+  const int vbase = (8 * h + (vi >> 2)) * D + dh * 16 + (vi & 3) * 4 +
+                    ((D == 128 ? (vi >> 2) : (vi >> 3)) << 5);
 
-  stage_load(0);
-  stage_write(0);
-  __syncthreads();
-
-  for (int kv0 = 0; kv0 < wg_kmax; kv0 += PF_KBLK) {
-    const bool has_next = kv0 + PF_KBLK < wg_kmax;
-    if (has_next) stage_load(kv0 + PF_KBLK);  // overlaps this tile's compute
-
-    if (wave_active && kv0 < wave_kmax) {
-      // ---- S = Q K^T: 4 col-tiles x 4 k-steps -----------------------------
-      f32x4 s[4];
-#pragma unroll
-      for (int n = 0; n < 4; n++) s[n] = f32x4{0, 0, 0, 0};
-#pragma unroll
-      for (int n = 0; n < 4; n++) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-          bf16x8 bk = *reinterpret_cast<const bf16x8*>(
-              &k_lds[n * 16 + frow][ks * 32 + fcol8]);
-          s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[ks], bk, s[n],
-                                                         0, 0, 0);
-        }
-      }
-      // ---- mask + online softmax ------------------------------------------
-      float alpha[4];
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int qrow = wq0 + crow4 + r;
-        const int qpos = ctx + qrow;
-        float smax = -INFINITY;
-        float pv[4];
-#pragma unroll
-        for (int n = 0; n < 4; n++) {
-          const int key = kv0 + n * 16 + frow;
-          float sv = s[n][r] * scale;
-          if (key > qpos || key >= seq_len || qrow >= q_len) sv = -INFINITY;
-          pv[n] = sv;
-          smax = fmaxf(smax, sv);
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1)
-          smax = fmaxf(smax, __shfl_xor(smax, off, 64));
-        const float m_new = fmaxf(m_r[r], smax);
-        alpha[r] = (m_new == -INFINITY) ? 1.0f : __expf(m_r[r] - m_new);
-        float psum = 0.0f;
-#pragma unroll
-        for (int n = 0; n < 4; n++) {
-          const float p = (pv[n] == -INFINITY) ? 0.0f : __expf(pv[n] - m_new);
-          psum += p;
-          p_lds[wid][crow4 + r][n * 16 + frow] = f32_to_bf16(p);
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1)
-          psum += __shfl_xor(psum, off, 64);
-        m_r[r] = m_new;
-        l_r[r] = l_r[r] * alpha[r] + psum;
-      }
-#pragma unroll
-      for (int n = 0; n < 8; n++) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) o_acc[n][r] *= alpha[r];
-      }
-      // ---- O += P V over the two 32-key halves ----------------------------
-      // (B-fragments from the tr16 image; per-lane tr address = image base
-      // + (l>>4)*128B + (l&15)*8B; each 32-key half needs TWO 8-read
-      // batches — one per 4 d-tiles — reusing one 16-VGPR tr[] set)
-      const unsigned vbase =
-          (unsigned)(unsigned long long)(&v_img[0][0]) +
-          ((lane >> 4) * 128u + (lane & 15) * 8u);
-      u32x2 tr[8];
-#define PF_TR8(OFF)                                                        \
-      asm volatile(                                                        \
-          "ds_read_b64_tr_b16 %[t0], %[a] offset:" #OFF "+0\n\t"           \
-          "ds_read_b64_tr_b16 %[t1], %[a] offset:" #OFF "+512\n\t"         \
-          "ds_read_b64_tr_b16 %[t2], %[a] offset:" #OFF "+1024\n\t"        \
-          "ds_read_b64_tr_b16 %[t3], %[a] offset:" #OFF "+1536\n\t"        \
-          "ds_read_b64_tr_b16 %[t4], %[a] offset:" #OFF "+2048\n\t"        \
-          "ds_read_b64_tr_b16 %[t5], %[a] offset:" #OFF "+2560\n\t"        \
-          "ds_read_b64_tr_b16 %[t6], %[a] offset:" #OFF "+3072\n\t"        \
-          "ds_read_b64_tr_b16 %[t7], %[a] offset:" #OFF "+3584\n\t"        \
-          "s_waitcnt lgkmcnt(0)"                                           \
-          : [t0] "=&v"(tr[0]), [t1] "=&v"(tr[1]), [t2] "=&v"(tr[2]),       \
-            [t3] "=&v"(tr[3]), [t4] "=&v"(tr[4]), [t5] "=&v"(tr[5]),       \
-            [t6] "=&v"(tr[6]), [t7] "=&v"(tr[7])                           \
-          : [a] "v"(vbase)                                                 \
-          : "memory")
-#define PF_PV4(HALF)                                                       \
-      do {                                                                 \
-        __builtin_amdgcn_sched_barrier(0);                                 \
-        _Pragma("unroll")                                                  \
-        for (int nn = 0; nn < 4; nn++) {                                   \
-          const int n = (HALF) * 4 + nn;                                   \
-          bf16x8 bv;                                                       \
-          unsigned* bw = reinterpret_cast<unsigned*>(&bv);                 \
-          bw[0] = tr[2 * nn][0];                                           \
-          bw[1] = tr[2 * nn][1];                                           \
-          bw[2] = tr[2 * nn + 1][0];                                       \
-          bw[3] = tr[2 * nn + 1][1];                                       \
-          o_acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(               \
-              pa, bv, o_acc[n], 0, 0, 0);                                  \
-        }                                                                  \
-      } while (0)
-      {
-        bf16x8 pa = *reinterpret_cast<const bf16x8*>(
-            &p_lds[wid][frow][fcol8]);
-        PF_TR8(0);     PF_PV4(0);
-        PF_TR8(4096);  PF_PV4(1);
-      }
-      {
-        bf16x8 pa = *reinterpret_cast<const bf16x8*>(
-            &p_lds[wid][frow][32 + fcol8]);
-        PF_TR8(8192);  PF_PV4(0);
-        PF_TR8(12288); PF_PV4(1);
-      }
-#undef PF_TR8
-#undef PF_PV4
-    }
-    // single buffer: all waves must be done READING this tile before the
-    // next tile's write lands (the co-resident second workgroup hides
-    // both barriers)
+  int pages = 0;
+  if (t_begin < t_end) {
+    pages = pages_from(t_begin);
+    stage(t_begin, __builtin_amdgcn_readlane(pages, 0), 0);
+  }
+  for (int t = t_begin; t < t_end; t++) {
+    const int buf = (t - t_begin) & 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (has_next) {
-      stage_write(kv0 + PF_KBLK);
-      __syncthreads();
+    if (t + 1 < t_end) {
+      if (t + 1 - tb == 64) {
+        tb += 64;
+        pages = pages_from(tb);
+      }
+      stage(t + 1, __builtin_amdgcn_readlane(pages, t + 1 - tb), buf ^ 1);
     }
+    const int k0 = t * PF_KT;
+    if (!wave_on || k0 >= wmax) continue;
+    const lds_u16* kt = (const lds_u16*)kv_lds + buf * 2 * TILE;
+    const lds_u16* vt = kt + TILE;
+
+    // ---- scores: keys [32 i, 32 i + 32) of the tile ------------------------
+    // (two independent chains of products, four K rows in flight)
+    f32x16 s[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[i][r] = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const bf16x8 a = *reinterpret_cast<const lds_bf16x8*>(
+            kt + ((kbase ^ (ks << 4)) + i * 32 * D));
+        s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], s[i], 0, 0,
+                                                       0);
+      }
+    }
+    if (k0 + PF_KT > wmin) {                   // uniform: tile on the diagonal
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int key = k0 + i * 32 + 16 * (r >> 3) + 8 * h +
+                          4 * ((r >> 2) & 1) + (r & 3);
+          if (key >= limit) s[i][r] = -INFINITY;
+        }
+    }
+    // ---- online softmax ----------------------------------------------------
+    float mt = s[0][0];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) mt = fmaxf(mt, s[i][r]);
+    mt = pair_max(mt);
+    if (__any(mt > m)) {
+      const float m_new = fmaxf(m, mt);
+      const float alpha =
+          __builtin_amdgcn_exp2f((m - (m_new == -INFINITY ? 0.f : m_new)) * c);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < DT; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o_acc[i][r] *= alpha;
+    }
+    const float mc = m == -INFINITY ? 0.0f : m * c;
+    bf16x8 p[TERMS][4];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        float a = __builtin_amdgcn_exp2f(fmaf(s[i][r], c, -mc));
+        float b = __builtin_amdgcn_exp2f(fmaf(s[i][r + 1], c, -mc));
+        l += a + b;
+#pragma unroll
+        for (int x = 0; x < TERMS; x++) {
+          const unsigned u = pack_bf16(a, b);
+          reinterpret_cast<unsigned*>(
+              &p[x][i * 2 + (r >> 3)])[(r & 7) >> 1] = u;
+          a -= __uint_as_float(u << 16);       // what is left, exactly
+          b -= __uint_as_float(u & 0xffff0000u);
+        }
+      }
+    // ---- O^T += V^T P^T ------------------------------------------------------
+#pragma unroll
+    for (int st = 0; st < 4; st++)
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) {
+        const lds_u16* vp = vt + ((vbase ^ (dt << 5)) + st * 16 * D);
+        s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)vp);
+        s16x4 hi =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp + 4 * D));
+        const bf16x8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+        for (int x = 0; x < TERMS; x++)
+          o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              a, p[x][st], o_acc[dt], 0, 0, 0);
+      }
   }
 
-  // ---- epilogue ------------------------------------------------------------
-  if (wave_active) {
+  // ---- epilogue: o_acc[dt][r] = O[row][dt*32 + 8*(r>>2) + 4h + (r&3)] --------
+  l = pair_sum(l);
+  if (!row_ok) return;
+  const long grow = (long)(q_start + qi) * n_qheads + head;
+  if (n_part == 1) {
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    unsigned short* o = out + (long)(q_start + qi) * out_stride +
+                        (long)head * D + 4 * h;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int qrow = wq0 + crow4 + r;
-      if (qrow >= q_len) continue;
-      const float inv = (l_r[r] > 0.0f) ? 1.0f / l_r[r] : 0.0f;
-      const long obase =
-          (long)(q_start + qrow) * out_stride + (long)qh * PF_D;
+    for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-      for (int n = 0; n < 8; n++)
-        out[obase + n * 16 + frow] = f32_to_bf16(o_acc[n][r] * inv);
-    }
+      for (int r = 0; r < 16; r += 4) {
+        uint2 x;
+        x.x = pack_bf16(o_acc[dt][r] * inv, o_acc[dt][r + 1] * inv);
+        x.y = pack_bf16(o_acc[dt][r + 2] * inv, o_acc[dt][r + 3] * inv);
+        *reinterpret_cast<uint2*>(o + dt * 32 + 2 * r) = x;
+      }
+    return;
   }
+  const long slot = grow * n_part + part;
+  if (h == 0) {
+    ws_ml[slot * 2] = m * c;
+    ws_ml[slot * 2 + 1] = l;
+  }
+  if (t_begin >= t_end) return;              // an empty part: l = 0
+  float* o = ws_o + slot * D + 4 * h;
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *reinterpret_cast<float4*>(o + dt * 32 + 2 * r) =
+          make_float4(o_acc[dt][r], o_acc[dt][r + 1], o_acc[dt][r + 2],
+                      o_acc[dt][r + 3]);
 }
 
-void launch_paged_attn_prefill(unsigned short* out, const unsigned short* q,
+// out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
+// row, four columns each
+template <int D>
+__global__ __launch_bounds__(256) void paged_attn_prefill_merge_kernel(
+    unsigned short* __restrict__ out, const float* __restrict__ ws_o,
+    const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
+    const long out_stride, const long rows) {
+  constexpr int LPR = D / 4;
+  const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
+  const int col = (threadIdx.x % LPR) * 4;
+  if (row >= rows) return;
+  const float* ml = ws_ml + row * n_part * 2;
+  float M = -INFINITY;
+  for (int p = 0; p < n_part; p++) M = fmaxf(M, ml[2 * p]);
+  if (M == -INFINITY) M = 0.0f;
+  float L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int p = 0; p < n_part; p++) {
+    if (ml[2 * p + 1] <= 0.0f) continue;     // nothing was written
+    const float w = __builtin_amdgcn_exp2f(ml[2 * p] - M);
+    L += ml[2 * p + 1] * w;
+    const float4 x = *reinterpret_cast<const float4*>(
+        ws_o + (row * n_part + p) * D + col);
+    a[0] += x.x * w; a[1] += x.y * w; a[2] += x.z * w; a[3] += x.w * w;
+  }
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  uint2 y;
+  y.x = pack_bf16(a[0] * inv, a[1] * inv);
+  y.y = pack_bf16(a[2] * inv, a[3] * inv);
+  const long tok = row / n_qheads;
+  *reinterpret_cast<uint2*>(out + tok * out_stride +
+                            (row - tok * n_qheads) * D + col) = y;
+}
+
+// Row tiles a batch has at most, and the parts its keys are split into: about
+// two workgroups per CU are wanted, and a part under eight tiles of keys costs
+// more in its merge than it saves.
+static long pf_tiles(long tokens, int n_seqs, int G) {
+  return tokens * G / PF_ROWS + n_seqs;
+}
+int paged_attn_prefill_parts(long tokens, int n_seqs, int G, int n_kv,
+                             int max_blocks) {
+  const long wgs = pf_tiles(tokens, n_seqs, G) * n_kv;
+  const long most = (long)max_blocks * PF_BS / (8 * PF_KT);
+  long p = wgs > 0 ? 512 / wgs : 1;
+  if (p > most) p = most;
+  return (int)(p < 1 ? 1 : p > 16 ? 16 : p);
+}
+
+void launch_paged_attn_prefill(unsigned short* out, float* ws_o, float* ws_ml,
+                               const unsigned short* q,
                                const unsigned short* k_cache,
                                const unsigned short* v_cache,
                                const int* block_tables, const int* cu_q,
-                               const int* seq_lens, const int* tile_seq,
-                               const int* tile_q0, int total_tiles, float scale,
-                               int n_qheads, int n_kv_heads,
-                               int max_blocks_per_seq, long q_stride,
-                               long out_stride, hipStream_t stream) {
-  dim3 grid(total_tiles, n_qheads), block(512);
-  hipLaunchKernelGGL(paged_attn_prefill_kernel, grid, block, 0, stream, out, q,
-                     k_cache, v_cache, block_tables, cu_q, seq_lens, tile_seq,
-                     tile_q0, scale, n_qheads, n_kv_heads, max_blocks_per_seq,
-                     q_stride, out_stride);
+                               const int* seq_lens, long tokens, int n_seqs,
+                               float scale, int n_qheads, int n_kv, int D,
+                               int max_blocks, long q_stride, long out_stride,
+                               int n_part, hipStream_t stream) {
+  const int G = n_qheads / n_kv;
+  if (tokens == 0 || n_seqs == 0) return;
+  dim3 grid((unsigned)(pf_tiles(tokens, n_seqs, G) * n_kv * n_part));
+#define PF_LAUNCH(DV, TERMS)                                                   \
+  do {                                                                         \
+    hipLaunchKernelGGL((paged_attn_prefill_kernel<DV, TERMS>), grid,           \
+                       dim3(256), 0, stream, out, ws_o, ws_ml, q, k_cache,     \
+                       v_cache, block_tables, cu_q, seq_lens, n_seqs, scale, G, \
+                       n_kv, max_blocks, q_stride, out_stride, n_part);        \
+    if (n_part > 1) {                                                          \
+      const long rows = tokens * n_qheads;                                     \
+      hipLaunchKernelGGL((paged_attn_prefill_merge_kernel<DV>),                \
+                         dim3((unsigned)((rows * (DV / 4) + 255) / 256)),      \
+                         dim3(256), 0, stream, out, ws_o, ws_ml, n_qheads,     \
+                         n_part, out_stride, rows);                            \
+    }                                                                          \
+  } while (0)
+  // 64-wide heads ran on fp32 weights before they had a kernel and still do
+  if (D == 128) PF_LAUNCH(128, 1);
+  else PF_LAUNCH(64, 3);
+#undef PF_LAUNCH
 }
 
 // ---------------------------------------------------------------------------------

@@ -211,9 +211,8 @@ class PrefillGraphRunner:
         only pad rows can see);
       * positions run chunk_start..chunk_start+B-1, so the graph is only
         used when chunk_start + B <= max_model_len (rope table bound).
-    Tile decomposition is precomputed per bucket (meta.prefill_tiles) —
-    deriving it from cu_q calls .cpu(), and a sync inside capture aborts
-    the capture."""
+    The attention kernel finds its rows from cu_q on the device: nothing in
+    the forward waits for the host."""
 
     def __init__(self, model, kv_caches, device, max_model_len: int = 4096,
                  max_tokens: int = 8192, pool=None):
@@ -248,15 +247,12 @@ class PrefillGraphRunner:
                                      device=dev),
         )
         cu_q = torch.tensor([0, B], dtype=torch.int32, device=dev)
-        tiles = (torch.zeros((B + 127) // 128, dtype=torch.int32, device=dev),
-                 torch.arange(0, B, 128, dtype=torch.int32, device=dev))
         meta = AttnMetadata(
             num_prefill_tokens=B, num_decode_tokens=0,
             slot_mapping=static["slot_mapping"],
             cu_q=cu_q,
             prefill_seq_lens=static["seq_lens"],
-            prefill_block_tables=static["block_tables"],
-            prefill_tiles=tiles)
+            prefill_block_tables=static["block_tables"])
 
         def fwd():
             return self.model(static["input_ids"], static["positions"],

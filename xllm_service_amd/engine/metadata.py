@@ -24,9 +24,8 @@ class AttnMetadata:
     prefill_seq_lens: Optional[torch.Tensor] = None   # [n_prefill] int32 (ctx+chunk)
     prefill_block_tables: Optional[torch.Tensor] = None  # [n_prefill, max_blk] int32
 
-    # precomputed prefill tile decomposition (tile_seq, tile_q0) — set by
-    # the prefill graph runner so capture never calls cu_q.cpu() (a sync
-    # inside hipGraph capture aborts it); None = derive from cu_q
+    # a prefill tile decomposition (tile_seq, tile_q0); the kernel finds its
+    # rows from cu_q on the device and does not need one
     prefill_tiles: Optional[tuple] = None
 
     # decode half

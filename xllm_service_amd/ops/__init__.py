@@ -134,25 +134,37 @@ def paged_attn_decode(q, k_cache, v_cache, block_tables, seq_lens, scale,
     return res
 
 
-def _prefill_tiles(cu_q):
-    """Host-side tile decomposition for the prefill kernel (128 q rows/WG)."""
-    tile_seq, tile_q0 = [], []
-    for s in range(len(cu_q) - 1):
-        qlen = int(cu_q[s + 1]) - int(cu_q[s])
-        for q0 in range(0, qlen, 128):
-            tile_seq.append(s)
-            tile_q0.append(q0)
-    return tile_seq, tile_q0
+def _prefill_native(q, k_cache, v_cache, block_tables, cu_q, seq_lens, out):
+    """Whether the MFMA prefill kernel takes this call. 128-wide heads always
+    do (what it cannot take raises there); 64-wide ones where layout, types and
+    alignment are the kernel's."""
+    D = k_cache.shape[-1]
+    if D != 64:
+        return D == 128
+    heads = [q] if out is None else [q, out]
+    return (all(t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous()
+                and t.data_ptr() % 16 == 0 for t in (k_cache, v_cache))
+            and all(t.dtype == torch.bfloat16 and t.dim() == 3
+                    and t.shape[2] == D and t.stride(2) == 1
+                    and t.stride(1) == D and t.stride(0) % 8 == 0
+                    and t.data_ptr() % 16 == 0 for t in heads)
+            and all(t.is_cuda and t.dtype == torch.int32 and t.is_contiguous()
+                    for t in (block_tables, cu_q, seq_lens))
+            and k_cache.shape[2] == 16 and v_cache.shape == k_cache.shape
+            and q.shape[1] % k_cache.shape[1] == 0
+            and seq_lens.shape[0] == cu_q.shape[0] - 1
+            and block_tables.shape[0] >= seq_lens.shape[0])
 
 
 def paged_attn_prefill(q, k_cache, v_cache, block_tables, cu_q, seq_lens,
                        scale, out=None, tiles=None):
+    """tiles: accepted from callers that made a tile list; the kernel finds
+    its rows from cu_q on the device."""
     if q.is_cuda:
         _require_ext()
-        if k_cache.shape[-1] != 128:
-            # the MFMA prefill kernel is head_dim-128 only; other head dims
-            # (e.g. OPT/tiny-VL 64) run an eager torch path ON GPU — loud
-            # and documented, not a silent bypass of the native 128 path
+        if not _prefill_native(q, k_cache, v_cache, block_tables, cu_q,
+                               seq_lens, out):
+            # other head widths run an eager torch path ON GPU
             res = ref.paged_attn_prefill(q, k_cache, v_cache, block_tables,
                                          cu_q, seq_lens, scale)
             if out is not None:
@@ -161,14 +173,8 @@ def paged_attn_prefill(q, k_cache, v_cache, block_tables, cu_q, seq_lens,
             return res
         if out is None:
             out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        dev = q.device
-        if tiles is None:
-            tile_seq, tile_q0 = _prefill_tiles(cu_q.cpu())
-            tiles = (torch.tensor(tile_seq, dtype=torch.int32, device=dev),
-                     torch.tensor(tile_q0, dtype=torch.int32, device=dev))
-        _ops.paged_attn_prefill(
-            out, q, k_cache, v_cache, block_tables, cu_q, seq_lens,
-            tiles[0], tiles[1], scale)
+        _ops.paged_attn_prefill(out, q, k_cache, v_cache, block_tables, cu_q,
+                                seq_lens, scale)
         return out
     res = ref.paged_attn_prefill(q, k_cache, v_cache, block_tables, cu_q,
                                  seq_lens, scale)

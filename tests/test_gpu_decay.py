@@ -1,0 +1,88 @@
+"""Decayed linear attention of bf16 prompt rows at the edges of its chunks and
+tiles, against the token recurrence in fp64.
+
+The features silu(x) are rounded to bf16; inputs whose feature lies within
+2^-6 of an ulp of the middle between two bf16 numbers become zero, so that
+oracle and kernel round alike. What remains are 32-bit products and sums:
+every output may be off by 2^-20 of the same sum over absolute values (a
+weight is a product of two rounded powers; up to 2^4 roundings in a chain)."""
+import pytest
+import torch
+
+from xllm_service_amd.ops import hybrid as H
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+
+
+def features(x):
+    y = x.to(F64) * torch.sigmoid(x.to(F64))
+    ulp = 2.0 ** (torch.floor(torch.log2(y.abs().clamp(min=1e-30))) - 7)
+    frac = (y.abs() / ulp) % 1.0
+    x = torch.where((frac - 0.5).abs() < 2.0 ** -6, torch.zeros_like(x), x)
+    y = x.to(F64) * torch.sigmoid(x.to(F64))
+    return x, y.to(torch.bfloat16).to(F64)
+
+
+def recur(q, k, v, a, S):
+    """[n, H, *] features, S [H, D, V]: outputs and the state after."""
+    out = []
+    for t in range(q.shape[0]):
+        S = a[:, None, None] * S + k[t][:, :, None] * v[t][:, None, :]
+        out.append((q[t][:, None, :] @ S)[:, 0])
+    return torch.stack(out), S
+
+
+def run(D, V, lens, ctx, slots, decay, bound, seed):
+    g = torch.Generator().manual_seed(seed)
+    heads, T = len(decay), sum(lens)
+    width = heads * (2 * D + V)
+    rows = torch.randn(T, width + 8, generator=g).to(torch.bfloat16)
+    rows[:, :width], f = features(rows[:, :width])
+    cut = (0, heads * D, 2 * heads * D, width)
+    a = torch.tensor(decay, dtype=torch.float32)
+    state = torch.randn(max(slots) + 2, heads, D, V, generator=g)
+    sd, rd = state.cuda(), rows.cuda()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    out = torch.full((T, heads, V), 9.0, device="cuda")
+    starts = [0]
+    for n in lens:
+        starts.append(starts[-1] + n)
+    H.decay_attn(*(rd[:, x:y] for x, y in zip(cut, cut[1:])), a.cuda(), sd,
+                 torch.tensor(slots, **i32), torch.tensor(starts, **i32),
+                 torch.tensor(ctx, **i32), out, max_q_len=bound)
+    out, sd, used = out.cpu().to(F64), sd.cpu(), set()
+    for s, (n, c, slot) in enumerate(zip(lens, ctx, slots)):
+        x = [f[starts[s]:starts[s + 1], p:e].reshape(n, heads, -1)
+             for p, e in zip(cut, cut[1:])]
+        S = state[slot].to(F64) if slot >= 0 and c > 0 else torch.zeros(
+            heads, D, V, dtype=F64)
+        a64 = a.to(F64)
+        want, after = recur(*x, a64, S)
+        big, top = recur(*(z.abs() for z in x), a64.abs(), S.abs())
+        off = (out[starts[s]:starts[s + 1]] - want).abs() - 2.0 ** -20 * big
+        assert off.max() <= 1e-30, f"sequence {s}: over by {off.max():.3g}"
+        if slot >= 0:
+            used.add(slot)
+            off = (sd[slot].to(F64) - after).abs() - 2.0 ** -20 * top
+            assert off.max() <= 1e-30, f"state {s}: over by {off.max():.3g}"
+    for slot in range(state.shape[0]):
+        if slot not in used:
+            assert torch.equal(sd[slot], state[slot])
+
+
+@pytest.mark.parametrize("D,V", [(128, 128), (64, 128), (128, 64), (64, 64)])
+@pytest.mark.parametrize("lens,bound", [
+    ([1, 15, 16, 17], 17), ([31, 32, 33, 128], 128),      # one chunk each
+    ([127, 128, 129, 1], 129), ([64, 65, 300, 256], 0),   # chunks and a scan
+])
+def test_prompt_rows(D, V, lens, bound):
+    """Fresh and continued sequences, one without a slot."""
+    run(D, V, lens, [0, 7, 0, 40], [3, 0, 1, -1], [0.999, 0.75, 1.0], bound,
+        sum(lens) + D + V)
+
+
+def test_many_chunks_and_hard_decays():
+    """More chunks than the scan holds in flight; decays whose powers leave
+    fp32's normal range within a chunk, and none at all."""
+    run(128, 128, [1300, 200], [0, 9], [0, 2], [0.3, 0.0, 0.996], 1300, 4)

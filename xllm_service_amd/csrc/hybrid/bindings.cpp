@@ -69,6 +69,13 @@ void launch_latent_attn_mfma(float*, float*, float*, const unsigned short*,
                              const unsigned short*, const int*, const int*,
                              const int*, int, int, int, int, int, int, int,
                              float, int, int, hipStream_t);
+long decay_attn_mfma_chunks(long, long);
+int decay_attn_mfma_chunk();
+void launch_decay_attn_mfma(float*, const unsigned short*,
+                            const unsigned short*, const unsigned short*,
+                            const float*, float*, const int*, const int*,
+                            const int*, long, int, int, int, int, long, long,
+                            long, float*, hipStream_t);
 template <typename T>
 void launch_decay_attn(float*, const T*, const T*, const T*, const float*,
                        float*, const int*, const int*, const int*, int, int,
@@ -619,6 +626,32 @@ void decay_attn(Tensor out, Tensor q, Tensor k, Tensor v, Tensor decay,
     cu = ptr<int>(*cu_q);
   } else {
     TORCH_CHECK(n_seqs == T, "decode: one sequence per token");
+  }
+  // prompt rows in bf16 with 64- or 128-wide heads: the matrix-pipe form,
+  // while its scratch stays under 2 GiB
+  auto rows8 = [](const Tensor& t) {
+    return t.stride(0) % 8 == 0 && t.stride(1) == 1 &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  auto aligned = [](const Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  if (cu != nullptr && is_bf16(q) && (D == 64 || D == 128) &&
+      (Dv == 64 || Dv == 128) && rows8(q) && rows8(k) && rows8(v) &&
+      aligned(out) && aligned(state)) {
+    const long longest = max_q_len > 0 ? std::min<long>(max_q_len, T) : T;
+    const bool one = longest <= hy::decay_attn_mfma_chunk();
+    const long n = hy::decay_attn_mfma_chunks(T, n_seqs) * H * D * Dv;
+    if (one || n * 4 <= (1L << 31)) {
+      Tensor ws;
+      if (!one) ws = torch::empty({n}, state.options());
+      hy::launch_decay_attn_mfma(
+          ptr<float>(out), ptr<bf>(q), ptr<bf>(k), ptr<bf>(v),
+          ptr<float>(decay), ptr<float>(state), ptr<int>(slots), cu,
+          ptr<int>(ctx_lens), T, n_seqs, H, D, Dv, q.stride(0), k.stride(0),
+          v.stride(0), one ? nullptr : ptr<float>(ws), cur());
+      return;
+    }
   }
   int chunk = 128, max_chunks = 1;
   Tensor ws;

@@ -36,7 +36,7 @@
 // product j is column (j / 4) * 64 + m * 4 + j % 4, so a lane fetches the
 // operands of four products with one 16 B read and ends up with four
 // neighbouring output columns. The key rows of pass 1 are dealt the same way.
-#include "hybrid_common.h"
+#include "recurrent_chunks.h"
 
 namespace xllm {
 namespace hyb {
@@ -130,24 +130,6 @@ XLLM_DEV void rt_stage(float* dst, const RTRows<T>& R, long row0, int rows,
   }
 }
 
-// chunk number b of the batch -> sequence, its chunk, first token, length
-XLLM_DEV bool rt_locate(int b, const int* cu_q, int n_seqs, int* s, int* c,
-                        int* t0, int* len) {
-  int acc = 0;
-  for (int i = 0; i < n_seqs; ++i) {
-    const int a = cu_q[i], e = cu_q[i + 1];
-    const int nc = (e - a + RT_C - 1) / RT_C;
-    if (b < acc + nc) {
-      *s = i; *c = b - acc;
-      *t0 = a + *c * RT_C;
-      *len = min(RT_C, e - *t0);
-      return true;
-    }
-    acc += nc;
-  }
-  return false;
-}
-
 // ---- pass 1: what a chunk adds to the state -----------------------------------
 // ws [chunks][H][D][Dv]; DP, VP: widths padded to the tile grid; blockIdx.z
 // is the block of VP value columns
@@ -164,7 +146,7 @@ __launch_bounds__(256, DP == 256 ? 2 : 4) retention_sum_kernel(
   float* ks = smem;                               // [RT_S][LK]
   float* vs = ks + RT_S * LK;                     // [RT_S][LV]
   int s, c, t0, len;
-  if (!rt_locate(blockIdx.x, cu_q, n_seqs, &s, &c, &t0, &len)) return;
+  if (!chunk_locate<RT_C>(blockIdx.x, cu_q, n_seqs, &s, &c, &t0, &len)) return;
   const int h = blockIdx.y, v0 = blockIdx.z * VP;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, n = lane & 15;
@@ -228,54 +210,6 @@ __launch_bounds__(256, DP == 256 ? 2 : 4) retention_sum_kernel(
     }
 }
 
-// ---- scan: one thread per (sequence, state element) -----------------------------
-__global__ void retention_scan_kernel(float* __restrict__ ws,
-                                      float* __restrict__ state,
-                                      const float* __restrict__ decay,
-                                      const int* __restrict__ slots,
-                                      const int* __restrict__ cu_q,
-                                      const int* __restrict__ ctx_lens,
-                                      int heads, long per_head) {
-  const int s = blockIdx.y;
-  const long per_seq = per_head * heads;
-  const long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (e >= per_seq) return;
-  long base = 0;
-  for (int i = 0; i < s; ++i)
-    base += (cu_q[i + 1] - cu_q[i] + RT_C - 1) / RT_C;
-  const int qlen = cu_q[s + 1] - cu_q[s];
-  if (qlen <= 0) return;
-  const int full = qlen / RT_C, rest = qlen - full * RT_C;
-  const int slot = slots[s];
-  const float a = decay[(int)(e / per_head)];
-  float S = (slot >= 0 && ctx_lens[s] > 0) ? state[slot * per_seq + e] : 0.f;
-  const float a_full = powf(a, (float)RT_C);
-  float* w = ws + base * per_seq + e;
-  constexpr int U = 8;                    // records in flight
-  int c = 0;
-  for (; c + U <= full; c += U) {
-    float x[U];
-#pragma unroll
-    for (int i = 0; i < U; ++i) x[i] = w[(c + i) * per_seq];
-#pragma unroll
-    for (int i = 0; i < U; ++i) {
-      w[(c + i) * per_seq] = S;
-      S = a_full * S + x[i];
-    }
-  }
-  for (; c < full; ++c) {
-    const float x = w[c * per_seq];
-    w[c * per_seq] = S;
-    S = a_full * S + x;
-  }
-  if (rest) {
-    const float x = w[c * per_seq];
-    w[c * per_seq] = S;
-    S = powf(a, (float)rest) * S + x;
-  }
-  if (slot >= 0) state[slot * per_seq + e] = S;
-}
-
 // four neighbouring outputs of one head, normed and gated
 template <typename T, bool VEC>
 XLLM_DEV void rt_store4(T* dst, const T* gate, const f32x4& o, float rs,
@@ -313,7 +247,7 @@ __global__ void __launch_bounds__(256, 3) retention_out_kernel(
   float* vs = ks + RT_S * LK;                     // [RT_S][LV]
   float* ss = smem;                               // [64][LV], later
   int s, c, t0, len;
-  if (!rt_locate(blockIdx.x, cu_q, n_seqs, &s, &c, &t0, &len)) return;
+  if (!chunk_locate<RT_C>(blockIdx.x, cu_q, n_seqs, &s, &c, &t0, &len)) return;
   const int h = blockIdx.y, v0 = blockIdx.z * VP;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int g = lane >> 4, n = lane & 15;
@@ -611,10 +545,10 @@ static void rt_prefill(T* out, long out_stride, float* o_raw, const T* gate,
                      lds, st, ws, K, V, rot, k_scale, decay, cu_q, n_seqs,
                      heads, D, Dv);
   const long per_head = (long)D * Dv, per_seq = per_head * heads;
-  hipLaunchKernelGGL(retention_scan_kernel,
+  hipLaunchKernelGGL((chunk_scan_kernel<RT_C>),
                      dim3((unsigned)((per_seq + 255) / 256), n_seqs),
                      dim3(256), 0, st, ws, state, decay, slots, cu_q, ctx_lens,
-                     heads, per_head);
+                     heads, per_head, false);
 #define RT_OUT(FUSED)                                                         \
   hipLaunchKernelGGL((retention_out_kernel<T, DP, VP, FUSED, VEC>), grid,     \
                      dim3(256), lds2, st, out, out_stride, o_raw, gate,       \

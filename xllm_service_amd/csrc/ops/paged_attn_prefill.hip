@@ -21,10 +21,6 @@
 //   O^T[d][row] += V^T P^T       A = V^T by hardware transpose reads, B = the
 //                                lane's own weights, rounded to bf16: no trip
 //                                through LDS
-// The C layout of S^T hands lane half h the rows 8i + 4h + r; feeding key
-// 16(i>>1) + 8h + 4(i&1) + r as A row 8i + 4h + r makes those the keys
-// 16t + 8h + 0..7 that the B operand of step t wants of that lane.
-//
 // K and V tiles go from memory straight to LDS (no registers, no ds_write),
 // double-buffered with one barrier per tile. The loads place 16 B per lane in
 // lane order, so rows cannot be padded; the 16 B chunks of a row are permuted
@@ -46,47 +42,16 @@
 // made on the host; before: 110 us and 48 us of copies and waiting. 8 prompts
 // of 109-438 tokens, 12 heads of 64: 11 us, an eager loop before: 14 ms.
 //
-// Fragments (lane l, h = l >> 5) of v_mfma_f32_32x32x16_bf16:
-//   A[l&31][h*8 + j], B[h*8 + j][l&31], C[8*(r>>2) + 4h + (r&3)][l&31]
+// Fragment layouts, the order of the keys and of the LDS images: mfma_rows.h.
 //
 // Parity: reference engine's paged-attention prefill.
-#include "common.h"
+#include "mfma_rows.h"
 
 namespace xllm {
-
-typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
-typedef __attribute__((ext_vector_type(2))) __bf16 bfx2;
-typedef __attribute__((ext_vector_type(2))) float fx2;
-typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
 
 #define PF_ROWS 128        // rows per workgroup
 #define PF_KT 64           // keys per tile
 #define PF_BS 16           // cache block size
-
-typedef __attribute__((address_space(3))) unsigned short lds_u16;
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-typedef __attribute__((address_space(3))) void lds_void;
-typedef const __attribute__((address_space(1))) void glb_void;
-
-// larger of a lane's and its partner's (l ^ 32) value
-XLLM_DEV float pair_max(float v) {
-  const unsigned u = __float_as_uint(v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-XLLM_DEV float pair_sum(float v) {
-  const unsigned u = __float_as_uint(v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-XLLM_DEV unsigned pack_bf16(float a, float b) {
-  const fx2 f = {a, b};
-  const bfx2 x = __builtin_convertvector(f, bfx2);
-  return __builtin_bit_cast(unsigned, x);
-}
 
 // Row tile `b` of the batch -> sequence and tile within it; later tiles of a
 // sequence (more keys) come first. False: past the last one. One wave looks
@@ -197,9 +162,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
 
   f32x16 o_acc[DT];
 #pragma unroll
-  for (int i = 0; i < DT; i++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) o_acc[i][r] = 0.0f;
+  for (int i = 0; i < DT; i++) o_acc[i] = mr_zero();
   float m = -INFINITY, l = 0.0f;
 
   // ---- staging: a wave moves the tile's page `wid` ---------------------------
@@ -210,8 +173,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
   // byte offset in a page of what this lane moves: row r of the page, its
   // chunk permuted by the row's key
   auto off_of = [&](int r, int key, bool val) {
-    const int x = val ? (D == 128 ? (key & 3) << 2 : ((key >> 1) & 1) << 2)
-                      : (D == 128 ? key & 15 : (key >> 1) & 7);
+    const int x = val ? mr_swz_cols<D>(key) : mr_swz_rows<D>(key);
     return (unsigned)(r * (2 * D) + ((spos ^ x) << 4));
   };
   unsigned koff[NI], voff[NI];
@@ -256,16 +218,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
     }
   };
 
-  // ---- LDS addresses (elements) --------------------------------------------
-  // K row of A row m = lane & 31, chunk 2 ks + h
-  const int km = ((c32 >> 4) << 4) | (((c32 >> 2) & 1) << 3) |
-                 (((c32 >> 3) & 1) << 2) | (c32 & 3);
-  const int kbase =
-      km * D + ((h ^ (D == 128 ? (km & 15) : ((km >> 1) & 7))) << 3);
-  // V: rows 16t + 8h + (i >> 2) (+4), columns dt*32 + dhalf*16 + (i & 3)*4
-  const int vi = lane & 15, dh = (lane >> 4) & 1;
-  const int vbase = (8 * h + (vi >> 2)) * D + dh * 16 + (vi & 3) * 4 +
-                    ((D == 128 ? (vi >> 2) : (vi >> 3)) << 5);
+  const int kbase = mr_row_base<D>(lane), vbase = mr_col_base<D>(lane);
 
   int pages = 0;
   if (t_begin < t_end) {
@@ -290,30 +243,21 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
 
     // ---- scores: keys [32 i, 32 i + 32) of the tile ------------------------
     // (two independent chains of products, four K rows in flight)
-    f32x16 s[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) s[i][r] = 0.0f;
+    f32x16 s[2] = {mr_zero(), mr_zero()};
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
 #pragma unroll
-      for (int i = 0; i < 2; i++) {
-        const bf16x8 a = *reinterpret_cast<const lds_bf16x8*>(
-            kt + ((kbase ^ (ks << 4)) + i * 32 * D));
-        s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], s[i], 0, 0,
-                                                       0);
-      }
+      for (int i = 0; i < 2; i++)
+        s[i] = mr_mma(*reinterpret_cast<const lds_bf16x8*>(
+                          kt + (kbase ^ (ks << 4)) + i * 32 * D),
+                      qf[ks], s[i]);
     }
     if (k0 + PF_KT > wmin) {                   // uniform: tile on the diagonal
 #pragma unroll
       for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int key = k0 + i * 32 + 16 * (r >> 3) + 8 * h +
-                          4 * ((r >> 2) & 1) + (r & 3);
-          if (key >= limit) s[i][r] = -INFINITY;
-        }
+        for (int r = 0; r < 16; r++)
+          if (k0 + i * 32 + mr_key_of(r, h) >= limit) s[i][r] = -INFINITY;
     }
     // ---- online softmax ----------------------------------------------------
     float mt = s[0][0];
@@ -347,8 +291,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
           const unsigned u = pack_bf16(a, b);
           reinterpret_cast<unsigned*>(
               &p[x][i * 2 + (r >> 3)])[(r & 7) >> 1] = u;
-          a -= __uint_as_float(u << 16);       // what is left, exactly
-          b -= __uint_as_float(u & 0xffff0000u);
+          drop_bf16(a, b, u);
         }
       }
     // ---- O^T += V^T P^T ------------------------------------------------------
@@ -356,15 +299,10 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
     for (int st = 0; st < 4; st++)
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) {
-        const lds_u16* vp = vt + ((vbase ^ (dt << 5)) + st * 16 * D);
-        s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)vp);
-        s16x4 hi =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vp + 4 * D));
-        const bf16x8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        const bf16x8 a = mr_cols<D>(vt + (vbase ^ (dt << 5)) + st * 16 * D);
 #pragma unroll
         for (int x = 0; x < TERMS; x++)
-          o_acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              a, p[x][st], o_acc[dt], 0, 0, 0);
+          o_acc[dt] = mr_mma(a, p[x][st], o_acc[dt]);
       }
   }
 

@@ -1,5 +1,5 @@
-"""Paged attention of prompt rows at the edges of its tiles, pages and key
-parts, against fp64 on the CPU. Results are bf16, off by up to 2^-9 of
+"""Paged attention of prompt rows and of decoded rows at the edges of their
+tiles, pages and key parts, against fp64 on the CPU. Results are bf16, off by up to 2^-9 of
 themselves. The weights that meet 128-wide values are rounded to bf16 as well:
 2^-9 of the weighted sum of |v|; twice both is allowed (the weights' sum is not
 rounded the same way). 64-wide heads keep 32-bit weights: 2^-18 for their
@@ -123,3 +123,41 @@ def test_prefill_needs_no_host():
         graph.replay()
         torch.cuda.synchronize()
         check(out, *want(q, k, v, table, lens, ctx, 0.1))
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("keys,kv_heads,per", [
+    ([1], 1, 1), ([15, 16, 17, 31, 32, 33], 2, 8),          # pages and tiles
+    ([127, 128, 129, 255, 256, 257, 700], 4, 7),            # waves
+    ([2049, 5, 4500], 3, 2), ([9001], 2, 4),                # parts
+    ([40 + 7 * i for i in range(70)], 4, 3),                # many pairs
+    ([18000, 33], 1, 5),              # over 32 tiles of one wave
+])
+def test_decode_edges(dim, keys, kv_heads, per):
+    ctx = [n - 1 for n in keys]
+    rows, k, v, table = make([1] * len(keys), ctx, kv_heads, per, dim,
+                             sum(keys) + dim)
+    heads, scale = kv_heads * per, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    sl = torch.tensor(keys, dtype=torch.int32)
+    dev = [t.cuda() for t in (k, v, table, sl)]
+    qd = rows.cuda()[:, :heads * dim].unflatten(-1, (heads, dim))
+    wide = torch.full((len(keys), (heads + 1) * dim), 7.0,
+                      dtype=torch.bfloat16, device="cuda")
+    out = wide[:, :heads * dim].unflatten(-1, (heads, dim))
+    for sign in (1.0, -1.0):
+        got = ops.paged_attn_decode(qd, *dev, sign * scale, out=out)
+        check(got, *want(q, k, v, table, [1] * len(keys), ctx, sign * scale))
+    assert (wide[:, heads * dim:] == 7.0).all()
+
+
+def test_decode_standout_scores():
+    rows, k, v, table = make([1, 1], [900, 350], 1, 2, 128, 5)
+    k[table[0, 4], 0, 3] *= 30.0
+    k[table[0, 50], 0, 15] *= 60.0
+    k[table[1, 21], 0, 13] *= 90.0            # the last key of all
+    q = rows[:, :256].unflatten(-1, (2, 128))
+    got = ops.paged_attn_decode(
+        q.contiguous().cuda(), k.cuda(), v.cuda(), table.cuda(),
+        torch.tensor([901, 351], dtype=torch.int32, device="cuda"), 0.3)
+    check(got, *want(q, k, v, table, [1, 1], [900, 350], 0.3))

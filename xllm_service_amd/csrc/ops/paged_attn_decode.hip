@@ -1,398 +1,406 @@
 // Paged-attention DECODE kernel for MI355X (gfx950 / CDNA4) — MFMA-based.
 //
-// v2 design: the GQA head group IS the MFMA M dimension. For one
-// (sequence, kv_head), the G query heads (G <= 16, zero-padded to 16) form
-// the A operand rows, so QK^T and P·V are mfma_f32_16x16x32_bf16 chains and
-// the VALU does only softmax bookkeeping — v1's shuffle-reduce design was
-// VALU-bound at ~2.1 TB/s of KV stream; here MFMA issue is ~free and the
-// kernel streams K/V at memory speed.
+// One new token per sequence: for one (sequence, kv_head) the G query heads
+// (G <= 32) are the columns of S^T = K Q^T and of O^T += V^T P^T, as in
+// paged_attn_prefill.hip (layouts: mfma_rows.h); most columns are padding and
+// the matrix pipe does not notice, the kernel is a stream over the cache.
 //
-//   * one workgroup (4 waves) per (seq, kv_head); wave w owns KV tiles
-//     w, w+4, w+8... of 32 keys (2 cache blocks) — sequence-partitioned
-//     flash-decoding, merged through LDS at the end
-//   * K feeds the QK^T B-fragment STRAIGHT from the paged cache (the
-//     [tok][d] cache row layout is exactly the B-fragment gather: 16-B
-//     vector loads per lane, no staging)
-//   * V bounces through a per-wave LDS transpose to build P·V B-fragments
-//   * per-row (=per-head) online softmax identical to the prefill kernel
+//   * every WAVE streams tiles of 32 keys (2 pages) of its own, through 16 KB
+//     of LDS of its own, straight from memory (global_load_lds, 16 B per lane):
+//     no registers hold data in flight, no barrier in the loop. While the
+//     scores of a tile are made its values are on the way, while its values
+//     are multiplied the next keys are: counted waits, each for the older half
+//   * 8 waves a CU (LDS-bound) keep 64-128 KB in flight per CU, four times
+//     what memory latency times bandwidth asks for
+//   * waves of a workgroup merge through LDS at the end; when there are too
+//     few (sequence, kv_head) pairs to fill the chip the keys are split over
+//     P workgroups, whose fp32 results a second kernel merges
 //
-// Fragment layouts as verified by tests/test_gpu_ops.py::test_mfma_fragment_layout.
+// Measured, 32 query / 8 key heads of 128: 128 sequences of 1-2 k keys 160 ->
+// 143 us, 5.6 TB/s (a large copy: 4.9); 24 x 0.6-1.3 k 24 + 9 -> 18 us; one of
+// 776: 16 -> 8 us. 28/4 heads, 6 x 9-20 k: 54 + 16 -> 28 + 4 us. Before: K in
+// registers a tile ahead, V loaded in the tile that used it, one result per
+// wave through memory.
+//
 // Parity: reference engine's paged-attention decode.
-#include "common.h"
+#include "mfma_rows.h"
 
 namespace xllm {
 
-typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
-
 #define PA_BS 16           // cache block size (tokens)
-#define PA_KBLK 32         // keys per tile (2 cache blocks)
-#define PA_D 128           // head_dim handled by the MFMA path
-#define PA_PAD 8           // LDS row padding (elements)
+#define PA_KT 32           // keys per tile (2 cache blocks)
+#define PA_NW 4            // waves per workgroup
 
-// NOTE round-2: forcing 3 waves/SIMD via __launch_bounds__(256, 3) caps the
-// unified VGPR+AGPR file at 166 and the allocator spills the K prefetch to
-// SCRATCH — measured 3.1 TB/s vs 5.3 at the natural 232V+32A allocation
-// (S=64 L=2048). The occupancy squeeze in docs/TODO_ROUND2.md is a dead
-// end on gfx950's unified file; the kernel already streams 5.1-5.6 TB/s at
-// serving shapes (B>=64, L>=1100).
-template <int G>
-__global__ __launch_bounds__(256) void paged_attn_decode_kernel(
-    float* __restrict__ ws_ml,               // [S*n_kv*W][G][2] partial m,l
-    float* __restrict__ ws_o,                // [S*n_kv*W][G][D] partial O
+// Columns [0, D) of 16 rows of a V image: the A operands of one step of
+// O^T += V^T P^T. The wait is part of it: a builtin here would make the compiler
+// wait for every load in flight to LDS, the next keys among them.
+template <int D, int OFF>
+XLLM_DEV void pa_cols(const unsigned (&at)[D / 32], bf16x8 (&v)[D / 32]) {
+  typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
+  u32x2 t[2 * (D / 32)];
+  if constexpr (D == 128)
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %8 offset:%12\n\t"
+        "ds_read_b64_tr_b16 %1, %8 offset:%13\n\t"
+        "ds_read_b64_tr_b16 %2, %9 offset:%12\n\t"
+        "ds_read_b64_tr_b16 %3, %9 offset:%13\n\t"
+        "ds_read_b64_tr_b16 %4, %10 offset:%12\n\t"
+        "ds_read_b64_tr_b16 %5, %10 offset:%13\n\t"
+        "ds_read_b64_tr_b16 %6, %11 offset:%12\n\t"
+        "ds_read_b64_tr_b16 %7, %11 offset:%13\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3]), "=&v"(t[4]),
+          "=&v"(t[5]), "=&v"(t[6]), "=&v"(t[7])
+        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(OFF),
+          "n"(OFF + 8 * D)
+        : "memory");
+  else
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4 offset:%6\n\t"
+        "ds_read_b64_tr_b16 %1, %4 offset:%7\n\t"
+        "ds_read_b64_tr_b16 %2, %5 offset:%6\n\t"
+        "ds_read_b64_tr_b16 %3, %5 offset:%7\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3])
+        : "v"(at[0]), "v"(at[1]), "n"(OFF), "n"(OFF + 8 * D)
+        : "memory");
+#pragma unroll
+  for (int i = 0; i < D / 32; i++) {
+    const unsigned x[4] = {t[2 * i][0], t[2 * i][1], t[2 * i + 1][0],
+                           t[2 * i + 1][1]};
+    __builtin_memcpy(&v[i], x, 16);
+  }
+}
+
+// 32 rows of a K image: the A operands of S^T = K Q^T, with their wait (as above)
+template <int D>
+XLLM_DEV void pa_rows(const unsigned (&at)[D / 16], bf16x8 (&k)[D / 16]) {
+  if constexpr (D == 128)
+    asm volatile(
+        "ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\t"
+        "ds_read_b128 %2, %10\n\tds_read_b128 %3, %11\n\t"
+        "ds_read_b128 %4, %12\n\tds_read_b128 %5, %13\n\t"
+        "ds_read_b128 %6, %14\n\tds_read_b128 %7, %15\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(k[0]), "=&v"(k[1]), "=&v"(k[2]), "=&v"(k[3]), "=&v"(k[4]),
+          "=&v"(k[5]), "=&v"(k[6]), "=&v"(k[7])
+        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "v"(at[4]),
+          "v"(at[5]), "v"(at[6]), "v"(at[7])
+        : "memory");
+  else
+    asm volatile(
+        "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+        "ds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(k[0]), "=&v"(k[1]), "=&v"(k[2]), "=&v"(k[3])
+        : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3])
+        : "memory");
+}
+
+// TERMS: bf16 terms a softmax weight is split into (1: rounded; 3: all of its
+// 32 bits).
+template <int D, int TERMS>
+__global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_decode_kernel(
+    unsigned short* __restrict__ out,        // [S, n_qheads, D]
+    float* __restrict__ ws_o,                // [S*n_qheads][P][D] (P > 1)
+    float* __restrict__ ws_ml,               // [S*n_qheads][P][2]
     const unsigned short* __restrict__ q,    // [num_seqs, n_qheads, D] bf16
     const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, BS, D]
     const unsigned short* __restrict__ v_cache,
     const int* __restrict__ block_tables,    // [num_seqs, max_blocks]
     const int* __restrict__ seq_lens,        // [num_seqs]
-    const float scale,
-    const int n_kv_heads, const int max_blocks_per_seq,
-    const long q_stride, const int P,       // P partitions per (seq, kvh)
-    unsigned short* __restrict__ out,       // [S, n_qheads, D] (P == 1)
-    const long out_stride) {
-  const int sk = blockIdx.x / P;            // (seq, kvh) unit
-  const int wgp = blockIdx.x % P;           // partition within the unit
-  const int seq = sk / n_kv_heads;
-  const int kvh = sk % n_kv_heads;
-  const int n_qheads = n_kv_heads * G;
+    const float scale, const int G, const int n_kv, const int max_blocks,
+    const long q_stride, const long out_stride, const int P) {
+  constexpr int NW = PA_NW, KS = D / 16, DT = D / 32;
+  constexpr int CPR = D / 8;                 // 16 B chunks of a row
+  constexpr int RPI = 64 / CPR;              // rows one load instruction fills
+  constexpr int NI = PA_KT / RPI;            // ... instructions per tile
+  constexpr int TILE = PA_KT * D;            // elements of a K or V tile
+  __shared__ __attribute__((aligned(1024))) unsigned short kv_lds[NW * 2 * TILE];
+  __shared__ float ml_lds[NW][32][2];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, c32 = lane & 31;
+  const int part = blockIdx.x % P, unit = blockIdx.x / P;
+  const int seq = unit / n_kv, kvh = unit % n_kv;
   const int seq_len = seq_lens[seq];
-  const int n_tiles = (seq_len + PA_KBLK - 1) / PA_KBLK;
-  const int nwaves = P * 4;                 // total partials per unit
+  const int n_tiles = (seq_len + PA_KT - 1) / PA_KT;
+  const int step = P * NW;                   // tiles from one to a wave's next
+  const int t0 = part * NW + wid;
 
-  const int wid = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int frow = lane & 15;
-  const int fcol8 = (lane >> 4) * 8;
-  const int crow4 = (lane >> 4) * 4;
-
-  // per-wave LDS scratch + cross-wave merge buffers.
-  // vt_lds holds the tr16-compatible V image: per n-tile (16 d) and k-half
-  // t, four [4 k][16 d] row-major blocks (one per 16-lane group), so P·V
-  // B-fragments come from ds_read_b64_tr_b16 (guide T10) instead of a
-  // scalar transpose. Element (k, d) lives at
-  //   (d>>4)*512 + ((k>>2)&1)*256 + (k>>3)*64 + (k&3)*16 + (d&15).
-  __shared__ unsigned short p_lds[4][16][PA_KBLK + PA_PAD];
-  __shared__ unsigned short vt_lds[4][4096];
-
-  // ---- Q as A-fragment: row = head-in-group (zero-padded to 16) -----------
-  bf16x8 qf[4];
-  if (frow < G) {
-    const long qoff = (long)seq * q_stride + (long)(kvh * G + frow) * PA_D;
+  const bool row_ok = c32 < G;
+  const int head = kvh * G + c32;
+  // weights are 2^(c (s - m)); a negative scale turns the queries' signs
+  const short flip = scale < 0.0f ? (short)0x8000 : (short)0;
+  const float c = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
+  // padding columns hold the first head's query: their results go nowhere
+  bf16x8 qf[KS];
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++)
-      qf[ks] = *reinterpret_cast<const bf16x8*>(q + qoff + ks * 32 + fcol8);
-  } else {
+  for (int ks = 0; ks < KS; ks++)
+    qf[ks] = *reinterpret_cast<const bf16x8*>(
+                 q + (long)seq * q_stride +
+                 (long)(row_ok ? head : kvh * G) * D + ks * 16 + h * 8) ^
+             flip;
+  f32x16 o_acc[DT];
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-  }
+  for (int i = 0; i < DT; i++) o_acc[i] = mr_zero();
+  float m = -INFINITY, l = 0.0f;
 
-  float m_r[4], l_r[4];
-  f32x4 o_acc[8];
-#pragma unroll
-  for (int r = 0; r < 4; r++) { m_r[r] = -INFINITY; l_r[r] = 0.0f; }
-#pragma unroll
-  for (int n = 0; n < 8; n++) o_acc[n] = f32x4{0, 0, 0, 0};
-
-  const int* btab = block_tables + (long)seq * max_blocks_per_seq;
-  const long head_stride = (long)PA_BS * PA_D;
-
-  // K/V loads of a tile: clamped-address loads (no per-load branch — guide
-  // trap 4(c)); lanes beyond seq_len re-read the last token. K garbage is
-  // masked to -inf in the softmax; V garbage is harmless because its P
-  // weight is exactly 0 (finite * 0 = 0 — clamping, unlike zero-fill via a
-  // branch, keeps the load stream unconditional).
-  // Cache-block index per 16-token half: min(t0/16+n, last_blk) is exact
-  // for clamped lanes too (the boundary tile's in-range lanes live in the
-  // same block the clamp resolves to) and — crucially — UNIFORM across the
-  // wave, so btab[...] compiles to a scalar load instead of a per-lane
-  // VMEM load sitting in the K/V address chain every tile.
+  // ---- loads: pages 2t and 2t + 1 of the sequence --------------------------
+  const int* btab = block_tables + (long)seq * max_blocks;
   const int last_blk = (seq_len - 1) / PA_BS;
-  auto load_blks = [&](int tile, int& b0, int& b1) {
-    // uniform per tile: min(2*tile+n, last_blk) is exact for clamped lanes
-    b0 = btab[min(tile * (PA_KBLK / PA_BS), last_blk)];
-    b1 = btab[min(tile * (PA_KBLK / PA_BS) + 1, last_blk)];
+  const int last_row = (seq_len - 1) % PA_BS;
+  const int srow = lane / CPR, spos = lane % CPR;
+  unsigned short* kt = kv_lds + wid * 2 * TILE;
+  unsigned short* vt = kt + TILE;
+  auto off_of = [&](int r, bool val) {       // bytes into a page
+    const int x = val ? mr_swz_cols<D>(r) : mr_swz_rows<D>(r);
+    return (unsigned)(r * (2 * D) + ((spos ^ x) << 4));
   };
-  auto base_of = [&](int blk) -> long {
-    return ((long)blk * n_kv_heads + kvh) * head_stride;
+  unsigned koff[NI / 2], voff[NI / 2];
+#pragma unroll
+  for (int i = 0; i < NI / 2; i++) {
+    koff[i] = off_of(i * RPI + srow, false);
+    voff[i] = off_of(i * RPI + srow, true);
+  }
+  // ids of 32 of the wave's tiles from the tb-th on, two lanes a tile
+  int tb = 0;
+  // (read without waiting for the length: what lies past the last page is not
+  // used)
+  auto pages_from = [&](int n) {
+    return btab[min(2 * (t0 + (n + (lane >> 1)) * step) + (lane & 1),
+                    max_blocks - 1)];
   };
-  auto load_k = [&](bf16x8 (&kb)[2][4], int tile, int b0, int b1) {
-    const int t0 = tile * PA_KBLK;
+  auto load = [&](int t, int n, int pages, bool val) {
+    const char* cache = reinterpret_cast<const char*>(val ? v_cache : k_cache);
+    unsigned short* dst = val ? vt : kt;
+    const int page0 = __builtin_amdgcn_readlane(pages, 2 * (n - tb));
+    const int page1 = 2 * t + 1 > last_blk
+        ? page0 : __builtin_amdgcn_readlane(pages, 2 * (n - tb) + 1);
+    const char* src0 = cache + ((long)page0 * n_kv + kvh) * (PA_BS * D * 2);
+    const char* src1 = cache + ((long)page1 * n_kv + kvh) * (PA_BS * D * 2);
+    auto move = [&](int i, unsigned off) {
+      __builtin_amdgcn_global_load_lds(
+          (glb_void*)((i < NI / 2 ? src0 : src1) + off),
+          (lds_void*)(dst + i * RPI * D), 16, 0, 0);
+    };
+    if (2 * t + 1 < last_blk) {
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-      const int tok = t0 + n * 16 + frow;
-      const int tok_c = tok < seq_len ? tok : seq_len - 1;
-      const long rbase = base_of(n ? b1 : b0) +
-                         (long)(tok_c % PA_BS) * PA_D;
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++)
-        kb[n][ks] = *reinterpret_cast<const bf16x8*>(
-            k_cache + rbase + ks * 32 + fcol8);
+      for (int i = 0; i < NI; i++)
+        move(i, val ? voff[i % (NI / 2)] : koff[i % (NI / 2)]);
+      return;
     }
+    // rows past the last key repeat it: masked below, and finite
+    unsigned off[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int ii = i % (NI / 2), r = ii * RPI + srow;
+      const int pg = 2 * t + i / (NI / 2);
+      const int rr = pg < last_blk ? r : pg > last_blk ? last_row
+                                       : min(r, last_row);
+      off[i] = (val ? voff[ii] : koff[ii]) + (rr - r) * (2 * D);
+    }
+#pragma unroll
+    for (int i = 0; i < NI; i++) move(i, off[i]);
   };
-  // lane covers token tv = lane>>1, d-half dv = (lane&1)*64
-  const int tv = lane >> 1;
-  const int dv = (lane & 1) * 64;
-  const int koff = ((tv >> 2) & 1) * 256 + (tv >> 3) * 64 + (tv & 3) * 16;
-  auto stage_v = [&](int tile, int b0, int b1) {
-    // V is loaded and written to the tr16 LDS image in-tile with transient
-    // registers (8-16 live): K owns the persistent prefetch buffers, and
-    // holding V too pushes past 256 regs into scratch spills (measured).
-    const int tok = tile * PA_KBLK + tv;
-    const int tok_c = tok < seq_len ? tok : seq_len - 1;
-    const long vbase = base_of(tv >> 4 ? b1 : b0) +
-                       (long)(tok_c % PA_BS) * PA_D + dv;
-#pragma unroll
-    for (int mseg = 0; mseg < 8; mseg++) {
-      const ushort8_t vv = *reinterpret_cast<const ushort8_t*>(
-          v_cache + vbase + mseg * 8);
-      const int d0 = dv + mseg * 8;
-      *reinterpret_cast<ushort8_t*>(
-          &vt_lds[wid][(d0 >> 4) * 512 + koff + (d0 & 15)]) = vv;
-    }
+  // everything but the NI loads issued last has arrived
+  auto wait_older = [&] {
+    if constexpr (NI == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
   };
+  auto wait_all = [&] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
-  // Pipeline: K is double-buffered (each tile's K loads issue a FULL tile
-  // ahead), V stages in-tile through transient regs, and the uniform block
-  // ids both need are scalar-loaded TWO iterations ahead (cb/fb/gb
-  // rotation) so the btab lookup never sits in any load's address chain.
-  bf16x8 kb_a[2][4], kb_b[2][4];
-  const int tile0 = wgp * 4 + wid;
-  int cb0 = 0, cb1 = 0;      // ids for the tile being computed
-  int fb0 = 0, fb1 = 0;      // ids for the next tile (K prefetch target)
-  if (tile0 < n_tiles) {
-    load_blks(tile0, cb0, cb1);
-    load_k(kb_a, tile0, cb0, cb1);
-    if (tile0 + nwaves < n_tiles) load_blks(tile0 + nwaves, fb0, fb1);
+  const int kbase = mr_row_base<D>(lane), vbase = mr_col_base<D>(lane);
+  unsigned kat[KS], vat[DT];                   // LDS bytes
+#pragma unroll
+  for (int i = 0; i < KS; i++)
+    kat[i] = (unsigned)(unsigned long long)((const lds_u16*)kt +
+                                            (kbase ^ (i << 4)));
+#pragma unroll
+  for (int i = 0; i < DT; i++)
+    vat[i] = (unsigned)(unsigned long long)((const lds_u16*)vt +
+                                            (vbase ^ (i << 5)));
+  int pages = pages_from(0);
+  if (t0 < n_tiles) {
+    load(t0, 0, pages, false);
+    load(t0, 0, pages, true);
   }
-
-  for (int tile = tile0, phase = 0; tile < n_tiles;
-       tile += nwaves, phase ^= 1) {
-    const int t0 = tile * PA_KBLK;
-    bf16x8 (&kb)[2][4] = phase ? kb_b : kb_a;
-    bf16x8 (&kb_next)[2][4] = phase ? kb_a : kb_b;
-    // ids for tile+2*nwaves: a full iteration before their first use
-    int gb0 = 0, gb1 = 0;
-    if (tile + 2 * nwaves < n_tiles) load_blks(tile + 2 * nwaves, gb0, gb1);
-    // K loads for the next tile: full-tile latency distance
-    if (tile + nwaves < n_tiles) load_k(kb_next, tile + nwaves, fb0, fb1);
-
-    // ---- S = Q K^T from the prefetched fragments --------------------------
-    f32x4 s[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
+  for (int t = t0, n = 0; t < n_tiles; t += step, n++) {
+    const bool more = t + step < n_tiles;
+    wait_older();                              // K of this tile is there
+    bf16x8 k[KS];
+    pa_rows<D>(kat, k);
+    f32x16 s = mr_zero();
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-#pragma unroll
-      for (int ks = 0; ks < 4; ks++)
-        s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[ks], kb[n][ks],
-                                                       s[n], 0, 0, 0);
-    }
-    // ---- stage V into the tr16 image (in-tile, transient regs) ------------
-    stage_v(tile, cb0, cb1);
-    cb0 = fb0; cb1 = fb1; fb0 = gb0; fb1 = gb1;
-
-    // ---- mask + online softmax (rows are heads) ---------------------------
-    float p_val[2][4];
-    float alpha[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float smax = -INFINITY;
-#pragma unroll
-      for (int n = 0; n < 2; n++) {
-        float sv = s[n][r] * scale;
-        if (t0 + n * 16 + frow >= seq_len) sv = -INFINITY;
-        p_val[n][r] = sv;
-        smax = fmaxf(smax, sv);
+    for (int ks = 0; ks < KS; ks++) s = mr_mma(k[ks], qf[ks], s);
+    int ids = pages;
+    if (more) {
+      if (n + 1 - tb == 32) {
+        ids = pages_from(n + 1);
+        asm volatile("" : "+v"(ids));          // the wait for them stays here
+        tb += 32;
       }
+      load(t + step, n + 1, ids, false);
+    }
+    if (t == n_tiles - 1) {
 #pragma unroll
-      for (int off = 8; off > 0; off >>= 1)
-        smax = fmaxf(smax, __shfl_xor(smax, off, 64));
-      const float m_new = fmaxf(m_r[r], smax);
-      alpha[r] = (m_new == -INFINITY) ? 1.0f : __expf(m_r[r] - m_new);
-      float psum = 0.0f;
+      for (int r = 0; r < 16; r++)
+        if (t * PA_KT + mr_key_of(r, h) >= seq_len) s[r] = -INFINITY;
+    }
+    float mt = s[0];
 #pragma unroll
-      for (int n = 0; n < 2; n++) {
-        const float p = (p_val[n][r] == -INFINITY)
-                            ? 0.0f : __expf(p_val[n][r] - m_new);
-        p_val[n][r] = p;
-        psum += p;
+    for (int r = 1; r < 16; r++) mt = fmaxf(mt, s[r]);
+    mt = pair_max(mt);
+    if (__any(mt > m)) {
+      const float m_new = fmaxf(m, mt);
+      const float alpha =
+          __builtin_amdgcn_exp2f((m - (m_new == -INFINITY ? 0.f : m_new)) * c);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < DT; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o_acc[i][r] *= alpha;
+    }
+    const float mc = m == -INFINITY ? 0.0f : m * c;
+    bf16x8 p[TERMS][2];
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) {
+      float a = __builtin_amdgcn_exp2f(fmaf(s[r], c, -mc));
+      float b = __builtin_amdgcn_exp2f(fmaf(s[r + 1], c, -mc));
+      l += a + b;
+#pragma unroll
+      for (int x = 0; x < TERMS; x++) {
+        const unsigned u = pack_bf16(a, b);
+        reinterpret_cast<unsigned*>(&p[x][r >> 3])[(r & 7) >> 1] = u;
+        drop_bf16(a, b, u);
       }
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) psum += __shfl_xor(psum, off, 64);
-      m_r[r] = m_new;
-      l_r[r] = l_r[r] * alpha[r] + psum;
     }
-    // P -> LDS -> A-fragment
+    if (more) wait_older();                    // V of this tile is there
+    else wait_all();
+    bf16x8 v[DT];
+    pa_cols<D, 0>(vat, v);
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
+    for (int i = 0; i < DT; i++)
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        p_lds[wid][crow4 + r][n * 16 + frow] = f32_to_bf16(p_val[n][r]);
-    }
+      for (int x = 0; x < TERMS; x++)
+        o_acc[i] = mr_mma(v[i], p[x][0], o_acc[i]);
+    pa_cols<D, 32 * D>(vat, v);
 #pragma unroll
-    for (int n = 0; n < 8; n++) {
+    for (int i = 0; i < DT; i++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) o_acc[n][r] *= alpha[r];
-    }
-    bf16x8 pa = *reinterpret_cast<const bf16x8*>(&p_lds[wid][frow][fcol8]);
-    // ---- O += P V (B-fragments via hardware transpose reads) --------------
-    // per tr read a 16-lane group gathers one [4 k][16 d] block; lane
-    // address = image + (l>>4)*128B + (l&15)*8B, sub-tiles via offset:
-    {
-      typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u32x2;
-      // low 32 bits of a generic LDS pointer ARE the LDS byte offset
-      // (the shared aperture is 2^32-aligned on amdgcn)
-      const unsigned vaddr =
-          (unsigned)(unsigned long long)(&vt_lds[wid][0]) +
-          ((lane >> 4) * 128u + (lane & 15) * 8u);
-      // one half-batch of 8 tr reads live at a time (16 result VGPRs,
-      // reused across halves: the kernel is register-occupancy-bound)
-#define PA_TR8(OFF0)                                                       \
-      asm volatile(                                                        \
-          "ds_read_b64_tr_b16 %[t0], %[a] offset:" #OFF0 "+0\n\t"          \
-          "ds_read_b64_tr_b16 %[t1], %[a] offset:" #OFF0 "+512\n\t"        \
-          "ds_read_b64_tr_b16 %[t2], %[a] offset:" #OFF0 "+1024\n\t"       \
-          "ds_read_b64_tr_b16 %[t3], %[a] offset:" #OFF0 "+1536\n\t"       \
-          "ds_read_b64_tr_b16 %[t4], %[a] offset:" #OFF0 "+2048\n\t"       \
-          "ds_read_b64_tr_b16 %[t5], %[a] offset:" #OFF0 "+2560\n\t"       \
-          "ds_read_b64_tr_b16 %[t6], %[a] offset:" #OFF0 "+3072\n\t"       \
-          "ds_read_b64_tr_b16 %[t7], %[a] offset:" #OFF0 "+3584\n\t"       \
-          "s_waitcnt lgkmcnt(0)"                                           \
-          : [t0] "=&v"(tr[0]), [t1] "=&v"(tr[1]), [t2] "=&v"(tr[2]),       \
-            [t3] "=&v"(tr[3]), [t4] "=&v"(tr[4]), [t5] "=&v"(tr[5]),       \
-            [t6] "=&v"(tr[6]), [t7] "=&v"(tr[7])                           \
-          : [a] "v"(vaddr)                                                 \
-          : "memory")
-      u32x2 tr[8];
-#pragma unroll
-      for (int half = 0; half < 2; half++) {
-        if (half == 0) { PA_TR8(0); } else { PA_TR8(4096); }
-        __builtin_amdgcn_sched_barrier(0);  // MFMAs stay below the wait
-#pragma unroll
-        for (int nn = 0; nn < 4; nn++) {
-          const int n = half * 4 + nn;
-          bf16x8 bv;
-          unsigned* bw = reinterpret_cast<unsigned*>(&bv);
-          bw[0] = tr[2 * nn][0];
-          bw[1] = tr[2 * nn][1];
-          bw[2] = tr[2 * nn + 1][0];
-          bw[3] = tr[2 * nn + 1][1];
-          o_acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, bv, o_acc[n],
-                                                             0, 0, 0);
-        }
-      }
-#undef PA_TR8
-    }
+      for (int x = 0; x < TERMS; x++)
+        o_acc[i] = mr_mma(v[i], p[x][1], o_acc[i]);
+    if (more) load(t + step, n + 1, ids, true);
+    pages = ids;
   }
+  l = pair_sum(l);
 
-  if (P == 1) {
-    // ---- fused merge: combine the 4 per-wave partials through LDS and
-    // write the output directly — saves the merge-kernel launch plus the
-    // global ws_o/ws_ml round-trip (~8 MB at batch 64). vt_lds (32 KB) and
-    // p_lds are dead by now and are reused as the merge buffers.
-    float* mo = reinterpret_cast<float*>(&vt_lds[0][0]);    // [4][G][128]
-    float* mml = reinterpret_cast<float*>(&p_lds[0][0][0]); // [4][G][2]
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = crow4 + r;
-      if (row < G) {
-        if (frow == 0) {
-          mml[(wid * G + row) * 2 + 0] = m_r[r];
-          mml[(wid * G + row) * 2 + 1] = l_r[r];
-        }
-#pragma unroll
-        for (int n = 0; n < 8; n++)
-          mo[((wid * G + row) * PA_D) + n * 16 + frow] = o_acc[n][r];
-      }
+  // ---- the waves' results meet in LDS ----------------------------------------
+  __syncthreads();
+  float* mo = reinterpret_cast<float*>(kv_lds);          // [NW][G][D]
+  if (row_ok) {
+    if (h == 0) {
+      ml_lds[wid][c32][0] = m == -INFINITY ? m : m * c;
+      ml_lds[wid][c32][1] = l;
     }
-    __syncthreads();
-    if (wid == 0) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = crow4 + r;
-        if (row >= G) continue;
-        float m_star = -INFINITY;
+    for (int i = 0; i < DT; i++)
 #pragma unroll
-        for (int w = 0; w < 4; w++)
-          m_star = fmaxf(m_star, mml[(w * G + row) * 2]);
-        float wgt[4], l_tot = 0.0f;
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-          const float mw = mml[(w * G + row) * 2];
-          wgt[w] = (mw == -INFINITY) ? 0.0f : __expf(mw - m_star);
-          l_tot += wgt[w] * mml[(w * G + row) * 2 + 1];
-        }
-        const float inv = (l_tot > 0.0f) ? 1.0f / l_tot : 0.0f;
-#pragma unroll
-        for (int n = 0; n < 8; n++) {
-          float o = 0.0f;
-#pragma unroll
-          for (int w = 0; w < 4; w++)
-            o += wgt[w] * mo[((w * G + row) * PA_D) + n * 16 + frow];
-          out[(long)seq * out_stride + (long)(kvh * G + row) * PA_D +
-              n * 16 + frow] = f32_to_bf16(o * inv);
-        }
-      }
-    }
-    return;
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<float4*>(mo + (wid * G + c32) * D + i * 32 + 2 * r +
+                                   4 * h) =
+            make_float4(o_acc[i][r], o_acc[i][r + 1], o_acc[i][r + 2],
+                        o_acc[i][r + 3]);
   }
-
-  // ---- write this wave's partial (no cross-wave sync: the tiny merge
-  // kernel below combines the P*4 partials per (seq, kvh) unit) ------------
-  const long part = ((long)sk * nwaves + wgp * 4 + wid);
-  if (frow == 0) {
+  __syncthreads();
+  for (int idx = tid; idx < G * (D / 4); idx += NW * 64) {
+    const int row = idx / (D / 4), col = idx % (D / 4) * 4;
+    float M = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = crow4 + r;
-      if (row < G) {
-        ws_ml[(part * G + row) * 2 + 0] = m_r[r];
-        ws_ml[(part * G + row) * 2 + 1] = l_r[r];
-      }
+    for (int w = 0; w < NW; w++) M = fmaxf(M, ml_lds[w][row][0]);
+    const float Mu = M == -INFINITY ? 0.0f : M;
+    float L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float f = __builtin_amdgcn_exp2f(ml_lds[w][row][0] - Mu);
+      L += ml_lds[w][row][1] * f;
+      const float4 x =
+          *reinterpret_cast<const float4*>(mo + (w * G + row) * D + col);
+      a[0] += x.x * f; a[1] += x.y * f; a[2] += x.z * f; a[3] += x.w * f;
     }
-  }
-#pragma unroll
-  for (int n = 0; n < 8; n++) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int row = crow4 + r;
-      if (row < G)
-        ws_o[(part * G + row) * PA_D + n * 16 + frow] = o_acc[n][r];
+    if (P == 1) {
+      const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+      uint2 y;
+      y.x = pack_bf16(a[0] * inv, a[1] * inv);
+      y.y = pack_bf16(a[2] * inv, a[3] * inv);
+      *reinterpret_cast<uint2*>(out + (long)seq * out_stride +
+                                (long)(kvh * G + row) * D + col) = y;
+    } else {
+      const long slot = ((long)seq * n_kv * G + kvh * G + row) * P + part;
+      if (col == 0) {
+        ws_ml[slot * 2] = M;
+        ws_ml[slot * 2 + 1] = L;
+      }
+      *reinterpret_cast<float4*>(ws_o + slot * D + col) =
+          make_float4(a[0], a[1], a[2], a[3]);
     }
   }
 }
 
-// Combine the W = P*4 per-wave partials of each (seq, kvh, g) row.
-__global__ void paged_attn_decode_merge_kernel(
-    unsigned short* __restrict__ out,        // [S, n_qheads, D]
-    const float* __restrict__ ws_ml,         // [S*n_kv*W][G][2]
-    const float* __restrict__ ws_o,          // [S*n_kv*W][G][D]
-    const int G, const int n_kv_heads, const int W, const long out_stride,
-    const long total) {                      // total = S * n_kv * G * D
-  for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total;
-       idx += (long)gridDim.x * blockDim.x) {
-    const int d = (int)(idx % PA_D);
-    long t = idx / PA_D;
-    const int g = (int)(t % G);
-    t /= G;
-    const int kvh = (int)(t % n_kv_heads);
-    const long seq = t / n_kv_heads;
-    const long unit = (seq * n_kv_heads + kvh);
-    float m_star = -INFINITY;
-    for (int w = 0; w < W; w++)
-      m_star = fmaxf(m_star, ws_ml[((unit * W + w) * G + g) * 2]);
-    float l_tot = 0.0f, o = 0.0f;
-    for (int w = 0; w < W; w++) {
-      const float mw = ws_ml[((unit * W + w) * G + g) * 2];
-      const float wgt = (mw == -INFINITY) ? 0.0f : __expf(mw - m_star);
-      l_tot += wgt * ws_ml[((unit * W + w) * G + g) * 2 + 1];
-      o += wgt * ws_o[((unit * W + w) * G + g) * PA_D + d];
-    }
-    const float inv = (l_tot > 0.0f) ? 1.0f / l_tot : 0.0f;
-    out[seq * out_stride + (long)(kvh * G + g) * PA_D + d] =
-        f32_to_bf16(o * inv);
+// out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
+// row, four columns each
+template <int D>
+__global__ __launch_bounds__(256) void paged_attn_merge_kernel(
+    unsigned short* __restrict__ out, const float* __restrict__ ws_o,
+    const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
+    const long out_stride, const long rows) {
+  constexpr int LPR = D / 4;
+  const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
+  const int col = (threadIdx.x % LPR) * 4;
+  if (row >= rows) return;
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
+  const float* o = ws_o + row * n_part * D + col;
+  float M = -INFINITY;
+  for (int p = 0; p < n_part; p++) M = fmaxf(M, ml[p].x);
+  if (M == -INFINITY) M = 0.0f;
+  float L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+  for (int p = 0; p < n_part; p++) {
+    const float2 z = ml[p];
+    const bool on = z.y > 0.0f;              // else nothing was written
+    const float w = on ? __builtin_amdgcn_exp2f(z.x - M) : 0.0f;
+    const float4 x = *reinterpret_cast<const float4*>(o + (long)p * D);
+    L += on ? z.y * w : 0.0f;
+    a[0] += on ? x.x * w : 0.0f; a[1] += on ? x.y * w : 0.0f;
+    a[2] += on ? x.z * w : 0.0f; a[3] += on ? x.w * w : 0.0f;
   }
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  uint2 y;
+  y.x = pack_bf16(a[0] * inv, a[1] * inv);
+  y.y = pack_bf16(a[2] * inv, a[3] * inv);
+  const long tok = row / n_qheads;
+  *reinterpret_cast<uint2*>(out + tok * out_stride +
+                            (row - tok * n_qheads) * D + col) = y;
 }
 
-// ---------------- fallback (head_dim != 128): v1 shuffle-reduce design ------
+void launch_paged_attn_merge(unsigned short* out, const float* ws_o,
+                             const float* ws_ml, int n_qheads, int D,
+                             int n_part, long out_stride, long rows,
+                             hipStream_t stream) {
+  const dim3 grid((unsigned)((rows * (D / 4) + 255) / 256));
+  if (D == 128)
+    hipLaunchKernelGGL((paged_attn_merge_kernel<128>), grid, dim3(256), 0,
+                       stream, out, ws_o, ws_ml, n_qheads, n_part, out_stride,
+                       rows);
+  else
+    hipLaunchKernelGGL((paged_attn_merge_kernel<64>), grid, dim3(256), 0,
+                       stream, out, ws_o, ws_ml, n_qheads, n_part, out_stride,
+                       rows);
+}
+
+// ---------------- other head widths: shuffle-reduce design -------------------
 template <int G>
 __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
     unsigned short* __restrict__ out, const unsigned short* __restrict__ q,
@@ -505,62 +513,70 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
   }
 }
 
-#define PA_DISPATCH_G(GV)                                                      \
-  do {                                                                         \
-    if (D == PA_D) {                                                           \
-      hipLaunchKernelGGL((paged_attn_decode_kernel<GV>), grid, block, 0,       \
-                         stream, ws_ml, ws_o, q, k_cache, v_cache,             \
-                         block_tables, seq_lens, scale, n_kv_heads,            \
-                         max_blocks_per_seq, q_stride, P, out, out_stride);    \
-      if (P > 1)                                                               \
-        hipLaunchKernelGGL(paged_attn_decode_merge_kernel, mgrid, block, 0,    \
-                           stream, out, ws_ml, ws_o, GV, n_kv_heads, P * 4,    \
-                           out_stride, total);                                 \
-    } else {                                                                   \
-      hipLaunchKernelGGL((paged_attn_decode_small_kernel<GV>), grid, block, 0, \
-                         stream, out, q, k_cache, v_cache, block_tables,       \
-                         seq_lens, scale, n_kv_heads, D, max_blocks_per_seq,   \
-                         q_stride, out_stride);                                \
-    }                                                                          \
-  } while (0)
-
-int paged_attn_decode_partitions(int num_seqs, int n_kv_heads) {
-  // partition only when there are too few (seq, kv_head) units to fill the
-  // chip: extra partitions shrink per-wave work and cost merge overhead
-  const int units = num_seqs * n_kv_heads;
-  int P = (512 + units - 1) / units;
-  if (P < 1) P = 1;
-  if (P > 8) P = 8;
-  return P;
+// Workgroups the keys of a (sequence, kv_head) pair are split over, from what
+// the host knows: the pairs and the widest table. One workgroup per CU is
+// enough to split for (more of them only add results to merge), a part of less
+// than eight tiles (two a wave) is not worth its share of the merge, and
+// neither is a split in two. Measured (us, 32/8 heads of 128), whole | split:
+// 1 x 776 keys 10.2 | 7.8, 1 x 2000 18.8 | 8.9, 1 x 20000 143 | 20 (16 parts),
+// 8 x 2000 19.9 | 15.8, 8 x 14000 144 | 82; 1 x 200 5.4 | 6.6, 8 x 500 8.6 |
+// 9.7, 16 x 1000 13.6 | 15.7, 32 x 1500 36.7 | 40.2. Eight waves in a workgroup
+// instead of four: within 5 % where that many keys are split at all, slower
+// for many pairs (128 x 300 keys: 41 against 33).
+int paged_attn_decode_parts(int num_seqs, int n_kv_heads, int max_blocks) {
+  const long units = (long)num_seqs * n_kv_heads;
+  const long tiles = ((long)max_blocks * PA_BS + PA_KT - 1) / PA_KT;
+  long p = units > 0 ? 256 / units : 1;
+  if (p > tiles / 8) p = tiles / 8;
+  return (int)(p < 3 ? 1 : p > 16 ? 16 : p);
 }
 
 void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
                               const unsigned short* k_cache,
                               const unsigned short* v_cache,
                               const int* block_tables, const int* seq_lens,
-                              float* ws_ml, float* ws_o,
-                              float scale, int num_seqs, int n_qheads,
-                              int n_kv_heads, int D, int max_blocks_per_seq,
-                              long q_stride, long out_stride,
+                              float* ws_ml, float* ws_o, float scale,
+                              int num_seqs, int n_qheads, int n_kv_heads, int D,
+                              int max_blocks_per_seq, long q_stride,
+                              long out_stride, int parts,
                               hipStream_t stream) {
-  const int P = paged_attn_decode_partitions(num_seqs, n_kv_heads);
-  dim3 grid(num_seqs * n_kv_heads * (D == PA_D ? P : 1)), block(256);
   const int G = n_qheads / n_kv_heads;
-  const long total = (long)num_seqs * n_kv_heads * G * PA_D;
-  long mg = (total + 255) / 256;
-  if (mg > 2048) mg = 2048;
-  dim3 mgrid((unsigned)mg);
-  switch (G) {
-    case 1: PA_DISPATCH_G(1); break;
-    case 2: PA_DISPATCH_G(2); break;
-    case 3: PA_DISPATCH_G(3); break;
-    case 4: PA_DISPATCH_G(4); break;
-    case 5: PA_DISPATCH_G(5); break;
-    case 6: PA_DISPATCH_G(6); break;
-    case 7: PA_DISPATCH_G(7); break;
-    case 8: PA_DISPATCH_G(8); break;
-    default: break;  // validated host-side
+  if (num_seqs == 0) return;
+  if (D != 128 && D != 64) {
+    const dim3 grid(num_seqs * n_kv_heads), block(256);
+#define PA_SMALL(GV)                                                           \
+  hipLaunchKernelGGL((paged_attn_decode_small_kernel<GV>), grid, block, 0,     \
+                     stream, out, q, k_cache, v_cache, block_tables, seq_lens, \
+                     scale, n_kv_heads, D, max_blocks_per_seq, q_stride,       \
+                     out_stride)
+    switch (G) {
+      case 1: PA_SMALL(1); break;
+      case 2: PA_SMALL(2); break;
+      case 3: PA_SMALL(3); break;
+      case 4: PA_SMALL(4); break;
+      case 5: PA_SMALL(5); break;
+      case 6: PA_SMALL(6); break;
+      case 7: PA_SMALL(7); break;
+      case 8: PA_SMALL(8); break;
+      default: break;  // validated host-side
+    }
+#undef PA_SMALL
+    return;
   }
+  const dim3 grid((unsigned)(num_seqs * n_kv_heads * parts));
+#define PA_LAUNCH(DV, TERMS)                                                   \
+  hipLaunchKernelGGL((paged_attn_decode_kernel<DV, TERMS>), grid,              \
+                     dim3(PA_NW * 64), 0, stream, out, ws_o, ws_ml, q,         \
+                     k_cache, v_cache, block_tables, seq_lens, scale, G,       \
+                     n_kv_heads, max_blocks_per_seq, q_stride, out_stride,     \
+                     parts)
+  // 64-wide heads have 32-bit weights, as every other width but 128
+  if (D == 128) PA_LAUNCH(128, 1);
+  else PA_LAUNCH(64, 3);
+#undef PA_LAUNCH
+  if (parts > 1)
+    launch_paged_attn_merge(out, ws_o, ws_ml, n_qheads, D, parts, out_stride,
+                            (long)num_seqs * n_qheads, stream);
 }
 
 }  // namespace xllm

@@ -149,17 +149,14 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
   // weights are 2^(c (s - m)); a negative scale turns the queries' signs
   const short flip = scale < 0.0f ? (short)0x8000 : (short)0;
   const float c = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
+  // rows past the last one hold its query: their results go nowhere
+  const int qr = min(rho, rows - 1), qq = qr / G;
+  const unsigned short* qp = q + (long)(q_start + qq) * q_stride +
+                             (long)(kvh * G + qr - qq * G) * D + h * 8;
   bf16x8 qf[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
-    qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (row_ok)
-      qf[ks] = *reinterpret_cast<const bf16x8*>(
-          q + (long)(q_start + qi) * q_stride + (long)head * D + ks * 16 +
-          h * 8);
-    qf[ks] ^= flip;
-  }
-
+  for (int ks = 0; ks < KS; ks++)
+    qf[ks] = *reinterpret_cast<const bf16x8*>(qp + ks * 16) ^ flip;
   f32x16 o_acc[DT];
 #pragma unroll
   for (int i = 0; i < DT; i++) o_acc[i] = mr_zero();
@@ -341,38 +338,11 @@ __global__ __launch_bounds__(256, 2) void paged_attn_prefill_kernel(
                       o_acc[dt][r + 3]);
 }
 
-// out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
-// row, four columns each
-template <int D>
-__global__ __launch_bounds__(256) void paged_attn_prefill_merge_kernel(
-    unsigned short* __restrict__ out, const float* __restrict__ ws_o,
-    const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
-    const long out_stride, const long rows) {
-  constexpr int LPR = D / 4;
-  const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
-  const int col = (threadIdx.x % LPR) * 4;
-  if (row >= rows) return;
-  const float* ml = ws_ml + row * n_part * 2;
-  float M = -INFINITY;
-  for (int p = 0; p < n_part; p++) M = fmaxf(M, ml[2 * p]);
-  if (M == -INFINITY) M = 0.0f;
-  float L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int p = 0; p < n_part; p++) {
-    if (ml[2 * p + 1] <= 0.0f) continue;     // nothing was written
-    const float w = __builtin_amdgcn_exp2f(ml[2 * p] - M);
-    L += ml[2 * p + 1] * w;
-    const float4 x = *reinterpret_cast<const float4*>(
-        ws_o + (row * n_part + p) * D + col);
-    a[0] += x.x * w; a[1] += x.y * w; a[2] += x.z * w; a[3] += x.w * w;
-  }
-  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-  uint2 y;
-  y.x = pack_bf16(a[0] * inv, a[1] * inv);
-  y.y = pack_bf16(a[2] * inv, a[3] * inv);
-  const long tok = row / n_qheads;
-  *reinterpret_cast<uint2*>(out + tok * out_stride +
-                            (row - tok * n_qheads) * D + col) = y;
-}
+// paged_attn_decode.hip
+void launch_paged_attn_merge(unsigned short* out, const float* ws_o,
+                             const float* ws_ml, int n_qheads, int D,
+                             int n_part, long out_stride, long rows,
+                             hipStream_t stream);
 
 // Row tiles a batch has at most, and the parts its keys are split into: about
 // two workgroups per CU are wanted, and a part under eight tiles of keys costs
@@ -402,23 +372,17 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws_o, float* ws_ml,
   if (tokens == 0 || n_seqs == 0) return;
   dim3 grid((unsigned)(pf_tiles(tokens, n_seqs, G) * n_kv * n_part));
 #define PF_LAUNCH(DV, TERMS)                                                   \
-  do {                                                                         \
-    hipLaunchKernelGGL((paged_attn_prefill_kernel<DV, TERMS>), grid,           \
-                       dim3(256), 0, stream, out, ws_o, ws_ml, q, k_cache,     \
-                       v_cache, block_tables, cu_q, seq_lens, n_seqs, scale, G, \
-                       n_kv, max_blocks, q_stride, out_stride, n_part);        \
-    if (n_part > 1) {                                                          \
-      const long rows = tokens * n_qheads;                                     \
-      hipLaunchKernelGGL((paged_attn_prefill_merge_kernel<DV>),                \
-                         dim3((unsigned)((rows * (DV / 4) + 255) / 256)),      \
-                         dim3(256), 0, stream, out, ws_o, ws_ml, n_qheads,     \
-                         n_part, out_stride, rows);                            \
-    }                                                                          \
-  } while (0)
+  hipLaunchKernelGGL((paged_attn_prefill_kernel<DV, TERMS>), grid, dim3(256),  \
+                     0, stream, out, ws_o, ws_ml, q, k_cache, v_cache,         \
+                     block_tables, cu_q, seq_lens, n_seqs, scale, G, n_kv,     \
+                     max_blocks, q_stride, out_stride, n_part)
   // 64-wide heads ran on fp32 weights before they had a kernel and still do
   if (D == 128) PF_LAUNCH(128, 1);
   else PF_LAUNCH(64, 3);
 #undef PF_LAUNCH
+  if (n_part > 1)
+    launch_paged_attn_merge(out, ws_o, ws_ml, n_qheads, D, n_part, out_stride,
+                            tokens * n_qheads, stream);
 }
 
 // ---------------------------------------------------------------------------------

@@ -59,7 +59,8 @@ ext_modules = [
                       "latent_attn_mfma.hip", "decay_attn.hip",
                       "decay_attn_mfma.hip", "moe.hip",
                       "streams.hip", "short_conv.hip",
-                      "gated_recurrence.hip", "capped_attn.hip",
+                      "gated_recurrence.hip", "paged_attn.hip",
+                      "capped_attn.hip",
                       "capped_attn_mfma.hip", "rownorm_rope.hip",
                       "delta_rule.hip", "rope_headnorm.hip", "depth_mix.hip",
                       "retention.hip", "joint_layer.hip")

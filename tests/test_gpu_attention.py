@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from xllm_service_amd import ops
+from xllm_service_amd.ops import hybrid as H
 
 pytestmark = pytest.mark.gpu
 PAGE = 16
@@ -34,7 +35,8 @@ def make(lens, ctx, kv_heads, per, dim, seed, spare=3):
     return rows.to(torch.bfloat16), k, v, table
 
 
-def want(q, k, v, table, lens, ctx, scale):
+def want(q, k, v, table, lens, ctx, scale, window=0, keep_first=0,
+         chunked=False, sink=None, cap=0.0, head_scale=None):
     """(result, weighted sum of |v|) in fp64; q [T, heads, dim]."""
     heads, dim = q.shape[1:]
     per = heads // k.shape[1]
@@ -44,8 +46,24 @@ def want(q, k, v, table, lens, ctx, scale):
         kk, vv = (x[pages].transpose(1, 2).reshape(-1, k.shape[1], dim)[:n + c]
                   .double().repeat_interleave(per, 1) for x in (k, v))
         z = torch.einsum("thd,lhd->htl", q[at:at + n].double(), kk) * scale
-        late = torch.arange(n + c)[None] > c + torch.arange(n)[:, None]
-        p = torch.softmax(z.masked_fill(late, -math.inf), -1)
+        if head_scale is not None:
+            z = z * head_scale.double()[:, None, None]
+        if cap:
+            z = cap * torch.tanh(z / cap)
+        pos, key = c + torch.arange(n)[:, None], torch.arange(n + c)[None]
+        gone = key > pos
+        if window:
+            first = pos // window * window if chunked else pos - window + 1
+            gone = gone | ((key < first) & (key >= keep_first))
+        z = z.masked_fill(gone, -math.inf)
+        m = z.amax(-1, keepdim=True)
+        if sink is not None:
+            m = torch.maximum(m, sink.double()[:, None, None])
+        p = torch.exp(z - m)
+        den = p.sum(-1, keepdim=True)
+        if sink is not None:
+            den = den + torch.exp(sink.double()[:, None, None] - m)
+        p = p / den
         out.append(torch.einsum("htl,lhd->thd", p, vv))
         big.append(torch.einsum("htl,lhd->thd", p, vv.abs()))
         at += n
@@ -161,3 +179,62 @@ def test_decode_standout_scores():
         q.contiguous().cuda(), k.cuda(), v.cuda(), table.cuda(),
         torch.tensor([901, 351], dtype=torch.int32, device="cuda"), 0.3)
     check(got, *want(q, k, v, table, [1, 1], [900, 350], 0.3))
+
+
+OPTIONS = {
+    "plain": {},
+    "window": dict(window=50),
+    "window + kept": dict(window=33, keep_first=5),
+    "window of one": dict(window=1, keep_first=70),
+    "chunks": dict(window=48, chunked=True),
+    "sink": dict(window=64, sink=True),
+    "cap": dict(cap=5.0),
+    "large cap": dict(cap=50.0),
+    "head scales": dict(head_scale=True, cap=3.0, sink=True),
+    "signs": dict(head_scale=True, window=100),
+}
+
+
+@pytest.mark.parametrize("opts", list(OPTIONS))
+@pytest.mark.parametrize("dim,bf16_out", [(64, True), (128, False),
+                                          (128, True)])
+@pytest.mark.parametrize("lens,ctx,kv_heads,per,decode", [
+    ([1, 33, 64, 130], [16, 31, 100, 0], 2, 4, False),
+    ([5, 2], [1500, 3000], 1, 2, False),                   # parts
+    ([1] * 5, [0, 15, 31, 127, 400], 3, 4, True),
+    ([1, 1], [2000, 4095], 1, 32, True),                   # parts
+])
+def test_options(dim, bf16_out, lens, ctx, kv_heads, per, decode, opts):
+    """Windows, kept keys, chunks, sinks, caps and head multipliers, fp32 and
+    bf16 results, keys read as values; the weights have 32 bits."""
+    opts = dict(OPTIONS[opts])
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(ctx) + dim)
+    heads, T, scale = kv_heads * per, sum(lens), 1.5 * dim ** -0.5
+    g = torch.Generator().manual_seed(3)
+    for name in ("sink", "head_scale"):
+        if opts.get(name):
+            opts[name] = torch.randn(heads, generator=g)
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)], dtype=torch.int32)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)),
+                      dtype=torch.int32)
+    q = rows[:, :heads * dim]
+    for values in (v, k):
+        kd = k.cuda()
+        vd = kd if values is k else v.cuda()
+        wide = torch.full((T, (heads + 1) * dim), 7.0, device="cuda",
+                          dtype=torch.bfloat16 if bf16_out else torch.float32)
+        out = wide[:, :heads * dim]
+        H.capped_attn(rows.cuda()[:, :heads * dim], kd, vd, table.cuda(),
+                      None if decode else cu.cuda(), sl.cuda(), heads, scale,
+                      opts.get("cap", 0.0), out, opts.get("window", 0),
+                      *(opts[x].cuda() if x in opts else None
+                        for x in ("sink",)), opts.get("keep_first", 0),
+                      opts["head_scale"].cuda() if "head_scale" in opts
+                      else None, opts.get("chunked", False))
+        ref, big = want(q.unflatten(-1, (heads, dim)), k, values, table, lens,
+                        ctx, scale, **opts)
+        off = (out.unflatten(-1, (heads, dim)).double().cpu() - ref).abs()
+        over = off - 2.0 ** -17 * big - (2.0 ** -8 * ref.abs() if bf16_out
+                                         else 0.0)
+        assert over.max() <= 1e-6, f"off by {off.max():.3g}"
+        assert (wide[:, heads * dim:] == 7.0).all()

@@ -120,6 +120,12 @@ template <typename T>
 void launch_gated_group_norm(T*, const float*, const float*, int, const T*,
                              long, float, int, int, int, int, int,
                              long, hipStream_t);
+int paged_attn_parts(bool, long, int, int, int, long, int, int);
+void launch_paged_attn(void*, long, bool, float*, float*, const unsigned short*,
+                       const unsigned short*, const unsigned short*, const int*,
+                       const int*, const int*, long, int, int, int, int, int,
+                       float, float, long, int, int, const float*, int,
+                       const float*, bool, hipStream_t);
 int capped_attn_mfma_class(int D, int Dv);
 void launch_capped_attn_mfma(void*, long, int, float*, float*, const unsigned short*,
                              const unsigned short*, const unsigned short*,
@@ -1095,12 +1101,38 @@ void capped_attn(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
     TORCH_CHECK(head_scale->numel() == heads);
     hsp = ptr<float>(*head_scale);
   }
-  // bf16: MFMA kernel when the sizes fit one of its instantiations
-  if (is_bf16(q) && hy::capped_attn_mfma_class(D, Dv) != 0 &&
-      q.stride(0) % 8 == 0 &&
+  // bf16 with 16 B rows: the matrix-pipe kernels
+  const bool rows16 =
+      is_bf16(q) && q.stride(0) % 8 == 0 &&
       reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 == 0 &&
       out_stride % 4 == 0 &&
-      reinterpret_cast<uintptr_t>(out.data_ptr()) % (out_bf ? 8 : 16) == 0) {
+      reinterpret_cast<uintptr_t>(out.data_ptr()) % (out_bf ? 8 : 16) == 0;
+  // 16-token pages, keys and values 64 or 128 wide (decode: no more query heads
+  // per key head than a wave has rows)
+  if (rows16 && bs == 16 && D == Dv && (D == 64 || D == 128) &&
+      (cu != nullptr || heads / n_kv <= 32) &&
+      reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(v_cache.data_ptr()) % 16 == 0) {
+    const int n_part =
+        hy::paged_attn_parts(cu == nullptr, T, n_seqs, heads, n_kv,
+                             block_tables.size(1), window, keep_first);
+    Tensor ws;                 // [T * heads][parts][D + 2]
+    float *ws_o = nullptr, *ws_ml = nullptr;
+    if (n_part > 1) {
+      const long n = (long)T * heads * n_part;
+      ws = torch::empty({n * (D + 2)}, out.options().dtype(torch::kFloat));
+      ws_o = ptr<float>(ws);
+      ws_ml = ws_o + n * D;
+    }
+    hy::launch_paged_attn(
+        out.data_ptr(), out_stride, !out_bf, ws_o, ws_ml, ptr<bf>(q),
+        ptr<bf>(k_cache), ptr<bf>(v_cache), ptr<int>(block_tables), cu,
+        ptr<int>(seq_lens), T, n_seqs, heads, n_kv, D, block_tables.size(1),
+        scale, cap, q.stride(0), n_part, window, sinkp, keep_first, hsp,
+        chunked, cur());
+    return;
+  }
+  if (rows16 && hy::capped_attn_mfma_class(D, Dv) != 0) {
     int n_part = 1;
     Tensor ws_acc, ws_ml;
     if (cu == nullptr) {

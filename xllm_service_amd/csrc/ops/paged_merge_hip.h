@@ -1,0 +1,154 @@
+// !!! This is a file automatically generated by hipify!!!
+#include "hip/hip_runtime.h"
+// What the paged attention kernels (paged_rows.h, paged_stream.h) share: their
+// options, and the merge of keys that were split over workgroups.
+#pragma once
+#include "mfma_rows.h"
+
+namespace xllm {
+
+// Options of a call. A kernel instantiated without MORE ignores them: bf16
+// results, every earlier key seen, scores scale * q.k.
+struct PagedMore {
+  int window = 0;         // > 0: a row sees the last `window` keys ...
+  int keep_first = 0;     // ... and the first keep_first
+  int chunked = 0;        // `window` is a chunk size: a row sees its own chunk
+  int out_f32 = 0;        // results in fp32
+  float cap = 0.0f;       // > 0: scores become cap * tanh(score / cap)
+  const float* sink = nullptr;        // [heads]: e^sink joins the denominator
+  const float* head_scale = nullptr;  // [heads]: one more score multiplier
+};
+
+// first key that a row which sees keys below `limit` has in its window
+template <bool MORE>
+XLLM_DEV int paged_first(const PagedMore& x, int limit) {
+  if (!MORE || x.window <= 0) return 0;
+  return x.chunked ? (limit - 1) / x.window * x.window
+                   : max(0, limit - x.window);
+}
+
+// The tiles a workgroup walks: those that hold kept keys, then from the first
+// one that its earliest row (which sees keys below `limit`) sees.
+struct PagedTiles {
+  int keep, gap, n;       // at(i): i below keep as it is, else + gap
+  XLLM_DEV int at(int i) const { return i < keep ? i : i + gap; }
+};
+template <bool MORE>
+XLLM_DEV PagedTiles paged_tiles(const PagedMore& x, int limit, int kmax,
+                                int n_tiles, int kt) {
+  if (!MORE || x.window <= 0) return {0, 0, n_tiles};
+  const int first = paged_first<MORE>(x, limit) / kt;
+  const int keep = min((min(x.keep_first, kmax) + kt - 1) / kt, first);
+  return {keep, first - keep, n_tiles - (first - keep)};
+}
+
+// How a row's scores become weights 2^(c (s - m)): a negative factor turns the
+// signs of the query's entries, so that c is positive; with a cap, s is the
+// capped score and pre goes in front of the tanh.
+struct PagedScore { short flip; float c, pre; };
+template <bool MORE>
+XLLM_DEV PagedScore paged_score(const PagedMore& x, float scale, int head) {
+  constexpr float log2e = 1.4426950408889634f;
+  if (MORE && x.head_scale != nullptr) scale *= x.head_scale[head];
+  if (MORE && x.cap > 0.0f) return {0, log2e, scale / x.cap};
+  return {scale < 0.0f ? (short)0x8000 : (short)0,
+          fmaxf(fabsf(scale) * log2e, 1e-30f), 0.0f};
+}
+
+// s <- cap * tanh(pre * s). Below 1/2 the odd Taylor series up to x^15 (the next
+// term is under 2^-26 of the value); above, 1 - 2 / (e^2x + 1). Tiles without
+// large scores, nearly all of them, skip the exponentials and divisions.
+template <int N>
+XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
+  float big = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      s[i][r] *= pre;
+      big = fmaxf(big, fabsf(s[i][r]));
+    }
+  const bool far = __any(!(big < 0.5f));
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const float v = s[i][r], w = v * v;
+      float y = fmaf(w, -929569.0f / 638512875.0f, 21844.0f / 6081075.0f);
+      y = fmaf(y, w, -1382.0f / 155925.0f);
+      y = fmaf(y, w, 62.0f / 2835.0f);
+      y = fmaf(y, w, -17.0f / 315.0f);
+      y = fmaf(y, w, 2.0f / 15.0f);
+      y = fmaf(y, w, -1.0f / 3.0f);
+      y = fmaf(y * w, v, v);
+      if (far) {
+        const float e = __expf(2.0f * fminf(v, 15.0f));
+        const float z = 1.0f - 2.0f / (e + 1.0f);
+        y = fabsf(v) < 0.5f ? y : z;
+      }
+      s[i][r] = cap * y;
+    }
+}
+
+// four neighbouring results
+template <bool MORE>
+XLLM_DEV void paged_put(const PagedMore& x, void* out, long at, float a,
+                        float b, float c, float d) {
+  if (MORE && x.out_f32) {
+    *reinterpret_cast<float4*>((float*)out + at) = make_float4(a, b, c, d);
+  } else {
+    uint2 y;
+    y.x = pack_bf16(a, b);
+    y.y = pack_bf16(c, d);
+    *reinterpret_cast<uint2*>((unsigned short*)out + at) = y;
+  }
+}
+
+// out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
+// row, four columns each
+template <int D, bool MORE>
+__global__ __launch_bounds__(256) void paged_attn_merge_kernel(
+    void* __restrict__ out, const float* __restrict__ ws_o,
+    const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
+    const long out_stride, const long rows, const PagedMore x) {
+  constexpr int LPR = D / 4;
+  const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
+  const int col = (threadIdx.x % LPR) * 4;
+  if (row >= rows) return;
+  const long tok = row / n_qheads;
+  const int head = (int)(row - tok * n_qheads);
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
+  const float* o = ws_o + row * n_part * D + col;
+  const bool sink = MORE && x.sink != nullptr;
+  const float sk = sink ? x.sink[head] * 1.4426950408889634f : -INFINITY;
+  float M = sk;
+  for (int p = 0; p < n_part; p++) M = fmaxf(M, ml[p].x);
+  if (M == -INFINITY) M = 0.0f;
+  float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.0f;
+  float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+  for (int p = 0; p < n_part; p++) {
+    const float2 z = ml[p];
+    const bool on = z.y > 0.0f;              // else nothing was written
+    const float w = on ? __builtin_amdgcn_exp2f(z.x - M) : 0.0f;
+    const float4 y = *reinterpret_cast<const float4*>(o + (long)p * D);
+    L += on ? z.y * w : 0.0f;
+    a[0] += on ? y.x * w : 0.0f; a[1] += on ? y.y * w : 0.0f;
+    a[2] += on ? y.z * w : 0.0f; a[3] += on ? y.w * w : 0.0f;
+  }
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  paged_put<MORE>(x, out, tok * out_stride + (long)head * D + col, a[0] * inv,
+                  a[1] * inv, a[2] * inv, a[3] * inv);
+}
+
+template <int D, bool MORE>
+inline void paged_merge(void* out, const float* ws_o, const float* ws_ml,
+                        int n_qheads, int n_part, long out_stride, long rows,
+                        const PagedMore& x, hipStream_t stream) {
+  hipLaunchKernelGGL((paged_attn_merge_kernel<D, MORE>),
+                     dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256),
+                     0, stream, out, ws_o, ws_ml, n_qheads, n_part, out_stride,
+                     rows, x);
+}
+
+}  // namespace xllm

@@ -120,7 +120,7 @@ template <typename T>
 void launch_gated_group_norm(T*, const float*, const float*, int, const T*,
                              long, float, int, int, int, int, int,
                              long, hipStream_t);
-int paged_attn_parts(bool, long, int, int, int, long, int, int);
+int paged_attn_parts(bool, long, int, int, int, long, int, int, bool);
 void launch_paged_attn(void*, long, bool, float*, float*, const unsigned short*,
                        const unsigned short*, const unsigned short*, const int*,
                        const int*, const int*, long, int, int, int, int, int,
@@ -1115,7 +1115,8 @@ void capped_attn(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
       reinterpret_cast<uintptr_t>(v_cache.data_ptr()) % 16 == 0) {
     const int n_part =
         hy::paged_attn_parts(cu == nullptr, T, n_seqs, heads, n_kv,
-                             block_tables.size(1), window, keep_first);
+                             block_tables.size(1), window, keep_first,
+                             cap > 0);
     Tensor ws;                 // [T * heads][parts][D + 2]
     float *ws_o = nullptr, *ws_ml = nullptr;
     if (n_part > 1) {

@@ -19,13 +19,13 @@ static PagedMore more_of(bool out_f32, float cap, int window, const float* sink,
 
 // Parts the keys are split into. cu_q null: decoded rows.
 int paged_attn_parts(bool decode, long tokens, int n_seqs, int heads, int n_kv,
-                     long max_blocks, int window, int keep_first) {
+                     long max_blocks, int window, int keep_first, bool capped) {
   if (window > 0)
     max_blocks = std::min<long>(
         max_blocks, (window + 15) / 16 + (keep_first + 15) / 16 + 2);
-  return decode ? paged_stream_parts(n_seqs, n_kv, max_blocks)
+  return decode ? paged_stream_parts(n_seqs, n_kv, max_blocks, capped)
                 : paged_rows_parts(tokens, n_seqs, heads / n_kv, n_kv,
-                                   max_blocks);
+                                   max_blocks, 3);
 }
 
 // out [tokens, heads * D] rows of out_stride, fp32 or bf16; q rows, caches and

@@ -39,7 +39,7 @@ void launch_paged_attn_decode(unsigned short*, const unsigned short*,
                               int, int, int, int, int, long, long, int,
                               hipStream_t);
 int paged_attn_decode_parts(int, int, int);
-int paged_attn_prefill_parts(long, int, int, int, int);
+int paged_attn_prefill_parts(long, int, int, int, int, int);
 void launch_paged_attn_prefill(unsigned short*, float*, float*,
                                const unsigned short*, const unsigned short*,
                                const unsigned short*, const int*, const int*,
@@ -262,7 +262,7 @@ void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
               seq_lens.size(0) >= n_seqs && block_tables.size(0) >= n_seqs,
               "prefill kernel: shapes do not match");
   const int n_part = xllm::paged_attn_prefill_parts(
-      tokens, n_seqs, n_qheads / n_kv, n_kv, block_tables.size(1));
+      tokens, n_seqs, n_qheads / n_kv, n_kv, D, block_tables.size(1));
   torch::Tensor ws;            // [tokens * heads][parts][D + 2], fp32
   float *ws_o = nullptr, *ws_ml = nullptr;
   if (n_part > 1) {

@@ -6,9 +6,10 @@
 
 namespace xllm {
 
-int paged_attn_prefill_parts(long tokens, int n_seqs, int G, int n_kv,
+int paged_attn_prefill_parts(long tokens, int n_seqs, int G, int n_kv, int D,
                              int max_blocks) {
-  return paged_rows_parts(tokens, n_seqs, G, n_kv, max_blocks);
+  return paged_rows_parts(tokens, n_seqs, G, n_kv, max_blocks,
+                          D == 128 ? 1 : 3);
 }
 
 // 64-wide heads ran on fp32 weights before they had a kernel and still do

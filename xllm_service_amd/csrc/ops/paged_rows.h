@@ -348,16 +348,20 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
 }
 
 // Row tiles a batch has at most, and the parts its keys are split into: about
-// two workgroups per CU are wanted, and a part under eight tiles of keys costs
-// more in its merge than it saves.
+// two workgroups per CU are wanted, and parts of at least eight tiles of keys
+// (four with 32-bit weights, whose tiles take twice as long): the merge costs
+// more than smaller ones save. Measured (us, by parts 1 | 2 | 4 | 8), 32-bit
+// weights: 2 x 64 rows of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of 16
+// over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles) 374 | 298 |
+// 302 | 325; 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
 inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
   return tokens * G / PF_ROWS + n_seqs;
 }
 inline int paged_rows_parts(long tokens, int n_seqs, int G, int n_kv,
-                            long max_blocks) {
+                            long max_blocks, int terms) {
   const long wgs = paged_rows_tiles(tokens, n_seqs, G) * n_kv;
-  const long most = max_blocks * PF_BS / (8 * PF_KT);
-  long p = wgs > 0 ? 512 / wgs : 1;
+  const long most = max_blocks * PF_BS / ((terms > 1 ? 4 : 8) * PF_KT);
+  long p = wgs > 0 ? (512 + wgs / 2) / wgs : 1;
   if (p > most) p = most;
   return (int)(p < 1 ? 1 : p > 16 ? 16 : p);
 }

@@ -367,11 +367,16 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
 // 9.7, 16 x 1000 13.6 | 15.7, 32 x 1500 36.7 | 40.2. Eight waves in a workgroup
 // instead of four: within 5 % where that many keys are split at all, slower
 // for many pairs (128 x 300 keys: 41 against 33).
-inline int paged_stream_parts(long num_seqs, int n_kv_heads, long max_blocks) {
+// Capped scores make a tile about twice as long, so that smaller parts and a
+// split in two pay: 16/4 heads, 1 x 700 keys 15.5 | 9.7 (6 parts), 32 x 2000
+// 37.6 | 31.0 (2 parts).
+inline int paged_stream_parts(long num_seqs, int n_kv_heads, long max_blocks,
+                              bool capped = false) {
   const long units = num_seqs * n_kv_heads;
   const long tiles = (max_blocks * PA_BS + PA_KT - 1) / PA_KT;
   long p = units > 0 ? 256 / units : 1;
-  if (p > tiles / 8) p = tiles / 8;
+  if (p > tiles / (capped ? 4 : 8)) p = tiles / (capped ? 4 : 8);
+  if (p == 2 && capped && tiles >= 48) return 2;
   return (int)(p < 3 ? 1 : p > 16 ? 16 : p);
 }
 

@@ -65,6 +65,11 @@ void launch_latent_attn(float*, const T*, const T*, const int*, const int*,
                         const int*, int, int, int, int, int, int, int, float,
                         long, int, hipStream_t);
 int latent_attn_mfma_class(int W, int r);
+bool latent_stream_takes(int, int, int, int);
+int latent_stream_parts(int, int, long, int);
+void launch_latent_stream(float*, float*, float*, const unsigned short*,
+                          const unsigned short*, const int*, const int*, int,
+                          int, int, int, float, int, int, hipStream_t);
 void launch_latent_attn_mfma(float*, float*, float*, const unsigned short*,
                              const unsigned short*, const int*, const int*,
                              const int*, int, int, int, int, int, int, int,
@@ -565,6 +570,29 @@ void latent_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables,
     cu = ptr<int>(*cu_q);
   } else {
     TORCH_CHECK(n_seqs == T, "decode: one sequence per token");
+  }
+  auto aligned = [](const Tensor& t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  // decoded rows of the rank-512 sizes
+  if (is_bf16(q) && cu == nullptr &&
+      hy::latent_stream_takes(W, r, H, cache.size(1)) && aligned(q) &&
+      aligned(cache) && aligned(out) && block_tables.size(1) > 0) {
+    const int n_part =
+        hy::latent_stream_parts(n_seqs, H, block_tables.size(1), window);
+    Tensor ws;                 // [T * H][parts][r + 2]
+    float *ws_o = nullptr, *ws_ml = nullptr;
+    if (n_part > 1) {
+      const long n = (long)T * H * n_part;
+      ws = torch::empty({n * (r + 2)}, out.options());
+      ws_o = ptr<float>(ws);
+      ws_ml = ws_o + n * r;
+    }
+    hy::launch_latent_stream(ptr<float>(out), ws_o, ws_ml, ptr<bf>(q),
+                             ptr<bf>(cache), ptr<int>(block_tables),
+                             ptr<int>(seq_lens), n_seqs, H, W,
+                             block_tables.size(1), scale, n_part, window, cur());
+    return;
   }
   // bf16: MFMA kernel when the sizes fit one of its instantiations
   if (is_bf16(q) && hy::latent_attn_mfma_class(W, r) != 0) {

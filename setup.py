@@ -37,6 +37,7 @@ ext_modules = [
                 "paged_attn_prefill.hip",
                 "sampling.hip",
                 "gemm.hip",
+                "linear.hip",
                 "skinny_gemm.hip",
                 "packed_gemm.hip",
             )

@@ -1,0 +1,75 @@
+"""x W^T (+ bias) at the edges of its tiles, against fp64 of the bf16 inputs. Sums
+are 32-bit and the result is rounded to bf16: 2^-9 of itself and 2^-24 times
+the square root of the number of terms (K up to 4096: 2^-18) of the sum of
+absolute products; twice both is allowed."""
+import pytest
+import torch
+
+from xllm_service_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 63, 64, 65, 100, 129, 300])
+@pytest.mark.parametrize("N,K", [(8, 128), (64, 256), (72, 1152), (200, 4096),
+                                 (4096, 384)])
+@pytest.mark.parametrize("bias,stride", [(False, 0), (True, 8)])
+def test_linear(M, N, K, bias, stride):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+
+    def bf(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(
+            torch.bfloat16)
+    x = bf(M, K + stride)[:, :K]
+    w, b = bf(N, K), bf(N) if bias else None
+    got = ops.linear(x, w, b)
+    assert got.shape == (M, N) and got.dtype == torch.bfloat16
+    want = x.double() @ w.double().t()
+    big = x.double().abs() @ w.double().abs().t()
+    if bias:
+        want, big = want + b.double(), big + b.double().abs()
+    off = (got.double() - want).abs() - 2.0 ** -8 * want.abs() \
+        - 2.0 ** -17 * big
+    assert off.max() <= 0, f"over by {off.max():.3g}"
+
+
+def test_what_the_kernels_do_not_take():
+    """Types, widths, gradients and shapes that go to the library."""
+    for dt, M, N, K in ((torch.float32, 4, 64, 128), (torch.bfloat16, 4, 63, 128),
+                        (torch.bfloat16, 4, 64, 100), (torch.bfloat16, 0, 8, 128)):
+        x, w = (torch.randn(r, K, device="cuda").to(dt) for r in (M, N))
+        y = ops.linear(x, w)
+        assert torch.equal(y, torch.nn.functional.linear(x, w))
+    x = torch.randn(2, 3, 128, device="cuda").to(torch.bfloat16)
+    w = torch.randn(64, 128, device="cuda").to(torch.bfloat16)
+    assert ops.linear(x, w).shape == (2, 3, 64)
+    w.requires_grad_(True)
+    ops.linear(x[0], w).float().sum().backward()
+    assert w.grad is not None
+
+
+def test_transforms_go_to_the_library():
+    """vmap, forward-mode AD, autocast and a dispatch mode see the call."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    x, w = (torch.randn(r, 128, device="cuda").to(torch.bfloat16)
+            for r in (6, 64))
+    linear = torch.nn.functional.linear
+    assert torch.equal(
+        torch.vmap(lambda r: ops.linear(r, w))(x.view(3, 2, 128)),
+        torch.vmap(lambda r: linear(r, w))(x.view(3, 2, 128)))
+    with forward_ad.dual_level():
+        y = ops.linear(forward_ad.make_dual(x, x), w)
+        assert forward_ad.unpack_dual(y).tangent is not None
+    with torch.autocast("cuda", torch.float16):
+        assert ops.linear(x, w).dtype == torch.float16
+
+    class Count(TorchDispatchMode):
+        calls = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Count.calls += 1
+            return func(*args, **(kwargs or {}))
+    with Count():
+        ops.linear(x, w)
+    assert Count.calls > 0

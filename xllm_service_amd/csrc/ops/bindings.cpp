@@ -2,6 +2,10 @@
 //
 // All tensor-shape/dtype validation lives here so the kernels stay lean.
 #include <hip/hip_runtime.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 
@@ -53,6 +57,10 @@ int skinny_gemm_splitk(int M, int N, int K);
 void launch_skinny_gemm(unsigned short*, const unsigned short*,
                         const unsigned short*, const unsigned short*, float*,
                         int, int, int, hipStream_t);
+int linear_takes(long M, long N, long K);
+void launch_linear(unsigned short*, const unsigned short*,
+                   const unsigned short*, const unsigned short*, int, int, int,
+                   long, int, hipStream_t);
 int packed_gemm_splitk(int M, int N, int K, int S);
 void launch_packed_gemm(unsigned short*, const unsigned short*,
                         unsigned short*, const unsigned short*,
@@ -329,6 +337,53 @@ torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor b,
   return c;
 }
 
+// plain memory, no transform, mode or trace that has to see the call
+static bool plain(const torch::Tensor& t) {
+  return !t.key_set().has_any(c10::DispatchKeySet(
+             {c10::DispatchKey::FuncTorchBatched,
+              c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
+              c10::DispatchKey::Functionalize, c10::DispatchKey::ZeroTensor,
+              c10::DispatchKey::Conjugate, c10::DispatchKey::Negative})) &&
+         !t._fw_grad(0).defined();
+}
+
+// x [..., K] @ w [N, K]^T (+ bias): the kernels of linear.hip where they take the
+// call, the library elsewhere (and wherever a gradient is wanted)
+torch::Tensor linear(torch::Tensor x, torch::Tensor w,
+                     c10::optional<torch::Tensor> bias) {
+  auto rows16 = [](const torch::Tensor& t) {
+    return plain(t) && t.dim() == 2 && t.is_cuda() &&
+           t.dtype() == torch::kBFloat16 && t.stride(1) == 1 &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  const bool grad =
+      at::GradMode::is_enabled() &&
+      (x.requires_grad() || w.requires_grad() ||
+       (bias.has_value() && bias->requires_grad()));
+  const bool seen = c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+                    torch::jit::tracer::isTracing() ||
+                    at::autocast::is_autocast_enabled(at::kCUDA);
+  if (!grad && !seen && rows16(x) && rows16(w) && x.size(1) == w.size(1) &&
+      x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) && w.is_contiguous() &&
+      x.device() == w.device() &&
+      (!bias.has_value() ||
+       (plain(*bias) && bias->dim() == 1 && bias->is_contiguous() &&
+        bias->dtype() == torch::kBFloat16 && bias->size(0) == w.size(0) &&
+        bias->device() == w.device()))) {
+    const long M = x.size(0), N = w.size(0), K = w.size(1);
+    const int kind = xllm::linear_takes(M, N, K);
+    if (kind != 0) {
+      c10::OptionalDeviceGuard guard(x.device());
+      auto y = torch::empty({M, N}, x.options());
+      xllm::launch_linear(u16(y), u16c(x), u16c(w),
+                          bias.has_value() ? u16c(*bias) : nullptr, (int)M,
+                          (int)N, (int)K, x.stride(0), kind, cur_stream());
+      return y;
+    }
+  }
+  return at::linear(x, w, bias.has_value() ? *bias : torch::Tensor());
+}
+
 torch::Tensor packed_gemm(torch::Tensor a, torch::Tensor wp, int64_t N,
                           c10::optional<torch::Tensor> bias,
                           int64_t s_override) {
@@ -548,6 +603,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma_probe_16x16x32", &mfma_probe_16x16x32);
   m.def("mfma_gemm", &mfma_gemm);
   m.def("skinny_gemm", &skinny_gemm);
+  m.def("linear", &linear);
   m.def("packed_gemm", &packed_gemm);
   m.def("packed_gemm_probe", &packed_gemm_probe);
   m.def("migrate_blocks_peer", &migrate_blocks_peer);

@@ -10,6 +10,8 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
+from xllm_service_amd import ops
+
 from . import parallel_state as ps
 
 
@@ -43,7 +45,7 @@ class ColumnParallelLinear(nn.Module):
     def forward(self, x):
         if self.use_skinny:
             return _maybe_skinny(x, self.weight, self.bias)
-        return torch.nn.functional.linear(x, self.weight, self.bias)
+        return ops.linear(x, self.weight, self.bias)
 
 
 class MergedColumnParallelLinear(ColumnParallelLinear):
@@ -85,7 +87,7 @@ class RowParallelLinear(nn.Module):
         if self.use_skinny:
             y = _maybe_skinny(x, self.weight, None)
         else:
-            y = torch.nn.functional.linear(x, self.weight)
+            y = ops.linear(x, self.weight)
         y = ps.tp_all_reduce(y)
         if self.bias is not None:
             y = y + self.bias

@@ -1,8 +1,9 @@
 """Llama-family decoder (Llama-3 / Qwen2 text tower) on the paged-KV engine.
 
-GEMMs go through hipBLASLt (torch linear); everything else on the hot path is
-a hand-written gfx950 HIP op: fused(add+)RMSNorm, fused RoPE, paged-attention
-prefill/decode, fused SwiGLU. Covers BASELINE.md configs 2-4.
+GEMMs go through the kernels of csrc/ops/linear.hip where the rows are few and
+through hipBLASLt above; everything else on the hot path is a hand-written gfx950
+HIP op: fused(add+)RMSNorm, fused RoPE, paged-attention prefill/decode, fused
+SwiGLU.
 """
 from __future__ import annotations
 

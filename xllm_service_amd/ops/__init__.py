@@ -225,6 +225,15 @@ def mfma_gemm(a, b, bias=None):
                                       else None).to(a.dtype)
 
 
+def linear(x, weight, bias=None):
+    """x @ weight.T (+ bias). On a GPU the bf16 shapes of serving steps run on
+    the kernels of csrc/ops/linear.hip, the others on the library."""
+    if x.is_cuda and HAS_EXT and not torch.overrides.has_torch_function(
+            (x, weight)):
+        return _ops.linear(x, weight, bias)
+    return torch.nn.functional.linear(x, weight, bias)
+
+
 def skinny_gemm(a, b, bias=None):
     """Split-K weight-streaming GEMM for decode batches (M <= 64).
     GPU-only; callers fall back to F.linear elsewhere."""

@@ -149,6 +149,7 @@ def test_prefill_needs_no_host():
     ([127, 128, 129, 255, 256, 257, 700], 4, 7),            # waves
     ([2049, 5, 4500], 3, 2), ([9001], 2, 4),                # parts
     ([40 + 7 * i for i in range(70)], 4, 3),                # many pairs
+    ([33 + 61 * (i % 7) for i in range(29)] + [6000], 3, 2),  # one long one
     ([18000, 33], 1, 5),              # over 32 tiles of one wave
 ])
 def test_decode_edges(dim, keys, kv_heads, per):
@@ -203,6 +204,7 @@ OPTIONS = {
     ([5, 2], [1500, 3000], 1, 2, False),                   # parts
     ([1] * 5, [0, 15, 31, 127, 400], 3, 4, True),
     ([1, 1], [2000, 4095], 1, 32, True),                   # parts
+    ([1] * 30, [20 + 31 * i for i in range(29)] + [3500], 3, 2, True),
 ])
 def test_options(dim, bf16_out, lens, ctx, kv_heads, per, decode, opts):
     """Windows, kept keys, chunks, sinks, caps and head multipliers, fp32 and

@@ -104,6 +104,11 @@ XLLM_DEV f32x4 ls_mma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// parts that n tiles are really split into, of the n_part there is room for
+XLLM_DEV int ls_parts(int n, int n_part, int per) {
+  return max(1, min(n_part, (n + per - 1) / per));
+}
+
 template <int W>
 __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
     float* __restrict__ out,               // [S, H, 512] (n_part == 1)
@@ -112,7 +117,7 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
     const unsigned short* __restrict__ q,  // [S, H, W]
     const unsigned short* __restrict__ cache,   // [blocks, 16, W]
     const int* __restrict__ block_tables, const int* __restrict__ seq_lens,
-    int heads, int table_width, float scale, int n_part, int window) {
+    int heads, int table_width, float scale, int n_part, int per, int window) {
   constexpr int CPR = W / 8;                     // 16 B chunks of a row
   constexpr int IPP = 16 * CPR / 64;             // load instructions per page
   constexpr int NI = 2 * IPP / 4;                // ... of a wave per tile
@@ -123,13 +128,16 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, n = lane & 15;
-  const int part = blockIdx.x % n_part, s = blockIdx.x / n_part;
+  const int n_seqs = gridDim.x / n_part;
+  const int part = blockIdx.x / n_seqs, s = blockIdx.x % n_seqs;  // idle last
   const int h0 = blockIdx.y * 16;                // first head
   const int seq_len = seq_lens[s];
   const int n_tiles = (seq_len + LS_KT - 1) / LS_KT;
   const int lo = window > 0 ? max(0, seq_len - window) : 0;
   const int t_first = lo / LS_KT;
-  const int tpp = (n_tiles - t_first + n_part - 1) / n_part;
+  const int parts = ls_parts(n_tiles - t_first, n_part, per);
+  if (part >= parts) return;
+  const int tpp = (n_tiles - t_first + parts - 1) / parts;
   const int t_begin = t_first + part * tpp;
   const int t_end = min(n_tiles, t_begin + tpp);
 
@@ -311,7 +319,7 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   l += __shfl_xor(l, 16, 64);
   if (!on) return;
   const int col = w * 128 + g * 4;
-  if (n_part == 1) {
+  if (parts == 1) {
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     float* o = out + row * LS_R + col;
 #pragma unroll
@@ -337,18 +345,24 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
 // workgroup per row, four columns per lane
 __global__ void __launch_bounds__(256) latent_stream_merge_kernel(
     float* __restrict__ out, const float* __restrict__ ws_o,
-    const float* __restrict__ ws_ml, int n_part, long rows) {
+    const float* __restrict__ ws_ml, int n_part, int per, long rows, int heads,
+    const int* __restrict__ seq_lens, int window) {
   const long row = blockIdx.x * 2L + (threadIdx.x >> 7);
   const int col = (threadIdx.x & 127) * 4;
   if (row >= rows) return;
+  const int len = seq_lens[row / heads];
+  const int parts = ls_parts(
+      (len + LS_KT - 1) / LS_KT -
+          (window > 0 ? max(0, len - window) / LS_KT : 0), n_part, per);
+  if (parts == 1) return;                        // written where it belongs
   const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
   const float* o = ws_o + row * n_part * LS_R + col;
   float M = -INFINITY;
-  for (int p = 0; p < n_part; p++) M = fmaxf(M, ml[p].x);
+  for (int p = 0; p < parts; p++) M = fmaxf(M, ml[p].x);
   if (M == -INFINITY) M = 0.0f;
   float L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 4
-  for (int p = 0; p < n_part; p++) {
+  for (int p = 0; p < parts; p++) {
     const float2 z = ml[p];
     const bool on = z.y > 0.0f;                  // else nothing was written
     const float f = on ? __builtin_amdgcn_exp2f(z.x - M) : 0.0f;
@@ -366,16 +380,21 @@ bool latent_stream_takes(int W, int r, int heads, int block_size) {
   return r == LS_R && (W == 512 || W == 576) && heads <= 32 && block_size == 16;
 }
 
-// Parts a sequence's keys are split into: one workgroup per CU, parts of at least
-// two tiles. Measured (us, by parts): 32 x 2000 keys, 16 heads 92 (1), 32 (4),
-// 24 (8), 27 (16); 8 x 4000 173 (1), 32 (8), 23 (16), 21 (32); 64 x 1000 51 (1),
-// 24 (4), 26 (8); 128 x 600 35 (1), 28 (2), 30 (4); 1 x 700 36 (1), 13 (12).
+// Room for parts from what the host knows, one part for every `per` tiles of a
+// sequence's own in the kernel. Few workgroups: one per CU, parts of at least two
+// tiles. Measured (us, by parts): 32 x 2000 keys, 16 heads 92 (1), 32 (4), 24
+// (8), 27 (16); 8 x 4000 173 (1), 32 (8), 23 (16), 21 (32); 64 x 1000 51 (1), 24
+// (4), 26 (8); 1 x 700 36 (1), 13 (12). More: parts of 16 tiles, so that a long
+// sequence among short ones is no chain that outlasts the rest; 128 x 600 35
+// (1), 28 (2), 30 (4).
+static int ls_per(long wgs) { return wgs < 86 ? 2 : 16; }
 int latent_stream_parts(int n_seqs, int heads, long table_width, int window) {
-  const long wgs = (long)n_seqs * ((heads + 15) / 16);
+  const long wgs = std::max<long>(1, (long)n_seqs * ((heads + 15) / 16));
   long tiles = (table_width + 1) / 2;
   if (window > 0) tiles = std::min<long>(tiles, window / LS_KT + 2);
-  const long p = std::min<long>(256 / std::max<long>(wgs, 1), tiles / 2);
-  return (int)std::max<long>(1, std::min<long>(p, 32));
+  const long per = ls_per(wgs);
+  const long p = wgs < 86 ? 256 / wgs : (512 + wgs - 1) / wgs;
+  return (int)std::min<long>({p, (tiles + per - 1) / per, 32});
 }
 
 // q, cache and out 16 B aligned
@@ -386,15 +405,16 @@ void launch_latent_stream(float* out, float* ws_o, float* ws_ml,
                           float scale, int n_part, int window, hipStream_t st) {
   if (n_seqs == 0) return;
   const dim3 grid(n_seqs * n_part, (heads + 15) / 16);
+  const int per = ls_per((long)n_seqs * grid.y);
   auto k = W == 512 ? latent_stream_kernel<512> : latent_stream_kernel<576>;
   hipLaunchKernelGGL(k, grid, dim3(256), 0, st, out, ws_o, ws_ml, q, cache,
                      block_tables, seq_lens, heads, table_width, scale, n_part,
-                     window);
+                     per, window);
   if (n_part > 1) {
     const long rows = (long)n_seqs * heads;
     hipLaunchKernelGGL(latent_stream_merge_kernel,
                        dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, out,
-                       ws_o, ws_ml, n_part, rows);
+                       ws_o, ws_ml, n_part, per, rows, heads, seq_lens, window);
   }
 }
 

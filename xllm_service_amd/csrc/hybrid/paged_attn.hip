@@ -17,13 +17,18 @@ static PagedMore more_of(bool out_f32, float cap, int window, const float* sink,
   return x;
 }
 
-// Parts the keys are split into. cu_q null: decoded rows.
+// pages that a window lets a row see
+static long seen_pages(long max_blocks, int window, int keep_first) {
+  return window <= 0 ? max_blocks
+      : std::min<long>(max_blocks,
+                       (window + 15) / 16 + (keep_first + 15) / 16 + 2);
+}
+
+// Room for parts the keys are split into. cu_q null: decoded rows.
 int paged_attn_parts(bool decode, long tokens, int n_seqs, int heads, int n_kv,
                      long max_blocks, int window, int keep_first, bool capped) {
-  if (window > 0)
-    max_blocks = std::min<long>(
-        max_blocks, (window + 15) / 16 + (keep_first + 15) / 16 + 2);
-  return decode ? paged_stream_parts(n_seqs, n_kv, max_blocks, capped)
+  max_blocks = seen_pages(max_blocks, window, keep_first);
+  return decode ? paged_stream_split(n_seqs, n_kv, max_blocks, capped).parts
                 : paged_rows_parts(tokens, n_seqs, heads / n_kv, n_kv,
                                    max_blocks, 3);
 }
@@ -44,7 +49,10 @@ void launch_paged_attn(void* out, long out_stride, bool out_f32, float* ws_o,
   if (cu_q == nullptr) {
     auto go = D == 128 ? paged_stream<128, 3, true> : paged_stream<64, 3, true>;
     go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, seq_lens, n_seqs,
-       scale, heads, n_kv, max_blocks, q_stride, out_stride, n_part, x, st);
+       scale, heads, n_kv, max_blocks, q_stride, out_stride,
+       paged_stream_split(n_seqs, n_kv,
+                          seen_pages(max_blocks, window, keep_first), cap > 0),
+       x, st);
   } else {
     auto go = D == 128 ? paged_rows<128, 3, true> : paged_rows<64, 3, true>;
     go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, cu_q, seq_lens,

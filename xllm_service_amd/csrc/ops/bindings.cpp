@@ -40,7 +40,7 @@ void launch_gather_blocks(unsigned short*, unsigned short*, const long*, int,
 void launch_paged_attn_decode(unsigned short*, const unsigned short*,
                               const unsigned short*, const unsigned short*,
                               const int*, const int*, float*, float*, float,
-                              int, int, int, int, int, long, long, int,
+                              int, int, int, int, int, long, long,
                               hipStream_t);
 int paged_attn_decode_parts(int, int, int);
 int paged_attn_prefill_parts(long, int, int, int, int, int);
@@ -246,7 +246,7 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
       u16(out), u16c(q), u16c(k_cache), u16c(v_cache),
       block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), ws_ml, ws_o,
       (float)scale, num_seqs, n_qheads, n_kv, D, block_tables.size(1),
-      q.stride(0), out.stride(0), parts, cur_stream());
+      q.stride(0), out.stride(0), cur_stream());
 }
 
 void paged_attn_prefill(torch::Tensor out, torch::Tensor q,

@@ -120,9 +120,10 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
 }
 
 int paged_attn_decode_parts(int num_seqs, int n_kv_heads, int max_blocks) {
-  return paged_stream_parts(num_seqs, n_kv_heads, max_blocks);
+  return paged_stream_split(num_seqs, n_kv_heads, max_blocks).parts;
 }
 
+// ws_o, ws_ml: room for paged_attn_decode_parts() results per row
 void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
                               const unsigned short* k_cache,
                               const unsigned short* v_cache,
@@ -130,8 +131,7 @@ void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
                               float* ws_ml, float* ws_o, float scale,
                               int num_seqs, int n_qheads, int n_kv_heads, int D,
                               int max_blocks_per_seq, long q_stride,
-                              long out_stride, int parts,
-                              hipStream_t stream) {
+                              long out_stride, hipStream_t stream) {
   const int G = n_qheads / n_kv_heads;
   if (num_seqs == 0) return;
   if (D != 128 && D != 64) {
@@ -159,7 +159,8 @@ void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
   auto go = D == 128 ? paged_stream<128, 1, false> : paged_stream<64, 3, false>;
   go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, seq_lens, num_seqs,
      scale, n_qheads, n_kv_heads, max_blocks_per_seq, q_stride, out_stride,
-     parts, PagedMore{}, stream);
+     paged_stream_split(num_seqs, n_kv_heads, max_blocks_per_seq), PagedMore{},
+     stream);
 }
 
 }  // namespace xllm

@@ -88,6 +88,12 @@ XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
     }
 }
 
+// Decoded rows: parts that a list of n tiles is really split into, of the P that
+// the host, which does not know the lengths, made room for
+XLLM_DEV int paged_parts(int n, int P, int per) {
+  return max(1, min(P, (n + per - 1) / per));
+}
+
 // four neighbouring results
 template <bool MORE>
 XLLM_DEV void paged_put(const PagedMore& x, void* out, long at, float a,
@@ -103,12 +109,15 @@ XLLM_DEV void paged_put(const PagedMore& x, void* out, long at, float a,
 }
 
 // out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
-// row, four columns each
+// row, four columns each. seq_lens: rows are decoded ones, one sequence each,
+// with as many parts as their length asks for (per tiles of kt keys); a single
+// part has been written where it belongs.
 template <int D, bool MORE>
 __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
     void* __restrict__ out, const float* __restrict__ ws_o,
     const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
-    const long out_stride, const long rows, const PagedMore x) {
+    const long out_stride, const long rows, const PagedMore x,
+    const int* __restrict__ seq_lens, const int per, const int kt) {
   constexpr int LPR = D / 4;
   const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
   const int col = (threadIdx.x % LPR) * 4;
@@ -117,15 +126,22 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
   const int head = (int)(row - tok * n_qheads);
   const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
   const float* o = ws_o + row * n_part * D + col;
+  int parts = n_part;
+  if (seq_lens != nullptr) {
+    const int len = seq_lens[tok];
+    parts = paged_parts(
+        paged_tiles<MORE>(x, len, len, (len + kt - 1) / kt, kt).n, n_part, per);
+    if (parts == 1) return;
+  }
   const bool sink = MORE && x.sink != nullptr;
   const float sk = sink ? x.sink[head] * 1.4426950408889634f : -INFINITY;
   float M = sk;
-  for (int p = 0; p < n_part; p++) M = fmaxf(M, ml[p].x);
+  for (int p = 0; p < parts; p++) M = fmaxf(M, ml[p].x);
   if (M == -INFINITY) M = 0.0f;
   float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.0f;
   float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 4
-  for (int p = 0; p < n_part; p++) {
+  for (int p = 0; p < parts; p++) {
     const float2 z = ml[p];
     const bool on = z.y > 0.0f;              // else nothing was written
     const float w = on ? __builtin_amdgcn_exp2f(z.x - M) : 0.0f;
@@ -142,11 +158,13 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
 template <int D, bool MORE>
 inline void paged_merge(void* out, const float* ws_o, const float* ws_ml,
                         int n_qheads, int n_part, long out_stride, long rows,
-                        const PagedMore& x, hipStream_t stream) {
+                        const PagedMore& x, hipStream_t stream,
+                        const int* seq_lens = nullptr, int per = 1,
+                        int kt = 1) {
   hipLaunchKernelGGL((paged_attn_merge_kernel<D, MORE>),
                      dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256),
                      0, stream, out, ws_o, ws_ml, n_qheads, n_part, out_stride,
-                     rows, x);
+                     rows, x, seq_lens, per, kt);
 }
 
 }  // namespace xllm

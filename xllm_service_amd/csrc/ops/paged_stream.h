@@ -12,9 +12,11 @@
 //     are multiplied the next keys are: counted waits, each for the older half
 //   * 8 waves a CU (LDS-bound) keep 64-128 KB in flight per CU, four times
 //     what memory latency times bandwidth asks for
-//   * waves of a workgroup merge through LDS at the end; when there are too
-//     few (sequence, kv_head) pairs to fill the chip the keys are split over
-//     P workgroups, whose fp32 results a second kernel merges
+//   * waves of a workgroup merge through LDS at the end; where there are too
+//     few (sequence, kv_head) pairs to fill the chip, or tables long enough for
+//     one sequence to outlast the others, the keys are split over up to P
+//     workgroups, as many as a sequence's own length asks for, whose fp32
+//     results a second kernel merges
 //
 // Measured, 32 query / 8 key heads of 128: 128 sequences of 1-2 k keys 160 ->
 // 143 us, 5.6 TB/s (a large copy: 4.9); 24 x 0.6-1.3 k 24 + 9 -> 18 us; one of
@@ -22,6 +24,8 @@
 // registers a tile ahead, V loaded in the tile that used it, one result per
 // wave through memory.
 #pragma once
+#include <algorithm>
+
 #include "paged_merge.h"
 
 namespace xllm {
@@ -109,7 +113,7 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
     const int* __restrict__ block_tables,    // [num_seqs, max_blocks]
     const int* __restrict__ seq_lens,        // [num_seqs]
     const float scale, const int G, const int n_kv, const int max_blocks,
-    const long q_stride, const long out_stride, const int P,
+    const long q_stride, const long out_stride, const int P, const int per,
     const PagedMore x) {
   constexpr int NW = PA_NW, KS = D / 16, DT = D / 32;
   constexpr int CPR = D / 8;                 // 16 B chunks of a row
@@ -122,14 +126,19 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, c32 = lane & 31;
-  const int part = blockIdx.x % P, unit = blockIdx.x / P;
+  // first the first parts of all: idle ones are then the last and not all of one
+  // XCD (16 x 1000 keys of 8 heads with room for 8: 55 us the other way, 22 so)
+  const int units = gridDim.x / P;
+  const int part = blockIdx.x / units, unit = blockIdx.x % units;
   const int seq = unit / n_kv, kvh = unit % n_kv;
   const int seq_len = seq_lens[seq];
   const int n_tiles = (seq_len + PA_KT - 1) / PA_KT;
   // a wave's tiles are every step-th of the list, from the i0-th on
   const PagedTiles list =
       paged_tiles<MORE>(x, seq_len, seq_len, n_tiles, PA_KT);
-  const int step = P * NW, i0 = part * NW + wid;
+  const int parts = paged_parts(list.n, P, per);
+  if (part >= parts) return;
+  const int step = parts * NW, i0 = part * NW + wid;
   const int lo = paged_first<MORE>(x, seq_len);   // first key in the window
 
   const bool row_ok = c32 < G;
@@ -337,7 +346,7 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
           *reinterpret_cast<const float4*>(mo + (w * G + row) * D + col);
       a[0] += y.x * f; a[1] += y.y * f; a[2] += y.z * f; a[3] += y.w * f;
     }
-    if (P == 1) {
+    if (parts == 1) {
       if (MORE && x.sink != nullptr)
         L += __builtin_amdgcn_exp2f(
             x.sink[kvh * G + row] * 1.4426950408889634f - M);
@@ -357,27 +366,43 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
   }
 }
 
-// Workgroups the keys of a (sequence, kv_head) pair are split over, from what
-// the host knows: the pairs and the widest table. One workgroup per CU is
-// enough to split for (more of them only add results to merge), a part of less
-// than eight tiles (two a wave) is not worth its share of the merge, and
-// neither is a split in two. Measured (us, 32/8 heads of 128), whole | split:
-// 1 x 776 keys 10.2 | 7.8, 1 x 2000 18.8 | 8.9, 1 x 20000 143 | 20 (16 parts),
-// 8 x 2000 19.9 | 15.8, 8 x 14000 144 | 82; 1 x 200 5.4 | 6.6, 8 x 500 8.6 |
-// 9.7, 16 x 1000 13.6 | 15.7, 32 x 1500 36.7 | 40.2. Eight waves in a workgroup
-// instead of four: within 5 % where that many keys are split at all, slower
-// for many pairs (128 x 300 keys: 41 against 33).
-// Capped scores make a tile about twice as long, so that smaller parts and a
-// split in two pay: 16/4 heads, 1 x 700 keys 15.5 | 9.7 (6 parts), 32 x 2000
-// 37.6 | 31.0 (2 parts).
-inline int paged_stream_parts(long num_seqs, int n_kv_heads, long max_blocks,
-                              bool capped = false) {
-  const long units = num_seqs * n_kv_heads;
-  const long tiles = (max_blocks * PA_BS + PA_KT - 1) / PA_KT;
-  long p = units > 0 ? 256 / units : 1;
-  if (p > tiles / (capped ? 4 : 8)) p = tiles / (capped ? 4 : 8);
-  if (p == 2 && capped && tiles >= 48) return 2;
-  return (int)(p < 3 ? 1 : p > 16 ? 16 : p);
+// Parts the keys of a (sequence, kv_head) pair are split into: room for P of them
+// from what the host knows (the pairs and the widest table), one for every `per`
+// tiles of a sequence's own in the kernel.
+//   Few pairs: one workgroup per CU is enough to split for (more only add
+// results to merge), a part of less than eight tiles (two a wave) is not worth its
+// share of the merge, neither is room for two. Measured (us), whole | split: 1 x
+// 776 keys 10.2 | 7.8, 1 x 2000 18.8 | 8.9, 1 x 20000 143 | 20 (16 parts), 8 x
+// 2000 19.9 | 15.8, 8 x 14000 144 | 82; 1 x 200 5.4 | 6.6, 8 x 500 8.6 | 9.7.
+//   More pairs fill the chip, and equal ones lose by a split what the merge costs
+// (16 x 1000 keys, 8 key heads, 13.9 | 15.6; 32 x 1-2 k 36.7 | 40.2), but a long
+// sequence among short ones is a chain of tiles that outlasts the rest. By parts of
+// 32 tiles, at most 8: 23 x 0.3-12 k, 4 key heads 122 | 70; 8 key heads, 16 x 2-16 k
+// 173 | 142, 48 x 0.3-8 k 184 | 159, 32 x 0.3-6 k 83.3 | 82.4, 16 x 0.3-2 k 20.3
+// | 20.3. The host sees no lengths, and in a captured step the widest table there can
+// be: whole below 3000 keys, and up to 128 pairs (which bring the least bytes to
+// hide a chain behind) above, up to 4096 for more pairs.
+//   Capped scores make a tile about twice as long: four tiles a part instead of
+// eight, and with many pairs, of any number, from 1500 keys on at most four parts of
+// 20 tiles. 4 key heads: 32 x 0.7-3 k 47 | 30, 32 x 0-4 k 61 | 37, 64 x 0.3-3 k
+// 54 | 51, 24 x 0.1-1 k in tables of 4096 20 | 19 (parts of 16: 31, 37, 50, 17; of
+// 32: 31, 36, 54, 22).
+//   Eight waves in a workgroup instead of four: within 5 % where keys are split,
+// slower for many pairs (128 x 300 keys: 41 against 33).
+struct PagedSplit { int parts, per; };
+inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
+                                     long max_blocks, bool capped = false) {
+  const long units = num_seqs * n_kv_heads, f = capped ? 2 : 1;
+  const long tiles = f * ((max_blocks * PA_BS + PA_KT - 1) / PA_KT);
+  const bool few = units < 86;
+  const int per = few ? (int)(8 / f) : capped ? 20 : 32;
+  if (few && units > 0) {
+    const long p = std::min<long>({256 / units, tiles / 8, 16});
+    return {p < 3 ? 1 : (int)p, per};
+  }
+  if (units == 0 || tiles < 96 || (units > 128 && !capped && tiles <= 128))
+    return {1, per};
+  return {(int)std::min<long>(8 / f, (tiles + 31) / 32), per};
 }
 
 // Decoded rows (at most 32 query heads per key head) and the merge of their
@@ -388,17 +413,19 @@ inline void paged_stream(void* out, float* ws_o, float* ws_ml,
                          const unsigned short* v_cache, const int* block_tables,
                          const int* seq_lens, int num_seqs, float scale,
                          int n_qheads, int n_kv, int max_blocks, long q_stride,
-                         long out_stride, int parts, const PagedMore& x,
+                         long out_stride, PagedSplit split, const PagedMore& x,
                          hipStream_t stream) {
   if (num_seqs == 0) return;
-  const dim3 grid((unsigned)(num_seqs * n_kv * parts));
+  const dim3 grid((unsigned)(num_seqs * n_kv * split.parts));
   hipLaunchKernelGGL((paged_attn_stream_kernel<D, TERMS, MORE>), grid,
                      dim3(PA_NW * 64), 0, stream, out, ws_o, ws_ml, q, k_cache,
                      v_cache, block_tables, seq_lens, scale, n_qheads / n_kv,
-                     n_kv, max_blocks, q_stride, out_stride, parts, x);
-  if (parts > 1)
-    paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, parts, out_stride,
-                         (long)num_seqs * n_qheads, x, stream);
+                     n_kv, max_blocks, q_stride, out_stride, split.parts,
+                     split.per, x);
+  if (split.parts > 1)
+    paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, split.parts, out_stride,
+                         (long)num_seqs * n_qheads, x, stream, seq_lens,
+                         split.per, PA_KT);
 }
 
 }  // namespace xllm

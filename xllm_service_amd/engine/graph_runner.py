@@ -18,27 +18,11 @@ import numpy as np
 import torch
 
 from .metadata import AttnMetadata
+from .staging import Staging
 
 log = logging.getLogger("xllm.graph")
 
 BUCKETS = (1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256)
-
-
-def _wait_staging(pin: dict) -> None:
-    """Block until the async host-to-device copies of the previous replay
-    have read the pinned staging buffers; only then may the host refill
-    them. A caller that syncs every step (sampling does) never waits here,
-    one that replays without reading results back would otherwise race."""
-    ev = pin.get("copied")
-    if ev is not None:
-        ev.synchronize()
-
-
-def _mark_staging(pin: dict) -> None:
-    ev = pin.get("copied")
-    if ev is None:
-        ev = pin["copied"] = torch.cuda.Event()
-    ev.record()
 
 
 @contextlib.contextmanager
@@ -66,12 +50,11 @@ class DecodeGraphRunner:
         self.device = device
         self.max_blocks = (max_model_len + 15) // 16
         self.buckets = [b for b in BUCKETS if b <= max_batch]
-        self.graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, dict,
+        # graph, its inputs (with a pinned image, so that the copy before a
+        # replay is truly async) and its logits
+        self.graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, Staging,
                                      torch.Tensor]] = {}
         self.pool = None
-        # pinned host staging (one per bucket) so the per-replay H2D copies
-        # are truly async; unpinned numpy->GPU copies serialize the stream
-        self._pinned: Dict[int, dict] = {}
         # per-request padded block-table rows (numpy, cheap incremental update)
         self._bt_rows: Dict[str, Tuple[np.ndarray, int]] = {}
 
@@ -85,16 +68,17 @@ class DecodeGraphRunner:
     @torch.inference_mode()
     def _capture(self, bs: int):
         dev = self.device
-        static = dict(
-            input_ids=torch.zeros(bs, dtype=torch.long, device=dev),
-            positions=torch.zeros(bs, dtype=torch.long, device=dev),
-            slot_mapping=torch.full((bs,), -1, dtype=torch.long, device=dev),
-            seq_lens=torch.full((bs,), 16, dtype=torch.int32, device=dev),
-            block_tables=torch.zeros(bs, self.max_blocks, dtype=torch.int32,
-                                     device=dev),
+        # padding rows must hold valid token and block ids: the first ones (or
+        # stale ones of a larger batch, which were valid once)
+        staging = Staging([
+            ("input_ids", (bs,), np.int64, 0),
+            ("positions", (bs,), np.int64, 0),
+            ("slot_mapping", (bs,), np.int64, -1),
+            ("seq_lens", (bs,), np.int32, 16),
             # recurrent-state slot per row; -1 (padding) touches no state
-            state_slots=torch.full((bs,), -1, dtype=torch.int32, device=dev),
-        )
+            ("state_slots", (bs,), np.int32, -1),
+            ("block_tables", (bs, self.max_blocks), np.int32, 0)], dev)
+        static = staging.dev
         meta = AttnMetadata(
             num_prefill_tokens=0, num_decode_tokens=bs,
             slot_mapping=static["slot_mapping"],
@@ -118,19 +102,7 @@ class DecodeGraphRunner:
             logits = fwd()
         if self.pool is None:
             self.pool = graph.pool()
-        self.graphs[bs] = (graph, static, logits)
-        # zero-init: padding rows of the FULL-width copies must hold valid
-        # token ids / block ids (stale entries from a larger batch are fine
-        # — they were valid once)
-        self._pinned[bs] = dict(
-            i64=torch.zeros(3, bs, dtype=torch.long, pin_memory=True),
-            seq_lens=torch.full((bs,), 16, dtype=torch.int32,
-                                pin_memory=True),
-            block_tables=torch.zeros(bs, self.max_blocks, dtype=torch.int32,
-                                     pin_memory=True),
-            state_slots=torch.full((bs,), -1, dtype=torch.int32,
-                                   pin_memory=True),
-        )
+        self.graphs[bs] = (graph, staging, logits)
 
     # ------------------------------------------------------------------ run
     def bucket_for(self, n: int) -> Optional[int]:
@@ -163,32 +135,21 @@ class DecodeGraphRunner:
             state_slots: Optional[np.ndarray] = None) -> torch.Tensor:
         n = len(input_ids)
         bs = self.bucket_for(n)
-        graph, static, logits = self.graphs[bs]
-        pin = self._pinned[bs]
-        _wait_staging(pin)
-        i64 = pin["i64"].numpy()
-        i64[0, :n] = input_ids
-        i64[1, :n] = positions
-        i64[2, :n] = slots
+        graph, staging, logits = self.graphs[bs]
+        staging.wait()
+        h = staging.host
+        h["input_ids"][:n] = input_ids
+        h["positions"][:n] = positions
+        h["slot_mapping"][:n] = slots
+        h["seq_lens"][:n] = seq_lens
         if n < bs:  # neutralize padding rows
-            i64[2, n:bs] = -1
-        pin["seq_lens"].numpy()[:n] = seq_lens
-        if n < bs:
-            pin["seq_lens"].numpy()[n:bs] = 16
-        np.stack(bt_rows, out=pin["block_tables"].numpy()[:n])
+            h["slot_mapping"][n:] = -1
+            h["seq_lens"][n:] = 16
+        np.stack(bt_rows, out=h["block_tables"][:n])
         if state_slots is not None:
-            ss = pin["state_slots"].numpy()
-            ss[:n] = state_slots
-            ss[n:bs] = -1
-            static["state_slots"].copy_(pin["state_slots"],
-                                        non_blocking=True)
-        static["input_ids"].copy_(pin["i64"][0], non_blocking=True)
-        static["positions"].copy_(pin["i64"][1], non_blocking=True)
-        static["slot_mapping"].copy_(pin["i64"][2], non_blocking=True)
-        static["seq_lens"].copy_(pin["seq_lens"], non_blocking=True)
-        static["block_tables"][:n].copy_(pin["block_tables"][:n],
-                                         non_blocking=True)
-        _mark_staging(pin)
+            h["state_slots"][:n] = state_slots
+            h["state_slots"][n:] = -1
+        staging.flush(n)
         graph.replay()
         return logits[:n]
 
@@ -223,10 +184,9 @@ class PrefillGraphRunner:
         self.max_blocks = (max_model_len + 15) // 16
         self.buckets = [b for b in PREFILL_BUCKETS
                         if b <= min(max_tokens, max_model_len)]
-        self.graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, dict,
+        self.graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, Staging,
                                      torch.Tensor]] = {}
         self.pool = pool
-        self._pinned: Dict[int, dict] = {}
 
     def capture_all(self):
         with collector_paused():
@@ -238,14 +198,13 @@ class PrefillGraphRunner:
     @torch.inference_mode()
     def _capture(self, B: int):
         dev = self.device
-        static = dict(
-            input_ids=torch.zeros(B, dtype=torch.long, device=dev),
-            positions=torch.arange(B, dtype=torch.long, device=dev),
-            slot_mapping=torch.full((B,), -1, dtype=torch.long, device=dev),
-            seq_lens=torch.full((1,), B, dtype=torch.int32, device=dev),
-            block_tables=torch.zeros(1, self.max_blocks, dtype=torch.int32,
-                                     device=dev),
-        )
+        staging = Staging([
+            ("input_ids", (B,), np.int64, 0),
+            ("positions", (B,), np.int64, np.arange(B)),
+            ("slot_mapping", (B,), np.int64, -1),
+            ("seq_lens", (1,), np.int32, B),
+            ("block_tables", (1, self.max_blocks), np.int32, 0)], dev)
+        static = staging.dev
         cu_q = torch.tensor([0, B], dtype=torch.int32, device=dev)
         meta = AttnMetadata(
             num_prefill_tokens=B, num_decode_tokens=0,
@@ -268,13 +227,7 @@ class PrefillGraphRunner:
             hidden = fwd()
         if self.pool is None:
             self.pool = graph.pool()
-        self.graphs[B] = (graph, static, hidden)
-        self._pinned[B] = dict(
-            i64=torch.zeros(3, B, dtype=torch.long, pin_memory=True),
-            seq_len=torch.full((1,), B, dtype=torch.int32, pin_memory=True),
-            block_tables=torch.zeros(1, self.max_blocks, dtype=torch.int32,
-                                     pin_memory=True),
-        )
+        self.graphs[B] = (graph, staging, hidden)
 
     def bucket_for(self, n: int) -> Optional[int]:
         for b in self.buckets:
@@ -290,24 +243,18 @@ class PrefillGraphRunner:
         tokens; returns the static hidden buffer (read rows < len(tokens)
         before the next replay)."""
         L = len(tokens)
-        graph, static, hidden = self.graphs[B]
-        pin = self._pinned[B]
-        _wait_staging(pin)
-        i64 = pin["i64"].numpy()
-        i64[0, :L] = tokens
-        i64[1, :L] = positions
-        i64[1, L:B] = np.arange(chunk_start + L, chunk_start + B)
-        i64[2, :L] = slots
-        i64[2, L:B] = -1
-        pin["seq_len"].numpy()[0] = chunk_start + B
-        bt = pin["block_tables"].numpy()
+        graph, staging, hidden = self.graphs[B]
+        staging.wait()
+        h = staging.host
+        h["input_ids"][:L] = tokens
+        h["positions"][:L] = positions
+        h["positions"][L:] = np.arange(chunk_start + L, chunk_start + B)
+        h["slot_mapping"][:L] = slots
+        h["slot_mapping"][L:] = -1
+        h["seq_lens"][0] = chunk_start + B
+        bt = h["block_tables"]
         bt[0, :] = 0
         bt[0, :len(block_table)] = block_table
-        static["input_ids"].copy_(pin["i64"][0], non_blocking=True)
-        static["positions"].copy_(pin["i64"][1], non_blocking=True)
-        static["slot_mapping"].copy_(pin["i64"][2], non_blocking=True)
-        static["seq_lens"].copy_(pin["seq_len"], non_blocking=True)
-        static["block_tables"].copy_(pin["block_tables"], non_blocking=True)
-        _mark_staging(pin)
+        staging.flush(1)
         graph.replay()
         return hidden

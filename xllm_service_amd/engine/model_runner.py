@@ -8,6 +8,7 @@ from __future__ import annotations
 
 from typing import Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from xllm_service_amd import ops
@@ -19,6 +20,7 @@ from .cache_spec import (CacheGroup, ConvState, PagedKV, PagedLatent,
 from .metadata import AttnMetadata
 from .scheduler import StepPlan
 from .sequence import Sequence
+from .staging import upload
 
 BLOCK_SIZE = 16
 UNPAGED_BLOCKS = 1 << 20     # pool of a model without block-addressed caches
@@ -201,76 +203,63 @@ class ModelRunner:
             d_tables.append(seq.block_table)
             d_state.append(seq.state_slot)
 
-        import numpy as _np
         if mrope_spans:
-            pos_np = _np.tile(_np.asarray(positions, dtype=_np.int64), (3, 1))
+            pos_np = np.tile(np.asarray(positions, dtype=np.int64), (3, 1))
             for row0, sp in mrope_spans:
                 pos_np[:, row0:row0 + sp.chunk_len] = \
                     sp.seq.mrope_pos[:, sp.chunk_start:
                                      sp.chunk_start + sp.chunk_len]
         else:
-            pos_np = _np.asarray(positions, dtype=_np.int64)
+            pos_np = np.asarray(positions, dtype=np.int64)
 
-        def pad_tables(tables: List[List[int]]) -> torch.Tensor:
+        def tables_np(tables):
             if not tables:
-                return torch.zeros(0, 1, dtype=torch.int32, device=self.device)
+                return None
             w = max(len(t) for t in tables)
-            out = torch.zeros(len(tables), w, dtype=torch.int32)
+            out = np.zeros((len(tables), w), dtype=np.int32)
             for i, t in enumerate(tables):
-                out[i, :len(t)] = torch.tensor(t, dtype=torch.int32)
-            return out.to(self.device)
+                out[i, :len(t)] = t
+            return out
 
-        dev = self.device
+        def arr(values, dtype=np.int32):
+            return np.asarray(values, dtype=dtype)
+
+        host = dict(slot_mapping=arr(slots, np.int64),
+                    input_ids=arr(tokens, np.int64), positions=pos_np)
+        if plan.prefills:
+            host.update(cu_q=arr(cu_q), prefill_seq_lens=arr(p_seq_lens),
+                        prefill_block_tables=tables_np(p_tables))
+        if plan.decodes:
+            host.update(decode_seq_lens=arr(d_seq_lens),
+                        decode_block_tables=tables_np(d_tables))
         np_ = cu_q[-1]
         from xllm_service_amd.distributed import parallel_state as ps
         if ps.tp_size() > 1 and ps.tp_rank() == 0:
-            def tables_np(tables):
-                if not tables:
-                    return None
-                w = max(len(t) for t in tables)
-                out = _np.zeros((len(tables), w), dtype=_np.int32)
-                for i, t in enumerate(tables):
-                    out[i, :len(t)] = t
-                return out
             self._tp_batch = dict(
                 kind="eager", np=np_, nd=len(plan.decodes),
-                input_ids=_np.asarray(tokens, dtype=_np.int64),
-                positions=pos_np,
-                slots=_np.asarray(slots, dtype=_np.int64),
-                cu_q=_np.asarray(cu_q, dtype=_np.int32)
-                if plan.prefills else None,
-                p_seq_lens=_np.asarray(p_seq_lens, dtype=_np.int32)
-                if plan.prefills else None,
-                p_tables=tables_np(p_tables) if plan.prefills else None,
-                d_seq_lens=_np.asarray(d_seq_lens, dtype=_np.int32)
-                if plan.decodes else None,
-                d_tables=tables_np(d_tables) if plan.decodes else None,
+                input_ids=host["input_ids"], positions=pos_np,
+                slots=host["slot_mapping"], cu_q=host.get("cu_q"),
+                p_seq_lens=host.get("prefill_seq_lens"),
+                p_tables=host.get("prefill_block_tables"),
+                d_seq_lens=host.get("decode_seq_lens"),
+                d_tables=host.get("decode_block_tables"),
             )
-        meta = AttnMetadata(
-            num_prefill_tokens=np_,
-            num_decode_tokens=len(plan.decodes),
-            slot_mapping=torch.tensor(slots, dtype=torch.long, device=dev),
-            cu_q=(torch.tensor(cu_q, dtype=torch.int32, device=dev)
-                  if plan.prefills else None),
-            prefill_seq_lens=(torch.tensor(p_seq_lens, dtype=torch.int32,
-                                           device=dev) if plan.prefills else None),
-            prefill_block_tables=pad_tables(p_tables) if plan.prefills else None,
-            decode_seq_lens=(torch.tensor(d_seq_lens, dtype=torch.int32,
-                                          device=dev) if plan.decodes else None),
-            decode_block_tables=pad_tables(d_tables) if plan.decodes else None,
-        )
         if self.uses_state_slots:
-            i32 = dict(dtype=torch.int32, device=dev)
             if plan.prefills:
-                meta.max_prefill_len = max(sp.chunk_len
-                                           for sp in plan.prefills)
-                meta.prefill_ctx_lens = torch.tensor(p_ctx, **i32)
-                meta.prefill_state_slots = torch.tensor(p_state, **i32)
+                host.update(prefill_ctx_lens=arr(p_ctx),
+                            prefill_state_slots=arr(p_state))
             if plan.decodes:
-                meta.decode_state_slots = torch.tensor(d_state, **i32)
-        input_ids = torch.tensor(tokens, dtype=torch.long, device=dev)
-        pos_t = torch.from_numpy(pos_np).to(dev)
+                host["decode_state_slots"] = arr(d_state)
+        on_dev = dict(zip(host, upload(list(host.values()), self.device)))
+        input_ids, pos_t = on_dev.pop("input_ids"), on_dev.pop("positions")
+        meta = AttnMetadata(num_prefill_tokens=np_,
+                            num_decode_tokens=len(plan.decodes), **on_dev)
+        if self.uses_state_slots and plan.prefills:
+            meta.max_prefill_len = max(sp.chunk_len for sp in plan.prefills)
         return input_ids, pos_t, meta
+
+    def _row_index(self, rows: List[int]) -> torch.Tensor:
+        return upload([np.asarray(rows, dtype=np.int64)], self.device)[0]
 
     # ---- sampling -----------------------------------------------------------
     def _logprobs(self, logits: torch.Tensor, seqs: List[Sequence],
@@ -403,15 +392,14 @@ class ModelRunner:
             if not rows:
                 return logits.new_zeros((0, logits.shape[-1]),
                                         dtype=torch.float32)
-            idx = torch.tensor(rows, dtype=torch.long, device=logits.device)
-            return logits[idx].float()
+            return logits[self._row_index(rows)].float()
         input_ids, positions, meta = self._build_batch(plan, bm)
         self._tp_batch = None
         hidden = self.model(input_ids, positions, self.kv_caches, meta)
         if not rows:
             return torch.zeros(0, self.cfg.vocab_size, dtype=torch.float32)
-        idx = torch.tensor(rows, dtype=torch.long, device=hidden.device)
-        return self.model.compute_logits(hidden[idx]).float()
+        return self.model.compute_logits(
+            hidden[self._row_index(rows)]).float()
 
     # ---- one step -----------------------------------------------------------
     @torch.inference_mode()
@@ -437,10 +425,11 @@ class ModelRunner:
         if tp_batch is not None:
             # rows that will need logits (followers must join the logits
             # all-gather with the same selection size)
-            rows_pre = []
-            for i, sp in enumerate(plan.prefills):
+            rows_pre, end = [], 0
+            for sp in plan.prefills:
+                end += sp.chunk_len
                 if sp.chunk_start + sp.chunk_len >= sp.seq.prompt_len:
-                    rows_pre.append(int(meta.cu_q[i + 1]) - 1)
+                    rows_pre.append(end - 1)
             rows_pre.extend(meta.num_prefill_tokens + j
                             for j in range(len(plan.decodes)))
             tp_batch["rows"] = rows_pre
@@ -455,9 +444,11 @@ class ModelRunner:
         # plus every decode row
         rows: List[int] = []
         seqs: List[Sequence] = []
-        for i, sp in enumerate(plan.prefills):
+        end = 0
+        for sp in plan.prefills:
+            end += sp.chunk_len
             if sp.chunk_start + sp.chunk_len >= sp.seq.prompt_len:
-                rows.append(int(meta.cu_q[i + 1]) - 1)
+                rows.append(end - 1)
                 seqs.append(sp.seq)
         np_ = meta.num_prefill_tokens
         for j, seq in enumerate(plan.decodes):
@@ -465,7 +456,7 @@ class ModelRunner:
             seqs.append(seq)
         if not rows:
             return {}
-        sel = hidden[torch.tensor(rows, dtype=torch.long, device=hidden.device)]
+        sel = hidden[self._row_index(rows)]
         logits = self.model.compute_logits(sel)
         tokens = self._sample(logits, seqs)
         lps = self._logprobs(logits, seqs, tokens)
@@ -497,7 +488,6 @@ class ModelRunner:
     def _execute_prefill_graph(self, sp, b) -> Dict[str, int]:
         """Single-sequence prefill chunk via the captured graph (the
         serving arrival fast path; see PrefillGraphRunner padding notes)."""
-        import numpy as np
         seq = sp.seq
         cs, L = sp.chunk_start, sp.chunk_len
         tokens = np.asarray(seq.prompt_token_ids[cs:cs + L], dtype=np.int64)
@@ -521,7 +511,6 @@ class ModelRunner:
     def _decode_graph_logits(self, plan: StepPlan, bm) -> torch.Tensor:
         """Logits [n_decodes, vocab] of a decode-only plan via the captured
         graph of its batch-size bucket."""
-        import numpy as np
         seqs = plan.decodes
         n = len(seqs)
         input_ids = np.empty(n, dtype=np.int64)

@@ -1,8 +1,8 @@
 // Fused activation kernels (SwiGLU / GEGLU) for MI355X (gfx950).
 //
-// out[t, i] = act(x[t, i]) * x[t, I + i] — one fused pass, bf16x8
-// vectorized, flattened grid-stride over (t, i) so small decode batches
-// still fill the chip (grid is sized by total work, not by rows).
+// out[t, i] = act(x[t, i]) * x[t, I + i] — one fused pass, 16 B per lane; the
+// grid is workgroups of a row by rows, so that nothing is divided.
+// 300 rows of 14336 5.72 -> 5.31 us, 8192 135 -> 120 us (5.9 TB/s).
 #include "common.h"
 
 namespace xllm {
@@ -11,12 +11,10 @@ template <bool GELU>
 __global__ void act_and_mul_kernel(
     unsigned short* __restrict__ out,      // [T, I]
     const unsigned short* __restrict__ x,  // [T, 2*I]
-    const int I, const long total_vec) {   // total_vec = T * I/8
-  const int iv = I / 8;
-  for (long v = blockIdx.x * (long)blockDim.x + threadIdx.x; v < total_vec;
-       v += (long)gridDim.x * blockDim.x) {
-    const long row = v / iv;
-    const int col = (int)(v % iv) * 8;
+    const int I, const int T) {
+  const int col = (blockIdx.x * 256 + threadIdx.x) * 8;
+  if (col >= I) return;
+  for (long row = blockIdx.y; row < T; row += gridDim.y) {
     ushort8_t g = *reinterpret_cast<const ushort8_t*>(x + row * 2 * I + col);
     ushort8_t u = *reinterpret_cast<const ushort8_t*>(x + row * 2 * I + I + col);
     ushort8_t r;
@@ -37,25 +35,23 @@ __global__ void act_and_mul_kernel(
   }
 }
 
-static inline dim3 act_grid(long total_vec) {
-  long g = (total_vec + 255) / 256;
-  if (g > 2048) g = 2048;  // grid-stride the rest (Guideline 11)
-  if (g < 1) g = 1;
-  return dim3((unsigned)g);
+template <bool GELU>
+static void act_launch(unsigned short* out, const unsigned short* x, int T,
+                       int I, hipStream_t stream) {
+  if (T <= 0 || I <= 0) return;
+  const dim3 grid((unsigned)((I / 8 + 255) / 256), (unsigned)(T < 65535 ? T : 65535));
+  hipLaunchKernelGGL((act_and_mul_kernel<GELU>), grid, dim3(256), 0, stream,
+                     out, x, I, T);
 }
 
 void launch_silu_and_mul(unsigned short* out, const unsigned short* x, int T,
                          int I, hipStream_t stream) {
-  const long total = (long)T * (I / 8);
-  hipLaunchKernelGGL((act_and_mul_kernel<false>), act_grid(total), dim3(256),
-                     0, stream, out, x, I, total);
+  act_launch<false>(out, x, T, I, stream);
 }
 
 void launch_gelu_and_mul(unsigned short* out, const unsigned short* x, int T,
                          int I, hipStream_t stream) {
-  const long total = (long)T * (I / 8);
-  hipLaunchKernelGGL((act_and_mul_kernel<true>), act_grid(total), dim3(256),
-                     0, stream, out, x, I, total);
+  act_launch<true>(out, x, T, I, stream);
 }
 
 }  // namespace xllm

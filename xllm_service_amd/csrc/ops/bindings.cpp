@@ -364,7 +364,8 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor w,
                     torch::jit::tracer::isTracing() ||
                     at::autocast::is_autocast_enabled(at::kCUDA);
   if (!grad && !seen && rows16(x) && rows16(w) && x.size(1) == w.size(1) &&
-      x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) && w.is_contiguous() &&
+      x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) &&
+      x.stride(0) < (1L << 24) && w.is_contiguous() &&
       x.device() == w.device() &&
       (!bias.has_value() ||
        (plain(*bias) && bias->dim() == 1 && bias->is_contiguous() &&

@@ -34,7 +34,7 @@
 //
 // Fragments of 16x16x32 (lane l, g = l >> 4): A[l&15][g*8 + j], B[g*8 +
 // j][l&15], C[g*4 + r][l&15].
-#include "../ops/mfma_rows.h"
+#include "../ops/paged_merge.h"
 #include "hybrid_common.h"
 
 namespace xllm {
@@ -355,22 +355,9 @@ __global__ void __launch_bounds__(256) latent_stream_merge_kernel(
       (len + LS_KT - 1) / LS_KT -
           (window > 0 ? max(0, len - window) / LS_KT : 0), n_part, per);
   if (parts == 1) return;                        // written where it belongs
-  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
-  const float* o = ws_o + row * n_part * LS_R + col;
-  float M = -INFINITY;
-  for (int p = 0; p < parts; p++) M = fmaxf(M, ml[p].x);
-  if (M == -INFINITY) M = 0.0f;
-  float L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-  for (int p = 0; p < parts; p++) {
-    const float2 z = ml[p];
-    const bool on = z.y > 0.0f;                  // else nothing was written
-    const float f = on ? __builtin_amdgcn_exp2f(z.x - M) : 0.0f;
-    const float4 y = *reinterpret_cast<const float4*>(o + (long)p * LS_R);
-    L += on ? z.y * f : 0.0f;
-    a[0] += on ? y.x * f : 0.0f; a[1] += on ? y.y * f : 0.0f;
-    a[2] += on ? y.z * f : 0.0f; a[3] += on ? y.w * f : 0.0f;
-  }
+  float M = -INFINITY, L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  paged_add_parts<8>(reinterpret_cast<const float2*>(ws_ml) + row * n_part,
+                     ws_o + row * n_part * LS_R + col, parts, LS_R, M, L, a);
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   *reinterpret_cast<float4*>(out + row * LS_R + col) =
       make_float4(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);

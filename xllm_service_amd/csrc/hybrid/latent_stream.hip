@@ -331,9 +331,9 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   const long slot = row * n_part + part;
   if (w == 0 && g == 0) {
     ws_ml[slot * 2] = m * c;
-    ws_ml[slot * 2 + 1] = l;
+    ws_ml[slot * 2 + 1] = t_begin < t_end ? l : PAGED_ABSENT;
   }
-  if (t_begin >= t_end) return;                  // an empty part: l = 0
+  if (t_begin >= t_end) return;
   float* o = ws_o + slot * LS_R + col;
 #pragma unroll
   for (int i = 0; i < 8; i++)

@@ -108,12 +108,16 @@ XLLM_DEV void paged_put(const PagedMore& x, void* out, long at, float a,
   }
 }
 
+#define PAGED_ABSENT (-1.0f)
+
 // Parts of a row, B at a time, added to (M, L, a): their maxima, sums and results
 // are all on the way at once, the first maximum is not waited for before the first
 // result is fetched. A merge is a launch and this chain: 32 rows x 16 heads, up to
 // four parts 4.67 -> 4.07 us, 17 k rows of three parts 6.55 -> 5.95; by eights where
 // there is room for more than four.
-// ml, o: of the row's first part, stride floats between results.
+// ml, o: of the row's first part, stride floats between results. A part without
+// keys has written no results and the sum PAGED_ABSENT: any other sum, NaN
+// among them, counts.
 template <int B>
 XLLM_DEV void paged_add_parts(const float2* ml, const float* o, int parts,
                               int stride, float& M, float& L, float (&a)[4]) {
@@ -129,7 +133,7 @@ XLLM_DEV void paged_add_parts(const float2* ml, const float* o, int parts,
     float top = M;
 #pragma unroll
     for (int k = 0; k < B; k++) {
-      if (p0 + k >= parts) z[k].y = 0.0f;
+      if (p0 + k >= parts) z[k].y = PAGED_ABSENT;
       top = fmaxf(top, z[k].x);
     }
     if (top == -INFINITY) top = 0.0f;
@@ -140,7 +144,7 @@ XLLM_DEV void paged_add_parts(const float2* ml, const float* o, int parts,
     for (int c = 0; c < 4; c++) a[c] *= keep;
 #pragma unroll
     for (int k = 0; k < B; k++) {
-      const bool on = z[k].y > 0.0f;             // else nothing was written
+      const bool on = !(z[k].y < 0.0f);
       const float w = on ? __builtin_amdgcn_exp2f(z[k].x - M) : 0.0f;
       L += on ? z[k].y * w : 0.0f;
       a[0] += on ? y[k].x * w : 0.0f; a[1] += on ? y[k].y * w : 0.0f;

@@ -334,9 +334,9 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
   const long slot = grow * n_part + part;
   if (h == 0) {
     ws_ml[slot * 2] = m * sc.c;
-    ws_ml[slot * 2 + 1] = l;
+    ws_ml[slot * 2 + 1] = i_begin < i_end ? l : PAGED_ABSENT;
   }
-  if (i_begin >= i_end) return;              // an empty part: l = 0
+  if (i_begin >= i_end) return;
   float* o = ws_o + slot * D + 4 * h;
 #pragma unroll
   for (int dt = 0; dt < DT; dt++)

@@ -86,3 +86,33 @@ def test_many_chunks_and_hard_decays():
     """More chunks than the scan holds in flight; decays whose powers leave
     fp32's normal range within a chunk, and none at all."""
     run(128, 128, [1300, 200], [0, 9], [0, 2], [0.3, 0.0, 0.996], 1300, 4)
+
+
+@pytest.mark.parametrize("long", [40, 300])         # one chunk each; a scan
+def test_sequences_without_new_tokens(long):
+    """A carried state stays bit for bit, a fresh one becomes zero, a sequence
+    without a slot touches nothing, and the others do not notice."""
+    g = torch.Generator().manual_seed(long)
+    heads, D, bound = 2, 64, max(long, 17)
+    a = torch.tensor([0.9, 0.99]).cuda()
+    first = torch.randn(5, heads, D, D, generator=g).cuda()
+    rows = torch.randn(long + 17, 3 * heads * D, generator=g).to(
+        torch.bfloat16).cuda()
+    i32 = dict(dtype=torch.int32, device="cuda")
+
+    def go(starts, ctx, slots):
+        state = first.clone()
+        out = torch.full((long + 17, heads, D), 9.0, device="cuda")
+        H.decay_attn(*rows.chunk(3, 1), a, state, torch.tensor(slots, **i32),
+                     torch.tensor(starts, **i32), torch.tensor(ctx, **i32),
+                     out, max_q_len=bound)
+        return out, state
+    out, state = go([0, 0, long, long, long, long + 17, long + 17],
+                    [5, 3, 4, 0, 0, 7], [0, 1, -1, 2, 3, 4])
+    want, alone = go([0, long, long + 17], [3, 0], [1, 3])
+    assert torch.equal(out, want)
+    for slot in (0, 4):
+        assert torch.equal(state[slot], first[slot])
+    assert (state[2] == 0).all()
+    for slot in (1, 3):
+        assert torch.equal(state[slot], alone[slot])

@@ -174,16 +174,19 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
     }
   }
   float* dst;
-  float keep = 0.f;                               // factor of what is there
+  bool add = false;                               // to what is there,
+  float keep = 0.f;                               // by this factor
   if (P.ws != nullptr) {
     dst = P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V);
   } else {
     const int slot = P.slots[s];
     if (slot < 0) return;
     dst = P.state + ((long)slot * P.heads + hd) * (D * V);
-    if (P.ctx_lens[s] > 0) keep = pw[len];
+    add = P.ctx_lens[s] > 0;
+    // no new tokens: a carried state stays (and no barrier has made pw visible)
+    if (add && len <= 0) return;
+    if (add) keep = pw[len];
   }
-  const bool add = P.ws == nullptr && P.ctx_lens[s] > 0;
 #pragma unroll
   for (int i = 0; i < DT; ++i)
 #pragma unroll

@@ -106,6 +106,30 @@ def test_prefill_edges(dim, lens, ctx, kv_heads, per):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("ctx", [[3, 0], [2600, 900]])      # whole; in parts
+def test_prefill_leaves_other_rows(dim, ctx):
+    """Rows of q and out outside of every prompt (cu_q) are not written."""
+    lens, heads = [5, 9], 4
+    rows, k, v, table = make(lens, ctx, 1, heads, dim, 21)
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    pad = torch.randn(2, heads, dim).to(torch.bfloat16)
+    tail = torch.randn(6, heads, dim).to(torch.bfloat16)
+    cu = torch.tensor([2, 7, 16], dtype=torch.int32)
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)], dtype=torch.int32)
+    dev = [t.cuda() for t in (k, v, table, cu, sl)]
+    qd, scale = torch.cat([pad, q, tail]).cuda(), dim ** -0.5
+    ref, big = want(q, k, v, table, lens, ctx, scale)
+    out = torch.full_like(qd, 7.0)
+    ops.paged_attn_prefill(qd, *dev, scale, out=out)
+    check(out[2:16], ref, big)
+    assert (out[:2] == 7.0).all() and (out[16:] == 7.0).all()
+    out = torch.full((22, heads * dim), 7.0, device="cuda")
+    H.capped_attn(qd.flatten(1), *dev[:3], *dev[3:], heads, scale, 0.0, out)
+    check(out[2:16].unflatten(-1, (heads, dim)), ref, big)
+    assert (out[:2] == 7.0).all() and (out[16:] == 7.0).all()
+
+
 def test_prefill_standout_scores():
     """Scores far apart: the running maximum moves within and across tiles."""
     lens, ctx = [40], [150]

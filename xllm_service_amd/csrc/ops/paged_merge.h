@@ -156,13 +156,16 @@ XLLM_DEV void paged_add_parts(const float2* ml, const float* o, int parts,
 // out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
 // row, four columns each. seq_lens: rows are decoded ones, one sequence each,
 // with as many parts as their length asks for (per tiles of kt keys); a single
-// part has been written where it belongs. B: parts fetched at once.
+// part has been written where it belongs. cu_q: rows are those of n_seqs prompts;
+// tokens outside of all of them have no parts and stay as they are. B: parts
+// fetched at once.
 template <int D, bool MORE, int B>
 __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
     void* __restrict__ out, const float* __restrict__ ws_o,
     const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
     const long out_stride, const long rows, const PagedMore x,
-    const int* __restrict__ seq_lens, const int per, const int kt) {
+    const int* __restrict__ seq_lens, const int per, const int kt,
+    const int* __restrict__ cu_q, const int n_seqs) {
   constexpr int LPR = D / 4;
   const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
   const int col = (threadIdx.x % LPR) * 4;
@@ -170,6 +173,7 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
   const long tok = row / n_qheads;
   const int head = (int)(row - tok * n_qheads);
   int parts = n_part;
+  if (cu_q != nullptr && (tok < cu_q[0] || tok >= cu_q[n_seqs])) return;
   if (seq_lens != nullptr) {
     const int len = seq_lens[tok];
     parts = paged_parts(
@@ -191,13 +195,13 @@ template <int D, bool MORE>
 inline void paged_merge(void* out, const float* ws_o, const float* ws_ml,
                         int n_qheads, int n_part, long out_stride, long rows,
                         const PagedMore& x, hipStream_t stream,
-                        const int* seq_lens = nullptr, int per = 1,
-                        int kt = 1) {
+                        const int* seq_lens, int per, int kt,
+                        const int* cu_q = nullptr, int n_seqs = 0) {
 #define PM_GO(B)                                                               \
   hipLaunchKernelGGL((paged_attn_merge_kernel<D, MORE, B>),                    \
                      dim3((unsigned)((rows * (D / 4) + 255) / 256)),           \
                      dim3(256), 0, stream, out, ws_o, ws_ml, n_qheads, n_part, \
-                     out_stride, rows, x, seq_lens, per, kt)
+                     out_stride, rows, x, seq_lens, per, kt, cu_q, n_seqs)
   if (n_part <= 4) PM_GO(4);
   else PM_GO(8);
 #undef PM_GO

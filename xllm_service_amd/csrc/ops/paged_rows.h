@@ -385,7 +385,8 @@ inline void paged_rows(void* out, float* ws_o, float* ws_ml,
                      max_blocks, q_stride, out_stride, n_part, x);
   if (n_part > 1)
     paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, n_part, out_stride,
-                         tokens * n_qheads, x, stream);
+                         tokens * n_qheads, x, stream, nullptr, 1, 1, cu_q,
+                         n_seqs);
 }
 
 }  // namespace xllm

@@ -68,6 +68,28 @@ def test_paged(entry, dim, how, where, bad):
 
 
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("where", ["q", "k"])
+@pytest.mark.parametrize("how", ["whole", "split"])
+@pytest.mark.parametrize("dim", [64, 128, 96])
+@pytest.mark.parametrize("decode", [True, False])
+def test_capped_scores(decode, dim, how, where, bad):
+    """Scores of every size meet the cap: a NaN stays one, an infinite one
+    becomes the cap (96: the kernel for other widths)."""
+    lens, ctx, kv_heads, per = (DECODE if decode else PREFILL)[how]
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, 8)
+    plant(bad, where, rows, k, v, table, dim)
+    heads, cap, scale = kv_heads * per, 3.0, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0))).int().cuda()
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)]).int().cuda()
+    out = torch.zeros(sum(lens), heads, dim, device="cuda")
+    H.capped_attn(rows.cuda()[:, :heads * dim],
+                  *(t.cuda() for t in (k, v, table)),
+                  None if decode else cu, sl, heads, scale, cap, out)
+    agree(out, want(q, k, v, table, lens, ctx, scale, cap=cap)[0])
+
+
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
 @pytest.mark.parametrize("where", ["q", "key", "tail"])
 @pytest.mark.parametrize("keys", [[30, 20], [90, 2600]])
 def test_latent(keys, where, bad):

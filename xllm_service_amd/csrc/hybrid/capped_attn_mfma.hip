@@ -65,7 +65,7 @@ XLLM_DEV bf16x8 cm_ld8(const unsigned short* p) {
 }
 
 XLLM_DEV float cm_tanh(float x) {          // 1 - 2 / (e^(2x) + 1)
-  const float e = __expf(2.0f * fminf(x, 15.0f));
+  const float e = __expf(2.0f * (x > 15.0f ? 15.0f : x));  // NaN stays
   return 1.0f - 2.0f / (e + 1.0f);
 }
 

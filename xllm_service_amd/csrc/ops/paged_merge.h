@@ -80,7 +80,7 @@ XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
       y = fmaf(y, w, -1.0f / 3.0f);
       y = fmaf(y * w, v, v);
       if (far) {
-        const float e = __expf(2.0f * fminf(v, 15.0f));
+        const float e = __expf(2.0f * (v > 15.0f ? 15.0f : v));  // NaN stays
         const float z = 1.0f - 2.0f / (e + 1.0f);
         y = fabsf(v) < 0.5f ? y : z;
       }

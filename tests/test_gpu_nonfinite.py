@@ -114,3 +114,36 @@ def test_latent(keys, where, bad):
         k = cache[table[s, :need[s]].long()].reshape(-1, W)[:n].double()
         ref.append(torch.softmax(q[s].double() @ k.t() * scale, -1) @ k[:, :r])
     agree(out, torch.stack(ref))
+
+
+@pytest.mark.parametrize("how", ["whole", "split"])
+@pytest.mark.parametrize("decode", [True, False])
+def test_nan_factors(decode, how):
+    """A NaN scale, or the NaN multiplier or sink of one head."""
+    lens, ctx, kv_heads, per = (DECODE if decode else PREFILL)[how]
+    rows, k, v, table = make(lens, ctx, kv_heads, per, 128, 9)
+    heads = kv_heads * per
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0))).int().cuda()
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)]).int().cuda()
+    dev = [t.cuda() for t in (k, v, table)]
+    q = rows.cuda()[:, :heads * 128]
+    for cap in (0.0, 5.0):
+        mult = torch.ones(heads, device="cuda")
+        mult[2] = math.nan
+        out = torch.zeros(sum(lens), heads, 128, device="cuda")
+        for more in (dict(head_scale=mult), dict(sink=mult)):
+            H.capped_attn(q, *dev, None if decode else cu, sl, heads, 0.1, cap,
+                          out, **more)
+            gone = torch.isnan(out)
+            assert gone[:, 2].all() and gone.sum() == gone[:, 2].numel()
+    q = q.unflatten(-1, (heads, 128))
+    out = ops.paged_attn_decode(q, *dev, sl, math.nan) if decode else \
+        ops.paged_attn_prefill(q, *dev, cu, sl, math.nan)
+    assert torch.isnan(out).all()
+    if decode:
+        latent = torch.randn(dev[0].shape[0], 16, 512, device="cuda").to(
+            torch.bfloat16)
+        out = torch.zeros(len(lens), 8, 512, device="cuda")
+        H.latent_attn(torch.ones_like(out, dtype=torch.bfloat16), latent,
+                      dev[2], None, sl, math.nan, 512, out)
+        assert torch.isnan(out).all()

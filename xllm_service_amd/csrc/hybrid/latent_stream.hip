@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   const bool on = h0 + n < heads;
   const long row = (long)s * heads + (on ? h0 + n : h0);
   const short flip = scale < 0.0f ? (short)0x8000 : (short)0;
-  const float c = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);
+  const float c = paged_factor(scale);
   bf16x8 qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++)
@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   if (!on) return;
   const int col = w * 128 + g * 4;
   if (parts == 1) {
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float inv = l != 0.0f ? 1.0f / l : 0.0f;
     float* o = out + row * LS_R + col;
 #pragma unroll
     for (int i = 0; i < 8; i++)
@@ -358,7 +358,7 @@ __global__ void __launch_bounds__(256) latent_stream_merge_kernel(
   float M = -INFINITY, L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   paged_add_parts<8>(reinterpret_cast<const float2*>(ws_ml) + row * n_part,
                      ws_o + row * n_part * LS_R + col, parts, LS_R, M, L, a);
-  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  const float inv = L != 0.0f ? 1.0f / L : 0.0f;
   *reinterpret_cast<float4*>(out + row * LS_R + col) =
       make_float4(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
 }

@@ -40,6 +40,12 @@ XLLM_DEV PagedTiles paged_tiles(const PagedMore& x, int limit, int kmax,
   return {keep, first - keep, n_tiles - (first - keep)};
 }
 
+// |scale| log2(e), above zero; a NaN stays one
+XLLM_DEV float paged_factor(float scale) {
+  const float c = fabsf(scale) * 1.4426950408889634f;
+  return c < 1e-30f ? 1e-30f : c;
+}
+
 // How a row's scores become weights 2^(c (s - m)): a negative factor turns the
 // signs of the query's entries, so that c is positive; with a cap, s is the
 // capped score and pre goes in front of the tanh.
@@ -50,7 +56,7 @@ XLLM_DEV PagedScore paged_score(const PagedMore& x, float scale, int head) {
   if (MORE && x.head_scale != nullptr) scale *= x.head_scale[head];
   if (MORE && x.cap > 0.0f) return {0, log2e, scale / x.cap};
   return {scale < 0.0f ? (short)0x8000 : (short)0,
-          fmaxf(fabsf(scale) * log2e, 1e-30f), 0.0f};
+          paged_factor(scale), 0.0f};
 }
 
 // s <- cap * tanh(pre * s). Below 1/2 the odd Taylor series up to x^15 (the next
@@ -186,7 +192,7 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
   float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   paged_add_parts<B>(reinterpret_cast<const float2*>(ws_ml) + row * n_part,
                      ws_o + row * n_part * D + col, parts, D, M, L, a);
-  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  const float inv = L != 0.0f ? 1.0f / L : 0.0f;
   paged_put<MORE>(x, out, tok * out_stride + (long)head * D + col, a[0] * inv,
                   a[1] * inv, a[2] * inv, a[3] * inv);
 }

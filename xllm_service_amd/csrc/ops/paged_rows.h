@@ -320,7 +320,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
     if (MORE && x.sink != nullptr)
       l += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f -
                                   m * sc.c);
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float inv = l != 0.0f ? 1.0f / l : 0.0f;
     const long at = (long)(q_start + qi) * out_stride + (long)head * D + 4 * h;
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)

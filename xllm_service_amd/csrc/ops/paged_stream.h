@@ -350,7 +350,7 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
       if (MORE && x.sink != nullptr)
         L += __builtin_amdgcn_exp2f(
             x.sink[kvh * G + row] * 1.4426950408889634f - M);
-      const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+      const float inv = L != 0.0f ? 1.0f / L : 0.0f;
       paged_put<MORE>(x, out, (long)seq * out_stride +
                       (long)(kvh * G + row) * D + col,
                       a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);

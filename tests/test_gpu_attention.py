@@ -206,6 +206,22 @@ def test_decode_standout_scores():
     check(got, *want(q, k, v, table, [1, 1], [900, 350], 0.3))
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("width", [0, 1])
+def test_decode_without_keys(dim, width):
+    """Sequences of no keys, in tables with and without columns: zeros."""
+    k = torch.randn(3, 2, PAGE, dim, device="cuda").to(torch.bfloat16)
+    q = torch.randn(3, 8, dim, device="cuda").to(torch.bfloat16)
+    table = torch.zeros(3, width, dtype=torch.int32, device="cuda")
+    sl = torch.zeros(3, dtype=torch.int32, device="cuda")
+    assert (ops.paged_attn_decode(q, k, k, table, sl, 0.1) == 0).all()
+    for sink in (None, torch.zeros(8, device="cuda")):
+        out = torch.full((3, 8, dim), 7.0, device="cuda")
+        H.capped_attn(q.flatten(1), k, k, table, None, sl, 8, 0.1, 0.0, out,
+                      sink=sink)
+        assert (out == 0).all()
+
+
 OPTIONS = {
     "plain": {},
     "window": dict(window=50),

@@ -177,10 +177,12 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
   // ids of 32 of the wave's tiles from the tb-th on, two lanes a tile
   int tb = 0;
   // (read without waiting for the length: what lies past the last page is not
-  // used)
+  // used; a table without columns has no entry to read)
   auto pages_from = [&](int n) {
-    return btab[min(2 * list.at(i0 + (n + (lane >> 1)) * step) + (lane & 1),
-                    max_blocks - 1)];
+    return max_blocks <= 0
+        ? 0
+        : btab[min(2 * list.at(i0 + (n + (lane >> 1)) * step) + (lane & 1),
+                   max_blocks - 1)];
   };
   auto load = [&](int t, int n, int pages, bool val) {
     const char* cache = reinterpret_cast<const char*>(val ? v_cache : k_cache);

@@ -194,6 +194,40 @@ def test_decode_edges(dim, keys, kv_heads, per):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("odd", ["caches", "rows", "all"])
+@pytest.mark.parametrize("decode", [True, False])
+def test_any_alignment(dim, odd, decode):
+    """Caches, queries and results at odd addresses (2 B) and row strides."""
+    lens, ctx = ([1, 1], [70, 3000]) if decode else ([5, 20], [2100, 40])
+    heads, scale = 8, dim ** -0.5
+    rows, k, v, table = make(lens, ctx, 2, 4, dim, dim)
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0))).int().cuda()
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)]).int().cuda()
+
+    def shifted(t, on):
+        if not on:
+            return t.cuda()
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        flat[1:].copy_(t.flatten())
+        return flat[1:].view(t.shape)
+    kd, vd = (shifted(t, odd != "rows") for t in (k, v))
+    extra = odd != "caches"
+    wide = torch.full((sum(lens), heads * dim + extra), 7.0,
+                      dtype=torch.bfloat16, device="cuda")
+    qd = wide.clone()[:, extra:].unflatten(-1, (heads, dim)).copy_(q)
+    out = wide[:, extra:].unflatten(-1, (heads, dim))
+    if decode:
+        got = ops.paged_attn_decode(qd, kd, vd, table.cuda(), sl, scale,
+                                    out=out)
+    else:
+        got = ops.paged_attn_prefill(qd, kd, vd, table.cuda(), cu, sl, scale,
+                                     out=out)
+    check(got, *want(q, k, v, table, lens, ctx, scale))
+    assert (wide[:, :extra] == 7.0).all()
+
+
 def test_decode_standout_scores():
     rows, k, v, table = make([1, 1], [900, 350], 1, 2, 128, 5)
     k[table[0, 4], 0, 3] *= 30.0

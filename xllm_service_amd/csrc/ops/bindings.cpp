@@ -40,7 +40,7 @@ void launch_gather_blocks(unsigned short*, unsigned short*, const long*, int,
 void launch_paged_attn_decode(unsigned short*, const unsigned short*,
                               const unsigned short*, const unsigned short*,
                               const int*, const int*, float*, float*, float,
-                              int, int, int, int, int, long, long,
+                              int, int, int, int, int, long, long, bool,
                               hipStream_t);
 int paged_attn_decode_parts(int, int, int);
 int paged_attn_prefill_parts(long, int, int, int, int, int);
@@ -95,6 +95,11 @@ inline unsigned short* u16(torch::Tensor& t) {
 }
 inline const unsigned short* u16c(const torch::Tensor& t) {
   return reinterpret_cast<const unsigned short*>(t.data_ptr());
+}
+// every row starts at a multiple of n bytes
+inline bool on_bytes(const torch::Tensor& t, int n) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % n == 0 &&
+         (t.size(0) <= 1 || t.stride(0) * 2 % n == 0);
 }
 inline hipStream_t cur_stream() {
   return at::hip::getCurrentHIPStream().stream();
@@ -232,7 +237,10 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   int parts = 1;
   torch::Tensor ws;            // [seqs * heads][parts][D + 2], fp32
   float *ws_o = nullptr, *ws_ml = nullptr;
-  if (D == 128 || D == 64) {
+  const bool stream = (D == 128 || D == 64) && on_bytes(k_cache, 16) &&
+                      on_bytes(v_cache, 16) && on_bytes(q, 16) &&
+                      on_bytes(out, 8);
+  if (stream) {
     parts = xllm::paged_attn_decode_parts(num_seqs, n_kv,
                                           block_tables.size(1));
     if (parts > 1) {
@@ -246,7 +254,7 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
       u16(out), u16c(q), u16c(k_cache), u16c(v_cache),
       block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(), ws_ml, ws_o,
       (float)scale, num_seqs, n_qheads, n_kv, D, block_tables.size(1),
-      q.stride(0), out.stride(0), cur_stream());
+      q.stride(0), out.stride(0), stream, cur_stream());
 }
 
 void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
@@ -269,6 +277,17 @@ void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
               n_qheads % n_kv == 0 && out.sizes() == q.sizes() &&
               seq_lens.size(0) >= n_seqs && block_tables.size(0) >= n_seqs,
               "prefill kernel: shapes do not match");
+  // the kernel moves caches and queries by 16 B and results by 8 B: copies of
+  // what lies at other addresses
+  if (!on_bytes(out, 8)) {
+    auto rows = out.clone(at::MemoryFormat::Contiguous);
+    paged_attn_prefill(rows, q, k_cache, v_cache, block_tables, cu_q, seq_lens,
+                       scale);
+    out.copy_(rows);
+    return;
+  }
+  for (auto* t : {&q, &k_cache, &v_cache})
+    if (!on_bytes(*t, 16)) *t = t->clone(at::MemoryFormat::Contiguous);
   const int n_part = xllm::paged_attn_prefill_parts(
       tokens, n_seqs, n_qheads / n_kv, n_kv, D, block_tables.size(1));
   torch::Tensor ws;            // [tokens * heads][parts][D + 2], fp32

@@ -7,6 +7,13 @@
 namespace xllm {
 
 // ---------------- other head widths: shuffle-reduce design -------------------
+// (and 64- and 128-wide heads at addresses that are not multiples of 16 B, which
+// loads straight to LDS ask for)
+XLLM_DEV ushort8_t pa_eight(const unsigned short* p) {   // any alignment
+  ushort8_t v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
 template <int G>
 __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
     unsigned short* __restrict__ out, const unsigned short* __restrict__ q,
@@ -31,7 +38,7 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
   for (int g = 0; g < G; g++) {
     const long qoff = (long)seq * q_stride + (long)(kvh * G + g) * D + 8 * d8;
     if (dvalid) {
-      ushort8_t v = *reinterpret_cast<const ushort8_t*>(q + qoff);
+      ushort8_t v = pa_eight(q + qoff);
 #pragma unroll
       for (int j = 0; j < 8; j++) qf[g][j] = bf16_to_f32(v.x[j]);
     } else {
@@ -58,8 +65,8 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
       const long roff = base + (long)t * D + 8 * d8;
       float kf[8], vf[8];
       if (dvalid) {
-        ushort8_t k8 = *reinterpret_cast<const ushort8_t*>(k_cache + roff);
-        ushort8_t v8 = *reinterpret_cast<const ushort8_t*>(v_cache + roff);
+        ushort8_t k8 = pa_eight(k_cache + roff);
+        ushort8_t v8 = pa_eight(v_cache + roff);
 #pragma unroll
         for (int u = 0; u < 8; u++) { kf[u] = bf16_to_f32(k8.x[u]); vf[u] = bf16_to_f32(v8.x[u]); }
       } else {
@@ -123,7 +130,8 @@ int paged_attn_decode_parts(int num_seqs, int n_kv_heads, int max_blocks) {
   return paged_stream_split(num_seqs, n_kv_heads, max_blocks).parts;
 }
 
-// ws_o, ws_ml: room for paged_attn_decode_parts() results per row
+// streamed: rows of q and the caches on 16 B, of out on 8 B, and heads 64 or 128
+// wide; ws_o, ws_ml: room for paged_attn_decode_parts() results per row
 void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
                               const unsigned short* k_cache,
                               const unsigned short* v_cache,
@@ -131,10 +139,11 @@ void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
                               float* ws_ml, float* ws_o, float scale,
                               int num_seqs, int n_qheads, int n_kv_heads, int D,
                               int max_blocks_per_seq, long q_stride,
-                              long out_stride, hipStream_t stream) {
+                              long out_stride, bool streamed,
+                              hipStream_t stream) {
   const int G = n_qheads / n_kv_heads;
   if (num_seqs == 0) return;
-  if (D != 128 && D != 64) {
+  if (!streamed) {
     const dim3 grid(num_seqs * n_kv_heads), block(256);
 #define PA_SMALL(GV)                                                           \
   hipLaunchKernelGGL((paged_attn_decode_small_kernel<GV>), grid, block, 0,     \

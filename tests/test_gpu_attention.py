@@ -194,6 +194,27 @@ def test_decode_edges(dim, keys, kv_heads, per):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("ctx", [[3, 0], [2600, 900]])      # whole; in parts
+@pytest.mark.parametrize("flat", [False, True])
+def test_prefill_shapes_of_results(ctx, flat):
+    """Results as rows of heads * dim, with more rows than there are queries;
+    caches of different sizes."""
+    lens, heads, dim = [5, 9], 4, 128
+    rows, k, v, table = make(lens, ctx, 1, heads, dim, 22)
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim)).contiguous()
+    cu = torch.tensor([0, 5, 14], dtype=torch.int32)
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)], dtype=torch.int32)
+    more = torch.cat([v, v[:2]])
+    out = torch.full((20, heads * dim), 7.0, dtype=torch.bfloat16,
+                     device="cuda")
+    ops.paged_attn_prefill(
+        *(t.cuda() for t in (q, k, more, table, cu, sl)), 0.1,
+        out=out if flat else out.unflatten(-1, (heads, dim)))
+    check(out[:14].unflatten(-1, (heads, dim)),
+          *want(q, k, v, table, lens, ctx, 0.1))
+    assert (out[14:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("odd", ["caches", "rows", "all"])
 @pytest.mark.parametrize("decode", [True, False])

@@ -273,8 +273,14 @@ void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
   const int n_seqs = cu_q.size(0) - 1;
   TORCH_CHECK(D == 128 || D == 64, "prefill kernel: head_dim 64 or 128");
   TORCH_CHECK(k_cache.size(2) == 16, "block_size must be 16");
-  TORCH_CHECK(k_cache.size(3) == D && v_cache.sizes() == k_cache.sizes() &&
-              n_qheads % n_kv == 0 && out.sizes() == q.sizes() &&
+  // out: [tokens, heads, D] or [tokens, heads * D]; q and out may have rows
+  // beyond the last prompt's, either cache pages that no table names
+  const long row = (long)n_qheads * D;
+  TORCH_CHECK(k_cache.size(3) == D &&
+              v_cache.sizes().slice(1) == k_cache.sizes().slice(1) &&
+              n_qheads % n_kv == 0 &&
+              (out.dim() == 3 ? out.size(1) * out.size(2)
+                              : out.size(1)) == row &&
               seq_lens.size(0) >= n_seqs && block_tables.size(0) >= n_seqs,
               "prefill kernel: shapes do not match");
   // the kernel moves caches and queries by 16 B and results by 8 B: copies of

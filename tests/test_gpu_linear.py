@@ -73,3 +73,19 @@ def test_transforms_go_to_the_library():
     with Count():
         ops.linear(x, w)
     assert Count.calls > 0
+
+
+def test_bias_that_overrides_the_call():
+    """A bias of a class with __torch_function__ is asked, like x and weight."""
+    calls = []
+
+    class Seen(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            calls.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+    x, w = (torch.randn(r, 128, device="cuda").to(torch.bfloat16)
+            for r in (6, 64))
+    b = torch.randn(64, device="cuda").to(torch.bfloat16).as_subclass(Seen)
+    assert isinstance(ops.linear(x, w, b), Seen)
+    assert torch.nn.functional.linear in calls

@@ -362,9 +362,10 @@ torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor b,
   return c;
 }
 
-// plain memory, no transform, mode or trace that has to see the call
+// plain memory without a transform or a tangent
 static bool plain(const torch::Tensor& t) {
-  return !t.key_set().has_any(c10::DispatchKeySet(
+  return t.layout() == torch::kStrided && !t.is_nested() &&
+         !t.key_set().has_any(c10::DispatchKeySet(
              {c10::DispatchKey::FuncTorchBatched,
               c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
               c10::DispatchKey::Functionalize, c10::DispatchKey::ZeroTensor,
@@ -372,28 +373,35 @@ static bool plain(const torch::Tensor& t) {
          !t._fw_grad(0).defined();
 }
 
+// Whether a call may go past torch's dispatcher: no gradient is wanted, and no
+// transform, mode, trace or autocast has to see it
+bool direct(const std::vector<torch::Tensor>& tensors) {
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+      torch::jit::tracer::isTracing() ||
+      at::autocast::is_autocast_enabled(at::kCUDA))
+    return false;
+  const bool grad = at::GradMode::is_enabled();
+  for (const auto& t : tensors)
+    if (!plain(t) || (grad && t.requires_grad())) return false;
+  return true;
+}
+
 // x [..., K] @ w [N, K]^T (+ bias): the kernels of linear.hip where they take the
 // call, the library elsewhere (and wherever a gradient is wanted)
 torch::Tensor linear(torch::Tensor x, torch::Tensor w,
                      c10::optional<torch::Tensor> bias) {
   auto rows16 = [](const torch::Tensor& t) {
-    return plain(t) && t.dim() == 2 && t.is_cuda() &&
-           t.dtype() == torch::kBFloat16 && t.stride(1) == 1 &&
+    return t.dim() == 2 && t.is_cuda() && t.dtype() == torch::kBFloat16 &&
+           t.stride(1) == 1 &&
            reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  const bool grad =
-      at::GradMode::is_enabled() &&
-      (x.requires_grad() || w.requires_grad() ||
-       (bias.has_value() && bias->requires_grad()));
-  const bool seen = c10::impl::TorchDispatchModeTLS::any_modes_set() ||
-                    torch::jit::tracer::isTracing() ||
-                    at::autocast::is_autocast_enabled(at::kCUDA);
-  if (!grad && !seen && rows16(x) && rows16(w) && x.size(1) == w.size(1) &&
+  if ((bias.has_value() ? direct({x, w, *bias}) : direct({x, w})) &&
+      rows16(x) && rows16(w) && x.size(1) == w.size(1) &&
       x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) &&
       x.stride(0) < (1L << 24) && w.is_contiguous() &&
       x.device() == w.device() &&
       (!bias.has_value() ||
-       (plain(*bias) && bias->dim() == 1 && bias->is_contiguous() &&
+       (bias->dim() == 1 && bias->is_contiguous() &&
         bias->dtype() == torch::kBFloat16 && bias->size(0) == w.size(0) &&
         bias->device() == w.device()))) {
     const long M = x.size(0), N = w.size(0), K = w.size(1);
@@ -630,6 +638,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma_gemm", &mfma_gemm);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("linear", &linear);
+  m.def("direct", &direct);
   m.def("packed_gemm", &packed_gemm);
   m.def("packed_gemm_probe", &packed_gemm_probe);
   m.def("migrate_blocks_peer", &migrate_blocks_peer);

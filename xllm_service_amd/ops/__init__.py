@@ -229,7 +229,7 @@ def linear(x, weight, bias=None):
     """x @ weight.T (+ bias). On a GPU the bf16 shapes of serving steps run on
     the kernels of csrc/ops/linear.hip, the others on the library."""
     if x.is_cuda and HAS_EXT and not torch.overrides.has_torch_function(
-            (x, weight)):
+            (x, weight, bias)):
         return _ops.linear(x, weight, bias)
     return torch.nn.functional.linear(x, weight, bias)
 

@@ -194,6 +194,24 @@ def test_decode_edges(dim, keys, kv_heads, per):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+def test_narrow_prefill_has_gradients():
+    """64-wide prompt rows: wanted gradients come from torch's operations."""
+    lens, ctx, heads, dim = [5, 9], [3, 20], 4, 64
+    rows, k, v, table = make(lens, ctx, 2, 2, dim, 23)
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim)).contiguous()
+    cu = torch.tensor([0, 5, 14], dtype=torch.int32, device="cuda")
+    sl = torch.tensor([8, 29], dtype=torch.int32, device="cuda")
+    qd, kd, vd = (t.cuda().requires_grad_(True) for t in (q, k, v))
+    out = ops.paged_attn_prefill(qd, kd, vd, table.cuda(), cu, sl, 0.1)
+    assert out.requires_grad
+    out.float().sum().backward()
+    for t in (qd, kd, vd):
+        assert t.grad is not None and (t.grad != 0).any()
+    with torch.no_grad():
+        got = ops.paged_attn_prefill(qd, kd, vd, table.cuda(), cu, sl, 0.1)
+    check(got, *want(q, k, v, table, lens, ctx, 0.1))
+
+
 @pytest.mark.parametrize("ctx", [[3, 0], [2600, 900]])      # whole; in parts
 @pytest.mark.parametrize("flat", [False, True])
 def test_prefill_shapes_of_results(ctx, flat):

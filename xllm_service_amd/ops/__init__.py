@@ -137,10 +137,14 @@ def paged_attn_decode(q, k_cache, v_cache, block_tables, seq_lens, scale,
 def _prefill_native(q, k_cache, v_cache, block_tables, cu_q, seq_lens, out):
     """Whether the MFMA prefill kernel takes this call. 128-wide heads always
     do (what it cannot take raises there); 64-wide ones where layout, types and
-    alignment are the kernel's."""
+    alignment are the kernel's and nothing asks for torch's own operations
+    (gradients, transforms, modes, autocast)."""
     D = k_cache.shape[-1]
     if D != 64:
         return D == 128
+    if torch.overrides.has_torch_function((q, k_cache, v_cache)) or \
+            not _ops.direct([q, k_cache, v_cache]):
+        return False
     heads = [q] if out is None else [q, out]
     return (all(t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous()
                 and t.data_ptr() % 16 == 0 for t in (k_cache, v_cache))

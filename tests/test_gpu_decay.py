@@ -116,3 +116,36 @@ def test_sequences_without_new_tokens(long):
     assert (state[2] == 0).all()
     for slot in (1, 3):
         assert torch.equal(state[slot], alone[slot])
+
+
+def test_every_activation():
+    """silu of every bf16 number below 2^100, read off as values of one-token
+    sequences whose query and key meet in 2^24: those of a division, within one
+    rounding to bf16, and zero where e^-x is infinite in 32 bits."""
+    x = torch.arange(-2 ** 15, 2 ** 15).to(torch.int16).view(torch.bfloat16)
+    x = torch.where(torch.isfinite(x) & (x.abs() < 2.0 ** 100), x,
+                    torch.zeros_like(x))
+    n, V = 512, 128
+    q = torch.zeros(n, 64, dtype=torch.bfloat16)
+    q[:, 0] = 4096.0                                 # its own activation
+    i32 = dict(dtype=torch.int32, device="cuda")
+    out = torch.zeros(n, 1, V, device="cuda")
+    H.decay_attn(q.cuda(), q.cuda(), x.view(n, V).cuda(),
+                 torch.ones(1, device="cuda"),
+                 torch.zeros(1, 1, 64, V, device="cuda"),
+                 torch.full((n,), -1, **i32), torch.arange(n + 1, **i32),
+                 torch.zeros(n, **i32), out, max_q_len=1)
+    plain = torch.zeros_like(out)                    # decoded rows: a division
+    H.decay_attn(q.cuda(), q.cuda(), x.view(n, V).cuda(),
+                 torch.ones(1, device="cuda"),
+                 torch.zeros(1, 1, 64, V, device="cuda"),
+                 torch.full((n,), -1, **i32), None, torch.zeros(n, **i32),
+                 plain)
+    assert torch.equal(out, plain)
+    got = out.cpu().double().flatten() / 2.0 ** 24
+    x = x.double()
+    want = torch.where(x < -88.7, 0.0, x * torch.sigmoid(x))
+    tiny = want.abs() < 2.0 ** -126                  # not normal
+    off = (got - want).abs()
+    assert (off[~tiny] <= 2.0 ** -8 * want[~tiny].abs()).all()
+    assert (off[tiny] <= 2.0 ** -126).all()

@@ -57,16 +57,18 @@ struct alignas(16) dm_u4 { unsigned x[4]; };
 
 // 8 neighbouring activations, packed. x / (1 + e^-x) with v_rcp and one Newton
 // step in place of a division: half its instructions, and the same bf16 for
-// every bf16 input (but for the three next to -87.5, whose 1e-36 becomes zero).
+// every bf16 input. The denominator is 2^-24 of itself: the reciprocal of 1e38
+// would be below what v_rcp returns.
 XLLM_DEV dm_u4 dm_act(const unsigned short* p) {
+  constexpr float s = 0x1p-24f;
   const ushort8_t x = *reinterpret_cast<const ushort8_t*>(p);
   float v[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float z = bf16_to_f32(x.x[j]);
-    const float d = fminf(1.0f + __expf(-z), 3e38f);
+    const float d = fmaf(__expf(-z), s, s);       // infinite below -88.7: r = 0
     const float r = __builtin_amdgcn_rcpf(d);
-    v[j] = z * fmaf(fmaf(-d, r, 1.0f), r, r);
+    v[j] = z * (s * fmaf(fmaf(-fminf(d, 3e38f), r, 1.0f), r, r));
   }
   dm_u4 y;
 #pragma unroll

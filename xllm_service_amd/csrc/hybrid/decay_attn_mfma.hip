@@ -230,7 +230,11 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
           bf16x8, dm_act(P.q + (long)(t0 + qi) * P.q_stride + hd * D + ks * 16 +
                          h * 8));
   }
-  f32x16 acc[2][VT];                              // apart as above
+  // Apart as above, and the leading products of four steps (of two within the
+  // chunk) are summed before they meet the large sum, which then is rounded 6
+  // times instead of 16. Error against 64 bits, 3 prompts of 853-1657 tokens:
+  // 8.2e-8 -> 6.7e-8 (the recurrence: 7.1e-8), for 3 us of 71.
+  f32x16 acc[2][VT];
 #pragma unroll
   for (int j = 0; j < VT; ++j) acc[0][j] = acc[1][j] = mr_zero();
   const int vbase = mr_col_base<V>(lane);
@@ -257,15 +261,20 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
       __syncthreads();
       if (!on) continue;
 #pragma unroll
-      for (int st = 0; st < 4; ++st)
+      for (int j = 0; j < VT; ++j) {
+        f32x16 z = mr_zero();
 #pragma unroll
-        for (int t = 0; t < 3; ++t)
+        for (int st = 0; st < 4; ++st)
 #pragma unroll
-          for (int j = 0; j < VT; ++j)
-            acc[t > 0][j] =
-                mr_mma(mr_cols<V>((const lds_u16*)lds + t * 64 * V +
-                                  (vbase ^ (j << 5)) + st * 16 * V),
-                       qf[d0 / 16 + st], acc[t > 0][j]);
+          for (int t = 0; t < 3; ++t) {
+            const bf16x8 x =
+                mr_cols<V>((const lds_u16*)lds + t * 64 * V +
+                           (vbase ^ (j << 5)) + st * 16 * V);
+            if (t == 0) z = mr_mma(x, qf[d0 / 16 + st], z);
+            else acc[1][j] = mr_mma(x, qf[d0 / 16 + st], acc[1][j]);
+          }
+        acc[0][j] += z;
+      }
     }
     __syncthreads();                              // also: pw is there
     const float fade = pw[min(qi, DM_C - 1) + 1];
@@ -323,15 +332,18 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
       }
     }
 #pragma unroll
-    for (int st = 0; st < 2; ++st)
+    for (int j = 0; j < VT; ++j) {
+      f32x16 y = mr_zero();
 #pragma unroll
-      for (int j = 0; j < VT; ++j) {
+      for (int st = 0; st < 2; ++st) {
         const bf16x8 x = mr_cols<V>((const lds_u16*)vs + (vbase ^ (j << 5)) +
                                     (kt * 32 + st * 16) * V);
+        y = mr_mma(x, p[0][st], y);
 #pragma unroll
-        for (int t = 0; t < 3; ++t)
-          acc[t > 0][j] = mr_mma(x, p[t][st], acc[t > 0][j]);
+        for (int t = 1; t < 3; ++t) acc[1][j] = mr_mma(x, p[t][st], acc[1][j]);
       }
+      acc[0][j] += y;
+    }
   }
   if (qi >= len) return;
   float* o = P.out + ((long)(t0 + qi) * P.heads + hd) * V + 4 * h;

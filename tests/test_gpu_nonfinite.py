@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from test_gpu_attention import make, want
+from test_gpu_decay import features, recur
 from xllm_service_amd import ops
 from xllm_service_amd.ops import hybrid as H
 
@@ -147,3 +148,31 @@ def test_nan_factors(decode, how):
         H.latent_attn(torch.ones_like(out, dtype=torch.bfloat16), latent,
                       dev[2], None, sl, math.nan, 512, out)
         assert torch.isnan(out).all()
+
+
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("T,at", [(100, 0), (100, 15), (100, 37),  # one chunk
+                                  (300, 0), (300, 37), (300, 127), (300, 200)])
+def test_decayed(T, at, where, bad):
+    """One entry of one token: the tokens before it do not see it, and the state
+    is lost where 64-bit arithmetic loses it."""
+    g = torch.Generator().manual_seed(T + at)
+    heads, D, V = 2, 64, 128
+    a = torch.tensor([0.9, 0.99])
+    x = torch.randn(T, heads * (2 * D + V), generator=g).to(torch.bfloat16)
+    cut = (0, heads * D, 2 * heads * D, x.shape[1])
+    x[at, cut["qkv".index(where)] + D + 5] = bad         # second head
+    x, f = features(x)
+    ref, after = recur(*(f[:, b:e].reshape(T, heads, -1)
+                         for b, e in zip(cut, cut[1:])), a.double(),
+                       torch.zeros(heads, D, V, dtype=torch.float64))
+    i32 = dict(dtype=torch.int32, device="cuda")
+    state = torch.zeros(1, heads, D, V, device="cuda")
+    out = torch.zeros(T, heads, V, device="cuda")
+    xd = x.cuda()
+    H.decay_attn(*(xd[:, b:e] for b, e in zip(cut, cut[1:])), a.cuda(), state,
+                 torch.zeros(1, **i32), torch.tensor([0, T], **i32),
+                 torch.zeros(1, **i32), out, max_q_len=T)
+    agree(out, ref)
+    agree(state[0], after)

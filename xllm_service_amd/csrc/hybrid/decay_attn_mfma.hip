@@ -75,6 +75,10 @@ XLLM_DEV dm_u4 dm_act(const unsigned short* p) {
   for (int j = 0; j < 4; ++j) y.x[j] = pack_bf16(v[2 * j], v[2 * j + 1]);
   return y;
 }
+// not zero where one of the two bf16 numbers is infinite or NaN
+XLLM_DEV unsigned dm_odd(unsigned u) {
+  return ((u & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
+}
 // v's three bf16 terms to the images at dst, dst + step, dst + 2 step
 XLLM_DEV void dm_split(float v[8], unsigned short* dst, int step) {
 #pragma unroll
@@ -212,6 +216,7 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
   __shared__ __attribute__((aligned(1024))) unsigned short
       lds[KV > SI ? KV : SI];
   __shared__ float pw[DM_C + 1];
+  __shared__ int lost[V];      // first token with a non-finite value, if any has
   int s, c, t0, len;
   if (!dm_locate(P, &s, &c, &t0, &len)) return;
   const int hd = blockIdx.y;
@@ -298,14 +303,32 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
     *reinterpret_cast<dm_u4*>(ks_ + r * D + ((ch ^ mr_swz_rows<D>(r)) << 3)) =
         y;
   }
+  unsigned odd = 0u;
 #pragma unroll 4
   for (int i = 0; i < DM_C * (V / 8) / 256; ++i) {
     const int idx = tid + i * 256, r = idx / (V / 8), ch = idx % (V / 8);
     dm_u4 y = {{0u, 0u, 0u, 0u}};
     if (r < len) y = dm_act(P.v + (long)(t0 + r) * P.v_stride + hd * V + ch * 8);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) odd |= dm_odd(y.x[j]);
     *reinterpret_cast<dm_u4*>(vs + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3)) = y;
   }
-  __syncthreads();
+  // A weight of zero keeps a key out of a row unless its value is not finite: the
+  // products see zero instead, and rows from that token on are NaN at the end.
+  const bool any_lost = __syncthreads_or(odd != 0u);
+  if (any_lost) {
+    for (int i = tid; i < V; i += 256) lost[i] = DM_C;
+    __syncthreads();
+    for (int i = tid; i < DM_C * V; i += 256) {
+      const int r = i / V, e = i % V;
+      unsigned short* x = vs + r * V + (((e >> 3) ^ mr_swz_cols<V>(r)) << 3) +
+                          (e & 7);
+      if (dm_odd(*x) == 0u) continue;
+      *x = 0;
+      atomicMin(lost + e, r);
+    }
+    __syncthreads();
+  }
   if (!on) return;
   const int kbase = mr_row_base<D>(lane);
   for (int kt = 0; kt <= w; ++kt) {
@@ -346,6 +369,14 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
     }
   }
   if (qi >= len) return;
+  if (any_lost) {
+#pragma unroll
+    for (int j = 0; j < VT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (lost[j * 32 + 8 * (r >> 2) + 4 * h + (r & 3)] <= qi)
+          acc[0][j][r] = NAN;
+  }
   float* o = P.out + ((long)(t0 + qi) * P.heads + hd) * V + 4 * h;
 #pragma unroll
   for (int j = 0; j < VT; ++j)

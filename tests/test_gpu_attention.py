@@ -267,6 +267,25 @@ def test_any_alignment(dim, odd, decode):
     assert (wide[:, :extra] == 7.0).all()
 
 
+@pytest.mark.parametrize("keys,per", [
+    ([777], 4), ([200], 8), ([5001], 1), ([600 + 33 * i for i in range(24)], 4),
+    ([40 + 70 * i for i in range(70)], 7)])
+def test_decode_weights(keys, per):
+    """The softmax weights of 128-wide heads have 16 bits: what the results are
+    off by is their rounding to bf16 (half a step of 2^-7 of their power of two),
+    and 2^-15 of the weighted sum of |v| for the weights and 32-bit sums."""
+    ctx = [n - 1 for n in keys]
+    rows, k, v, table = make([1] * len(keys), ctx, 4, per, 128, sum(keys))
+    q = rows[:, :512 * per].unflatten(-1, (4 * per, 128))
+    got = ops.paged_attn_decode(
+        q.cuda(), k.cuda(), v.cuda(), table.cuda(),
+        torch.tensor(keys, dtype=torch.int32, device="cuda"), 0.13)
+    ref, big = want(q, k, v, table, [1] * len(keys), ctx, 0.13)
+    over = (got.double().cpu() - ref).abs() - 2.0 ** -15 * big \
+        - 2.0 ** (torch.floor(torch.log2(ref.abs())) - 8)
+    assert over.max() <= 0, f"over by {over.max():.3g}"
+
+
 def test_decode_standout_scores():
     rows, k, v, table = make([1, 1], [900, 350], 1, 2, 128, 5)
     k[table[0, 4], 0, 3] *= 30.0

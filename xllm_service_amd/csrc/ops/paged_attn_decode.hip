@@ -164,8 +164,9 @@ void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
 #undef PA_SMALL
     return;
   }
-  // 64-wide heads have 32-bit weights, as every other width but 128
-  auto go = D == 128 ? paged_stream<128, 1, false> : paged_stream<64, 3, false>;
+  // 64-wide heads have 32-bit weights, as every other width but 128, whose
+  // weights have 16 (G is at most 8)
+  auto go = D == 128 ? paged_stream<128, 2, false> : paged_stream<64, 3, false>;
   go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, seq_lens, num_seqs,
      scale, n_qheads, n_kv_heads, max_blocks_per_seq, q_stride, out_stride,
      paged_stream_split(num_seqs, n_kv_heads, max_blocks_per_seq), PagedMore{},

@@ -100,8 +100,16 @@ XLLM_DEV void pa_rows(const unsigned (&at)[D / 16], bf16x8 (&k)[D / 16]) {
         : "memory");
 }
 
-// TERMS: bf16 terms a softmax weight is split into (1: rounded; 3: all of its
-// 32 bits). MORE: the options of PagedMore.
+// TERMS: bf16 terms a softmax weight is split into (2: its upper 16 bits of
+// mantissa; 3: all of them). MORE: the options of PagedMore.
+//   Two terms cost no product of their own: columns 16 and up are padding where
+// at most 8 heads share a key head. They hold the queries of columns 0 to 15
+// again, and their lanes, which make the same weights, keep the second terms.
+// With one rounded term the results' error depended on how many weights were the
+// largest of their wave, and so exact: 24 x 0.6-1.4 k keys 0.00192 of the result,
+// by 32 waves a row 0.00186; with two 0.00166, which is the rounding to bf16. Us,
+// one term | two by a product of their own | here: 1 x 776 keys 9.0 | 9.6 | 9.5,
+// 24 x 0.6-1.4 k 18.9 | 19.6 | 19.1, 128 x 1-2 k 142.5 | 142.8 | 142.0.
 template <int D, int TERMS, bool MORE>
 __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
     void* __restrict__ out,                  // [S, n_qheads, D]
@@ -116,6 +124,8 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
     const long q_stride, const long out_stride, const int P, const int per,
     const PagedMore x) {
   constexpr int NW = PA_NW, KS = D / 16, DT = D / 32;
+  constexpr bool FOLD = TERMS == 2;          // G <= 8
+  constexpr int NP = FOLD ? 1 : TERMS;       // products per weight
   constexpr int CPR = D / 8;                 // 16 B chunks of a row
   constexpr int RPI = 64 / CPR;              // rows one load instruction fills
   constexpr int NI = PA_KT / RPI;            // ... instructions per tile
@@ -141,8 +151,11 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
   const int step = parts * NW, i0 = part * NW + wid;
   const int lo = paged_first<MORE>(x, seq_len);   // first key in the window
 
-  const bool row_ok = c32 < G;
-  const int head = kvh * G + c32;
+  const int col = FOLD ? c32 & 15 : c32;
+  const bool second = FOLD && c32 >= 16;     // second terms of column col
+  const unsigned first = second ? 0xffff0000u : 0u;   // what the others keep
+  const bool row_ok = col < G;
+  const int head = kvh * G + col;
   const PagedScore sc = paged_score<MORE>(x, scale, row_ok ? head : kvh * G);
   // padding columns hold the first head's query: their results go nowhere
   bf16x8 qf[KS];
@@ -282,17 +295,25 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
         for (int r = 0; r < 16; r++) o_acc[j][r] *= alpha;
     }
     const float mc = m == -INFINITY ? 0.0f : m * c;
-    bf16x8 p[TERMS][2];
+    bf16x8 p[NP][2];
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
       float a = __builtin_amdgcn_exp2f(fmaf(s[0][r], c, -mc));
       float b = __builtin_amdgcn_exp2f(fmaf(s[0][r + 1], c, -mc));
       l += a + b;
 #pragma unroll
-      for (int e = 0; e < TERMS; e++) {
-        const unsigned u = pack_bf16(a, b);
+      for (int e = 0; e < NP; e++) {
+        unsigned u;
+        if constexpr (FOLD) {
+          a -= __uint_as_float(__float_as_uint(a) & first);
+          b -= __uint_as_float(__float_as_uint(b) & first);
+          u = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a),
+                                    0x07060302u);
+        } else {
+          u = pack_bf16(a, b);
+          drop_bf16(a, b, u);
+        }
         reinterpret_cast<unsigned*>(&p[e][r >> 3])[(r & 7) >> 1] = u;
-        drop_bf16(a, b, u);
       }
     }
     if (more) wait_older();                    // V of this tile is there
@@ -302,13 +323,13 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
 #pragma unroll
     for (int j = 0; j < DT; j++)
 #pragma unroll
-      for (int e = 0; e < TERMS; e++)
+      for (int e = 0; e < NP; e++)
         o_acc[j] = mr_mma(v[j], p[e][0], o_acc[j]);
     pa_cols<D, 32 * D>(vat, v);
 #pragma unroll
     for (int j = 0; j < DT; j++)
 #pragma unroll
-      for (int e = 0; e < TERMS; e++)
+      for (int e = 0; e < NP; e++)
         o_acc[j] = mr_mma(v[j], p[e][1], o_acc[j]);
     if (more) load(list.at(i + step), n + 1, ids, true);
     pages = ids;
@@ -317,24 +338,26 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
 
   // ---- the waves' results meet in LDS ----------------------------------------
   __syncthreads();
-  float* mo = reinterpret_cast<float*>(kv_lds);          // [NW][G][D]
+  const int R = FOLD ? 2 * G : G;                        // second terms apart
+  constexpr int DP = FOLD ? D + 4 : D;                   // rows on other banks
+  float* mo = reinterpret_cast<float*>(kv_lds);          // [NW][R][DP]
   if (row_ok) {
-    if (h == 0) {
-      ml_lds[wid][c32][0] = m == -INFINITY ? m : m * sc.c;
-      ml_lds[wid][c32][1] = l;
+    if (h == 0 && !second) {
+      ml_lds[wid][col][0] = m == -INFINITY ? m : m * sc.c;
+      ml_lds[wid][col][1] = l;
     }
+    float* mine = mo + (wid * R + (second ? G : 0) + col) * DP + 4 * h;
 #pragma unroll
     for (int i = 0; i < DT; i++)
 #pragma unroll
       for (int r = 0; r < 16; r += 4)
-        *reinterpret_cast<float4*>(mo + (wid * G + c32) * D + i * 32 + 2 * r +
-                                   4 * h) =
+        *reinterpret_cast<float4*>(mine + i * 32 + 2 * r) =
             make_float4(o_acc[i][r], o_acc[i][r + 1], o_acc[i][r + 2],
                         o_acc[i][r + 3]);
   }
   __syncthreads();
   for (int idx = tid; idx < G * (D / 4); idx += NW * 64) {
-    const int row = idx / (D / 4), col = idx % (D / 4) * 4;
+    const int row = idx / (D / 4), at = idx % (D / 4) * 4;
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NW; w++) M = fmaxf(M, ml_lds[w][row][0]);
@@ -344,8 +367,12 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
     for (int w = 0; w < NW; w++) {
       const float f = __builtin_amdgcn_exp2f(ml_lds[w][row][0] - Mu);
       L += ml_lds[w][row][1] * f;
-      const float4 y =
-          *reinterpret_cast<const float4*>(mo + (w * G + row) * D + col);
+      const float* from = mo + (w * R + row) * DP + at;
+      float4 y = *reinterpret_cast<const float4*>(from);
+      if (FOLD) {
+        const float4 z = *reinterpret_cast<const float4*>(from + G * DP);
+        y.x += z.x; y.y += z.y; y.z += z.z; y.w += z.w;
+      }
       a[0] += y.x * f; a[1] += y.y * f; a[2] += y.z * f; a[3] += y.w * f;
     }
     if (parts == 1) {
@@ -354,15 +381,15 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
             x.sink[kvh * G + row] * 1.4426950408889634f - M);
       const float inv = L != 0.0f ? 1.0f / L : 0.0f;
       paged_put<MORE>(x, out, (long)seq * out_stride +
-                      (long)(kvh * G + row) * D + col,
+                      (long)(kvh * G + row) * D + at,
                       a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
     } else {
       const long slot = ((long)seq * n_kv * G + kvh * G + row) * P + part;
-      if (col == 0) {
+      if (at == 0) {
         ws_ml[slot * 2] = M;
         ws_ml[slot * 2 + 1] = L;
       }
-      *reinterpret_cast<float4*>(ws_o + slot * D + col) =
+      *reinterpret_cast<float4*>(ws_o + slot * D + at) =
           make_float4(a[0], a[1], a[2], a[3]);
     }
   }
@@ -407,8 +434,8 @@ inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
   return {(int)std::min<long>(8 / f, (tiles + 31) / 32), per};
 }
 
-// Decoded rows (at most 32 query heads per key head) and the merge of their
-// parts
+// Decoded rows (at most 32 query heads per key head, 8 with two terms) and the
+// merge of their parts
 template <int D, int TERMS, bool MORE>
 inline void paged_stream(void* out, float* ws_o, float* ws_ml,
                          const unsigned short* q, const unsigned short* k_cache,

@@ -134,7 +134,7 @@ def test_every_activation():
                  torch.ones(1, device="cuda"),
                  torch.zeros(1, 1, 64, V, device="cuda"),
                  torch.full((n,), -1, **i32), torch.arange(n + 1, **i32),
-                 torch.zeros(n, **i32), out, max_q_len=1)
+                 torch.zeros(n, **i32), out, max_q_len=128)   # not as short
     plain = torch.zeros_like(out)                    # decoded rows: a division
     H.decay_attn(q.cuda(), q.cuda(), x.view(n, V).cuda(),
                  torch.ones(1, device="cuda"),
@@ -175,3 +175,13 @@ def test_no_less_precise_than_the_recurrence():
         off.append([float((y.cpu().to(F64) - w).norm() / w.norm())
                     for y, w in ((out, want), (state[0], after))])
     assert off[0][0] <= off[1][0] and off[0][1] <= off[1][1], off
+
+
+@pytest.mark.parametrize("heads,D,V", [(1, 128, 128), (48, 64, 64),
+                                       (40, 128, 64), (20, 64, 128)])
+def test_short_batches(heads, D, V):
+    """Lengths on both sides of the line between the recurrence and the
+    matrix-pipe form, for few and for many states."""
+    for n in (1, 3, 9, 12, 13, 16, 17, 24, 25):
+        run(D, V, [n, max(1, n // 2), n], [0, 5, 3], [1, -1, 0],
+            [0.75 + 0.24 * h / heads for h in range(heads)], n, n)

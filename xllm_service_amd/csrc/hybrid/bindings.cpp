@@ -76,6 +76,7 @@ void launch_latent_attn_mfma(float*, float*, float*, const unsigned short*,
                              float, int, int, hipStream_t);
 long decay_attn_mfma_chunks(long, long);
 int decay_attn_mfma_chunk();
+bool decay_attn_short(long, long, int, int);
 void launch_decay_attn_mfma(float*, const unsigned short*,
                             const unsigned short*, const unsigned short*,
                             const float*, float*, const int*, const int*,
@@ -661,8 +662,8 @@ void decay_attn(Tensor out, Tensor q, Tensor k, Tensor v, Tensor decay,
   } else {
     TORCH_CHECK(n_seqs == T, "decode: one sequence per token");
   }
-  // prompt rows in bf16 with 64- or 128-wide heads: the matrix-pipe form,
-  // while its scratch stays under 2 GiB
+  // prompt rows in bf16 with 64- or 128-wide heads: the matrix-pipe form from a
+  // few tokens on, while its scratch stays under 2 GiB
   auto rows8 = [](const Tensor& t) {
     return t.stride(0) % 8 == 0 && t.stride(1) == 1 &&
            reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
@@ -676,7 +677,8 @@ void decay_attn(Tensor out, Tensor q, Tensor k, Tensor v, Tensor decay,
     const long longest = max_q_len > 0 ? std::min<long>(max_q_len, T) : T;
     const bool one = longest <= hy::decay_attn_mfma_chunk();
     const long n = hy::decay_attn_mfma_chunks(T, n_seqs) * H * D * Dv;
-    if (one || n * 4 <= (1L << 31)) {
+    if (!hy::decay_attn_short(longest, (long)n_seqs * H, D, Dv) &&
+        (one || n * 4 <= (1L << 31))) {
       Tensor ws;
       if (!one) ws = torch::empty({n}, state.options());
       hy::launch_decay_attn_mfma(

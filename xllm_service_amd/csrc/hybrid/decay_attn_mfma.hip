@@ -394,6 +394,23 @@ long decay_attn_mfma_chunks(long tokens, long n_seqs) {
 }
 int decay_attn_mfma_chunk() { return DM_C; }
 
+// Whether a batch is too short for this form: a sequence of a few tokens costs it
+// nearly as much as one of 32 (both passes move the whole state through LDS), where
+// the recurrence of decay_attn.hip walks token by token, one workgroup per 16
+// columns of a state, whose rate falls once they fill the chip. Measured (us, the
+// recurrence | here), 128 x 128, 8 states: 2 tokens 5.8 | 24, 16 16.8 | 24.6, 24 23.3 |
+// 25.6, 32 29.6 | 25.9; 256 states: 8 22.6 | 26.7, 12 28.7 | 26.7; 1024: 8 68 | 82, 12
+// 88 | 82. 64 x 64, 8 states: 8 8.6 | 12.0, 14 12.2 | 12.1; 512: 4 13.4 | 14.0, 6 16.3 |
+// 13.9. 64 x 128, 64: 16 14.2 | 16.6, 20 17.1 | 17.2; 128 x 64, 256: 10 16.3 | 18.4, 14
+// 20.2 | 18.4.
+bool decay_attn_short(long longest, long states, int D, int V) {
+  const int most = D != V ? 16 : D == 128 ? 24 : 12;   // tokens, few workgroups
+  const long wgs = states * (V / 16);
+  const int tenths = wgs <= 512 ? 10 : wgs <= 1024 ? 8 : wgs <= 1536 ? 6
+                     : wgs <= 2048 ? 4 : D == 64 ? 3 : V == 64 ? 6 : 4;
+  return longest * 10 <= most * tenths;
+}
+
 // D, V in {64, 128}; rows 16 B aligned. ws null: no sequence has more than
 // DM_C tokens.
 void launch_decay_attn_mfma(float* out, const unsigned short* q,

@@ -1,5 +1,6 @@
 """Rotation and cache writes in 16 B pieces against the kernel for any alignment,
-which rows shifted by 8 bytes take: the same arithmetic, so the same bits."""
+which few tokens and rows shifted by 8 bytes take: the same arithmetic, so the same
+bits."""
 import pytest
 import torch
 
@@ -8,12 +9,14 @@ from xllm_service_amd import ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("T", [1, 5, 300])
+@pytest.mark.parametrize("T", [1, 5, 300, None])
 @pytest.mark.parametrize("heads,kv_heads,dim", [(32, 8, 128), (28, 4, 128),
                                                 (12, 12, 64), (3, 1, 80),
                                                 (5, 2, 96), (1, 1, 16)])
 @pytest.mark.parametrize("sections", [None, "eights", "odd"])
 def test_both_kernels(T, heads, kv_heads, dim, sections):
+    if T is None:                          # as few as the 16 B kernel takes
+        T = 16384 // ((heads + 2 * kv_heads) * (dim // 16)) + 1
     g = torch.Generator(device="cuda").manual_seed(T + heads + dim)
     width = (heads + 2 * kv_heads) * dim
     data = torch.randn(T, width, generator=g, device="cuda").to(torch.bfloat16)

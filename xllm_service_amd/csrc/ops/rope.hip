@@ -140,11 +140,12 @@ __global__ void fused_rope_cache_kernel(
 
 // The same where whole heads are rotated and everything is in steps of eight: a lane
 // has eight pairs, 16 B each, and its loads do not wait for each other (but for
-// cos and sin, which the position leads to). One token per row of workgroups.
+// cos and sin, which the position leads to). One token per row of workgroups, which
+// are no larger than its lanes.
 // 32/8 heads of 128, (one pair per lane, a wave per head and token) -> here: 8192
-// tokens 92.8 -> 33.4 us, 2048 27.1 -> 8.3, 300 5.10 -> 3.13, 128 3.36 -> 2.67, 24
-// 2.42 -> 2.40 (an empty launch: 2.0). That kernel stays for partial rotary and for
-// rows that are not aligned.
+// tokens 92.8 -> 33.4 us, 2048 27.1 -> 8.3, 300 5.10 -> 3.13, 128 3.36 -> 2.67 (an empty
+// launch: 2.0). That kernel stays for partial rotary, for rows that are not aligned
+// and for few tokens.
 __global__ void fused_rope_cache8_kernel(
     unsigned short* __restrict__ q, const unsigned short* __restrict__ k,
     const unsigned short* __restrict__ v, unsigned short* __restrict__ k_cache,
@@ -157,7 +158,7 @@ __global__ void fused_rope_cache8_kernel(
   long pos = positions[token];
   const long slot = slot_mapping[token];
   const unsigned half = D / 2, lanes = half / 8;    // lanes of a head
-  const unsigned at = blockIdx.y * 256 + threadIdx.x;
+  const unsigned at = blockIdx.y * blockDim.x + threadIdx.x;
   const int h = at / lanes, i = (at - h * lanes) * 8;
   if (h >= n_q + 2 * n_kv) return;
   const int kvh = h - n_q < n_kv ? h - n_q : h - n_q - n_kv;
@@ -208,16 +209,19 @@ void launch_fused_rope_cache(unsigned short* q, const unsigned short* k,
                              long q_stride, long kv_stride, int block_size,
                              int ms0, int ms1, hipStream_t stream) {
   // 16 B accesses of q, k, v, the caches and the table; rows of the M-RoPE
-  // sections in steps of eight
+  // sections in steps of eight. Few lanes stay with the other kernel, which finds
+  // its place without a division: 3 heads of 64, 1000 tokens 3.0 | 3.3 us here, 48
+  // heads of 80, 8 tokens 2.6 | 2.8, 32 2.7 | 2.9, 64 3.0 | 2.9.
   const auto on16 = [](const void* p) {
     return reinterpret_cast<uintptr_t>(p) % 16 == 0;
   };
-  if (T > 0 && rot == D && D % 16 == 0 && q_stride % 8 == 0 &&
+  const int lanes = (n_q + 2 * n_kv) * (D / 16);       // of a token
+  if ((long)T * lanes >= 16384 && rot == D && D % 16 == 0 && q_stride % 8 == 0 &&
       kv_stride % 8 == 0 && ms0 % 8 == 0 && ms1 % 8 == 0 && on16(q) &&
       on16(k) && on16(v) && on16(k_cache) && on16(v_cache) && on16(cos_sin)) {
-    const dim3 grid((unsigned)T,
-                    (unsigned)(((long)(n_q + 2 * n_kv) * (D / 16) + 255) / 256));
-    hipLaunchKernelGGL(fused_rope_cache8_kernel, grid, dim3(256), 0, stream, q,
+    const int wg = lanes < 256 ? (lanes + 63) / 64 * 64 : 256;
+    const dim3 grid((unsigned)T, (unsigned)((lanes + wg - 1) / wg));
+    hipLaunchKernelGGL(fused_rope_cache8_kernel, grid, dim3(wg), 0, stream, q,
                        k, v, k_cache, v_cache, positions, slot_mapping, cos_sin,
                        n_q, n_kv, D, q_stride, kv_stride, block_size, T, ms0,
                        ms1);

@@ -286,6 +286,22 @@ def test_decode_weights(keys, per):
     assert over.max() <= 0, f"over by {over.max():.3g}"
 
 
+@pytest.mark.parametrize("keys,kv_heads,per", [
+    ([1, 16, 9], 12, 1), ([64] * 29 + [17, 3], 12, 1),       # shuffled
+    ([17] * 24, 12, 1), ([65, 64, 1] * 10, 12, 2),           # streamed
+    ([33 * i + 1 for i in range(64)], 12, 1),                # by two waves
+    ([5000] + [40] * 29, 3, 1)])                             # never in parts
+def test_narrow_decode_forms(keys, kv_heads, per):
+    """64-wide heads on both sides of the lines between their forms."""
+    ctx = [n - 1 for n in keys]
+    rows, k, v, table = make([1] * len(keys), ctx, kv_heads, per, 64, sum(keys))
+    q = rows[:, :kv_heads * per * 64].unflatten(-1, (kv_heads * per, 64))
+    got = ops.paged_attn_decode(
+        q.cuda(), k.cuda(), v.cuda(), table.cuda(),
+        torch.tensor(keys, dtype=torch.int32, device="cuda"), 0.125)
+    check(got, *want(q, k, v, table, [1] * len(keys), ctx, 0.125))
+
+
 def test_decode_standout_scores():
     rows, k, v, table = make([1, 1], [900, 350], 1, 2, 128, 5)
     k[table[0, 4], 0, 3] *= 30.0

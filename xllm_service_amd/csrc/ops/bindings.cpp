@@ -42,7 +42,7 @@ void launch_paged_attn_decode(unsigned short*, const unsigned short*,
                               const int*, const int*, float*, float*, float,
                               int, int, int, int, int, long, long, bool,
                               hipStream_t);
-int paged_attn_decode_parts(int, int, int);
+int paged_attn_decode_parts(int, int, int, int);
 int paged_attn_prefill_parts(long, int, int, int, int, int);
 void launch_paged_attn_prefill(unsigned short*, float*, float*,
                                const unsigned short*, const unsigned short*,
@@ -241,7 +241,7 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
                       on_bytes(v_cache, 16) && on_bytes(q, 16) &&
                       on_bytes(out, 8);
   if (stream) {
-    parts = xllm::paged_attn_decode_parts(num_seqs, n_kv,
+    parts = xllm::paged_attn_decode_parts(num_seqs, n_kv, D,
                                           block_tables.size(1));
     if (parts > 1) {
       const long n = (long)num_seqs * n_qheads * parts;

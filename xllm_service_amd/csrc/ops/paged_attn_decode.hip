@@ -126,8 +126,32 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
   }
 }
 
-int paged_attn_decode_parts(int num_seqs, int n_kv_heads, int max_blocks) {
-  return paged_stream_split(num_seqs, n_kv_heads, max_blocks).parts;
+// 64-wide heads had one workgroup per pair and no merge before they were streamed
+// (by the shuffle kernel above), so the split of the 128-wide ones does not pay
+// for many pairs: 128 sequences of 12 heads, 64 keys each in tables of 8192,
+// shuffle 7.9 | split 17.1 | whole 9.2 us, 500 keys 35 | 38.5 | 32. From 768 pairs on
+// workgroups of two waves, twice as many at a time: 64 keys 9.2 -> 6.8, 16 8.0 -> 5.9
+// (384 pairs of 500 keys 11.8 -> 15.7, so not there).
+//   Few pairs: as for 128-wide heads. In tables of 768 keys and more that costs the
+// shortest sequences the merge (64 keys 4.7 -> 5.6 us) for what the others gain (200
+// keys 9.3 -> 6.5, 1000 32 -> 7.7); eight waves without a merge would be 4.6, 5.2 and
+// 9.1, 2000 keys 13.9 instead of 7.7.
+static PagedSplit decode_split(long num_seqs, int n_kv_heads, int D,
+                               long max_blocks) {
+  const long units = num_seqs * n_kv_heads;
+  if (D == 64 && units >= 86) return {1, 1, units >= 768 ? 2 : 4};
+  return paged_stream_split(num_seqs, n_kv_heads, max_blocks);
+}
+// Tables of a page or of a few, one or two query heads per key head: the shuffle
+// kernel, whose chain is shorter. One page, 12 heads x 16 sequences 3.4-4.5 | 4.3 us,
+// x 128 3.9-5.2 | 5.9; four pages, x 32 4.8 | 5.2.
+static bool decode_tiny(long units, int G, int D, long max_blocks) {
+  return D == 64 && G <= 2 &&
+         (max_blocks <= 1 || (max_blocks <= 4 && units >= 300 && units < 768));
+}
+int paged_attn_decode_parts(int num_seqs, int n_kv_heads, int D,
+                            int max_blocks) {
+  return decode_split(num_seqs, n_kv_heads, D, max_blocks).parts;
 }
 
 // streamed: rows of q and the caches on 16 B, of out on 8 B, and heads 64 or 128
@@ -143,7 +167,8 @@ void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
                               hipStream_t stream) {
   const int G = n_qheads / n_kv_heads;
   if (num_seqs == 0) return;
-  if (!streamed) {
+  if (!streamed ||
+      decode_tiny((long)num_seqs * n_kv_heads, G, D, max_blocks_per_seq)) {
     const dim3 grid(num_seqs * n_kv_heads), block(256);
 #define PA_SMALL(GV)                                                           \
   hipLaunchKernelGGL((paged_attn_decode_small_kernel<GV>), grid, block, 0,     \
@@ -169,7 +194,7 @@ void launch_paged_attn_decode(unsigned short* out, const unsigned short* q,
   auto go = D == 128 ? paged_stream<128, 2, false> : paged_stream<64, 3, false>;
   go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, seq_lens, num_seqs,
      scale, n_qheads, n_kv_heads, max_blocks_per_seq, q_stride, out_stride,
-     paged_stream_split(num_seqs, n_kv_heads, max_blocks_per_seq), PagedMore{},
+     decode_split(num_seqs, n_kv_heads, D, max_blocks_per_seq), PagedMore{},
      stream);
 }
 

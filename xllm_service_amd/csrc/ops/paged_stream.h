@@ -32,7 +32,6 @@ namespace xllm {
 
 #define PA_BS 16           // cache block size (tokens)
 #define PA_KT 32           // keys per tile (2 cache blocks)
-#define PA_NW 4            // waves per workgroup
 
 // Columns [0, D) of 16 rows of a V image: the A operands of one step of
 // O^T += V^T P^T. The wait is part of it: a builtin here would make the compiler
@@ -110,8 +109,10 @@ XLLM_DEV void pa_rows(const unsigned (&at)[D / 16], bf16x8 (&k)[D / 16]) {
 // by 32 waves a row 0.00186; with two 0.00166, which is the rounding to bf16. Us,
 // one term | two by a product of their own | here: 1 x 776 keys 9.0 | 9.6 | 9.5,
 // 24 x 0.6-1.4 k 18.9 | 19.6 | 19.1, 128 x 1-2 k 142.5 | 142.8 | 142.0.
-template <int D, int TERMS, bool MORE>
-__global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
+//   NW: waves of a workgroup, four but where the 64-wide form asks for two.
+template <int D, int TERMS, bool MORE, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 2 ? 8 : 2) void
+paged_attn_stream_kernel(
     void* __restrict__ out,                  // [S, n_qheads, D]
     float* __restrict__ ws_o,                // [S*n_qheads][P][D] (P > 1)
     float* __restrict__ ws_ml,               // [S*n_qheads][P][2]
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
     const float scale, const int G, const int n_kv, const int max_blocks,
     const long q_stride, const long out_stride, const int P, const int per,
     const PagedMore x) {
-  constexpr int NW = PA_NW, KS = D / 16, DT = D / 32;
+  constexpr int KS = D / 16, DT = D / 32;
   constexpr bool FOLD = TERMS == 2;          // G <= 8
   constexpr int NP = FOLD ? 1 : TERMS;       // products per weight
   constexpr int CPR = D / 8;                 // 16 B chunks of a row
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(PA_NW * 64, 2) void paged_attn_stream_kernel(
 // 32: 31, 36, 54, 22).
 //   Eight waves in a workgroup instead of four: within 5 % where keys are split,
 // slower for many pairs (128 x 300 keys: 41 against 33).
-struct PagedSplit { int parts, per; };
+struct PagedSplit { int parts, per, waves = 4; };
 inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
                                      long max_blocks, bool capped = false) {
   const long units = num_seqs * n_kv_heads, f = capped ? 2 : 1;
@@ -446,11 +447,19 @@ inline void paged_stream(void* out, float* ws_o, float* ws_ml,
                          hipStream_t stream) {
   if (num_seqs == 0) return;
   const dim3 grid((unsigned)(num_seqs * n_kv * split.parts));
-  hipLaunchKernelGGL((paged_attn_stream_kernel<D, TERMS, MORE>), grid,
-                     dim3(PA_NW * 64), 0, stream, out, ws_o, ws_ml, q, k_cache,
-                     v_cache, block_tables, seq_lens, scale, n_qheads / n_kv,
-                     n_kv, max_blocks, q_stride, out_stride, split.parts,
-                     split.per, x);
+#define PS_GO(NW)                                                              \
+  hipLaunchKernelGGL((paged_attn_stream_kernel<D, TERMS, MORE, NW>), grid,     \
+                     dim3(NW * 64), 0, stream, out, ws_o, ws_ml, q, k_cache,   \
+                     v_cache, block_tables, seq_lens, scale, n_qheads / n_kv,  \
+                     n_kv, max_blocks, q_stride, out_stride, split.parts,      \
+                     split.per, x)
+  if constexpr (D == 64 && !MORE) {
+    if (split.waves == 2) PS_GO(2);
+    else PS_GO(4);
+  } else {
+    PS_GO(4);
+  }
+#undef PS_GO
   if (split.parts > 1)
     paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, split.parts, out_stride,
                          (long)num_seqs * n_qheads, x, stream, seq_lens,

@@ -350,6 +350,7 @@ OPTIONS = {
 @pytest.mark.parametrize("lens,ctx,kv_heads,per,decode", [
     ([1, 33, 64, 130], [16, 31, 100, 0], 2, 4, False),
     ([5, 2], [1500, 3000], 1, 2, False),                   # parts
+    ([1, 2, 5, 33] * 6, [100, 31, 400, 0] * 6, 2, 4, False),   # few keys, many
     ([1] * 5, [0, 15, 31, 127, 400], 3, 4, True),
     ([1, 1], [2000, 4095], 1, 32, True),                   # parts
     ([1] * 30, [20 + 31 * i for i in range(29)] + [3500], 3, 2, True),

@@ -127,6 +127,7 @@ void launch_gated_group_norm(T*, const float*, const float*, int, const T*,
                              long, float, int, int, int, int, int,
                              long, hipStream_t);
 int paged_attn_parts(bool, long, int, int, int, long, int, int, bool);
+bool paged_attn_small(bool, long, int, int, int, int, long, int, int, bool);
 void launch_paged_attn(void*, long, bool, float*, float*, const unsigned short*,
                        const unsigned short*, const unsigned short*, const int*,
                        const int*, const int*, long, int, int, int, int, int,
@@ -1138,9 +1139,11 @@ void capped_attn(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
       out_stride % 4 == 0 &&
       reinterpret_cast<uintptr_t>(out.data_ptr()) % (out_bf ? 8 : 16) == 0;
   // 16-token pages, keys and values 64 or 128 wide (decode: no more query heads
-  // per key head than a wave has rows)
+  // per key head than a wave has rows), and more than a few keys per row
   if (rows16 && bs == 16 && D == Dv && (D == 64 || D == 128) &&
       (cu != nullptr || heads / n_kv <= 32) &&
+      !hy::paged_attn_small(cu == nullptr, T, n_seqs, heads, n_kv, D,
+                            block_tables.size(1), window, keep_first, cap > 0) &&
       reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(v_cache.data_ptr()) % 16 == 0) {
     const int n_part =

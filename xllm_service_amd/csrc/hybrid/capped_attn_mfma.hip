@@ -64,9 +64,11 @@ XLLM_DEV bf16x8 cm_ld8(const unsigned short* p) {
   return *reinterpret_cast<const bf16x8*>(p);
 }
 
-XLLM_DEV float cm_tanh(float x) {          // 1 - 2 / (e^(2x) + 1)
-  const float e = __expf(2.0f * (x > 15.0f ? 15.0f : x));  // NaN stays
-  return 1.0f - 2.0f / (e + 1.0f);
+// (scores below half the cap, nearly all of them, need no exponential)
+XLLM_DEV float cm_tanh(float x) {
+  const float y = tanh_near(x);
+  const bool far = !(fabsf(x) < 0.5f);
+  return __any(far) && far ? tanh_far(x) : y;
 }
 
 // KQ = 32-column chunks of a key row (D padded), NO = 16-column tiles of a
@@ -348,7 +350,7 @@ capped_attn_mfma_kernel(
   if (!wave_on || !row_ok) return;
   // acc[lb*4+nn][rr] = O^T[col = ((lb*CS+cpart)*4+nn)*16 + g*4 + rr][row n]
   if (n_part == 1 && sink != nullptr) l += __expf(sink[head] - m);
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  const float inv = l != 0.f ? 1.0f / l : 0.f;
   const long base = grow * n_part + blockIdx.y;
   const float mul = (n_part == 1) ? inv : 1.0f;
   const long orow = tok * out_stride + (long)head * Dv;
@@ -392,7 +394,7 @@ __global__ void __launch_bounds__(256) capped_attn_merge_kernel(
     if (M == -INFINITY) M = 0.f;
     const float e = on ? __expf(mp - M) : 0.f;
     const float L = wave_reduce_sum(lp * e) + (sink ? __expf(sk - M) : 0.f);
-    wgt[tid] = (L > 0.f) ? e / L : 0.f;
+    wgt[tid] = (L != 0.f) ? e / L : 0.f;
   }
   __syncthreads();
   const float* base = ws_acc + row * n_part * (long)r;

@@ -78,4 +78,22 @@ XLLM_DEV float block_reduce_sum(float v, float* tmp) {
   return tmp[0];
 }
 
+// tanh below 1/2: the odd Taylor series up to x^15 (the next term is under 2^-26 of
+// the value)
+XLLM_DEV float tanh_near(float v) {
+  const float w = v * v;
+  float y = fmaf(w, -929569.0f / 638512875.0f, 21844.0f / 6081075.0f);
+  y = fmaf(y, w, -1382.0f / 155925.0f);
+  y = fmaf(y, w, 62.0f / 2835.0f);
+  y = fmaf(y, w, -17.0f / 315.0f);
+  y = fmaf(y, w, 2.0f / 15.0f);
+  y = fmaf(y, w, -1.0f / 3.0f);
+  return fmaf(y * w, v, v);
+}
+// 1 - 2 / (e^2x + 1): from 1/2 on; a NaN stays one
+XLLM_DEV float tanh_far(float v) {
+  const float e = __expf(2.0f * (v > 15.0f ? 15.0f : v));
+  return 1.0f - 2.0f / (e + 1.0f);
+}
+
 }  // namespace xllm

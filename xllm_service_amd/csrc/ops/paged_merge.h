@@ -59,9 +59,8 @@ XLLM_DEV PagedScore paged_score(const PagedMore& x, float scale, int head) {
           paged_factor(scale), 0.0f};
 }
 
-// s <- cap * tanh(pre * s). Below 1/2 the odd Taylor series up to x^15 (the next
-// term is under 2^-26 of the value); above, 1 - 2 / (e^2x + 1). Tiles without
-// large scores, nearly all of them, skip the exponentials and divisions.
+// s <- cap * tanh(pre * s). Tiles without large scores, nearly all of them, skip
+// the exponentials and divisions.
 template <int N>
 XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
   float big = 0.0f;
@@ -77,17 +76,10 @@ XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
   for (int i = 0; i < N; i++)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-      const float v = s[i][r], w = v * v;
-      float y = fmaf(w, -929569.0f / 638512875.0f, 21844.0f / 6081075.0f);
-      y = fmaf(y, w, -1382.0f / 155925.0f);
-      y = fmaf(y, w, 62.0f / 2835.0f);
-      y = fmaf(y, w, -17.0f / 315.0f);
-      y = fmaf(y, w, 2.0f / 15.0f);
-      y = fmaf(y, w, -1.0f / 3.0f);
-      y = fmaf(y * w, v, v);
+      const float v = s[i][r];
+      float y = tanh_near(v);
       if (far) {
-        const float e = __expf(2.0f * (v > 15.0f ? 15.0f : v));  // NaN stays
-        const float z = 1.0f - 2.0f / (e + 1.0f);
+        const float z = tanh_far(v);
         y = fabsf(v) < 0.5f ? y : z;
       }
       s[i][r] = cap * y;

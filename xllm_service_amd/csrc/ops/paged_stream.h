@@ -412,25 +412,30 @@ paged_attn_stream_kernel(
 // | 20.3. The host sees no lengths, and in a captured step the widest table there can
 // be: whole below 3000 keys, and up to 128 pairs (which bring the least bytes to
 // hide a chain behind) above, up to 4096 for more pairs.
-//   Capped scores make a tile about twice as long: four tiles a part instead of
-// eight, and with many pairs, of any number, from 1500 keys on at most four parts of
-// 20 tiles. 4 key heads: 32 x 0.7-3 k 47 | 30, 32 x 0-4 k 61 | 37, 64 x 0.3-3 k
+//   With options (a window, a cap, a sink) weights have 32 bits and a tile is longer,
+// with a cap about twice as long: four tiles a part instead of eight (8 key heads, a
+// window of 512 11.7 -> 10.3, 300 keys in tables of 4096 9.8 -> 8.6), and for capped
+// scores, with many pairs below 512, from 1500 keys on at most four parts of 20 tiles
+// (1024 pairs of 16 keys in tables of 4096 8.6 in one | 16.5). 4 key heads: 32 x 0.7-3 k 47 | 30, 32 x 0-4 k 61 | 37, 64 x 0.3-3 k
 // 54 | 51, 24 x 0.1-1 k in tables of 4096 20 | 19 (parts of 16: 31, 37, 50, 17; of
 // 32: 31, 36, 54, 22).
 //   Eight waves in a workgroup instead of four: within 5 % where keys are split,
 // slower for many pairs (128 x 300 keys: 41 against 33).
 struct PagedSplit { int parts, per, waves = 4; };
 inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
-                                     long max_blocks, bool capped = false) {
-  const long units = num_seqs * n_kv_heads, f = capped ? 2 : 1;
-  const long tiles = f * ((max_blocks * PA_BS + PA_KT - 1) / PA_KT);
+                                     long max_blocks, bool options = false,
+                                     bool capped = false) {
+  const long units = num_seqs * n_kv_heads;
   const bool few = units < 86;
+  const long f = (few ? options : capped) ? 2 : 1;
+  const long tiles = f * ((max_blocks * PA_BS + PA_KT - 1) / PA_KT);
   const int per = few ? (int)(8 / f) : capped ? 20 : 32;
   if (few && units > 0) {
     const long p = std::min<long>({256 / units, tiles / 8, 16});
     return {p < 3 ? 1 : (int)p, per};
   }
-  if (units == 0 || tiles < 96 || (units > 128 && !capped && tiles <= 128))
+  if (units == 0 || tiles < 96 || (units > 128 && !capped && tiles <= 128) ||
+      (units >= 512 && capped))
     return {1, per};
   return {(int)std::min<long>(8 / f, (tiles + 31) / 32), per};
 }

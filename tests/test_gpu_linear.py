@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M", [1, 31, 32, 33, 63, 64, 65, 100, 129, 300])
 @pytest.mark.parametrize("N,K", [(8, 128), (64, 256), (72, 1152), (200, 4096),
-                                 (4096, 384)])
+                                 (4096, 384), (4104, 384), (2056, 2048),
+                                 (3080, 4096), (8192, 2048)])
 @pytest.mark.parametrize("bias,stride", [(False, 0), (True, 8)])
 def test_linear(M, N, K, bias, stride):
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
@@ -89,3 +90,39 @@ def test_bias_that_overrides_the_call():
     b = torch.randn(64, device="cuda").to(torch.bfloat16).as_subclass(Seen)
     assert isinstance(ops.linear(x, w, b), Seen)
     assert torch.nn.functional.linear in calls
+
+
+def test_tuned_choices_are_kept():
+    """A product that the loaded table of tuned kernels names runs on the library
+    where its own kernel is the slower one."""
+    import os
+
+    import torch.cuda.tunable as tunable
+    from torch.profiler import ProfilerActivity, profile
+    table = os.path.join(os.path.dirname(__file__), "..", "configs",
+                         "tunableop_gfx950.csv")
+    x, w = (torch.randn(r, 4096, device="cuda").to(torch.bfloat16)
+            for r in (128, 4096))
+
+    def own():
+        """Whether a kernel of linear.hip ran."""
+        ops.linear(x, w)
+        with profile(activities=[ProfilerActivity.CUDA]) as seen:
+            ops.linear(x, w)
+            torch.cuda.synchronize()
+        names = [e.key for e in seen.key_averages()]
+        if not any(n.startswith(("void xllm", "Cijk")) for n in names):
+            pytest.skip(f"no kernel names from the profiler: {names}")
+        return any("linear_tile" in n or "linear_stream" in n for n in names)
+    was = tunable.is_enabled(), tunable.tuning_is_enabled()
+    try:
+        tunable.enable(True)
+        tunable.tuning_enable(False)
+        if not tunable.read_file(table):
+            pytest.skip("the table is for other versions of the library")
+        assert not own()
+        tunable.enable(False)
+        assert own()
+    finally:
+        tunable.enable(was[0])
+        tunable.tuning_enable(was[1])

@@ -3,6 +3,7 @@
 // All tensor-shape/dtype validation lives here so the kernels stay lean.
 #include <hip/hip_runtime.h>
 #include <ATen/autocast_mode.h>
+#include <ATen/hip/tunable/Tunable.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -386,6 +387,20 @@ bool direct(const std::vector<torch::Tensor>& tensors) {
   return true;
 }
 
+// Whether torch's table of tuned products, if it is in use, names a kernel of the
+// library for y [M, N] = x [M, K] w [N, K]^T
+static bool tuned(long M, long N, long K, long x_stride) {
+  auto* ctx = at::cuda::tunable::getTuningContext();
+  if (!ctx->IsTunableOpEnabled()) return false;
+  char shape[160];
+  snprintf(shape, sizeof shape, "tn_%ld_%ld_%ld_ld_%ld_%ld_%ld", N, M, K, K,
+           x_stride, N);
+  const auto entry = ctx->GetTuningResultsManager().Lookup(
+      "GemmTunableOp_BFloat16_TN", shape);
+  return entry != at::cuda::tunable::ResultEntry::Null() &&
+         entry != at::cuda::tunable::ResultEntry::Default();
+}
+
 // x [..., K] @ w [N, K]^T (+ bias): the kernels of linear.hip where they take the
 // call, the library elsewhere (and wherever a gradient is wanted)
 torch::Tensor linear(torch::Tensor x, torch::Tensor w,
@@ -406,7 +421,8 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor w,
         bias->device() == w.device()))) {
     const long M = x.size(0), N = w.size(0), K = w.size(1);
     const int kind = xllm::linear_takes(M, N, K);
-    if (kind != 0) {
+    if (kind != 0 &&
+        !(M > 48 && !bias.has_value() && tuned(M, N, K, x.stride(0)))) {
       c10::OptionalDeviceGuard guard(x.device());
       auto y = torch::empty({M, N}, x.options());
       xllm::launch_linear(u16(y), u16c(x), u16c(w),

@@ -268,12 +268,21 @@ __global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
 //            | 50-104 (tuned 50)
 //   M 300    2048 x 2048 10.8 | 10.5, 4096 x 2048 16.6 | 15.7, 4096 x 4096 29 | 25
 //   M 512    3072 x 2048 16.5 | 15.3, 4096 x 2048 17.6 | 17.1; M 1024 30 | 24
+//   M 96-256, few tiles   512 x 4096 17.7 | 8.8-12, 1024 x 2048 10.5 | 8.4, 1536 x 3072
+//            16 | 10.7, 2048 x 4096 18.8-20.4 | 12.8-15.9, 2560 x 4096 19 | 13; 1024 x
+//            1024 and 3072 x 4096 are still faster here
+//   M 16     32000 x 4096 as above, 128256 x 4096 193 | 189 (tuned 178); 8 177 | 188
+// A tuned choice of the library is preferred above 48 rows (linear in bindings.cpp):
+//   4096 x 4096, here | tuned | not   M 48 12.6 | 13.7 | 13.7, 64 14.5 | 13.6 | 15.1,
+//            96 19.6 | 17.2 | 22.0, 128 21.4 | 16.9 | 24.5
 int linear_takes(long M, long N, long K) {
   if (M <= 0 || K < LN_K || K % LN_K != 0 || N % 8 != 0) return 0;
   if (N * K >= (1L << 31) || M * K >= (1L << 30)) return 0;
-  if (M <= 16) return 1;
+  if (M <= 16) return M <= 8 || N * K <= 1L << 28 ? 1 : 0;
   if (M <= 64) return N * K <= 4096L * 4096 ? 1 : 0;
   const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  // few tiles with long rows leave most of the chip waiting for their chain
+  if (tiles <= 128 && ((K > 2048 && N < 3072) || (K > 1024 && N < 2048))) return 0;
   return K <= 4096 && (tiles <= 256 || (tiles <= 512 && K <= 2048)) ? 2 : 0;
 }
 

@@ -46,3 +46,45 @@ def test_decode_edges(tail, heads, window, keys):
             off = (out[s].double().cpu() - p @ k[:, :r]).abs()
             over = off - 2.0 ** -17 * (p @ k[:, :r].abs())
             assert over.max() <= 1e-7, f"sequence {s}: off by {off.max():.3g}"
+
+
+@pytest.mark.parametrize("op", ["latent", "capped"])
+def test_fixed_parts(op, monkeypatch):
+    """XLLM_LATENT_PARTS and XLLM_CAPPED_PARTS fix the parts of decoded rows: one
+    part needs no workspace, 16 need one, and the results agree."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    keys, heads = 900, 8
+    table = torch.randperm(60, generator=g, device="cuda").int().view(1, 60)
+    sl = torch.tensor([keys], dtype=torch.int32, device="cuda")
+    if op == "latent":
+        cache = torch.randn(60, 16, 576, generator=g, device="cuda").to(
+            torch.bfloat16)
+        q = torch.randn(1, heads, 576, generator=g, device="cuda").to(
+            torch.bfloat16)
+        out = torch.zeros(1, heads, 512, device="cuda")
+
+        def run():
+            H.latent_attn(q, cache, table, None, sl, 0.07, 512, out)
+    else:
+        k, v = (torch.randn(60, 2, 16, 128, generator=g, device="cuda").to(
+            torch.bfloat16) for _ in range(2))
+        q = torch.randn(1, heads * 128, generator=g, device="cuda").to(
+            torch.bfloat16)
+        out = torch.zeros(1, heads, 128, device="cuda")
+
+        def run():
+            H.capped_attn(q, k, v, table, None, sl, heads, 0.08, 0.0, out)
+    run()
+    free = out.clone()
+    used = {}
+    for parts in (1, 16):
+        monkeypatch.setenv(f"XLLM_{op.upper()}_PARTS", str(parts))
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        out.zero_()
+        run()
+        torch.cuda.synchronize()
+        used[parts] = torch.cuda.max_memory_allocated() - before
+        assert (out - free).abs().max() <= 1e-5
+    assert used[1] == 0 and used[16] > 0, used

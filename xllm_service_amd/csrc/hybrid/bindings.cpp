@@ -576,8 +576,10 @@ void latent_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables,
   auto aligned = [](const Tensor& t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  // decoded rows of the rank-512 sizes
+  // decoded rows of the rank-512 sizes (XLLM_LATENT_PARTS asks for the kernel with a
+  // fixed number of parts)
   if (is_bf16(q) && cu == nullptr &&
+      std::getenv("XLLM_LATENT_PARTS") == nullptr &&
       hy::latent_stream_takes(W, r, H, cache.size(1)) && aligned(q) &&
       aligned(cache) && aligned(out) && block_tables.size(1) > 0) {
     const int n_part =
@@ -1139,9 +1141,11 @@ void capped_attn(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
       out_stride % 4 == 0 &&
       reinterpret_cast<uintptr_t>(out.data_ptr()) % (out_bf ? 8 : 16) == 0;
   // 16-token pages, keys and values 64 or 128 wide (decode: no more query heads
-  // per key head than a wave has rows), and more than a few keys per row
+  // per key head than a wave has rows), and more than a few keys per row.
+  // XLLM_CAPPED_PARTS asks for the decode kernel with a fixed number of parts
   if (rows16 && bs == 16 && D == Dv && (D == 64 || D == 128) &&
-      (cu != nullptr || heads / n_kv <= 32) &&
+      (cu != nullptr || (heads / n_kv <= 32 &&
+                         std::getenv("XLLM_CAPPED_PARTS") == nullptr)) &&
       !hy::paged_attn_small(cu == nullptr, T, n_seqs, heads, n_kv, D,
                             block_tables.size(1), window, keep_first, cap > 0) &&
       reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&

@@ -1,9 +1,10 @@
 """Paged attention of prompt rows and of decoded rows at the edges of their
-tiles, pages and key parts, against fp64 on the CPU. Results are bf16, off by up to 2^-9 of
-themselves. The weights that meet 128-wide values are rounded to bf16 as well:
-2^-9 of the weighted sum of |v|; twice both is allowed (the weights' sum is not
-rounded the same way). 64-wide heads keep 32-bit weights: 2^-18 for their
-exponentials, whose arguments are rounded products of up to 2^5."""
+tiles, pages and key parts, against fp64 on the CPU. Results are bf16, off by up to
+2^-8 of themselves (half a step of 2^-7 at a power of two). The weights that meet
+128-wide values of prompts are rounded to bf16 as well, each by up to 2^-8 of itself,
+2^-9 on average: 2^-8 of the weighted sum of |v| is allowed, for decoded rows too,
+whose weights have 16 bits (test_decode_weights). 64-wide heads keep 32-bit weights:
+2^-18 for their exponentials, whose arguments are rounded products of up to 2^5."""
 import math
 
 import pytest

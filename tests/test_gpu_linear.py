@@ -1,7 +1,7 @@
 """x W^T (+ bias) at the edges of its tiles, against fp64 of the bf16 inputs. Sums
-are 32-bit and the result is rounded to bf16: 2^-9 of itself and 2^-24 times
-the square root of the number of terms (K up to 4096: 2^-18) of the sum of
-absolute products; twice both is allowed."""
+are 32-bit and the result is rounded to bf16: 2^-8 of itself (half a step of 2^-7 at
+a power of two) and 2^-24 times the square root of the number of terms (K up to
+4096: 2^-18) of the sum of absolute products, of which twice as much is allowed."""
 import pytest
 import torch
 

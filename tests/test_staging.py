@@ -25,7 +25,12 @@ def test_staging_sections():
     s.host["a"][:] = 9
     s.host["t"][:] = np.arange(24).reshape(4, 6)
     assert s._last % 4 == 0 and s._row == 6
-    n = s._last + 2 * s._row           # what flush(2) copies
-    s._dev[:n].copy_(s._pin[:n])
+    s.wait()                           # nothing is on its way yet
+    s.flush(2)
+    s.wait()
     assert s.dev["a"].tolist() == [9] * 3
     assert s.dev["t"].flatten().tolist() == list(range(12)) + [0] * 12
+    s.host["b"][:] = 4
+    s.flush(4)
+    assert s.dev["b"].tolist() == [4] * 5
+    assert s.dev["t"].flatten().tolist() == list(range(24))

@@ -26,8 +26,7 @@
 // pieces of 32 B) that share an LDS cycle fall on different banks.
 //
 // Measured, 32 sequences of 1.5-2.4 k keys, 16 heads, rows of 576: 67 + 5 us before,
-// 24 us with the merge now; the rows alone take 15 us
-// at the rate of a large copy.
+// 24 us with the merge now; the rows alone take 15 us at the rate of a large copy.
 //
 // The LDS reads are asm with their wait: in front of a builtin the compiler
 // waits for every load to LDS in flight.
@@ -104,11 +103,6 @@ XLLM_DEV f32x4 ls_mma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// parts that n tiles are really split into, of the n_part there is room for
-XLLM_DEV int ls_parts(int n, int n_part, int per) {
-  return max(1, min(n_part, (n + per - 1) / per));
-}
-
 template <int W>
 __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
     float* __restrict__ out,               // [S, H, 512] (n_part == 1)
@@ -135,7 +129,7 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   const int n_tiles = (seq_len + LS_KT - 1) / LS_KT;
   const int lo = window > 0 ? max(0, seq_len - window) : 0;
   const int t_first = lo / LS_KT;
-  const int parts = ls_parts(n_tiles - t_first, n_part, per);
+  const int parts = paged_parts(n_tiles - t_first, n_part, per);
   if (part >= parts) return;
   const int tpp = (n_tiles - t_first + parts - 1) / parts;
   const int t_begin = t_first + part * tpp;
@@ -351,7 +345,7 @@ __global__ void __launch_bounds__(256) latent_stream_merge_kernel(
   const int col = (threadIdx.x & 127) * 4;
   if (row >= rows) return;
   const int len = seq_lens[row / heads];
-  const int parts = ls_parts(
+  const int parts = paged_parts(
       (len + LS_KT - 1) / LS_KT -
           (window > 0 ? max(0, len - window) / LS_KT : 0), n_part, per);
   if (parts == 1) return;                        // written where it belongs

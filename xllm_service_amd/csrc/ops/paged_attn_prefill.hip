@@ -29,10 +29,10 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws_o, float* ws_ml,
 }
 
 // ---------------------------------------------------------------------------------
-// MFMA layout probe: C[16][16] = A[16][32] x B[32][16] with the fragment
-// layout assumptions documented above. tests/test_gpu_ops.py checks this
-// against torch.matmul on random data — if the lane mappings are wrong, that
-// test fails (and so would the prefill kernel).
+// Probe of the 16x16x32 fragments, A[l&15][8 (l>>4) + j], B[8 (l>>4) + j][l&15],
+// C[4 (l>>4) + r][l&15], which linear.hip's stream kernel and the 16-row kernels of
+// ../hybrid rely on (the 32x32x16 ones of this directory: mfma_rows.h):
+// tests/test_gpu_ops.py compares it with torch.matmul on random data.
 __global__ void mfma_probe_kernel(float* __restrict__ c,
                                   const unsigned short* __restrict__ a,
                                   const unsigned short* __restrict__ b) {

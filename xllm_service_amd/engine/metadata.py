@@ -24,10 +24,6 @@ class AttnMetadata:
     prefill_seq_lens: Optional[torch.Tensor] = None   # [n_prefill] int32 (ctx+chunk)
     prefill_block_tables: Optional[torch.Tensor] = None  # [n_prefill, max_blk] int32
 
-    # a prefill tile decomposition (tile_seq, tile_q0); the kernel finds its
-    # rows from cu_q on the device and does not need one
-    prefill_tiles: Optional[tuple] = None
-
     # decode half
     decode_seq_lens: Optional[torch.Tensor] = None    # [n_decode] int32
     decode_block_tables: Optional[torch.Tensor] = None

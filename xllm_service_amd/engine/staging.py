@@ -87,6 +87,8 @@ class Staging:
     def flush(self, rows: int) -> None:
         n = self._last + rows * self._row
         self._dev[:n].copy_(self._pin[:n], non_blocking=True)
+        if not self._dev.is_cuda:
+            return
         if self._copied is None:
             self._copied = torch.cuda.Event()
         self._copied.record()

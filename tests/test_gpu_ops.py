@@ -53,6 +53,27 @@ def test_rmsnorm(dev):
         _assert_close(got, want, atol=3e-2, label=f"rmsnorm {T}x{H}")
 
 
+@pytest.mark.parametrize("H", [4096, 4104, 8192, 8200, 16384, 32768])
+def test_rmsnorm_wide_rows(dev, H):
+    """Rows of one to eight pieces per thread, with and without the residual, on
+    both sides of the line up to which the weights come with the row. 2^-8: the
+    rounding of the result, and of the sum that both write back; 2^-18: fp32."""
+    g = torch.Generator(device=dev).manual_seed(H)
+    x, r = (torch.randn(3, H, generator=g, device=dev).to(torch.bfloat16)
+            for _ in range(2))
+    w = torch.randn(H, generator=g, device=dev).to(torch.bfloat16)
+
+    def want(z):
+        return z * (z.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * w.double()
+    ref0, s = want(x.double()), x.double() + r.double()
+    assert ((ops.rmsnorm(x, w, 1e-5).double() - ref0).abs()
+            <= (2.0 ** -8 + 2.0 ** -18) * ref0.abs()).all()
+    got, res = ops.fused_add_rmsnorm(x.clone(), r.clone(), w, 1e-5)
+    assert ((res.double() - s).abs() <= 2.0 ** -8 * s.abs()).all()
+    assert ((got.double() - want(s)).abs()
+            <= (2.0 ** -8 + 2.0 ** -18) * want(s).abs()).all()
+
+
 def test_fused_add_rmsnorm(dev):
     torch.manual_seed(0)
     T, H = 33, 4096

@@ -27,7 +27,9 @@ XLLM_DEV float row_sum(float v, float* tmp) {
 
 // A few rows (decoding): a chain of latencies; the weights come with the row, not
 // after its sum. 24 rows of 4096 2.60 -> 2.56 us, of 8192 3.25 -> 3.03 (an empty
-// launch: 2.0); 8192 of 4096 39.5 us, 6.8 TB/s, as before.
+// launch: 2.0); 8192 of 4096 39.5 us, 6.8 TB/s, as before. Rows above 8192, of which
+// a thread has three pieces and more, have no registers to spare for that: 300 x
+// 32768 with the residual 19.5 that way, 13.3 with weights after the sum.
 // ELEMS = number of ushort8 octets each thread owns (H <= block*8*ELEMS)
 template <bool FUSED_ADD, int ELEMS>
 __global__ void rmsnorm_kernel(
@@ -46,15 +48,17 @@ __global__ void rmsnorm_kernel(
   unsigned short* rr = FUSED_ADD ? residual + (long)row * H : nullptr;
   unsigned short* orow = out + (long)row * H;
 
+  constexpr bool EARLY = ELEMS <= 2;         // weights with the row
   float v[ELEMS][8];
-  ushort8_t wv[ELEMS];
+  ushort8_t wv[EARLY ? ELEMS : 1];
   float sumsq = 0.0f;
 #pragma unroll
   for (int e = 0; e < ELEMS; e++) {
     const int i = (tid + e * nthread) * 8;
     if (i < H) {
       ushort8_t u = *reinterpret_cast<const ushort8_t*>(xr + i);
-      wv[e] = *reinterpret_cast<const ushort8_t*>(w + i);
+      if constexpr (EARLY)
+        wv[e] = *reinterpret_cast<const ushort8_t*>(w + i);
 #pragma unroll
       for (int j = 0; j < 8; j++) v[e][j] = bf16_to_f32(u.x[j]);
       if constexpr (FUSED_ADD) {
@@ -78,10 +82,13 @@ __global__ void rmsnorm_kernel(
   for (int e = 0; e < ELEMS; e++) {
     const int i = (tid + e * nthread) * 8;
     if (i < H) {
+      const ushort8_t g =
+          EARLY ? wv[EARLY ? e : 0]
+                : *reinterpret_cast<const ushort8_t*>(w + i);
       ushort8_t o;
 #pragma unroll
       for (int j = 0; j < 8; j++)
-        o.x[j] = f32_to_bf16(v[e][j] * rrms * bf16_to_f32(wv[e].x[j]));
+        o.x[j] = f32_to_bf16(v[e][j] * rrms * bf16_to_f32(g.x[j]));
       *reinterpret_cast<ushort8_t*>(orow + i) = o;
     }
   }

@@ -34,6 +34,21 @@ def test_linear(M, N, K, bias, stride):
     assert off.max() <= 0, f"over by {off.max():.3g}"
 
 
+@pytest.mark.parametrize("M,N,K", [(64, 72, 1152), (65, 72, 1152),
+                                   (129, 2056, 2048), (300, 3080, 2048)])
+def test_rows_of_a_wider_tensor(M, N, K):
+    """Without a bias, with which the library takes over above 64 rows."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x, w = (torch.randn(r, K + 8, generator=g, device="cuda").to(torch.bfloat16)
+            for r in (M, N))
+    x, w = x[:, :K], w[:, :K].contiguous()
+    want = x.double() @ w.double().t()
+    big = x.double().abs() @ w.double().abs().t()
+    off = (ops.linear(x, w).double() - want).abs() - 2.0 ** -8 * want.abs() \
+        - 2.0 ** -17 * big
+    assert off.max() <= 0, f"over by {off.max():.3g}"
+
+
 def test_what_the_kernels_do_not_take():
     """Types, widths, gradients and shapes that go to the library."""
     for dt, M, N, K in ((torch.float32, 4, 64, 128), (torch.bfloat16, 4, 63, 128),

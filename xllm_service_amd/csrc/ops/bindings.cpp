@@ -58,7 +58,7 @@ int skinny_gemm_splitk(int M, int N, int K);
 void launch_skinny_gemm(unsigned short*, const unsigned short*,
                         const unsigned short*, const unsigned short*, float*,
                         int, int, int, hipStream_t);
-int linear_takes(long M, long N, long K);
+int linear_takes(long M, long N, long K, bool bias);
 void launch_linear(unsigned short*, const unsigned short*,
                    const unsigned short*, const unsigned short*, int, int, int,
                    long, int, hipStream_t);
@@ -420,7 +420,7 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor w,
         bias->dtype() == torch::kBFloat16 && bias->size(0) == w.size(0) &&
         bias->device() == w.device()))) {
     const long M = x.size(0), N = w.size(0), K = w.size(1);
-    const int kind = xllm::linear_takes(M, N, K);
+    const int kind = xllm::linear_takes(M, N, K, bias.has_value());
     if (kind != 0 &&
         !(M > 48 && !bias.has_value() && tuned(M, N, K, x.stride(0)))) {
       c10::OptionalDeviceGuard guard(x.device());

@@ -173,8 +173,7 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
 template <int S>
 __global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
-    const unsigned short* __restrict__ w,
-    const unsigned short* __restrict__ bias, const int M, const int N,
+    const unsigned short* __restrict__ w, const int M, const int N,
     const int K, const long x_stride, const int n_tiles_n) {
   constexpr int HALF = 64 * LN_K, TILE = 2 * HALF;
   __shared__ __attribute__((aligned(1024))) unsigned short lds[S * TILE];
@@ -234,15 +233,9 @@ __global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
   constexpr int ROW = 64 + 8;                    // bf16 of a row, padded
 #pragma unroll
   for (int r = 0; r < 16; r += 4) {
-    float s[4];
-    const long n = n0 + wn * 32 + 2 * r + 4 * h;
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-      s[k] = acc[r + k] + (bias != nullptr && n + k < N
-                               ? bf16_to_f32(bias[n + k]) : 0.0f);
     uint2 o;
-    o.x = pack_bf16(s[0], s[1]);
-    o.y = pack_bf16(s[2], s[3]);
+    o.x = pack_bf16(acc[r], acc[r + 1]);
+    o.y = pack_bf16(acc[r + 2], acc[r + 3]);
     *reinterpret_cast<uint2*>(lds + (wm * 32 + c32) * ROW + wn * 32 + 2 * r +
                               4 * h) = o;
   }
@@ -272,14 +265,18 @@ __global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
 //            16 | 10.7, 2048 x 4096 18.8-20.4 | 12.8-15.9, 2560 x 4096 19 | 13; 1024 x
 //            1024 and 3072 x 4096 are still faster here
 //   M 16     32000 x 4096 as above, 128256 x 4096 193 | 189 (tuned 178); 8 177 | 188
+// With a bias the library chooses among other kernels, which are faster from 65 rows
+// on, here | library: 96 x 2048 x 2048 11.8 | 6.9, 128 x 2048 x 1536 9.9 | 6.3, 300 x
+// 4096 x 2048 16.1 | 13.6, 96 x 4608 x 3584 18.2 | 16.5, 512 x 3072 x 2048 16.5 | 13.6.
 // A tuned choice of the library is preferred above 48 rows (linear in bindings.cpp):
 //   4096 x 4096, here | tuned | not   M 48 12.6 | 13.7 | 13.7, 64 14.5 | 13.6 | 15.1,
 //            96 19.6 | 17.2 | 22.0, 128 21.4 | 16.9 | 24.5
-int linear_takes(long M, long N, long K) {
+int linear_takes(long M, long N, long K, bool bias) {
   if (M <= 0 || K < LN_K || K % LN_K != 0 || N % 8 != 0) return 0;
   if (N * K >= (1L << 31) || M * K >= (1L << 30)) return 0;
   if (M <= 16) return M <= 8 || N * K <= 1L << 28 ? 1 : 0;
   if (M <= 64) return N * K <= 4096L * 4096 ? 1 : 0;
+  if (bias) return 0;
   const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
   // few tiles with long rows leave most of the chip waiting for their chain
   if (tiles <= 128 && ((K > 2048 && N < 3072) || (K > 1024 && N < 2048))) return 0;
@@ -305,10 +302,10 @@ void launch_linear(unsigned short* y, const unsigned short* x,
   const int tn = (N + 63) / 64, tm = (M + 63) / 64;
   if (tn * tm <= 256)
     hipLaunchKernelGGL((linear_tile_kernel<4>), dim3(tn * tm), dim3(256), 0,
-                       stream, y, x, w, bias, M, N, K, x_stride, tn);
+                       stream, y, x, w, M, N, K, x_stride, tn);
   else
     hipLaunchKernelGGL((linear_tile_kernel<2>), dim3(tn * tm), dim3(256), 0,
-                       stream, y, x, w, bias, M, N, K, x_stride, tn);
+                       stream, y, x, w, M, N, K, x_stride, tn);
 }
 
 }  // namespace xllm

@@ -260,6 +260,19 @@ def test_skinny_gemm(dev, M, N, K):
                   label=f"skinny {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,rows", [(33, 64), (65, 128), (129, 256)])
+def test_skinny_gemm_workspace(dev, M, rows):
+    """The kernel writes partial results of whole groups of row tiles, six of them
+    for 1536 entries: all have room."""
+    a, b = (torch.ones(r, 1536, device=dev, dtype=torch.bfloat16)
+            for r in (M, 512))
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    assert (ops.skinny_gemm(a, b) == 1536).all()
+    assert torch.cuda.max_memory_allocated() - base >= 6 * rows * 512 * 4
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (64, 6144, 4096),
                                    (64, 4096, 4096), (64, 28672, 4096),
                                    (64, 4096, 14336), (33, 512, 1536),

@@ -55,6 +55,7 @@ void launch_mfma_gemm(unsigned short*, const unsigned short*,
                       const unsigned short*, const unsigned short*, int, int,
                       int, hipStream_t);
 int skinny_gemm_splitk(int M, int N, int K);
+int skinny_gemm_rows(int M);
 void launch_skinny_gemm(unsigned short*, const unsigned short*,
                         const unsigned short*, const unsigned short*, float*,
                         int, int, int, hipStream_t);
@@ -350,7 +351,7 @@ torch::Tensor skinny_gemm(torch::Tensor a, torch::Tensor b,
   TORCH_CHECK(K % 64 == 0 && N % 4 == 0);
   auto c = torch::empty({M, N}, a.options());
   const int SK = xllm::skinny_gemm_splitk(M, N, K);
-  const long mpad = ((M + 15) / 16) * 16;
+  const long mpad = xllm::skinny_gemm_rows(M);   // rows of a partial result
   torch::Tensor ws;
   if (SK > 1)
     ws = torch::empty({(long)SK * mpad * N}, a.options().dtype(torch::kFloat));

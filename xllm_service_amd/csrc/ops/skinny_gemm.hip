@@ -36,6 +36,8 @@ static inline int skinny_gemm_mt(int M) {
   return 16;
 }
 
+int skinny_gemm_rows(int M) { return 16 * skinny_gemm_mt(M); }
+
 static inline int skinny_gemm_strips(int MT) {  // n-strips per wave
   const int s = 16 / MT;
   return s > 8 ? 8 : s;      // cap: 16 strips of B double-buffer spills
@@ -59,7 +61,7 @@ int skinny_gemm_splitk(int M, int N, int K) {
 
 template <int MT, bool DIRECT>  // DIRECT: write bf16 C, add bias inline
 __global__ __launch_bounds__(256) void skinny_gemm_kernel(
-    float* __restrict__ ws,                // [SK, 64, N] fp32 partials
+    float* __restrict__ ws,                // [SK, 16 MT, N] fp32 partials
     unsigned short* __restrict__ c,        // [M, N] bf16 (DIRECT only)
     const unsigned short* __restrict__ a,  // [M, K] bf16
     const unsigned short* __restrict__ w,  // [N, K] bf16

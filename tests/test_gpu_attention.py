@@ -390,3 +390,22 @@ def test_options(dim, bf16_out, lens, ctx, kv_heads, per, decode, opts):
                                          else 0.0)
         assert over.max() <= 1e-6, f"off by {off.max():.3g}"
         assert (wide[:, heads * dim:] == 7.0).all()
+
+
+@pytest.mark.parametrize("seqs,kv_heads,per,keys,width", [
+    (191, 4, 2, 70, 512), (192, 4, 2, 70, 512),      # parts | whole
+    (191, 4, 2, 250, 16), (192, 4, 2, 250, 16), (192, 4, 2, 250, 17),  # waves
+    (3, 2, 8, 32, 2), (3, 2, 8, 33, 3)])
+def test_decode_forms(seqs, kv_heads, per, keys, width):
+    """Both sides of the lines between parts and waves of 128-wide heads."""
+    lens, ctx, scale = [1] * seqs, [(keys * (i + 1)) // seqs - 1 if keys > 40
+                                    else keys - 1 for i in range(seqs)], 0.088
+    ctx = [max(c, 0) for c in ctx]
+    rows, k, v, table = make(lens, ctx, kv_heads, per, 128, 35)
+    wide = torch.zeros(seqs, max(width, table.shape[1]), dtype=torch.int32)
+    wide[:, :table.shape[1]] = table
+    q = rows[:, :kv_heads * per * 128].unflatten(-1, (kv_heads * per, 128))
+    sl = torch.tensor(ctx, dtype=torch.int32) + 1
+    got = ops.paged_attn_decode(q.cuda(), k.cuda(), v.cuda(), wide.cuda(),
+                                sl.cuda(), scale)
+    check(got, *want(q, k, v, table, lens, ctx, scale))

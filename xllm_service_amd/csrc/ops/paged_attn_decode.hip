@@ -136,11 +136,18 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
 // shortest sequences the merge (64 keys 4.7 -> 5.6 us) for what the others gain (200
 // keys 9.3 -> 6.5, 1000 32 -> 7.7); eight waves without a merge would be 4.6, 5.2 and
 // 9.1, 2000 keys 13.9 instead of 7.7.
+//   128-wide heads: two waves only where tables have few tiles, of which four leave
+// waves idle that hold LDS (32 key heads, 32 x 16 keys 10.1 -> 8.4). In wide tables long
+// sequences may be there, which two waves walk more slowly (30 x 0.1-3.6 k, 32 key heads
+// 113 -> 123; 69 x 7.0-7.8 k, 8 key heads 311 -> 336); 16 keys in tables of 4096 stay
+// at 10.3.
 static PagedSplit decode_split(long num_seqs, int n_kv_heads, int D,
                                long max_blocks) {
   const long units = num_seqs * n_kv_heads;
   if (D == 64 && units >= 86) return {1, 1, units >= 768 ? 2 : 4};
-  return paged_stream_split(num_seqs, n_kv_heads, max_blocks);
+  PagedSplit x = paged_stream_split(num_seqs, n_kv_heads, max_blocks);
+  if (max_blocks <= 2 || (units >= 768 && max_blocks <= 16)) x.waves = 2;
+  return x;
 }
 // Tables of a page or of a few, one or two query heads per key head: the shuffle
 // kernel, whose chain is shorter. One page, 12 heads x 16 sequences 3.4-4.5 | 4.3 us,

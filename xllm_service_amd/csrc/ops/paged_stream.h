@@ -109,9 +109,9 @@ XLLM_DEV void pa_rows(const unsigned (&at)[D / 16], bf16x8 (&k)[D / 16]) {
 // by 32 waves a row 0.00186; with two 0.00166, which is the rounding to bf16. Us,
 // one term | two by a product of their own | here: 1 x 776 keys 9.0 | 9.6 | 9.5,
 // 24 x 0.6-1.4 k 18.9 | 19.6 | 19.1, 128 x 1-2 k 142.5 | 142.8 | 142.0.
-//   NW: waves of a workgroup, four but where the 64-wide form asks for two.
+//   NW: waves of a workgroup, four but where the host asks for two.
 template <int D, int TERMS, bool MORE, int NW>
-__global__ __launch_bounds__(NW * 64, NW == 2 ? 8 : 2) void
+__global__ __launch_bounds__(NW * 64, NW == 2 && D == 64 ? 8 : 2) void
 paged_attn_stream_kernel(
     void* __restrict__ out,                  // [S, n_qheads, D]
     float* __restrict__ ws_o,                // [S*n_qheads][P][D] (P > 1)
@@ -411,7 +411,12 @@ paged_attn_stream_kernel(
 // 173 | 142, 48 x 0.3-8 k 184 | 159, 32 x 0.3-6 k 83.3 | 82.4, 16 x 0.3-2 k 20.3
 // | 20.3. The host sees no lengths, and in a captured step the widest table there can
 // be: whole below 3000 keys, and up to 128 pairs (which bring the least bytes to
-// hide a chain behind) above, up to 4096 for more pairs.
+// hide a chain behind) above, up to 4096 for more pairs. From 768 pairs
+// on they are whole in any table: idle parts and the merge cost short sequences up to
+// twice their time (tables of 8192, 8 key heads, 128 x 16 keys 12.3 whole | 18.1, x 64
+// 15.4 | 19.2; 32 key heads, 256 x 16 65 | 113), and neither even nor uneven lengths
+// gain by parts there. 512 to 767 pairs do: 8 key heads, 66 x 3.6-7.3 k 232 | 212, 32
+// key heads, 22 x 0.2-8.7 k 277 | 241, against 64 x 16 keys 7.9 | 10.9, x 200 15.5 | 16.7.
 //   With options (a window, a cap, a sink) weights have 32 bits and a tile is longer,
 // with a cap about twice as long: four tiles a part instead of eight (8 key heads, a
 // window of 512 11.7 -> 10.3, 300 keys in tables of 4096 9.8 -> 8.6), and for capped
@@ -435,7 +440,7 @@ inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
     return {p < 3 ? 1 : (int)p, per};
   }
   if (units == 0 || tiles < 96 || (units > 128 && !capped && tiles <= 128) ||
-      (units >= 512 && capped))
+      (capped && units >= 512) || (!options && units >= 768))
     return {1, per};
   return {(int)std::min<long>(8 / f, (tiles + 31) / 32), per};
 }
@@ -458,7 +463,7 @@ inline void paged_stream(void* out, float* ws_o, float* ws_ml,
                      v_cache, block_tables, seq_lens, scale, n_qheads / n_kv,  \
                      n_kv, max_blocks, q_stride, out_stride, split.parts,      \
                      split.per, x)
-  if constexpr (D == 64 && !MORE) {
+  if constexpr (!MORE) {
     if (split.waves == 2) PS_GO(2);
     else PS_GO(4);
   } else {

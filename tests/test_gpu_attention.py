@@ -392,6 +392,18 @@ def test_options(dim, bf16_out, lens, ctx, kv_heads, per, decode, opts):
         assert (wide[:, heads * dim:] == 7.0).all()
 
 
+def test_prefill_without_prompts():
+    """cu_q of one entry, or of none, names no rows: out stays as it is."""
+    rows, k, v, table = make([300], [0], 1, 4, 128, 34)
+    q = rows[:, :512].unflatten(-1, (4, 128)).cuda()
+    for n in (1, 0):
+        empty = torch.zeros(n, dtype=torch.int32, device="cuda")
+        out = torch.full_like(q, 7.0)
+        ops.paged_attn_prefill(q, k.cuda(), v.cuda(), table[:0].cuda(), empty,
+                               empty[:0], 0.1, out=out)
+        assert (out == 7.0).all()
+
+
 @pytest.mark.parametrize("seqs,kv_heads,per,keys,width", [
     (191, 4, 2, 70, 512), (192, 4, 2, 70, 512),      # parts | whole
     (191, 4, 2, 250, 16), (192, 4, 2, 250, 16), (192, 4, 2, 250, 17),  # waves

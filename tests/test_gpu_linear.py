@@ -34,6 +34,15 @@ def test_linear(M, N, K, bias, stride):
     assert off.max() <= 0, f"over by {off.max():.3g}"
 
 
+@pytest.mark.parametrize("M", [8, 9, 16, 17, 24, 25, 32, 48, 49])
+@pytest.mark.parametrize("N,K", [(4096, 128), (4112, 640), (6152, 1152),
+                                 (8200, 256), (8200, 4096)])
+def test_rows_in_steps_of_eight(M, N, K):
+    """One and two row tiles of W, with and without a CU for each workgroup;
+    fewer steps than waves."""
+    test_linear(M, N, K, True, 8)
+
+
 @pytest.mark.parametrize("M,N,K", [(64, 72, 1152), (65, 72, 1152),
                                    (129, 2056, 2048), (300, 3080, 2048)])
 def test_rows_of_a_wider_tensor(M, N, K):

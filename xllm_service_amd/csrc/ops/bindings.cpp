@@ -423,7 +423,8 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor w,
     const long M = x.size(0), N = w.size(0), K = w.size(1);
     const int kind = xllm::linear_takes(M, N, K, bias.has_value());
     if (kind != 0 &&
-        !(M > 48 && !bias.has_value() && tuned(M, N, K, x.stride(0)))) {
+        !(M > (N > 8192 ? 32 : 48) && !bias.has_value() &&
+          tuned(M, N, K, x.stride(0)))) {
       c10::OptionalDeviceGuard guard(x.device());
       auto y = torch::empty({M, N}, x.options());
       xllm::launch_linear(u16(y), u16c(x), u16c(w),

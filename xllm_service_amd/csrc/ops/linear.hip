@@ -72,78 +72,116 @@ struct LnTile {
 };
 
 // ---- decode batches: a stream over W -------------------------------------------
-// A workgroup owns 16 rows of W and up to 16 MT rows of x (16x16x32 products);
-// its NW waves take the steps of K in turn, each through tiles of its own and
-// without a barrier. The sums of the waves meet in LDS. Sixteen rows and not
-// more, because the projections of a layer have few thousand of them: N = 4096
-// fills the 256 CUs once, and what a CU moves besides W, the rows of x, comes
-// from L2.
-template <int MT, int NW>
+// A workgroup owns 16 NT rows of W and XR rows of x (16x16x32 products); its NW
+// waves take the steps of K in turn, each through a ring of D tiles of its own and
+// without a barrier. The sums of the waves meet in LDS.
+//   What bounds it: W from memory (a kernel that only reads takes 7.0 us for 32 MB,
+// 12.4 for 64, 47 for 256), and beside it the rows of x, which every workgroup
+// fetches from L2: 24 of them weigh as much as 24 rows of W. So no more rows of x
+// are loaded than there are (in steps of eight), and two row tiles of W share them
+// where that leaves a workgroup for most CUs. Workgroups start at different
+// steps, so that not all ask for the same columns of x at a time. Us, N x K, before
+// (16 rows of W, 16 or 32 of x, one tile a wave) -> here:
+//   M 8   4096 x 4096 8.7 -> 7.7, 6144 x 4096 12.7 -> 10.7, 8192 x 4096 14.9 -> 12.8
+//   M 24  4096 x 4096 10.1 -> 9.1, 6144 x 4096 15.2 -> 12.4, 8192 x 4096 16.9 -> 14.3,
+//         32000 x 4096 57 -> 48, 4096 x 14336 27.5 -> 25.3
+//   M 64  4096 x 4096 14.4 -> 13.2, 6144 x 4096 22.0 -> 17.2, 8192 x 4096 23.5 -> 18.5
+template <int NT, int XR, int NW, int D>
 __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w,
     const unsigned short* __restrict__ bias, const int M, const int N,
     const int K, const long x_stride) {
-  constexpr int T = 16 * LN_K, TILE = T * (1 + MT);
-  constexpr int ROW = 20;                        // fp32 of a part's row, padded
+  constexpr int WR = 16 * NT;                    // rows of W
+  constexpr int MT = (XR + 15) / 16;             // row tiles of x
+  constexpr int T = WR * LN_K, TILE = T + XR * LN_K;
+  constexpr int ROW = WR + 4;                    // fp32 of a part's row, padded
   constexpr int PART = NW * 16 * MT * ROW * 2;
+  constexpr int RING = NW * D * TILE;
   __shared__ __attribute__((aligned(1024))) unsigned short
-      lds[NW * TILE > PART ? NW * TILE : PART];
+      lds[RING > PART ? RING : PART];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
-  const long n0 = blockIdx.x * 16L;
-  unsigned short* wt = lds + wid * TILE;
-  unsigned short* xt = wt + T;
-  LnTile<16> lw;
-  LnTile<16 * MT> lx;
+  const long n0 = blockIdx.x * (long)WR;
+  unsigned short* wt = lds + wid * (D * TILE);
+  LnTile<WR> lw;
+  LnTile<XR> lx;
   lw.init(n0, N, K, lane);
   lx.init(0, M, x_stride, lane);
   const unsigned short* wp = w + n0 * K;
-  unsigned at[4];                                // chunk 4 ks + g of row c16
+  // bytes of chunk 4 ks + g of row c16; a last tile of eight rows is read twice
+  const unsigned base = (unsigned)(unsigned long long)(const lds_u16*)wt;
+  const int half = XR % 16 != 0 ? c16 & 7 : c16;
+  unsigned at[4], last[4];
 #pragma unroll
-  for (int ks = 0; ks < 4; ks++)
-    at[ks] = (unsigned)(unsigned long long)(const lds_u16*)wt +
-             2 * (c16 * LN_K + (((4 * ks + g) ^ c16) << 3));
-  f32x4 acc[MT];
-#pragma unroll
-  for (int j = 0; j < MT; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int steps = K / LN_K;
-  if (wid < steps) {
-    lw.load(wp + wid * LN_K, wt);
-    lx.load(x + wid * LN_K, xt);
+  for (int ks = 0; ks < 4; ks++) {
+    at[ks] = 2 * (c16 * LN_K + (((4 * ks + g) ^ c16) << 3));
+    last[ks] = 2 * (half * LN_K + (((4 * ks + g) ^ half) << 3));
   }
-  for (int t = wid; t < steps; t += NW) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    bf16x8 a[4], b[MT][4];
-    unsigned xat[MT][4];
+  f32x4 acc[NT][MT];
 #pragma unroll
-    for (int j = 0; j < MT; j++)
+  for (int i = 0; i < NT; i++)
 #pragma unroll
-      for (int ks = 0; ks < 4; ks++) xat[j][ks] = at[ks] + (1 + j) * (2 * T);
-    ln_read2(at, xat[0], a, b[0]);
-    if (t + NW < steps) lw.load(wp + (t + NW) * LN_K, wt);
+    for (int j = 0; j < MT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = K / LN_K, turn = blockIdx.x % steps;
+  const int mine = (steps - wid + NW - 1) / NW;  // of this wave
+  auto load = [&](int i, int slot) {
+    int t = wid + i * NW + turn;
+    t = (t >= steps ? t - steps : t) * LN_K;
+    lw.load(wp + t, wt + slot * TILE);
+    lx.load(x + t, wt + slot * TILE + T);
+  };
 #pragma unroll
-    for (int j = 1; j < MT; j++) ln_read(xat[j], b[j]);
-    if (t + NW < steps) lx.load(x + (t + NW) * LN_K, xt);
+  for (int d = 0; d < D; d++)
+    if (d < mine) load(d, d);
+  for (int i = 0, slot = 0; i < mine; i++, slot = slot + 1 == D ? 0 : slot + 1) {
+    if (D == 2 && i + 1 < mine)                  // the next tile may be on the way
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((WR + XR) / 4) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    constexpr int TILES = NT + MT;               // row tiles of W, then of x
+    bf16x8 v[TILES][4];
+    auto rows = [&](int r, unsigned (&to)[4]) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++)
+        to[ks] = base + slot * (2 * TILE) + r * (2 * 16 * LN_K) +
+                 (r == TILES - 1 ? last[ks] : at[ks]);
+    };
+    unsigned r0[4], r1[4];
+#pragma unroll
+    for (int r = 0; r + 1 < TILES; r += 2) {
+      rows(r, r0);
+      rows(r + 1, r1);
+      ln_read2(r0, r1, v[r], v[r + 1]);
+    }
+    if constexpr (TILES % 2 != 0) {
+      rows(TILES - 1, r0);
+      ln_read(r0, v[TILES - 1]);
+    }
+    if (i + D < mine) load(i + D, slot);
 #pragma unroll
     for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-      for (int j = 0; j < MT; j++)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks], b[j][ks],
-                                                         acc[j], 0, 0, 0);
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+          acc[n][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              v[n][ks], v[NT + j][ks], acc[n][j], 0, 0, 0);
   }
-  // acc[j][r] = y[m = 16 j + c16][n = 4 g + r]
+  // acc[n][j][r] = y[m = 16 j + c16][16 n + 4 g + r]
   __syncthreads();
   float* part = reinterpret_cast<float*>(lds);   // [NW][16 MT][ROW]
 #pragma unroll
-  for (int j = 0; j < MT; j++)
-    *reinterpret_cast<float4*>(part + ((wid * MT + j) * 16 + c16) * ROW +
-                               4 * g) =
-        make_float4(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
+  for (int n = 0; n < NT; n++)
+#pragma unroll
+    for (int j = 0; j < MT; j++)
+      *reinterpret_cast<float4*>(part + ((wid * MT + j) * 16 + c16) * ROW +
+                                 16 * n + 4 * g) =
+          make_float4(acc[n][j][0], acc[n][j][1], acc[n][j][2], acc[n][j][3]);
   __syncthreads();
-  for (int i = tid; i < 16 * MT * 4; i += NW * 64) {
-    const int m = i >> 2, col = (i & 3) * 4;
+  constexpr int C4 = WR / 4;                     // columns in fours
+  for (int i = tid; i < 16 * MT * C4; i += NW * 64) {
+    const int m = i / C4, col = (i % C4) * 4;
     const long n = n0 + col;
     if (m >= M || n >= N) continue;
     float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -252,11 +290,18 @@ __global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
 // 0: the library's; 1: stream; 2: tiles. Besides its time on the GPU a library
 // call costs 28 us of host time (its choice of a kernel), these cost 6.
 // Measured, us on the GPU, here | library, weights from memory (N x K):
-//   M 1-8    2048 x 2048 4.2 | 8.3, 4096 x 4096 8.5 | 14.5, 8192 x 4096 15.1 |
-//            17, 4096 x 14336 24 | 26, 28672 x 4096 42 | 61, 32000 x 4096 46 | 58
-//   M 24-32  2048 x 2048 5.0 | 8.6, 4096 x 4096 10.5 | 12.7, 6144 x 4096 16.5 |
-//            16, 8192 x 4096 19 | 17.5: x rows weigh as much as W from here on
-//   M 64     4096 x 2048 9.9 | 12.4, 4096 x 4096 14.2 | 14.6, 6144 x 4096 22 | 18
+//   M 8      2048 x 2048 4.1 | 8.9, 4096 x 4096 7.7 | 15.3, 4096 x 14336 21 | 25, 28672 x
+//            4096 39 | 60, 32000 x 4096 44 | 57
+//   M 16     32000 x 4096 48 | 57; 128256 x 4096, another kernel, 193 | 189
+//   M 24-32  512 x 14336 20.4 | 18.1, 23.1 | 24.5; 4096 x 4096 9.1-10 | 13.2, 8192 x 4096
+//            14.4-15 | 16, 14336 x 4096 24.5-26.1 | 25.6, 32000 x 4096 48.4-50.6 | 62;
+//            12288 x 8192 45-46.5 | 41
+//   M 48     4096 x 4096 11.8 | 13.6, 8192 x 4096 16.9 | 17.9, 14336 x 4096 28.4 | 26.2,
+//            28672 x 4096 53 | 60, 14336 x 2048 16.4 | 16.8; 512 x 8192 12.7 | 9.7, 2048 x
+//            8192 17.9 | 15.1, 6144 x 14336 47 | 52
+//   M 64     4096 x 4096 13.2 | 14.9, 8192 x 4096 18.5 | 18.9, 12288 x 4096 31.4 | 24.7, 12288
+//            x 2048 18.8 | 16.1; 1024 x 8192 20 | 13.6, 4096 x 8192 22.7 | 23.9, 6144 x
+//            8192 30 | 29.3, 4096 x 14336 38.8 | 38.8
 //   M 96-192 4096 x 2048 12 | 14-21, 4096 x 4096 20 | 21-31, 4096 x 14336 60-68
 //            | 50-104 (tuned 50)
 //   M 300    2048 x 2048 10.8 | 10.5, 4096 x 2048 16.6 | 15.7, 4096 x 4096 29 | 25
@@ -264,18 +309,27 @@ __global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
 //   M 96-256, few tiles   512 x 4096 17.7 | 8.8-12, 1024 x 2048 10.5 | 8.4, 1536 x 3072
 //            16 | 10.7, 2048 x 4096 18.8-20.4 | 12.8-15.9, 2560 x 4096 19 | 13; 1024 x
 //            1024 and 3072 x 4096 are still faster here
-//   M 16     32000 x 4096 as above, 128256 x 4096 193 | 189 (tuned 178); 8 177 | 188
 // With a bias the library chooses among other kernels, which are faster from 65 rows
 // on, here | library: 96 x 2048 x 2048 11.8 | 6.9, 128 x 2048 x 1536 9.9 | 6.3, 300 x
 // 4096 x 2048 16.1 | 13.6, 96 x 4608 x 3584 18.2 | 16.5, 512 x 3072 x 2048 16.5 | 13.6.
-// A tuned choice of the library is preferred above 48 rows (linear in bindings.cpp):
-//   4096 x 4096, here | tuned | not   M 48 12.6 | 13.7 | 13.7, 64 14.5 | 13.6 | 15.1,
+// A tuned choice of the library is preferred above 48 rows, above 32 where N > 8192
+// (linear in bindings.cpp): M 32, 28672 x 4096 48.9 | 48.2, M 48 53.5 | 49.3 | 60.5 not,
+//   4096 x 4096, here | tuned | not   M 48 11.8 | 13.7 | 13.7, 64 13.2 | 13.6 | 15.1,
 //            96 19.6 | 17.2 | 22.0, 128 21.4 | 16.9 | 24.5
 int linear_takes(long M, long N, long K, bool bias) {
   if (M <= 0 || K < LN_K || K % LN_K != 0 || N % 8 != 0) return 0;
   if (N * K >= (1L << 31) || M * K >= (1L << 30)) return 0;
   if (M <= 16) return M <= 8 || N * K <= 1L << 28 ? 1 : 0;
-  if (M <= 64) return N * K <= 4096L * 4096 ? 1 : 0;
+  // few workgroups with long rows
+  if (M <= 32)
+    return (N > 1024 || K <= 8192) &&
+           (N <= 8192 || (K <= 4096 && N * K <= 1L << 28)) ? 1 : 0;
+  if (M <= 48)
+    return N <= 8192 ? (N > 2048 || K < 8192 ? 1 : 0)
+                     : N * K <= 1L << 28 &&
+                       (K <= 2048 || (K <= 4096 && N >= 18432)) ? 1 : 0;
+  if (M <= 64)
+    return N <= 8192 && (K <= 4096 || (N >= 2048 && N <= 4096 && K <= 8192)) ? 1 : 0;
   if (bias) return 0;
   const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
   // few tiles with long rows leave most of the chip waiting for their chain
@@ -283,20 +337,53 @@ int linear_takes(long M, long N, long K, bool bias) {
   return K <= 4096 && (tiles <= 256 || (tiles <= 512 && K <= 2048)) ? 2 : 0;
 }
 
+// Row tiles of W: one up to 4096 rows of it, one workgroup a CU then; two above.
+// Up to 16 rows of x weigh little, and where W has many columns and its row
+// tiles leave few CUs without one in the last turn, one tile is the better again:
+// M 8, 8192 x 4096 12.8 one | 13.5 two, 12288 x 4096 17.9 | 19.9, 8192 x 8192 26.2 |
+// 29.8; but 4608 x 4096 10.5 | 9.4 (a ninth of the CUs have two), 14336 x 4096
+// 22.2 | 21.1, 8192 x 2048 9.1 | 8.0; M 24, 8192 x 4096 15.6 | 14.4.
+static bool linear_one_tile(int M, int N, int K) {
+  const int wgs = (N + 15) / 16;
+  return wgs <= 256 ||
+         (M <= 16 && K >= 4096 && 10 * wgs >= 9 * ((wgs + 255) / 256 * 256));
+}
+// A workgroup that has a CU to itself takes all of its LDS: two tiles a wave, or
+// more waves. Where there are more than CUs, two of them share one: M 24, 32000 x
+// 4096 48.4, with two tiles 49.2; 18944 x 4096 33.4 | 34.5.
+static void launch_stream(unsigned short* y, const unsigned short* x,
+                          const unsigned short* w, const unsigned short* bias,
+                          int M, int N, int K, long x_stride,
+                          hipStream_t stream) {
+  const bool one = linear_one_tile(M, N, K);
+  const dim3 grid((N + (one ? 15 : 31)) / (one ? 16 : 32));
+  const bool few = grid.x <= 256;
+#define LN_STREAM(NT, XR, NW, D)                                               \
+  hipLaunchKernelGGL((linear_stream_kernel<NT, XR, NW, D>), grid,              \
+                     dim3(NW * 64), 0, stream, y, x, w, bias, M, N, K, x_stride)
+  if (one) {
+    if (M <= 8) LN_STREAM(1, 8, 4, 2);
+    else if (M <= 16) LN_STREAM(1, 16, 4, 2);
+    else if (M <= 24) LN_STREAM(1, 24, 4, 2);
+    else if (M <= 32) LN_STREAM(1, 32, 4, 2);
+    else if (M <= 48) LN_STREAM(1, 48, 4, 2);
+    else LN_STREAM(1, 64, 4, 2);
+  } else {
+    if (M <= 8) LN_STREAM(2, 8, 4, 2);
+    else if (M <= 16) { if (few) LN_STREAM(2, 16, 4, 2); else LN_STREAM(2, 16, 2, 2); }
+    else if (M <= 24) { if (few) LN_STREAM(2, 24, 4, 2); else LN_STREAM(2, 24, 4, 1); }
+    else if (M <= 32) { if (few) LN_STREAM(2, 32, 4, 2); else LN_STREAM(2, 32, 4, 1); }
+    else if (M <= 48) { if (few) LN_STREAM(2, 48, 7, 1); else LN_STREAM(2, 48, 4, 1); }
+    else LN_STREAM(2, 64, 6, 1);
+  }
+#undef LN_STREAM
+}
+
 void launch_linear(unsigned short* y, const unsigned short* x,
                    const unsigned short* w, const unsigned short* bias, int M,
                    int N, int K, long x_stride, int kind, hipStream_t stream) {
   if (kind == 1) {
-    const dim3 grid((N + 15) / 16);
-    const bool few = grid.x <= 256;              // a CU each
-#define LN_STREAM(MT, NW)                                                      \
-  hipLaunchKernelGGL((linear_stream_kernel<MT, NW>), grid, dim3(NW * 64), 0,   \
-                     stream, y, x, w, bias, M, N, K, x_stride)
-    if (M <= 16) LN_STREAM(1, 8);
-    else if (M <= 32) { if (few) LN_STREAM(2, 8); else LN_STREAM(2, 4); }
-    else if (M <= 48) { if (few) LN_STREAM(3, 8); else LN_STREAM(3, 4); }
-    else LN_STREAM(4, 4);
-#undef LN_STREAM
+    launch_stream(y, x, w, bias, M, N, K, x_stride, stream);
     return;
   }
   const int tn = (N + 63) / 64, tm = (M + 63) / 64;

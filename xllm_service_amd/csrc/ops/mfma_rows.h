@@ -48,6 +48,12 @@ XLLM_DEV unsigned pack_bf16(float a, float b) {
   const bfx2 x = __builtin_convertvector(f, bfx2);
   return __builtin_bit_cast(unsigned, x);
 }
+// c + both of a packed pair
+XLLM_DEV float sum_bf16(unsigned u, float c) {
+  const bfx2 one = {(__bf16)1.0f, (__bf16)1.0f};
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bfx2, u), one, c,
+                                         false);
+}
 // a, b <- what the packed pair leaves of them (exact)
 XLLM_DEV void drop_bf16(float& a, float& b, unsigned u) {
   a -= __uint_as_float(u << 16);
@@ -89,6 +95,25 @@ template <int W> XLLM_DEV bf16x8 mr_cols(const lds_u16* p) {
   const s16x4 hi =
       __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * W));
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// The same where the caller has waited for what it reads: through a pointer without
+// alias information the compiler waits for all loads to LDS first.
+template <int W>
+XLLM_DEV bf16x8 mr_cols_own(const lds_u16* __restrict__ p) {
+  return mr_cols<W>(p);
+}
+// `bytes` of memory for loads to LDS. Those through global addresses are flat
+// instructions to the compiler, which from then on lets no LDS read pass another:
+// every use of one waits for all.
+XLLM_DEV __amdgpu_buffer_rsrc_t mr_buffer(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes,
+                                           0x00020000);
+}
+// 16 bytes per lane, in lane order from dst on; zeros from out of the bounds
+XLLM_DEV void mr_to_lds(__amdgpu_buffer_rsrc_t src, unsigned off,
+                        unsigned short* dst) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void*)dst, 16, off, 0, 0,
+                                           0);
 }
 XLLM_DEV f32x16 mr_zero() {
   f32x16 z;

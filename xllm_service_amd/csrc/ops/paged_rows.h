@@ -34,13 +34,16 @@
 // Bound by the matrix pipe and the vector unit in turn: a tile costs a wave
 // 32 products (about 1000 cycles) and about as many cycles of exponentials,
 // maxima and conversions, which the second wave of the SIMD overlaps; LDS
-// reads feed 32 rows each and stay just below the pipe's rate. Measured, 4
-// prompts of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads: 371 us,
-// 873 TFLOP/s (a large bf16 matrix product: 1466); one head and 16 rows per
-// wave on 16x16x32 products, P through LDS: 1209 us. 3 chunks of 93-261 tokens
-// over 0.5-1.8 k, 28 heads, with the key split: 31 us, without a list of tiles
-// made on the host; before: 110 us and 48 us of copies and waiting. 8 prompts
-// of 109-438 tokens, 12 heads of 64: 13.6 us, an eager loop before: 14 ms.
+// reads feed 32 rows each and stay just below the pipe's rate. Loads to LDS go
+// through buffers: after those through global addresses, which are flat
+// instructions to the compiler, every use of an LDS read waited for all reads in
+// flight, and the first transpose read for the next tile too. With that and
+// three steps of K on the way ahead of their products, before -> after: 4 prompts
+// of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads 366 -> 354 us,
+// 3 chunks of 93-261 tokens over 0.5-1.8 k, 28 heads, keys split 30.9 -> 30.1, 2
+// of 1.8-2.3 k in a window of 1024, three terms 63.3 -> 61.3, 8 prompts of 109-438,
+// 12 heads of 64 13.6. (One head and 16 rows per wave on 16x16x32 products, P
+// through LDS: 1209 us for the first; an eager loop 14 ms for the last.)
 //
 // Fragment layouts, the order of the keys and of the LDS images: mfma_rows.h.
 #pragma once
@@ -188,18 +191,16 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
   auto pages_from = [&](int i) {
     return btab[min(list.at(i + lane) * (PF_KT / PF_BS) + wid, last_blk)];
   };
-  auto put = [&](const char* kp, const char* vp, unsigned ko, unsigned vo,
-                 unsigned short* dst) {
-    __builtin_amdgcn_global_load_lds((glb_void*)(kp + ko), (lds_void*)dst, 16,
-                                     0, 0);
-    __builtin_amdgcn_global_load_lds((glb_void*)(vp + vo),
-                                     (lds_void*)(dst + TILE), 16, 0, 0);
+  auto put = [&](__amdgpu_buffer_rsrc_t kp, __amdgpu_buffer_rsrc_t vp,
+                 unsigned ko, unsigned vo, unsigned short* dst) {
+    mr_to_lds(kp, ko, dst);
+    mr_to_lds(vp, vo, dst + TILE);
   };
   auto stage = [&](int t, int page, int buf) {
     const int pg = t * (PF_KT / PF_BS) + wid;
-    const long base = ((long)page * n_kv + kvh) * (PF_BS * D * 2);
-    const char* kp = reinterpret_cast<const char*>(k_cache) + base;
-    const char* vp = reinterpret_cast<const char*>(v_cache) + base;
+    const long base = ((long)page * n_kv + kvh) * (PF_BS * D);
+    const auto kp = mr_buffer(k_cache + base, PF_BS * D * 2);
+    const auto vp = mr_buffer(v_cache + base, PF_BS * D * 2);
     unsigned short* dst = kv_lds + buf * 2 * TILE + wid * 16 * D;
     if (pg < last_blk) {
 #pragma unroll
@@ -252,6 +253,14 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
                           kt + (kbase ^ (ks << 4)) + i * 32 * D),
                       qf[ks], s[i]);
     }
+    // three steps of K are on the way while one is multiplied
+    __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+    for (int ks = 0; ks < KS - 3; ks++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
     if (MORE && x.cap > 0.0f) paged_cap<2>(s, sc.pre, x.cap);
     // uniform: a tile on the diagonal or on the edge of a window
     if (k0 + PF_KT > wmin || (MORE && k0 < whi)) {
@@ -291,12 +300,13 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
       for (int r = 0; r < 16; r += 2) {
         float a = __builtin_amdgcn_exp2f(fmaf(s[i][r], c, -mc));
         float b = __builtin_amdgcn_exp2f(fmaf(s[i][r + 1], c, -mc));
-        l += a + b;
+        if (TERMS > 1) l += a + b;
 #pragma unroll
         for (int e = 0; e < TERMS; e++) {
           const unsigned u = pack_bf16(a, b);
           reinterpret_cast<unsigned*>(
               &p[e][i * 2 + (r >> 3)])[(r & 7) >> 1] = u;
+          if (TERMS == 1) l = sum_bf16(u, l);
           drop_bf16(a, b, u);
         }
       }
@@ -305,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
     for (int st = 0; st < 4; st++)
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) {
-        const bf16x8 a = mr_cols<D>(vt + (vbase ^ (dt << 5)) + st * 16 * D);
+        const bf16x8 a = mr_cols_own<D>(vt + (vbase ^ (dt << 5)) + st * 16 * D);
 #pragma unroll
         for (int e = 0; e < TERMS; e++)
           o_acc[dt] = mr_mma(a, p[e][st], o_acc[dt]);

@@ -58,6 +58,25 @@ def test_rows_of_a_wider_tensor(M, N, K):
     assert off.max() <= 0, f"over by {off.max():.3g}"
 
 
+@pytest.mark.parametrize("M,N,K,stride", [
+    (65, 64, 128, 0), (97, 136, 256, 8), (128, 3080, 384, 0),    # 32 rows of x
+    (200, 2056, 640, 8), (250, 3080, 1152, 0), (300, 4104, 256, 8),
+    (380, 4040, 128, 0), (500, 3080, 2048, 8),                   # 128 of W
+    (70, 3080, 4736, 0), (2048, 200, 384, 0), (8000, 72, 256, 8)])
+def test_shapes_of_prompt_tiles(M, N, K, stride):
+    """Every shape of a tile, with remainders of both sides and fewer steps than
+    buffers; longest rows. 2^-17 covers K up to 4096, 2^-16.8 up to 4736."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w = (torch.randn(r, K + stride, generator=g, device="cuda").to(
+        torch.bfloat16)[:, :K] for r in (M, N))
+    w = w.contiguous()
+    want = x.double() @ w.double().t()
+    big = x.double().abs() @ w.double().abs().t()
+    off = (ops.linear(x, w).double() - want).abs() - 2.0 ** -8 * want.abs() \
+        - 2.0 ** -16.8 * big
+    assert off.max() <= 0, f"over by {off.max():.3g}"
+
+
 def test_what_the_kernels_do_not_take():
     """Types, widths, gradients and shapes that go to the library."""
     for dt, M, N, K in ((torch.float32, 4, 64, 128), (torch.bfloat16, 4, 63, 128),

@@ -6,23 +6,15 @@
 // both are rows x 128 entries, loaded straight to LDS (global_load_lds, 16 B per
 // lane, 256 B of a row at a time) with the 16 B chunks of a row permuted by the
 // row: whole-row reads then meet no bank twice. W rows are the A operand, x rows
-// the B operand of 32x32x16 products (layouts: mfma_rows.h); sums are fp32.
-//
-// The LDS reads are asm with their wait: in front of a builtin the compiler
-// waits for every load to LDS in flight.
+// the B operand of 16x16x32 products; sums are fp32.
 #include "mfma_rows.h"
 
 namespace xllm {
 
 #define LN_K 128           // entries of a row per step
 
-// bytes into a [rows][128] image of chunk 2 ks + h of a lane's row
-XLLM_DEV void ln_addresses(unsigned base, int row, int h, unsigned (&at)[8]) {
-#pragma unroll
-  for (int ks = 0; ks < 8; ks++)
-    at[ks] = base + 2 * (row * LN_K + (((2 * ks + h) ^ (row & 15)) << 3));
-}
-// four steps of 32 rows
+// Four chunks of a lane's row, with their wait in the same asm: after loads to LDS through
+// global addresses the compiler waits for more than it has to.
 XLLM_DEV void ln_read(const unsigned* at, bf16x8* v) {
   asm volatile(
       "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
@@ -202,88 +194,162 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
   }
 }
 
-// ---- short prompts: 64 x 64 tiles -----------------------------------------------
-// Four waves, a quarter of the tile each; one barrier per step. S buffers: four
-// where a workgroup has a CU to itself (three steps are on the way while one
-// is multiplied: 300 x 2048 x 2048 10.8 us, with two 11.8), two where two share
-// it (300 x 4096 x 2048 16.6 us, with four 21.6). Bound by the chain of a step:
-// LDS reads, their wait, four products on one accumulator.
-template <int S>
-__global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
+// ---- short prompts ---------------------------------------------------------------
+// A workgroup owns 16 NW rows of W and 16 MT of x. Tiles of LK columns go through a
+// ring of S buffers; a wave multiplies 32 rows of W by all of x over one half of a
+// tile's columns, with the operands of the next tile read from LDS meanwhile and one
+// barrier per tile. At the end the waves of the two halves swap a row tile of W.
+//   What bounds it: what a CU pulls from L2, (16 NW + 16 MT) K entries at 70 KB/us with
+// W from memory (98 where it is cached; a loop of loads alone 107-115): without
+// products 300 x 3072 x 2048 takes 10.2 us of 11.6, without the epilogue 10.5. Longer
+// rings and other orders of the columns changed nothing, and rows of 64 B instead of
+// 256, as the products want their operands straight from memory, come at a third of
+// the rate. So the shape that a CU pulls least for is taken (linear_shape), all
+// products run beside the loads, and loads go through buffers: after global ones the
+// compiler lets no LDS read pass another. Us, 64 x 64 tiles of four waves, a quarter
+// of the products each -> here: 300 x 2048 x 2048 11.2 -> 9.4, 4096 x 2048 16.3 -> 13.2,
+// 4096 x 4096 29.5 -> 22.5, 3072 x 2048 11.7 -> 11.6; 96 x 3072 x 2048 10.9 -> 9.6;
+// 192 x 6144 x 4096 30.1 -> 25.7; 512 x 3072 x 2048 16.5 -> 16.7; 256 x 3072 x 2048, as many
+// tiles of 64 x 64 either way, 11.8 -> 12.1.
+template <int NW, int MT, int LK, int S>
+__global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w, const int M, const int N,
     const int K, const long x_stride, const int n_tiles_n) {
-  constexpr int HALF = 64 * LN_K, TILE = 2 * HALF;
+  constexpr int WR = 16 * NW;                    // rows of W
+  constexpr int WT = WR * LK, TILE = WT + 16 * MT * LK;
+  constexpr int KS = LK / 64;                    // products a wave makes of a step
+  constexpr int CPR = LK / 8, RPI = 64 / CPR;    // chunks of a row, rows a load
+  constexpr int WI = 16 / RPI, XI = 16 * MT / (RPI * NW);   // loads of a wave
+  static_assert(XI * RPI * NW == 16 * MT, "");
   __shared__ __attribute__((aligned(1024))) unsigned short lds[S * TILE];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h = lane >> 5, c32 = lane & 31;
-  const long n0 = (blockIdx.x % n_tiles_n) * 64L;
-  const long m0 = (blockIdx.x / n_tiles_n) * 64L;
-  const int wn = wid & 1, wm = wid >> 1;
-  // a wave loads 16 rows of both
-  LnTile<16> lw, lx;
-  const long nr = min(n0 + wid * 16, (long)N - 1);
-  const long mr = min(m0 + wid * 16, (long)M - 1);
-  lw.init(nr, N, K, lane);
-  lx.init(mr, M, x_stride, lane);
-  const unsigned short* wp = w + nr * K;
-  const unsigned short* xp = x + mr * x_stride;
-  unsigned short* mine = lds + wid * 16 * LN_K;
-  unsigned wat[8], xat[8];
-  const unsigned base = (unsigned)(unsigned long long)(const lds_u16*)lds;
-  ln_addresses(base, wn * 32 + c32, h, wat);
-  ln_addresses(base + 2 * HALF, wm * 32 + c32, h, xat);
-  f32x16 acc = mr_zero();
-  const int steps = K / LN_K;
-  auto stage = [&](int t) {                      // eight loads
-    unsigned short* dst = mine + (t & (S - 1)) * TILE;
-    lw.load(wp + t * LN_K, dst);
-    lx.load(xp + t * LN_K, dst + HALF);
+  const int g = lane >> 4, c16 = lane & 15;
+  const long n0 = (blockIdx.x % n_tiles_n) * (long)WR;
+  const long m0 = (blockIdx.x / n_tiles_n) * (16L * MT);
+  const int n_rows = (int)min((long)WR, N - n0);
+  const int m_rows = (int)min(16L * MT, M - m0);
+  const unsigned short* wp = w + n0 * K;
+  const unsigned short* xp = x + m0 * x_stride;
+  const unsigned w_bytes = (unsigned)n_rows * K * 2;
+  const unsigned x_bytes = (unsigned)((m_rows - 1) * x_stride + K) * 2;
+  // a wave loads 16 rows of W and its share of x, RPI at a time; rows past the last
+  // one repeat it: their results go nowhere
+  unsigned w_off[WI], x_off[XI];
+  auto offset = [&](int r, int last, long stride) {
+    const int swz = LK == 128 ? r & 15 : (r >> 1) & 7;
+    return (unsigned)(min(r, last) * stride * 2) +
+           (((lane % CPR) ^ swz) << 4);
   };
-  for (int t = 0; t < min(S - 1, steps); t++) stage(t);
-  for (int t = 0; t < steps; t++) {
-    const int buf = t & (S - 1);
-    // this step has arrived; what was issued later may be on the way
-    if (S == 4 && t + 2 < steps)
-      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-    else if (S == 4 && t + 1 < steps)
-      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    if (t + S - 1 < steps) stage(t + S - 1);
 #pragma unroll
-    for (int k = 0; k < 8; k += 4) {
-      unsigned a_at[4], b_at[4];
+  for (int i = 0; i < WI; i++)
+    w_off[i] = offset((wid * WI + i) * RPI + lane / CPR, n_rows - 1, K);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        a_at[i] = wat[k + i] + buf * (2 * TILE);
-        b_at[i] = xat[k + i] + buf * (2 * TILE);
-      }
-      bf16x8 a[4], b[4];
-      ln_read2(a_at, b_at, a, b);
+  for (int i = 0; i < XI; i++)
+    x_off[i] = offset((wid * XI + i) * RPI + lane / CPR, m_rows - 1, x_stride);
+  const int steps = K / LK;
+  auto stage = [&](int t, int slot) {
+    const bool on = t < steps;                   // past the end: zeros
+    const auto ws = mr_buffer(wp, on ? w_bytes : 0u);
+    const auto xs = mr_buffer(xp, on ? x_bytes : 0u);
+    unsigned short* dst = lds + slot * TILE;
 #pragma unroll
-      for (int i = 0; i < 4; i++) acc = mr_mma(a[i], b[i], acc);
+    for (int i = 0; i < WI; i++)
+      mr_to_lds(ws, w_off[i], dst + (wid * WI + i) * 512, t * (LK * 2));
+#pragma unroll
+    for (int i = 0; i < XI; i++)
+      mr_to_lds(xs, x_off[i], dst + WT + (wid * XI + i) * 512, t * (LK * 2));
+  };
+  // a wave multiplies 32 rows of W by all of x over half of the step's columns
+  const int hw = wid % (NW / 2), hk = wid / (NW / 2);
+  int at[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++)
+    at[ks] = c16 * LK + (((4 * (KS * hk + ks) + g) ^
+                          (LK == 128 ? c16 : c16 >> 1)) << 3);
+  struct Frags { bf16x8 w[KS][2], x[KS][MT]; };
+  auto fetch = [&](Frags& f, int slot) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      const lds_u16* p = (const lds_u16*)lds + slot * TILE + at[ks];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+        f.w[ks][i] =
+            *reinterpret_cast<const lds_bf16x8*>(p + (hw * 2 + i) * 16 * LK);
+#pragma unroll
+      for (int j = 0; j < MT; j++)
+        f.x[ks][j] = *reinterpret_cast<const lds_bf16x8*>(p + WT + j * 16 * LK);
     }
-  }
-  // through LDS to whole rows
-  __syncthreads();
-  constexpr int ROW = 64 + 8;                    // bf16 of a row, padded
+  };
+  f32x4 acc[2][MT];
 #pragma unroll
-  for (int r = 0; r < 16; r += 4) {
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < MT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < S - 1; t++) stage(t, t);
+  // the next step's tile has arrived, those after it may be on the way
+  auto meet = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 3) * (WI + XI)) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * (WI + XI)) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  Frags f[2];
+  fetch(f[0], 0);
+  int slot = 0;
+  auto step = [&](int t, const Frags& now, Frags& next) {
+    meet();
+    stage(t + S - 1, slot == 0 ? S - 1 : slot - 1);
+    slot = slot == S - 1 ? 0 : slot + 1;
+    fetch(next, slot);
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              now.w[ks][i], now.x[ks][j], acc[i][j], 0, 0, 0);
+  };
+  for (int t = 0;;) {
+    step(t, f[0], f[1]);
+    if (++t == steps) break;
+    step(t, f[1], f[0]);
+    if (++t == steps) break;
+  }
+  // acc[i][j][r] = a half of y[m = 16 j + c16][n = 32 hw + 16 i + 4 g + r]. The
+  // waves of the two halves swap a row tile of W, then whole rows go out.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  f32x4* swap = reinterpret_cast<f32x4*>(lds);   // [NW][MT][64]
+#pragma unroll
+  for (int j = 0; j < MT; j++) swap[(wid * MT + j) * 64 + lane] = hk ? acc[0][j] : acc[1][j];
+  __syncthreads();
+  constexpr int ROW = WR + 8;                    // bf16 of a row, padded
+  unsigned short* out = lds + NW * MT * 64 * 8;
+  const int col0 = 32 * hw + 16 * hk + 4 * g;
+#pragma unroll
+  for (int j = 0; j < MT; j++) {
+    const f32x4 z = (hk ? acc[1][j] : acc[0][j]) + swap[((wid ^ (NW / 2)) * MT + j) * 64 + lane];
     uint2 o;
-    o.x = pack_bf16(acc[r], acc[r + 1]);
-    o.y = pack_bf16(acc[r + 2], acc[r + 3]);
-    *reinterpret_cast<uint2*>(lds + (wm * 32 + c32) * ROW + wn * 32 + 2 * r +
-                              4 * h) = o;
+    o.x = pack_bf16(z[0], z[1]);
+    o.y = pack_bf16(z[2], z[3]);
+    *reinterpret_cast<uint2*>(out + (16 * j + c16) * ROW + col0) = o;
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int idx = tid + i * 256, row = idx >> 3, col = (idx & 7) * 8;
-    if (m0 + row < M && n0 + col < N)
+  for (int k = 0; k < (MT + 1) / 2; k++) {
+    const int idx = tid + k * NW * 64;
+    const int row = idx / (WR / 8), col = idx % (WR / 8) * 8;
+    if (row < m_rows && col < n_rows)
       *reinterpret_cast<uint4*>(y + (m0 + row) * N + n0 + col) =
-          *reinterpret_cast<const uint4*>(lds + row * ROW + col);
+          *reinterpret_cast<const uint4*>(out + row * ROW + col);
   }
 }
 
@@ -302,20 +368,43 @@ __global__ __launch_bounds__(256, S == 4 ? 1 : 2) void linear_tile_kernel(
 //   M 64     4096 x 4096 13.2 | 14.9, 8192 x 4096 18.5 | 18.9, 12288 x 4096 31.4 | 24.7, 12288
 //            x 2048 18.8 | 16.1; 1024 x 8192 20 | 13.6, 4096 x 8192 22.7 | 23.9, 6144 x
 //            8192 30 | 29.3, 4096 x 14336 38.8 | 38.8
-//   M 96-192 4096 x 2048 12 | 14-21, 4096 x 4096 20 | 21-31, 4096 x 14336 60-68
-//            | 50-104 (tuned 50)
-//   M 300    2048 x 2048 10.8 | 10.5, 4096 x 2048 16.6 | 15.7, 4096 x 4096 29 | 25
-//   M 512    3072 x 2048 16.5 | 15.3, 4096 x 2048 17.6 | 17.1; M 1024 30 | 24
-//   M 96-256, few tiles   512 x 4096 17.7 | 8.8-12, 1024 x 2048 10.5 | 8.4, 1536 x 3072
-//            16 | 10.7, 2048 x 4096 18.8-20.4 | 12.8-15.9, 2560 x 4096 19 | 13; 1024 x
-//            1024 and 3072 x 4096 are still faster here
-// With a bias the library chooses among other kernels, which are faster from 65 rows
-// on, here | library: 96 x 2048 x 2048 11.8 | 6.9, 128 x 2048 x 1536 9.9 | 6.3, 300 x
-// 4096 x 2048 16.1 | 13.6, 96 x 4608 x 3584 18.2 | 16.5, 512 x 3072 x 2048 16.5 | 13.6.
+//   M 96-192 2048 x 2048 9.2 | 11.2-12, 4096 x 2048 10-11 | 13.3-21.5, 4096 x 4096
+//            16.6-18.7 | 22-33, 6144 x 4096 20.6-25.7 | 23-34, 8192 x 4096 23.5-28.5 | 24.3-35,
+//            4096 x 8192 30-34 | 36-59, 3584 x 18944 55-67 | 98-124
+//   M 300    2048 x 2048 9.3 | 12.9, 4096 x 2048 13.1 | 15.5, 4096 x 4096 22.4 | 25.8, 6144 x
+//            4096 30.3 | 30, 4096 x 14336 71 | 75; not in one turn of the CUs: 8192 x 4096
+//            46 | 37, 14336 x 2048 49 | 30
+//   M 512-1024   3072 x 2048 16.7 | 15.2, 4096 x 4096 30.7 | 30.2, 2048 x 2048 12-17.3 |
+//            12.8-17.1, 1024 x 4096 15.5-20.7 | 15.8-21.1; M 2048, 512 x 2048 13 | 10.8, M 3072 18 |
+//            12.9; but M 8192, 64 x 2048 8.7 | 10
+//   long rows, few tiles   M 96, 1024 x 4096 15.2 | 11.8, 2560 x 4096 15.9 | 13.2; M 128,
+//            1536 x 3072 12.7 | 10.5, 2048 x 4096 15.4 | 12.6, M 192 15.3 | 15.8; M 192, 1024 x
+//            4096 15 | 12.3, M 300 13.9 | 15.4; at K 2048 1024 x 2048 6.6 | 8.3
+// With a bias the library chooses among other kernels, which were faster from 65 rows
+// on: 96 x 2048 x 2048 6.9, 128 x 2048 x 1536 6.3, 96 x 4608 x 3584 16.5.
 // A tuned choice of the library is preferred above 48 rows, above 32 where N > 8192
 // (linear in bindings.cpp): M 32, 28672 x 4096 48.9 | 48.2, M 48 53.5 | 49.3 | 60.5 not,
 //   4096 x 4096, here | tuned | not   M 48 11.8 | 13.7 | 13.7, 64 13.2 | 13.6 | 15.1,
-//            96 19.6 | 17.2 | 22.0, 128 21.4 | 16.9 | 24.5
+//            96 16.6 | 17.2 | 22.0, 128 16.6 | 16.9 | 24.5
+
+// Of the shapes that linear_tile_kernel has, the one that a CU pulls least for: turns
+// of the CUs times the rows of a tile. x rows of 64 rows of W, or 0: 64 of 128.
+static int linear_shape(long M, long N, long* turns) {
+  int best = 0;
+  long least = 0;
+  for (int mt = 0; mt <= 6; mt++) {
+    if (mt == 1) continue;
+    const long wr = mt == 0 ? 128 : 64, xr = mt == 0 ? 64 : 16 * mt;
+    const long t = ((N + wr - 1) / wr * ((M + xr - 1) / xr) + 255) / 256;
+    const long cost = t * (wr + xr);
+    if (least != 0 && cost >= least) continue;
+    least = cost;
+    best = mt;
+    *turns = t;
+  }
+  return best;
+}
+
 int linear_takes(long M, long N, long K, bool bias) {
   if (M <= 0 || K < LN_K || K % LN_K != 0 || N % 8 != 0) return 0;
   if (N * K >= (1L << 31) || M * K >= (1L << 30)) return 0;
@@ -331,10 +420,13 @@ int linear_takes(long M, long N, long K, bool bias) {
   if (M <= 64)
     return N <= 8192 && (K <= 4096 || (N >= 2048 && N <= 4096 && K <= 8192)) ? 1 : 0;
   if (bias) return 0;
-  const long tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  long turns;
+  linear_shape(M, N, &turns);
+  if (turns > 1 || N > 8192 || (M > 2048 && N > 128)) return 0;
+  if (K > 4096) return N >= 3072 && N <= 4608 && M <= 192 ? 2 : 0;
   // few tiles with long rows leave most of the chip waiting for their chain
-  if (tiles <= 128 && ((K > 2048 && N < 3072) || (K > 1024 && N < 2048))) return 0;
-  return K <= 4096 && (tiles <= 256 || (tiles <= 512 && K <= 2048)) ? 2 : 0;
+  if (K > 2048 && ((N < 3072 && M <= 128) || (N < 2048 && M <= 256))) return 0;
+  return 2;
 }
 
 // Row tiles of W: one up to 4096 rows of it, one workgroup a CU then; two above.
@@ -386,13 +478,22 @@ void launch_linear(unsigned short* y, const unsigned short* x,
     launch_stream(y, x, w, bias, M, N, K, x_stride, stream);
     return;
   }
-  const int tn = (N + 63) / 64, tm = (M + 63) / 64;
-  if (tn * tm <= 256)
-    hipLaunchKernelGGL((linear_tile_kernel<4>), dim3(tn * tm), dim3(256), 0,
-                       stream, y, x, w, M, N, K, x_stride, tn);
-  else
-    hipLaunchKernelGGL((linear_tile_kernel<2>), dim3(tn * tm), dim3(256), 0,
-                       stream, y, x, w, M, N, K, x_stride, tn);
+#define LN_TILE(NW, MT, LK, S)                                                 \
+  hipLaunchKernelGGL((linear_tile_kernel<NW, MT, LK, S>),                      \
+                     dim3((unsigned)((N + 16 * NW - 1) / (16 * NW) *           \
+                                     ((M + 16 * MT - 1) / (16 * MT)))),        \
+                     dim3(NW * 64), 0, stream, y, x, w, M, N, K, x_stride,     \
+                     (N + 16 * NW - 1) / (16 * NW))
+  long turns;
+  switch (linear_shape(M, N, &turns)) {
+    case 0: LN_TILE(8, 4, 64, 6); break;
+    case 2: LN_TILE(4, 2, 128, 6); break;
+    case 3: LN_TILE(4, 3, 128, 5); break;
+    case 4: LN_TILE(4, 4, 128, 5); break;
+    case 5: LN_TILE(4, 5, 128, 4); break;
+    default: LN_TILE(4, 6, 128, 4);
+  }
+#undef LN_TILE
 }
 
 }  // namespace xllm

@@ -111,9 +111,9 @@ XLLM_DEV __amdgpu_buffer_rsrc_t mr_buffer(const void* p, unsigned bytes) {
 }
 // 16 bytes per lane, in lane order from dst on; zeros from out of the bounds
 XLLM_DEV void mr_to_lds(__amdgpu_buffer_rsrc_t src, unsigned off,
-                        unsigned short* dst) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void*)dst, 16, off, 0, 0,
-                                           0);
+                        unsigned short* dst, unsigned base = 0) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void*)dst, 16, off, base,
+                                           0, 0);
 }
 XLLM_DEV f32x16 mr_zero() {
   f32x16 z;

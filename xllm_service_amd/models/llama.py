@@ -12,6 +12,7 @@ from typing import List, Optional, Tuple
 
 import torch
 import torch.nn as nn
+import torch.nn.modules.module as module_hooks
 
 from xllm_service_amd import ops
 from xllm_service_amd.distributed import parallel_state as ps
@@ -90,6 +91,13 @@ class LlamaMLP(nn.Module):
         return self.down(ops.silu_and_mul(self.gate_up(x)))
 
 
+def _plain(module, kind):
+    """A module of this very class that nothing observes or replaces."""
+    return (type(module) is kind and not module._forward_hooks
+            and not module._forward_pre_hooks
+            and "forward" not in module.__dict__)
+
+
 class LlamaDecoderLayer(nn.Module):
     def __init__(self, cfg: ModelConfig, dtype):
         super().__init__()
@@ -99,7 +107,47 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = LlamaMLP(cfg, dtype)
         self.eps = cfg.rms_eps
 
+    def _native(self, x, residual, positions, kv_cache, meta, cos_sin):
+        """The layer as one native call, or None where a module in it is not the
+        plain one or torch has to see the calls: gradients, modes, tracing."""
+        if not (x.is_cuda and ops.HAS_EXT and torch.is_inference_mode_enabled()
+                and ps.tp_size() == 1) or module_hooks._global_forward_hooks \
+                or module_hooks._global_forward_pre_hooks \
+                or torch.compiler.is_compiling():
+            return None
+        attn, mlp = self._modules["attn"], self._modules["mlp"]
+        if not (_plain(attn, LlamaAttention) and _plain(mlp, LlamaMLP)):
+            return None
+        qkv, o = attn._modules["qkv_proj"], attn._modules["o_proj"]
+        gate_up, down = mlp._modules["gate_up"], mlp._modules["down"]
+        for m, kind in ((qkv, MergedColumnParallelLinear),
+                        (o, RowParallelLinear),
+                        (gate_up, MergedColumnParallelLinear),
+                        (down, RowParallelLinear)):
+            if not _plain(m, kind) or m.use_skinny:
+                return None
+        if o.bias is not None or down.bias is not None \
+                or attn.head_dim != 128 or kv_cache[0].shape[-1] != 128:
+            return None
+        w = (self.input_norm, qkv.weight, qkv.bias, o.weight, self.post_norm,
+             gate_up.weight, gate_up.bias, down.weight)
+        if torch.overrides.has_torch_function((x, residual, *w, *kv_cache)):
+            return None
+        ms0 = ms1 = 0
+        if attn.mrope_sections and positions.dim() != 1:
+            ms0 = int(attn.mrope_sections[0])
+            ms1 = ms0 + int(attn.mrope_sections[1])
+        return ops.decoder_layer(
+            x, residual, *w, self.eps, attn.n_heads, attn.scale, positions,
+            meta.slot_mapping, cos_sin, *kv_cache, ms0, ms1,
+            meta.num_prefill_tokens, meta.num_decode_tokens,
+            meta.prefill_block_tables, meta.cu_q, meta.prefill_seq_lens,
+            meta.decode_block_tables, meta.decode_seq_lens)
+
     def forward(self, x, residual, positions, kv_cache, meta, cos_sin):
+        done = self._native(x, residual, positions, kv_cache, meta, cos_sin)
+        if done is not None:
+            return done
         if residual is None:
             residual = x
             x = ops.rmsnorm(x, self.input_norm, self.eps)

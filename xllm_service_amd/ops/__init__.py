@@ -238,6 +238,13 @@ def linear(x, weight, bias=None):
     return torch.nn.functional.linear(x, weight, bias)
 
 
+def decoder_layer(*args):
+    """One layer of the dense decoders as a native call (GPU only): the layer's
+    new (x, residual), or None where torch's dispatcher must not be passed by."""
+    _require_ext()
+    return _ops.decoder_layer(*args)
+
+
 def skinny_gemm(a, b, bias=None):
     """Split-K weight-streaming GEMM for decode batches (M <= 64).
     GPU-only; callers fall back to F.linear elsewhere."""

@@ -77,6 +77,29 @@ def test_shapes_of_prompt_tiles(M, N, K, stride):
     assert off.max() <= 0, f"over by {off.max():.3g}"
 
 
+@pytest.mark.parametrize("M", [1, 8, 24, 33, 64, 65, 100, 250, 500])
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (4112, 640), (8208, 384),
+                                 (3088, 2048)])
+def test_gated(M, N, K):
+    """Gates and their partners in one product, against fp64 of the rounded sums:
+    the two roundings of 2^-8 of a sum (silu turns one of the gate into at most
+    1.1 of its size) and that of the result; 2^-17 as above, times the other
+    factor."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = (torch.randn(r, K, generator=g, device="cuda").to(torch.bfloat16)
+            for r in (M, N))
+    got = ops.linear_gated(x, w).double()
+    assert got.shape == (M, N // 2)
+    want = x.double() @ w.double().t()
+    big = x.double().abs() @ w.double().abs().t()
+    off = (2.0 ** -8 * want.abs() + 2.0 ** -17 * big).chunk(2, 1)
+    gate, up = want.chunk(2, 1)
+    y = torch.nn.functional.silu(gate) * up
+    bound = 2.0 ** -8 * y.abs() + 1.1 * off[0] * up.abs() \
+        + torch.nn.functional.silu(gate).abs() * off[1] + 1.1 * off[0] * off[1]
+    assert ((got - y).abs() - 1.01 * bound).max() <= 0
+
+
 def test_what_the_kernels_do_not_take():
     """Types, widths, gradients and shapes that go to the library."""
     for dt, M, N, K in ((torch.float32, 4, 64, 128), (torch.bfloat16, 4, 63, 128),

@@ -62,7 +62,7 @@ void launch_skinny_gemm(unsigned short*, const unsigned short*,
 int linear_takes(long M, long N, long K, bool bias);
 void launch_linear(unsigned short*, const unsigned short*,
                    const unsigned short*, const unsigned short*, int, int, int,
-                   long, int, hipStream_t);
+                   long, int, bool, hipStream_t);
 int packed_gemm_splitk(int M, int N, int K, int S);
 void launch_packed_gemm(unsigned short*, const unsigned short*,
                         unsigned short*, const unsigned short*,
@@ -402,38 +402,69 @@ static bool tuned(long M, long N, long K, long x_stride) {
          entry != at::cuda::tunable::ResultEntry::Default();
 }
 
-// x [..., K] @ w [N, K]^T (+ bias): the kernels of linear.hip where they take the
-// call, the library elsewhere (and wherever a gradient is wanted)
-torch::Tensor linear(torch::Tensor x, torch::Tensor w,
-                     c10::optional<torch::Tensor> bias) {
+// Which kernels of linear.hip take x @ w^T (+ bias): linear_takes, 0 for none
+static int linear_kind(const torch::Tensor& x, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias) {
   auto rows16 = [](const torch::Tensor& t) {
     return t.dim() == 2 && t.is_cuda() && t.dtype() == torch::kBFloat16 &&
            t.stride(1) == 1 &&
            reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  if ((bias.has_value() ? direct({x, w, *bias}) : direct({x, w})) &&
-      rows16(x) && rows16(w) && x.size(1) == w.size(1) &&
-      x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) &&
-      x.stride(0) < (1L << 24) && w.is_contiguous() &&
-      x.device() == w.device() &&
-      (!bias.has_value() ||
-       (bias->dim() == 1 && bias->is_contiguous() &&
-        bias->dtype() == torch::kBFloat16 && bias->size(0) == w.size(0) &&
-        bias->device() == w.device()))) {
+  if (!((bias.has_value() ? direct({x, w, *bias}) : direct({x, w})) &&
+        rows16(x) && rows16(w) && x.size(1) == w.size(1) &&
+        x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) &&
+        x.stride(0) < (1L << 24) && w.is_contiguous() &&
+        x.device() == w.device() &&
+        (!bias.has_value() ||
+         (bias->dim() == 1 && bias->is_contiguous() &&
+          bias->dtype() == torch::kBFloat16 && bias->size(0) == w.size(0) &&
+          bias->device() == w.device()))))
+    return 0;
+  const long M = x.size(0), N = w.size(0), K = w.size(1);
+  const int kind = xllm::linear_takes(M, N, K, bias.has_value());
+  return kind != 0 && M > (N > 8192 ? 32 : 48) && !bias.has_value() &&
+                 tuned(M, N, K, x.stride(0))
+             ? 0
+             : kind;
+}
+
+// x [..., K] @ w [N, K]^T (+ bias): the kernels of linear.hip where they take the
+// call, the library elsewhere (and wherever a gradient is wanted)
+torch::Tensor linear(torch::Tensor x, torch::Tensor w,
+                     c10::optional<torch::Tensor> bias) {
+  if (const int kind = linear_kind(x, w, bias)) {
     const long M = x.size(0), N = w.size(0), K = w.size(1);
-    const int kind = xllm::linear_takes(M, N, K, bias.has_value());
-    if (kind != 0 &&
-        !(M > (N > 8192 ? 32 : 48) && !bias.has_value() &&
-          tuned(M, N, K, x.stride(0)))) {
+    c10::OptionalDeviceGuard guard(x.device());
+    auto y = torch::empty({M, N}, x.options());
+    xllm::launch_linear(u16(y), u16c(x), u16c(w),
+                        bias.has_value() ? u16c(*bias) : nullptr, (int)M,
+                        (int)N, (int)K, x.stride(0), kind, false, cur_stream());
+    return y;
+  }
+  return at::linear(x, w, bias.has_value() ? *bias : torch::Tensor());
+}
+
+// silu(x gates^T) (x ups^T), w = [gates | ups] by rows: one kernel where linear.hip
+// takes the product (a launch, and twice the result written and read again: 24 rows,
+// 2 x 4096 x 4096 18.5 us as two kernels), the same two calls as always elsewhere
+torch::Tensor linear_gated(torch::Tensor x, torch::Tensor w,
+                           c10::optional<torch::Tensor> bias) {
+  if (!bias.has_value() && w.dim() == 2 && w.size(0) % 16 == 0) {
+    if (const int kind = linear_kind(x, w, bias)) {
+      const long M = x.size(0), N = w.size(0), K = w.size(1);
       c10::OptionalDeviceGuard guard(x.device());
-      auto y = torch::empty({M, N}, x.options());
-      xllm::launch_linear(u16(y), u16c(x), u16c(w),
-                          bias.has_value() ? u16c(*bias) : nullptr, (int)M,
-                          (int)N, (int)K, x.stride(0), kind, cur_stream());
+      auto y = torch::empty({M, N / 2}, x.options());
+      xllm::launch_linear(u16(y), u16c(x), u16c(w), nullptr, (int)M, (int)N,
+                          (int)K, x.stride(0), kind, true, cur_stream());
       return y;
     }
   }
-  return at::linear(x, w, bias.has_value() ? *bias : torch::Tensor());
+  const auto h = ::linear(x, w, bias);
+  auto shape = h.sizes().vec();
+  shape.back() /= 2;
+  auto y = torch::empty(shape, h.options());
+  silu_and_mul(y, h);
+  return y;
 }
 
 // One layer of the dense decoders (models/llama.py) over prompt rows and decode
@@ -489,10 +520,8 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layer(
                       scale);
   h = ::linear(out, o_w, c10::nullopt);
   fused_add_rmsnorm(h, res, post_norm, eps);
-  h = ::linear(h, gate_up_w, gate_up_b);
-  auto act = torch::empty({h.size(0), h.size(1) / 2}, h.options());
-  silu_and_mul(act, h);
-  return std::make_tuple(::linear(act, down_w, c10::nullopt), res);
+  h = linear_gated(h, gate_up_w, gate_up_b);
+  return std::make_tuple(::linear(h, down_w, c10::nullopt), res);
 }
 
 torch::Tensor packed_gemm(torch::Tensor a, torch::Tensor wp, int64_t N,
@@ -715,6 +744,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma_gemm", &mfma_gemm);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("linear", &linear);
+  m.def("linear_gated", &linear_gated);
   m.def("direct", &direct);
   m.def("decoder_layer", &decoder_layer);
   m.def("packed_gemm", &packed_gemm);

@@ -39,6 +39,21 @@ XLLM_DEV void ln_read2(const unsigned* a, const unsigned* b, bf16x8* v,
       : "memory");
 }
 
+// Gated products: W = [gates | ups] by rows, half of each, and a tile of ROWS rows has
+// as many of both. Row of the matrix that row r of the tile from gate `first` on is;
+// rows past the last one repeat it
+template <int ROWS>
+XLLM_DEV long ln_gate_row(long first, long half, int r) {
+  return r < ROWS / 2 ? min(first + r, half - 1)
+                      : half + min(first + r - ROWS / 2, half - 1);
+}
+// silu(gate) up of two sums, as act_and_mul_kernel makes it of rounded ones
+XLLM_DEV float ln_gated(float gate, float up) {
+  const unsigned u = pack_bf16(gate, up);
+  const float a = __uint_as_float(u << 16);
+  return a / (1.0f + __expf(-a)) * __uint_as_float(u & 0xffff0000u);
+}
+
 // Rows r0 .. of a matrix into an image: instruction i moves four rows
 template <int ROWS>
 struct LnTile {
@@ -50,6 +65,17 @@ struct LnTile {
     for (int i = 0; i < NI; i++) {
       const int r = i * 4 + (lane >> 4);
       const long row = min(first + r, rows - 1) - first;
+      off[i] = (unsigned)(row * stride * 2 +
+                          (((lane & 15) ^ (r & 15)) << 4));
+    }
+  }
+  // the first half of the rows from `first` on, the other half as many rows further
+  // on as there are in a half of the matrix
+  XLLM_DEV void init_gate(long first, long half, long stride, int lane) {
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int r = i * 4 + (lane >> 4);
+      const long row = ln_gate_row<ROWS>(first, half, r) - first;
       off[i] = (unsigned)(row * stride * 2 +
                           (((lane & 15) ^ (r & 15)) << 4));
     }
@@ -78,7 +104,7 @@ struct LnTile {
 //   M 24  4096 x 4096 10.1 -> 9.1, 6144 x 4096 15.2 -> 12.4, 8192 x 4096 16.9 -> 14.3,
 //         32000 x 4096 57 -> 48, 4096 x 14336 27.5 -> 25.3
 //   M 64  4096 x 4096 14.4 -> 13.2, 6144 x 4096 22.0 -> 17.2, 8192 x 4096 23.5 -> 18.5
-template <int NT, int XR, int NW, int D>
+template <int NT, int XR, int NW, int D, bool GATE>
 __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w,
@@ -95,11 +121,14 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
-  const long n0 = blockIdx.x * (long)WR;
+  constexpr int OUT = GATE ? WR / 2 : WR;        // columns of the result
+  const int n_out = GATE ? N / 2 : N;
+  const long n0 = blockIdx.x * (long)OUT;
   unsigned short* wt = lds + wid * (D * TILE);
   LnTile<WR> lw;
   LnTile<XR> lx;
-  lw.init(n0, N, K, lane);
+  if (GATE) lw.init_gate(n0, n_out, K, lane);
+  else lw.init(n0, N, K, lane);
   lx.init(0, M, x_stride, lane);
   const unsigned short* wp = w + n0 * K;
   // bytes of chunk 4 ks + g of row c16; a last tile of eight rows is read twice
@@ -171,26 +200,35 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
                                  16 * n + 4 * g) =
           make_float4(acc[n][j][0], acc[n][j][1], acc[n][j][2], acc[n][j][3]);
   __syncthreads();
-  constexpr int C4 = WR / 4;                     // columns in fours
-  for (int i = tid; i < 16 * MT * C4; i += NW * 64) {
-    const int m = i / C4, col = (i % C4) * 4;
-    const long n = n0 + col;
-    if (m >= M || n >= N) continue;
-    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto sum = [&](int m, int col, float (&s)[4]) {
 #pragma unroll
     for (int k = 0; k < NW; k++) {
       const float4 z = *reinterpret_cast<const float4*>(
           part + (k * 16 * MT + m) * ROW + col);
-      s[0] += z.x; s[1] += z.y; s[2] += z.z; s[3] += z.w;
+      if (k == 0) { s[0] = z.x; s[1] = z.y; s[2] = z.z; s[3] = z.w; }
+      else { s[0] += z.x; s[1] += z.y; s[2] += z.z; s[3] += z.w; }
     }
-    if (bias != nullptr) {
+  };
+  constexpr int C4 = OUT / 4;                    // columns in fours
+  for (int i = tid; i < 16 * MT * C4; i += NW * 64) {
+    const int m = i / C4, col = (i % C4) * 4;
+    const long n = n0 + col;
+    if (m >= M || n >= n_out) continue;
+    float s[4];
+    sum(m, col, s);
+    if constexpr (GATE) {
+      float u[4];
+      sum(m, OUT + col, u);
+#pragma unroll
+      for (int k = 0; k < 4; k++) s[k] = ln_gated(s[k], u[k]);
+    } else if (bias != nullptr) {
 #pragma unroll
       for (int k = 0; k < 4; k++) s[k] += bf16_to_f32(bias[n + k]);
     }
     uint2 o;
     o.x = pack_bf16(s[0], s[1]);
     o.y = pack_bf16(s[2], s[3]);
-    *reinterpret_cast<uint2*>(y + (long)m * N + n) = o;
+    *reinterpret_cast<uint2*>(y + (long)m * n_out + n) = o;
   }
 }
 
@@ -211,7 +249,7 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
 // 4096 x 4096 29.5 -> 22.5, 3072 x 2048 11.7 -> 11.6; 96 x 3072 x 2048 10.9 -> 9.6;
 // 192 x 6144 x 4096 30.1 -> 25.7; 512 x 3072 x 2048 16.5 -> 16.7; 256 x 3072 x 2048, as many
 // tiles of 64 x 64 either way, 11.8 -> 12.1.
-template <int NW, int MT, int LK, int S>
+template <int NW, int MT, int LK, int S, bool GATE>
 __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w, const int M, const int N,
@@ -226,28 +264,34 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
-  const long n0 = (blockIdx.x % n_tiles_n) * (long)WR;
+  constexpr int OUT = GATE ? WR / 2 : WR;        // columns of the result
+  const int n_out = GATE ? N / 2 : N;
+  const long n0 = (blockIdx.x % n_tiles_n) * (long)OUT;
   const long m0 = (blockIdx.x / n_tiles_n) * (16L * MT);
-  const int n_rows = (int)min((long)WR, N - n0);
+  const int n_cols = (int)min((long)OUT, n_out - n0);
   const int m_rows = (int)min(16L * MT, M - m0);
   const unsigned short* wp = w + n0 * K;
   const unsigned short* xp = x + m0 * x_stride;
-  const unsigned w_bytes = (unsigned)n_rows * K * 2;
+  const unsigned w_bytes = (unsigned)(n_cols + (GATE ? n_out : 0)) * K * 2;
   const unsigned x_bytes = (unsigned)((m_rows - 1) * x_stride + K) * 2;
   // a wave loads 16 rows of W and its share of x, RPI at a time; rows past the last
   // one repeat it: their results go nowhere
   unsigned w_off[WI], x_off[XI];
-  auto offset = [&](int r, int last, long stride) {
+  auto offset = [&](int r, long row, long stride) {
     const int swz = LK == 128 ? r & 15 : (r >> 1) & 7;
-    return (unsigned)(min(r, last) * stride * 2) +
-           (((lane % CPR) ^ swz) << 4);
+    return (unsigned)(row * stride * 2) + (((lane % CPR) ^ swz) << 4);
   };
 #pragma unroll
-  for (int i = 0; i < WI; i++)
-    w_off[i] = offset((wid * WI + i) * RPI + lane / CPR, n_rows - 1, K);
+  for (int i = 0; i < WI; i++) {
+    const int r = (wid * WI + i) * RPI + lane / CPR;
+    w_off[i] = offset(r, GATE ? ln_gate_row<WR>(n0, n_out, r) - n0
+                              : min(r, n_cols - 1), K);
+  }
 #pragma unroll
-  for (int i = 0; i < XI; i++)
-    x_off[i] = offset((wid * XI + i) * RPI + lane / CPR, m_rows - 1, x_stride);
+  for (int i = 0; i < XI; i++) {
+    const int r = (wid * XI + i) * RPI + lane / CPR;
+    x_off[i] = offset(r, min(r, m_rows - 1), x_stride);
+  }
   const int steps = K / LK;
   auto stage = [&](int t, int slot) {
     const bool on = t < steps;                   // past the end: zeros
@@ -343,13 +387,24 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     *reinterpret_cast<uint2*>(out + (16 * j + c16) * ROW + col0) = o;
   }
   __syncthreads();
+  constexpr int C8 = OUT / 8;                    // columns in eights
 #pragma unroll
-  for (int k = 0; k < (MT + 1) / 2; k++) {
+  for (int k = 0; k < (16 * MT * C8 + NW * 64 - 1) / (NW * 64); k++) {
     const int idx = tid + k * NW * 64;
-    const int row = idx / (WR / 8), col = idx % (WR / 8) * 8;
-    if (row < m_rows && col < n_rows)
-      *reinterpret_cast<uint4*>(y + (m0 + row) * N + n0 + col) =
-          *reinterpret_cast<const uint4*>(out + row * ROW + col);
+    const int row = idx / C8, col = idx % C8 * 8;
+    if (row >= m_rows || col >= n_cols) continue;
+    uint4 v = *reinterpret_cast<const uint4*>(out + row * ROW + col);
+    if constexpr (GATE) {
+      const uint4 u = *reinterpret_cast<const uint4*>(out + row * ROW + OUT + col);
+      auto two = [](unsigned a, unsigned b) {
+        return pack_bf16(
+            ln_gated(__uint_as_float(a << 16), __uint_as_float(b << 16)),
+            ln_gated(__uint_as_float(a & 0xffff0000u),
+                     __uint_as_float(b & 0xffff0000u)));
+      };
+      v = make_uint4(two(v.x, u.x), two(v.y, u.y), two(v.z, u.z), two(v.w, u.w));
+    }
+    *reinterpret_cast<uint4*>(y + (m0 + row) * n_out + n0 + col) = v;
   }
 }
 
@@ -443,15 +498,17 @@ static bool linear_one_tile(int M, int N, int K) {
 // A workgroup that has a CU to itself takes all of its LDS: two tiles a wave, or
 // more waves. Where there are more than CUs, two of them share one: M 24, 32000 x
 // 4096 48.4, with two tiles 49.2; 18944 x 4096 33.4 | 34.5.
+template <bool GATE>
 static void launch_stream(unsigned short* y, const unsigned short* x,
                           const unsigned short* w, const unsigned short* bias,
                           int M, int N, int K, long x_stride,
                           hipStream_t stream) {
   const bool one = linear_one_tile(M, N, K);
-  const dim3 grid((N + (one ? 15 : 31)) / (one ? 16 : 32));
+  const int out = (one ? 16 : 32) / (GATE ? 2 : 1), n_out = N / (GATE ? 2 : 1);
+  const dim3 grid((n_out + out - 1) / out);
   const bool few = grid.x <= 256;
 #define LN_STREAM(NT, XR, NW, D)                                               \
-  hipLaunchKernelGGL((linear_stream_kernel<NT, XR, NW, D>), grid,              \
+  hipLaunchKernelGGL((linear_stream_kernel<NT, XR, NW, D, GATE>), grid,        \
                      dim3(NW * 64), 0, stream, y, x, w, bias, M, N, K, x_stride)
   if (one) {
     if (M <= 8) LN_STREAM(1, 8, 4, 2);
@@ -471,19 +528,19 @@ static void launch_stream(unsigned short* y, const unsigned short* x,
 #undef LN_STREAM
 }
 
-void launch_linear(unsigned short* y, const unsigned short* x,
-                   const unsigned short* w, const unsigned short* bias, int M,
-                   int N, int K, long x_stride, int kind, hipStream_t stream) {
-  if (kind == 1) {
-    launch_stream(y, x, w, bias, M, N, K, x_stride, stream);
-    return;
-  }
+template <bool GATE>
+static void launch_tile(unsigned short* y, const unsigned short* x,
+                        const unsigned short* w, int M, int N, int K,
+                        long x_stride, hipStream_t stream) {
+  const int n_out = N / (GATE ? 2 : 1);
 #define LN_TILE(NW, MT, LK, S)                                                 \
-  hipLaunchKernelGGL((linear_tile_kernel<NW, MT, LK, S>),                      \
-                     dim3((unsigned)((N + 16 * NW - 1) / (16 * NW) *           \
-                                     ((M + 16 * MT - 1) / (16 * MT)))),        \
-                     dim3(NW * 64), 0, stream, y, x, w, M, N, K, x_stride,     \
-                     (N + 16 * NW - 1) / (16 * NW))
+  do {                                                                         \
+    constexpr int OUT = 16 * NW / (GATE ? 2 : 1);                              \
+    const int tn = (n_out + OUT - 1) / OUT, tm = (M + 16 * MT - 1) / (16 * MT); \
+    hipLaunchKernelGGL((linear_tile_kernel<NW, MT, LK, S, GATE>),              \
+                       dim3((unsigned)(tn * tm)), dim3(NW * 64), 0, stream, y, \
+                       x, w, M, N, K, x_stride, tn);                           \
+  } while (0)
   long turns;
   switch (linear_shape(M, N, &turns)) {
     case 0: LN_TILE(8, 4, 64, 6); break;
@@ -494,6 +551,19 @@ void launch_linear(unsigned short* y, const unsigned short* x,
     default: LN_TILE(4, 6, 128, 4);
   }
 #undef LN_TILE
+}
+
+// gate: W = [gates | ups], y [M, N / 2] = silu(x gates^T) (x ups^T)
+void launch_linear(unsigned short* y, const unsigned short* x,
+                   const unsigned short* w, const unsigned short* bias, int M,
+                   int N, int K, long x_stride, int kind, bool gate,
+                   hipStream_t stream) {
+  if (kind == 1)
+    (gate ? launch_stream<true> : launch_stream<false>)(
+        y, x, w, bias, M, N, K, x_stride, stream);
+  else
+    (gate ? launch_tile<true> : launch_tile<false>)(y, x, w, M, N, K, x_stride,
+                                                    stream);
 }
 
 }  // namespace xllm

@@ -24,6 +24,13 @@ from xllm_service_amd.models.config import ModelConfig
 from xllm_service_amd.ops import ref as op_ref
 
 
+def _plain(module, kind):
+    """A module of this very class that nothing observes or replaces."""
+    return (type(module) is kind and not module._forward_hooks
+            and not module._forward_pre_hooks
+            and "forward" not in module.__dict__)
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: ModelConfig, dtype):
         super().__init__()
@@ -88,14 +95,10 @@ class LlamaMLP(nn.Module):
                                       dtype=dtype)
 
     def forward(self, x):
-        return self.down(ops.silu_and_mul(self.gate_up(x)))
-
-
-def _plain(module, kind):
-    """A module of this very class that nothing observes or replaces."""
-    return (type(module) is kind and not module._forward_hooks
-            and not module._forward_pre_hooks
-            and "forward" not in module.__dict__)
+        g = self.gate_up
+        if _plain(g, MergedColumnParallelLinear) and not g.use_skinny:
+            return self.down(ops.linear_gated(x, g.weight, g.bias))
+        return self.down(ops.silu_and_mul(g(x)))
 
 
 class LlamaDecoderLayer(nn.Module):

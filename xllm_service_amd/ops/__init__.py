@@ -238,6 +238,15 @@ def linear(x, weight, bias=None):
     return torch.nn.functional.linear(x, weight, bias)
 
 
+def linear_gated(x, weight, bias=None):
+    """silu(gate) * up of the two halves of x @ weight.T (+ bias): one kernel for the
+    bf16 shapes of serving steps, `linear` and `silu_and_mul` elsewhere."""
+    if x.is_cuda and HAS_EXT and not torch.overrides.has_torch_function(
+            (x, weight, bias)):
+        return _ops.linear_gated(x, weight, bias)
+    return silu_and_mul(linear(x, weight, bias))
+
+
 def decoder_layer(*args):
     """One layer of the dense decoders as a native call (GPU only): the layer's
     new (x, residual), or None where torch's dispatcher must not be passed by."""

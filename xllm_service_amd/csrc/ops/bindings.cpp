@@ -1,6 +1,7 @@
 // PyTorch bindings for the MI355X (gfx950) HIP kernels.
 //
 // All tensor-shape/dtype validation lives here so the kernels stay lean.
+#include "linear.h"
 #include <hip/hip_runtime.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/tunable/Tunable.h>
@@ -60,9 +61,10 @@ void launch_skinny_gemm(unsigned short*, const unsigned short*,
                         const unsigned short*, const unsigned short*, float*,
                         int, int, int, hipStream_t);
 int linear_takes(long M, long N, long K, bool bias);
+int linear_tiles(int M, int N, int K, int kind);
 void launch_linear(unsigned short*, const unsigned short*,
                    const unsigned short*, const unsigned short*, int, int, int,
-                   long, int, bool, hipStream_t);
+                   long, int, int, const LinearEnds&, hipStream_t);
 int packed_gemm_splitk(int M, int N, int K, int S);
 void launch_packed_gemm(unsigned short*, const unsigned short*,
                         unsigned short*, const unsigned short*,
@@ -438,7 +440,7 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor w,
     auto y = torch::empty({M, N}, x.options());
     xllm::launch_linear(u16(y), u16c(x), u16c(w),
                         bias.has_value() ? u16c(*bias) : nullptr, (int)M,
-                        (int)N, (int)K, x.stride(0), kind, false, cur_stream());
+                        (int)N, (int)K, x.stride(0), kind, 0, {}, cur_stream());
     return y;
   }
   return at::linear(x, w, bias.has_value() ? *bias : torch::Tensor());
@@ -455,7 +457,8 @@ torch::Tensor linear_gated(torch::Tensor x, torch::Tensor w,
       c10::OptionalDeviceGuard guard(x.device());
       auto y = torch::empty({M, N / 2}, x.options());
       xllm::launch_linear(u16(y), u16c(x), u16c(w), nullptr, (int)M, (int)N,
-                          (int)K, x.stride(0), kind, true, cur_stream());
+                          (int)K, x.stride(0), kind, xllm::LN_GATE, {},
+                          cur_stream());
       return y;
     }
   }
@@ -467,61 +470,151 @@ torch::Tensor linear_gated(torch::Tensor x, torch::Tensor w,
   return y;
 }
 
-// One layer of the dense decoders (models/llama.py) over prompt rows and decode
-// rows: what its modules call, in their order, without the interpreter between two
+// Rows between two products of a layer: as an RMS norm leaves them, or without their
+// factors and with the sums of their squares' parts [rows][tiles]
+struct Rows { torch::Tensor x, squares; };
+
+static xllm::LinearEnds scale_of(const Rows& in, double eps) {
+  xllm::LinearEnds e;
+  e.squares = in.squares.data_ptr<float>();
+  e.n_squares = in.squares.size(1);
+  e.eps = (float)eps;
+  return e;
+}
+
+// in W^T (+ bias), or of W = [gates | ups] silu(in gates^T) (in ups^T)
+static torch::Tensor product(const Rows& in, const torch::Tensor& w,
+                             const c10::optional<torch::Tensor>& bias, bool gate,
+                             double eps) {
+  if (!in.squares.defined())
+    return gate ? linear_gated(in.x, w, bias) : ::linear(in.x, w, bias);
+  const long M = in.x.size(0), N = w.size(0), K = w.size(1);
+  auto y = torch::empty({M, gate ? N / 2 : N}, in.x.options());
+  xllm::launch_linear(u16(y), u16c(in.x), u16c(w),
+                      bias.has_value() ? u16c(*bias) : nullptr, (int)M, (int)N,
+                      (int)K, in.x.stride(0), linear_kind(in.x, w, bias),
+                      xllm::LN_SCALE | (gate ? xllm::LN_GATE : 0),
+                      scale_of(in, eps), cur_stream());
+  return y;
+}
+
+// The rows of the next product: res += x w^T, normed. One kernel where linear.hip
+// takes this product and the next one (next_w), else product and norm.
+static Rows product_normed(const torch::Tensor& x, const torch::Tensor& w,
+                           const torch::Tensor& res, const torch::Tensor& norm,
+                           const torch::Tensor& next_w,
+                           const c10::optional<torch::Tensor>& next_bias,
+                           bool next_gate, double eps) {
+  const c10::optional<torch::Tensor> none;
+  const int kind = linear_kind(x, w, none);
+  const long M = x.size(0), N = w.size(0), K = w.size(1);
+  if (kind != 0 && res.dim() == 2 && res.is_contiguous() && res.size(0) == M &&
+      res.size(1) == N && res.dtype() == torch::kBFloat16 && on_bytes(res, 16) &&
+      norm.dim() == 1 && norm.size(0) == N && norm.is_contiguous() &&
+      norm.dtype() == torch::kBFloat16 &&
+      reinterpret_cast<uintptr_t>(norm.data_ptr()) % 16 == 0 &&
+      res.is_cuda() && norm.is_cuda() &&
+      !(next_gate && (next_bias.has_value() || next_w.size(0) % 16 != 0))) {
+    Rows out{torch::empty({M, N}, x.options()), {}};
+    const int next = linear_kind(out.x, next_w, next_bias);
+    const int tiles = xllm::linear_tiles((int)M, (int)N, (int)K, kind);
+    if (next != 0 && tiles % 4 == 0 && tiles <= (next == 1 ? 256 : 64)) {
+      out.squares = torch::empty({M, tiles}, x.options().dtype(torch::kFloat));
+      xllm::LinearEnds e;
+      e.residual = reinterpret_cast<unsigned short*>(res.data_ptr());
+      e.norm = u16c(norm);
+      e.sums = out.squares.data_ptr<float>();
+      xllm::launch_linear(u16(out.x), u16c(x), u16c(w), nullptr, (int)M, (int)N,
+                          (int)K, x.stride(0), kind, xllm::LN_ADD, e,
+                          cur_stream());
+      return out;
+    }
+  }
+  auto h = ::linear(x, w, none);
+  fused_add_rmsnorm(h, res, norm, eps);
+  return {h, {}};
+}
+
+struct DecoderLayer {
+  torch::Tensor input_norm, qkv_w;
+  c10::optional<torch::Tensor> qkv_b;
+  torch::Tensor o_w, post_norm, gate_up_w;
+  c10::optional<torch::Tensor> gate_up_b;
+  torch::Tensor down_w, k_cache, v_cache;
+};
+
+// Layers of the dense decoders (models/llama.py) over prompt rows and decode rows:
+// what their modules call, in their order, without the interpreter between two
 // launches (75 us of host time a layer, 25 here, where the kernels of 300 rows of 2048
-// take 70). Nothing, with nothing done, where torch has to see the calls.
-c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layer(
+// take 70), and without launches for the norms between two products. Nothing, with
+// nothing done, where torch has to see the calls.
+c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layers(
     torch::Tensor x, c10::optional<torch::Tensor> residual,
-    torch::Tensor input_norm, torch::Tensor qkv_w,
-    c10::optional<torch::Tensor> qkv_b, torch::Tensor o_w,
-    torch::Tensor post_norm, torch::Tensor gate_up_w,
-    c10::optional<torch::Tensor> gate_up_b, torch::Tensor down_w, double eps,
+    std::vector<std::vector<c10::optional<torch::Tensor>>> weights, double eps,
     long heads, double scale, torch::Tensor positions,
-    torch::Tensor slot_mapping, torch::Tensor cos_sin, torch::Tensor k_cache,
-    torch::Tensor v_cache, long ms0, long ms1, long n_prefill, long n_decode,
-    c10::optional<torch::Tensor> prefill_tables,
+    torch::Tensor slot_mapping, torch::Tensor cos_sin, long ms0, long ms1,
+    long n_prefill, long n_decode, c10::optional<torch::Tensor> prefill_tables,
     c10::optional<torch::Tensor> cu_q,
     c10::optional<torch::Tensor> prefill_lens,
     c10::optional<torch::Tensor> decode_tables,
     c10::optional<torch::Tensor> decode_lens) {
-  if (!direct({x, input_norm, qkv_w, o_w, post_norm, gate_up_w, down_w, k_cache,
-               v_cache}))
-    return c10::nullopt;
-  torch::Tensor h = x, res;
+  std::vector<DecoderLayer> layers;
+  for (const auto& w : weights) {
+    TORCH_CHECK(w.size() == 10, "decoder layer: ten tensors");
+    layers.push_back({w[0].value(), w[1].value(), w[2], w[3].value(),
+                      w[4].value(), w[5].value(), w[6], w[7].value(),
+                      w[8].value(), w[9].value()});
+  }
+  TORCH_CHECK(!layers.empty(), "decoder layers: none");
+  for (const auto& p : layers)
+    if (!direct({x, p.input_norm, p.qkv_w, p.o_w, p.post_norm, p.gate_up_w,
+                 p.down_w, p.k_cache, p.v_cache}))
+      return c10::nullopt;
+  c10::OptionalDeviceGuard guard(x.device());
+  torch::Tensor res;
+  Rows in;
   if (residual.has_value()) {
     res = *residual;
-    fused_add_rmsnorm(h, res, input_norm, eps);
+    in.x = x;
+    fused_add_rmsnorm(in.x, res, layers[0].input_norm, eps);
   } else {
     res = x;
-    h = torch::empty_like(x);
-    rmsnorm(h, x, input_norm, eps);
+    in.x = torch::empty_like(x);
+    rmsnorm(in.x, x, layers[0].input_norm, eps);
   }
-  const auto qkv = ::linear(h, qkv_w, qkv_b);
-  const long T = qkv.size(0), D = k_cache.size(3), n_kv = k_cache.size(1);
-  const long row = qkv.stride(0), at = qkv.storage_offset();
-  TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (heads + 2 * n_kv) * D &&
-              qkv.stride(1) == 1, "decoder layer: shapes do not match");
-  const auto q = qkv.as_strided({T, heads, D}, {row, D, 1}, at);
-  const auto k = qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + heads * D);
-  const auto v =
-      qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + (heads + n_kv) * D);
-  fused_rope_cache(positions, q, k, v, k_cache, v_cache, slot_mapping, cos_sin,
-                   D, ms0, ms1);
-  auto out = torch::empty({T, heads * D}, qkv.options());
-  const auto out3 = out.view({T, heads, D});
-  if (n_prefill > 0)
-    paged_attn_prefill(out3.slice(0, 0, n_prefill), q.slice(0, 0, n_prefill),
-                       k_cache, v_cache, prefill_tables.value(), cu_q.value(),
-                       prefill_lens.value(), scale);
-  if (n_decode > 0)
-    paged_attn_decode(out3.slice(0, n_prefill), q.slice(0, n_prefill), k_cache,
-                      v_cache, decode_tables.value(), decode_lens.value(),
-                      scale);
-  h = ::linear(out, o_w, c10::nullopt);
-  fused_add_rmsnorm(h, res, post_norm, eps);
-  h = linear_gated(h, gate_up_w, gate_up_b);
-  return std::make_tuple(::linear(h, down_w, c10::nullopt), res);
+  for (size_t i = 0; i < layers.size(); i++) {
+    const auto& p = layers[i];
+    const auto qkv = product(in, p.qkv_w, p.qkv_b, false, eps);
+    const long T = qkv.size(0), D = p.k_cache.size(3), n_kv = p.k_cache.size(1);
+    const long row = qkv.stride(0), at = qkv.storage_offset();
+    TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (heads + 2 * n_kv) * D &&
+                qkv.stride(1) == 1, "decoder layer: shapes do not match");
+    const auto q = qkv.as_strided({T, heads, D}, {row, D, 1}, at);
+    const auto k = qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + heads * D);
+    const auto v =
+        qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + (heads + n_kv) * D);
+    fused_rope_cache(positions, q, k, v, p.k_cache, p.v_cache, slot_mapping,
+                     cos_sin, D, ms0, ms1);
+    auto out = torch::empty({T, heads * D}, qkv.options());
+    const auto out3 = out.view({T, heads, D});
+    if (n_prefill > 0)
+      paged_attn_prefill(out3.slice(0, 0, n_prefill), q.slice(0, 0, n_prefill),
+                         p.k_cache, p.v_cache, prefill_tables.value(),
+                         cu_q.value(), prefill_lens.value(), scale);
+    if (n_decode > 0)
+      paged_attn_decode(out3.slice(0, n_prefill), q.slice(0, n_prefill),
+                        p.k_cache, p.v_cache, decode_tables.value(),
+                        decode_lens.value(), scale);
+    in = product_normed(out, p.o_w, res, p.post_norm, p.gate_up_w, p.gate_up_b,
+                        true, eps);
+    const auto act = product(in, p.gate_up_w, p.gate_up_b, true, eps);
+    if (i + 1 == layers.size())
+      return std::make_tuple(::linear(act, p.down_w, c10::nullopt), res);
+    const auto& next = layers[i + 1];
+    in = product_normed(act, p.down_w, res, next.input_norm, next.qkv_w,
+                        next.qkv_b, false, eps);
+  }
+  return c10::nullopt;
 }
 
 torch::Tensor packed_gemm(torch::Tensor a, torch::Tensor wp, int64_t N,
@@ -746,7 +839,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear", &linear);
   m.def("linear_gated", &linear_gated);
   m.def("direct", &direct);
-  m.def("decoder_layer", &decoder_layer);
+  m.def("decoder_layers", &decoder_layers);
   m.def("packed_gemm", &packed_gemm);
   m.def("packed_gemm_probe", &packed_gemm_probe);
   m.def("migrate_blocks_peer", &migrate_blocks_peer);

@@ -7,6 +7,7 @@
 // lane, 256 B of a row at a time) with the 16 B chunks of a row permuted by the
 // row: whole-row reads then meet no bank twice. W rows are the A operand, x rows
 // the B operand of 16x16x32 products; sums are fp32.
+#include "linear.h"
 #include "mfma_rows.h"
 
 namespace xllm {
@@ -52,6 +53,17 @@ XLLM_DEV float ln_gated(float gate, float up) {
   const unsigned u = pack_bf16(gate, up);
   const float a = __uint_as_float(u << 16);
   return a / (1.0f + __expf(-a)) * __uint_as_float(u & 0xffff0000u);
+}
+
+// two neighbours, packed: joined with the residual's, their squares added to sq
+XLLM_DEV unsigned ln_join(unsigned y, unsigned& r, unsigned w, float& sq) {
+  const float a = __uint_as_float(y << 16) + __uint_as_float(r << 16);
+  const float b = __uint_as_float(y & 0xffff0000u) +
+                  __uint_as_float(r & 0xffff0000u);
+  sq += a * a + b * b;
+  r = pack_bf16(a, b);
+  return pack_bf16(a * __uint_as_float(w << 16),
+                   b * __uint_as_float(w & 0xffff0000u));
 }
 
 // Rows r0 .. of a matrix into an image: instruction i moves four rows
@@ -104,12 +116,14 @@ struct LnTile {
 //   M 24  4096 x 4096 10.1 -> 9.1, 6144 x 4096 15.2 -> 12.4, 8192 x 4096 16.9 -> 14.3,
 //         32000 x 4096 57 -> 48, 4096 x 14336 27.5 -> 25.3
 //   M 64  4096 x 4096 14.4 -> 13.2, 6144 x 4096 22.0 -> 17.2, 8192 x 4096 23.5 -> 18.5
-template <int NT, int XR, int NW, int D, bool GATE>
+template <int NT, int XR, int NW, int D, int MODE>
 __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w,
     const unsigned short* __restrict__ bias, const int M, const int N,
-    const int K, const long x_stride) {
+    const int K, const long x_stride, const LinearEnds ends) {
+  constexpr bool GATE = MODE & LN_GATE, SCALE = MODE & LN_SCALE,
+                 ADD = MODE & LN_ADD;
   constexpr int WR = 16 * NT;                    // rows of W
   constexpr int MT = (XR + 15) / 16;             // row tiles of x
   constexpr int T = WR * LN_K, TILE = T + XR * LN_K;
@@ -117,7 +131,7 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
   constexpr int PART = NW * 16 * MT * ROW * 2;
   constexpr int RING = NW * D * TILE;
   __shared__ __attribute__((aligned(1024))) unsigned short
-      lds[RING > PART ? RING : PART];
+      lds[RING > PART + 32 * MT ? RING : PART + 32 * MT];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
@@ -139,6 +153,33 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
   for (int ks = 0; ks < 4; ks++) {
     at[ks] = 2 * (c16 * LN_K + (((4 * ks + g) ^ c16) << 3));
     last[ks] = 2 * (half * LN_K + (((4 * ks + g) ^ half) << 3));
+  }
+  // squares of this wave's rows, wid + NW i: fetched here, summed at the end
+  constexpr int SR = SCALE ? (XR + NW - 1) / NW : 1;
+  uint4 sq[SR];
+  if constexpr (SCALE) {
+#pragma unroll
+    for (int i = 0; i < SR; i++) {
+      const int m = wid + NW * i;
+      sq[i] = mr_load(mr_buffer(ends.squares + (long)m * ends.n_squares,
+                                m < M ? ends.n_squares * 4 : 0), lane * 16);
+    }
+  }
+  // what is added at the end: this lane's columns of up to OWN rows
+  constexpr int C4 = OUT / 4;                    // columns in fours
+  constexpr int OWN = (16 * MT * C4 + NW * 64 - 1) / (NW * 64);
+  uint2 res[ADD ? OWN : 1], norm[ADD ? OWN : 1];
+  if constexpr (ADD) {
+#pragma unroll
+    for (int k = 0; k < OWN; k++) {
+      const int i = tid + k * NW * 64, m = i / C4;
+      const long n = n0 + (i % C4) * 4;
+      res[k] = norm[k] = make_uint2(0u, 0u);
+      if (m >= M || n >= n_out) continue;
+      res[k] = *reinterpret_cast<const uint2*>(ends.residual +
+                                               (long)m * n_out + n);
+      norm[k] = *reinterpret_cast<const uint2*>(ends.norm + n);
+    }
   }
   f32x4 acc[NT][MT];
 #pragma unroll
@@ -199,6 +240,29 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
       *reinterpret_cast<float4*>(part + ((wid * MT + j) * 16 + c16) * ROW +
                                  16 * n + 4 * g) =
           make_float4(acc[n][j][0], acc[n][j][1], acc[n][j][2], acc[n][j][3]);
+  float* factor = reinterpret_cast<float*>(lds + PART);
+  if constexpr (SCALE) {
+    // all rows in step: one after the other they took 2 us
+    float v[SR];
+#pragma unroll
+    for (int i = 0; i < SR; i++)
+      v[i] = __uint_as_float(sq[i].x) + __uint_as_float(sq[i].y) +
+             __uint_as_float(sq[i].z) + __uint_as_float(sq[i].w);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      float u[SR];
+#pragma unroll
+      for (int i = 0; i < SR; i++) u[i] = __shfl_xor(v[i], off, 64);
+#pragma unroll
+      for (int i = 0; i < SR; i++) v[i] += u[i];
+    }
+    float mine = v[0];
+#pragma unroll
+    for (int i = 1; i < SR; i++) mine = lane == i ? v[i] : mine;
+    const int m = wid + NW * lane;
+    if (lane < SR && m < 16 * MT)
+      factor[m] = rsqrtf(mine / (float)K + ends.eps);
+  }
   __syncthreads();
   auto sum = [&](int m, int col, float (&s)[4]) {
 #pragma unroll
@@ -209,26 +273,48 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
       else { s[0] += z.x; s[1] += z.y; s[2] += z.z; s[3] += z.w; }
     }
   };
-  constexpr int C4 = OUT / 4;                    // columns in fours
-  for (int i = tid; i < 16 * MT * C4; i += NW * 64) {
+#pragma unroll
+  for (int k = 0; k < OWN; k++) {
+    const int i = tid + k * NW * 64;
+    if (i >= 16 * MT * C4) break;
     const int m = i / C4, col = (i % C4) * 4;
     const long n = n0 + col;
-    if (m >= M || n >= n_out) continue;
+    const bool ok = m < M && n < n_out;
+    if (!ADD && !ok) continue;
     float s[4];
     sum(m, col, s);
+    const float f = SCALE ? factor[m] : 1.0f;
     if constexpr (GATE) {
       float u[4];
       sum(m, OUT + col, u);
 #pragma unroll
-      for (int k = 0; k < 4; k++) s[k] = ln_gated(s[k], u[k]);
-    } else if (bias != nullptr) {
+      for (int e = 0; e < 4; e++) s[e] = ln_gated(s[e] * f, u[e] * f);
+    } else if constexpr (SCALE) {
 #pragma unroll
-      for (int k = 0; k < 4; k++) s[k] += bf16_to_f32(bias[n + k]);
+      for (int e = 0; e < 4; e++) s[e] *= f;
+    }
+    if (MODE % 4 != LN_GATE && !ADD && bias != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) s[e] += bf16_to_f32(bias[n + e]);
     }
     uint2 o;
     o.x = pack_bf16(s[0], s[1]);
     o.y = pack_bf16(s[2], s[3]);
-    *reinterpret_cast<uint2*>(y + (long)m * n_out + n) = o;
+    const long at = (long)m * n_out + n;
+    if constexpr (ADD) {
+      float q = 0.0f;
+      if (ok) {
+        o.x = ln_join(o.x, res[k].x, norm[k].x, q);
+        o.y = ln_join(o.y, res[k].y, norm[k].y, q);
+        *reinterpret_cast<uint2*>(ends.residual + at) = res[k];
+      }
+#pragma unroll
+      for (int off = C4 / 2; off > 0; off >>= 1) q += __shfl_xor(q, off, 64);
+      if (col == 0 && m < M)
+        ends.sums[(long)m * gridDim.x + blockIdx.x] = q;
+      if (!ok) continue;
+    }
+    *reinterpret_cast<uint2*>(y + at) = o;
   }
 }
 
@@ -249,11 +335,14 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
 // 4096 x 4096 29.5 -> 22.5, 3072 x 2048 11.7 -> 11.6; 96 x 3072 x 2048 10.9 -> 9.6;
 // 192 x 6144 x 4096 30.1 -> 25.7; 512 x 3072 x 2048 16.5 -> 16.7; 256 x 3072 x 2048, as many
 // tiles of 64 x 64 either way, 11.8 -> 12.1.
-template <int NW, int MT, int LK, int S, bool GATE>
+template <int NW, int MT, int LK, int S, int MODE>
 __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w, const int M, const int N,
-    const int K, const long x_stride, const int n_tiles_n) {
+    const int K, const long x_stride, const int n_tiles_n,
+    const LinearEnds ends) {
+  constexpr bool GATE = MODE & LN_GATE, SCALE = MODE & LN_SCALE,
+                 ADD = MODE & LN_ADD;
   constexpr int WR = 16 * NW;                    // rows of W
   constexpr int WT = WR * LK, TILE = WT + 16 * MT * LK;
   constexpr int KS = LK / 64;                    // products a wave makes of a step
@@ -291,6 +380,20 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   for (int i = 0; i < XI; i++) {
     const int r = (wid * XI + i) * RPI + lane / CPR;
     x_off[i] = offset(r, min(r, m_rows - 1), x_stride);
+  }
+  // squares of the rows, SL lanes to each: fetched here, summed at the end
+  constexpr int SL = NW * 64 / (16 * MT) >= 8 ? 8 : NW * 64 / (16 * MT) >= 4 ? 4 : 2;
+  constexpr int SQ = SCALE ? 64 / (4 * SL) : 1;
+  uint4 sq[SQ];
+  if constexpr (SCALE) {
+    const auto src = mr_buffer(ends.squares + m0 * ends.n_squares,
+                               (unsigned)m_rows * ends.n_squares * 4);
+#pragma unroll
+    for (int i = 0; i < SQ; i++) {
+      const int p = (i * SL + tid % SL) * 4;
+      sq[i] = mr_load(src, p < ends.n_squares
+                               ? (tid / SL * ends.n_squares + p) * 4 : ~15u);
+    }
   }
   const int steps = K / LK;
   auto stage = [&](int t, int slot) {
@@ -378,9 +481,24 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   constexpr int ROW = WR + 8;                    // bf16 of a row, padded
   unsigned short* out = lds + NW * MT * 64 * 8;
   const int col0 = 32 * hw + 16 * hk + 4 * g;
+  float* factor = reinterpret_cast<float*>(out + 16 * MT * ROW);
+  if constexpr (SCALE) {
+    float v = 0.0f;
+#pragma unroll
+    for (int i = 0; i < SQ; i++)
+      v += __uint_as_float(sq[i].x) + __uint_as_float(sq[i].y) +
+           __uint_as_float(sq[i].z) + __uint_as_float(sq[i].w);
+#pragma unroll
+    for (int off = SL / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (tid % SL == 0 && tid / SL < 16 * MT)
+      factor[tid / SL] = rsqrtf(v / (float)K + ends.eps);
+    __syncthreads();
+  }
 #pragma unroll
   for (int j = 0; j < MT; j++) {
-    const f32x4 z = (hk ? acc[1][j] : acc[0][j]) + swap[((wid ^ (NW / 2)) * MT + j) * 64 + lane];
+    f32x4 z = (hk ? acc[1][j] : acc[0][j]) +
+              swap[((wid ^ (NW / 2)) * MT + j) * 64 + lane];
+    if (SCALE) z *= factor[16 * j + c16];
     uint2 o;
     o.x = pack_bf16(z[0], z[1]);
     o.y = pack_bf16(z[2], z[3]);
@@ -392,8 +510,10 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   for (int k = 0; k < (16 * MT * C8 + NW * 64 - 1) / (NW * 64); k++) {
     const int idx = tid + k * NW * 64;
     const int row = idx / C8, col = idx % C8 * 8;
-    if (row >= m_rows || col >= n_cols) continue;
-    uint4 v = *reinterpret_cast<const uint4*>(out + row * ROW + col);
+    const bool ok = row < m_rows && col < n_cols;
+    if (!ADD && !ok) continue;
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (ok) v = *reinterpret_cast<const uint4*>(out + row * ROW + col);
     if constexpr (GATE) {
       const uint4 u = *reinterpret_cast<const uint4*>(out + row * ROW + OUT + col);
       auto two = [](unsigned a, unsigned b) {
@@ -404,7 +524,23 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
       };
       v = make_uint4(two(v.x, u.x), two(v.y, u.y), two(v.z, u.z), two(v.w, u.w));
     }
-    *reinterpret_cast<uint4*>(y + (m0 + row) * n_out + n0 + col) = v;
+    const long at = (m0 + row) * n_out + n0 + col;
+    if constexpr (ADD) {
+      float q = 0.0f;
+      if (ok) {
+        uint4 r = *reinterpret_cast<const uint4*>(ends.residual + at);
+        const uint4 n = *reinterpret_cast<const uint4*>(ends.norm + n0 + col);
+        v = make_uint4(ln_join(v.x, r.x, n.x, q), ln_join(v.y, r.y, n.y, q),
+                       ln_join(v.z, r.z, n.z, q), ln_join(v.w, r.w, n.w, q));
+        *reinterpret_cast<uint4*>(ends.residual + at) = r;
+      }
+#pragma unroll
+      for (int off = C8 / 2; off > 0; off >>= 1) q += __shfl_xor(q, off, 64);
+      if (idx % C8 == 0 && row < m_rows)
+        ends.sums[(m0 + row) * n_tiles_n + blockIdx.x % n_tiles_n] = q;
+      if (!ok) continue;
+    }
+    *reinterpret_cast<uint4*>(y + at) = v;
   }
 }
 
@@ -498,18 +634,20 @@ static bool linear_one_tile(int M, int N, int K) {
 // A workgroup that has a CU to itself takes all of its LDS: two tiles a wave, or
 // more waves. Where there are more than CUs, two of them share one: M 24, 32000 x
 // 4096 48.4, with two tiles 49.2; 18944 x 4096 33.4 | 34.5.
-template <bool GATE>
+template <int MODE>
 static void launch_stream(unsigned short* y, const unsigned short* x,
                           const unsigned short* w, const unsigned short* bias,
                           int M, int N, int K, long x_stride,
-                          hipStream_t stream) {
+                          const LinearEnds& ends, hipStream_t stream) {
+  constexpr bool GATE = MODE & LN_GATE;
   const bool one = linear_one_tile(M, N, K);
   const int out = (one ? 16 : 32) / (GATE ? 2 : 1), n_out = N / (GATE ? 2 : 1);
   const dim3 grid((n_out + out - 1) / out);
   const bool few = grid.x <= 256;
 #define LN_STREAM(NT, XR, NW, D)                                               \
-  hipLaunchKernelGGL((linear_stream_kernel<NT, XR, NW, D, GATE>), grid,        \
-                     dim3(NW * 64), 0, stream, y, x, w, bias, M, N, K, x_stride)
+  hipLaunchKernelGGL((linear_stream_kernel<NT, XR, NW, D, MODE>), grid,        \
+                     dim3(NW * 64), 0, stream, y, x, w, bias, M, N, K,         \
+                     x_stride, ends)
   if (one) {
     if (M <= 8) LN_STREAM(1, 8, 4, 2);
     else if (M <= 16) LN_STREAM(1, 16, 4, 2);
@@ -528,18 +666,20 @@ static void launch_stream(unsigned short* y, const unsigned short* x,
 #undef LN_STREAM
 }
 
-template <bool GATE>
+template <int MODE>
 static void launch_tile(unsigned short* y, const unsigned short* x,
                         const unsigned short* w, int M, int N, int K,
-                        long x_stride, hipStream_t stream) {
+                        long x_stride, const LinearEnds& ends,
+                        hipStream_t stream) {
+  constexpr bool GATE = MODE & LN_GATE;
   const int n_out = N / (GATE ? 2 : 1);
 #define LN_TILE(NW, MT, LK, S)                                                 \
   do {                                                                         \
     constexpr int OUT = 16 * NW / (GATE ? 2 : 1);                              \
     const int tn = (n_out + OUT - 1) / OUT, tm = (M + 16 * MT - 1) / (16 * MT); \
-    hipLaunchKernelGGL((linear_tile_kernel<NW, MT, LK, S, GATE>),              \
+    hipLaunchKernelGGL((linear_tile_kernel<NW, MT, LK, S, MODE>),              \
                        dim3((unsigned)(tn * tm)), dim3(NW * 64), 0, stream, y, \
-                       x, w, M, N, K, x_stride, tn);                           \
+                       x, w, M, N, K, x_stride, tn, ends);                     \
   } while (0)
   long turns;
   switch (linear_shape(M, N, &turns)) {
@@ -553,17 +693,34 @@ static void launch_tile(unsigned short* y, const unsigned short* x,
 #undef LN_TILE
 }
 
-// gate: W = [gates | ups], y [M, N / 2] = silu(x gates^T) (x ups^T)
+// Tiles of N that such a product has: parts of LN_ADD's sums
+int linear_tiles(int M, int N, int K, int kind) {
+  if (kind == 1) return linear_one_tile(M, N, K) ? (N + 15) / 16 : (N + 31) / 32;
+  long turns;
+  return linear_shape(M, N, &turns) == 0 ? (N + 127) / 128 : (N + 63) / 64;
+}
+
+// mode: LN_GATE: W = [gates | ups], y [M, N / 2] = silu(x gates^T) (x ups^T);
+// LN_SCALE with or without it, or LN_ADD alone: see there
 void launch_linear(unsigned short* y, const unsigned short* x,
                    const unsigned short* w, const unsigned short* bias, int M,
-                   int N, int K, long x_stride, int kind, bool gate,
-                   hipStream_t stream) {
-  if (kind == 1)
-    (gate ? launch_stream<true> : launch_stream<false>)(
-        y, x, w, bias, M, N, K, x_stride, stream);
-  else
-    (gate ? launch_tile<true> : launch_tile<false>)(y, x, w, M, N, K, x_stride,
-                                                    stream);
+                   int N, int K, long x_stride, int kind, int mode,
+                   const LinearEnds& ends, hipStream_t stream) {
+#define LN_MODE(MODE)                                                          \
+  case MODE:                                                                   \
+    if (kind == 1)                                                             \
+      launch_stream<MODE>(y, x, w, bias, M, N, K, x_stride, ends, stream);     \
+    else                                                                       \
+      launch_tile<MODE>(y, x, w, M, N, K, x_stride, ends, stream);             \
+    break
+  switch (mode) {
+    LN_MODE(0);
+    LN_MODE(LN_GATE);
+    LN_MODE(LN_SCALE);
+    LN_MODE(LN_SCALE | LN_GATE);
+    LN_MODE(LN_ADD);
+  }
+#undef LN_MODE
 }
 
 }  // namespace xllm

@@ -115,6 +115,12 @@ XLLM_DEV void mr_to_lds(__amdgpu_buffer_rsrc_t src, unsigned off,
   __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_void*)dst, 16, off, base,
                                            0, 0);
 }
+// the same to registers
+XLLM_DEV uint4 mr_load(__amdgpu_buffer_rsrc_t src, unsigned off) {
+  typedef __attribute__((ext_vector_type(4))) unsigned u4;
+  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(src, off, 0, 0);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 XLLM_DEV f32x16 mr_zero() {
   f32x16 z;
 #pragma unroll

@@ -110,14 +110,9 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = LlamaMLP(cfg, dtype)
         self.eps = cfg.rms_eps
 
-    def _native(self, x, residual, positions, kv_cache, meta, cos_sin):
-        """The layer as one native call, or None where a module in it is not the
-        plain one or torch has to see the calls: gradients, modes, tracing."""
-        if not (x.is_cuda and ops.HAS_EXT and torch.is_inference_mode_enabled()
-                and ps.tp_size() == 1) or module_hooks._global_forward_hooks \
-                or module_hooks._global_forward_pre_hooks \
-                or torch.compiler.is_compiling():
-            return None
+    def _native_weights(self, kv_cache):
+        """What the native layers take of this one, or None where a module in it
+        is not the plain one."""
         attn, mlp = self._modules["attn"], self._modules["mlp"]
         if not (_plain(attn, LlamaAttention) and _plain(mlp, LlamaMLP)):
             return None
@@ -133,22 +128,12 @@ class LlamaDecoderLayer(nn.Module):
                 or attn.head_dim != 128 or kv_cache[0].shape[-1] != 128:
             return None
         w = (self.input_norm, qkv.weight, qkv.bias, o.weight, self.post_norm,
-             gate_up.weight, gate_up.bias, down.weight)
-        if torch.overrides.has_torch_function((x, residual, *w, *kv_cache)):
-            return None
-        ms0 = ms1 = 0
-        if attn.mrope_sections and positions.dim() != 1:
-            ms0 = int(attn.mrope_sections[0])
-            ms1 = ms0 + int(attn.mrope_sections[1])
-        return ops.decoder_layer(
-            x, residual, *w, self.eps, attn.n_heads, attn.scale, positions,
-            meta.slot_mapping, cos_sin, *kv_cache, ms0, ms1,
-            meta.num_prefill_tokens, meta.num_decode_tokens,
-            meta.prefill_block_tables, meta.cu_q, meta.prefill_seq_lens,
-            meta.decode_block_tables, meta.decode_seq_lens)
+             gate_up.weight, gate_up.bias, down.weight, *kv_cache)
+        return None if torch.overrides.has_torch_function(w) else w
 
     def forward(self, x, residual, positions, kv_cache, meta, cos_sin):
-        done = self._native(x, residual, positions, kv_cache, meta, cos_sin)
+        done = _native_layers([self], x, residual, positions, [kv_cache], meta,
+                              cos_sin)
         if done is not None:
             return done
         if residual is None:
@@ -161,6 +146,36 @@ class LlamaDecoderLayer(nn.Module):
         x, residual = ops.fused_add_rmsnorm(x, residual, self.post_norm, self.eps)
         x = self.mlp(x)
         return x, residual
+
+
+def _native_layers(layers, x, residual, positions, kv_caches, meta, cos_sin):
+    """Layers as one native call, or None where one of their modules is not the
+    plain one or torch has to see the calls: gradients, modes, tracing."""
+    if not (x.is_cuda and ops.HAS_EXT and torch.is_inference_mode_enabled()
+            and ps.tp_size() == 1) or module_hooks._global_forward_hooks \
+            or module_hooks._global_forward_pre_hooks \
+            or torch.compiler.is_compiling() \
+            or torch.overrides.has_torch_function((x, residual)):
+        return None
+    weights = []
+    for layer, kv_cache in zip(layers, kv_caches):
+        w = layer._native_weights(kv_cache)
+        if w is None:
+            return None
+        weights.append(w)
+    first = layers[0]
+    attn = first.attn
+    if any(layer.eps != first.eps for layer in layers):
+        return None
+    ms0 = ms1 = 0
+    if attn.mrope_sections and positions.dim() != 1:
+        ms0 = int(attn.mrope_sections[0])
+        ms1 = ms0 + int(attn.mrope_sections[1])
+    return ops.decoder_layers(
+        x, residual, weights, first.eps, attn.n_heads, attn.scale, positions,
+        meta.slot_mapping, cos_sin, ms0, ms1, meta.num_prefill_tokens,
+        meta.num_decode_tokens, meta.prefill_block_tables, meta.cu_q,
+        meta.prefill_seq_lens, meta.decode_block_tables, meta.decode_seq_lens)
 
 
 class LlamaForCausalLM(nn.Module):
@@ -203,10 +218,17 @@ class LlamaForCausalLM(nn.Module):
                 meta: AttnMetadata,
                 inputs_embeds: Optional[torch.Tensor] = None):
         x = inputs_embeds if inputs_embeds is not None else self.embed(input_ids)
-        residual = None
-        for i, layer in enumerate(self.layers):
-            x, residual = layer(x, residual, positions, kv_caches[i], meta,
-                                self.cos_sin)
+        layers, done = list(self.layers), None
+        if layers and all(_plain(m, LlamaDecoderLayer) for m in layers):
+            done = _native_layers(layers, x, None, positions, kv_caches, meta,
+                                  self.cos_sin)
+        if done is not None:
+            x, residual = done
+        else:
+            residual = None
+            for i, layer in enumerate(layers):
+                x, residual = layer(x, residual, positions, kv_caches[i], meta,
+                                    self.cos_sin)
         x, _ = ops.fused_add_rmsnorm(x, residual, self.final_norm, self.cfg.rms_eps)
         return x
 

@@ -247,11 +247,11 @@ def linear_gated(x, weight, bias=None):
     return silu_and_mul(linear(x, weight, bias))
 
 
-def decoder_layer(*args):
-    """One layer of the dense decoders as a native call (GPU only): the layer's
-    new (x, residual), or None where torch's dispatcher must not be passed by."""
+def decoder_layers(*args):
+    """Layers of the dense decoders as a native call (GPU only): the last one's new
+    (x, residual), or None where torch's dispatcher must not be passed by."""
     _require_ext()
-    return _ops.decoder_layer(*args)
+    return _ops.decoder_layers(*args)
 
 
 def skinny_gemm(a, b, bias=None):

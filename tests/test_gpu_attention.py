@@ -107,6 +107,30 @@ def test_prefill_edges(dim, lens, ctx, kv_heads, per):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("lens,ctx,sign", [
+    ([300, 1, 257, 32, 0, 333], [0, 2300, 17, 5, 9, 100], 1.0),  # row tiles
+    ([60, 850], [4500, 0], -1.0),                   # over 64 tiles of keys
+    ([13] * 70, [2100] + [3] * 69, 1.0),            # more than 64 sequences
+])
+def test_prefill_many_tiles(lens, ctx, sign):
+    """Calls of two turns of workgroups and 2048 keys and more."""
+    kv_heads, per, dim = 16, 8, 128
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(lens))
+    heads, scale = kv_heads * per, sign * dim ** -0.5
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)))
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)])
+    dev = [t.cuda() for t in (k, v, table, cu.int(), sl.int())]
+    wide = torch.full((sum(lens), (heads + 1) * dim), 7.0,
+                      dtype=torch.bfloat16, device="cuda")
+    out = wide[:, :heads * dim].unflatten(-1, (heads, dim))
+    got = ops.paged_attn_prefill(
+        rows.cuda()[:, :heads * dim].unflatten(-1, (heads, dim)), *dev, scale,
+        out=out)
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    check(got, *want(q, k, v, table, lens, ctx, scale))
+    assert (wide[:, heads * dim:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("ctx", [[3, 0], [2600, 900]])      # whole; in parts
 def test_prefill_leaves_other_rows(dim, ctx):

@@ -1,8 +1,8 @@
 // Paged attention of prompt rows for the dense decoders: bf16 in and out, causal
-// (kernel and its reasons: paged_rows.h).
+// (kernels and their reasons: paged_rows.h, paged_long.h).
 //
 // Parity: reference engine's paged-attention prefill.
-#include "paged_rows.h"
+#include "paged_long.h"
 
 namespace xllm {
 
@@ -22,6 +22,13 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws_o, float* ws_ml,
                                float scale, int n_qheads, int n_kv, int D,
                                int max_blocks, long q_stride, long out_stride,
                                int n_part, hipStream_t stream) {
+  if (D == 128 && n_part == 1 &&
+      paged_long_takes(tokens, n_seqs, n_qheads / n_kv, n_kv, max_blocks)) {
+    paged_long(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens,
+               n_seqs, scale, n_qheads, n_kv, max_blocks, q_stride, out_stride,
+               stream);
+    return;
+  }
   auto go = D == 128 ? paged_rows<128, 1, false> : paged_rows<64, 3, false>;
   go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, cu_q, seq_lens,
      tokens, n_seqs, scale, n_qheads, n_kv, max_blocks, q_stride, out_stride,

@@ -58,6 +58,7 @@ namespace xllm {
 // Row tile `b` of the batch -> sequence and tile within it; later tiles of a
 // sequence (more keys) come first. False: past the last one. One wave looks
 // 64 sequences over at a time.
+template <int ROWS>
 XLLM_DEV bool pf_locate(int b, const int* cu_q, int n_seqs, int G, int lane,
                         int* s, int* lt) {
   int acc = 0;
@@ -65,7 +66,7 @@ XLLM_DEV bool pf_locate(int b, const int* cu_q, int n_seqs, int G, int lane,
     const int i = base + lane;
     int nt = 0;
     if (i < n_seqs)
-      nt = ((cu_q[i + 1] - cu_q[i]) * G + PF_ROWS - 1) / PF_ROWS;
+      nt = ((cu_q[i + 1] - cu_q[i]) * G + ROWS - 1) / ROWS;
     int sum = nt;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
   const int kvh = blockIdx.x % n_kv;
   const int part = (blockIdx.x / n_kv) % n_part;
   int seq, lt;
-  if (!pf_locate(blockIdx.x / (n_kv * n_part), cu_q, n_seqs, G, lane, &seq,
+  if (!pf_locate<PF_ROWS>(blockIdx.x / (n_kv * n_part), cu_q, n_seqs, G, lane, &seq,
                  &lt))
     return;
   const int q_start = cu_q[seq];
@@ -364,12 +365,13 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
 // weights: 2 x 64 rows of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of 16
 // over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles) 374 | 298 |
 // 302 | 325; 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
+template <int ROWS>
 inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
-  return tokens * G / PF_ROWS + n_seqs;
+  return tokens * G / ROWS + n_seqs;
 }
 inline int paged_rows_parts(long tokens, int n_seqs, int G, int n_kv,
                             long max_blocks, int terms) {
-  const long wgs = paged_rows_tiles(tokens, n_seqs, G) * n_kv;
+  const long wgs = paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv;
   const long most = max_blocks * PF_BS / ((terms > 1 ? 4 : 8) * PF_KT);
   long p = wgs > 0 ? (512 + wgs / 2) / wgs : 1;
   if (p > most) p = most;
@@ -388,7 +390,7 @@ inline void paged_rows(void* out, float* ws_o, float* ws_ml,
   const int G = n_qheads / n_kv;
   if (tokens == 0 || n_seqs <= 0) return;
   const dim3 grid(
-      (unsigned)(paged_rows_tiles(tokens, n_seqs, G) * n_kv * n_part));
+      (unsigned)(paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv * n_part));
   hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE>), grid, dim3(256),
                      0, stream, out, ws_o, ws_ml, q, k_cache, v_cache,
                      block_tables, cu_q, seq_lens, n_seqs, scale, G, n_kv,

@@ -33,13 +33,16 @@ namespace xllm {
 // 4200 new tokens before 100 behind 3000 cached ones were 4% slower than with the
 // kernel of paged_rows.h.
 XLLM_DEV bool pl_locate(int b, const int* cu_q, const int* seq_lens, int n_seqs,
-                        int G, int lane, int* s, int* lt) {
-  if (n_seqs > 64) return pf_locate<PL_ROWS>(b, cu_q, n_seqs, G, lane, s, lt);
-  int nt = 0, top = 0;                           // of sequence `lane`
+                        int G, int lane, PfPlace* place) {
+  if (n_seqs > 64)
+    return pf_locate<PL_ROWS>(b, cu_q, seq_lens, n_seqs, G, lane, place);
+  int start = 0, len = 0, keys = 0;              // of sequence `lane`
   if (lane < n_seqs) {
-    nt = ((cu_q[lane + 1] - cu_q[lane]) * G + PL_ROWS - 1) / PL_ROWS;
-    top = seq_lens[lane] * G;
+    start = cu_q[lane];
+    len = cu_q[lane + 1] - start;
+    keys = seq_lens[lane];
   }
+  const int nt = (len * G + PL_ROWS - 1) / PL_ROWS, top = keys * G;
   int most = nt > 0 ? top : 0;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, 64));
@@ -67,8 +70,10 @@ XLLM_DEV bool pl_locate(int b, const int* cu_q, const int* seq_lens, int n_seqs,
       unsigned long long at = __ballot(level >= first && level < last);
       for (; r > 0; r--) at &= at - 1;
       const int i = __builtin_amdgcn_readfirstlane(__ffsll(at) - 1);
-      *s = i;
-      *lt = __builtin_amdgcn_readlane(last, i) - 1 - level;
+      *place = {i, __builtin_amdgcn_readlane(last, i) - 1 - level,
+                __builtin_amdgcn_readlane(start, i),
+                __builtin_amdgcn_readlane(len, i),
+                __builtin_amdgcn_readlane(keys, i)};
       return true;
     }
     acc += __shfl(sum, 63, 64);
@@ -102,12 +107,11 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
   const int h = lane >> 5, c32 = lane & 31;
 
   const int kvh = blockIdx.x % n_kv;
-  int seq, lt;
-  if (!pl_locate(blockIdx.x / n_kv, cu_q, seq_lens, n_seqs, G, lane, &seq, &lt))
+  PfPlace place;
+  if (!pl_locate(blockIdx.x / n_kv, cu_q, seq_lens, n_seqs, G, lane, &place))
     return;
-  const int q_start = cu_q[seq];
-  const int q_len = cu_q[seq + 1] - q_start;
-  const int seq_len = seq_lens[seq];
+  const int seq = place.seq, lt = place.lt, q_start = place.q_start,
+            q_len = place.q_len, seq_len = place.seq_len;
   const int ctx = seq_len - q_len;
   const int rows = q_len * G;
 

@@ -1,6 +1,6 @@
 """Decoder layers as one native call against the calls of their modules. What enters
-and leaves attention of a first layer is the same bits. Norms between two products
-are split over these: as many roundings, of other values, so that a layer's result
+and leaves attention of a first layer is the same bits. Norms and gates between two
+products are made by these, without some of the roundings, so that a layer's result
 differs by a few independent errors of 2^-9: within 2^-7 in the 2-norm, 2^-6 after
 three layers."""
 import pytest
@@ -92,8 +92,6 @@ def test_native_layers(name, prompts, decodes, first, n_layers, monkeypatch):
         assert torch.equal(a, b)
     for a, b in zip(got, want):
         assert _off(a, b) < 2.0 ** (-7 if n_layers == 1 else -6)
-    if n_layers == 1:
-        assert torch.equal(got[1], want[1])
     with torch.no_grad():                     # gradients could be asked for
         _step(layers, cfg, prompts, decodes, first)
     assert len(calls) == 1

@@ -81,10 +81,10 @@ def test_shapes_of_prompt_tiles(M, N, K, stride):
 @pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (4112, 640), (8208, 384),
                                  (3088, 2048)])
 def test_gated(M, N, K):
-    """Gates and their partners in one product, against fp64 of the rounded sums:
-    the two roundings of 2^-8 of a sum (silu turns one of the gate into at most
-    1.1 of its size) and that of the result; 2^-17 as above, times the other
-    factor."""
+    """Gates and their partners in one product, against fp64: 2^-8 for the result's
+    rounding, and of each sum, where a caller's two products round them, 2^-8 more
+    and 2^-17 as above, times the other factor (silu turns an error of the gate
+    into at most 1.1 of its size)."""
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x, w = (torch.randn(r, K, generator=g, device="cuda").to(torch.bfloat16)
             for r in (M, N))

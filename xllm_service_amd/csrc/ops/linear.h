@@ -10,8 +10,9 @@ namespace xllm {
 // weights (the rows of the next product but for their factors), sums the squares of
 // this tile's columns. So a norm needs no launch of its own between two products: 4.6 us
 // of a decode step, 3.4 of a prompt's, for 1.5 more in the two products. 8 layers, 24
-// rows of 4096: 701 -> 677 us, 300 of 2048 589 -> 563. What is rounded is what was
-// rounded before: the sum, the residual, the row times the weights.
+// rows of 4096: 701 -> 677 us, 300 of 2048 589 -> 563. Of the norm's and the gate's own
+// roundings the residual's and the rows' are left, the sums' in between are not made:
+// error against 64 bits 0.0189 -> 0.0158 and 0.0132 -> 0.0118.
 enum { LN_GATE = 1, LN_SCALE = 2, LN_ADD = 4 };
 struct LinearEnds {
   const float* squares = nullptr;            // [M][n_squares]

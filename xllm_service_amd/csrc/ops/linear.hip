@@ -48,18 +48,15 @@ XLLM_DEV long ln_gate_row(long first, long half, int r) {
   return r < ROWS / 2 ? min(first + r, half - 1)
                       : half + min(first + r - ROWS / 2, half - 1);
 }
-// silu(gate) up of two sums, as act_and_mul_kernel makes it of rounded ones
+// silu(gate) up of two sums
 XLLM_DEV float ln_gated(float gate, float up) {
-  const unsigned u = pack_bf16(gate, up);
-  const float a = __uint_as_float(u << 16);
-  return a / (1.0f + __expf(-a)) * __uint_as_float(u & 0xffff0000u);
+  return gate / (1.0f + __expf(-gate)) * up;
 }
 
-// two neighbours, packed: joined with the residual's, their squares added to sq
-XLLM_DEV unsigned ln_join(unsigned y, unsigned& r, unsigned w, float& sq) {
-  const float a = __uint_as_float(y << 16) + __uint_as_float(r << 16);
-  const float b = __uint_as_float(y & 0xffff0000u) +
-                  __uint_as_float(r & 0xffff0000u);
+// two neighbours: joined with the residual's, their squares added to sq
+XLLM_DEV unsigned ln_join(float a, float b, unsigned& r, unsigned w, float& sq) {
+  a += __uint_as_float(r << 16);
+  b += __uint_as_float(r & 0xffff0000u);
   sq += a * a + b * b;
   r = pack_bf16(a, b);
   return pack_bf16(a * __uint_as_float(w << 16),
@@ -304,8 +301,8 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
     if constexpr (ADD) {
       float q = 0.0f;
       if (ok) {
-        o.x = ln_join(o.x, res[k].x, norm[k].x, q);
-        o.y = ln_join(o.y, res[k].y, norm[k].y, q);
+        o.x = ln_join(s[0], s[1], res[k].x, norm[k].x, q);
+        o.y = ln_join(s[2], s[3], res[k].y, norm[k].y, q);
         *reinterpret_cast<uint2*>(ends.residual + at) = res[k];
       }
 #pragma unroll
@@ -478,7 +475,9 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
 #pragma unroll
   for (int j = 0; j < MT; j++) swap[(wid * MT + j) * 64 + lane] = hk ? acc[0][j] : acc[1][j];
   __syncthreads();
-  constexpr int ROW = WR + 8;                    // bf16 of a row, padded
+  // rows on their way out: bf16, or what something is still done to, padded
+  constexpr bool WIDE = GATE || ADD;
+  constexpr int ROW = WIDE ? 2 * (WR + 4) : WR + 8;
   unsigned short* out = lds + NW * MT * 64 * 8;
   const int col0 = 32 * hw + 16 * hk + 4 * g;
   float* factor = reinterpret_cast<float*>(out + 16 * MT * ROW);
@@ -499,10 +498,14 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     f32x4 z = (hk ? acc[1][j] : acc[0][j]) +
               swap[((wid ^ (NW / 2)) * MT + j) * 64 + lane];
     if (SCALE) z *= factor[16 * j + c16];
-    uint2 o;
-    o.x = pack_bf16(z[0], z[1]);
-    o.y = pack_bf16(z[2], z[3]);
-    *reinterpret_cast<uint2*>(out + (16 * j + c16) * ROW + col0) = o;
+    if constexpr (WIDE) {
+      *reinterpret_cast<f32x4*>(out + (16 * j + c16) * ROW + 2 * col0) = z;
+    } else {
+      uint2 o;
+      o.x = pack_bf16(z[0], z[1]);
+      o.y = pack_bf16(z[2], z[3]);
+      *reinterpret_cast<uint2*>(out + (16 * j + c16) * ROW + col0) = o;
+    }
   }
   __syncthreads();
   constexpr int C8 = OUT / 8;                    // columns in eights
@@ -513,16 +516,25 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     const bool ok = row < m_rows && col < n_cols;
     if (!ADD && !ok) continue;
     uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (ok) v = *reinterpret_cast<const uint4*>(out + row * ROW + col);
-    if constexpr (GATE) {
-      const uint4 u = *reinterpret_cast<const uint4*>(out + row * ROW + OUT + col);
-      auto two = [](unsigned a, unsigned b) {
-        return pack_bf16(
-            ln_gated(__uint_as_float(a << 16), __uint_as_float(b << 16)),
-            ln_gated(__uint_as_float(a & 0xffff0000u),
-                     __uint_as_float(b & 0xffff0000u)));
+    float f[8];
+    if constexpr (WIDE) {
+      auto eight = [&](int at, float (&to)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          *reinterpret_cast<f32x4*>(to + e) = *reinterpret_cast<const f32x4*>(
+              out + row * ROW + 2 * (at + e));
       };
-      v = make_uint4(two(v.x, u.x), two(v.y, u.y), two(v.z, u.z), two(v.w, u.w));
+      if (ok) eight(col, f);
+      if constexpr (GATE) {
+        float u[8];
+        eight(OUT + col, u);
+#pragma unroll
+        for (int e = 0; e < 8; e++) f[e] = ln_gated(f[e], u[e]);
+        v = make_uint4(pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]),
+                       pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7]));
+      }
+    } else {
+      v = *reinterpret_cast<const uint4*>(out + row * ROW + col);
     }
     const long at = (m0 + row) * n_out + n0 + col;
     if constexpr (ADD) {
@@ -530,8 +542,10 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
       if (ok) {
         uint4 r = *reinterpret_cast<const uint4*>(ends.residual + at);
         const uint4 n = *reinterpret_cast<const uint4*>(ends.norm + n0 + col);
-        v = make_uint4(ln_join(v.x, r.x, n.x, q), ln_join(v.y, r.y, n.y, q),
-                       ln_join(v.z, r.z, n.z, q), ln_join(v.w, r.w, n.w, q));
+        v = make_uint4(ln_join(f[0], f[1], r.x, n.x, q),
+                       ln_join(f[2], f[3], r.y, n.y, q),
+                       ln_join(f[4], f[5], r.z, n.z, q),
+                       ln_join(f[6], f[7], r.w, n.w, q));
         *reinterpret_cast<uint4*>(ends.residual + at) = r;
       }
 #pragma unroll

@@ -131,6 +131,32 @@ def test_prefill_many_tiles(lens, ctx, sign):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [
+    (1, 1, 128, [1, 127], [127, 0], 1.0),            # a tile for some waves only
+    (3, 1, 64, [33, 31, 32], [96, 64, 65], -1.0),    # edges of row and key tiles
+    (2, 7, 128, [9, 30, 0, 2], [640, 1, 64, 255], 1.0),
+    (1, 5, 64, [40], [984], 1.0),                    # four turns of waves
+    (1, 3, 128, [100, 5], [1948, 0], -1.0),          # eight
+    (2, 1, 64, [3] * 70, [150] + [0] * 69, 1.0),     # more than 64 sequences
+])
+def test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign):
+    """Waves of a workgroup that share out the keys of its rows."""
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(lens))
+    heads, scale = kv_heads * per, sign * dim ** -0.5
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)))
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)])
+    dev = [t.cuda() for t in (k, v, table, cu.int(), sl.int())]
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    wide = torch.full((sum(lens), (heads + 1) * dim), 7.0,
+                      dtype=torch.bfloat16, device="cuda")
+    out = wide[:, :heads * dim].unflatten(-1, (heads, dim))
+    got = ops.paged_attn_prefill(
+        rows.cuda()[:, :heads * dim].unflatten(-1, (heads, dim)), *dev, scale,
+        out=out)
+    check(got, *want(q, k, v, table, lens, ctx, scale))
+    assert (wide[:, heads * dim:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("ctx", [[3, 0], [2600, 900]])      # whole; in parts
 def test_prefill_leaves_other_rows(dim, ctx):

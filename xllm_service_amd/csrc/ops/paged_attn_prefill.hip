@@ -1,15 +1,18 @@
 // Paged attention of prompt rows for the dense decoders: bf16 in and out, causal
-// (kernels and their reasons: paged_rows.h, paged_long.h).
+// (kernels and their reasons: paged_rows.h, paged_long.h, paged_short.h).
 //
 // Parity: reference engine's paged-attention prefill.
 #include "paged_long.h"
+#include "paged_short.h"
 
 namespace xllm {
 
 int paged_attn_prefill_parts(long tokens, int n_seqs, int G, int n_kv, int D,
                              int max_blocks) {
-  return paged_rows_parts(tokens, n_seqs, G, n_kv, max_blocks,
-                          D == 128 ? 1 : 3);
+  const int terms = D == 128 ? 1 : 3;
+  return paged_short_takes(tokens, n_seqs, G, n_kv, max_blocks, terms)
+             ? 1
+             : paged_rows_parts(tokens, n_seqs, G, n_kv, max_blocks, terms);
 }
 
 // 64-wide heads ran on fp32 weights before they had a kernel and still do
@@ -22,6 +25,14 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws_o, float* ws_ml,
                                float scale, int n_qheads, int n_kv, int D,
                                int max_blocks, long q_stride, long out_stride,
                                int n_part, hipStream_t stream) {
+  if (tokens == 0 || n_seqs <= 0) return;
+  if (paged_short_takes(tokens, n_seqs, n_qheads / n_kv, n_kv, max_blocks,
+                        D == 128 ? 1 : 3)) {
+    auto go = D == 128 ? paged_short<128, 1> : paged_short<64, 3>;
+    go(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
+       scale, n_qheads, n_kv, max_blocks, q_stride, out_stride, stream);
+    return;
+  }
   if (D == 128 && n_part == 1 &&
       paged_long_takes(tokens, n_seqs, n_qheads / n_kv, n_kv, max_blocks)) {
     paged_long(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens,

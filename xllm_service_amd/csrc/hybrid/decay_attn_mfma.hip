@@ -20,10 +20,12 @@
 // Chunks of 128 tokens halve the scratch traffic of 64 (a record is a whole
 // state per head), and the products within a chunk they add are cheap.
 //
-// Measured, 3 prompts of 853-1657 tokens, 16 heads of 128 x 128: sum 20 us, scan
-// 15 us (70 MB), out 31 us; 665 us as a recurrence on the vector unit, two
-// passes and a scan. out and sum run one round of workgroups whose phases
-// (fetch, activate, split, multiply) follow each other; two share a CU.
+// Measured, 3 prompts of 853-1657 tokens, 16 heads of 128 x 128: sum 18.7 us (64 MB),
+// scan 14.4 (70 MB, the rate of a copy), out 30.6 (111 MB); 665 us as a recurrence on
+// the vector unit, two passes and a scan. out and sum run one round of workgroups whose
+// phases (activate, split, multiply) follow each other, two to a CU, and are bound by
+// the vector unit: activations and splits. What a phase reads is fetched during the one
+// before it: 68.0 -> 61.9 us in all.
 #include "../ops/mfma_rows.h"
 #include "recurrent_chunks.h"
 
@@ -55,20 +57,24 @@ XLLM_DEV bool dm_locate(const DMArgs& P, int* s, int* c, int* t0, int* len) {
 
 struct alignas(16) dm_u4 { unsigned x[4]; };
 
-// 8 neighbouring activations, packed. x / (1 + e^-x) with v_rcp and one Newton
-// step in place of a division: half its instructions, and the same bf16 for
-// every bf16 input. The denominator is 2^-24 of itself: the reciprocal of 1e38
-// would be below what v_rcp returns.
-XLLM_DEV dm_u4 dm_act(const unsigned short* p) {
-  constexpr float s = 0x1p-24f;
-  const ushort8_t x = *reinterpret_cast<const ushort8_t*>(p);
+XLLM_DEV ushort8_t dm_row(const unsigned short* p) {
+  return *reinterpret_cast<const ushort8_t*>(p);
+}
+// 8 neighbouring activations, packed. x / (1 + e^-x) with v_rcp in place of a
+// division. The denominator is 2^-24 of itself: the reciprocal of 1e38 would be below
+// what v_rcp returns. Its 1 is a step of 2^-23 larger: what v_rcp and v_exp return is
+// then rounded to the bf16 number that the division gives for every bf16 input (without
+// it for all but one; e^-x from a log2(e) up to 5 steps smaller or 2 larger changes
+// none, so this is no close call). A Newton step on the reciprocal, which does that too,
+// costs 2.3 us of 70.
+XLLM_DEV dm_u4 dm_act(const ushort8_t& x) {
+  constexpr float s = 0x1p-24f, one = s * (1.0f + 0x1p-23f);
   float v[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const float z = bf16_to_f32(x.x[j]);
-    const float d = fmaf(__expf(-z), s, s);       // infinite below -88.7: r = 0
-    const float r = __builtin_amdgcn_rcpf(d);
-    v[j] = z * (s * fmaf(fmaf(-fminf(d, 3e38f), r, 1.0f), r, r));
+    const float d = fmaf(__expf(-z), s, one);     // infinite below -88.7: 0
+    v[j] = z * (s * __builtin_amdgcn_rcpf(d));
   }
   dm_u4 y;
 #pragma unroll
@@ -132,15 +138,31 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
   const int kbase = mr_col_base<D>(lane), vbase = mr_col_base<V>(lane);
   const int d0 = (w & 1) * DT, e0 = (w >> 1) * VT;   // first tiles
 
+  constexpr int KI = ST * (D / 8) / 256, VI = ST * (V / 8) / 256;
+  ushort8_t kr[KI], vr[VI];
+  auto fetch = [&](int b0) {                      // rows past the end: the last
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const int idx = tid + i * 256, r = min(b0 + idx / (D / 8), len - 1);
+      kr[i] = dm_row(P.k + (long)(t0 + r) * P.k_stride + hd * D +
+                     idx % (D / 8) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < VI; ++i) {
+      const int idx = tid + i * 256, r = min(b0 + idx / (V / 8), len - 1);
+      vr[i] = dm_row(P.v + (long)(t0 + r) * P.v_stride + hd * V +
+                     idx % (V / 8) * 8);
+    }
+  };
+  if (len > 0) fetch(0);
   for (int b0 = 0; b0 < len; b0 += ST) {
     __syncthreads();                              // also: pw is there
 #pragma unroll
-    for (int i = 0; i < ST * (D / 8) / 256; ++i) {
+    for (int i = 0; i < KI; ++i) {
       const int idx = tid + i * 256, r = idx / (D / 8), ch = idx % (D / 8);
       float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if (b0 + r < len) {
-        const dm_u4 y =
-            dm_act(P.k + (long)(t0 + b0 + r) * P.k_stride + hd * D + ch * 8);
+        const dm_u4 y = dm_act(kr[i]);
         const float wgt = pw[len - 1 - b0 - r];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -151,15 +173,15 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
       dm_split(x, ks + r * D + ((ch ^ mr_swz_cols<D>(r)) << 3), ST * D);
     }
 #pragma unroll
-    for (int i = 0; i < ST * (V / 8) / 256; ++i) {
+    for (int i = 0; i < VI; ++i) {
       const int idx = tid + i * 256, r = idx / (V / 8), ch = idx % (V / 8);
       dm_u4 y = {{0u, 0u, 0u, 0u}};
-      if (b0 + r < len)
-        y = dm_act(P.v + (long)(t0 + b0 + r) * P.v_stride + hd * V + ch * 8);
+      if (b0 + r < len) y = dm_act(vr[i]);
       *reinterpret_cast<dm_u4*>(vs + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3)) =
           y;
     }
     __syncthreads();
+    if (b0 + ST < len) fetch(b0 + ST);            // beside the products
 #pragma unroll
     for (int st = 0; st < ST / 16; ++st) {
       bf16x8 b[VT];
@@ -226,43 +248,79 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
   if (tid <= DM_C) pw[tid] = dm_pow(P.decay[hd], tid);
   const int qi = w * 32 + n;
   const bool on = w * 32 < len;
-  bf16x8 qf[KS];
+  // half of the state before the chunk, on its way while what comes before it
+  // is made
+  const int slot = P.slots[s];
+  const bool carried = slot >= 0 && P.ctx_lens[s] > 0;
+  const bool before = c > 0 || carried;           // uniform
+  const float* S =
+      (P.ws != nullptr
+           ? P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V)
+           : P.state + ((long)max(slot, 0) * P.heads + hd) * (D * V));
+  constexpr int SN = 64 * (V / 8) / 256;
+  float sr[SN][8];
+  auto fetch_state = [&](int d0) {
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (qi < len)
-      qf[ks] = __builtin_bit_cast(
-          bf16x8, dm_act(P.q + (long)(t0 + qi) * P.q_stride + hd * D + ks * 16 +
-                         h * 8));
+    for (int i = 0; i < SN; ++i) {
+      const float* p = S + d0 * V + (tid + i * 256) * 8;
+      Quad<float>::ld(p, sr[i]);
+      Quad<float>::ld(p + 4, sr[i] + 4);
+    }
+  };
+  bf16x8 qf[KS];
+  {
+    ushort8_t qr[KS];
+    const unsigned short* p = P.q + (long)(t0 + min(qi, len - 1)) * P.q_stride +
+                              hd * D + h * 8;
+    if (len > 0) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) qr[ks] = dm_row(p + ks * 16);
+    }
+    if (before) fetch_state(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      qf[ks] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (qi < len) qf[ks] = __builtin_bit_cast(bf16x8, dm_act(qr[ks]));
+    }
   }
   // Apart as above, and the leading products of four steps (of two within the
   // chunk) are summed before they meet the large sum, which then is rounded 6
   // times instead of 16. Error against 64 bits, 3 prompts of 853-1657 tokens:
-  // 8.2e-8 -> 6.7e-8 (the recurrence: 7.1e-8), for 3 us of 71.
+  // 8.2e-8 -> 6.7e-8 (the recurrence: 7.1e-8), for 3 us.
   f32x16 acc[2][VT];
 #pragma unroll
   for (int j = 0; j < VT; ++j) acc[0][j] = acc[1][j] = mr_zero();
   const int vbase = mr_col_base<V>(lane);
 
+  // K, then V: batches of four pieces a lane, one on its way while another one is
+  // activated
+  constexpr int NB = DM_C * (D / 8 + V / 8) / 1024;
+  ushort8_t raw[2][4];
+  auto fetch = [&](int b) {
+    const bool key = b < DM_C * (D / 8) / 1024;
+    const int W = key ? D : V;
+    const unsigned short* p = key ? P.k : P.v;
+    const long stride = key ? P.k_stride : P.v_stride;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int idx = tid + (b * 4 + i) * 256 - (key ? 0 : DM_C * (D / 8));
+      const int r = min(idx / (W / 8), len - 1);  // rows past the end: the last
+      raw[b & 1][i] =
+          dm_row(p + (long)(t0 + r) * stride + hd * W + idx % (W / 8) * 8);
+    }
+  };
+
   // ---- through the state before the chunk ------------------------------------
-  const int slot = P.slots[s];
-  const bool carried = slot >= 0 && P.ctx_lens[s] > 0;
-  if (c > 0 || carried) {                         // uniform
-    const float* S =
-        (P.ws != nullptr
-             ? P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V)
-             : P.state + ((long)slot * P.heads + hd) * (D * V));
+  if (before) {
 #pragma unroll
     for (int d0 = 0; d0 < D; d0 += 64) {
       if (d0) __syncthreads();
 #pragma unroll
-      for (int i = 0; i < 64 * (V / 8) / 256; ++i) {
+      for (int i = 0; i < SN; ++i) {
         const int idx = tid + i * 256, r = idx / (V / 8), ch = idx % (V / 8);
-        float x[8];
-        Quad<float>::ld(S + (d0 + r) * V + ch * 8, x);
-        Quad<float>::ld(S + (d0 + r) * V + ch * 8 + 4, x + 4);
-        dm_split(x, lds + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3), 64 * V);
+        dm_split(sr[i], lds + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3), 64 * V);
       }
+      if (d0 + 64 < D) fetch_state(d0 + 64);
       __syncthreads();
       if (!on) continue;
 #pragma unroll
@@ -281,6 +339,7 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
         acc[0][j] += z;
       }
     }
+    if (len > 0) fetch(0);
     __syncthreads();                              // also: pw is there
     const float fade = pw[min(qi, DM_C - 1) + 1];
 #pragma unroll
@@ -290,28 +349,36 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
         acc[0][j][r] *= fade;
         acc[1][j][r] *= fade;
       }
+  } else if (len > 0) {
+    fetch(0);
   }
+  if (len <= 0) return;                           // uniform
 
   // ---- within the chunk --------------------------------------------------------
   unsigned short* ks_ = lds;
   unsigned short* vs = lds + DM_C * D;
-#pragma unroll 4
-  for (int i = 0; i < DM_C * (D / 8) / 256; ++i) {
-    const int idx = tid + i * 256, r = idx / (D / 8), ch = idx % (D / 8);
-    dm_u4 y = {{0u, 0u, 0u, 0u}};
-    if (r < len) y = dm_act(P.k + (long)(t0 + r) * P.k_stride + hd * D + ch * 8);
-    *reinterpret_cast<dm_u4*>(ks_ + r * D + ((ch ^ mr_swz_rows<D>(r)) << 3)) =
-        y;
-  }
   unsigned odd = 0u;
-#pragma unroll 4
-  for (int i = 0; i < DM_C * (V / 8) / 256; ++i) {
-    const int idx = tid + i * 256, r = idx / (V / 8), ch = idx % (V / 8);
-    dm_u4 y = {{0u, 0u, 0u, 0u}};
-    if (r < len) y = dm_act(P.v + (long)(t0 + r) * P.v_stride + hd * V + ch * 8);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) odd |= dm_odd(y.x[j]);
-    *reinterpret_cast<dm_u4*>(vs + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3)) = y;
+  for (int b = 0; b < NB; ++b) {
+    if (b + 1 < NB) fetch(b + 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool key = b < DM_C * (D / 8) / 1024;
+      const int W = key ? D : V;
+      const int idx = tid + (b * 4 + i) * 256 - (key ? 0 : DM_C * (D / 8));
+      const int r = idx / (W / 8), ch = idx % (W / 8);
+      dm_u4 y = {{0u, 0u, 0u, 0u}};
+      if (r < len) y = dm_act(raw[b & 1][i]);
+      if (key) {
+        *reinterpret_cast<dm_u4*>(ks_ + r * D +
+                                  ((ch ^ mr_swz_rows<D>(r)) << 3)) = y;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) odd |= dm_odd(y.x[j]);
+        *reinterpret_cast<dm_u4*>(vs + r * V +
+                                  ((ch ^ mr_swz_cols<V>(r)) << 3)) = y;
+      }
+    }
   }
   // A weight of zero keeps a key out of a row unless its value is not finite: the
   // products see zero instead, and rows from that token on are NaN at the end.

@@ -10,8 +10,9 @@
 // one barrier per tile, so that a tile is on the way while the other is
 // computed. Before, tiles went through registers between two barriers.
 //
-//   S^T[key][head] = K Q^T       16x16x32 products, every wave makes all of it
-//                                (A = K rows from LDS, B = Q in registers)
+//   S^T[key][head] = K Q^T       16x16x32 products, a wave multiplies a quarter of
+//                                the columns (A = K rows from LDS, B = Q in
+//                                registers); shares are added through LDS
 //   online softmax               a lane holds 8 keys of ONE head
 //   O^T[col][head] += V^T P^T    wave w owns columns 128 w .. 128 w + 127;
 //                                A = V^T by transpose reads of the same image,
@@ -25,8 +26,12 @@
 // between the halves of the banks and need three; either way the 16 rows (or 8
 // pieces of 32 B) that share an LDS cycle fall on different banks.
 //
-// Measured, 32 sequences of 1.5-2.4 k keys, 16 heads, rows of 576: 67 + 5 us before,
-// 24 us with the merge now; the rows alone take 15 us at the rate of a large copy.
+// Measured, 32 sequences of 1.5-2.5 k keys, 16 heads, rows of 576: 67 + 5 us before,
+// 24.2 us with the merge now (25.6 when every wave made all scores, and read all of a
+// tile for them); the rows alone take 15 us at the rate of a large copy. Bound by a tile's
+// chain of LDS reads, products and weights, 1.7 us for 36 KB: more tiles on their way
+// (four buffers) did not help, nor did two teams of waves with tiles of their own in a
+// workgroup, which beside 144 KB of LDS gained nothing over more parts.
 //
 // The LDS reads are asm with their wait: in front of a builtin the compiler
 // waits for every load to LDS in flight.
@@ -47,34 +52,53 @@ template <int W> XLLM_DEV int ls_swz(int k) {
   return W == 512 ? ((k & 3) << 2) | lo : (((k >> 1) & 1) << 2) | lo;
 }
 
-// Eight K fragments: four steps of both halves. W == 512: one address per step;
-// W == 576: two, and two offsets.
-template <int W, int OFF>
-XLLM_DEV void ls_keys(const unsigned (&at)[4], bf16x8 (&k)[2][4]) {
-  constexpr int H = 8 * W;                       // bytes of four rows
-  constexpr int O1 = W == 512 ? OFF : OFF + 128;
+// K fragments of four steps, both halves
+template <int W>
+XLLM_DEV void ls_keys(const unsigned* at, bf16x8 (&k)[2][4]) {
   asm volatile(
-      "ds_read_b128 %0, %8 offset:%12\n\tds_read_b128 %1, %9 offset:%12\n\t"
-      "ds_read_b128 %2, %10 offset:%13\n\tds_read_b128 %3, %11 offset:%13\n\t"
-      "ds_read_b128 %4, %8 offset:%14\n\tds_read_b128 %5, %9 offset:%14\n\t"
-      "ds_read_b128 %6, %10 offset:%15\n\tds_read_b128 %7, %11 offset:%15\n\t"
+      "ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\t"
+      "ds_read_b128 %2, %10\n\tds_read_b128 %3, %11\n\t"
+      "ds_read_b128 %4, %8 offset:%12\n\tds_read_b128 %5, %9 offset:%12\n\t"
+      "ds_read_b128 %6, %10 offset:%12\n\tds_read_b128 %7, %11 offset:%12\n\t"
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[0][2]), "=&v"(k[0][3]),
         "=&v"(k[1][0]), "=&v"(k[1][1]), "=&v"(k[1][2]), "=&v"(k[1][3])
-      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(OFF), "n"(O1),
-        "n"(OFF + H), "n"(O1 + H)
+      : "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]), "n"(8 * W)
       : "memory");
 }
-// the last two steps of 576
-template <int OFF>
-XLLM_DEV void ls_keys_end(const unsigned (&at)[4], bf16x8 (&k)[2][2]) {
+// of one step
+template <int W>
+XLLM_DEV void ls_key(unsigned at, bf16x8 (&k)[2]) {
   asm volatile(
-      "ds_read_b128 %0, %4 offset:%6\n\tds_read_b128 %1, %5 offset:%6\n\t"
-      "ds_read_b128 %2, %4 offset:%7\n\tds_read_b128 %3, %5 offset:%7\n\t"
+      "ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:%3\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[1][0]), "=&v"(k[1][1])
-      : "v"(at[0]), "v"(at[1]), "n"(OFF), "n"(OFF + 8 * 576)
+      : "=&v"(k[0]), "=&v"(k[1])
+      : "v"(at), "n"(8 * W)
       : "memory");
+}
+// The waves' shares of the scores, [wave][half][lane]: `mine` goes out, their sum
+// comes back, added in the same order by all
+XLLM_DEV void ls_share(unsigned to, unsigned from, f32x4 (&sc)[2]) {
+  // the compiler does not see what an asm block reads of a product under way: it
+  // ends within 16 states
+  asm volatile(
+      "s_nop 15\n\ts_nop 7\n\tds_write_b128 %0, %1\n\tds_write_b128 %0, %2 offset:1024\n\t"
+      "s_waitcnt lgkmcnt(0)" ::"v"(to), "v"(sc[0]), "v"(sc[1])
+      : "memory");
+  __builtin_amdgcn_s_barrier();
+  f32x4 x[8];
+  asm volatile(
+      "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:1024\n\t"
+      "ds_read_b128 %2, %8 offset:2048\n\tds_read_b128 %3, %8 offset:3072\n\t"
+      "ds_read_b128 %4, %8 offset:4096\n\tds_read_b128 %5, %8 offset:5120\n\t"
+      "ds_read_b128 %6, %8 offset:6144\n\tds_read_b128 %7, %8 offset:7168\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]),
+        "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
+      : "v"(from)
+      : "memory");
+#pragma unroll
+  for (int i = 0; i < 2; i++) sc[i] = (x[i] + x[2 + i]) + (x[4 + i] + x[6 + i]);
 }
 // Four V^T fragments (16 columns, 32 keys each)
 template <int W>
@@ -117,7 +141,8 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   constexpr int NI = 2 * IPP / 4;                // ... of a wave per tile
   constexpr int KS = W / 32;                     // steps of a score product
   constexpr int TILE = LS_KT * W;
-  __shared__ __attribute__((aligned(1024))) unsigned short lds[2 * TILE];
+  __shared__ __attribute__((aligned(1024))) unsigned short
+      lds[2 * TILE + 4 * 2 * 64 * 8];            // and the shares of the scores
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -139,11 +164,15 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   const long row = (long)s * heads + (on ? h0 + n : h0);
   const short flip = scale < 0.0f ? (short)0x8000 : (short)0;
   const float c = paged_factor(scale);
-  bf16x8 qf[KS];
+  // this wave's steps of the score product
+  const int k0 = W == 512 ? 4 * w : 4 * w + min(w, 2);
+  const bool five = W == 576 && w < 2;
+  bf16x8 qf[5];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++)
-    qf[ks] = *reinterpret_cast<const bf16x8*>(q + row * W + ks * 32 + g * 8) ^
-             flip;
+  for (int i = 0; i < 5; i++)
+    qf[i] = *reinterpret_cast<const bf16x8*>(
+                q + row * W + min(k0 + i, KS - 1) * 32 + g * 8) ^
+            flip;
 
   // ---- loads: instruction i of wave w is the (4 i + w)-th of the tile --------
   const int last_blk = (seq_len - 1) / 16, last_row = (seq_len - 1) % 16;
@@ -195,12 +224,12 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   // ---- LDS addresses (bytes, first buffer) -------------------------------------
   const unsigned base = (unsigned)(unsigned long long)(const lds_u16*)lds;
   const int km = (n >> 2) * 8 + (n & 3);         // key of A row n, half 0
-  unsigned kat[4];
+  unsigned kat[5];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int ch = W == 512 ? i * 4 + g : (i & 1) * 4 + g;
-    kat[i] = base + 2 * (km * W + ((ch ^ ls_swz<W>(km)) << 3));
-  }
+  for (int i = 0; i < 5; i++)
+    kat[i] = base + 2 * (km * W + (((min(k0 + i, KS - 1) * 4 + g) ^
+                                    ls_swz<W>(km)) << 3));
+  const unsigned from = base + 2 * (2 * TILE) + lane * 16, to = from + w * 2048;
   const int vk = g * 8 + (n >> 2);               // key of a value piece
   unsigned vat[8];
 #pragma unroll
@@ -231,34 +260,27 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
       stage(t + 1, pages, buf ^ 1);
     }
     const unsigned shift = buf * (2 * TILE);
-    unsigned ka[4];
+    unsigned ka[5];
 #pragma unroll
-    for (int i = 0; i < 4; i++) ka[i] = kat[i] + shift;
+    for (int i = 0; i < 5; i++) ka[i] = kat[i] + shift;
     // ---- scores ----------------------------------------------------------------
     f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    auto four = [&](const bf16x8 (&k)[2][4], int ks) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        sc[0] = ls_mma(k[0][i], qf[ks + i], sc[0]);
-        sc[1] = ls_mma(k[1][i], qf[ks + i], sc[1]);
-      }
-    };
     {
       bf16x8 k[2][4];
-      ls_keys<W, 0>(ka, k); four(k, 0);
-      ls_keys<W, 256>(ka, k); four(k, 4);
-      ls_keys<W, 512>(ka, k); four(k, 8);
-      ls_keys<W, 768>(ka, k); four(k, 12);
-      if constexpr (W == 576) {
-        bf16x8 e[2][2];
-        ls_keys_end<1024>(ka, e);
+      ls_keys<W>(ka, k);
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-          sc[0] = ls_mma(e[0][i], qf[16 + i], sc[0]);
-          sc[1] = ls_mma(e[1][i], qf[16 + i], sc[1]);
-        }
+      for (int i = 0; i < 4; i++) {
+        sc[0] = ls_mma(k[0][i], qf[i], sc[0]);
+        sc[1] = ls_mma(k[1][i], qf[i], sc[1]);
+      }
+      if (five) {
+        bf16x8 e[2];
+        ls_key<W>(ka[4], e);
+        sc[0] = ls_mma(e[0], qf[4], sc[0]);
+        sc[1] = ls_mma(e[1], qf[4], sc[1]);
       }
     }
+    ls_share(to, from, sc);
     // sc[h2][r]: key t*32 + g*8 + h2*4 + r, head n
     if (t == n_tiles - 1 || t * LS_KT < lo) {    // uniform
 #pragma unroll
@@ -363,19 +385,30 @@ bool latent_stream_takes(int W, int r, int heads, int block_size) {
 
 // Room for parts from what the host knows, one part for every `per` tiles of a
 // sequence's own in the kernel. Few workgroups: one per CU, parts of at least two
-// tiles. Measured (us, by parts): 32 x 2000 keys, 16 heads 92 (1), 32 (4), 24
-// (8), 27 (16); 8 x 4000 173 (1), 32 (8), 23 (16), 21 (32); 64 x 1000 51 (1), 24
-// (4), 26 (8); 1 x 700 36 (1), 13 (12). More: parts of 16 tiles, so that a long
-// sequence among short ones is no chain that outlasts the rest; 128 x 600 35
-// (1), 28 (2), 30 (4).
-static int ls_per(long wgs) { return wgs < 86 ? 2 : 16; }
-int latent_stream_parts(int n_seqs, int heads, long table_width, int window) {
-  const long wgs = std::max<long>(1, (long)n_seqs * ((heads + 15) / 16));
+// tiles. Measured (us, by parts): 32 x 2000 keys, 16 heads 37 (4), 25 (8), 24 (16); 8 x
+// 4000 35 (8), 23 (16), 20 (32); 1 x 700 16 (4), 12 (8). More, up to where a part is a
+// long chain: one turn of two per CU, 43 x 1500 28 (5), 25 (10), 43 x 0.1-6 k 62 (5), 42
+// (10), 64 x 1000 25 (4), 24 (8), 64 x 0.1-6 k 78 (4), 55 (8). Still more in short
+// tables the same: 90 x 600 33 (parts of 16 tiles), 23 (of 4), 128 x 0.1-0.9 k 35, 27. In
+// long ones parts of 16 tiles, so that a long sequence among short ones is no chain that
+// outlasts the rest: 90 x 0.1-6 k 74 (6), 84 (5, of 4 tiles), 300 x 0.1-4 k 188 (2), 210
+// (1).
+struct LsParts { long room, per; };
+static LsParts ls_parts(long wgs, long table_width, int window) {
   long tiles = (table_width + 1) / 2;
   if (window > 0) tiles = std::min<long>(tiles, window / LS_KT + 2);
-  const long per = ls_per(wgs);
-  const long p = wgs < 86 ? 256 / wgs : (512 + wgs - 1) / wgs;
-  return (int)std::min<long>({p, (tiles + per - 1) / per, 32});
+  LsParts x;
+  if (wgs < 43) x = {256 / wgs, 2};
+  else if (wgs < 86 || (wgs <= 256 && tiles <= 32)) x = {512 / wgs, 4};
+  else x = {(512 + wgs - 1) / wgs, 16};
+  x.room = std::min<long>({x.room, (tiles + x.per - 1) / x.per, 32});
+  return x;
+}
+static long ls_wgs(int n_seqs, int heads) {
+  return std::max<long>(1, (long)n_seqs * ((heads + 15) / 16));
+}
+int latent_stream_parts(int n_seqs, int heads, long table_width, int window) {
+  return (int)ls_parts(ls_wgs(n_seqs, heads), table_width, window).room;
 }
 
 // q, cache and out 16 B aligned
@@ -386,7 +419,8 @@ void launch_latent_stream(float* out, float* ws_o, float* ws_ml,
                           float scale, int n_part, int window, hipStream_t st) {
   if (n_seqs == 0) return;
   const dim3 grid(n_seqs * n_part, (heads + 15) / 16);
-  const int per = ls_per((long)n_seqs * grid.y);
+  const int per =
+      (int)ls_parts(ls_wgs(n_seqs, heads), table_width, window).per;
   auto k = W == 512 ? latent_stream_kernel<512> : latent_stream_kernel<576>;
   hipLaunchKernelGGL(k, grid, dim3(256), 0, st, out, ws_o, ws_ml, q, cache,
                      block_tables, seq_lens, heads, table_width, scale, n_part,

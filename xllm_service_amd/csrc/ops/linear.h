@@ -6,7 +6,7 @@ namespace xllm {
 // What a product does with its rows on the way in and out, by bits of MODE.
 // LN_SCALE: x holds the rows of an RMS norm without their factors, which come from the
 // sums of their squares' parts: results times 1 / sqrt(sum / K + eps).
-// LN_ADD: results, rounded, join the residual; y gets the new residual times the norm's
+// LN_ADD: results join the residual before either is rounded; y gets the new residual times the norm's
 // weights (the rows of the next product but for their factors), sums the squares of
 // this tile's columns. So a norm needs no launch of its own between two products: 4.6 us
 // of a decode step, 3.4 of a prompt's, for 1.5 more in the two products. 8 layers, 24

@@ -15,7 +15,7 @@ from xllm_service_amd.ops import ref
 pytestmark = pytest.mark.gpu
 
 
-def _step(layers, cfg, prompts, decodes, first):
+def _step(layers, cfg, prompts, decodes, first, no_slot=()):
     """One pass over chunks of `prompts` tokens behind 20 cached ones and rows of
     `decodes` cached ones; fresh inputs and caches every time."""
     g = torch.Generator(device="cuda").manual_seed(3)
@@ -34,6 +34,7 @@ def _step(layers, cfg, prompts, decodes, first):
     seq = [i for i, n in enumerate(prompts) for _ in range(n)] \
         + list(range(len(prompts), len(prompts) + len(decodes)))
     slots = [int(tables[s, p // 16]) * 16 + p % 16 for s, p in zip(seq, pos)]
+    slots = [-1 if i in no_slot else s for i, s in enumerate(slots)]
     cu = [0]
     for n in prompts:
         cu.append(cu[-1] + n)
@@ -95,3 +96,32 @@ def test_native_layers(name, prompts, decodes, first, n_layers, monkeypatch):
     with torch.no_grad():                     # gradients could be asked for
         _step(layers, cfg, prompts, decodes, first)
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("name", ["llama-2k", "llama-4k"])
+@pytest.mark.parametrize("prompts,decodes", [
+    ([], [1]), ([5], [17, 90, 3]), ([8, 9], [31] * 7), ([20, 9], [8]), ([41], []),
+    ([33, 31], []), ([70, 60], []), ([100, 105, 107], [4])])
+def test_rotated_products(name, prompts, decodes):
+    """Keys and values that the first product of a second layer leaves in its caches:
+    as above within 2^-6, elsewhere, and where a row has no slot, what was there."""
+    cfg = get_config(name)
+    with torch.device("cuda"):
+        layers = [LlamaDecoderLayer(cfg, torch.bfloat16) for _ in range(2)]
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for n, p in torch.nn.ModuleList(layers).named_parameters():
+        p.data.normal_(1.0 if "norm" in n else 0.0, 0.02, generator=g)
+    T = sum(prompts) + len(decodes)
+    no_slot = (T - 1,) if T > 1 else ()
+    with torch.inference_mode():
+        got, caches = _step(layers, cfg, prompts, decodes, True, no_slot)
+        none, before = _step(layers, cfg, prompts, decodes, True, range(T))
+        layers[0].mlp.down.register_forward_hook(lambda *a: None)
+        want, plain = _step(layers, cfg, prompts, decodes, True, no_slot)
+    for a, b, was in zip(caches[1], plain[1], before[1]):
+        new = (b != was).any(-1)                     # rows of heads
+        assert int(new.sum()) == (T - len(no_slot)) * cfg.num_kv_heads
+        assert torch.equal(a[~new], was[~new])
+        assert _off(a[new], b[new]) < 2.0 ** -6
+        off = (a[new].double() - b[new].double()).norm(dim=-1)
+        assert (off < 2.0 ** -5 * b[new].double().norm(dim=-1)).all()

@@ -543,10 +543,35 @@ struct DecoderLayer {
   torch::Tensor down_w, k_cache, v_cache;
 };
 
+// Whether the first product of a layer rotates its heads and fills the caches itself:
+// rows of a product before it, one position to a row, heads of 128 without a bias
+static bool rotates(const Rows& in, const DecoderLayer& p, long heads,
+                    const torch::Tensor& positions, const torch::Tensor& slots,
+                    const torch::Tensor& cos_sin) {
+  const long T = in.x.size(0);
+  auto cache = [&](const torch::Tensor& t) {
+    return t.is_cuda() && t.dim() == 4 && t.dtype() == torch::kBFloat16 &&
+           t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  auto rows = [&](const torch::Tensor& t) {
+    return t.is_cuda() && t.dtype() == torch::kLong && t.dim() == 1 &&
+           t.is_contiguous() && t.size(0) == T;
+  };
+  return in.squares.defined() && !p.qkv_b.has_value() && cache(p.k_cache) &&
+         cache(p.v_cache) && p.k_cache.sizes() == p.v_cache.sizes() &&
+         p.k_cache.size(3) == xllm::LN_HEAD &&
+         p.qkv_w.size(0) == (heads + 2 * p.k_cache.size(1)) * xllm::LN_HEAD &&
+         rows(positions) && rows(slots) && cos_sin.is_cuda() &&
+         cos_sin.dtype() == torch::kFloat && cos_sin.is_contiguous() &&
+         cos_sin.dim() == 2 && cos_sin.size(1) == xllm::LN_HEAD &&
+         reinterpret_cast<uintptr_t>(cos_sin.data_ptr()) % 16 == 0;
+}
+
 // Layers of the dense decoders (models/llama.py) over prompt rows and decode rows:
 // what their modules call, in their order, without the interpreter between two
 // launches (75 us of host time a layer, 25 here, where the kernels of 300 rows of 2048
-// take 70), and without launches for the norms between two products. Nothing, with
+// take 70), and without launches for the norms between two products and for the rotation
+// and the cache rows of what comes out of one (LN_ROPE). Nothing, with
 // nothing done, where torch has to see the calls.
 c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layers(
     torch::Tensor x, c10::optional<torch::Tensor> residual,
@@ -584,18 +609,36 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layers(
   }
   for (size_t i = 0; i < layers.size(); i++) {
     const auto& p = layers[i];
-    const auto qkv = product(in, p.qkv_w, p.qkv_b, false, eps);
-    const long T = qkv.size(0), D = p.k_cache.size(3), n_kv = p.k_cache.size(1);
-    const long row = qkv.stride(0), at = qkv.storage_offset();
-    TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (heads + 2 * n_kv) * D &&
-                qkv.stride(1) == 1, "decoder layer: shapes do not match");
-    const auto q = qkv.as_strided({T, heads, D}, {row, D, 1}, at);
-    const auto k = qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + heads * D);
-    const auto v =
-        qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + (heads + n_kv) * D);
-    fused_rope_cache(positions, q, k, v, p.k_cache, p.v_cache, slot_mapping,
-                     cos_sin, D, ms0, ms1);
-    auto out = torch::empty({T, heads * D}, qkv.options());
+    const long T = in.x.size(0), D = p.k_cache.size(3), n_kv = p.k_cache.size(1);
+    torch::Tensor q;
+    if (ms0 == 0 && rotates(in, p, heads, positions, slot_mapping, cos_sin)) {
+      q = torch::empty({T, heads, D}, in.x.options());
+      auto e = scale_of(in, eps);
+      e.positions = positions.data_ptr<long>();
+      e.slots = slot_mapping.data_ptr<long>();
+      e.cos_sin = cos_sin.data_ptr<float>();
+      e.k_cache = reinterpret_cast<unsigned short*>(p.k_cache.data_ptr());
+      e.v_cache = reinterpret_cast<unsigned short*>(p.v_cache.data_ptr());
+      e.n_q = (int)heads;
+      e.n_kv = (int)n_kv;
+      e.block = (int)p.k_cache.size(2);
+      xllm::launch_linear(u16(q), u16c(in.x), u16c(p.qkv_w), nullptr, (int)T,
+                          (int)p.qkv_w.size(0), (int)p.qkv_w.size(1),
+                          in.x.stride(0), linear_kind(in.x, p.qkv_w, p.qkv_b),
+                          xllm::LN_SCALE | xllm::LN_ROPE, e, cur_stream());
+    } else {
+      const auto qkv = product(in, p.qkv_w, p.qkv_b, false, eps);
+      const long row = qkv.stride(0), at = qkv.storage_offset();
+      TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (heads + 2 * n_kv) * D &&
+                  qkv.stride(1) == 1, "decoder layer: shapes do not match");
+      q = qkv.as_strided({T, heads, D}, {row, D, 1}, at);
+      const auto k = qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + heads * D);
+      const auto v =
+          qkv.as_strided({T, n_kv, D}, {row, D, 1}, at + (heads + n_kv) * D);
+      fused_rope_cache(positions, q, k, v, p.k_cache, p.v_cache, slot_mapping,
+                       cos_sin, D, ms0, ms1);
+    }
+    auto out = torch::empty({T, heads * D}, q.options());
     const auto out3 = out.view({T, heads, D});
     if (n_prefill > 0)
       paged_attn_prefill(out3.slice(0, 0, n_prefill), q.slice(0, 0, n_prefill),

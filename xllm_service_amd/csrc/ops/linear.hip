@@ -48,6 +48,55 @@ XLLM_DEV long ln_gate_row(long first, long half, int r) {
   return r < ROWS / 2 ? min(first + r, half - 1)
                       : half + min(first + r - ROWS / 2, half - 1);
 }
+// Rotated products: a tile of ROWS rows has ROWS / 2 of the first half of a head and
+// their partners of the other one. Its first row, and row r of it from there
+template <int ROWS> XLLM_DEV int ln_rope_first(int tile) {
+  constexpr int TILES = LN_HEAD / ROWS;          // of a head
+  return tile / TILES * LN_HEAD + tile % TILES * (ROWS / 2);
+}
+template <int ROWS> XLLM_DEV int ln_rope_row(int r) {
+  return r < ROWS / 2 ? r : LN_HEAD / 2 + r - ROWS / 2;
+}
+// what becomes of row m of the columns from `first` on: the columns' place, null for
+// none, in a query, a key or a value
+struct LnRope {
+  long pos, slot;
+  XLLM_DEV void init(const LinearEnds& e, long m, bool ok) {
+    pos = ok ? e.positions[m] : 0;
+    slot = ok ? e.slots[m] : -1;
+  }
+  XLLM_DEV unsigned short* place(const LinearEnds& e, unsigned short* y, long m,
+                                 int first) const {
+    const int h = first / LN_HEAD, at = first % LN_HEAD;
+    if (h < e.n_q) return y + (m * e.n_q + h) * LN_HEAD + at;
+    if (slot < 0) return nullptr;
+    const long blk = slot >> 31 == 0 ? (unsigned)slot / (unsigned)e.block
+                                     : slot / e.block;
+    const bool val = h >= e.n_q + e.n_kv;
+    return (val ? e.v_cache : e.k_cache) +
+           ((blk * e.n_kv + h - e.n_q - (val ? e.n_kv : 0)) * e.block +
+            (slot - blk * e.block)) * LN_HEAD + at;
+  }
+  // cos and sin of four columns' pairs
+  XLLM_DEV void angles(const LinearEnds& e, int first, float4& c, float4& s) const {
+    const float* p = e.cos_sin + pos * LN_HEAD + first % LN_HEAD;
+    c = make_float4(1.f, 1.f, 1.f, 1.f);
+    s = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (first / LN_HEAD >= e.n_q + e.n_kv) return;   // values stay
+    c = *reinterpret_cast<const float4*>(p);
+    s = *reinterpret_cast<const float4*>(p + LN_HEAD / 2);
+  }
+};
+// four pairs
+XLLM_DEV void ln_turn(float* a, float* b, const float4& c, const float4& s) {
+  const float cc[4] = {c.x, c.y, c.z, c.w}, ss[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const float x = a[e], y = b[e];
+    a[e] = x * cc[e] - y * ss[e];
+    b[e] = y * cc[e] + x * ss[e];
+  }
+}
 // silu(gate) up of two sums
 XLLM_DEV float ln_gated(float gate, float up) {
   return gate / (1.0f + __expf(-gate)) * up;
@@ -89,6 +138,14 @@ struct LnTile {
                           (((lane & 15) ^ (r & 15)) << 4));
     }
   }
+  XLLM_DEV void init_rope(long stride, int lane) {
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+      const int r = i * 4 + (lane >> 4);
+      off[i] = (unsigned)(ln_rope_row<ROWS>(r) * stride * 2 +
+                          (((lane & 15) ^ (r & 15)) << 4));
+    }
+  }
   XLLM_DEV void load(const unsigned short* p, unsigned short* dst) const {
 #pragma unroll
     for (int i = 0; i < NI; i++)
@@ -120,7 +177,8 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
     const unsigned short* __restrict__ bias, const int M, const int N,
     const int K, const long x_stride, const LinearEnds ends) {
   constexpr bool GATE = MODE & LN_GATE, SCALE = MODE & LN_SCALE,
-                 ADD = MODE & LN_ADD;
+                 ADD = MODE & LN_ADD, ROPE = MODE & LN_ROPE;
+  constexpr bool PAIR = GATE || ROPE;            // two rows of W to a column
   constexpr int WR = 16 * NT;                    // rows of W
   constexpr int MT = (XR + 15) / 16;             // row tiles of x
   constexpr int T = WR * LN_K, TILE = T + XR * LN_K;
@@ -132,13 +190,14 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
-  constexpr int OUT = GATE ? WR / 2 : WR;        // columns of the result
+  constexpr int OUT = PAIR ? WR / 2 : WR;        // columns of the result
   const int n_out = GATE ? N / 2 : N;
-  const long n0 = blockIdx.x * (long)OUT;
+  const long n0 = ROPE ? (long)ln_rope_first<WR>(blockIdx.x) : blockIdx.x * (long)OUT;
   unsigned short* wt = lds + wid * (D * TILE);
   LnTile<WR> lw;
   LnTile<XR> lx;
-  if (GATE) lw.init_gate(n0, n_out, K, lane);
+  if (ROPE) lw.init_rope(K, lane);
+  else if (GATE) lw.init_gate(n0, n_out, K, lane);
   else lw.init(n0, N, K, lane);
   lx.init(0, M, x_stride, lane);
   const unsigned short* wp = w + n0 * K;
@@ -176,6 +235,16 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
       res[k] = *reinterpret_cast<const uint2*>(ends.residual +
                                                (long)m * n_out + n);
       norm[k] = *reinterpret_cast<const uint2*>(ends.norm + n);
+    }
+  }
+  LnRope rope[ROPE ? OWN : 1];
+  float4 cosv[ROPE ? OWN : 1], sinv[ROPE ? OWN : 1];
+  if constexpr (ROPE) {
+#pragma unroll
+    for (int k = 0; k < OWN; k++) {
+      const int i = tid + k * NW * 64, m = i / C4;
+      rope[k].init(ends, m, m < M);
+      rope[k].angles(ends, (int)n0 + (i % C4) * 4, cosv[k], sinv[k]);
     }
   }
   f32x4 acc[NT][MT];
@@ -286,11 +355,24 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
       sum(m, OUT + col, u);
 #pragma unroll
       for (int e = 0; e < 4; e++) s[e] = ln_gated(s[e] * f, u[e] * f);
+    } else if constexpr (ROPE) {
+      float u[4];
+      sum(m, OUT + col, u);
+#pragma unroll
+      for (int e = 0; e < 4; e++) s[e] *= f, u[e] *= f;
+      ln_turn(s, u, cosv[k], sinv[k]);
+      unsigned short* to = rope[k].place(ends, y, m, (int)n);
+      if (to == nullptr) continue;
+      *reinterpret_cast<uint2*>(to) =
+          make_uint2(pack_bf16(s[0], s[1]), pack_bf16(s[2], s[3]));
+      *reinterpret_cast<uint2*>(to + LN_HEAD / 2) =
+          make_uint2(pack_bf16(u[0], u[1]), pack_bf16(u[2], u[3]));
+      continue;
     } else if constexpr (SCALE) {
 #pragma unroll
       for (int e = 0; e < 4; e++) s[e] *= f;
     }
-    if (MODE % 4 != LN_GATE && !ADD && bias != nullptr) {
+    if (!ROPE && MODE % 4 != LN_GATE && !ADD && bias != nullptr) {
 #pragma unroll
       for (int e = 0; e < 4; e++) s[e] += bf16_to_f32(bias[n + e]);
     }
@@ -339,7 +421,8 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     const int K, const long x_stride, const int n_tiles_n,
     const LinearEnds ends) {
   constexpr bool GATE = MODE & LN_GATE, SCALE = MODE & LN_SCALE,
-                 ADD = MODE & LN_ADD;
+                 ADD = MODE & LN_ADD, ROPE = MODE & LN_ROPE;
+  constexpr bool PAIR = GATE || ROPE;            // two rows of W to a column
   constexpr int WR = 16 * NW;                    // rows of W
   constexpr int WT = WR * LK, TILE = WT + 16 * MT * LK;
   constexpr int KS = LK / 64;                    // products a wave makes of a step
@@ -350,15 +433,17 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, c16 = lane & 15;
-  constexpr int OUT = GATE ? WR / 2 : WR;        // columns of the result
+  constexpr int OUT = PAIR ? WR / 2 : WR;        // columns of the result
   const int n_out = GATE ? N / 2 : N;
-  const long n0 = (blockIdx.x % n_tiles_n) * (long)OUT;
+  const int tile_n = blockIdx.x % n_tiles_n;
+  const long n0 = ROPE ? (long)ln_rope_first<WR>(tile_n) : tile_n * (long)OUT;
   const long m0 = (blockIdx.x / n_tiles_n) * (16L * MT);
   const int n_cols = (int)min((long)OUT, n_out - n0);
   const int m_rows = (int)min(16L * MT, M - m0);
   const unsigned short* wp = w + n0 * K;
   const unsigned short* xp = x + m0 * x_stride;
-  const unsigned w_bytes = (unsigned)(n_cols + (GATE ? n_out : 0)) * K * 2;
+  const unsigned w_bytes =
+      (unsigned)(n_cols + (GATE ? n_out : ROPE ? LN_HEAD / 2 : 0)) * K * 2;
   const unsigned x_bytes = (unsigned)((m_rows - 1) * x_stride + K) * 2;
   // a wave loads 16 rows of W and its share of x, RPI at a time; rows past the last
   // one repeat it: their results go nowhere
@@ -370,8 +455,9 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
 #pragma unroll
   for (int i = 0; i < WI; i++) {
     const int r = (wid * WI + i) * RPI + lane / CPR;
-    w_off[i] = offset(r, GATE ? ln_gate_row<WR>(n0, n_out, r) - n0
-                              : min(r, n_cols - 1), K);
+    w_off[i] = offset(r, ROPE   ? ln_rope_row<WR>(r)
+                         : GATE ? ln_gate_row<WR>(n0, n_out, r) - n0
+                                : min(r, n_cols - 1), K);
   }
 #pragma unroll
   for (int i = 0; i < XI; i++) {
@@ -390,6 +476,16 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
       const int p = (i * SL + tid % SL) * 4;
       sq[i] = mr_load(src, p < ends.n_squares
                                ? (tid / SL * ends.n_squares + p) * 4 : ~15u);
+    }
+  }
+  constexpr int C8 = OUT / 8;                    // columns in eights
+  constexpr int OWN = (16 * MT * C8 + NW * 64 - 1) / (NW * 64);
+  LnRope rope[ROPE ? OWN : 1];
+  if constexpr (ROPE) {
+#pragma unroll
+    for (int k = 0; k < OWN; k++) {
+      const int row = (tid + k * NW * 64) / C8;
+      rope[k].init(ends, m0 + row, row < m_rows);
     }
   }
   const int steps = K / LK;
@@ -467,6 +563,15 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     step(t, f[1], f[0]);
     if (++t == steps) break;
   }
+  float4 cosv[ROPE ? OWN : 1][2], sinv[ROPE ? OWN : 1][2];
+  if constexpr (ROPE) {
+#pragma unroll
+    for (int k = 0; k < OWN; k++)
+#pragma unroll
+      for (int e = 0; e < 2; e++)
+        rope[k].angles(ends, (int)n0 + (tid + k * NW * 64) % C8 * 8 + 4 * e,
+                       cosv[k][e], sinv[k][e]);
+  }
   // acc[i][j][r] = a half of y[m = 16 j + c16][n = 32 hw + 16 i + 4 g + r]. The
   // waves of the two halves swap a row tile of W, then whole rows go out.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -476,7 +581,7 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   for (int j = 0; j < MT; j++) swap[(wid * MT + j) * 64 + lane] = hk ? acc[0][j] : acc[1][j];
   __syncthreads();
   // rows on their way out: bf16, or what something is still done to, padded
-  constexpr bool WIDE = GATE || ADD;
+  constexpr bool WIDE = PAIR || ADD;
   constexpr int ROW = WIDE ? 2 * (WR + 4) : WR + 8;
   unsigned short* out = lds + NW * MT * 64 * 8;
   const int col0 = 32 * hw + 16 * hk + 4 * g;
@@ -508,9 +613,8 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     }
   }
   __syncthreads();
-  constexpr int C8 = OUT / 8;                    // columns in eights
 #pragma unroll
-  for (int k = 0; k < (16 * MT * C8 + NW * 64 - 1) / (NW * 64); k++) {
+  for (int k = 0; k < OWN; k++) {
     const int idx = tid + k * NW * 64;
     const int row = idx / C8, col = idx % C8 * 8;
     const bool ok = row < m_rows && col < n_cols;
@@ -525,6 +629,21 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
               out + row * ROW + 2 * (at + e));
       };
       if (ok) eight(col, f);
+      if constexpr (ROPE) {
+        float u[8];
+        eight(OUT + col, u);
+        ln_turn(f, u, cosv[k][0], sinv[k][0]);
+        ln_turn(f + 4, u + 4, cosv[k][1], sinv[k][1]);
+        unsigned short* to = rope[k].place(ends, y, m0 + row, (int)n0 + col);
+        if (to == nullptr) continue;
+        *reinterpret_cast<uint4*>(to) =
+            make_uint4(pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]),
+                       pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7]));
+        *reinterpret_cast<uint4*>(to + LN_HEAD / 2) =
+            make_uint4(pack_bf16(u[0], u[1]), pack_bf16(u[2], u[3]),
+                       pack_bf16(u[4], u[5]), pack_bf16(u[6], u[7]));
+        continue;
+      }
       if constexpr (GATE) {
         float u[8];
         eight(OUT + col, u);
@@ -653,9 +772,9 @@ static void launch_stream(unsigned short* y, const unsigned short* x,
                           const unsigned short* w, const unsigned short* bias,
                           int M, int N, int K, long x_stride,
                           const LinearEnds& ends, hipStream_t stream) {
-  constexpr bool GATE = MODE & LN_GATE;
+  constexpr int PAIR = MODE & (LN_GATE | LN_ROPE) ? 2 : 1;
   const bool one = linear_one_tile(M, N, K);
-  const int out = (one ? 16 : 32) / (GATE ? 2 : 1), n_out = N / (GATE ? 2 : 1);
+  const int out = (one ? 16 : 32) / PAIR, n_out = N / PAIR;
   const dim3 grid((n_out + out - 1) / out);
   const bool few = grid.x <= 256;
 #define LN_STREAM(NT, XR, NW, D)                                               \
@@ -685,11 +804,11 @@ static void launch_tile(unsigned short* y, const unsigned short* x,
                         const unsigned short* w, int M, int N, int K,
                         long x_stride, const LinearEnds& ends,
                         hipStream_t stream) {
-  constexpr bool GATE = MODE & LN_GATE;
-  const int n_out = N / (GATE ? 2 : 1);
+  constexpr int PAIR = MODE & (LN_GATE | LN_ROPE) ? 2 : 1;
+  const int n_out = N / PAIR;
 #define LN_TILE(NW, MT, LK, S)                                                 \
   do {                                                                         \
-    constexpr int OUT = 16 * NW / (GATE ? 2 : 1);                              \
+    constexpr int OUT = 16 * NW / PAIR;                                         \
     const int tn = (n_out + OUT - 1) / OUT, tm = (M + 16 * MT - 1) / (16 * MT); \
     hipLaunchKernelGGL((linear_tile_kernel<NW, MT, LK, S, MODE>),              \
                        dim3((unsigned)(tn * tm)), dim3(NW * 64), 0, stream, y, \
@@ -715,7 +834,7 @@ int linear_tiles(int M, int N, int K, int kind) {
 }
 
 // mode: LN_GATE: W = [gates | ups], y [M, N / 2] = silu(x gates^T) (x ups^T);
-// LN_SCALE with or without it, or LN_ADD alone: see there
+// LN_SCALE with or without it, LN_ADD alone, LN_SCALE | LN_ROPE: see there
 void launch_linear(unsigned short* y, const unsigned short* x,
                    const unsigned short* w, const unsigned short* bias, int M,
                    int N, int K, long x_stride, int kind, int mode,
@@ -733,6 +852,7 @@ void launch_linear(unsigned short* y, const unsigned short* x,
     LN_MODE(LN_SCALE);
     LN_MODE(LN_SCALE | LN_GATE);
     LN_MODE(LN_ADD);
+    LN_MODE(LN_SCALE | LN_ROPE);
   }
 #undef LN_MODE
 }

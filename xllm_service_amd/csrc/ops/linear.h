@@ -16,7 +16,7 @@ namespace xllm {
 // LN_ROPE, heads of 128: W = [queries | keys | values] by heads; y [M, queries] gets
 // queries rotated by their rows' positions, the caches keys (rotated) and values. A
 // tile has columns of one half of a head and their partners of the other one. A launch
-// less, 4.0 us of 300 rows and 4.7 of 24, for 0.8 and 2.2 more in the product: 548 -> 526 us,
+// less, 4.0 us of 300 rows and 4.7 of 24, for 0.5 to 1.5 more in the product: 548 -> 526 us,
 // 675 -> 657.
 enum { LN_GATE = 1, LN_SCALE = 2, LN_ADD = 4, LN_ROPE = 8 };
 constexpr int LN_HEAD = 128;

@@ -27,7 +27,7 @@
 // pieces of 32 B) that share an LDS cycle fall on different banks.
 //
 // Measured, 32 sequences of 1.5-2.5 k keys, 16 heads, rows of 576: 67 + 5 us before,
-// 24.2 us with the merge now (25.6 when every wave made all scores, and read all of a
+// 23.6 us with the merge now (25.6 when every wave made all scores, and read all of a
 // tile for them); the rows alone take 15 us at the rate of a large copy. Bound by a tile's
 // chain of LDS reads, products and weights, 1.7 us for 36 KB: more tiles on their way
 // (four buffers) did not help, nor did two teams of waves with tiles of their own in a
@@ -385,11 +385,12 @@ bool latent_stream_takes(int W, int r, int heads, int block_size) {
 
 // Room for parts from what the host knows, one part for every `per` tiles of a
 // sequence's own in the kernel. Few workgroups: one per CU, parts of at least two
-// tiles. Measured (us, by parts): 32 x 2000 keys, 16 heads 37 (4), 25 (8), 24 (16); 8 x
-// 4000 35 (8), 23 (16), 20 (32); 1 x 700 16 (4), 12 (8). More, up to where a part is a
-// long chain: one turn of two per CU, 43 x 1500 28 (5), 25 (10), 43 x 0.1-6 k 62 (5), 42
-// (10), 64 x 1000 25 (4), 24 (8), 64 x 0.1-6 k 78 (4), 55 (8). Still more in short
-// tables the same: 90 x 600 33 (parts of 16 tiles), 23 (of 4), 128 x 0.1-0.9 k 35, 27. In
+// tiles. Measured (us, by parts): 1 x 700 keys, 16 heads 16 (4), 12 (8); 8 x 4000 35
+// (8), 23 (16), 20 (32); 16 x 2000 18.5 (16), 20.3 (32). More, up to where a part is a
+// long chain: one turn of two per CU, 24 x 2000 22.8 (10), 22.3 (21), 24 x 0.1-6 k 34.8
+// (10), 29.1 (21), 32 x 700 15.7 (8), 16.0 (16), 32 x 2000 24.8 (8), 23.8 (16), 32 x 0.1-6 k
+// 40.9 (8), 33.0 (16), 43 x 1500 28 (5), 25 (10), 43 x 0.1-6 k 62 (5), 42 (10), 64 x 1000
+// 25 (4), 24 (8), 64 x 0.1-6 k 78 (4), 55 (8). Still more in short tables the same: 90 x 600 33 (parts of 16 tiles), 23 (of 4), 128 x 0.1-0.9 k 35, 27. In
 // long ones parts of 16 tiles, so that a long sequence among short ones is no chain that
 // outlasts the rest: 90 x 0.1-6 k 74 (6), 84 (5, of 4 tiles), 300 x 0.1-4 k 188 (2), 210
 // (1).
@@ -398,7 +399,7 @@ static LsParts ls_parts(long wgs, long table_width, int window) {
   long tiles = (table_width + 1) / 2;
   if (window > 0) tiles = std::min<long>(tiles, window / LS_KT + 2);
   LsParts x;
-  if (wgs < 43) x = {256 / wgs, 2};
+  if (wgs < 24) x = {256 / wgs, 2};
   else if (wgs < 86 || (wgs <= 256 && tiles <= 32)) x = {512 / wgs, 4};
   else x = {(512 + wgs - 1) / wgs, 16};
   x.room = std::min<long>({x.room, (tiles + x.per - 1) / x.per, 32});

@@ -157,6 +157,40 @@ def test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("lens,ctx,kv_heads,per", [
+    ([9], [120], 4, 1),                 # waves that share the keys
+    ([80], [300], 16, 8),               # whole chains
+    ([900], [1300], 16, 8),             # eight waves in turn
+])
+def test_prefill_sums_whole_weights(lens, ctx, kv_heads, per):
+    """One key has the weight 1 and the only value, all others a weight that bf16
+    would round by nearly 2^-8 of itself: what is left of a result's error is the
+    rounding of v / sum, up to 2^-9 and of either sign, so that the mean over many
+    is far below 2^-12; sums of rounded weights are off by 2^-9.2 and more."""
+    dim, weight = 128, 0.5 + 2.0 ** -9 - 2.0 ** -16
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, 3)
+    heads, first = kv_heads * per, table[0, 0].long()
+    q = torch.zeros(lens[0], heads, dim, dtype=torch.bfloat16)
+    q[..., 0] = 1.0
+    k.zero_()
+    k[first, :, 0, 0] = 1.0
+    only = torch.rand(kv_heads, dim, generator=torch.Generator().manual_seed(
+        per)).add_(1.0).to(torch.bfloat16)
+    v.zero_()
+    v[first, :, 0] = only
+    got = ops.paged_attn_prefill(
+        q.cuda(), k.cuda(), v.cuda(), table.cuda(),
+        torch.tensor([0, lens[0]], dtype=torch.int32, device="cuda"),
+        torch.tensor([lens[0] + ctx[0]], dtype=torch.int32, device="cuda"),
+        -math.log(weight)).double().cpu()
+    keys = ctx[0] + 1 + torch.arange(lens[0])
+    ref = only.double().repeat_interleave(per, 0)[None] \
+        / (1.0 + (keys.double() - 1.0) * weight)[:, None, None]
+    off = got / ref - 1.0
+    assert off.abs().max() < 2.0 ** -8
+    assert off.mean().abs() < 2.0 ** -12
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("ctx", [[3, 0], [2600, 900]])      # whole; in parts
 def test_prefill_leaves_other_rows(dim, ctx):

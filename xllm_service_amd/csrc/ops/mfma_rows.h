@@ -48,12 +48,6 @@ XLLM_DEV unsigned pack_bf16(float a, float b) {
   const bfx2 x = __builtin_convertvector(f, bfx2);
   return __builtin_bit_cast(unsigned, x);
 }
-// c + both of a packed pair
-XLLM_DEV float sum_bf16(unsigned u, float c) {
-  const bfx2 one = {(__bf16)1.0f, (__bf16)1.0f};
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bfx2, u), one, c,
-                                         false);
-}
 // a, b <- what the packed pair leaves of them (exact)
 XLLM_DEV void drop_bf16(float& a, float& b, unsigned u) {
   a -= __uint_as_float(u << 16);

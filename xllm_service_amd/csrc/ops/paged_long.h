@@ -216,9 +216,8 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
     for (int r = 8 * (st & 1); r < 8 * (st & 1) + 8; r += 2) {
       const float a = __builtin_amdgcn_exp2f(fmaf(s[i][r], c, -mc));
       const float b = __builtin_amdgcn_exp2f(fmaf(s[i][r + 1], c, -mc));
-      const unsigned u = pack_bf16(a, b);
-      reinterpret_cast<unsigned*>(&p[st])[(r & 7) >> 1] = u;
-      l = sum_bf16(u, l);
+      l += a + b;
+      reinterpret_cast<unsigned*>(&p[st])[(r & 7) >> 1] = pack_bf16(a, b);
     }
   };
   // operands of four products: 16 values' rows, or two steps of the keys'

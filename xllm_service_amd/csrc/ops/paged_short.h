@@ -196,13 +196,12 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
       for (int r = 0; r < 16; r += 2) {
         float a = __builtin_amdgcn_exp2f(fmaf(s[j][r], c, -mc));
         float b = __builtin_amdgcn_exp2f(fmaf(s[j][r + 1], c, -mc));
-        if (TERMS > 1) l += a + b;
+        l += a + b;
 #pragma unroll
         for (int e = 0; e < TERMS; e++) {
           const unsigned u = pack_bf16(a, b);
           reinterpret_cast<unsigned*>(
               &p[e][j * 2 + (r >> 3)])[(r & 7) >> 1] = u;
-          if (TERMS == 1) l = sum_bf16(u, l);
           drop_bf16(a, b, u);
         }
       }

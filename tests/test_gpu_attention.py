@@ -157,6 +157,32 @@ def test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign):
     assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("lens,keys,kv_heads,per", [
+    ([40, 7], [130, 0], 2, 2),                       # waves that share the keys
+    ([300, 50, 9], [60, 0, 300], 16, 8),             # whole chains
+    ([900, 300, 5], [450, 0, 2300], 16, 8),          # eight waves in turn
+])
+def test_prefill_rows_without_keys(dim, lens, keys, kv_heads, per):
+    """More new tokens than keys, or no keys at all: rows in front of the first key
+    are zero, the others see what they see."""
+    ctx = [n - m for n, m in zip(keys, lens)]
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, 31)
+    heads, scale = kv_heads * per, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)))
+    dev = [t.cuda() for t in (k, v, table, cu.int(),
+                              torch.tensor(keys, dtype=torch.int32))]
+    got = ops.paged_attn_prefill(
+        rows.cuda()[:, :heads * dim].unflatten(-1, (heads, dim)), *dev, scale)
+    sees = torch.cat([torch.arange(n) + c >= 0 for n, c in zip(lens, ctx)])
+    on = [i for i, n in enumerate(keys) if n > 0]
+    left = [min(lens[i], keys[i]) for i in on]
+    check(got[sees.cuda()], *want(q[sees], k, v, table[on], left,
+                                  [max(ctx[i], 0) for i in on], scale))
+    assert (got[~sees.cuda()] == 0).all()
+
+
 @pytest.mark.parametrize("lens,ctx,kv_heads,per", [
     ([9], [120], 4, 1),                 # waves that share the keys
     ([80], [300], 16, 8),               # whole chains

@@ -117,7 +117,7 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
 
   const int row0 = lt * PL_ROWS;
   const int kmax = ctx + (min(row0 + PL_ROWS, rows) - 1) / G + 1;
-  const int n = (kmax + PF_KT - 1) / PF_KT;      // tiles
+  const int n = (max(kmax, 0) + PF_KT - 1) / PF_KT;   // tiles; rows without keys: 0
 
   // ---- this lane's row -----------------------------------------------------
   const int wrow0 = row0 + wid * 32;
@@ -166,7 +166,8 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
   int tb = 0;
   unsigned from_lo = 0, from_hi = 0, bytes = 0;
   auto look_up = [&]() {
-    const int t = tb + lane, pg = min(t, n - 1) * (PF_KT / PF_BS) + page4;
+    const int t = tb + lane,
+              pg = max(min(t, n - 1), 0) * (PF_KT / PF_BS) + page4;
     const long id = btab[min(pg, last_blk)];
     const unsigned long long at = (unsigned long long)(
         cache + (id * n_kv + kvh) * (PF_BS * D));
@@ -295,7 +296,8 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
   };
 
   // tiles with keys that this wave's rows see
-  const unsigned mine = wave_on ? (unsigned)((wmax + PF_KT - 1) / PF_KT) : 0;
+  const unsigned mine =
+      wave_on ? (unsigned)(max(wmax, 0) + PF_KT - 1) / PF_KT : 0;
   look_up();
 #pragma unroll
   for (int i = 0; i < PL_BUFS - 1; i++)

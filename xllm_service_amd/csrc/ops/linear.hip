@@ -490,16 +490,19 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   }
   const int steps = K / LK;
   auto stage = [&](int t, int slot) {
-    const bool on = t < steps;                   // past the end: zeros
+    // past the end: zeros, by an empty buffer; an offset in front of its bounds check
+    // would be taken from a size of 0
+    const bool on = t < steps;
+    const unsigned col = on ? t * (LK * 2) : 0u;
     const auto ws = mr_buffer(wp, on ? w_bytes : 0u);
     const auto xs = mr_buffer(xp, on ? x_bytes : 0u);
     unsigned short* dst = lds + slot * TILE;
 #pragma unroll
     for (int i = 0; i < WI; i++)
-      mr_to_lds(ws, w_off[i], dst + (wid * WI + i) * 512, t * (LK * 2));
+      mr_to_lds(ws, w_off[i], dst + (wid * WI + i) * 512, col);
 #pragma unroll
     for (int i = 0; i < XI; i++)
-      mr_to_lds(xs, x_off[i], dst + WT + (wid * XI + i) * 512, t * (LK * 2));
+      mr_to_lds(xs, x_off[i], dst + WT + (wid * XI + i) * 512, col);
   };
   // a wave multiplies 32 rows of W by all of x over half of the step's columns
   const int hw = wid % (NW / 2), hk = wid / (NW / 2);

@@ -15,9 +15,10 @@ from xllm_service_amd.ops import ref
 pytestmark = pytest.mark.gpu
 
 
-def _step(layers, cfg, prompts, decodes, first, no_slot=()):
+def _step(layers, cfg, prompts, decodes, first, no_slot=(), held=list):
     """One pass over chunks of `prompts` tokens behind 20 cached ones and rows of
-    `decodes` cached ones; fresh inputs and caches every time."""
+    `decodes` cached ones; fresh inputs and caches every time. `held`: what holds
+    the caches of the layers."""
     g = torch.Generator(device="cuda").manual_seed(3)
     T, pages = sum(prompts) + len(decodes), 80
 
@@ -52,7 +53,7 @@ def _step(layers, cfg, prompts, decodes, first, no_slot=()):
     x, residual = bf(T, cfg.hidden_size), bf(T, cfg.hidden_size)
     pos = torch.tensor(pos, device="cuda")
     residual = None if first else residual
-    done = _native_layers(layers, x, residual, pos, caches, meta, cos_sin)
+    done = _native_layers(layers, x, residual, pos, held(caches), meta, cos_sin)
     if done is None:
         done = x, residual
         for layer, kv in zip(layers, caches):
@@ -125,3 +126,20 @@ def test_rotated_products(name, prompts, decodes):
         assert _off(a[new], b[new]) < 2.0 ** -6
         off = (a[new].double() - b[new].double()).norm(dim=-1)
         assert (off < 2.0 ** -5 * b[new].double().norm(dim=-1)).all()
+
+
+def test_caches_by_index():
+    """A cache for every layer, found by its number: too few are refused."""
+    cfg = get_config("llama-2k")
+    with torch.device("cuda"):
+        layers = [LlamaDecoderLayer(cfg, torch.bfloat16) for _ in range(3)]
+    for p in torch.nn.ModuleList(layers).parameters():
+        p.data.normal_(0.0, 0.02)
+    with torch.inference_mode():
+        want, _ = _step(layers, cfg, [5], [31], True)
+        got, _ = _step(layers, cfg, [5], [31], True,
+                       held=lambda c: dict(reversed(list(enumerate(c)))))
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        for held in (lambda c: c[:2], lambda c: tuple(c[:1]), lambda c: []):
+            with pytest.raises(IndexError):
+                _step(layers, cfg, [5], [31], True, held=held)

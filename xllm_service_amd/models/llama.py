@@ -158,8 +158,8 @@ def _native_layers(layers, x, residual, positions, kv_caches, meta, cos_sin):
             or torch.overrides.has_torch_function((x, residual)):
         return None
     weights = []
-    for layer, kv_cache in zip(layers, kv_caches):
-        w = layer._native_weights(kv_cache)
+    for i, layer in enumerate(layers):
+        w = layer._native_weights(kv_caches[i])
         if w is None:
             return None
         weights.append(w)

@@ -15,10 +15,11 @@ from xllm_service_amd.ops import ref
 pytestmark = pytest.mark.gpu
 
 
-def _step(layers, cfg, prompts, decodes, first, no_slot=(), held=list):
+def _step(layers, cfg, prompts, decodes, first, no_slot=(), held=list,
+          mrope=False):
     """One pass over chunks of `prompts` tokens behind 20 cached ones and rows of
     `decodes` cached ones; fresh inputs and caches every time. `held`: what holds
-    the caches of the layers."""
+    the caches of the layers; `mrope`: three rows of positions, each its own."""
     g = torch.Generator(device="cuda").manual_seed(3)
     T, pages = sum(prompts) + len(decodes), 80
 
@@ -52,6 +53,8 @@ def _step(layers, cfg, prompts, decodes, first, no_slot=(), held=list):
     cos_sin = ref.rope_table(cfg.head_dim, 256, cfg.rope_theta).cuda()
     x, residual = bf(T, cfg.hidden_size), bf(T, cfg.hidden_size)
     pos = torch.tensor(pos, device="cuda")
+    if mrope:
+        pos = torch.stack([pos, pos // 2, pos // 3 + 7])
     residual = None if first else residual
     done = _native_layers(layers, x, residual, pos, held(caches), meta, cos_sin)
     if done is None:
@@ -143,3 +146,31 @@ def test_caches_by_index():
         for held in (lambda c: c[:2], lambda c: tuple(c[:1]), lambda c: []):
             with pytest.raises(IndexError):
                 _step(layers, cfg, [5], [31], True, held=held)
+
+
+@pytest.mark.parametrize("name,value", [("scale", 0.5), ("eps", 0.25),
+                                        ("mrope_sections", (16, 24, 24))])
+def test_settings_of_a_layer(name, value):
+    """What one layer has its own of acts on this one: results as the modules give
+    them, not as all layers with the first one's settings do."""
+    cfg = get_config("llama-2k")
+    with torch.device("cuda"):
+        layers = [LlamaDecoderLayer(cfg, torch.bfloat16) for _ in range(3)]
+    g = torch.Generator(device="cuda").manual_seed(1)
+    for n, p in torch.nn.ModuleList(layers).named_parameters():
+        p.data.normal_(1.0 if "norm" in n else 0.0, 0.02, generator=g)
+    rows = name == "mrope_sections"
+    args = layers, cfg, [40, 33], [17], True
+    if rows:
+        for layer in layers:
+            layer.attn.mrope_sections = (64, 0, 0)
+    with torch.inference_mode():
+        same, _ = _step(*args, mrope=rows)
+        setattr(layers[1] if name == "eps" else layers[1].attn, name, value)
+        got, _ = _step(*args, mrope=rows)
+        for layer in layers:
+            layer.mlp.down.register_forward_hook(lambda *a: None)
+        want, _ = _step(*args, mrope=rows)
+    assert max(_off(a, b) for a, b in zip(same, want)) > 2.0 ** -5
+    for a, b in zip(got, want):
+        assert _off(a, b) < 2.0 ** -6

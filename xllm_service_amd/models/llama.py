@@ -165,7 +165,11 @@ def _native_layers(layers, x, residual, positions, kv_caches, meta, cos_sin):
         weights.append(w)
     first = layers[0]
     attn = first.attn
-    if any(layer.eps != first.eps for layer in layers):
+
+    def settings(layer):
+        a = layer.attn
+        return layer.eps, a.n_heads, a.n_kv_heads, a.scale, a.mrope_sections
+    if any(settings(layer) != settings(first) for layer in layers):
         return None
     ms0 = ms1 = 0
     if attn.mrope_sections and positions.dim() != 1:

@@ -24,10 +24,21 @@ from xllm_service_amd.models.config import ModelConfig
 from xllm_service_amd.ops import ref as op_ref
 
 
+# hooks of all modules: the dicts that a module's call looks at
+_EVERY_HOOK = (module_hooks._global_forward_hooks,
+               module_hooks._global_forward_pre_hooks,
+               module_hooks._global_backward_hooks,
+               module_hooks._global_backward_pre_hooks)
+
+
 def _plain(module, kind):
-    """A module of this very class that nothing observes or replaces."""
-    return (type(module) is kind and not module._forward_hooks
-            and not module._forward_pre_hooks
+    """A module of this very class that nothing observes or replaces: what its call
+    would do besides its forward is nothing."""
+    return (type(module) is kind
+            and not (module._forward_hooks or module._forward_pre_hooks
+                     or module._backward_hooks or module._backward_pre_hooks
+                     or any(_EVERY_HOOK))
+            and module._compiled_call_impl is None
             and "forward" not in module.__dict__)
 
 
@@ -152,9 +163,7 @@ def _native_layers(layers, x, residual, positions, kv_caches, meta, cos_sin):
     """Layers as one native call, or None where one of their modules is not the
     plain one or torch has to see the calls: gradients, modes, tracing."""
     if not (x.is_cuda and ops.HAS_EXT and torch.is_inference_mode_enabled()
-            and ps.tp_size() == 1) or module_hooks._global_forward_hooks \
-            or module_hooks._global_forward_pre_hooks \
-            or torch.compiler.is_compiling() \
+            and ps.tp_size() == 1) or torch.compiler.is_compiling() \
             or torch.overrides.has_torch_function((x, residual)):
         return None
     weights = []

@@ -471,8 +471,10 @@ torch::Tensor linear_gated(torch::Tensor x, torch::Tensor w,
 }
 
 // Rows between two products of a layer: as an RMS norm leaves them, or without their
-// factors and with the sums of their squares' parts [rows][tiles]
-struct Rows { torch::Tensor x, squares; };
+// factors, with the sums of their squares' parts [rows][tiles] and the kernels that
+// take the product which they were made for (linear_kind, asked once: torch's table
+// of tuned products may change meanwhile)
+struct Rows { torch::Tensor x, squares; int kind = 0; };
 
 static xllm::LinearEnds scale_of(const Rows& in, double eps) {
   xllm::LinearEnds e;
@@ -492,7 +494,7 @@ static torch::Tensor product(const Rows& in, const torch::Tensor& w,
   auto y = torch::empty({M, gate ? N / 2 : N}, in.x.options());
   xllm::launch_linear(u16(y), u16c(in.x), u16c(w),
                       bias.has_value() ? u16c(*bias) : nullptr, (int)M, (int)N,
-                      (int)K, in.x.stride(0), linear_kind(in.x, w, bias),
+                      (int)K, in.x.stride(0), in.kind,
                       xllm::LN_SCALE | (gate ? xllm::LN_GATE : 0),
                       scale_of(in, eps), cur_stream());
   return y;
@@ -515,9 +517,10 @@ static Rows product_normed(const torch::Tensor& x, const torch::Tensor& w,
       reinterpret_cast<uintptr_t>(norm.data_ptr()) % 16 == 0 &&
       res.is_cuda() && norm.is_cuda() &&
       !(next_gate && (next_bias.has_value() || next_w.size(0) % 16 != 0))) {
-    Rows out{torch::empty({M, N}, x.options()), {}};
+    Rows out{torch::empty({M, N}, x.options())};
     const int next = linear_kind(out.x, next_w, next_bias);
     const int tiles = xllm::linear_tiles((int)M, (int)N, (int)K, kind);
+    out.kind = next;
     if (next != 0 && tiles % 4 == 0 && tiles <= (next == 1 ? 256 : 64)) {
       out.squares = torch::empty({M, tiles}, x.options().dtype(torch::kFloat));
       xllm::LinearEnds e;
@@ -532,7 +535,7 @@ static Rows product_normed(const torch::Tensor& x, const torch::Tensor& w,
   }
   auto h = ::linear(x, w, none);
   fused_add_rmsnorm(h, res, norm, eps);
-  return {h, {}};
+  return {h};
 }
 
 struct DecoderLayer {
@@ -624,7 +627,7 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layers(
       e.block = (int)p.k_cache.size(2);
       xllm::launch_linear(u16(q), u16c(in.x), u16c(p.qkv_w), nullptr, (int)T,
                           (int)p.qkv_w.size(0), (int)p.qkv_w.size(1),
-                          in.x.stride(0), linear_kind(in.x, p.qkv_w, p.qkv_b),
+                          in.x.stride(0), in.kind,
                           xllm::LN_SCALE | xllm::LN_ROPE, e, cur_stream());
     } else {
       const auto qkv = product(in, p.qkv_w, p.qkv_b, false, eps);

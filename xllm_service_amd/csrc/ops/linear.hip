@@ -7,6 +7,8 @@
 // lane, 256 B of a row at a time) with the 16 B chunks of a row permuted by the
 // row: whole-row reads then meet no bank twice. W rows are the A operand, x rows
 // the B operand of 16x16x32 products; sums are fp32.
+#include <stdexcept>
+
 #include "linear.h"
 #include "mfma_rows.h"
 
@@ -842,6 +844,7 @@ void launch_linear(unsigned short* y, const unsigned short* x,
                    const unsigned short* w, const unsigned short* bias, int M,
                    int N, int K, long x_stride, int kind, int mode,
                    const LinearEnds& ends, hipStream_t stream) {
+  if (kind != 1 && kind != 2) throw std::invalid_argument("linear: kernels");
 #define LN_MODE(MODE)                                                          \
   case MODE:                                                                   \
     if (kind == 1)                                                             \
@@ -856,6 +859,7 @@ void launch_linear(unsigned short* y, const unsigned short* x,
     LN_MODE(LN_SCALE | LN_GATE);
     LN_MODE(LN_ADD);
     LN_MODE(LN_SCALE | LN_ROPE);
+    default: throw std::invalid_argument("linear: mode");
   }
 #undef LN_MODE
 }

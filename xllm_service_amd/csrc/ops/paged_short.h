@@ -19,6 +19,7 @@ namespace xllm {
 
 #define PS_ROWS 32         // rows per workgroup
 #define PS_WAVES 4
+#define PS_KEYS 2048       // of a table, at most
 
 template <int D, int TERMS>
 __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
@@ -94,13 +95,14 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
     koff[i] = (unsigned)(r * (2 * D) + ((spos ^ mr_swz_rows<D>(r)) << 4));
     voff[i] = (unsigned)(r * (2 * D) + ((spos ^ mr_swz_cols<D>(r)) << 4));
   }
-  // Where the pages of 16 of this wave's tiles from the tb-th on are, and how much of
-  // each is keys, one page per lane. Rows past the last key, and tiles past the last
-  // one, are out of the bounds: zeros.
-  int tb = 0;
+  // Where the pages of this wave's tiles are, and how much of each is keys, one page
+  // per lane: 16 tiles, where a table of PS_KEYS keys has 8 for a wave and one past them
+  // is asked for. Rows past the last key, and tiles past the last one, are out of the
+  // bounds: zeros.
+  static_assert((PS_KEYS / PF_KT / PS_WAVES + 1) * PAGES <= 64, "pages per lane");
   unsigned at_lo = 0, at_hi = 0, bytes = 0;
   auto look_up = [&]() {
-    const int t = wid + PS_WAVES * (tb + (lane >> 2));
+    const int t = wid + PS_WAVES * (lane >> 2);
     const int pg = min(t, n - 1) * PAGES + (lane & 3);
     const long at =
         ((long)btab[min(pg, last_blk)] * n_kv + kvh) * (PF_BS * D * 2);
@@ -114,7 +116,7 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
   auto stage = [&](int i, bool val) {
 #pragma unroll
     for (int p = 0; p < PAGES; p++) {
-      const int at = (i - tb) * PAGES + p;
+      const int at = i * PAGES + p;
       const unsigned lo = __builtin_amdgcn_readlane(at_lo, at);
       const unsigned hi = __builtin_amdgcn_readlane(at_hi, at);
       const auto src = mr_buffer(
@@ -159,11 +161,6 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
                           kt + (kbase ^ (ks << 4)) + j * 32 * D),
                       qf[ks], s[j]);
     read();
-    // this tile's values are on their way: its pages are not asked for again
-    if (i + 1 - tb == 16) {
-      tb += 16;
-      look_up();
-    }
     stage(i + 1, false);
     if (k0 + PF_KT > wmin) {                     // uniform: a tile on the diagonal
 #pragma unroll
@@ -280,7 +277,7 @@ inline bool paged_short_takes(long tokens, int n_seqs, int G, int n_kv,
                               long max_blocks, int terms) {
   return paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv <= 256 &&
          max_blocks * PF_BS >= 128 &&
-         max_blocks * PF_BS <= (terms > 1 ? 1024 : 2048);
+         max_blocks * PF_BS <= (terms > 1 ? PS_KEYS / 2 : PS_KEYS);
 }
 
 template <int D, int TERMS>

@@ -177,7 +177,8 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
     const unsigned short* __restrict__ w,
     const unsigned short* __restrict__ bias, const int M, const int N,
-    const int K, const long x_stride, const LinearEnds ends) {
+    const int K, const long x_stride, const unsigned turns,
+    const LinearEnds ends) {
   constexpr bool GATE = MODE & LN_GATE, SCALE = MODE & LN_SCALE,
                  ADD = MODE & LN_ADD, ROPE = MODE & LN_ROPE;
   constexpr bool PAIR = GATE || ROPE;            // two rows of W to a column
@@ -254,17 +255,19 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
   for (int i = 0; i < NT; i++)
 #pragma unroll
     for (int j = 0; j < MT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int steps = K / LN_K, turn = blockIdx.x % steps;
+  const int steps = K / LN_K;
+  const int turn = (int)__umulhi(blockIdx.x * turns, (unsigned)steps);
   const int mine = (steps - wid + NW - 1) / NW;  // of this wave
-  auto load = [&](int i, int slot) {
-    int t = wid + i * NW + turn;
-    t = (t >= steps ? t - steps : t) * LN_K;
-    lw.load(wp + t, wt + slot * TILE);
-    lx.load(x + t, wt + slot * TILE + T);
+  auto column = [&](int i) {
+    const int t = wid + i * NW + turn;
+    return (t >= steps ? t - steps : t) * LN_K;
   };
 #pragma unroll
   for (int d = 0; d < D; d++)
-    if (d < mine) load(d, d);
+    if (d < mine) {
+      lw.load(wp + column(d), wt + d * TILE);
+      lx.load(x + column(d), wt + d * TILE + T);
+    }
   for (int i = 0, slot = 0; i < mine; i++, slot = slot + 1 == D ? 0 : slot + 1) {
     if (D == 2 && i + 1 < mine)                  // the next tile may be on the way
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((WR + XR) / 4) : "memory");
@@ -283,12 +286,15 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
       rows(r, r0);
       rows(r + 1, r1);
       ln_read2(r0, r1, v[r], v[r + 1]);
+      // W is read, its next tile may come: 64 rows, 2560 x 2560 9.4 -> 9.1 us
+      if (r < NT && r + 2 >= NT && i + D < mine)
+        lw.load(wp + column(i + D), wt + slot * TILE);
     }
     if constexpr (TILES % 2 != 0) {
       rows(TILES - 1, r0);
       ln_read(r0, v[TILES - 1]);
     }
-    if (i + D < mine) load(i + D, slot);
+    if (i + D < mine) lx.load(x + column(i + D), wt + slot * TILE + T);
 #pragma unroll
     for (int ks = 0; ks < 4; ks++)
 #pragma unroll
@@ -759,19 +765,29 @@ int linear_takes(long M, long N, long K, bool bias) {
 }
 
 // Row tiles of W: one up to 4096 rows of it, one workgroup a CU then; two above.
-// Up to 16 rows of x weigh little, and where W has many columns and its row
-// tiles leave few CUs without one in the last turn, one tile is the better again:
-// M 8, 8192 x 4096 12.8 one | 13.5 two, 12288 x 4096 17.9 | 19.9, 8192 x 8192 26.2 |
-// 29.8; but 4608 x 4096 10.5 | 9.4 (a ninth of the CUs have two), 14336 x 4096
-// 22.2 | 21.1, 8192 x 2048 9.1 | 8.0; M 24, 8192 x 4096 15.6 | 14.4.
+// Up to 16 rows of x weigh little, and where W has long rows and many columns, one
+// tile is the better again if the last turn of the CUs leaves fewer of them idle with
+// it, or as few and no more than a tenth. M 8, one | two: 8192 x 4096 13.7 | 14.2, 9216 x
+// 4096 17.3 | 19.7, 12288 x 4096 19.5 | 21.6, 18944 x 3584 26.8 | 27.9, 28672 x 4096 40.4 |
+// 42.7; but 4608 x 3584 10.4 | 9.5 (a ninth of the CUs have two), 14336 x 4096 23.7 | 22.4,
+// 22016 x 4096 33.6 | 33, 24576 x 2048 22.9 | 19.8; M 24, 8192 x 4096 16.6 | 15.3.
+// Short rows have little to share: M 8, 8192 x 640 4.4 | 4.7, 7424 x 1536 6.5 | 6.7, 10240 x
+// 1536 8.3 | 9.3, but 4352 x 1536 5.8 | 5.6.
 static bool linear_one_tile(int M, int N, int K) {
-  const int wgs = (N + 15) / 16;
-  return wgs <= 256 ||
-         (M <= 16 && K >= 4096 && 10 * wgs >= 9 * ((wgs + 255) / 256 * 256));
+  const int wgs = (N + 15) / 16, turns = (wgs + 255) / 256;
+  const int of_two = ((N + 31) / 32 + 255) / 256;
+  if (wgs <= 256) return true;
+  if (M > 16) return false;
+  if (K >= 2048)
+    return K >= 2560 && (turns < 2 * of_two || 10 * wgs >= 9 * 256 * turns);
+  if (N <= 8192) return K <= 640 || (K <= 1536 && N > 6656);
+  return turns < 2 * of_two && K >= (M <= 8 ? 1024 : 1536);
 }
 // A workgroup that has a CU to itself takes all of its LDS: two tiles a wave, or
 // more waves. Where there are more than CUs, two of them share one: M 24, 32000 x
-// 4096 48.4, with two tiles 49.2; 18944 x 4096 33.4 | 34.5.
+// 4096 48.4, with two tiles 49.2; 18944 x 4096 33.4 | 34.5. Up to 16 rows, and up to 32 of
+// short rows of W, eight waves are up to 5% faster than four with two tiles each:
+// M 10, 768 x 3072 4.2 -> 4.1, M 32, 2560 x 2560 7.3 -> 6.9, but 4096 x 4096 10.4 | 10.5.
 template <int MODE>
 static void launch_stream(unsigned short* y, const unsigned short* x,
                           const unsigned short* w, const unsigned short* bias,
@@ -782,15 +798,22 @@ static void launch_stream(unsigned short* y, const unsigned short* x,
   const int out = (one ? 16 : 32) / PAIR, n_out = N / PAIR;
   const dim3 grid((n_out + out - 1) / out);
   const bool few = grid.x <= 256;
+  // Workgroup b starts at step b mod steps, which its product with 2^32 / steps holds in
+  // the upper bits; at the first one where a product is small (0): 10 rows, 768 x 768
+  // 2.9 us, with a division 3.0; 4096 x 4096 8.2, without turns 9.1.
+  const int steps = K / LN_K;
+  const unsigned turns =
+      (long)N * K < 1L << 23 ? 0u : (unsigned)(((1L << 32) + steps - 1) / steps);
 #define LN_STREAM(NT, XR, NW, D)                                               \
   hipLaunchKernelGGL((linear_stream_kernel<NT, XR, NW, D, MODE>), grid,        \
                      dim3(NW * 64), 0, stream, y, x, w, bias, M, N, K,         \
-                     x_stride, ends)
+                     x_stride, turns, ends)
   if (one) {
-    if (M <= 8) LN_STREAM(1, 8, 4, 2);
-    else if (M <= 16) LN_STREAM(1, 16, 4, 2);
+    const bool eight = few || K <= 1536;
+    if (M <= 8) { if (eight) LN_STREAM(1, 8, 8, 1); else LN_STREAM(1, 8, 4, 2); }
+    else if (M <= 16) { if (eight) LN_STREAM(1, 16, 8, 1); else LN_STREAM(1, 16, 4, 2); }
     else if (M <= 24) LN_STREAM(1, 24, 4, 2);
-    else if (M <= 32) LN_STREAM(1, 32, 4, 2);
+    else if (M <= 32) { if (K <= 2560) LN_STREAM(1, 32, 8, 1); else LN_STREAM(1, 32, 4, 2); }
     else if (M <= 48) LN_STREAM(1, 48, 4, 2);
     else LN_STREAM(1, 64, 4, 2);
   } else {

@@ -62,7 +62,11 @@ def test_rows_of_a_wider_tensor(M, N, K):
     (65, 64, 128, 0), (97, 136, 256, 8), (128, 3080, 384, 0),    # 32 rows of x
     (200, 2056, 640, 8), (250, 3080, 1152, 0), (300, 4104, 256, 8),
     (380, 4040, 128, 0), (500, 3080, 2048, 8),                   # 128 of W
-    (70, 3080, 4736, 0), (2048, 200, 384, 0), (8000, 72, 256, 8)])
+    (70, 3080, 4736, 0), (2048, 200, 384, 0), (8000, 72, 256, 8),
+    (140, 4040, 4224, 0),                                        # 64, not 48, of x
+    (70, 200, 128, 8), (350, 1544, 384, 0), (505, 2056, 256, 8),  # short rows
+    (126, 8456, 384, 8), (300, 4872, 1024, 0), (577, 2056, 128, 8),  # square tiles
+    (65, 16392, 2048, 0), (90, 8456, 1152, 8)])                  # many columns
 def test_shapes_of_prompt_tiles(M, N, K, stride):
     """Every shape of a tile, with remainders of both sides and fewer steps than
     buffers; longest rows. 2^-17 covers K up to 4096, 2^-16.8 up to 4736."""
@@ -79,7 +83,7 @@ def test_shapes_of_prompt_tiles(M, N, K, stride):
 
 @pytest.mark.parametrize("M", [1, 8, 24, 33, 64, 65, 100, 250, 500])
 @pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (4112, 640), (8208, 384),
-                                 (3088, 2048)])
+                                 (3088, 2048), (4880, 1024)])
 def test_gated(M, N, K):
     """Gates and their partners in one product, against fp64: 2^-8 for the result's
     rounding, and of each sum, where a caller's two products round them, 2^-8 more

@@ -430,6 +430,9 @@ static int linear_kind(const torch::Tensor& x, const torch::Tensor& w,
              : kind;
 }
 
+// Kernels that do more than the product (LinearEnds)
+static bool has_ends(int kind) { return kind == 1 || kind == 2; }
+
 // x [..., K] @ w [N, K]^T (+ bias): the kernels of linear.hip where they take the
 // call, the library elsewhere (and wherever a gradient is wanted)
 torch::Tensor linear(torch::Tensor x, torch::Tensor w,
@@ -452,7 +455,7 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor w,
 torch::Tensor linear_gated(torch::Tensor x, torch::Tensor w,
                            c10::optional<torch::Tensor> bias) {
   if (!bias.has_value() && w.dim() == 2 && w.size(0) % 16 == 0) {
-    if (const int kind = linear_kind(x, w, bias)) {
+    if (const int kind = linear_kind(x, w, bias); has_ends(kind)) {
       const long M = x.size(0), N = w.size(0), K = w.size(1);
       c10::OptionalDeviceGuard guard(x.device());
       auto y = torch::empty({M, N / 2}, x.options());
@@ -510,7 +513,7 @@ static Rows product_normed(const torch::Tensor& x, const torch::Tensor& w,
   const c10::optional<torch::Tensor> none;
   const int kind = linear_kind(x, w, none);
   const long M = x.size(0), N = w.size(0), K = w.size(1);
-  if (kind != 0 && res.dim() == 2 && res.is_contiguous() && res.size(0) == M &&
+  if (has_ends(kind) && res.dim() == 2 && res.is_contiguous() && res.size(0) == M &&
       res.size(1) == N && res.dtype() == torch::kBFloat16 && on_bytes(res, 16) &&
       norm.dim() == 1 && norm.size(0) == N && norm.is_contiguous() &&
       norm.dtype() == torch::kBFloat16 &&
@@ -521,7 +524,7 @@ static Rows product_normed(const torch::Tensor& x, const torch::Tensor& w,
     const int next = linear_kind(out.x, next_w, next_bias);
     const int tiles = xllm::linear_tiles((int)M, (int)N, (int)K, kind);
     out.kind = next;
-    if (next != 0 && tiles % 4 == 0 && tiles <= (next == 1 ? 256 : 64)) {
+    if (has_ends(next) && tiles % 4 == 0 && tiles <= (next == 1 ? 256 : 64)) {
       out.squares = torch::empty({M, tiles}, x.options().dtype(torch::kFloat));
       xllm::LinearEnds e;
       e.residual = reinterpret_cast<unsigned short*>(res.data_ptr());

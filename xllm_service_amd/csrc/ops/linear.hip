@@ -420,8 +420,8 @@ __global__ __launch_bounds__(NW * 64) void linear_stream_kernel(
 // compiler lets no LDS read pass another. Us, 64 x 64 tiles of four waves, a quarter
 // of the products each -> here: 300 x 2048 x 2048 11.2 -> 9.4, 4096 x 2048 16.3 -> 13.2,
 // 4096 x 4096 29.5 -> 22.5, 3072 x 2048 11.7 -> 11.6; 96 x 3072 x 2048 10.9 -> 9.6;
-// 192 x 6144 x 4096 30.1 -> 25.7; 512 x 3072 x 2048 16.5 -> 16.7; 256 x 3072 x 2048, as many
-// tiles of 64 x 64 either way, 11.8 -> 12.1.
+// 192 x 6144 x 4096 30.1 -> 25.7; 256 x 3072 x 2048, as many
+// tiles of 64 x 64 either way, 12.0 -> 11.9 (a ring of five there 12.2).
 template <int NW, int MT, int LK, int S, int MODE>
 __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
     unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
@@ -688,7 +688,91 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
   }
 }
 
-// 0: the library's; 1: stream; 2: tiles. Besides its time on the GPU a library
+// More tiles of 64 x 64 than CUs, rows of W up to 2048: two workgroups share a CU, four
+// waves, a quarter of the tile each; two buffers, one barrier per step of 128 columns.
+// Bound by what comes before and after its few steps, which two workgroups cover for
+// each other. Us, linear_tile_kernel | here: 256 x 6912 x 640 9.9 | 8.0, 300 x 4864 x 1024
+// 11.2 | 9.9, 500 x 4096 x 1536 14.5 | 13.8, 256 x 6912 x 128 5.1 | 4.1.
+__global__ __launch_bounds__(256, 2) void linear_square_kernel(
+    unsigned short* __restrict__ y, const unsigned short* __restrict__ x,
+    const unsigned short* __restrict__ w, const int M, const int N,
+    const int K, const long x_stride, const int n_tiles_n) {
+  constexpr int HALF = 64 * LN_K, TILE = 2 * HALF;
+  __shared__ __attribute__((aligned(1024))) unsigned short lds[2 * TILE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, c32 = lane & 31;
+  const long n0 = (blockIdx.x % n_tiles_n) * 64L;
+  const long m0 = (blockIdx.x / n_tiles_n) * 64L;
+  const int wn = wid & 1, wm = wid >> 1;
+  // a wave loads 16 rows of both; rows past the last one repeat it
+  LnTile<16> lw, lx;
+  const long nr = min(n0 + wid * 16, (long)N - 1);
+  const long mr = min(m0 + wid * 16, (long)M - 1);
+  lw.init(nr, N, K, lane);
+  lx.init(mr, M, x_stride, lane);
+  const unsigned short* wp = w + nr * K;
+  const unsigned short* xp = x + mr * x_stride;
+  unsigned short* mine = lds + wid * 16 * LN_K;
+  // bytes of chunk 2 k + h of a lane's row in either half
+  const unsigned base = (unsigned)(unsigned long long)(const lds_u16*)lds;
+  unsigned wat[8], xat[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const int rw = wn * 32 + c32, rx = wm * 32 + c32;
+    wat[k] = base + 2 * (rw * LN_K + (((2 * k + h) ^ (rw & 15)) << 3));
+    xat[k] = base + 2 * (HALF + rx * LN_K + (((2 * k + h) ^ (rx & 15)) << 3));
+  }
+  f32x16 acc = mr_zero();
+  const int steps = K / LN_K;
+  auto stage = [&](int t) {
+    unsigned short* dst = mine + (t & 1) * TILE;
+    lw.load(wp + t * LN_K, dst);
+    lx.load(xp + t * LN_K, dst + HALF);
+  };
+  stage(0);
+  for (int t = 0; t < steps; t++) {
+    const unsigned buf = (t & 1) * (2 * TILE);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    if (t + 1 < steps) stage(t + 1);
+#pragma unroll
+    for (int k = 0; k < 8; k += 4) {
+      unsigned a_at[4], b_at[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        a_at[i] = wat[k + i] + buf;
+        b_at[i] = xat[k + i] + buf;
+      }
+      bf16x8 a[4], b[4];
+      ln_read2(a_at, b_at, a, b);
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc = mr_mma(a[i], b[i], acc);
+    }
+  }
+  // through LDS to whole rows
+  __syncthreads();
+  constexpr int ROW = 64 + 8;                    // bf16 of a row, padded
+#pragma unroll
+  for (int r = 0; r < 16; r += 4) {
+    uint2 o;
+    o.x = pack_bf16(acc[r], acc[r + 1]);
+    o.y = pack_bf16(acc[r + 2], acc[r + 3]);
+    *reinterpret_cast<uint2*>(lds + (wm * 32 + c32) * ROW + wn * 32 + 2 * r +
+                              4 * h) = o;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int idx = tid + i * 256, row = idx >> 3, col = (idx & 7) * 8;
+    if (m0 + row < M && n0 + col < N)
+      *reinterpret_cast<uint4*>(y + (m0 + row) * N + n0 + col) =
+          *reinterpret_cast<const uint4*>(lds + row * ROW + col);
+  }
+}
+
+// 0: the library's; 1: stream; 2: tiles; 3: square ones, without LinearEnds' options.
+// Besides its time on the GPU a library
 // call costs 28 us of host time (its choice of a kernel), these cost 6.
 // Measured, us on the GPU, here | library, weights from memory (N x K):
 //   M 8      2048 x 2048 4.1 | 8.9, 4096 x 4096 7.7 | 15.3, 4096 x 14336 21 | 25, 28672 x
@@ -724,11 +808,14 @@ __global__ __launch_bounds__(NW * 64) void linear_tile_kernel(
 
 // Of the shapes that linear_tile_kernel has, the one that a CU pulls least for: turns
 // of the CUs times the rows of a tile. x rows of 64 rows of W, or 0: 64 of 128.
-static int linear_shape(long M, long N, long* turns) {
+// Three row tiles of 48 without a smaller fourth one, which would fetch W ahead of
+// the others, cost long rows more than two of 64 and a rest: M 144, 4096 x 14336 59.7 |
+// 52.7, 4096 x 8192 34.4 | 31.2, 3584 x 18944 74.6 | 66.1; M 152 48.3 | 54.8.
+static int linear_shape(long M, long N, long K, long* turns) {
   int best = 0;
   long least = 0;
   for (int mt = 0; mt <= 6; mt++) {
-    if (mt == 1) continue;
+    if (mt == 1 || (mt == 3 && K > 4096 && M > 128 && M <= 144)) continue;
     const long wr = mt == 0 ? 128 : 64, xr = mt == 0 ? 64 : 16 * mt;
     const long t = ((N + wr - 1) / wr * ((M + xr - 1) / xr) + 255) / 256;
     const long cost = t * (wr + xr);
@@ -744,24 +831,65 @@ int linear_takes(long M, long N, long K, bool bias) {
   if (M <= 0 || K < LN_K || K % LN_K != 0 || N % 8 != 0) return 0;
   if (N * K >= (1L << 31) || M * K >= (1L << 30)) return 0;
   if (M <= 16) return M <= 8 || N * K <= 1L << 28 ? 1 : 0;
-  // few workgroups with long rows
-  if (M <= 32)
-    return (N > 1024 || K <= 8192) &&
-           (N <= 8192 || (K <= 4096 && N * K <= 1L << 28)) ? 1 : 0;
-  if (M <= 48)
-    return N <= 8192 ? (N > 2048 || K < 8192 ? 1 : 0)
-                     : N * K <= 1L << 28 &&
-                       (K <= 2048 || (K <= 4096 && N >= 18432)) ? 1 : 0;
-  if (M <= 64)
-    return N <= 8192 && (K <= 4096 || (N >= 2048 && N <= 4096 && K <= 8192)) ? 1 : 0;
+  // More than 8192 columns: x rows weigh more and more, and the last turn of the CUs
+  // counts. Here | library, M 20 | M 28-32: 50272 x 768 20.7 | 20, 21.6 | 20.4, 9216 x
+  // 4096 22.6 | 20.5, 24.1 | 21.4, 12288 x 4096 24.2 | 23.4, 25.6 | 24, 14336 x 4096 25.2 |
+  // 25.8, 27.2 | 26.3, 16384 x 4096 27.1 | 32.5, 28.5 | 32.6, 24576 x 3072 31.5 | 31.3, 33.2 |
+  // 31.5, 37888 x 3584 53.6 | 54.9, 57 | 55.7
+  // The library splits long rows of whole 1024s over workgroups: few workgroups here
+  // wait longer for theirs. Here | library, 512 x 8192 | 512 x 8448: M 24 8.2 | 8.1, 8.6 |
+  // 17.7, M 40 10.9 | 7.9, 11.4 | 17.5, M 64 13.5 | 8.4, 14 | 17.8; M 32, 512 x 16384 18.4 | 19.2
+  const bool split = K >= 6144 && K % 1024 == 0;
+  if (M <= 32) {
+    if (N <= 8192)
+      return N > 1024 || K <= 8192 || !split || M > 24 || N <= 256 ? 1 : 0;
+    if (K <= 2048) return N <= 32768 ? 1 : 0;
+    return K <= 4096 && (M <= 24 ? N >= 14336 && N * K <= 1L << 28
+                                 : N >= 16384 && K > 3072 && N * K <= 1L << 27) ? 1 : 0;
+  }
+  // M 40: 14336 x 2048 16.9 | 17.4, 32000 x 1024 18.6 | 25.9; 24576 x 2048 25.4 | 25, 28672 x
+  // 4096 53.1 | 48.3 (M 48 55.4 | 58.5), 50272 x 768 23.7 | 21.7, 18944 x 3584 36.7 | 33.9
+  if (M <= 48) {
+    if (N <= 8192) return N > 2048 || !split || (N >= 1536 && K < 8192) ? 1 : 0;
+    return (K <= 2048 && N <= 16384) || (K <= 1024 && N <= 32768) ? 1 : 0;
+  }
+  if (M <= 64) {
+    if (N > 8192) return N * K <= 1L << 23 ? 1 : 0;   // M 57, 9600 x 384 6.7 | 8.2
+    if (K <= 4096 || (N >= 2048 && N <= 4096 && K <= 8192)) return 1;
+    return split ? (N >= 1280 && N <= 2048 && K < 8192 ? 1 : 0)
+                 : (N * K <= 1L << 24 ? 1 : 0);
+  }
   if (bias) return 0;
   long turns;
-  linear_shape(M, N, &turns);
-  if (turns > 1 || N > 8192 || (M > 2048 && N > 128)) return 0;
-  if (K > 4096) return N >= 3072 && N <= 4608 && M <= 192 ? 2 : 0;
-  // few tiles with long rows leave most of the chip waiting for their chain
-  if (K > 2048 && ((N < 3072 && M <= 128) || (N < 2048 && M <= 256))) return 0;
-  return 2;
+  const int shape = linear_shape(M, N, K, &turns);
+  const long squares = (M + 63) / 64 * ((N + 63) / 64);
+  // Up to two turns of square tiles where none of the others takes one, or has tiles
+  // of 128 rows: library | square, 126 x 8448 x 640 11.1 | 7.9, 160 x 9856 x 1536 19.8 | 17.3,
+  // 300 x 4864 x 1024 13.9 | 9.9, 256 x 6912 x 1536 20.8 | 14.9, 689 x 2688 x 1920 20.5 | 17;
+  // at 2048 no longer, 512 x 3072 x 2048 15.3 | 16.4, but 160 x 8448 x 2048 24.2 | 19.8
+  if (squares > 256 && squares <= 512 &&
+      K <= (shape == 0 || turns > 1 ? (N <= 8192 ? 1920 : 2048) : 512))
+    return 3;
+  if (turns > 1 || (M > 2048 && N > 128 && K > 1024)) return 0;
+  if (N > 8192 && (N > 16384 || K > 2048 || shape == 0)) return 0;
+  // 128 rows of W a tile, the library has as large ones from 257 rows on: M 512, 3072 x
+  // 2048 17 | 15.3, 3584 x 3584 27.6 | 25.8, M 300, 4608 x 3584 26.9 | 23.8; but M 256, 6144 x
+  // 4096 31.1 | 40.3, and short rows, M 512, 4096 x 1024 10.9 | 13.1
+  if (shape == 0 && M > 256 && K > 1536) return 0;
+  // M 80: 4096 x 14336 48.8 | 43.1, 4096 x 11008 40.9 | 35, 3584 x 8192 27.9 | 25.4 and at
+  // M 76 47.3 | 49.2, 39.6 | 40.7, 27 | 28.1; 3584 x 18944 61 | 130
+  if (K > 4096)
+    return N >= 3072 && N <= 4608 && M <= 192 &&
+           !(M > 76 && M <= 80 && N > 3072 && K <= 16384) ? 2 : 0;
+  // few tiles with long rows leave most of the chip waiting for their chain, many of
+  // them wait for each other: 256 x 4096, M 300 10 | 8.9, M 2048 16.2 | 13.8; M 1536, 640 x 2560
+  // 14.7 | 12.4, M 2048, 512 x 2048 13 | 10.8, 1024 x 4096 32.6 | 28.5
+  // 576 x 4096, M 300, 12.2 | 10.2, 832 x 3072, M 260, 11.1 | 8.7: where the tiles
+  // of W are no multiple of four, those that share one lie on several XCDs
+  if (K > 2048)
+    return N >= 512 && (N >= 1024 || N % 256 == 0) && M <= 1024 &&
+           !((N < 3072 && M <= 128) || (N < 2048 && M <= 256)) ? 2 : 0;
+  return M <= 1536 || K <= 1536 || N <= 128 ? 2 : 0;
 }
 
 // Row tiles of W: one up to 4096 rows of it, one workgroup a CU then; two above.
@@ -842,12 +970,15 @@ static void launch_tile(unsigned short* y, const unsigned short* x,
                        dim3((unsigned)(tn * tm)), dim3(NW * 64), 0, stream, y, \
                        x, w, M, N, K, x_stride, tn, ends);                     \
   } while (0)
+  // a ring longer than a row costs what its empty steps do: 300 x 1344 x 128 3.5 -> 3.1,
+  // 500 x 2048 x 256 4.3 -> 3.8
+  const bool short_row = K <= 384;
   long turns;
-  switch (linear_shape(M, N, &turns)) {
+  switch (linear_shape(M, N, K, &turns)) {
     case 0: LN_TILE(8, 4, 64, 6); break;
-    case 2: LN_TILE(4, 2, 128, 6); break;
-    case 3: LN_TILE(4, 3, 128, 5); break;
-    case 4: LN_TILE(4, 4, 128, 5); break;
+    case 2: if (short_row) LN_TILE(4, 2, 64, 4); else LN_TILE(4, 2, 128, 6); break;
+    case 3: if (short_row) LN_TILE(4, 3, 128, 3); else LN_TILE(4, 3, 128, 5); break;
+    case 4: if (short_row) LN_TILE(4, 4, 64, 4); else LN_TILE(4, 4, 128, 4); break;
     case 5: LN_TILE(4, 5, 128, 4); break;
     default: LN_TILE(4, 6, 128, 4);
   }
@@ -858,7 +989,7 @@ static void launch_tile(unsigned short* y, const unsigned short* x,
 int linear_tiles(int M, int N, int K, int kind) {
   if (kind == 1) return linear_one_tile(M, N, K) ? (N + 15) / 16 : (N + 31) / 32;
   long turns;
-  return linear_shape(M, N, &turns) == 0 ? (N + 127) / 128 : (N + 63) / 64;
+  return linear_shape(M, N, K, &turns) == 0 ? (N + 127) / 128 : (N + 63) / 64;
 }
 
 // mode: LN_GATE: W = [gates | ups], y [M, N / 2] = silu(x gates^T) (x ups^T);
@@ -867,6 +998,12 @@ void launch_linear(unsigned short* y, const unsigned short* x,
                    const unsigned short* w, const unsigned short* bias, int M,
                    int N, int K, long x_stride, int kind, int mode,
                    const LinearEnds& ends, hipStream_t stream) {
+  if (kind == 3 && mode == 0 && bias == nullptr) {
+    const int tn = (N + 63) / 64, tm = (M + 63) / 64;
+    hipLaunchKernelGGL(linear_square_kernel, dim3((unsigned)(tn * tm)), dim3(256),
+                       0, stream, y, x, w, M, N, K, x_stride, tn);
+    return;
+  }
   if (kind != 1 && kind != 2) throw std::invalid_argument("linear: kernels");
 #define LN_MODE(MODE)                                                          \
   case MODE:                                                                   \

@@ -112,9 +112,9 @@ def test_prefill_edges(dim, lens, ctx, kv_heads, per):
     ([60, 850], [4500, 0], -1.0),                   # over 64 tiles of keys
     ([13] * 70, [2100] + [3] * 69, 1.0),            # more than 64 sequences
 ])
-def test_prefill_many_tiles(lens, ctx, sign):
+def test_prefill_many_tiles(lens, ctx, sign, kv_heads=16, per=8):
     """Calls of two turns of workgroups and 2048 keys and more."""
-    kv_heads, per, dim = 16, 8, 128
+    dim = 128
     rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(lens))
     heads, scale = kv_heads * per, sign * dim ** -0.5
     cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)))
@@ -129,6 +129,18 @@ def test_prefill_many_tiles(lens, ctx, sign):
     q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
     check(got, *want(q, k, v, table, lens, ctx, scale))
     assert (wide[:, heads * dim:] == 7.0).all()
+
+
+@pytest.mark.parametrize("lens,ctx,kv_heads,per,sign", [
+    ([900, 1, 257, 32, 0, 433], [0, 2300, 17, 5, 9, 100], 16, 8, 1.0),  # row tiles
+    ([700, 333], [0, 2100], 15, 7, 1.0),            # tokens on both sides of a wave's
+    ([600, 500], [1500, 0], 32, 3, -1.0),
+    ([1100], [950], 88, 1, 0.0),                    # equal weights
+    ([260] * 65 + [300], [0] * 65 + [1800], 4, 2, 1.0),   # more than 64 sequences
+])
+def test_prefill_long_chains(lens, ctx, kv_heads, per, sign):
+    """Few sequences of many tokens, and many of some: eight waves in turn."""
+    test_prefill_many_tiles(lens, ctx, sign, kv_heads, per)
 
 
 @pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [

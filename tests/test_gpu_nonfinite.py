@@ -69,6 +69,26 @@ def test_paged(entry, dim, how, where, bad):
 
 
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("dim,lens,ctx,kv_heads,per", [
+    (128, [9, 33], [40, 170], 2, 4), (64, [9, 33], [40, 170], 2, 4),
+    (128, [610, 500], [40, 1600], 32, 3)])
+def test_prompts(dim, lens, ctx, kv_heads, per, where, bad):
+    """Waves that share the keys of few rows, and eight of long prompts in turn."""
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, 7)
+    plant(bad, where, rows, k, v, table, dim)
+    heads, scale = kv_heads * per, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0))).int().cuda()
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)]).int().cuda()
+    dev = [t.cuda() for t in (k, v, table)]
+    ref, _ = want(q, k, v, table, lens, ctx, scale)
+    agree(ops.paged_attn_prefill(
+        rows.cuda()[:, :heads * dim].unflatten(-1, (heads, dim)), *dev, cu, sl,
+        scale), ref)
+
+
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
 @pytest.mark.parametrize("where", ["q", "k"])
 @pytest.mark.parametrize("how", ["whole", "split"])
 @pytest.mark.parametrize("dim", [64, 128, 96])

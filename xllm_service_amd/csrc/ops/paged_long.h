@@ -384,11 +384,15 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
 // 4 x 1.6-2.3 k over up to 3.1 k 352 | 326, 4200 and 100 behind 3000 205 | 161, 3000 and 2000
 // behind 3000 228 | 218, 7 x 500 and 2100 86 | 82; 4000, 4 x 7 heads 136 | 121 (440); but
 // 1024 behind 1024 50 | 56 (136), 2500 71.5 | 74 (320), 5500, 4 x 4 heads 142 | 148 (344),
-// 8 x 512 44.7 | 45.4 and 2000, 2500 113 | 115 (576).
+// 8 x 512 44.7 | 45.4 and 2000, 2500 109 | 112 (576). Not many short prompts beside a long
+// one, 2200 and 20 x 100 65 | 68.5 (688), 40 x 100 behind 2000 207 | 217 (816), nor, of
+// more than four turns, short ones at all: with eight query heads to each 7 x 500 and 2100
+// 143 | 160 (1464), but 4096 294 | 284 (1032), 2000, 1300, 20 177 | 164 (848).
 inline bool paged_long_takes(long tokens, int n_seqs, int G, int n_kv,
                              long max_blocks) {
-  return paged_rows_tiles<PL_ROWS>(tokens, n_seqs, G) * n_kv >= 440 &&
-         max_blocks * PF_BS >= 2048;
+  const long wgs = paged_rows_tiles<PL_ROWS>(tokens, n_seqs, G) * n_kv;
+  return wgs >= 440 && max_blocks * PF_BS >= 2048 && tokens >= 256L * n_seqs &&
+         (wgs <= 1100 || tokens >= 1024L * n_seqs);
 }
 
 inline void paged_long(unsigned short* out, const unsigned short* q,

@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("keys", [[1, 15, 16, 17, 31, 32, 33, 64, 65, 100],
                                   [2100, 5], [300] * 40,
                                   [90] * 90 + [1500],
-                                  [200, 40] * 44 + [1000]])
+                                  [200, 40] * 44 + [1000],
+                                  [500, 30] * 12 + [1100]])
 def test_decode_edges(tail, heads, window, keys):
     g = torch.Generator().manual_seed(tail + heads + window + len(keys))
     W, r, scale = 512 + tail, 512, 192 ** -0.5

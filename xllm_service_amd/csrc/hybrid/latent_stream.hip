@@ -127,6 +127,12 @@ XLLM_DEV f32x4 ls_mma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// Parts of a sequence of n tiles: one for every `per` of them, or of up to `few` one for
+// every two
+XLLM_DEV int ls_own(int n, int n_part, int per, int few) {
+  return max(paged_parts(n, n_part, per), paged_parts(n, min(n_part, few), 2));
+}
+
 template <int W>
 __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
     float* __restrict__ out,               // [S, H, 512] (n_part == 1)
@@ -135,7 +141,8 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
     const unsigned short* __restrict__ q,  // [S, H, W]
     const unsigned short* __restrict__ cache,   // [blocks, 16, W]
     const int* __restrict__ block_tables, const int* __restrict__ seq_lens,
-    int heads, int table_width, float scale, int n_part, int per, int window) {
+    int heads, int table_width, float scale, int n_part, int per, int few,
+    int window) {
   constexpr int CPR = W / 8;                     // 16 B chunks of a row
   constexpr int IPP = 16 * CPR / 64;             // load instructions per page
   constexpr int NI = 2 * IPP / 4;                // ... of a wave per tile
@@ -154,7 +161,7 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
   const int n_tiles = (seq_len + LS_KT - 1) / LS_KT;
   const int lo = window > 0 ? max(0, seq_len - window) : 0;
   const int t_first = lo / LS_KT;
-  const int parts = paged_parts(n_tiles - t_first, n_part, per);
+  const int parts = ls_own(n_tiles - t_first, n_part, per, few);
   if (part >= parts) return;
   const int tpp = (n_tiles - t_first + parts - 1) / parts;
   const int t_begin = t_first + part * tpp;
@@ -361,15 +368,15 @@ __global__ void __launch_bounds__(256, 2) latent_stream_kernel(
 // workgroup per row, four columns per lane
 __global__ void __launch_bounds__(256) latent_stream_merge_kernel(
     float* __restrict__ out, const float* __restrict__ ws_o,
-    const float* __restrict__ ws_ml, int n_part, int per, long rows, int heads,
-    const int* __restrict__ seq_lens, int window) {
+    const float* __restrict__ ws_ml, int n_part, int per, int few, long rows,
+    int heads, const int* __restrict__ seq_lens, int window) {
   const long row = blockIdx.x * 2L + (threadIdx.x >> 7);
   const int col = (threadIdx.x & 127) * 4;
   if (row >= rows) return;
   const int len = seq_lens[row / heads];
-  const int parts = paged_parts(
+  const int parts = ls_own(
       (len + LS_KT - 1) / LS_KT -
-          (window > 0 ? max(0, len - window) / LS_KT : 0), n_part, per);
+          (window > 0 ? max(0, len - window) / LS_KT : 0), n_part, per, few);
   if (parts == 1) return;                        // written where it belongs
   float M = -INFINITY, L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   paged_add_parts<8>(reinterpret_cast<const float2*>(ws_ml) + row * n_part,
@@ -383,26 +390,31 @@ bool latent_stream_takes(int W, int r, int heads, int block_size) {
   return r == LS_R && (W == 512 || W == 576) && heads <= 32 && block_size == 16;
 }
 
-// Room for parts from what the host knows, one part for every `per` tiles of a
-// sequence's own in the kernel. Few workgroups: one per CU, parts of at least two
+// Room for parts from what the host knows; how many there are follows a sequence's own
+// length in the kernel (ls_own). Few workgroups: one per CU, parts of at least two
 // tiles. Measured (us, by parts): 1 x 700 keys, 16 heads 16 (4), 12 (8); 8 x 4000 35
-// (8), 23 (16), 20 (32); 16 x 2000 18.5 (16), 20.3 (32). More, up to where a part is a
-// long chain: one turn of two per CU, 24 x 2000 22.8 (10), 22.3 (21), 24 x 0.1-6 k 34.8
-// (10), 29.1 (21), 32 x 700 15.7 (8), 16.0 (16), 32 x 2000 24.8 (8), 23.8 (16), 32 x 0.1-6 k
-// 40.9 (8), 33.0 (16), 43 x 1500 28 (5), 25 (10), 43 x 0.1-6 k 62 (5), 42 (10), 64 x 1000
-// 25 (4), 24 (8), 64 x 0.1-6 k 78 (4), 55 (8). Still more in short tables the same: 90 x 600 33 (parts of 16 tiles), 23 (of 4), 128 x 0.1-0.9 k 35, 27. In
-// long ones parts of 16 tiles, so that a long sequence among short ones is no chain that
-// outlasts the rest: 90 x 0.1-6 k 74 (6), 84 (5, of 4 tiles), 300 x 0.1-4 k 188 (2), 210
-// (1).
-struct LsParts { long room, per; };
+// (8), 23 (16), 20 (32); 16 x 2000 18.5 (16), 20.3 (32). More, where a part is a long
+// chain: parts of four tiles up to one turn of two workgroups per CU, 24 x 2000 22.8
+// (10), 22.3 (21), 24 x 0.1-6 k 34.8 (10), 29.1 (21), 32 x 2000 24.8 (8), 23.8 (16), 32 x
+// 0.1-6 k 40.9 (8), 33.0 (16), 43 x 1500 28 (5), 25 (10), 43 x 0.1-6 k 62 (5), 42 (10), 64
+// x 1000 25 (4), 24 (8), 64 x 0.1-6 k 78 (4), 55 (8); and what one per CU leaves room for of
+// two: 24 x 500 15.8 (8), 17.7 (4), 32 x 1000 18.6 (8), 19.3 (16). Still more in tables of
+// 512 to 1024 keys the same: 90 x 600 33 (parts of 16 tiles), 23 (of 4), 128 x 0.1-0.9 k
+// 35, 27, but 256 x 300 26.5, 32. Else parts of 16 tiles, so that a long sequence among
+// short ones is no chain that outlasts the rest: 90 x 0.1-6 k 74 (6), 84 (5, of 4 tiles),
+// 300 x 0.1-4 k 188 (2), 210 (1).
+struct LsParts { long room, per, few; };
 static LsParts ls_parts(long wgs, long table_width, int window) {
   long tiles = (table_width + 1) / 2;
   if (window > 0) tiles = std::min<long>(tiles, window / LS_KT + 2);
   LsParts x;
-  if (wgs < 24) x = {256 / wgs, 2};
-  else if (wgs < 86 || (wgs <= 256 && tiles <= 32)) x = {512 / wgs, 4};
-  else x = {(512 + wgs - 1) / wgs, 16};
-  x.room = std::min<long>({x.room, (tiles + x.per - 1) / x.per, 32});
+  if (wgs < 24) x = {256 / wgs, 2, 0};
+  else if (wgs < 86) x = {512 / wgs, 4, 256 / wgs};
+  else if (wgs <= 256 && tiles > 16 && tiles <= 32) x = {512 / wgs, 4, 0};
+  else x = {(512 + wgs - 1) / wgs, 16, 0};
+  const long most = std::max((tiles + x.per - 1) / x.per,
+                             std::min(x.few, (tiles + 1) / 2));
+  x.room = std::min<long>({x.room, most, 32});
   return x;
 }
 static long ls_wgs(int n_seqs, int heads) {
@@ -420,17 +432,17 @@ void launch_latent_stream(float* out, float* ws_o, float* ws_ml,
                           float scale, int n_part, int window, hipStream_t st) {
   if (n_seqs == 0) return;
   const dim3 grid(n_seqs * n_part, (heads + 15) / 16);
-  const int per =
-      (int)ls_parts(ls_wgs(n_seqs, heads), table_width, window).per;
+  const LsParts p = ls_parts(ls_wgs(n_seqs, heads), table_width, window);
   auto k = W == 512 ? latent_stream_kernel<512> : latent_stream_kernel<576>;
   hipLaunchKernelGGL(k, grid, dim3(256), 0, st, out, ws_o, ws_ml, q, cache,
                      block_tables, seq_lens, heads, table_width, scale, n_part,
-                     per, window);
+                     (int)p.per, (int)p.few, window);
   if (n_part > 1) {
     const long rows = (long)n_seqs * heads;
     hipLaunchKernelGGL(latent_stream_merge_kernel,
                        dim3((unsigned)((rows + 1) / 2)), dim3(256), 0, st, out,
-                       ws_o, ws_ml, n_part, per, rows, heads, seq_lens, window);
+                       ws_o, ws_ml, n_part, (int)p.per, (int)p.few, rows, heads,
+                       seq_lens, window);
   }
 }
 

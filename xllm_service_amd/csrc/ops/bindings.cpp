@@ -60,7 +60,7 @@ int skinny_gemm_rows(int M);
 void launch_skinny_gemm(unsigned short*, const unsigned short*,
                         const unsigned short*, const unsigned short*, float*,
                         int, int, int, hipStream_t);
-int linear_takes(long M, long N, long K, bool bias);
+int linear_takes(long M, long N, long K, bool bias, bool ends);
 int linear_tiles(int M, int N, int K, int kind);
 void launch_linear(unsigned short*, const unsigned short*,
                    const unsigned short*, const unsigned short*, int, int, int,
@@ -404,9 +404,10 @@ static bool tuned(long M, long N, long K, long x_stride) {
          entry != at::cuda::tunable::ResultEntry::Default();
 }
 
-// Which kernels of linear.hip take x @ w^T (+ bias): linear_takes, 0 for none
+// Which kernels of linear.hip take x @ w^T (+ bias), with LinearEnds' options or
+// without: linear_takes, 0 for none
 static int linear_kind(const torch::Tensor& x, const torch::Tensor& w,
-                       const c10::optional<torch::Tensor>& bias) {
+                       const c10::optional<torch::Tensor>& bias, bool ends) {
   auto rows16 = [](const torch::Tensor& t) {
     return t.dim() == 2 && t.is_cuda() && t.dtype() == torch::kBFloat16 &&
            t.stride(1) == 1 &&
@@ -423,21 +424,18 @@ static int linear_kind(const torch::Tensor& x, const torch::Tensor& w,
           bias->device() == w.device()))))
     return 0;
   const long M = x.size(0), N = w.size(0), K = w.size(1);
-  const int kind = xllm::linear_takes(M, N, K, bias.has_value());
+  const int kind = xllm::linear_takes(M, N, K, bias.has_value(), ends);
   return kind != 0 && M > (N > 8192 ? 32 : 48) && !bias.has_value() &&
                  tuned(M, N, K, x.stride(0))
              ? 0
              : kind;
 }
 
-// Kernels that do more than the product (LinearEnds)
-static bool has_ends(int kind) { return kind == 1 || kind == 2; }
-
 // x [..., K] @ w [N, K]^T (+ bias): the kernels of linear.hip where they take the
 // call, the library elsewhere (and wherever a gradient is wanted)
 torch::Tensor linear(torch::Tensor x, torch::Tensor w,
                      c10::optional<torch::Tensor> bias) {
-  if (const int kind = linear_kind(x, w, bias)) {
+  if (const int kind = linear_kind(x, w, bias, false)) {
     const long M = x.size(0), N = w.size(0), K = w.size(1);
     c10::OptionalDeviceGuard guard(x.device());
     auto y = torch::empty({M, N}, x.options());
@@ -455,7 +453,7 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor w,
 torch::Tensor linear_gated(torch::Tensor x, torch::Tensor w,
                            c10::optional<torch::Tensor> bias) {
   if (!bias.has_value() && w.dim() == 2 && w.size(0) % 16 == 0) {
-    if (const int kind = linear_kind(x, w, bias); has_ends(kind)) {
+    if (const int kind = linear_kind(x, w, bias, true)) {
       const long M = x.size(0), N = w.size(0), K = w.size(1);
       c10::OptionalDeviceGuard guard(x.device());
       auto y = torch::empty({M, N / 2}, x.options());
@@ -511,9 +509,9 @@ static Rows product_normed(const torch::Tensor& x, const torch::Tensor& w,
                            const c10::optional<torch::Tensor>& next_bias,
                            bool next_gate, double eps) {
   const c10::optional<torch::Tensor> none;
-  const int kind = linear_kind(x, w, none);
+  const int kind = linear_kind(x, w, none, true);
   const long M = x.size(0), N = w.size(0), K = w.size(1);
-  if (has_ends(kind) && res.dim() == 2 && res.is_contiguous() && res.size(0) == M &&
+  if (kind != 0 && res.dim() == 2 && res.is_contiguous() && res.size(0) == M &&
       res.size(1) == N && res.dtype() == torch::kBFloat16 && on_bytes(res, 16) &&
       norm.dim() == 1 && norm.size(0) == N && norm.is_contiguous() &&
       norm.dtype() == torch::kBFloat16 &&
@@ -521,10 +519,10 @@ static Rows product_normed(const torch::Tensor& x, const torch::Tensor& w,
       res.is_cuda() && norm.is_cuda() &&
       !(next_gate && (next_bias.has_value() || next_w.size(0) % 16 != 0))) {
     Rows out{torch::empty({M, N}, x.options())};
-    const int next = linear_kind(out.x, next_w, next_bias);
+    const int next = linear_kind(out.x, next_w, next_bias, true);
     const int tiles = xllm::linear_tiles((int)M, (int)N, (int)K, kind);
     out.kind = next;
-    if (has_ends(next) && tiles % 4 == 0 && tiles <= (next == 1 ? 256 : 64)) {
+    if (next != 0 && tiles % 4 == 0 && tiles <= (next == 1 ? 256 : 64)) {
       out.squares = torch::empty({M, tiles}, x.options().dtype(torch::kFloat));
       xllm::LinearEnds e;
       e.residual = reinterpret_cast<unsigned short*>(res.data_ptr());

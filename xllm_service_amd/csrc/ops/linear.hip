@@ -827,7 +827,9 @@ static int linear_shape(long M, long N, long K, long* turns) {
   return best;
 }
 
-int linear_takes(long M, long N, long K, bool bias) {
+// ends: LinearEnds' options are wanted, which save a launch of 2.5 to 5 us. Then products
+// are taken too that the library is faster at by as much: 1, 2
+int linear_takes(long M, long N, long K, bool bias, bool ends) {
   if (M <= 0 || K < LN_K || K % LN_K != 0 || N % 8 != 0) return 0;
   if (N * K >= (1L << 31) || M * K >= (1L << 30)) return 0;
   if (M <= 16) return M <= 8 || N * K <= 1L << 28 ? 1 : 0;
@@ -843,6 +845,7 @@ int linear_takes(long M, long N, long K, bool bias) {
   if (M <= 32) {
     if (N <= 8192)
       return N > 1024 || K <= 8192 || !split || M > 24 || N <= 256 ? 1 : 0;
+    if (ends) return K <= 4096 && N * K <= 1L << 28 ? 1 : 0;
     if (K <= 2048) return N <= 32768 ? 1 : 0;
     return K <= 4096 && (M <= 24 ? N >= 14336 && N * K <= 1L << 28
                                  : N >= 16384 && K > 3072 && N * K <= 1L << 27) ? 1 : 0;
@@ -851,6 +854,8 @@ int linear_takes(long M, long N, long K, bool bias) {
   // 4096 53.1 | 48.3 (M 48 55.4 | 58.5), 50272 x 768 23.7 | 21.7, 18944 x 3584 36.7 | 33.9
   if (M <= 48) {
     if (N <= 8192) return N > 2048 || !split || (N >= 1536 && K < 8192) ? 1 : 0;
+    if (ends)
+      return N * K <= 1L << 28 && (K <= 2048 || (K <= 4096 && N >= 18432)) ? 1 : 0;
     return (K <= 2048 && N <= 16384) || (K <= 1024 && N <= 32768) ? 1 : 0;
   }
   if (M <= 64) {
@@ -865,17 +870,17 @@ int linear_takes(long M, long N, long K, bool bias) {
   const long squares = (M + 63) / 64 * ((N + 63) / 64);
   // Up to two turns of square tiles where none of the others takes one, or has tiles
   // of 128 rows: library | square, 126 x 8448 x 640 11.1 | 7.9, 160 x 9856 x 1536 19.8 | 17.3,
-  // 300 x 4864 x 1024 13.9 | 9.9, 256 x 6912 x 1536 20.8 | 14.9, 689 x 2688 x 1920 20.5 | 17;
-  // at 2048 no longer, 512 x 3072 x 2048 15.3 | 16.4, but 160 x 8448 x 2048 24.2 | 19.8
-  if (squares > 256 && squares <= 512 &&
-      K <= (shape == 0 || turns > 1 ? (N <= 8192 ? 1920 : 2048) : 512))
+  // 300 x 4864 x 1024 13.9 | 9.9, 256 x 6912 x 1536 20.8 | 14.9, 689 x 2688 x 1920 20.5 | 17,
+  // 160 x 8448 x 2048 24.2 | 19.8, 512 x 3072 x 2048 15.3 | 16.4
+  if (!ends && squares > 256 && squares <= 512 &&
+      K <= (shape == 0 || turns > 1 ? 2048 : 512))
     return 3;
   if (turns > 1 || (M > 2048 && N > 128 && K > 1024)) return 0;
   if (N > 8192 && (N > 16384 || K > 2048 || shape == 0)) return 0;
-  // 128 rows of W a tile, the library has as large ones from 257 rows on: M 512, 3072 x
-  // 2048 17 | 15.3, 3584 x 3584 27.6 | 25.8, M 300, 4608 x 3584 26.9 | 23.8; but M 256, 6144 x
+  // 128 rows of W a tile, the library has as large ones from 257 rows on: M 512, 3584 x
+  // 3584 27.6 | 25.8, M 300, 4608 x 3584 26.9 | 23.8; but M 256, 6144 x
   // 4096 31.1 | 40.3, and short rows, M 512, 4096 x 1024 10.9 | 13.1
-  if (shape == 0 && M > 256 && K > 1536) return 0;
+  if (!ends && shape == 0 && M > 256 && K > 1536) return 0;
   // M 80: 4096 x 14336 48.8 | 43.1, 4096 x 11008 40.9 | 35, 3584 x 8192 27.9 | 25.4 and at
   // M 76 47.3 | 49.2, 39.6 | 40.7, 27 | 28.1; 3584 x 18944 61 | 130
   if (K > 4096)
@@ -913,9 +918,9 @@ static bool linear_one_tile(int M, int N, int K) {
 }
 // A workgroup that has a CU to itself takes all of its LDS: two tiles a wave, or
 // more waves. Where there are more than CUs, two of them share one: M 24, 32000 x
-// 4096 48.4, with two tiles 49.2; 18944 x 4096 33.4 | 34.5. Up to 16 rows, and up to 32 of
-// short rows of W, eight waves are up to 5% faster than four with two tiles each:
-// M 10, 768 x 3072 4.2 -> 4.1, M 32, 2560 x 2560 7.3 -> 6.9, but 4096 x 4096 10.4 | 10.5.
+// 4096 48.4, with two tiles 49.2; 18944 x 4096 33.4 | 34.5. Of short rows eight waves with one
+// tile are faster: M 10, 8192 x 640 4.5 -> 4.4, M 32, 2560 x 2560 7.3 -> 6.9, but 4096 x 4096
+// 10.4 | 10.5.
 template <int MODE>
 static void launch_stream(unsigned short* y, const unsigned short* x,
                           const unsigned short* w, const unsigned short* bias,
@@ -927,17 +932,16 @@ static void launch_stream(unsigned short* y, const unsigned short* x,
   const dim3 grid((n_out + out - 1) / out);
   const bool few = grid.x <= 256;
   // Workgroup b starts at step b mod steps, which its product with 2^32 / steps holds in
-  // the upper bits; at the first one where a product is small (0): 10 rows, 768 x 768
-  // 2.9 us, with a division 3.0; 4096 x 4096 8.2, without turns 9.1.
+  // the upper bits: 10 rows, 768 x 768 2.9 us, with a division 3.0; 4096 x 4096 8.2, all
+  // at the first step 9.1.
   const int steps = K / LN_K;
-  const unsigned turns =
-      (long)N * K < 1L << 23 ? 0u : (unsigned)(((1L << 32) + steps - 1) / steps);
+  const unsigned turns = (unsigned)(((1L << 32) + steps - 1) / steps);
 #define LN_STREAM(NT, XR, NW, D)                                               \
   hipLaunchKernelGGL((linear_stream_kernel<NT, XR, NW, D, MODE>), grid,        \
                      dim3(NW * 64), 0, stream, y, x, w, bias, M, N, K,         \
                      x_stride, turns, ends)
   if (one) {
-    const bool eight = few || K <= 1536;
+    const bool eight = !few && K <= 1536;        // many workgroups of short rows
     if (M <= 8) { if (eight) LN_STREAM(1, 8, 8, 1); else LN_STREAM(1, 8, 4, 2); }
     else if (M <= 16) { if (eight) LN_STREAM(1, 16, 8, 1); else LN_STREAM(1, 16, 4, 2); }
     else if (M <= 24) LN_STREAM(1, 24, 4, 2);

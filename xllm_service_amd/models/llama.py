@@ -32,14 +32,14 @@ _EVERY_HOOK = (module_hooks._global_forward_hooks,
 
 
 def _plain(module, kind):
-    """A module of this very class that nothing observes or replaces: what its call
-    would do besides its forward is nothing."""
-    return (type(module) is kind
-            and not (module._forward_hooks or module._forward_pre_hooks
-                     or module._backward_hooks or module._backward_pre_hooks
-                     or any(_EVERY_HOOK))
-            and module._compiled_call_impl is None
-            and "forward" not in module.__dict__)
+    """A module of this very class that nothing observes or replaces: without a hook
+    of all modules, its call would do nothing besides its forward."""
+    if type(module) is not kind:
+        return False
+    d = module.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"]
+                or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                or d.get("_compiled_call_impl") or "forward" in d)
 
 
 class LlamaAttention(nn.Module):
@@ -107,7 +107,8 @@ class LlamaMLP(nn.Module):
 
     def forward(self, x):
         g = self.gate_up
-        if _plain(g, MergedColumnParallelLinear) and not g.use_skinny:
+        if not any(_EVERY_HOOK) and _plain(g, MergedColumnParallelLinear) \
+                and not g.use_skinny:
             return self.down(ops.linear_gated(x, g.weight, g.bias))
         return self.down(ops.silu_and_mul(g(x)))
 
@@ -163,7 +164,8 @@ def _native_layers(layers, x, residual, positions, kv_caches, meta, cos_sin):
     """Layers as one native call, or None where one of their modules is not the
     plain one or torch has to see the calls: gradients, modes, tracing."""
     if not (x.is_cuda and ops.HAS_EXT and torch.is_inference_mode_enabled()
-            and ps.tp_size() == 1) or torch.compiler.is_compiling() \
+            and ps.tp_size() == 1) or any(_EVERY_HOOK) \
+            or torch.compiler.is_compiling() \
             or torch.overrides.has_torch_function((x, residual)):
         return None
     weights = []
@@ -172,13 +174,13 @@ def _native_layers(layers, x, residual, positions, kv_caches, meta, cos_sin):
         if w is None:
             return None
         weights.append(w)
-    first = layers[0]
-    attn = first.attn
 
     def settings(layer):
-        a = layer.attn
+        a = layer._modules["attn"]
         return layer.eps, a.n_heads, a.n_kv_heads, a.scale, a.mrope_sections
-    if any(settings(layer) != settings(first) for layer in layers):
+    first = layers[0]
+    attn, shared = first._modules["attn"], settings(first)
+    if any(settings(layer) != shared for layer in layers):
         return None
     ms0 = ms1 = 0
     if attn.mrope_sections and positions.dim() != 1:

@@ -27,7 +27,7 @@
 // pieces of 32 B) that share an LDS cycle fall on different banks.
 //
 // Measured, 32 sequences of 1.5-2.5 k keys, 16 heads, rows of 576: 67 + 5 us before,
-// 23.6 us with the merge now (25.6 when every wave made all scores, and read all of a
+// 23.5 us with the merge now (25.6 when every wave made all scores, and read all of a
 // tile for them); the rows alone take 15 us at the rate of a large copy. Bound by a tile's
 // chain of LDS reads, products and weights, 1.7 us for 36 KB: more tiles on their way
 // (four buffers) did not help, nor did two teams of waves with tiles of their own in a

@@ -772,8 +772,8 @@ __global__ __launch_bounds__(256, 2) void linear_square_kernel(
 }
 
 // 0: the library's; 1: stream; 2: tiles; 3: square ones, without LinearEnds' options.
-// Besides its time on the GPU a library
-// call costs 28 us of host time (its choice of a kernel), these cost 6.
+// Besides its time on the GPU a library call costs 28 us of host time (its choice of a
+// kernel), these cost 6.
 // Measured, us on the GPU, here | library, weights from memory (N x K):
 //   M 8      2048 x 2048 4.1 | 8.9, 4096 x 4096 7.7 | 15.3, 4096 x 14336 21 | 25, 28672 x
 //            4096 39 | 60, 32000 x 4096 44 | 57

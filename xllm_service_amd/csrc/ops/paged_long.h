@@ -3,8 +3,8 @@
 //
 // Rows, tiles, products and LDS images are those of paged_rows.h. There each wave
 // does a tile's products and then its weights, and what the two waves of a SIMD overlap
-// is left to chance: 2130 cycles a tile and wave where products take 1024 and weights
-// 1180. Here a workgroup has eight waves and 256 rows, two waves to a SIMD, which
+// is left to chance: 2610 cycles a tile and wave, a whole call's by counters, of which
+// the matrix pipe works 1024 and the vector unit 1130. Here a workgroup has eight waves and 256 rows, two waves to a SIMD, which
 // take turns: while waves 0-3 multiply (weights of the last tile by its values, keys of
 // this one by the queries, 32 products without a pause), waves 4-7 make weights of
 // their scores, then the other way round, a barrier between two half steps. Operands of
@@ -13,8 +13,9 @@
 // share of a step is one page, whose address three v_readlane fetch from a table of 64
 // tiles made at once: by scalar arithmetic on the way a step's loads cost 700 cycles.
 //
-// Bound by the weights: 1500 cycles, the products 1600. 4 prompts of 1.6-2.3 k tokens
-// over up to 3.1 k cached ones, 32 heads of 128: 354 -> 326 us. What it costs is one
+// Bound by both in turn: 2210 cycles, the pipe 1024, the vector unit 1240 of them. 4
+// prompts of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads of 128: 353 -> 335
+// us. What it costs is one
 // workgroup per CU: nothing covers its start and its end, so it is taken for several
 // turns of workgroups with long chains only (paged_long_takes).
 #pragma once

@@ -39,7 +39,7 @@
 // instructions to the compiler, every use of an LDS read waited for all reads in
 // flight, and the first transpose read for the next tile too. With that and
 // three steps of K on the way ahead of their products, before -> after: 4 prompts
-// of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads 366 -> 354 us,
+// of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads 366 -> 353 us,
 // 3 chunks of 93-261 tokens over 0.5-1.8 k, 28 heads, keys split 30.9 -> 30.1, 2
 // of 1.8-2.3 k in a window of 1024, three terms 63.3 -> 61.3, 8 prompts of 109-438,
 // 12 heads of 64 13.6. (One head and 16 rows per wave on 16x16x32 products, P

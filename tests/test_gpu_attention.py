@@ -132,11 +132,16 @@ def test_prefill_many_tiles(lens, ctx, sign, kv_heads=16, per=8):
 
 
 @pytest.mark.parametrize("lens,ctx,kv_heads,per,sign", [
-    ([900, 1, 257, 32, 0, 433], [0, 2300, 17, 5, 9, 100], 16, 8, 1.0),  # row tiles
+    ([900, 1, 257, 32, 0, 433], [0, 2300, 17, 5, 9, 100], 16, 8, 1.0),
+    ([900, 1, 257, 32, 0, 433], [0, 3100, 17, 5, 9, 100], 16, 8, 1.0),  # row tiles
     ([700, 333], [0, 2100], 15, 7, 1.0),            # tokens on both sides of a wave's
     ([600, 500], [1500, 0], 32, 3, -1.0),
     ([1100], [950], 88, 1, 0.0),                    # equal weights
-    ([260] * 65 + [300], [0] * 65 + [1800], 4, 2, 1.0),   # more than 64 sequences
+    ([260] * 65 + [300], [0] * 65 + [1800], 4, 2, 1.0),
+    ([260] * 65 + [300], [0] * 65 + [2800], 4, 2, 1.0),   # more than 64 sequences
+    ([1150], [2100], 18, 8, 1.0),                   # before and behind the lines of the
+    ([1150], [2100], 14, 8, 1.0),                   # rule: 648, 504
+    ([1150], [1900], 18, 8, -1.0),                  # and 3072 keys
 ])
 def test_prefill_long_chains(lens, ctx, kv_heads, per, sign):
     """Few sequences of many tokens, and many of some: eight waves in turn."""
@@ -173,7 +178,8 @@ def test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign):
 @pytest.mark.parametrize("lens,keys,kv_heads,per", [
     ([40, 7], [130, 0], 2, 2),                       # waves that share the keys
     ([300, 50, 9], [60, 0, 300], 16, 8),             # whole chains
-    ([900, 300, 5], [450, 0, 2300], 16, 8),          # eight waves in turn
+    ([900, 300, 5], [450, 0, 2300], 16, 8),
+    ([900, 300, 5], [450, 0, 2300], 13, 8),          # eight waves in turn
 ])
 def test_prefill_rows_without_keys(dim, lens, keys, kv_heads, per):
     """More new tokens than keys, or no keys at all: rows in front of the first key

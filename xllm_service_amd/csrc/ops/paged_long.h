@@ -4,20 +4,20 @@
 // Rows, tiles, products and LDS images are those of paged_rows.h. There each wave
 // does a tile's products and then its weights, and what the two waves of a SIMD overlap
 // is left to chance: 2610 cycles a tile and wave, a whole call's by counters, of which
-// the matrix pipe works 1024 and the vector unit 1130. Here a workgroup has eight waves and 256 rows, two waves to a SIMD, which
-// take turns: while waves 0-3 multiply (weights of the last tile by its values, keys of
-// this one by the queries, 32 products without a pause), waves 4-7 make weights of
-// their scores, then the other way round, a barrier between two half steps. Operands of
-// the next four products are read from LDS during each four, the first ones before
-// the barrier. Four tiles of K and V in LDS: loads have two steps to arrive. A wave's
-// share of a step is one page, whose address three v_readlane fetch from a table of 64
-// tiles made at once: by scalar arithmetic on the way a step's loads cost 700 cycles.
+// the matrix pipe works 1024 and the vector unit 1130. Here a workgroup has eight waves
+// and 256 rows, two waves to a SIMD, which take turns: while waves 0-3 multiply (weights
+// of the last tile by its values, keys of this one by the queries, 32 products without a
+// pause), waves 4-7 make weights of their scores, then the other way round, a barrier
+// between two half steps. Operands of the next four products are read from LDS during
+// each four, the first ones before the barrier. Four tiles of K and V in LDS: loads have
+// two steps to arrive. A wave's share of a step is one page, whose address three
+// v_readlane fetch from a table of 64 tiles made at once: by scalar arithmetic on the way
+// a step's loads cost 700 cycles.
 //
 // Bound by both in turn: 2210 cycles, the pipe 1024, the vector unit 1240 of them. 4
 // prompts of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads of 128: 353 -> 335
-// us. What it costs is one
-// workgroup per CU: nothing covers its start and its end, so it is taken for several
-// turns of workgroups with long chains only (paged_long_takes).
+// us. What it costs is one workgroup per CU: nothing covers its start and its end, so it
+// is taken for whole turns of workgroups with long chains only (paged_long_takes).
 #pragma once
 #include "paged_rows.h"
 
@@ -379,21 +379,34 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
                        o_acc[dt][r + 2] * inv, o_acc[dt][r + 3] * inv);
 }
 
-// Two turns of workgroups, nearly, and chains of some length: the host knows the
-// width of the tables, not the lengths. Us, paged_rows.h | here, 8 key heads, four
-// query heads to each unless noted: 4096 new 159 | 143 (520 workgroups), 8192 543 | 508,
-// 4 x 1.6-2.3 k over up to 3.1 k 352 | 326, 4200 and 100 behind 3000 205 | 161, 3000 and 2000
-// behind 3000 228 | 218, 7 x 500 and 2100 86 | 82; 4000, 4 x 7 heads 136 | 121 (440); but
-// 1024 behind 1024 50 | 56 (136), 2500 71.5 | 74 (320), 5500, 4 x 4 heads 142 | 148 (344),
-// 8 x 512 44.7 | 45.4 and 2000, 2500 109 | 112 (576). Not many short prompts beside a long
-// one, 2200 and 20 x 100 65 | 68.5 (688), 40 x 100 behind 2000 207 | 217 (816), nor, of
-// more than four turns, short ones at all: with eight query heads to each 7 x 500 and 2100
-// 143 | 160 (1464), but 4096 294 | 284 (1032), 2000, 1300, 20 177 | 164 (848).
+// Workgroups that fill their turns, one to a CU: the host knows the width of the tables,
+// not the lengths, and counts as if sequences were equal. Us, paged_rows.h | here, by
+// query/key heads, workgroups in parentheses:
+//   nearly two turns   32/8: 4096 153 | 139 (512), 3760 133 | 120 (470), 3 x 1253 behind
+//            3132 246 | 225 (480); 64/8: 1880 behind 4700 348 | 321 (470); but fewer, 2500
+//            71.5 | 74 (320), 1024 behind 1024 50 | 56 (136)
+//   up to two and a half, a third turn for a few   32/8: 4128 behind 4128 453 | 467
+//            (516), 2 x 2064 behind 1444 184 | 202 (528), 3 x 1376 behind 3440 307 | 335
+//            (528); 64/8: 3 x 688 behind 1720 164 | 182 (528), 2064 85.7 | 87.9 (520);
+//            but 4200 and 100 behind 3000 205 | 161 (544), for the order of its chains
+//   more     32/8: 3 x 1866 behind 4665 512 | 481 (720), 5600 behind 14000 1484 | 1369
+//            (704); 64/8: 3 x 933 behind 2332 268 | 259 (720), but in tables of 2243 keys
+//            2 x 1320 behind 923 152 | 156 (672). One sequence with little before it has
+//            short chains for the last turn in both kernels: 64/8: 2800 141 | 149 (704),
+//            32/32: 5600 270 | 278 (704); but of 7200, 32/8, 414 | 398 (904)
+// Not many short prompts beside a long one, 2200 and 20 x 100 65 | 68.5 (688), 40 x 100
+// behind 2000 207 | 217 (816), nor, of more than four turns, short ones at all: with
+// eight query heads to each 7 x 500 and 2100 143 | 160 (1464), but 4096 294 | 284 (1032).
 inline bool paged_long_takes(long tokens, int n_seqs, int G, int n_kv,
                              long max_blocks) {
-  const long wgs = paged_rows_tiles<PL_ROWS>(tokens, n_seqs, G) * n_kv;
-  return wgs >= 440 && max_blocks * PF_BS >= 2048 && tokens >= 256L * n_seqs &&
-         (wgs <= 1100 || tokens >= 1024L * n_seqs);
+  const long keys = max_blocks * PF_BS, rows = tokens * G;
+  const long wgs = (rows + n_seqs * (long)PL_ROWS - 1) / (n_seqs * (long)PL_ROWS) *
+                   n_seqs * n_kv;
+  if (wgs < 440 || keys < 2048 || tokens < 256L * n_seqs) return false;
+  if (wgs <= 512) return true;
+  if (wgs <= 640 || keys < 3072) return false;
+  if (wgs > 1100 && tokens < 1024L * n_seqs) return false;
+  return n_seqs > 1 || 2 * keys >= 3 * tokens || keys >= 6144;
 }
 
 inline void paged_long(unsigned short* out, const unsigned short* q,

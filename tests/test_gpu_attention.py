@@ -155,6 +155,9 @@ def test_prefill_long_chains(lens, ctx, kv_heads, per, sign):
     (1, 5, 64, [40], [984], 1.0),                    # four turns of waves
     (1, 3, 128, [100, 5], [1948, 0], -1.0),          # eight
     (2, 1, 64, [3] * 70, [150] + [0] * 69, 1.0),     # more than 64 sequences
+    (1, 1, 128, [127], [1393], 1.0),                 # before 1536 keys
+    (1, 1, 128, [127], [1409], 1.0),                 # from there on too few rows
+    (1, 1, 128, [128], [1408], -1.0),                # and enough
 ])
 def test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign):
     """Waves of a workgroup that share out the keys of its rows."""

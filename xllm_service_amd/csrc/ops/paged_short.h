@@ -272,12 +272,16 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
 // tokens 6.3 | 7.0, 64 of 64-wide heads 5.4 | 6.1. Longer tables go to more
 // workgroups there: 32 tokens of 28/4 heads behind 1000 keys 18.5 | 15.9, 100 of 32/8
 // behind 1600 22.0 | 20.5, but 32 behind 3000 21.9 | 29.4; 16 of 64-wide heads behind
-// 1000 11.9 | 12.0.
+// 1000 11.9 | 12.0. From 1536 keys on, where there are three parts, only rows that fill
+// a tile: 17 of 32/32 heads behind 1400 21.3 | 19.2, behind 1600 18.1 | 21.2, 60 of them
+// 22.7 | 19.3, 19.8 | 21.3; 30 of 16/4 (120 rows) behind 1600 19.1 | 19.7, 45 behind 1930
+// 21.8 | 21.7.
 inline bool paged_short_takes(long tokens, int n_seqs, int G, int n_kv,
                               long max_blocks, int terms) {
+  const long keys = max_blocks * PF_BS;
   return paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv <= 256 &&
-         max_blocks * PF_BS >= 128 &&
-         max_blocks * PF_BS <= (terms > 1 ? PS_KEYS / 2 : PS_KEYS);
+         keys >= 128 && keys <= (terms > 1 ? PS_KEYS / 2 : PS_KEYS) &&
+         (keys < 1536 || tokens * G >= (long)PF_ROWS * n_seqs);
 }
 
 template <int D, int TERMS>

@@ -827,17 +827,13 @@ static int linear_shape(long M, long N, long K, long* turns) {
   return best;
 }
 
-// ends: LinearEnds' options are wanted, which save a launch of 2.5 to 5 us. Then products
-// are taken too that the library is faster at by as much: 1, 2
+// The choice (0 to 3, see above). ends: LinearEnds' options are wanted, which save a launch
+// of 2.5 to 5 us. Then products are taken too that the library is faster at by less than
+// that, and the answer is never 3.
 int linear_takes(long M, long N, long K, bool bias, bool ends) {
   if (M <= 0 || K < LN_K || K % LN_K != 0 || N % 8 != 0) return 0;
   if (N * K >= (1L << 31) || M * K >= (1L << 30)) return 0;
   if (M <= 16) return M <= 8 || N * K <= 1L << 28 ? 1 : 0;
-  // More than 8192 columns: x rows weigh more and more, and the last turn of the CUs
-  // counts. Here | library, M 20 | M 28-32: 50272 x 768 20.7 | 20, 21.6 | 20.4, 9216 x
-  // 4096 22.6 | 20.5, 24.1 | 21.4, 12288 x 4096 24.2 | 23.4, 25.6 | 24, 14336 x 4096 25.2 |
-  // 25.8, 27.2 | 26.3, 16384 x 4096 27.1 | 32.5, 28.5 | 32.6, 24576 x 3072 31.5 | 31.3, 33.2 |
-  // 31.5, 37888 x 3584 53.6 | 54.9, 57 | 55.7
   // The library splits long rows of whole 1024s over workgroups: few workgroups here
   // wait longer for theirs. Here | library, 512 x 8192 | 512 x 8448: M 24 8.2 | 8.1, 8.6 |
   // 17.7, M 40 10.9 | 7.9, 11.4 | 17.5, M 64 13.5 | 8.4, 14 | 17.8; M 32, 512 x 16384 18.4 | 19.2
@@ -846,6 +842,11 @@ int linear_takes(long M, long N, long K, bool bias, bool ends) {
     if (N <= 8192)
       return N > 1024 || K <= 8192 || !split || M > 24 || N <= 256 ? 1 : 0;
     if (ends) return K <= 4096 && N * K <= 1L << 28 ? 1 : 0;
+    // More than 8192 columns: x rows weigh more and more, and the last turn of the CUs
+    // counts. Here | library, M 20, M 28-32: 50272 x 768 20.7 | 20, 21.6 | 20.4; 9216 x 4096
+    // 22.6 | 20.5, 24.1 | 21.4; 12288 x 4096 24.2 | 23.4, 25.6 | 24; 14336 x 4096 25.2 | 25.8,
+    // 27.2 | 26.3; 16384 x 4096 27.1 | 32.5, 28.5 | 32.6; 24576 x 3072 31.5 | 31.3, 33.2 | 31.5;
+    // 37888 x 3584 53.6 | 54.9, 57 | 55.7
     if (K <= 2048) return N <= 32768 ? 1 : 0;
     return K <= 4096 && (M <= 24 ? N >= 14336 && N * K <= 1L << 28
                                  : N >= 16384 && K > 3072 && N * K <= 1L << 27) ? 1 : 0;
@@ -886,11 +887,17 @@ int linear_takes(long M, long N, long K, bool bias, bool ends) {
   if (K > 4096)
     return N >= 3072 && N <= 4608 && M <= 192 &&
            !(M > 76 && M <= 80 && N > 3072 && K <= 16384) ? 2 : 0;
+  // Fewer than 1024 columns in up to 32 tiles of 128 by 64, where the library steps to its
+  // next time: 512 x 3072, M 320 8.4 | 8.6; 768 x 3072, M 300 8.6 | 8.7, M 350 11.6 | 8.8;
+  // 768 x 4096, M 300 12.1 | 13.8, M 400 14.2 | 14.3, M 768 19.4 | 16.6; but 768 x 2560, M 300
+  // 9.6 | 8.3
+  if (!ends && K > 2560 && N < 1024 && (N + 127) / 128 * ((M + 63) / 64) <= 32)
+    return 0;
   // few tiles with long rows leave most of the chip waiting for their chain, many of
-  // them wait for each other: 256 x 4096, M 300 10 | 8.9, M 2048 16.2 | 13.8; M 1536, 640 x 2560
-  // 14.7 | 12.4, M 2048, 512 x 2048 13 | 10.8, 1024 x 4096 32.6 | 28.5
-  // 576 x 4096, M 300, 12.2 | 10.2, 832 x 3072, M 260, 11.1 | 8.7: where the tiles
-  // of W are no multiple of four, those that share one lie on several XCDs
+  // them wait for each other: 256 x 4096, M 300 10 | 8.9, M 2048 16.2 | 13.8; M 1536, 640 x
+  // 2560 14.7 | 12.4, M 2048, 512 x 2048 13 | 10.8, 1024 x 4096 32.6 | 28.5. Where the tiles of
+  // W are no multiple of four, those that share one lie on several XCDs: 576 x 4096, M 300,
+  // 12.2 | 10.2, 832 x 3072, M 260, 11.1 | 8.7
   if (K > 2048)
     return N >= 512 && (N >= 1024 || N % 256 == 0) && M <= 1024 &&
            !((N < 3072 && M <= 128) || (N < 2048 && M <= 256)) ? 2 : 0;

@@ -1,0 +1,261 @@
+// What the paged attention kernels (paged_rows.h, paged_stream.h) share: their
+// options, and the merge of keys that were split over workgroups.
+#pragma once
+#include <atomic>
+#include <random>
+
+#include "mfma_rows.h"
+
+namespace xllm {
+
+// Options of a call. A kernel instantiated without MORE ignores them: bf16
+// results, every earlier key seen, scores scale * q.k.
+struct PagedMore {
+  int window = 0;         // > 0: a row sees the last `window` keys ...
+  int keep_first = 0;     // ... and the first keep_first
+  int chunked = 0;        // `window` is a chunk size: a row sees its own chunk
+  int out_f32 = 0;        // results in fp32
+  float cap = 0.0f;       // > 0: scores become cap * tanh(score / cap)
+  const float* sink = nullptr;        // [heads]: e^sink joins the denominator
+  const float* head_scale = nullptr;  // [heads]: one more score multiplier
+};
+
+// first key that a row which sees keys below `limit` has in its window
+template <bool MORE>
+XLLM_DEV int paged_first(const PagedMore& x, int limit) {
+  if (!MORE || x.window <= 0) return 0;
+  return x.chunked ? (limit - 1) / x.window * x.window
+                   : max(0, limit - x.window);
+}
+
+// The tiles a workgroup walks: those that hold kept keys, then from the first
+// one that its earliest row (which sees keys below `limit`) sees.
+struct PagedTiles {
+  int keep, gap, n;       // at(i): i below keep as it is, else + gap
+  XLLM_DEV int at(int i) const { return i < keep ? i : i + gap; }
+};
+template <bool MORE>
+XLLM_DEV PagedTiles paged_tiles(const PagedMore& x, int limit, int kmax,
+                                int n_tiles, int kt) {
+  if (!MORE || x.window <= 0) return {0, 0, n_tiles};
+  const int first = paged_first<MORE>(x, limit) / kt;
+  const int keep = min((min(x.keep_first, kmax) + kt - 1) / kt, first);
+  return {keep, first - keep, n_tiles - (first - keep)};
+}
+
+// |scale| log2(e), above zero; a NaN stays one
+XLLM_DEV float paged_factor(float scale) {
+  const float c = fabsf(scale) * 1.4426950408889634f;
+  return c < 1e-30f ? 1e-30f : c;
+}
+
+// How a row's scores become weights 2^(c (s - m)): a negative factor turns the
+// signs of the query's entries, so that c is positive; with a cap, s is the
+// capped score and pre goes in front of the tanh.
+struct PagedScore { short flip; float c, pre; };
+template <bool MORE>
+XLLM_DEV PagedScore paged_score(const PagedMore& x, float scale, int head) {
+  constexpr float log2e = 1.4426950408889634f;
+  if (MORE && x.head_scale != nullptr) scale *= x.head_scale[head];
+  if (MORE && x.cap > 0.0f) return {0, log2e, scale / x.cap};
+  return {scale < 0.0f ? (short)0x8000 : (short)0,
+          paged_factor(scale), 0.0f};
+}
+
+// s <- cap * tanh(pre * s). Tiles without large scores, nearly all of them, skip
+// the exponentials and divisions.
+template <int N>
+XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
+  float big = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      s[i][r] *= pre;
+      big = fmaxf(big, fabsf(s[i][r]));
+    }
+  const bool far = __any(!(big < 0.5f));
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const float v = s[i][r];
+      float y = tanh_near(v);
+      if (far) {
+        const float z = tanh_far(v);
+        y = fabsf(v) < 0.5f ? y : z;
+      }
+      s[i][r] = cap * y;
+    }
+}
+
+// Decoded rows: parts that a list of n tiles is really split into, of the P that
+// the host, which does not know the lengths, made room for
+XLLM_DEV int paged_parts(int n, int P, int per) {
+  return max(1, min(P, (n + per - 1) / per));
+}
+
+// four neighbouring results
+template <bool MORE>
+XLLM_DEV void paged_put(const PagedMore& x, void* out, long at, float a,
+                        float b, float c, float d) {
+  if (MORE && x.out_f32) {
+    *reinterpret_cast<float4*>((float*)out + at) = make_float4(a, b, c, d);
+  } else {
+    uint2 y;
+    y.x = pack_bf16(a, b);
+    y.y = pack_bf16(c, d);
+    *reinterpret_cast<uint2*>((unsigned short*)out + at) = y;
+  }
+}
+
+#define PAGED_ABSENT (-1.0f)
+
+// Parts of a row, B at a time, added to (M, L, a): their maxima, sums and results
+// are all on the way at once, the first maximum is not waited for before the first
+// result is fetched. A merge is a chain of this and, in a kernel of its own, a launch:
+// 32 rows x 16 heads, up to four parts 4.67 -> 4.07 us, 17 k rows of three parts 6.55 ->
+// 5.95; by eights where there is room for more than four.
+// ml(p), o(p): maximum and sum, and four results of part p. A part without
+// keys has written no results and the sum PAGED_ABSENT: any other sum, NaN
+// among them, counts.
+template <int B, class Ml, class O>
+XLLM_DEV void paged_add_parts(const Ml& ml, const O& o, int parts, float& M,
+                              float& L, float (&a)[4]) {
+  for (int p0 = 0; p0 < parts; p0 += B) {
+    float2 z[B];
+    float4 y[B];
+#pragma unroll
+    for (int k = 0; k < B; k++) {
+      const int p = min(p0 + k, parts - 1);
+      z[k] = ml(p);
+      y[k] = o(p);
+    }
+    float top = M;
+#pragma unroll
+    for (int k = 0; k < B; k++) {
+      if (p0 + k >= parts) z[k].y = PAGED_ABSENT;
+      top = fmaxf(top, z[k].x);
+    }
+    if (top == -INFINITY) top = 0.0f;
+    const float keep = __builtin_amdgcn_exp2f(M - top);
+    M = top;
+    L *= keep;
+#pragma unroll
+    for (int c = 0; c < 4; c++) a[c] *= keep;
+#pragma unroll
+    for (int k = 0; k < B; k++) {
+      const bool on = !(z[k].y < 0.0f);
+      const float w = on ? __builtin_amdgcn_exp2f(z[k].x - M) : 0.0f;
+      L += on ? z[k].y * w : 0.0f;
+      a[0] += on ? y[k].x * w : 0.0f; a[1] += on ? y[k].y * w : 0.0f;
+      a[2] += on ? y[k].z * w : 0.0f; a[3] += on ? y[k].w * w : 0.0f;
+    }
+  }
+}
+
+// ---- the last of a unit's workgroups merges ------------------------------------
+// A unit is what is split into parts. Its workgroups count themselves when their parts
+// are in memory, and the one that finds all others counted merges: no second launch,
+// which cost 4 to 5 us of which two thirds were its start and the end of the kernel
+// before it.
+//   The counters are scratch like the parts, which nobody has cleared: a launch for that
+// would cost what the merge's did, and counters kept from call to call would have to
+// know of streams, threads and captured graphs. Instead each call has a tag of 56 random
+// bits, and whoever finds another value in a counter than its call's tag and a count
+// puts the tag and no count there: before its own part is counted, and only if the
+// counter still holds what it found. The last one sets it back, so a captured call finds
+// no count of its last replay. What lay there before would have to agree in 56 random
+// bits to pass for a count.
+//   Parts and counts pass between XCDs, whose L2s do not see each other's lines: parts
+// are stored and loaded past them (mr_store_far), a workgroup counts itself when all of
+// its waves have waited for their stores, counts are atomics at device scope.
+struct PagedMeet {
+  unsigned long long* count = nullptr;   // [units]
+  unsigned long long tag = 0;            // low 8 bits: none
+};
+typedef unsigned long long u64;
+// by one thread of a workgroup, early: at, its unit's counter
+XLLM_DEV void paged_open(u64* at, u64 seen, u64 tag) {
+  if (((seen ^ tag) >> 8) != 0)
+    __hip_atomic_compare_exchange_strong(at, &seen, tag, __ATOMIC_RELAXED,
+                                         __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+}
+XLLM_DEV u64 paged_seen(u64* at) {
+  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// by all of its threads, with their stores behind them: whether it is the last of `parts`
+XLLM_DEV bool paged_last(u64* at, int parts) {
+  __shared__ int last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const u64 old = __hip_atomic_fetch_add(at, 1ull, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+    last = (int)(old & 255) == parts - 1;
+    if (last)
+      __hip_atomic_store(at, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return last != 0;
+}
+// A call's counters, behind its parts: scratch is rows * parts * (D + 2) + 2 * units floats
+inline PagedMeet paged_meet(float* ws_ml, long rows, int parts) {
+  static std::atomic<u64> calls{[] {
+    std::random_device r;
+    return (u64)r() << 32 | r();
+  }()};
+  u64 z = calls.fetch_add(0x9e3779b97f4a7c15ull, std::memory_order_relaxed);
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;   // splitmix64 (Steele et al. 2014)
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  return {reinterpret_cast<u64*>(ws_ml + 2 * rows * parts), (z ^ (z >> 31)) << 8};
+}
+
+// out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
+// row, four columns each. Rows are those of n_seqs prompts; tokens outside of all of
+// them have no parts and stay as they are. B: parts fetched at once.
+template <int D, bool MORE, int B>
+__global__ __launch_bounds__(256) void paged_attn_merge_kernel(
+    void* __restrict__ out, const float* __restrict__ ws_o,
+    const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
+    const long out_stride, const long rows, const PagedMore x,
+    const int* __restrict__ cu_q, const int n_seqs) {
+  constexpr int LPR = D / 4;
+  const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
+  const int col = (threadIdx.x % LPR) * 4;
+  if (row >= rows) return;
+  const long tok = row / n_qheads;
+  const int head = (int)(row - tok * n_qheads);
+  if (tok < cu_q[0] || tok >= cu_q[n_seqs]) return;
+  const bool sink = MORE && x.sink != nullptr;
+  float M = sink ? x.sink[head] * 1.4426950408889634f : -INFINITY;
+  float L = sink ? 1.0f : 0.0f;
+  float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
+  const float* o = ws_o + row * n_part * D + col;
+  paged_add_parts<B>(
+      [&](int p) { return ml[p]; },
+      [&](int p) { return *reinterpret_cast<const float4*>(o + (long)p * D); },
+      n_part, M, L, a);
+  const float inv = L != 0.0f ? 1.0f / L : 0.0f;
+  paged_put<MORE>(x, out, tok * out_stride + (long)head * D + col, a[0] * inv,
+                  a[1] * inv, a[2] * inv, a[3] * inv);
+}
+
+template <int D, bool MORE>
+inline void paged_merge(void* out, const float* ws_o, const float* ws_ml,
+                        int n_qheads, int n_part, long out_stride, long rows,
+                        const PagedMore& x, hipStream_t stream,
+                        const int* cu_q, int n_seqs) {
+#define PM_GO(B)                                                               \
+  hipLaunchKernelGGL((paged_attn_merge_kernel<D, MORE, B>),                    \
+                     dim3((unsigned)((rows * (D / 4) + 255) / 256)),           \
+                     dim3(256), 0, stream, out, ws_o, ws_ml, n_qheads, n_part, \
+                     out_stride, rows, x, cu_q, n_seqs)
+  if (n_part <= 4) PM_GO(4);
+  else PM_GO(8);
+#undef PM_GO
+}
+
+}  // namespace xllm

@@ -1,0 +1,37 @@
+import sys, ctypes, statistics, json, torch
+def lib(p):
+    L = ctypes.CDLL(p); L.run.argtypes = [ctypes.c_int]+[ctypes.c_void_p]*3+[ctypes.c_int]*3+[ctypes.c_long, ctypes.c_void_p]; return L
+A, B = lib('_work/p/lv/lv.so'), lib('_work/p/lv/lv2.so')
+import importlib.util
+def load(path, name):
+    spec = importlib.util.spec_from_file_location(name, path); m = importlib.util.module_from_spec(spec); spec.loader.exec_module(m); return m
+S = load('_work/start/xllm_service_amd/_ops.cpython-310-x86_64-linux-gnu.so', 'old._ops')
+dev='cuda'; out=open('gpurun_out/tune2.txt','w')
+def graph(calls):
+    calls[0](); torch.cuda.synchronize(); g=torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        for c in calls: c()
+    return g
+xr=lambda M: next(a for a in (8,16,24,32,48,64) if M<=a)
+for N,K in [(768,768),(2304,768),(1024,1024),(512,2048),(1536,2048),(768,3072),(256,4096),(1024,4096),(640,2560),(2560,2560),(2048,2048),(2048,4096),(4096,4096),(4096,14336),(1024,8192),(4608,3584),(6144,4096),(8192,4096),(14336,4096),(28672,4096)]:
+    copies=int(max(6,min(40,(512<<20)//(2*N*K))))
+    W=[torch.randn(N,K,device=dev,dtype=torch.bfloat16) for _ in range(copies)]
+    for M in [1,8,12,16,24,28,32,40,48,56,64]:
+        x=torch.randn(M,K,device=dev,dtype=torch.bfloat16); y=torch.empty(M,N,device=dev,dtype=torch.bfloat16)
+        ref=torch.nn.functional.linear(x,W[0]).float()
+        gs={'start':graph([lambda w=w:S.linear(x,w,None) for w in W])}
+        vs=[0,1,8] if N<=4096 else [0,1,3,4,5,7]
+        for n,L in (('a',A),('b',B)):
+            for v in vs:
+                go=lambda w,v=v,L=L: L.run(xr(M)*100+v,y.data_ptr(),x.data_ptr(),w.data_ptr(),M,N,K,K,torch.cuda.current_stream().cuda_stream)
+                y.zero_()
+                if go(W[0]): continue
+                e=((y.float()-ref).norm()/ref.norm()).item(); assert e<.01,(n,v,M,N,K,e)
+                gs[f'{n}{v}']=graph([lambda w=w,go=go: go(w) for w in W])
+        ts={v:[] for v in gs}
+        for _ in range(9):
+            for v,g in gs.items():
+                e0,e1=torch.cuda.Event(True),torch.cuda.Event(True); e0.record(); g.replay(); e1.record(); torch.cuda.synchronize(); ts[v].append(e0.elapsed_time(e1)*1e3/copies)
+        m={v:round(statistics.median(t),2) for v,t in ts.items()}
+        print(N,K,M,json.dumps(m),file=out,flush=True)
+    print('ok',N,K,flush=True)

@@ -434,6 +434,48 @@ def test_narrow_decode_forms(keys, kv_heads, per):
     check(got, *want(q, k, v, table, [1] * len(keys), ctx, 0.125))
 
 
+@pytest.mark.parametrize("dim,keys,kv_heads,per", [
+    (128, [12 * 32, 12 * 32 + 1, 17 * 32], 8, 4),     # where parts begin
+    (128, [32 * 32 + 1, 65 * 32, 8 * 65 * 32 + 5], 1, 7),   # eight of them, more
+    (64, [16 * 32, 16 * 32 + 1, 21 * 32, 31, 2000], 16, 1),
+    (128, [23 * 32, 23 * 32 + 1, 3000, 40] * 3, 8, 3),      # 96 pairs
+    (64, [19 * 32, 19 * 32 + 1, 2000, 700] * 2, 12, 1),
+    (64, [39 * 32, 39 * 32 + 1, 2000, 9] * 4, 12, 2)])      # 192
+def test_decode_parts_meet(dim, keys, kv_heads, per):
+    """Sequences split into parts, whose last workgroup merges: over scratch that
+    held anything before, and in replays of a captured step whose lengths change."""
+    ctx = [n - 1 for n in keys]
+    rows, k, v, table = make([1] * len(keys), ctx, kv_heads, per, dim, sum(keys))
+    heads, scale = kv_heads * per, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim)).contiguous()
+    dev = [t.cuda() for t in (q, k, v, table)]
+    sl = torch.tensor(keys, dtype=torch.int32, device="cuda")
+    out = torch.empty_like(dev[0])
+
+    def litter():              # where scratch will be: any values
+        for fill in (0, -1, 0x7f7f7f7f7f7f7f01):
+            torch.full((1 << 18,), fill, dtype=torch.int64, device="cuda")
+
+    def step():
+        litter()
+        ops.paged_attn_decode(*dev, sl, scale, out=out)
+    step()
+    check(out, *want(q, k, v, table, [1] * len(keys), ctx, scale))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for lens in (keys, keys, [max(1, n // 2) for n in keys], keys):
+        sl.copy_(torch.tensor(lens))
+        out.fill_(3.0)
+        graph.replay()
+        got = out.clone()
+        ops.paged_attn_decode(*dev, sl, scale, out=out)
+        assert torch.equal(got, out)
+        check(got, *want(q, k, v, table, [1] * len(lens),
+                         [n - 1 for n in lens], scale))
+
+
 def test_decode_standout_scores():
     rows, k, v, table = make([1, 1], [900, 350], 1, 2, 128, 5)
     k[table[0, 4], 0, 3] *= 30.0

@@ -1154,11 +1154,11 @@ void capped_attn(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
         hy::paged_attn_parts(cu == nullptr, T, n_seqs, heads, n_kv,
                              block_tables.size(1), window, keep_first,
                              cap > 0);
-    Tensor ws;                 // [T * heads][parts][D + 2]
+    Tensor ws;                 // [T * heads][parts][D + 2], and counters
     float *ws_o = nullptr, *ws_ml = nullptr;
     if (n_part > 1) {
       const long n = (long)T * heads * n_part;
-      ws = torch::empty({n * (D + 2)}, out.options().dtype(torch::kFloat));
+      ws = torch::empty({n * (D + 2) + 2L * n_seqs * n_kv}, out.options().dtype(torch::kFloat));
       ws_o = ptr<float>(ws);
       ws_ml = ws_o + n * D;
     }

@@ -379,8 +379,12 @@ __global__ void __launch_bounds__(256) latent_stream_merge_kernel(
           (window > 0 ? max(0, len - window) / LS_KT : 0), n_part, per, few);
   if (parts == 1) return;                        // written where it belongs
   float M = -INFINITY, L = 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  paged_add_parts<8>(reinterpret_cast<const float2*>(ws_ml) + row * n_part,
-                     ws_o + row * n_part * LS_R + col, parts, LS_R, M, L, a);
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
+  const float* o = ws_o + row * n_part * LS_R + col;
+  paged_add_parts<8>(
+      [&](int p) { return ml[p]; },
+      [&](int p) { return *reinterpret_cast<const float4*>(o + (long)p * LS_R); },
+      parts, M, L, a);
   const float inv = L != 0.0f ? 1.0f / L : 0.0f;
   *reinterpret_cast<float4*>(out + row * LS_R + col) =
       make_float4(a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);

@@ -239,7 +239,7 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   TORCH_CHECK(n_qheads % n_kv == 0 && n_qheads / n_kv <= 8,
               "GQA group must be <= 8");
   int parts = 1;
-  torch::Tensor ws;            // [seqs * heads][parts][D + 2], fp32
+  torch::Tensor ws;            // [seqs * heads][parts][D + 2], fp32, and counters
   float *ws_o = nullptr, *ws_ml = nullptr;
   const bool stream = (D == 128 || D == 64) && on_bytes(k_cache, 16) &&
                       on_bytes(v_cache, 16) && on_bytes(q, 16) &&
@@ -249,7 +249,7 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
                                           block_tables.size(1));
     if (parts > 1) {
       const long n = (long)num_seqs * n_qheads * parts;
-      ws = torch::empty({n * (D + 2)}, q.options().dtype(torch::kFloat));
+      ws = torch::empty({n * (D + 2) + 2L * num_seqs * n_kv}, q.options().dtype(torch::kFloat));
       ws_o = ws.data_ptr<float>();
       ws_ml = ws_o + n * D;
     }

@@ -115,6 +115,28 @@ XLLM_DEV uint4 mr_load(__amdgpu_buffer_rsrc_t src, unsigned off) {
   const u4 v = __builtin_amdgcn_raw_buffer_load_b128(src, off, 0, 0);
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+// 16 and 8 bytes that a workgroup on another XCD wrote or will read: past the L2s,
+// each of which serves one XCD (device scope, the sc1 bit of loads and stores). A store
+// is there once the wave has waited for it.
+constexpr int MR_DEVICE = 16;
+XLLM_DEV float4 mr_load_far(__amdgpu_buffer_rsrc_t src, unsigned off) {
+  return __builtin_bit_cast(
+      float4, __builtin_amdgcn_raw_buffer_load_b128(src, off, 0, MR_DEVICE));
+}
+XLLM_DEV float2 mr_load_far2(__amdgpu_buffer_rsrc_t src, unsigned off) {
+  return __builtin_bit_cast(
+      float2, __builtin_amdgcn_raw_buffer_load_b64(src, off, 0, MR_DEVICE));
+}
+XLLM_DEV void mr_store_far(__amdgpu_buffer_rsrc_t dst, unsigned off, float4 v) {
+  typedef __attribute__((ext_vector_type(4))) unsigned u4;
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), dst, off, 0,
+                                         MR_DEVICE);
+}
+XLLM_DEV void mr_store_far2(__amdgpu_buffer_rsrc_t dst, unsigned off, float2 v) {
+  typedef __attribute__((ext_vector_type(2))) unsigned u2;
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), dst, off, 0,
+                                        MR_DEVICE);
+}
 XLLM_DEV f32x16 mr_zero() {
   f32x16 z;
 #pragma unroll

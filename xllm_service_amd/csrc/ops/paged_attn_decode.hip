@@ -132,10 +132,10 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
 // shuffle 7.9 | split 17.1 | whole 9.2 us, 500 keys 35 | 38.5 | 32. From 768 pairs on
 // workgroups of two waves, twice as many at a time: 64 keys 9.2 -> 6.8, 16 8.0 -> 5.9
 // (384 pairs of 500 keys 11.8 -> 15.7, so not there).
-//   Few pairs: as for 128-wide heads. In tables of 768 keys and more that costs the
-// shortest sequences the merge (64 keys 4.7 -> 5.6 us) for what the others gain (200
-// keys 9.3 -> 6.5, 1000 32 -> 7.7); eight waves without a merge would be 4.6, 5.2 and
-// 9.1, 2000 keys 13.9 instead of 7.7.
+//   Few pairs: as for 128-wide heads. 86 to 192, whole | by 16 tiles, at most four: 8
+// sequences of 12 heads, 1000 keys 13.1 | 11.1, 2000 22.1 | 15.5, 0.1-2 k 17.6 | 10.3, but 600
+// 8.9 | 9.1; 16 of 2000 25.6 | 24.2, 0.1-2 k 19.8 | 18.0, but 1300 19.1 | 19.9; 21 of 2000 27.5 |
+// 31.4.
 //   128-wide heads: two waves only where tables have few tiles, of which four leave
 // waves idle that hold LDS (32 key heads, 32 x 16 keys 10.1 -> 8.4). In wide tables long
 // sequences may be there, which two waves walk more slowly (30 x 0.1-3.6 k, 32 key heads
@@ -144,8 +144,16 @@ __global__ __launch_bounds__(256) void paged_attn_decode_small_kernel(
 static PagedSplit decode_split(long num_seqs, int n_kv_heads, int D,
                                long max_blocks) {
   const long units = num_seqs * n_kv_heads;
-  if (D == 64 && units >= 86) return {1, 1, units >= 768 ? 2 : 4};
-  PagedSplit x = paged_stream_split(num_seqs, n_kv_heads, max_blocks);
+  PagedSplit x;
+  if (D == 64 && units >= 86) {
+    if (units >= 768) x.waves = 2;
+    if (units > 192) return x;
+    x.per = 16;
+    x.least = units <= 128 ? 24 : 48;
+    x.parts = (int)std::min<long>(4, (max_blocks + 31) / 32);
+    return x;
+  }
+  x = paged_stream_split(num_seqs, n_kv_heads, max_blocks);
   if (max_blocks <= 2 || (units >= 768 && max_blocks <= 16)) x.waves = 2;
   return x;
 }

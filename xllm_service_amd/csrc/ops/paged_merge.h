@@ -1,6 +1,9 @@
 // What the paged attention kernels (paged_rows.h, paged_stream.h) share: their
 // options, and the merge of keys that were split over workgroups.
 #pragma once
+#include <atomic>
+#include <random>
+
 #include "mfma_rows.h"
 
 namespace xllm {
@@ -87,10 +90,26 @@ XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
 }
 
 // Decoded rows: parts that a list of n tiles is really split into, of the P that
-// the host, which does not know the lengths, made room for
-XLLM_DEV int paged_parts(int n, int P, int per) {
-  return max(1, min(P, (n + per - 1) / per));
+// the host, which does not know the lengths, made room for: one for every `per` tiles,
+// of up to eight one for every `near`
+__host__ __device__ inline int paged_parts(int n, int P, int per) {
+  const int p = (n + per - 1) / per;
+  return p < 1 ? 1 : p > P ? P : p;
 }
+struct PagedSplit {
+  int parts = 1, per = 1;
+  int near = 1 << 20;        // tiles
+  int least = 0;             // tiles of the shortest list that is split
+  bool twos = false;         // 2, 4 or 8 of them
+  int waves = 4;             // of a workgroup
+  __host__ __device__ int of(int n) const {
+    const int far = paged_parts(n, parts, per);
+    const int most = paged_parts(n, parts < 8 ? parts : 8, near);
+    if (n < least) return 1;
+    return twos ? far < 2 ? 1 : far < 5 ? 2 : far < 8 ? 4 : 8
+                : far > most ? far : most;
+  }
+};
 
 // four neighbouring results
 template <bool MORE>
@@ -110,23 +129,23 @@ XLLM_DEV void paged_put(const PagedMore& x, void* out, long at, float a,
 
 // Parts of a row, B at a time, added to (M, L, a): their maxima, sums and results
 // are all on the way at once, the first maximum is not waited for before the first
-// result is fetched. A merge is a launch and this chain: 32 rows x 16 heads, up to
-// four parts 4.67 -> 4.07 us, 17 k rows of three parts 6.55 -> 5.95; by eights where
-// there is room for more than four.
-// ml, o: of the row's first part, stride floats between results. A part without
+// result is fetched. A merge is a chain of this and, in a kernel of its own, a launch:
+// 32 rows x 16 heads, up to four parts 4.67 -> 4.07 us, 17 k rows of three parts 6.55 ->
+// 5.95; by eights where there is room for more than four.
+// ml(p), o(p): maximum and sum, and four results of part p. A part without
 // keys has written no results and the sum PAGED_ABSENT: any other sum, NaN
 // among them, counts.
-template <int B>
-XLLM_DEV void paged_add_parts(const float2* ml, const float* o, int parts,
-                              int stride, float& M, float& L, float (&a)[4]) {
+template <int B, class Ml, class O>
+XLLM_DEV void paged_add_parts(const Ml& ml, const O& o, int parts, float& M,
+                              float& L, float (&a)[4]) {
   for (int p0 = 0; p0 < parts; p0 += B) {
     float2 z[B];
     float4 y[B];
 #pragma unroll
     for (int k = 0; k < B; k++) {
       const int p = min(p0 + k, parts - 1);
-      z[k] = ml[p];
-      y[k] = *reinterpret_cast<const float4*>(o + (long)p * stride);
+      z[k] = ml(p);
+      y[k] = o(p);
     }
     float top = M;
 #pragma unroll
@@ -151,18 +170,73 @@ XLLM_DEV void paged_add_parts(const float2* ml, const float* o, int parts,
   }
 }
 
+// ---- the last of a unit's workgroups merges ------------------------------------
+// A unit is what is split into parts. Its workgroups count themselves when their parts
+// are in memory, and the one that finds all others counted merges: no second launch,
+// which cost 4 to 5 us of which two thirds were its start and the end of the kernel
+// before it.
+//   The counters are scratch like the parts, which nobody has cleared: a launch for that
+// would cost what the merge's did, and counters kept from call to call would have to
+// know of streams, threads and captured graphs. Instead each call has a tag of 56 random
+// bits, and whoever finds another value in a counter than its call's tag and a count
+// puts the tag and no count there: before its own part is counted, and only if the
+// counter still holds what it found. The last one sets it back, so a captured call finds
+// no count of its last replay. What lay there before would have to agree in 56 random
+// bits to pass for a count.
+//   Parts and counts pass between XCDs, whose L2s do not see each other's lines: parts
+// are stored and loaded past them (mr_store_far), a workgroup counts itself when all of
+// its waves have waited for their stores, counts are atomics at device scope.
+struct PagedMeet {
+  unsigned long long* count = nullptr;   // [units]
+  unsigned long long tag = 0;            // low 8 bits: none
+};
+typedef unsigned long long u64;
+// by one thread of a workgroup, early: at, its unit's counter
+XLLM_DEV void paged_open(u64* at, u64 seen, u64 tag) {
+  if (((seen ^ tag) >> 8) != 0)
+    __hip_atomic_compare_exchange_strong(at, &seen, tag, __ATOMIC_RELAXED,
+                                         __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+}
+XLLM_DEV u64 paged_seen(u64* at) {
+  return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// by all of its threads, with their stores behind them: whether it is the last of `parts`.
+// last: LDS that nothing else is in
+XLLM_DEV bool paged_last(u64* at, int parts, int* last) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const u64 old = __hip_atomic_fetch_add(at, 1ull, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+    const bool all = (int)(old & 255) == parts - 1;
+    *last = all;
+    if (all)
+      __hip_atomic_store(at, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return *last != 0;
+}
+// A call's counters, behind its parts: scratch is rows * parts * (D + 2) + 2 * units floats
+inline PagedMeet paged_meet(float* ws_ml, long rows, int parts) {
+  static std::atomic<u64> calls{[] {
+    std::random_device r;
+    return (u64)r() << 32 | r();
+  }()};
+  u64 z = calls.fetch_add(0x9e3779b97f4a7c15ull, std::memory_order_relaxed);
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;   // splitmix64 (Steele et al. 2014)
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  return {reinterpret_cast<u64*>(ws_ml + 2 * rows * parts), (z ^ (z >> 31)) << 8};
+}
+
 // out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
-// row, four columns each. seq_lens: rows are decoded ones, one sequence each,
-// with as many parts as their length asks for (per tiles of kt keys); a single
-// part has been written where it belongs. cu_q: rows are those of n_seqs prompts;
-// tokens outside of all of them have no parts and stay as they are. B: parts
-// fetched at once.
+// row, four columns each. Rows are those of n_seqs prompts; tokens outside of all of
+// them have no parts and stay as they are. B: parts fetched at once.
 template <int D, bool MORE, int B>
 __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
     void* __restrict__ out, const float* __restrict__ ws_o,
     const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
     const long out_stride, const long rows, const PagedMore x,
-    const int* __restrict__ seq_lens, const int per, const int kt,
     const int* __restrict__ cu_q, const int n_seqs) {
   constexpr int LPR = D / 4;
   const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
@@ -170,20 +244,17 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
   if (row >= rows) return;
   const long tok = row / n_qheads;
   const int head = (int)(row - tok * n_qheads);
-  int parts = n_part;
-  if (cu_q != nullptr && (tok < cu_q[0] || tok >= cu_q[n_seqs])) return;
-  if (seq_lens != nullptr) {
-    const int len = seq_lens[tok];
-    parts = paged_parts(
-        paged_tiles<MORE>(x, len, len, (len + kt - 1) / kt, kt).n, n_part, per);
-    if (parts == 1) return;
-  }
+  if (tok < cu_q[0] || tok >= cu_q[n_seqs]) return;
   const bool sink = MORE && x.sink != nullptr;
   float M = sink ? x.sink[head] * 1.4426950408889634f : -INFINITY;
   float L = sink ? 1.0f : 0.0f;
   float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  paged_add_parts<B>(reinterpret_cast<const float2*>(ws_ml) + row * n_part,
-                     ws_o + row * n_part * D + col, parts, D, M, L, a);
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
+  const float* o = ws_o + row * n_part * D + col;
+  paged_add_parts<B>(
+      [&](int p) { return ml[p]; },
+      [&](int p) { return *reinterpret_cast<const float4*>(o + (long)p * D); },
+      n_part, M, L, a);
   const float inv = L != 0.0f ? 1.0f / L : 0.0f;
   paged_put<MORE>(x, out, tok * out_stride + (long)head * D + col, a[0] * inv,
                   a[1] * inv, a[2] * inv, a[3] * inv);
@@ -193,13 +264,12 @@ template <int D, bool MORE>
 inline void paged_merge(void* out, const float* ws_o, const float* ws_ml,
                         int n_qheads, int n_part, long out_stride, long rows,
                         const PagedMore& x, hipStream_t stream,
-                        const int* seq_lens, int per, int kt,
-                        const int* cu_q = nullptr, int n_seqs = 0) {
+                        const int* cu_q, int n_seqs) {
 #define PM_GO(B)                                                               \
   hipLaunchKernelGGL((paged_attn_merge_kernel<D, MORE, B>),                    \
                      dim3((unsigned)((rows * (D / 4) + 255) / 256)),           \
                      dim3(256), 0, stream, out, ws_o, ws_ml, n_qheads, n_part, \
-                     out_stride, rows, x, seq_lens, per, kt, cu_q, n_seqs)
+                     out_stride, rows, x, cu_q, n_seqs)
   if (n_part <= 4) PM_GO(4);
   else PM_GO(8);
 #undef PM_GO

@@ -405,8 +405,7 @@ inline void paged_rows(void* out, float* ws_o, float* ws_ml,
                      max_blocks, q_stride, out_stride, n_part, x);
   if (n_part > 1)
     paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, n_part, out_stride,
-                         tokens * n_qheads, x, stream, nullptr, 1, 1, cu_q,
-                         n_seqs);
+                         tokens * n_qheads, x, stream, cu_q, n_seqs);
 }
 
 }  // namespace xllm

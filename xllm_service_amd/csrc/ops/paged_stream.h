@@ -15,14 +15,17 @@
 //   * waves of a workgroup merge through LDS at the end; where there are too
 //     few (sequence, kv_head) pairs to fill the chip, or tables long enough for
 //     one sequence to outlast the others, the keys are split over up to P
-//     workgroups, as many as a sequence's own length asks for, whose fp32
-//     results a second kernel merges
+//     workgroups, as many as a sequence's own length asks for, of whose fp32
+//     results the last one to finish makes the sequence's (paged_meet)
 //
 // Measured, 32 query / 8 key heads of 128: 128 sequences of 1-2 k keys 160 ->
 // 143 us, 5.6 TB/s (a large copy: 4.9); 24 x 0.6-1.3 k 24 + 9 -> 18 us; one of
 // 776: 16 -> 8 us. 28/4 heads, 6 x 9-20 k: 54 + 16 -> 28 + 4 us. Before: K in
 // registers a tile ahead, V loaded in the tile that used it, one result per
-// wave through memory.
+// wave through memory. What a second kernel for the merge cost, and parts that
+// were larger for it, us with its launch -> here: one of 776 10.6 -> 7.5, 6 x 9-20 k
+// 38.4 -> 37.0, 16 x 0.5-4 k 31.3 -> 25.5. What is left of it is a chain of three
+// trips to memory: results out, the count, all results in.
 #pragma once
 #include <algorithm>
 
@@ -109,8 +112,9 @@ XLLM_DEV void pa_rows(const unsigned (&at)[D / 16], bf16x8 (&k)[D / 16]) {
 // by 32 waves a row 0.00186; with two 0.00166, which is the rounding to bf16. Us,
 // one term | two by a product of their own | here: 1 x 776 keys 9.0 | 9.6 | 9.5,
 // 24 x 0.6-1.4 k 18.9 | 19.6 | 19.1, 128 x 1-2 k 142.5 | 142.8 | 142.0.
-//   NW: waves of a workgroup, four but where the host asks for two.
-template <int D, int TERMS, bool MORE, int NW>
+//   NW: waves of a workgroup, four but where the host asks for two. SPLIT: there is room
+// for parts (without the code for them 5.05 -> 4.93 us for a few keys).
+template <int D, int TERMS, bool MORE, int NW, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, NW == 2 && D == 64 ? 8 : 2) void
 paged_attn_stream_kernel(
     void* __restrict__ out,                  // [S, n_qheads, D]
@@ -122,8 +126,8 @@ paged_attn_stream_kernel(
     const int* __restrict__ block_tables,    // [num_seqs, max_blocks]
     const int* __restrict__ seq_lens,        // [num_seqs]
     const float scale, const int G, const int n_kv, const int max_blocks,
-    const long q_stride, const long out_stride, const int P, const int per,
-    const PagedMore x) {
+    const long q_stride, const long out_stride, const PagedSplit split,
+    const PagedMeet meet, const PagedMore x) {
   constexpr int KS = D / 16, DT = D / 32;
   constexpr bool FOLD = TERMS == 2;          // G <= 8
   constexpr int NP = FOLD ? 1 : TERMS;       // products per weight
@@ -139,7 +143,7 @@ paged_attn_stream_kernel(
   const int h = lane >> 5, c32 = lane & 31;
   // first the first parts of all: idle ones are then the last and not all of one
   // XCD (16 x 1000 keys of 8 heads with room for 8: 55 us the other way, 22 so)
-  const int units = gridDim.x / P;
+  const int P = SPLIT ? split.parts : 1, units = gridDim.x / P;
   const int part = blockIdx.x / units, unit = blockIdx.x % units;
   const int seq = unit / n_kv, kvh = unit % n_kv;
   const int seq_len = seq_lens[seq];
@@ -147,8 +151,10 @@ paged_attn_stream_kernel(
   // a wave's tiles are every step-th of the list, from the i0-th on
   const PagedTiles list =
       paged_tiles<MORE>(x, seq_len, seq_len, n_tiles, PA_KT);
-  const int parts = paged_parts(list.n, P, per);
-  if (part >= parts) return;
+  const int parts = SPLIT ? split.of(list.n) : 1;
+  if (SPLIT && part >= parts) return;
+  u64 seen = 0;
+  if (SPLIT && parts > 1 && tid == 0) seen = paged_seen(meet.count + unit);
   const int step = parts * NW, i0 = part * NW + wid;
   const int lo = paged_first<MORE>(x, seq_len);   // first key in the window
 
@@ -248,6 +254,7 @@ paged_attn_stream_kernel(
     vat[i] = (unsigned)(unsigned long long)((const lds_u16*)vt +
                                             (vbase ^ (i << 5)));
   int pages = pages_from(0);
+  if (SPLIT && parts > 1 && tid == 0) paged_open(meet.count + unit, seen, meet.tag);
   if (i0 < list.n) {
     load(list.at(i0), 0, pages, false);
     load(list.at(i0), 0, pages, true);
@@ -357,6 +364,10 @@ paged_attn_stream_kernel(
                         o_acc[i][r + 3]);
   }
   __syncthreads();
+  // parts of this unit's rows
+  const long rows_at = ((long)seq * n_kv + kvh) * G * P;
+  const auto unit_o = mr_buffer(ws_o + rows_at * D, parts == 1 ? 0 : G * P * D * 4);
+  const auto unit_ml = mr_buffer(ws_ml + rows_at * 2, parts == 1 ? 0 : G * P * 8);
   for (int idx = tid; idx < G * (D / 4); idx += NW * 64) {
     const int row = idx / (D / 4), at = idx % (D / 4) * 4;
     float M = -INFINITY;
@@ -376,7 +387,7 @@ paged_attn_stream_kernel(
       }
       a[0] += y.x * f; a[1] += y.y * f; a[2] += y.z * f; a[3] += y.w * f;
     }
-    if (parts == 1) {
+    if (!SPLIT || parts == 1) {
       if (MORE && x.sink != nullptr)
         L += __builtin_amdgcn_exp2f(
             x.sink[kvh * G + row] * 1.4426950408889634f - M);
@@ -385,64 +396,93 @@ paged_attn_stream_kernel(
                       (long)(kvh * G + row) * D + at,
                       a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
     } else {
-      const long slot = ((long)seq * n_kv * G + kvh * G + row) * P + part;
-      if (at == 0) {
-        ws_ml[slot * 2] = M;
-        ws_ml[slot * 2 + 1] = L;
-      }
-      *reinterpret_cast<float4*>(ws_o + slot * D + at) =
-          make_float4(a[0], a[1], a[2], a[3]);
+      const int slot = row * P + part;
+      if (at == 0) mr_store_far2(unit_ml, slot * 8, make_float2(M, L));
+      mr_store_far(unit_o, (slot * D + at) * 4,
+                   make_float4(a[0], a[1], a[2], a[3]));
     }
+  }
+  int* flag = reinterpret_cast<int*>(kv_lds);
+  if (!SPLIT || parts == 1 || !paged_last(meet.count + unit, parts, flag)) return;
+  // ---- all parts are there ----------------------------------------------------
+  for (int idx = tid; idx < G * (D / 4); idx += NW * 64) {
+    const int row = idx / (D / 4), at = idx % (D / 4) * 4;
+    const bool sink = MORE && x.sink != nullptr;
+    float M = sink ? x.sink[kvh * G + row] * 1.4426950408889634f : -INFINITY;
+    float L = sink ? 1.0f : 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int slot = row * P;
+    paged_add_parts<8>(
+        [&](int p) { return mr_load_far2(unit_ml, (slot + p) * 8); },
+        [&](int p) { return mr_load_far(unit_o, ((slot + p) * D + at) * 4); },
+        parts, M, L, a);
+    const float inv = L != 0.0f ? 1.0f / L : 0.0f;
+    paged_put<MORE>(x, out, (long)seq * out_stride +
+                    (long)(kvh * G + row) * D + at,
+                    a[0] * inv, a[1] * inv, a[2] * inv, a[3] * inv);
   }
 }
 
 // Parts the keys of a (sequence, kv_head) pair are split into: room for P of them
-// from what the host knows (the pairs and the widest table), one for every `per`
-// tiles of a sequence's own in the kernel.
-//   Few pairs: one workgroup per CU is enough to split for (more only add
-// results to merge), a part of less than eight tiles (two a wave) is not worth its
-// share of the merge, neither is room for two. Measured (us), whole | split: 1 x
-// 776 keys 10.2 | 7.8, 1 x 2000 18.8 | 8.9, 1 x 20000 143 | 20 (16 parts), 8 x
-// 2000 19.9 | 15.8, 8 x 14000 144 | 82; 1 x 200 5.4 | 6.6, 8 x 500 8.6 | 9.7.
-//   More pairs fill the chip, and equal ones lose by a split what the merge costs
-// (16 x 1000 keys, 8 key heads, 13.9 | 15.6; 32 x 1-2 k 36.7 | 40.2), but a long
-// sequence among short ones is a chain of tiles that outlasts the rest. By parts of
-// 32 tiles, at most 8: 23 x 0.3-12 k, 4 key heads 122 | 70; 8 key heads, 16 x 2-16 k
-// 173 | 142, 48 x 0.3-8 k 184 | 159, 32 x 0.3-6 k 83.3 | 82.4, 16 x 0.3-2 k 20.3
-// | 20.3. The host sees no lengths, and in a captured step the widest table there can
-// be: whole below 3000 keys, and up to 128 pairs (which bring the least bytes to
-// hide a chain behind) above, up to 4096 for more pairs. From 768 pairs
-// on they are whole in any table: idle parts and the merge cost short sequences up to
-// twice their time (tables of 8192, 8 key heads, 128 x 16 keys 12.3 whole | 18.1, x 64
-// 15.4 | 19.2; 32 key heads, 256 x 16 65 | 113), and neither even nor uneven lengths
-// gain by parts there. 512 to 767 pairs do: 8 key heads, 66 x 3.6-7.3 k 232 | 212, 32
+// from what the host knows (the pairs and the widest table), as many as a sequence's
+// own tiles ask for in the kernel (PagedSplit::of).
+//   Few pairs: one workgroup per CU is enough to split for. Up to eight parts one tile
+// for each wave is best, beyond them two, and what is done in three turns of a wave not
+// worth the merge. Us, 8 key heads, by parts: 1 x 776 keys 12.2 whole, 8.9 (4), 8.1 (8);
+// 1 x 2000 21, 9.4 (8), 10.0 (16); 1 x 20000 182, 22.8 (16); 1 x 300 7.7, 7.6 (3), 1 x 400
+// 8.7, 8.4 (2), 7.5 (4); 8 x 500 9.5, 9.1 (4), 8 x 2000 26, 17.7 (4); 64-wide, 4 x 400 7.9,
+// 7.5 (4), but 7 x 400, with room for three, 7.9, 8.4.
+//   With options (a window, a cap, a sink) weights have 32 bits and a tile is longer: four
+// tiles a part however many, from nine on (4 key heads, 1 x 300 keys, capped 10.5 whole,
+// 8.3 in three, 1 x 1000 19.7, 8.5 in eight; a window of 512 12.0, 8.2 in five).
+//   Up to 128 pairs, whole | by 16 tiles, 2, 4 or 8 parts: 11 x 1000 16.8 | 14.3, 16 x 1000
+// 17.7 | 17.6, 11 x 0.5-4 k 31.0 | 21.6, 16 x 0.2-2 k 25.3 | 20.5. Not 3: 264 workgroups for 256
+// CUs, 11 x 1500 20.4 | 23.2 and 19.0 in two; 11 x 2000 21.6 in two, 23.8 in four. Long
+// tables, up to 32 tiles a part: 22 x 1-20 k, 4 key heads, 84.0 | 86.9 by 16, 83.5 by 32.
+//   More pairs fill the chip, and equal ones lose by a split what the merge costs (24 x
+// 0.6-1.4 k 22.8 | 26.4; 32 x 1-2 k 38.2 | 41.3), but a long sequence among short ones is a
+// chain of tiles that outlasts the rest. By parts of 32 tiles, at most 8: 8 key heads, 16 x
+// 2-16 k 173 | 142, 48 x 0.3-8 k 184 | 159, 32 x 0.3-6 k 83.3 | 82.4. The host sees no
+// lengths, and in a captured step the widest table there can be: whole up to 4096 keys.
+// From 768 pairs on they are whole in any table: idle parts and the merge cost short
+// sequences up to twice their time (tables of 8192, 8 key heads, 128 x 16 keys 12.3 whole
+// | 18.1, x 64 15.4 | 19.2; 32 key heads, 256 x 16 65 | 113), and neither even nor uneven
+// lengths gain by parts there. 512 to 767 pairs do: 8 key heads, 66 x 3.6-7.3 k 232 | 212, 32
 // key heads, 22 x 0.2-8.7 k 277 | 241, against 64 x 16 keys 7.9 | 10.9, x 200 15.5 | 16.7.
-//   With options (a window, a cap, a sink) weights have 32 bits and a tile is longer,
-// with a cap about twice as long: four tiles a part instead of eight (8 key heads, a
-// window of 512 11.7 -> 10.3, 300 keys in tables of 4096 9.8 -> 8.6), and for capped
-// scores, with many pairs below 512, from 1500 keys on at most four parts of 20 tiles
-// (1024 pairs of 16 keys in tables of 4096 8.6 in one | 16.5). 4 key heads: 32 x 0.7-3 k 47 | 30, 32 x 0-4 k 61 | 37, 64 x 0.3-3 k
-// 54 | 51, 24 x 0.1-1 k in tables of 4096 20 | 19 (parts of 16: 31, 37, 50, 17; of
-// 32: 31, 36, 54, 22).
-//   Eight waves in a workgroup instead of four: within 5 % where keys are split,
-// slower for many pairs (128 x 300 keys: 41 against 33).
-struct PagedSplit { int parts, per, waves = 4; };
+//   Capped scores take twice as long: with many pairs below 512, from 1500 keys on at most
+// four parts of 20 tiles (1024 pairs of 16 keys in tables of 4096 8.6 in one | 16.5). 4 key
+// heads: 32 x 0.7-3 k 47 | 30, 32 x 0-4 k 61 | 37, 64 x 0.3-3 k 54 | 51, 24 x 0.1-1 k in tables
+// of 4096 20 | 19 (parts of 16: 31, 37, 50, 17; of 32: 31, 36, 54, 22).
+//   Eight waves in a workgroup instead of four: within 5 % where keys are split and where
+// they are not, slower for many pairs (128 x 300 keys: 41 against 33).
 inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
                                      long max_blocks, bool options = false,
                                      bool capped = false) {
   const long units = num_seqs * n_kv_heads;
-  const bool few = units < 86;
-  const long f = (few ? options : capped) ? 2 : 1;
-  const long tiles = f * ((max_blocks * PA_BS + PA_KT - 1) / PA_KT);
-  const int per = few ? (int)(8 / f) : capped ? 20 : 32;
-  if (few && units > 0) {
-    const long p = std::min<long>({256 / units, tiles / 8, 16});
-    return {p < 3 ? 1 : (int)p, per};
+  const long table = (max_blocks * PA_BS + PA_KT - 1) / PA_KT;
+  PagedSplit x;
+  if (units == 0) return x;
+  if (units < 86) {
+    x.parts = (int)std::min<long>(256 / units, 16);
+    x.per = options ? 4 : 8;
+    x.near = 4;
+    x.least = options ? 9 : x.parts < 4 ? 17 : 13;
+    x.parts = x.of((int)std::min<long>(table, 1 << 20));
+    return x;
   }
-  if (units == 0 || tiles < 96 || (units > 128 && !capped && tiles <= 128) ||
+  if (units <= 128 && !options) {
+    x.per = (int)std::min<long>(32, std::max<long>(16, table / 8));
+    x.least = 24;
+    x.twos = true;
+    x.parts = (int)std::min<long>(8, (table + x.per - 1) / x.per);
+    return x;
+  }
+  const long f = capped ? 2 : 1, tiles = f * table;
+  x.per = capped ? 20 : 32;
+  if (tiles < 96 || (units > 128 && !capped && tiles <= 128) ||
       (capped && units >= 512) || (!options && units >= 768))
-    return {1, per};
-  return {(int)std::min<long>(8 / f, (tiles + 31) / 32), per};
+    return x;
+  x.parts = (int)std::min<long>(8 / f, (tiles + 31) / 32);
+  return x;
 }
 
 // Decoded rows (at most 32 query heads per key head, 8 with two terms) and the
@@ -457,23 +497,19 @@ inline void paged_stream(void* out, float* ws_o, float* ws_ml,
                          hipStream_t stream) {
   if (num_seqs == 0) return;
   const dim3 grid((unsigned)(num_seqs * n_kv * split.parts));
-#define PS_GO(NW)                                                              \
-  hipLaunchKernelGGL((paged_attn_stream_kernel<D, TERMS, MORE, NW>), grid,     \
-                     dim3(NW * 64), 0, stream, out, ws_o, ws_ml, q, k_cache,   \
-                     v_cache, block_tables, seq_lens, scale, n_qheads / n_kv,  \
-                     n_kv, max_blocks, q_stride, out_stride, split.parts,      \
-                     split.per, x)
-  if constexpr (!MORE) {
-    if (split.waves == 2) PS_GO(2);
-    else PS_GO(4);
-  } else {
-    PS_GO(4);
-  }
-#undef PS_GO
+  PagedMeet meet;
   if (split.parts > 1)
-    paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, split.parts, out_stride,
-                         (long)num_seqs * n_qheads, x, stream, seq_lens,
-                         split.per, PA_KT);
+    meet = paged_meet(ws_ml, (long)num_seqs * n_qheads, split.parts);
+#define PS_GO(NW, SPLIT)                                                       \
+  hipLaunchKernelGGL((paged_attn_stream_kernel<D, TERMS, MORE, NW, SPLIT>),    \
+                     grid, dim3(NW * 64), 0, stream, out, ws_o, ws_ml, q,      \
+                     k_cache, v_cache, block_tables, seq_lens, scale,          \
+                     n_qheads / n_kv, n_kv, max_blocks, q_stride, out_stride,  \
+                     split, meet, x)
+  if (split.parts > 1) PS_GO(4, true);
+  else if (!MORE && split.waves == 2) PS_GO((MORE ? 4 : 2), false);
+  else PS_GO(4, false);
+#undef PS_GO
 }
 
 }  // namespace xllm

@@ -565,6 +565,41 @@ def test_options(dim, bf16_out, lens, ctx, kv_heads, per, decode, opts):
         assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [
+    (8, 4, 128, [650], [0], 1.0),                    # waves in two groups
+    (8, 4, 128, [60, 700, 1], [900, 0, 130], -1.0),  # tiles for one group only
+    (12, 3, 128, [1500], [0], 1.0),                  # more workgroups than CUs
+    (12, 1, 64, [448, 64, 65, 384] * 2 + [300], [0, 0, 1, 5] * 2 + [0], 1.0),
+    (8, 4, 128, [260, 64, 33, 250, 1, 320, 300], [0, 90, 4, 3, 270, 0, 0], 1.0),
+    (8, 4, 128, [40] * 40, [i % 5 * 60 for i in range(40)], 1.0),
+])
+def test_prefill_orders_and_groups(kv_heads, per, dim, lens, ctx, sign):
+    """Row tiles in the order of their chains, in one turn, two and more; groups
+    of waves that share out the keys of their rows."""
+    test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign)
+
+
+def test_prefill_groups_without_keys():
+    test_prefill_rows_without_keys(128, [700, 90, 5], [100, 660, 0], 8, 4)
+
+
+@pytest.mark.parametrize("opts", ["cap", "head scales", "window", "sink"])
+@pytest.mark.parametrize("lens,ctx,kv_heads,per,window", [
+    ([400, 390], [260, 30], 8, 4, 630),              # waves in two groups
+    ([30, 9, 128], [600, 0, 1], 2, 4, 700),          # few rows: up to 768 keys
+    ([130], [900], 4, 4, 640),
+])
+def test_prefill_options_of_forms(lens, ctx, kv_heads, per, window, opts):
+    name = opts + str(window)
+    OPTIONS[name] = dict(OPTIONS[opts])
+    if "window" in OPTIONS[name]:
+        OPTIONS[name].update(window=window, keep_first=9)
+    try:
+        test_options(128, False, lens, ctx, kv_heads, per, False, name)
+    finally:
+        del OPTIONS[name]
+
+
 def test_prefill_without_prompts():
     """cu_q of one entry, or of none, names no rows: out stays as it is."""
     rows, k, v, table = make([300], [0], 1, 4, 128, 34)

@@ -126,12 +126,12 @@ template <typename T>
 void launch_gated_group_norm(T*, const float*, const float*, int, const T*,
                              long, float, int, int, int, int, int,
                              long, hipStream_t);
-int paged_attn_parts(bool, long, int, int, int, long, int, int, bool);
+long paged_attn_scratch(bool, long, int, int, int, int, long, int, int, bool);
 bool paged_attn_small(bool, long, int, int, int, int, long, int, int, bool);
-void launch_paged_attn(void*, long, bool, float*, float*, const unsigned short*,
+void launch_paged_attn(void*, long, bool, float*, const unsigned short*,
                        const unsigned short*, const unsigned short*, const int*,
                        const int*, const int*, long, int, int, int, int, int,
-                       float, float, long, int, int, const float*, int,
+                       float, float, long, int, const float*, int,
                        const float*, bool, hipStream_t);
 int capped_attn_mfma_class(int D, int Dv);
 void launch_capped_attn_mfma(void*, long, int, float*, float*, const unsigned short*,
@@ -1150,24 +1150,16 @@ void capped_attn(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache,
                             block_tables.size(1), window, keep_first, cap > 0) &&
       reinterpret_cast<uintptr_t>(k_cache.data_ptr()) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(v_cache.data_ptr()) % 16 == 0) {
-    const int n_part =
-        hy::paged_attn_parts(cu == nullptr, T, n_seqs, heads, n_kv,
-                             block_tables.size(1), window, keep_first,
-                             cap > 0);
-    Tensor ws;                 // [T * heads][parts][D + 2], and counters
-    float *ws_o = nullptr, *ws_ml = nullptr;
-    if (n_part > 1) {
-      const long n = (long)T * heads * n_part;
-      ws = torch::empty({n * (D + 2) + 2L * n_seqs * n_kv}, out.options().dtype(torch::kFloat));
-      ws_o = ptr<float>(ws);
-      ws_ml = ws_o + n * D;
-    }
+    const long need = hy::paged_attn_scratch(
+        cu == nullptr, T, n_seqs, heads, n_kv, D, block_tables.size(1), window,
+        keep_first, cap > 0);
+    Tensor ws;
+    if (need > 0) ws = torch::empty({need}, out.options().dtype(torch::kFloat));
     hy::launch_paged_attn(
-        out.data_ptr(), out_stride, !out_bf, ws_o, ws_ml, ptr<bf>(q),
-        ptr<bf>(k_cache), ptr<bf>(v_cache), ptr<int>(block_tables), cu,
+        out.data_ptr(), out_stride, !out_bf, need > 0 ? ptr<float>(ws) : nullptr,
+        ptr<bf>(q), ptr<bf>(k_cache), ptr<bf>(v_cache), ptr<int>(block_tables), cu,
         ptr<int>(seq_lens), T, n_seqs, heads, n_kv, D, block_tables.size(1),
-        scale, cap, q.stride(0), n_part, window, sinkp, keep_first, hsp,
-        chunked, cur());
+        scale, cap, q.stride(0), window, sinkp, keep_first, hsp, chunked, cur());
     return;
   }
   if (rows16 && hy::capped_attn_mfma_class(D, Dv) != 0) {

@@ -2,7 +2,7 @@
 // value width 64 or 128: the kernels of the dense decoders (../ops/paged_rows.h,
 // ../ops/paged_stream.h) with their options, the softmax weights in 32 bits.
 // Other widths and pages: capped_attn_mfma.hip.
-#include "../ops/paged_rows.h"
+#include "../ops/paged_short.h"
 #include "../ops/paged_stream.h"
 
 namespace xllm {
@@ -24,13 +24,18 @@ static long seen_pages(long max_blocks, int window, int keep_first) {
                        (window + 15) / 16 + (keep_first + 15) / 16 + 2);
 }
 
-// Room for parts the keys are split into. cu_q null: decoded rows.
-int paged_attn_parts(bool decode, long tokens, int n_seqs, int heads, int n_kv,
-                     long max_blocks, int window, int keep_first, bool capped) {
+// Floats of scratch that a call asks for. cu_q null: decoded rows.
+long paged_attn_scratch(bool decode, long tokens, int n_seqs, int heads, int n_kv,
+                        int D, long max_blocks, int window, int keep_first,
+                        bool capped) {
+  if (tokens == 0 || n_seqs <= 0) return 0;
   max_blocks = seen_pages(max_blocks, window, keep_first);
-  return decode ? paged_stream_split(n_seqs, n_kv, max_blocks, true, capped).parts
-                : paged_rows_parts(tokens, n_seqs, heads / n_kv, n_kv,
-                                   max_blocks, 3);
+  if (!decode)
+    return paged_prompts(tokens, n_seqs, heads / n_kv, n_kv, D, max_blocks, 3,
+                         true).scratch;
+  const int parts =
+      paged_stream_split(n_seqs, n_kv, max_blocks, true, capped).parts;
+  return parts > 1 ? tokens * heads * parts * (D + 2) + 2L * n_seqs * n_kv : 0;
 }
 
 // Whether the kernels of capped_attn_mfma.hip are faster: they have 16 rows a wave
@@ -80,31 +85,37 @@ bool paged_attn_small(bool decode, long tokens, int n_seqs, int heads, int n_kv,
 
 // out [tokens, heads * D] rows of out_stride, fp32 or bf16; q rows, caches and
 // out 16 B aligned (a bf16 out 8 B); decode: at most 32 heads per key head
-void launch_paged_attn(void* out, long out_stride, bool out_f32, float* ws_o,
-                       float* ws_ml, const unsigned short* q,
+void launch_paged_attn(void* out, long out_stride, bool out_f32, float* ws,
+                       const unsigned short* q,
                        const unsigned short* k_cache,
                        const unsigned short* v_cache, const int* block_tables,
                        const int* cu_q, const int* seq_lens, long tokens,
                        int n_seqs, int heads, int n_kv, int D, int max_blocks,
-                       float scale, float cap, long q_stride, int n_part,
-                       int window, const float* sink, int keep_first,
+                       float scale, float cap, long q_stride, int window, const float* sink, int keep_first,
                        const float* head_scale, bool chunked, hipStream_t st) {
   const PagedMore x =
       more_of(out_f32, cap, window, sink, keep_first, head_scale, chunked);
+  if (tokens == 0 || n_seqs <= 0) return;
+  const long seen = seen_pages(max_blocks, window, keep_first);
   if (cu_q == nullptr) {
     auto go = D == 128 ? paged_stream<128, 3, true> : paged_stream<64, 3, true>;
-    go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, seq_lens, n_seqs,
-       scale, heads, n_kv, max_blocks, q_stride, out_stride,
-       paged_stream_split(n_seqs, n_kv,
-                          seen_pages(max_blocks, window, keep_first), true,
-                          cap > 0),
-       x, st);
-  } else {
-    auto go = D == 128 ? paged_rows<128, 3, true> : paged_rows<64, 3, true>;
-    go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, cu_q, seq_lens,
-       tokens, n_seqs, scale, heads, n_kv, max_blocks, q_stride, out_stride,
-       n_part, x, st);
+    const PagedSplit split = paged_stream_split(n_seqs, n_kv, seen, true, cap > 0);
+    go(out, ws, ws + tokens * heads * split.parts * D, q, k_cache, v_cache,
+       block_tables, seq_lens, n_seqs, scale, heads, n_kv, max_blocks, q_stride,
+       out_stride, split, x, st);
+    return;
   }
+  const PagedPrompts p =
+      paged_prompts(tokens, n_seqs, heads / n_kv, n_kv, D, seen, 3, true);
+  if (p.few) {
+    auto go = D == 128 ? paged_short<128, 3, true> : paged_short<64, 3, true>;
+    go(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
+       scale, heads, n_kv, max_blocks, q_stride, out_stride, x, st);
+    return;
+  }
+  auto go = D == 128 ? paged_rows<128, 3, true> : paged_rows<64, 3, true>;
+  go(out, ws, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
+     scale, heads, n_kv, max_blocks, q_stride, out_stride, p, x, st);
 }
 
 }  // namespace hyb

@@ -45,12 +45,12 @@ void launch_paged_attn_decode(unsigned short*, const unsigned short*,
                               int, int, int, int, int, long, long, bool,
                               hipStream_t);
 int paged_attn_decode_parts(int, int, int, int);
-int paged_attn_prefill_parts(long, int, int, int, int, int);
-void launch_paged_attn_prefill(unsigned short*, float*, float*,
+long paged_attn_prefill_scratch(long, int, int, int, int, int);
+void launch_paged_attn_prefill(unsigned short*, float*, const unsigned short*,
                                const unsigned short*, const unsigned short*,
-                               const unsigned short*, const int*, const int*,
-                               const int*, long, int, float, int, int, int,
-                               int, long, long, int, hipStream_t);
+                               const int*, const int*, const int*, long, int,
+                               float, int, int, int, int, long, long,
+                               hipStream_t);
 void launch_greedy_sample(long*, const unsigned short*, int, int, hipStream_t);
 void launch_mfma_gemm(unsigned short*, const unsigned short*,
                       const unsigned short*, const unsigned short*, int, int,
@@ -298,22 +298,16 @@ void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
   }
   for (auto* t : {&q, &k_cache, &v_cache})
     if (!on_bytes(*t, 16)) *t = t->clone(at::MemoryFormat::Contiguous);
-  const int n_part = xllm::paged_attn_prefill_parts(
+  const long need = xllm::paged_attn_prefill_scratch(
       tokens, n_seqs, n_qheads / n_kv, n_kv, D, block_tables.size(1));
-  torch::Tensor ws;            // [tokens * heads][parts][D + 2], fp32
-  float *ws_o = nullptr, *ws_ml = nullptr;
-  if (n_part > 1) {
-    const long n = tokens * n_qheads * n_part;
-    ws = torch::empty({n * (D + 2)}, q.options().dtype(torch::kFloat));
-    ws_o = ws.data_ptr<float>();
-    ws_ml = ws_o + n * D;
-  }
+  torch::Tensor ws;
+  if (need > 0) ws = torch::empty({need}, q.options().dtype(torch::kFloat));
   xllm::launch_paged_attn_prefill(
-      u16(out), ws_o, ws_ml, u16c(q), u16c(k_cache), u16c(v_cache),
-      block_tables.data_ptr<int>(), cu_q.data_ptr<int>(),
-      seq_lens.data_ptr<int>(), tokens, n_seqs, (float)scale, n_qheads, n_kv,
-      D, block_tables.size(1), q.stride(0), out.stride(0), n_part,
-      cur_stream());
+      u16(out), need > 0 ? ws.data_ptr<float>() : nullptr, u16c(q),
+      u16c(k_cache), u16c(v_cache), block_tables.data_ptr<int>(),
+      cu_q.data_ptr<int>(), seq_lens.data_ptr<int>(), tokens, n_seqs,
+      (float)scale, n_qheads, n_kv, D, block_tables.size(1), q.stride(0),
+      out.stride(0), cur_stream());
 }
 
 torch::Tensor greedy_sample(torch::Tensor logits) {

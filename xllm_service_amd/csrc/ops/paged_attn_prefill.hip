@@ -7,16 +7,20 @@
 
 namespace xllm {
 
-int paged_attn_prefill_parts(long tokens, int n_seqs, int G, int n_kv, int D,
-                             int max_blocks) {
-  const int terms = D == 128 ? 1 : 3;
-  return paged_short_takes(tokens, n_seqs, G, n_kv, max_blocks, terms)
-             ? 1
-             : paged_rows_parts(tokens, n_seqs, G, n_kv, max_blocks, terms);
+static PagedPrompts prompts(long tokens, int n_seqs, int G, int n_kv, int D,
+                            int max_blocks) {
+  // 64-wide heads ran on fp32 weights before they had a kernel and still do
+  return paged_prompts(tokens, n_seqs, G, n_kv, D, max_blocks, D == 128 ? 1 : 3,
+                       false);
+}
+// floats of scratch that a call asks for
+long paged_attn_prefill_scratch(long tokens, int n_seqs, int G, int n_kv, int D,
+                                int max_blocks) {
+  if (tokens == 0 || n_seqs <= 0) return 0;
+  return prompts(tokens, n_seqs, G, n_kv, D, max_blocks).scratch;
 }
 
-// 64-wide heads ran on fp32 weights before they had a kernel and still do
-void launch_paged_attn_prefill(unsigned short* out, float* ws_o, float* ws_ml,
+void launch_paged_attn_prefill(unsigned short* out, float* ws,
                                const unsigned short* q,
                                const unsigned short* k_cache,
                                const unsigned short* v_cache,
@@ -24,26 +28,28 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws_o, float* ws_ml,
                                const int* seq_lens, long tokens, int n_seqs,
                                float scale, int n_qheads, int n_kv, int D,
                                int max_blocks, long q_stride, long out_stride,
-                               int n_part, hipStream_t stream) {
+                               hipStream_t stream) {
   if (tokens == 0 || n_seqs <= 0) return;
-  if (paged_short_takes(tokens, n_seqs, n_qheads / n_kv, n_kv, max_blocks,
-                        D == 128 ? 1 : 3)) {
-    auto go = D == 128 ? paged_short<128, 1> : paged_short<64, 3>;
+  const int G = n_qheads / n_kv;
+  const PagedPrompts p = prompts(tokens, n_seqs, G, n_kv, D, max_blocks);
+  if (p.few) {
+    auto go = D == 128 ? paged_short<128, 1, false> : paged_short<64, 3, false>;
     go(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
-       scale, n_qheads, n_kv, max_blocks, q_stride, out_stride, stream);
+       scale, n_qheads, n_kv, max_blocks, q_stride, out_stride, PagedMore{},
+       stream);
     return;
   }
-  if (D == 128 && n_part == 1 &&
-      paged_long_takes(tokens, n_seqs, n_qheads / n_kv, n_kv, max_blocks)) {
+  if (D == 128 && p.parts == 1 &&
+      paged_long_takes(tokens, n_seqs, G, n_kv, max_blocks)) {
     paged_long(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens,
                n_seqs, scale, n_qheads, n_kv, max_blocks, q_stride, out_stride,
                stream);
     return;
   }
   auto go = D == 128 ? paged_rows<128, 1, false> : paged_rows<64, 3, false>;
-  go(out, ws_o, ws_ml, q, k_cache, v_cache, block_tables, cu_q, seq_lens,
-     tokens, n_seqs, scale, n_qheads, n_kv, max_blocks, q_stride, out_stride,
-     n_part, PagedMore{}, stream);
+  go(out, ws, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
+     scale, n_qheads, n_kv, max_blocks, q_stride, out_stride, p, PagedMore{},
+     stream);
 }
 
 // ---------------------------------------------------------------------------------

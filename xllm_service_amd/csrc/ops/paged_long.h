@@ -26,62 +26,6 @@ namespace xllm {
 #define PL_ROWS 256        // rows per workgroup
 #define PL_BUFS 4          // tiles of K and V in LDS
 
-// Row tile `b` of the batch, the longest chains of keys first whatever their
-// sequences: a tile of a sequence has PL_ROWS rows (of query and head) fewer before it
-// than the next one, so all tiles sort into levels of that width with one tile
-// of a sequence to a level. A lane counts the tiles of a level, 64 levels at a time.
-// Up to 64 sequences; of more, one sequence after the other (pf_locate). Without this
-// 4200 new tokens before 100 behind 3000 cached ones were 4% slower than with the
-// kernel of paged_rows.h.
-XLLM_DEV bool pl_locate(int b, const int* cu_q, const int* seq_lens, int n_seqs,
-                        int G, int lane, PfPlace* place) {
-  if (n_seqs > 64)
-    return pf_locate<PL_ROWS>(b, cu_q, seq_lens, n_seqs, G, lane, place);
-  int start = 0, len = 0, keys = 0;              // of sequence `lane`
-  if (lane < n_seqs) {
-    start = cu_q[lane];
-    len = cu_q[lane + 1] - start;
-    keys = seq_lens[lane];
-  }
-  const int nt = (len * G + PL_ROWS - 1) / PL_ROWS, top = keys * G;
-  int most = nt > 0 ? top : 0;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, 64));
-  const int first = (most - top) / PL_ROWS, last = first + nt;   // its levels
-  int levels = nt > 0 ? last : 0;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-    levels = max(levels, __shfl_xor(levels, off, 64));
-  int acc = 0;
-  for (int base = 0; base < levels; base += 64) {
-    int c = 0;
-    for (int i = 0; i < n_seqs; i++)
-      c += base + lane >= __builtin_amdgcn_readlane(first, i) &&
-           base + lane < __builtin_amdgcn_readlane(last, i);
-    int sum = c;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int up = __shfl_up(sum, off, 64);
-      if (lane >= off) sum += up;
-    }
-    const unsigned long long hit = __ballot(b < acc + sum);
-    if (hit != 0) {
-      const int l = __ffsll(hit) - 1, level = base + l;
-      int r = b - acc - (__shfl(sum, l, 64) - __shfl(c, l, 64));
-      unsigned long long at = __ballot(level >= first && level < last);
-      for (; r > 0; r--) at &= at - 1;
-      const int i = __builtin_amdgcn_readfirstlane(__ffsll(at) - 1);
-      *place = {i, __builtin_amdgcn_readlane(last, i) - 1 - level,
-                __builtin_amdgcn_readlane(start, i),
-                __builtin_amdgcn_readlane(len, i),
-                __builtin_amdgcn_readlane(keys, i)};
-      return true;
-    }
-    acc += __shfl(sum, 63, 64);
-  }
-  return false;
-}
-
 __global__ __launch_bounds__(512) void paged_attn_long_kernel(
     unsigned short* __restrict__ out,        // [total_q, n_qheads, D]
     const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
@@ -108,8 +52,10 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
   const int h = lane >> 5, c32 = lane & 31;
 
   const int kvh = blockIdx.x % n_kv;
+  int unit;
   PfPlace place;
-  if (!pl_locate(blockIdx.x / n_kv, cu_q, seq_lens, n_seqs, G, lane, &place))
+  if (!pf_longest<PL_ROWS, 1>(blockIdx.x / n_kv, 1, INT_MAX / 2, cu_q, seq_lens,
+                           n_seqs, G, lane, &place, &unit))
     return;
   const int seq = place.seq, lt = place.lt, q_start = place.q_start,
             q_len = place.q_len, seq_len = place.seq_len;

@@ -89,6 +89,33 @@ XLLM_DEV void paged_cap(f32x16 (&s)[N], float pre, float cap) {
     }
 }
 
+// Scores of keys that a row does not see are -inf: those from `limit` on and those below
+// lo but for the first keep_first. key(r): of entry r. Without kept keys that is one
+// comparison; written with || the compiler branched around each of the entries.
+template <bool MORE, int N, class Key>
+XLLM_DEV void paged_mask(const PagedMore& x, f32x16 (&s)[N], int limit, int lo,
+                         const Key& key) {
+  if (!MORE || x.keep_first <= 0) {
+    const unsigned span = (unsigned)max(limit - (MORE ? lo : 0), 0);
+#pragma unroll
+    for (int i = 0; i < N; i++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const unsigned at = (unsigned)(key(i, r) - (MORE ? lo : 0));
+        s[i][r] = at < span ? s[i][r] : -INFINITY;
+      }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < N; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int k = key(i, r);
+      const bool on = (k < limit) & ((k >= lo) | (k < x.keep_first));
+      s[i][r] = on ? s[i][r] : -INFINITY;
+    }
+}
+
 // Decoded rows: parts that a list of n tiles is really split into, of the P that
 // the host, which does not know the lengths, made room for: one for every `per` tiles,
 // of up to eight one for every `near`

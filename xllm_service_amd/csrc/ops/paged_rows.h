@@ -47,6 +47,9 @@
 //
 // Fragment layouts, the order of the keys and of the LDS images: mfma_rows.h.
 #pragma once
+#include <algorithm>
+#include <climits>
+
 #include "paged_merge.h"
 
 namespace xllm {
@@ -96,11 +99,90 @@ XLLM_DEV bool pf_locate(int b, const int* cu_q, const int* seq_lens, int n_seqs,
   return false;
 }
 
+// Sums (maxima) of the lanes up to and with this one, on the vector unit alone
+template <bool SUM>
+XLLM_DEV int pf_scan(int v) {
+#define PF_STEP(CTRL, ROWS)                                                    \
+  {                                                                            \
+    const int u = __builtin_amdgcn_update_dpp(SUM ? 0 : INT_MIN, v, CTRL, ROWS, \
+                                              0xf, false);                     \
+    v = SUM ? v + u : max(v, u);                                               \
+  }
+  PF_STEP(0x111, 0xf) PF_STEP(0x112, 0xf) PF_STEP(0x114, 0xf)   // row_shr
+  PF_STEP(0x118, 0xf)
+  PF_STEP(0x142, 0xa) PF_STEP(0x143, 0xc)                       // row_bcast
+#undef PF_STEP
+  return v;
+}
+
+// Row tile `b` of the batch, the longest chains of keys first whatever their
+// sequences: a tile of a sequence has ROWS rows (of query and head) fewer before it
+// than the next one, so all tiles sort into levels of WIDTH of those with at most
+// WIDTH tiles of a sequence to a level, which share its keys and stay together. The level
+// of tile b is found by halves, a lane counting its sequence's tiles above one. Up to 64
+// sequences; of more, one sequence after the other (pf_locate).
+//   units: b is one of so many per tile (parts), of which those past the first `turn` come
+// in the reverse order if they are no more than another `turn`: two workgroups share a
+// CU then, and the longest chains meet the shortest. By sequences, the tiles of two
+// equal prompts met their likes: 2 x 1.8-2.3 k in a window of 1024 59.5 -> 54.8 us, 4 x 512
+// of 32/8 heads 28.3 -> 22.8, 3 x 500 capped 51.5 -> 40.2. WIDTH 1, 2 and 4: 40 x 60 behind
+// 500, whose two tiles read the same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500 and
+// 300 of 64-wide heads 26.6, 26.6, 27.6.
+template <int ROWS, int WIDTH>
+XLLM_DEV bool pf_longest(int b, int units, int turn, const int* cu_q,
+                         const int* seq_lens, int n_seqs, int G, int lane,
+                         PfPlace* place, int* unit) {
+  if (n_seqs > 64) {
+    *unit = b % units;
+    return pf_locate<ROWS>(b / units, cu_q, seq_lens, n_seqs, G, lane, place);
+  }
+  int start = 0, len = 0, keys = 0;              // of sequence `lane`
+  if (lane < n_seqs) {
+    start = cu_q[lane];
+    len = cu_q[lane + 1] - start;
+    keys = seq_lens[lane];
+  }
+  const int nt = (len * G + ROWS - 1) / ROWS, top = keys * G;
+  const int most = __builtin_amdgcn_readlane(
+      pf_scan<false>(nt > 0 ? top : INT_MIN), 63);
+  const int total = __builtin_amdgcn_readlane(pf_scan<true>(nt), 63) * units;
+  if (b >= total) return false;
+  if (b >= turn && total <= 2 * turn) b = turn + total - 1 - b;
+  *unit = b % units;
+  b /= units;
+  // its tiles from the top: [first, first + nt)
+  const int first = nt > 0 ? (most - top) / ROWS : 0;
+  const int depth = __builtin_amdgcn_readlane(pf_scan<false>(first + nt), 63);
+  const int deepest = (depth - 1) / WIDTH;       // level, in tiles; tiles over it
+  int level = 0, above = 0;
+  for (int step = deepest > 0 ? 1 << (31 - __builtin_clz(deepest)) : 0; step > 0;
+       step >>= 1) {
+    const int mine = level + step * WIDTH;
+    const int c = __builtin_amdgcn_readlane(
+        pf_scan<true>(min(max(mine - first, 0), nt)), 63);
+    if (c <= b) level = mine, above = c;         // uniform
+  }
+  // sequence `lane`'s tiles over the level, and with those in it
+  const int over = min(max(level - first, 0), nt);
+  const int with = min(max(level + WIDTH - first, 0), nt);
+  const int upto = pf_scan<true>(with - over);
+  const int r = b - above;
+  const int i = __builtin_amdgcn_readfirstlane(__ffsll(__ballot(r < upto)) - 1);
+  const int k = r - __builtin_amdgcn_readlane(upto - with, i);
+  *place = {i, __builtin_amdgcn_readlane(nt, i) - 1 - k,
+            __builtin_amdgcn_readlane(start, i),
+            __builtin_amdgcn_readlane(len, i),
+            __builtin_amdgcn_readlane(keys, i)};
+  return true;
+}
+
 // TERMS: bf16 terms a softmax weight is split into. One rounds it to bf16;
 // three (8 + 8 + 8 mantissa bits) hold all of its 32-bit value, each with a
 // product of its own into the same fp32 sums. MORE: the options of PagedMore.
-template <int D, int TERMS, bool MORE>
-__global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
+// KG: groups of four waves, each with the same rows and its share of the tiles: what
+// splitting keys over workgroups does, without partial results in memory.
+template <int D, int TERMS, bool MORE, int KG>
+__global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     void* __restrict__ out,                  // [total_q, n_qheads, D]
     float* __restrict__ ws_o,                // [total_q*n_qheads][n_part][D]
     float* __restrict__ ws_ml,               // [total_q*n_qheads][n_part][2]
@@ -119,18 +201,21 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
   constexpr int RPI = 64 / CPR;              // rows one load instruction fills
   constexpr int NI = 16 / RPI;               // ... instructions per page
   constexpr int TILE = PF_KT * D;            // elements of a K or V tile
-  __shared__ __attribute__((aligned(1024))) unsigned short kv_lds[4 * TILE];
+  __shared__ __attribute__((aligned(1024))) unsigned short
+      kv_lds[KG * 4 * TILE];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wid = wave & 3, kg = KG > 1 ? wave >> 2 : 0;
   const int h = lane >> 5, c32 = lane & 31;
 
   const int kvh = blockIdx.x % n_kv;
-  const int part = (blockIdx.x / n_kv) % n_part;
+  int part;
   PfPlace at;
-  if (!pf_locate<PF_ROWS>(blockIdx.x / (n_kv * n_part), cu_q, seq_lens, n_seqs, G,
-                          lane, &at))
+  if (!pf_longest<PF_ROWS, 2>(blockIdx.x / n_kv, n_part,
+                              KG > 1 ? INT_MAX / 2 : 256 / n_kv, cu_q, seq_lens,
+                              n_seqs, G, lane, &at, &part))
     return;
   const int seq = at.seq, lt = at.lt, q_start = at.q_start, q_len = at.q_len,
             seq_len = at.seq_len;
@@ -146,8 +231,9 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
   // parts of at least four tiles; the rest of them stay empty
   const int parts = min(n_part, (list.n + 3) / 4);
   const int tpp = parts > 0 ? (list.n + parts - 1) / parts : 0;
-  const int i_begin = part * tpp;
-  const int i_end = min(list.n, i_begin + tpp);
+  const int p_begin = part * tpp;
+  const int i_end = min(list.n, p_begin + tpp);
+  const int i_begin = p_begin + kg;              // every KG-th of a group's
 
   // ---- this lane's row -----------------------------------------------------
   const int wrow0 = row0 + wid * 32;
@@ -195,11 +281,12 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
     koff[i] = off_of(r, r, false);
     voff[i] = off_of(r, r, true);
   }
-  // ids of this wave's pages of 64 tiles from the tb-th on, one per lane: a
+  // ids of this wave's pages of 64 of its tiles, one per lane: a
   // scalar load per tile would make every wait for LDS a wait for it too
-  int tb = i_begin;
-  auto pages_from = [&](int i) {
-    return btab[min(list.at(i + lane) * (PF_KT / PF_BS) + wid, last_blk)];
+  int tb = 0;                                    // from this one on
+  auto pages_from = [&](int n) {
+    return btab[min(list.at(i_begin + (n + lane) * KG) * (PF_KT / PF_BS) + wid,
+                    last_blk)];
   };
   auto put = [&](__amdgpu_buffer_rsrc_t kp, __amdgpu_buffer_rsrc_t vp,
                  unsigned ko, unsigned vo, unsigned short* dst) {
@@ -211,7 +298,7 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
     const long base = ((long)page * n_kv + kvh) * (PF_BS * D);
     const auto kp = mr_buffer(k_cache + base, PF_BS * D * 2);
     const auto vp = mr_buffer(v_cache + base, PF_BS * D * 2);
-    unsigned short* dst = kv_lds + buf * 2 * TILE + wid * 16 * D;
+    unsigned short* dst = kv_lds + (kg * 2 + buf) * 2 * TILE + wid * 16 * D;
     if (pg < last_blk) {
 #pragma unroll
       for (int i = 0; i < NI; i++)
@@ -231,25 +318,27 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
 
   int pages = 0;
   if (i_begin < i_end) {
-    pages = pages_from(i_begin);
+    pages = pages_from(0);
     stage(list.at(i_begin), __builtin_amdgcn_readlane(pages, 0), 0);
   }
-  for (int it = i_begin; it < i_end; it++) {
-    const int buf = (it - i_begin) & 1;
+  // a step: a tile of every group, the last of which may have none left
+  for (int at = p_begin, n = 0; at < i_end; at += KG, n++) {
+    const int buf = n & 1, it = at + kg;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (it + 1 < i_end) {
-      if (it + 1 - tb == 64) {
+    if (it + KG < i_end) {
+      if (n + 1 - tb == 64) {
         tb += 64;
         pages = pages_from(tb);
       }
-      stage(list.at(it + 1), __builtin_amdgcn_readlane(pages, it + 1 - tb),
+      stage(list.at(it + KG), __builtin_amdgcn_readlane(pages, n + 1 - tb),
             buf ^ 1);
     }
+    if (KG > 1 && it >= i_end) continue;
     const int k0 = list.at(it) * PF_KT;
     if (!wave_on || k0 >= wmax) continue;
     if (MORE && k0 + PF_KT <= wlo && k0 >= x.keep_first) continue;
-    const lds_u16* kt = (const lds_u16*)kv_lds + buf * 2 * TILE;
+    const lds_u16* kt = (const lds_u16*)kv_lds + (kg * 2 + buf) * 2 * TILE;
     const lds_u16* vt = kt + TILE;
 
     // ---- scores: keys [32 i, 32 i + 32) of the tile ------------------------
@@ -274,14 +363,9 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
     if (MORE && x.cap > 0.0f) paged_cap<2>(s, sc.pre, x.cap);
     // uniform: a tile on the diagonal or on the edge of a window
     if (k0 + PF_KT > wmin || (MORE && k0 < whi)) {
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          const int key = k0 + i * 32 + mr_key_of(r, h);
-          if (key >= limit || (MORE && key < lo && key >= x.keep_first))
-            s[i][r] = -INFINITY;
-        }
+      paged_mask<MORE>(x, s, limit, lo, [&](int i, int r) {
+        return k0 + i * 32 + mr_key_of(r, h);
+      });
     }
     // ---- online softmax: weights are 2^(c (s - m)) ---------------------------
     const float c = sc.c;
@@ -333,76 +417,146 @@ __global__ __launch_bounds__(256, 2) void paged_attn_rows_kernel(
 
   // ---- epilogue: o_acc[dt][r] = O[row][dt*32 + 8*(r>>2) + 4h + (r&3)] --------
   l = pair_sum(l);
+  m = m == -INFINITY ? m : m * sc.c;
+  constexpr int OWN = DT / KG;                   // column tiles a group finishes
+  const int dt0 = kg * OWN;
+  if constexpr (KG > 1) {
+    // the groups swap halves of their sums
+    __syncthreads();
+    f32x4* swap = reinterpret_cast<f32x4*>(kv_lds);   // [8 waves][OWN][4][64]
+    float2* ml = reinterpret_cast<float2*>(swap + 8 * OWN * 4 * 64);   // [8][32]
+    if (h == 0) ml[wave * 32 + c32] = make_float2(m, l);
+#pragma unroll
+    for (int j = 0; j < OWN; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const f32x16 o = kg ? o_acc[j] : o_acc[OWN + j];
+        swap[((wave * OWN + j) * 4 + r) * 64 + lane] =
+            f32x4{o[4 * r], o[4 * r + 1], o[4 * r + 2], o[4 * r + 3]};
+      }
+    __syncthreads();
+    const float2 z = ml[(wave ^ 4) * 32 + c32];
+    // a group without tiles has no part in the row
+    const bool mine = i_begin < i_end, other = p_begin + (kg ^ 1) < i_end;
+    float top = fmaxf(m, z.x);                   // which skips a NaN
+    if (m != m || z.x != z.x) top = NAN;
+    const float to = top == -INFINITY ? 0.0f : top;
+    const float f = mine ? __builtin_amdgcn_exp2f(m - to) : 0.0f;
+    const float g = other ? __builtin_amdgcn_exp2f(z.x - to) : 0.0f;
+    l = (mine ? l * f : 0.0f) + (other ? z.y * g : 0.0f);
+    m = top;
+#pragma unroll
+    for (int j = 0; j < OWN; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const f32x4 y = swap[(((wave ^ 4) * OWN + j) * 4 + r) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float x = kg ? o_acc[OWN + j][4 * r + e] : o_acc[j][4 * r + e];
+          o_acc[j][4 * r + e] =
+              (mine ? x * f : 0.0f) + (other ? y[e] * g : 0.0f);
+        }
+      }
+  }
   if (!row_ok) return;
   const long grow = (long)(q_start + qi) * n_qheads + head;
   if (n_part == 1) {
     if (MORE && x.sink != nullptr)
-      l += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f -
-                                  m * sc.c);
+      l += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f - m);
     const float inv = l != 0.0f ? 1.0f / l : 0.0f;
     const long to = (long)(q_start + qi) * out_stride + (long)head * D + 4 * h;
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++)
+    for (int j = 0; j < OWN; j++)
 #pragma unroll
       for (int r = 0; r < 16; r += 4)
-        paged_put<MORE>(x, out, to + dt * 32 + 2 * r, o_acc[dt][r] * inv,
-                        o_acc[dt][r + 1] * inv, o_acc[dt][r + 2] * inv,
-                        o_acc[dt][r + 3] * inv);
+        paged_put<MORE>(x, out, to + (dt0 + j) * 32 + 2 * r, o_acc[j][r] * inv,
+                        o_acc[j][r + 1] * inv, o_acc[j][r + 2] * inv,
+                        o_acc[j][r + 3] * inv);
     return;
   }
   const long slot = grow * n_part + part;
-  if (h == 0) {
-    ws_ml[slot * 2] = m * sc.c;
-    ws_ml[slot * 2 + 1] = i_begin < i_end ? l : PAGED_ABSENT;
+  if (h == 0 && kg == 0) {
+    ws_ml[slot * 2] = m;
+    ws_ml[slot * 2 + 1] = p_begin < i_end ? l : PAGED_ABSENT;
   }
-  if (i_begin >= i_end) return;
+  if (p_begin >= i_end) return;
   float* o = ws_o + slot * D + 4 * h;
 #pragma unroll
-  for (int dt = 0; dt < DT; dt++)
+  for (int j = 0; j < OWN; j++)
 #pragma unroll
     for (int r = 0; r < 16; r += 4)
-      *reinterpret_cast<float4*>(o + dt * 32 + 2 * r) =
-          make_float4(o_acc[dt][r], o_acc[dt][r + 1], o_acc[dt][r + 2],
-                      o_acc[dt][r + 3]);
+      *reinterpret_cast<float4*>(o + (dt0 + j) * 32 + 2 * r) =
+          make_float4(o_acc[j][r], o_acc[j][r + 1], o_acc[j][r + 2],
+                      o_acc[j][r + 3]);
 }
 
-// Row tiles a batch has at most, and the parts its keys are split into: about
-// two workgroups per CU are wanted, and parts of at least eight tiles of keys
-// (four with 32-bit weights, whose tiles take twice as long): the merge costs
-// more than smaller ones save. Measured (us, by parts 1 | 2 | 4 | 8), 32-bit
-// weights: 2 x 64 rows of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of 16
-// over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles) 374 | 298 |
-// 302 | 325; 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
+// Row tiles a batch has at most
 template <int ROWS>
 inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
-  return tokens * G / ROWS + n_seqs;
+  return (tokens * G + n_seqs * (ROWS - 1L)) / ROWS;
 }
-inline int paged_rows_parts(long tokens, int n_seqs, int G, int n_kv,
-                            long max_blocks, int terms) {
+// Groups of waves, and parts of the keys. Parts: about two workgroups per CU are wanted,
+// and parts of at least eight tiles of keys (four with 32-bit weights, whose tiles take
+// twice as long): the merge costs more than smaller ones save. Measured (us, by parts 1 | 2 |
+// 4 | 8), 32-bit weights: 2 x 64 rows of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of
+// 16 over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles) 374 | 298 | 302 | 325;
+// 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
+//   Two groups of waves instead where they fill one turn of the CUs, as one part: 128-wide
+// heads, up to 24 tiles, or for a single sequence that fills most of the CUs; us, as before
+// (parts) | two groups: 1024 tokens of 32/8 heads 34.5 (2) | 25.5, 28/4 32.5 (2) | 24.8, 3 x
+// 300 behind 1000 44 (2) | 33, 1000 behind 1000 49.5 (2) | 42.2, 700 20.9 (1) | 20.0, but 300
+// 13.2 (1) | 14.1; 300 behind 1000, 28/4 (66 workgroups) 27.3 | 28.5, 16/4 1000 behind 1000
+// (125) 34.9 (4) | 37.5; and one prompt in up to 448 workgroups, whose chains differ: 1400
+// of 32/8 39 | 32.8, 2048 of 28/4 (448) 54.2 | 50, 32/8 (512) 55.5 | 56.4, 850 of 64/8 (14 tiles)
+// 29 | 31.4. 32-bit weights, 2 x 400 behind 500 of 32/8 in a window 46.3 (2) | 33, capped 51.8 |
+// 40, but 300 behind 1000 (75) 37 (4) | 42, 2000 of 16/4 capped 71 (2) | 73.7. 64-wide, two
+// workgroups to a CU: 8 prompts of 64-448 13.3 (1) | 12.4, 1700 (168) 27.8 (3) | 32.7.
+// groups: KG; scratch: floats
+struct PagedRows { int parts = 1, groups = 1; long scratch = 0; };
+inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D,
+                                 long max_blocks, int terms) {
+  PagedRows x;
   const long wgs = paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv;
-  const long most = max_blocks * PF_BS / ((terms > 1 ? 4 : 8) * PF_KT);
-  long p = wgs > 0 ? (512 + wgs / 2) / wgs : 1;
-  if (p > most) p = most;
-  return (int)(p < 1 ? 1 : p > 16 ? 16 : p);
+  const long keys = max_blocks * PF_BS, tiles = keys / PF_KT;
+  const bool alone = n_seqs == 1 && 2 * keys < 3 * tokens;
+  if (D == 64)
+    x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 ? 2 : 1;
+  else if (terms > 1)
+    x.groups = keys >= 640 && tiles <= 20 && wgs >= 200 && wgs <= 256 ? 2 : 1;
+  else if (keys >= 640 && wgs >= 72)
+    x.groups = wgs <= 256 ? (tiles <= 24 || (n_seqs == 1 && wgs >= 200) ? 2 : 1)
+                          : (wgs <= 448 && alone && tiles >= 20 ? 2 : 1);
+  const long p = x.groups == 2 || wgs == 0 ? 1 : (512 + wgs / 2) / wgs;
+  const long most = keys / ((terms > 1 ? 4 : 8) * PF_KT);
+  x.parts = (int)std::max<long>(1, std::min<long>({p, most, 16}));
+  if (x.parts > 1) x.scratch = tokens * G * n_kv * x.parts * (D + 2);
+  return x;
 }
 
 // Prompt rows and the merge of their parts
 template <int D, int TERMS, bool MORE>
-inline void paged_rows(void* out, float* ws_o, float* ws_ml,
-                       const unsigned short* q, const unsigned short* k_cache,
+inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
+                       const unsigned short* k_cache,
                        const unsigned short* v_cache, const int* block_tables,
                        const int* cu_q, const int* seq_lens, long tokens,
                        int n_seqs, float scale, int n_qheads, int n_kv,
                        int max_blocks, long q_stride, long out_stride,
-                       int n_part, const PagedMore& x, hipStream_t stream) {
+                       const PagedRows& plan, const PagedMore& x,
+                       hipStream_t stream) {
+  const int n_part = plan.parts;
   const int G = n_qheads / n_kv;
   if (tokens == 0 || n_seqs <= 0) return;
+  float* ws_ml = ws_o + tokens * n_qheads * n_part * D;
   const dim3 grid(
       (unsigned)(paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv * n_part));
-  hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE>), grid, dim3(256),
-                     0, stream, out, ws_o, ws_ml, q, k_cache, v_cache,
-                     block_tables, cu_q, seq_lens, n_seqs, scale, G, n_kv,
-                     max_blocks, q_stride, out_stride, n_part, x);
+#define PF_GO(KG)                                                              \
+  hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG>), grid,       \
+                     dim3(KG * 256), 0, stream, out, ws_o, ws_ml, q, k_cache,  \
+                     v_cache, block_tables, cu_q, seq_lens, n_seqs, scale, G,  \
+                     n_kv, max_blocks, q_stride, out_stride, n_part, x)
+  if (plan.groups == 2) PF_GO(2);
+  else PF_GO(1);
+#undef PF_GO
   if (n_part > 1)
     paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, n_part, out_stride,
                          tokens * n_qheads, x, stream, cu_q, n_seqs);

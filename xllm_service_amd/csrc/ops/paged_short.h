@@ -10,8 +10,10 @@
 //
 // Bound by that chain and the launch. Measured (us, paged_rows.h, with its merge where
 // it splits | here): 300 tokens of 16/4 heads of 128 11.9 | 10.3, 512 of them
-// 16.0 | 10.7, 1000 of 8/1 25.1 | 14.9, 100 of 32/8 behind 800 22.8 | 14.6, 448 of
-// 12/12 heads of 64 12.7 | 8.8.
+// 16.8 | 11.7, 1000 of 8/1 25.1 | 14.9, 100 of 32/8 behind 800 22.8 | 14.6, 1000 of 12/12
+// heads of 64 19.8 | 14.6, 300 of 16/4 in a window 17.3 | 13.7, capped 22.2 | 16.1. What a CU
+// pulls (61 KB/us: each wave has tiles of its own) bounds longer chains: 64 rows a wave,
+// half as much to pull, were slower (300 tokens 17, 100 behind 4000 60 | 40 for 32 rows).
 #pragma once
 #include "paged_rows.h"
 
@@ -19,11 +21,11 @@ namespace xllm {
 
 #define PS_ROWS 32         // rows per workgroup
 #define PS_WAVES 4
-#define PS_KEYS 2048       // of a table, at most
+#define PS_KEYS 2048       // that a row sees, at most
 
-template <int D, int TERMS>
+template <int D, int TERMS, bool MORE>
 __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
-    unsigned short* __restrict__ out,        // [total_q, n_qheads, D]
+    void* __restrict__ out,                  // [total_q, n_qheads, D]
     const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
     const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
     const unsigned short* __restrict__ v_cache,
@@ -31,7 +33,8 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
     const int* __restrict__ cu_q,            // [num_seqs+1] query offsets
     const int* __restrict__ seq_lens,        // [num_seqs] total key len
     const int n_seqs, const float scale, const int G, const int n_kv,
-    const int max_blocks, const long q_stride, const long out_stride) {
+    const int max_blocks, const long q_stride, const long out_stride,
+    const PagedMore x) {
   constexpr int KS = D / 16;                 // k steps of a score product
   constexpr int DT = D / 32;                 // 32-wide tiles of the head
   constexpr int CPR = D / 8;                 // 16 B chunks of a row
@@ -65,9 +68,14 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
   const int limit = row_ok ? ctx + qi + 1 : 0;   // keys this row sees
   const int wmin = ctx + row0 / G + 1;           // fewest of a row
   const int kmax = ctx + (min(row0 + PS_ROWS, rows) - 1) / G + 1;
-  const int n = (kmax + PF_KT - 1) / PF_KT;      // tiles; this wave's: wid + 4 i
+  const PagedTiles list = paged_tiles<MORE>(x, wmin, kmax,
+                                            (kmax + PF_KT - 1) / PF_KT, PF_KT);
+  const int n = list.n;                          // this wave's tiles: wid + 4 i
+  // keys below lo are out of sight but for the kept ones
+  const int lo = paged_first<MORE>(x, row_ok ? limit : 1);
+  const int whi = paged_first<MORE>(x, kmax);
 
-  const PagedScore sc = paged_score<false>(PagedMore{}, scale, 0);
+  const PagedScore sc = paged_score<MORE>(x, scale, row_ok ? head : kvh * G);
   const float c = sc.c;
   // rows past the last one hold its query: their results go nowhere
   const int qr = min(rho, rows - 1), qq = qr / G;
@@ -96,19 +104,19 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
     voff[i] = (unsigned)(r * (2 * D) + ((spos ^ mr_swz_cols<D>(r)) << 4));
   }
   // Where the pages of this wave's tiles are, and how much of each is keys, one page
-  // per lane: 16 tiles, where a table of PS_KEYS keys has 8 for a wave and one past them
-  // is asked for. Rows past the last key, and tiles past the last one, are out of the
-  // bounds: zeros.
-  static_assert((PS_KEYS / PF_KT / PS_WAVES + 1) * PAGES <= 64, "pages per lane");
+  // per lane: 16 tiles, where a row that sees PS_KEYS keys has up to 9 for a wave and one
+  // past them is asked for. Rows past the last key, and tiles past the last one, are out
+  // of the bounds: zeros.
+  static_assert((PS_KEYS / PF_KT / PS_WAVES + 2) * PAGES <= 64, "pages per lane");
   unsigned at_lo = 0, at_hi = 0, bytes = 0;
   auto look_up = [&]() {
-    const int t = wid + PS_WAVES * (lane >> 2);
-    const int pg = min(t, n - 1) * PAGES + (lane & 3);
+    const int i = wid + PS_WAVES * (lane / PAGES);
+    const int pg = list.at(min(i, n - 1)) * PAGES + lane % PAGES;
     const long at =
         ((long)btab[min(pg, last_blk)] * n_kv + kvh) * (PF_BS * D * 2);
     at_lo = (unsigned)at;
     at_hi = (unsigned)(at >> 32);
-    bytes = t < n ? min(max(seq_len - pg * PF_BS, 0), PF_BS) * (D * 2) : 0;
+    bytes = i < n ? min(max(seq_len - pg * PF_BS, 0), PF_BS) * (D * 2) : 0;
     asm volatile("" : "+v"(at_lo), "+v"(at_hi), "+v"(bytes));   // waited for here
   };
   unsigned short* kv = kv_lds + wid * (2 * TILE);
@@ -117,11 +125,11 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
 #pragma unroll
     for (int p = 0; p < PAGES; p++) {
       const int at = i * PAGES + p;
-      const unsigned lo = __builtin_amdgcn_readlane(at_lo, at);
-      const unsigned hi = __builtin_amdgcn_readlane(at_hi, at);
+      const unsigned a = __builtin_amdgcn_readlane(at_lo, at);
+      const unsigned b = __builtin_amdgcn_readlane(at_hi, at);
       const auto src = mr_buffer(
           (const char*)(val ? v_cache : k_cache) +
-              (long)((unsigned long long)hi << 32 | lo),
+              (long)((unsigned long long)b << 32 | a),
           __builtin_amdgcn_readlane(bytes, at));
 #pragma unroll
       for (int k = 0; k < NI; k++)
@@ -150,7 +158,7 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
     stage(0, true);
   }
   for (int i = 0; wid + PS_WAVES * i < n; i++) {
-    const int k0 = (wid + PS_WAVES * i) * PF_KT;
+    const int k0 = list.at(wid + PS_WAVES * i) * PF_KT;
     arrived();                                   // keys
     f32x16 s[2] = {mr_zero(), mr_zero()};
 #pragma unroll
@@ -162,13 +170,12 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
                       qf[ks], s[j]);
     read();
     stage(i + 1, false);
-    if (k0 + PF_KT > wmin) {                     // uniform: a tile on the diagonal
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-          if (k0 + j * 32 + mr_key_of(r, h) >= limit) s[j][r] = -INFINITY;
-    }
+    if (MORE && x.cap > 0.0f) paged_cap<2>(s, sc.pre, x.cap);
+    // uniform: a tile on the diagonal or on the edge of a window
+    if (k0 + PF_KT > wmin || (MORE && k0 < whi))
+      paged_mask<MORE>(x, s, limit, lo, [&](int j, int r) {
+        return k0 + j * 32 + mr_key_of(r, h);
+      });
     // online softmax: weights are 2^(c (s - m))
     float mt = s[0][0];
 #pragma unroll
@@ -249,6 +256,8 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
                  : 0.0f;
     if (w < n) sum += z.y * f[w];
   }
+  if (MORE && x.sink != nullptr)
+    sum += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f - top);
   const float inv = sum != 0.0f ? 1.0f / sum : 0.0f;
   // a wave writes one (two) of every four pieces of its rows
   const long to = (long)(q_start + qi) * out_stride + (long)head * D + 4 * h;
@@ -259,45 +268,64 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
 #pragma unroll
     for (int w = 0; w < PS_WAVES; w++)
       if (w < n) o += part[((w * DT + dt) * 4 + r) * 64 + lane] * f[w];
-    paged_put<false>(PagedMore{}, out, to + dt * 32 + 8 * r, o[0] * inv,
-                     o[1] * inv, o[2] * inv, o[3] * inv);
+    paged_put<MORE>(x, out, to + dt * 32 + 8 * r, o[0] * inv, o[1] * inv,
+                    o[2] * inv, o[3] * inv);
   }
 }
 
-// One turn of workgroups (at 128 wide LDS holds one per CU) over tables of 128 to 2048
-// keys, half of that with 32-bit weights. More workgroups take a second turn for what
-// fewer waves do over the same keys (us, paged_rows.h | here): 300 tokens of 32/8 heads
-// (304 workgroups) 12.3 | 13.3, 900 of 12/12 of 64 (372) 10.2 | 10.5, 594 behind up to
-// 3000 keys (616) 50 | 68. In one or two tiles of keys there is nothing to share: 20
-// tokens 6.3 | 7.0, 64 of 64-wide heads 5.4 | 6.1. Longer tables go to more
-// workgroups there: 32 tokens of 28/4 heads behind 1000 keys 18.5 | 15.9, 100 of 32/8
-// behind 1600 22.0 | 20.5, but 32 behind 3000 21.9 | 29.4; 16 of 64-wide heads behind
-// 1000 11.9 | 12.0. From 1536 keys on, where there are three parts, only rows that fill
+// One turn of workgroups (at 128 wide LDS holds one per CU, at 64 two) over 128 to 2048
+// keys, half of that for 64-wide heads, 768 with options, where a tile takes twice as
+// long. More workgroups take a second turn for what fewer waves do over the same keys
+// (us, paged_rows.h | here): 300 tokens of 32/8 heads (304 workgroups) 12.3 | 13.3, in a
+// window 17.5 | 19.2, 8 prompts of 64-448 of 12/12 of 64 (764) 12.4 | 17.4, 594 behind up to
+// 3000 keys (616) 50 | 68; but 2 x 600 behind 200 (456) 22.3 | 16.5. In one or two tiles of keys
+// there is nothing to share: 20 tokens 6.3 | 7.0, 64 of 64-wide heads 5.4 | 6.1. Longer
+// tables go to more workgroups there: 32 tokens of 28/4 heads behind 1000 keys 18.5 | 15.9,
+// 100 of 32/8 behind 1600 22.0 | 20.5, but 32 behind 3000 21.9 | 29.4; 16 of 64-wide heads
+// behind 1000 11.9 | 12.0; 100 of 16/4 behind 1000, capped, 25.2 | 28.3, 30 of them in a window
+// of 1024 20.1 | 21.9. From 1536 keys on, where there are three parts, only rows that fill
 // a tile: 17 of 32/32 heads behind 1400 21.3 | 19.2, behind 1600 18.1 | 21.2, 60 of them
 // 22.7 | 19.3, 19.8 | 21.3; 30 of 16/4 (120 rows) behind 1600 19.1 | 19.7, 45 behind 1930
 // 21.8 | 21.7.
-inline bool paged_short_takes(long tokens, int n_seqs, int G, int n_kv,
-                              long max_blocks, int terms) {
+inline bool paged_short_takes(long tokens, int n_seqs, int G, int n_kv, int D,
+                              long max_blocks, bool options) {
   const long keys = max_blocks * PF_BS;
-  return paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv <= 256 &&
-         keys >= 128 && keys <= (terms > 1 ? PS_KEYS / 2 : PS_KEYS) &&
+  return paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv <=
+             (D == 64 ? 512 : 256) &&
+         keys >= 128 &&
+         keys <= (options ? 768 : D == 64 ? PS_KEYS / 2 : PS_KEYS) &&
          (keys < 1536 || tokens * G >= (long)PF_ROWS * n_seqs);
 }
 
-template <int D, int TERMS>
-inline void paged_short(unsigned short* out, const unsigned short* q,
+template <int D, int TERMS, bool MORE>
+inline void paged_short(void* out, const unsigned short* q,
                         const unsigned short* k_cache,
                         const unsigned short* v_cache, const int* block_tables,
                         const int* cu_q, const int* seq_lens, long tokens,
                         int n_seqs, float scale, int n_qheads, int n_kv,
                         int max_blocks, long q_stride, long out_stride,
-                        hipStream_t stream) {
+                        const PagedMore& x, hipStream_t stream) {
   const int G = n_qheads / n_kv;
   hipLaunchKernelGGL(
-      (paged_attn_short_kernel<D, TERMS>),
+      (paged_attn_short_kernel<D, TERMS, MORE>),
       dim3((unsigned)(paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv)),
       dim3(PS_WAVES * 64), 0, stream, out, q, k_cache, v_cache, block_tables,
-      cu_q, seq_lens, n_seqs, scale, G, n_kv, max_blocks, q_stride, out_stride);
+      cu_q, seq_lens, n_seqs, scale, G, n_kv, max_blocks, q_stride, out_stride, x);
+}
+
+// How a batch of prompts is run: by this kernel, or by paged_rows.h. max_blocks: pages
+// that a row sees
+struct PagedPrompts : PagedRows {
+  bool few = false;
+};
+inline PagedPrompts paged_prompts(long tokens, int n_seqs, int G, int n_kv, int D,
+                                  long max_blocks, int terms, bool options) {
+  PagedPrompts p;
+  p.few = paged_short_takes(tokens, n_seqs, G, n_kv, D, max_blocks, options);
+  if (!p.few)
+    static_cast<PagedRows&>(p) =
+        paged_rows_plan(tokens, n_seqs, G, n_kv, D, max_blocks, terms);
+  return p;
 }
 
 }  // namespace xllm

@@ -279,12 +279,9 @@ paged_attn_stream_kernel(
     }
     if (MORE && x.cap > 0.0f) paged_cap<1>(s, sc.pre, x.cap);
     if (t == n_tiles - 1 || (MORE && t * PA_KT < lo)) {      // uniform
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int key = t * PA_KT + mr_key_of(r, h);
-        if (key >= seq_len || (MORE && key < lo && key >= x.keep_first))
-          s[0][r] = -INFINITY;
-      }
+      paged_mask<MORE>(x, s, seq_len, lo, [&](int, int r) {
+        return t * PA_KT + mr_key_of(r, h);
+      });
     }
     const float c = sc.c;                      // weights are 2^(c (s - m))
     float mt = s[0][0];

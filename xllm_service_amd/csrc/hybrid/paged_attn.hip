@@ -110,12 +110,13 @@ void launch_paged_attn(void* out, long out_stride, bool out_f32, float* ws,
   if (p.few) {
     auto go = D == 128 ? paged_short<128, 3, true> : paged_short<64, 3, true>;
     go(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
-       scale, heads, n_kv, max_blocks, q_stride, out_stride, x, st);
+       scale, heads, n_kv, max_blocks, q_stride, out_stride, x, PagedAhead{}, st);
     return;
   }
   auto go = D == 128 ? paged_rows<128, 3, true> : paged_rows<64, 3, true>;
   go(out, ws, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
-     scale, heads, n_kv, max_blocks, q_stride, out_stride, p, x, st);
+     scale, heads, n_kv, max_blocks, q_stride, out_stride, p, x,
+     PagedAhead{}, st);
 }
 
 }  // namespace hyb

@@ -50,7 +50,7 @@ void launch_paged_attn_prefill(unsigned short*, float*, const unsigned short*,
                                const unsigned short*, const unsigned short*,
                                const int*, const int*, const int*, long, int,
                                float, int, int, int, int, long, long,
-                               hipStream_t);
+                               const void* const*, const long*, hipStream_t);
 void launch_greedy_sample(long*, const unsigned short*, int, int, hipStream_t);
 void launch_mfma_gemm(unsigned short*, const unsigned short*,
                       const unsigned short*, const unsigned short*, int, int,
@@ -261,10 +261,22 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
       q.stride(0), out.stride(0), stream, cur_stream());
 }
 
-void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
-                        torch::Tensor k_cache, torch::Tensor v_cache,
-                        torch::Tensor block_tables, torch::Tensor cu_q,
-                        torch::Tensor seq_lens, double scale) {
+// Weights that are read after an attention, in their order: PagedAhead
+struct Ahead {
+  const void* at[4] = {};
+  long bytes[4] = {};
+  void add(int i, const torch::Tensor& w) {
+    if (!w.is_contiguous()) return;
+    at[i] = w.data_ptr();
+    bytes[i] = w.numel() * w.element_size();
+  }
+};
+
+static void prefill_attn(torch::Tensor out, torch::Tensor q,
+                         torch::Tensor k_cache, torch::Tensor v_cache,
+                         torch::Tensor block_tables, torch::Tensor cu_q,
+                         torch::Tensor seq_lens, double scale,
+                         const Ahead* ahead) {
   CHECK_BF16_ROWVIEW(out); CHECK_BF16_ROWVIEW(q);
   CHECK_BF16_CUDA(k_cache); CHECK_BF16_CUDA(v_cache);
   for (auto* t : {&block_tables, &cu_q, &seq_lens}) {
@@ -291,8 +303,8 @@ void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
   // what lies at other addresses
   if (!on_bytes(out, 8)) {
     auto rows = out.clone(at::MemoryFormat::Contiguous);
-    paged_attn_prefill(rows, q, k_cache, v_cache, block_tables, cu_q, seq_lens,
-                       scale);
+    prefill_attn(rows, q, k_cache, v_cache, block_tables, cu_q, seq_lens, scale,
+                 ahead);
     out.copy_(rows);
     return;
   }
@@ -307,7 +319,15 @@ void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
       u16c(k_cache), u16c(v_cache), block_tables.data_ptr<int>(),
       cu_q.data_ptr<int>(), seq_lens.data_ptr<int>(), tokens, n_seqs,
       (float)scale, n_qheads, n_kv, D, block_tables.size(1), q.stride(0),
-      out.stride(0), cur_stream());
+      out.stride(0), ahead ? ahead->at : nullptr,
+      ahead ? ahead->bytes : nullptr, cur_stream());
+}
+void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
+                        torch::Tensor k_cache, torch::Tensor v_cache,
+                        torch::Tensor block_tables, torch::Tensor cu_q,
+                        torch::Tensor seq_lens, double scale) {
+  prefill_attn(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, scale,
+               nullptr);
 }
 
 torch::Tensor greedy_sample(torch::Tensor logits) {
@@ -638,10 +658,16 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layers(
     }
     auto out = torch::empty({T, heads * D}, q.options());
     const auto out3 = out.view({T, heads, D});
-    if (n_prefill > 0)
-      paged_attn_prefill(out3.slice(0, 0, n_prefill), q.slice(0, 0, n_prefill),
-                         p.k_cache, p.v_cache, prefill_tables.value(),
-                         cu_q.value(), prefill_lens.value(), scale);
+    if (n_prefill > 0) {
+      Ahead ahead;
+      ahead.add(0, p.o_w);
+      ahead.add(1, p.gate_up_w);
+      ahead.add(2, p.down_w);
+      if (i + 1 < layers.size()) ahead.add(3, layers[i + 1].qkv_w);
+      prefill_attn(out3.slice(0, 0, n_prefill), q.slice(0, 0, n_prefill),
+                   p.k_cache, p.v_cache, prefill_tables.value(), cu_q.value(),
+                   prefill_lens.value(), scale, &ahead);
+    }
     if (n_decode > 0)
       paged_attn_decode(out3.slice(0, n_prefill), q.slice(0, n_prefill),
                         p.k_cache, p.v_cache, decode_tables.value(),

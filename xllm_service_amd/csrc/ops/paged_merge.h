@@ -1,6 +1,7 @@
 // What the paged attention kernels (paged_rows.h, paged_stream.h) share: their
 // options, and the merge of keys that were split over workgroups.
 #pragma once
+#include <algorithm>
 #include <atomic>
 #include <random>
 
@@ -19,6 +20,52 @@ struct PagedMore {
   const float* sink = nullptr;        // [heads]: e^sink joins the denominator
   const float* head_scale = nullptr;  // [heads]: one more score multiplier
 };
+
+// What later kernels read from memory, for the CUs that attention over a few rows leaves
+// idle: workgroups past the last one's rows bring it into the cache in front of memory
+// (256 MB), and the products that follow find their weights there: 300 x 4096 x 2048 12.9 ->
+// 10.3 us, 3072 x 2048 11.3 -> 8.8, 4096 x 4096 21.6 -> 16.6. 8 layers, 300 rows of 2048
+// 532 -> 490, 120 448 -> 392, 2 x 90 471 -> 427, 600 795 -> 745; of 4096, 300 1145 -> 1120,
+// 90 774 -> 743, 150 826 -> 827. (Loads of the next weights among those of a product
+// itself cost 30 us instead: they return in order, and each step waited for memory
+// again. Decoded rows stream their weights at the rate of memory, and gained nothing.)
+struct PagedAhead {
+  static constexpr int N = 4;
+  const unsigned short* at[N] = {};
+  unsigned bytes[N] = {};
+  int wgs = 0;                        // that do so
+};
+// by workgroup `mine` of them, through LDS that it does not look at: 1 KB a wave
+XLLM_DEV void paged_fetch(const PagedAhead& a, int mine, unsigned short* lds) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned waves = blockDim.x >> 6, lane = threadIdx.x & 63;
+  const unsigned step = a.wgs * waves * 1024u;
+  for (int i = 0; i < PagedAhead::N; i++) {
+    const auto src = mr_buffer(a.at[i], a.bytes[i]);
+    for (unsigned at = (mine * waves + wave) * 1024u; at < a.bytes[i]; at += step)
+      mr_to_lds(src, at + lane * 16, lds + wave * 512);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// What the CUs that `wgs` workgroups leave can fetch of N pieces while those run: a CU
+// pulls 60 KB/us, memory 5 MB/us. 300 rows of 2048, 46 MB a layer: up to 24 MB 509 us, 32
+// 508, 41 (400 KB a CU) 502, all 490; 150 of 4096, 184 MB: 41 MB 821, 52 835.
+inline PagedAhead paged_ahead(long wgs, const void* const* at,
+                              const long* bytes) {
+  PagedAhead a;
+  if (at == nullptr || wgs > 256 - 32) return a;
+  a.wgs = (int)(256 - wgs);
+  long room = std::min<long>(48 << 20, a.wgs * (450L << 10));
+  for (int i = 0; i < PagedAhead::N; i++) {
+    const long n = std::min(bytes[i], room) / 1024 * 1024;
+    if (n <= 0) continue;
+    a.at[i] = static_cast<const unsigned short*>(at[i]);
+    a.bytes[i] = (unsigned)n;
+    room -= n;
+  }
+  return a;
+}
 
 // first key that a row which sees keys below `limit` has in its window
 template <bool MORE>

@@ -194,7 +194,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     const int* __restrict__ seq_lens,        // [num_seqs] total key len
     const int n_seqs, const float scale, const int G, const int n_kv,
     const int max_blocks, const long q_stride, const long out_stride,
-    const int n_part, const PagedMore x) {
+    const int n_part, const PagedMore x, const PagedAhead ahead) {
   constexpr int KS = D / 16;                 // k steps of a score product
   constexpr int DT = D / 32;                 // 32-wide tiles of the head
   constexpr int CPR = D / 8;                 // 16 B chunks of a row
@@ -210,6 +210,11 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   const int wid = wave & 3, kg = KG > 1 ? wave >> 2 : 0;
   const int h = lane >> 5, c32 = lane & 31;
 
+  const int beyond = (int)blockIdx.x - (int)(gridDim.x - ahead.wgs);
+  if (!MORE && beyond >= 0) {
+    paged_fetch(ahead, beyond, kv_lds);
+    return;
+  }
   const int kvh = blockIdx.x % n_kv;
   int part;
   PfPlace at;
@@ -542,18 +547,19 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
                        int n_seqs, float scale, int n_qheads, int n_kv,
                        int max_blocks, long q_stride, long out_stride,
                        const PagedRows& plan, const PagedMore& x,
-                       hipStream_t stream) {
+                       const PagedAhead& ahead, hipStream_t stream) {
   const int n_part = plan.parts;
   const int G = n_qheads / n_kv;
   if (tokens == 0 || n_seqs <= 0) return;
   float* ws_ml = ws_o + tokens * n_qheads * n_part * D;
   const dim3 grid(
-      (unsigned)(paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv * n_part));
+      (unsigned)(paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv * n_part +
+                 ahead.wgs));
 #define PF_GO(KG)                                                              \
   hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG>), grid,       \
                      dim3(KG * 256), 0, stream, out, ws_o, ws_ml, q, k_cache,  \
                      v_cache, block_tables, cu_q, seq_lens, n_seqs, scale, G,  \
-                     n_kv, max_blocks, q_stride, out_stride, n_part, x)
+                     n_kv, max_blocks, q_stride, out_stride, n_part, x, ahead)
   if (plan.groups == 2) PF_GO(2);
   else PF_GO(1);
 #undef PF_GO

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
     const int* __restrict__ seq_lens,        // [num_seqs] total key len
     const int n_seqs, const float scale, const int G, const int n_kv,
     const int max_blocks, const long q_stride, const long out_stride,
-    const PagedMore x) {
+    const PagedMore x, const PagedAhead ahead) {
   constexpr int KS = D / 16;                 // k steps of a score product
   constexpr int DT = D / 32;                 // 32-wide tiles of the head
   constexpr int CPR = D / 8;                 // 16 B chunks of a row
@@ -51,6 +51,11 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, c32 = lane & 31;
 
+  const int beyond = (int)blockIdx.x - (int)(gridDim.x - ahead.wgs);
+  if (!MORE && beyond >= 0) {
+    paged_fetch(ahead, beyond, kv_lds);
+    return;
+  }
   const int kvh = blockIdx.x % n_kv;
   PfPlace place;
   if (!pf_locate<PS_ROWS>(blockIdx.x / n_kv, cu_q, seq_lens, n_seqs, G, lane,
@@ -304,13 +309,16 @@ inline void paged_short(void* out, const unsigned short* q,
                         const int* cu_q, const int* seq_lens, long tokens,
                         int n_seqs, float scale, int n_qheads, int n_kv,
                         int max_blocks, long q_stride, long out_stride,
-                        const PagedMore& x, hipStream_t stream) {
+                        const PagedMore& x, const PagedAhead& ahead,
+                        hipStream_t stream) {
   const int G = n_qheads / n_kv;
   hipLaunchKernelGGL(
       (paged_attn_short_kernel<D, TERMS, MORE>),
-      dim3((unsigned)(paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv)),
+      dim3((unsigned)(paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv +
+                      ahead.wgs)),
       dim3(PS_WAVES * 64), 0, stream, out, q, k_cache, v_cache, block_tables,
-      cu_q, seq_lens, n_seqs, scale, G, n_kv, max_blocks, q_stride, out_stride, x);
+      cu_q, seq_lens, n_seqs, scale, G, n_kv, max_blocks, q_stride, out_stride, x,
+      ahead);
 }
 
 // How a batch of prompts is run: by this kernel, or by paged_rows.h. max_blocks: pages

@@ -300,7 +300,7 @@ def test_layers_against_64_bits(hidden, inter, heads, kv_heads, bias, gate_bias,
         no_further(a[new], b[new], w[new])
 
 
-@pytest.mark.parametrize("prompts", [[90], [120], [40, 70]])
+@pytest.mark.parametrize("prompts", [[90], [105], [40, 70]])
 def test_layers_of_small_weights(prompts):
     """Weights of no whole kilobytes, which CUs that attention leaves idle fetch."""
     test_layers_against_64_bits(136, 40, 2, 1, False, False, False, prompts, [])

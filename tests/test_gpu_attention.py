@@ -579,6 +579,27 @@ def test_prefill_orders_and_groups(kv_heads, per, dim, lens, ctx, sign):
     test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign)
 
 
+@pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [
+    (2, 4, 128, [50, 60, 0, 130, 20], [2500, 100, 30, 0, 700], 1.0),
+    (4, 4, 128, [3] * 68 + [64, 1], [0, 90] * 34 + [1300, 1100], -1.0),
+    (3, 5, 128, [9, 77], [1015, 1016], 1.0),         # parts of eight tiles, and nine
+    (1, 1, 128, [60, 1], [8200, 40], 1.0),          # sixteen parts
+    (12, 1, 64, [100, 5, 33], [1500, 0, 450], 1.0),
+    (8, 4, 128, [70], [3000], -1.0),                 # one sequence
+    (8, 4, 128, [300], [2000], 1.0),                 # in parts of two groups
+    (4, 7, 128, [1, 197, 0, 261], [900, 1750, 3, 524], 1.0),
+    (8, 4, 128, [600, 20, 33], [0, 1500, 100], 1.0),
+])
+def test_prefill_parts_by_length(kv_heads, per, dim, lens, ctx, sign):
+    """Keys split by a sequence's own length, over 64 sequences and more."""
+    test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign)
+
+
+@pytest.mark.parametrize("opts", ["cap", "window", "sink"])
+def test_prefill_parts_with_options(opts):
+    test_prefill_options_of_forms([40, 3, 200], [1700, 5, 600], 2, 4, 900, opts)
+
+
 def test_prefill_groups_without_keys():
     test_prefill_rows_without_keys(128, [700, 90, 5], [100, 660, 0], 8, 4)
 

@@ -44,7 +44,7 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws,
        stream);
     return;
   }
-  if (D == 128 && p.parts == 1 &&
+  if (D == 128 && p.least == 0 &&
       paged_long_takes(tokens, n_seqs, G, n_kv, max_blocks)) {
     paged_long(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens,
                n_seqs, scale, n_qheads, n_kv, max_blocks, q_stride, out_stride,
@@ -52,8 +52,7 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws,
     return;
   }
   const PagedAhead a = paged_ahead(
-      paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv * p.parts, ahead,
-      ahead_bytes);
+      paged_rows_wgs(p, tokens, n_seqs, G, n_kv), ahead, ahead_bytes);
   auto go = D == 128 ? paged_rows<128, 1, false> : paged_rows<64, 3, false>;
   go(out, ws, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
      scale, n_qheads, n_kv, max_blocks, q_stride, out_stride, p, PagedMore{},

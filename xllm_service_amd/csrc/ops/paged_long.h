@@ -52,10 +52,9 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
   const int h = lane >> 5, c32 = lane & 31;
 
   const int kvh = blockIdx.x % n_kv;
-  int unit;
   PfPlace place;
-  if (!pf_longest<PL_ROWS, 1>(blockIdx.x / n_kv, 1, INT_MAX / 2, cu_q, seq_lens,
-                           n_seqs, G, lane, &place, &unit))
+  if (!pf_longest<PL_ROWS, 1>(blockIdx.x / n_kv, INT_MAX / 2, cu_q, seq_lens,
+                              n_seqs, G, lane, &place))
     return;
   const int seq = place.seq, lt = place.lt, q_start = place.q_start,
             q_len = place.q_len, seq_len = place.seq_len;

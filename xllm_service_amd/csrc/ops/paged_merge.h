@@ -305,13 +305,14 @@ inline PagedMeet paged_meet(float* ws_ml, long rows, int parts) {
 
 // out[row] = sum_p o[row][p] 2^(m_p - M) / sum_p l_p 2^(m_p - M): D/4 lanes per
 // row, four columns each. Rows are those of n_seqs prompts; tokens outside of all of
-// them have no parts and stay as they are. B: parts fetched at once.
-template <int D, bool MORE, int B>
+// them have no parts and stay as they are, rows with one part are there. ws_at: slot of
+// a row's first part, parts; the others follow it.
+template <int D, bool MORE>
 __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
     void* __restrict__ out, const float* __restrict__ ws_o,
-    const float* __restrict__ ws_ml, const int n_qheads, const int n_part,
-    const long out_stride, const long rows, const PagedMore x,
-    const int* __restrict__ cu_q, const int n_seqs) {
+    const float* __restrict__ ws_ml, const int2* __restrict__ ws_at,
+    const int n_qheads, const long out_stride, const long rows,
+    const PagedMore x, const int* __restrict__ cu_q, const int n_seqs) {
   constexpr int LPR = D / 4;
   const long row = (blockIdx.x * 256L + threadIdx.x) / LPR;
   const int col = (threadIdx.x % LPR) * 4;
@@ -319,16 +320,20 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
   const long tok = row / n_qheads;
   const int head = (int)(row - tok * n_qheads);
   if (tok < cu_q[0] || tok >= cu_q[n_seqs]) return;
+  const int2 at = ws_at[row];
+  if (at.y <= 1) return;
   const bool sink = MORE && x.sink != nullptr;
   float M = sink ? x.sink[head] * 1.4426950408889634f : -INFINITY;
   float L = sink ? 1.0f : 0.0f;
   float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + row * n_part;
-  const float* o = ws_o + row * n_part * D + col;
-  paged_add_parts<B>(
-      [&](int p) { return ml[p]; },
-      [&](int p) { return *reinterpret_cast<const float4*>(o + (long)p * D); },
-      n_part, M, L, a);
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + at.x;
+  const float* o = ws_o + (long)at.x * D + col;
+  auto ml_of = [&](int p) { return ml[p]; };
+  auto o_of = [&](int p) {
+    return *reinterpret_cast<const float4*>(o + p * D);
+  };
+  if (at.y <= 4) paged_add_parts<4>(ml_of, o_of, at.y, M, L, a);
+  else paged_add_parts<8>(ml_of, o_of, at.y, M, L, a);
   const float inv = L != 0.0f ? 1.0f / L : 0.0f;
   paged_put<MORE>(x, out, tok * out_stride + (long)head * D + col, a[0] * inv,
                   a[1] * inv, a[2] * inv, a[3] * inv);
@@ -336,17 +341,13 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(
 
 template <int D, bool MORE>
 inline void paged_merge(void* out, const float* ws_o, const float* ws_ml,
-                        int n_qheads, int n_part, long out_stride, long rows,
-                        const PagedMore& x, hipStream_t stream,
-                        const int* cu_q, int n_seqs) {
-#define PM_GO(B)                                                               \
-  hipLaunchKernelGGL((paged_attn_merge_kernel<D, MORE, B>),                    \
-                     dim3((unsigned)((rows * (D / 4) + 255) / 256)),           \
-                     dim3(256), 0, stream, out, ws_o, ws_ml, n_qheads, n_part, \
-                     out_stride, rows, x, cu_q, n_seqs)
-  if (n_part <= 4) PM_GO(4);
-  else PM_GO(8);
-#undef PM_GO
+                        const int2* ws_at, int n_qheads,
+                        long out_stride, long rows, const PagedMore& x,
+                        hipStream_t stream, const int* cu_q, int n_seqs) {
+  hipLaunchKernelGGL((paged_attn_merge_kernel<D, MORE>),
+                     dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256), 0,
+                     stream, out, ws_o, ws_ml, ws_at, n_qheads, out_stride,
+                     rows, x, cu_q, n_seqs);
 }
 
 }  // namespace xllm

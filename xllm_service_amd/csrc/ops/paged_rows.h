@@ -28,8 +28,8 @@
 // the row reads of K and the transpose reads of V free of bank conflicts.
 //
 // Few row tiles over a long context leave most of the chip idle: then the
-// keys are split over n_part workgroups and a second kernel merges the fp32
-// partial results.
+// keys of a tile are split over workgroups, by the length of its own sequence
+// (pf_parts), and a second kernel merges the fp32 partial results.
 //
 // Bound by the matrix pipe and the vector unit in turn: a tile costs a wave
 // 32 products (about 1000 cycles) and about as many cycles of exponentials,
@@ -121,20 +121,23 @@ XLLM_DEV int pf_scan(int v) {
 // WIDTH tiles of a sequence to a level, which share its keys and stay together. The level
 // of tile b is found by halves, a lane counting its sequence's tiles above one. Up to 64
 // sequences; of more, one sequence after the other (pf_locate).
-//   units: b is one of so many per tile (parts), of which those past the first `turn` come
-// in the reverse order if they are no more than another `turn`: two workgroups share a
-// CU then, and the longest chains meet the shortest. By sequences, the tiles of two
-// equal prompts met their likes: 2 x 1.8-2.3 k in a window of 1024 59.5 -> 54.8 us, 4 x 512
-// of 32/8 heads 28.3 -> 22.8, 3 x 500 capped 51.5 -> 40.2. WIDTH 1, 2 and 4: 40 x 60 behind
-// 500, whose two tiles read the same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500 and
+//   Tiles past the first `turn` come in the reverse order if they are no more than another
+// `turn`: two workgroups share a CU then, and the longest chains meet the shortest. By
+// sequences, the tiles of two equal prompts met their likes: 2 x 1.8-2.3 k in a window of
+// 1024 59.5 -> 54.8 us, 4 x 512 of 32/8 heads 28.3 -> 22.8, 3 x 500 capped 51.5 -> 40.2.
+// WIDTH 1, 2 and 4: 40 x 60 behind 500, whose two tiles read the same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500 and
 // 300 of 64-wide heads 26.6, 26.6, 27.6.
 template <int ROWS, int WIDTH>
-XLLM_DEV bool pf_longest(int b, int units, int turn, const int* cu_q,
-                         const int* seq_lens, int n_seqs, int G, int lane,
-                         PfPlace* place, int* unit) {
-  if (n_seqs > 64) {
-    *unit = b % units;
-    return pf_locate<ROWS>(b / units, cu_q, seq_lens, n_seqs, G, lane, place);
+XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
+                         int n_seqs, int G, int lane, PfPlace* place) {
+  if (n_seqs > 64)
+    return pf_locate<ROWS>(b, cu_q, seq_lens, n_seqs, G, lane, place);
+  if (n_seqs == 1) {                             // without scans: 0.4 us of a small call
+    const int q0 = cu_q[0], n = cu_q[1] - q0, all = (n * G + ROWS - 1) / ROWS;
+    if (b >= all) return false;
+    if (b >= turn && all <= 2 * turn) b = turn + all - 1 - b;
+    *place = {0, all - 1 - b, q0, n, seq_lens[0]};
+    return true;
   }
   int start = 0, len = 0, keys = 0;              // of sequence `lane`
   if (lane < n_seqs) {
@@ -145,11 +148,9 @@ XLLM_DEV bool pf_longest(int b, int units, int turn, const int* cu_q,
   const int nt = (len * G + ROWS - 1) / ROWS, top = keys * G;
   const int most = __builtin_amdgcn_readlane(
       pf_scan<false>(nt > 0 ? top : INT_MIN), 63);
-  const int total = __builtin_amdgcn_readlane(pf_scan<true>(nt), 63) * units;
+  const int total = __builtin_amdgcn_readlane(pf_scan<true>(nt), 63);
   if (b >= total) return false;
   if (b >= turn && total <= 2 * turn) b = turn + total - 1 - b;
-  *unit = b % units;
-  b /= units;
   // its tiles from the top: [first, first + nt)
   const int first = nt > 0 ? (most - top) / ROWS : 0;
   const int depth = __builtin_amdgcn_readlane(pf_scan<false>(first + nt), 63);
@@ -176,16 +177,104 @@ XLLM_DEV bool pf_longest(int b, int units, int turn, const int* cu_q,
   return true;
 }
 
+#define PF_UNITS 448       // groups of waves that a batch's keys are split over,
+#define PF_TURN 512        // and that the CUs hold at once
+
+// Unit `b` of a batch whose keys are split: a row tile and one of its parts, b - part the
+// tile's first. One sequence: up to `most` equal parts, of at least four tiles of keys.
+// Several: parts of `per` tiles, so that all of the batch walk about as many, whatever its
+// sequences' lengths. Never more parts than ceil(n / per), or than `most` for one sequence:
+// the grid and the scratch hold that many units (PagedRows), and a row whose unit was not
+// in the grid would leave the merge without its place. PF_UNITS: just under two groups of
+// waves to a CU.
+//   The same number of parts for all, as many as the longest's table asks for, left one
+// sequence's chain to be waited for: 50, 60, 300 and 20 tokens behind 9000, 100, 0 and 700
+// of 32/8 heads 59.4 -> 34.4 us, of 28/4 51.4 -> 29, 31, 322 and 416 behind 4052, 20 and
+// 27 of 32/32 56 -> 30.5, 2 x 200 behind 3000 52.3 -> 41.1; equal ones (8 x 100 behind 500,
+// 20.1) gain nothing.
+template <int ROWS, bool MORE>
+XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& x,
+                       const int* cu_q, const int* seq_lens, int n_seqs, int G,
+                       int n_kv, int lane, PfPlace* at, int* part, int* parts,
+                       int* first) {
+  auto tiles_of = [&](int keys) {
+    const int n = (max(keys, 0) + PF_KT - 1) / PF_KT;
+    return MORE && x.window > 0
+               ? min(n, (x.window + x.keep_first) / PF_KT + 3) : n;
+  };
+  if (n_seqs == 1) {
+    const int q0 = cu_q[0], len = cu_q[1] - q0, keys = seq_lens[0];
+    const int p = max(min((tiles_of(keys) + 3) / 4, most), 1);
+    const int all = (len * G + ROWS - 1) / ROWS * p;
+    if (b >= all) return false;
+    const int turn = 256 / n_kv;                 // as in pf_longest
+    if (b >= turn && all <= 2 * turn) b = turn + all - 1 - b;
+    *part = b % p;
+    *parts = p;
+    *first = b - b % p;
+    *at = {0, (all - 1 - b) / p, q0, len, keys};
+    return true;
+  }
+  int start = 0, len = 0, keys = 0, nt = 0, n = 0;
+  auto look = [&](int i) {                       // sequence i, one to a lane
+    start = len = keys = 0;
+    if (i < n_seqs) {
+      start = cu_q[i];
+      len = cu_q[i + 1] - start;
+      keys = seq_lens[i];
+    }
+    nt = (len * G + ROWS - 1) / ROWS;
+    n = tiles_of(keys);
+  };
+  int work = 0;
+  for (int base = 0; base < n_seqs; base += 64) {
+    look(base + lane);
+    work += __builtin_amdgcn_readlane(pf_scan<true>(nt * n), 63);
+  }
+  const int some = PF_UNITS / groups;
+  int per = max(least, (work * n_kv + some - 1) / some);
+  // a few workgroups left for another turn cost up to a third
+  if (n_seqs <= 64)
+    for (int i = 0; i < 8; i++, per++) {
+      const int p = max(min((n + per - 1) / per, most), 1);
+      if (__builtin_amdgcn_readlane(pf_scan<true>(nt * p), 63) * n_kv <= PF_TURN / groups)
+        break;
+    }
+  int acc = 0;
+  for (int base = 0; base < n_seqs; base += 64) {
+    if (n_seqs > 64) look(base + lane);
+    const int p = max(min((n + per - 1) / per, most), 1);
+    const int upto = acc + pf_scan<true>(nt * p);
+    const unsigned long long hit = __ballot(b < upto);
+    if (hit != 0) {
+      const int l = __builtin_amdgcn_readfirstlane(__ffsll(hit) - 1);
+      const int pl = __builtin_amdgcn_readlane(p, l);
+      const int r = b - __builtin_amdgcn_readlane(upto - nt * p, l);
+      *part = r % pl;
+      *parts = pl;
+      *first = b - r % pl;
+      *at = {base + l, __builtin_amdgcn_readlane(nt, l) - 1 - r / pl,
+             __builtin_amdgcn_readlane(start, l),
+             __builtin_amdgcn_readlane(len, l),
+             __builtin_amdgcn_readlane(keys, l)};
+      return true;
+    }
+    acc = __builtin_amdgcn_readlane(upto, 63);
+  }
+  return false;
+}
+
 // TERMS: bf16 terms a softmax weight is split into. One rounds it to bf16;
 // three (8 + 8 + 8 mantissa bits) hold all of its 32-bit value, each with a
 // product of its own into the same fp32 sums. MORE: the options of PagedMore.
 // KG: groups of four waves, each with the same rows and its share of the tiles: what
 // splitting keys over workgroups does, without partial results in memory.
-template <int D, int TERMS, bool MORE, int KG>
+template <int D, int TERMS, bool MORE, int KG, bool SPLIT>
 __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     void* __restrict__ out,                  // [total_q, n_qheads, D]
-    float* __restrict__ ws_o,                // [total_q*n_qheads][n_part][D]
-    float* __restrict__ ws_ml,               // [total_q*n_qheads][n_part][2]
+    float* __restrict__ ws_o,                // [slots][D] (least > 0)
+    float* __restrict__ ws_ml,               // [slots][2]
+    int2* __restrict__ ws_at,                // [total_q*n_qheads]: first slot, parts
     const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
     const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
     const unsigned short* __restrict__ v_cache,
@@ -194,7 +283,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     const int* __restrict__ seq_lens,        // [num_seqs] total key len
     const int n_seqs, const float scale, const int G, const int n_kv,
     const int max_blocks, const long q_stride, const long out_stride,
-    const int n_part, const PagedMore x, const PagedAhead ahead) {
+    const int least, const int most, const PagedMore x, const PagedAhead ahead) {
   constexpr int KS = D / 16;                 // k steps of a score product
   constexpr int DT = D / 32;                 // 32-wide tiles of the head
   constexpr int CPR = D / 8;                 // 16 B chunks of a row
@@ -216,12 +305,19 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     return;
   }
   const int kvh = blockIdx.x % n_kv;
-  int part;
+  int part = 0, parts = 1, first = 0;
   PfPlace at;
-  if (!pf_longest<PF_ROWS, 2>(blockIdx.x / n_kv, n_part,
-                              KG > 1 ? INT_MAX / 2 : 256 / n_kv, cu_q, seq_lens,
-                              n_seqs, G, lane, &at, &part))
-    return;
+  if constexpr (SPLIT) {
+    if (!pf_parts<PF_ROWS, MORE>(blockIdx.x / n_kv, least, most, KG, x, cu_q,
+                                 seq_lens, n_seqs, G, n_kv, lane, &at, &part,
+                                 &parts, &first))
+      return;
+  } else {
+    if (!pf_longest<PF_ROWS, 2>(blockIdx.x / n_kv,
+                                KG > 1 ? INT_MAX / 2 : 256 / n_kv, cu_q, seq_lens,
+                                n_seqs, G, lane, &at))
+      return;
+  }
   const int seq = at.seq, lt = at.lt, q_start = at.q_start, q_len = at.q_len,
             seq_len = at.seq_len;
   const int ctx = seq_len - q_len;
@@ -233,9 +329,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   const int n_tiles = (kmax + PF_KT - 1) / PF_KT;
   const PagedTiles list = paged_tiles<MORE>(x, ctx + row0 / G + 1, kmax,
                                             n_tiles, PF_KT);
-  // parts of at least four tiles; the rest of them stay empty
-  const int parts = min(n_part, (list.n + 3) / 4);
-  const int tpp = parts > 0 ? (list.n + parts - 1) / parts : 0;
+  const int tpp = (max(list.n, 0) + parts - 1) / parts;
   const int p_begin = part * tpp;
   const int i_end = min(list.n, p_begin + tpp);
   const int i_begin = p_begin + kg;              // every KG-th of a group's
@@ -465,7 +559,12 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   }
   if (!row_ok) return;
   const long grow = (long)(q_start + qi) * n_qheads + head;
-  if (n_part == 1) {
+  // the parts of a row lie together (strided, the merge took up to 9 us more)
+  const int slot = (first * n_kv + kvh * parts) * PF_ROWS +
+                   (wid * 32 + c32) * parts + part;
+  if (SPLIT && part == 0 && h == 0 && kg == 0)
+    ws_at[grow] = make_int2(slot, parts);
+  if (!SPLIT || parts == 1) {
     if (MORE && x.sink != nullptr)
       l += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f - m);
     const float inv = l != 0.0f ? 1.0f / l : 0.0f;
@@ -479,13 +578,12 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
                         o_acc[j][r + 3] * inv);
     return;
   }
-  const long slot = grow * n_part + part;
   if (h == 0 && kg == 0) {
-    ws_ml[slot * 2] = m;
-    ws_ml[slot * 2 + 1] = p_begin < i_end ? l : PAGED_ABSENT;
+    ws_ml[slot * 2L] = m;
+    ws_ml[slot * 2L + 1] = p_begin < i_end ? l : PAGED_ABSENT;
   }
   if (p_begin >= i_end) return;
-  float* o = ws_o + slot * D + 4 * h;
+  float* o = ws_o + (long)slot * D + 4 * h;
 #pragma unroll
   for (int j = 0; j < OWN; j++)
 #pragma unroll
@@ -500,24 +598,36 @@ template <int ROWS>
 inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
   return (tokens * G + n_seqs * (ROWS - 1L)) / ROWS;
 }
-// Groups of waves, and parts of the keys. Parts: about two workgroups per CU are wanted,
-// and parts of at least eight tiles of keys (four with 32-bit weights, whose tiles take
-// twice as long): the merge costs more than smaller ones save. Measured (us, by parts 1 | 2 |
-// 4 | 8), 32-bit weights: 2 x 64 rows of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of
-// 16 over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles) 374 | 298 | 302 | 325;
-// 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
-//   Two groups of waves instead where they fill one turn of the CUs, as one part: 128-wide
+// Groups of waves, and parts of the keys. Parts (pf_parts): about two groups of waves per
+// CU are wanted, and parts of at least eight tiles of keys (four with 32-bit weights, whose
+// tiles take twice as long): the merge costs more than smaller ones save. At least six: 3
+// chunks of 93-261 tokens 36.5 us (eight: 31.8); up to 16 parts, not 8: 29.7 (34.9) for 50-300
+// tokens behind up to 9000. Measured (us, by parts 1 | 2 | 4 | 8), 32-bit weights: 2 x 64 rows
+// of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of 16 over 600 37 | 26 | 24 | 28; 1024
+// of 32 over 8000 (264 row tiles) 374 | 298 | 302 | 325; 4096 of 16 in a window (520 row
+// tiles) 69 | 87 | 111 | 182.
+//   Parts of two groups of waves, which leave half the partial results in memory (24 MB of
+// the 3 chunks'), where their larger units still fill the CUs, one turn of them and no more:
+// one sequence in 200-256 of at least three parts, several in up to 144 before they are
+// split; us, one | two groups: the 3 chunks 31.4 | 29.6, 2 x 200 behind 3000 43.7 | 41.1, 300 behind 2000 of 32/8
+// 37.2 | 31.5, 300 behind 12000 of 16/4 64.8 | 48.7, of 28/4 (204 units) 91 | 78, capped 1900
+// and 32/8 47.1 | 44; but 272 units of the last but one 110, two parts (256 units) of 1000
+// behind 500 of 16/4 capped 38.6 | 42.8, 31, 322 and 416 tokens of 32 heads (288) 30.5 | 35.7.
+//   Two groups of waves and one part where these fill one turn of the CUs: 128-wide
 // heads, up to 24 tiles, or for a single sequence that fills most of the CUs; us, as before
 // (parts) | two groups: 1024 tokens of 32/8 heads 34.5 (2) | 25.5, 28/4 32.5 (2) | 24.8, 3 x
 // 300 behind 1000 44 (2) | 33, 1000 behind 1000 49.5 (2) | 42.2, 700 20.9 (1) | 20.0, but 300
 // 13.2 (1) | 14.1; 300 behind 1000, 28/4 (66 workgroups) 27.3 | 28.5, 16/4 1000 behind 1000
-// (125) 34.9 (4) | 37.5; and one prompt in up to 448 workgroups, whose chains differ: 1400
+// (125) 34.9 (4) | 37.5; and one prompt in up to 448 workgroups, whose chains differ: 1200 of
+// 32/32 (19 tiles) 44 | 30, 1400
 // of 32/8 39 | 32.8, 2048 of 28/4 (448) 54.2 | 50, 32/8 (512) 55.5 | 56.4, 850 of 64/8 (14 tiles)
-// 29 | 31.4. 32-bit weights, 2 x 400 behind 500 of 32/8 in a window 46.3 (2) | 33, capped 51.8 |
+// 29 | 31.4. 32-bit weights, 2 x 400 behind 500 of 32/8 in a window 46.3 (2) | 33, in
+// one of 512 41 (2) | 29.5, capped 51.8 |
 // 40, but 300 behind 1000 (75) 37 (4) | 42, 2000 of 16/4 capped 71 (2) | 73.7. 64-wide, two
 // workgroups to a CU: 8 prompts of 64-448 13.3 (1) | 12.4, 1700 (168) 27.8 (3) | 32.7.
-// groups: KG; scratch: floats
-struct PagedRows { int parts = 1, groups = 1; long scratch = 0; };
+// groups: KG; least: tiles of a part, 0 without parts; most: parts of a tile; units: tiles
+// and parts a grid holds; scratch: floats
+struct PagedRows { int groups = 1, least = 0, most = 1; long units = 0, scratch = 0; };
 inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D,
                                  long max_blocks, int terms) {
   PagedRows x;
@@ -527,15 +637,32 @@ inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D
   if (D == 64)
     x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 ? 2 : 1;
   else if (terms > 1)
-    x.groups = keys >= 640 && tiles <= 20 && wgs >= 200 && wgs <= 256 ? 2 : 1;
+    x.groups = keys >= 512 && tiles <= 20 && wgs >= 200 && wgs <= 256 ? 2 : 1;
   else if (keys >= 640 && wgs >= 72)
     x.groups = wgs <= 256 ? (tiles <= 24 || (n_seqs == 1 && wgs >= 200) ? 2 : 1)
-                          : (wgs <= 448 && alone && tiles >= 20 ? 2 : 1);
-  const long p = x.groups == 2 || wgs == 0 ? 1 : (512 + wgs / 2) / wgs;
-  const long most = keys / ((terms > 1 ? 4 : 8) * PF_KT);
-  x.parts = (int)std::max<long>(1, std::min<long>({p, most, 16}));
-  if (x.parts > 1) x.scratch = tokens * G * n_kv * x.parts * (D + 2);
+                          : (wgs <= 448 && alone && tiles >= 18 ? 2 : 1);
+  const int least = terms == 1 ? 8 : 4;
+  if (x.groups == 1 && wgs > 0 && wgs <= 340 && tiles >= 2 * least) {
+    const long row_tiles = paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G);
+    const long twos = std::min<long>({256 / wgs, tiles / (terms == 1 ? 8 : 5), 16});
+    if (D == 128 && (n_seqs > 1 ? terms == 1 && wgs <= 144
+                                : twos > 2 && wgs * twos >= 200))
+      x.groups = 2;
+    x.most = n_seqs > 1 ? 16
+             : x.groups == 2 ? (int)twos
+                 : (int)std::min<long>({(512 + wgs / 2) / wgs, tiles / least, 16});
+    x.least = x.groups == 2 ? 12 : D == 64 ? 4 : least;
+    x.units = n_seqs > 1 ? row_tiles + PF_UNITS / x.groups / n_kv + 1
+                         : row_tiles * x.most;
+    x.scratch = x.units * n_kv * PF_ROWS * (D + 2) + tokens * G * n_kv * 2;
+  }
   return x;
+}
+
+inline long paged_rows_wgs(const PagedRows& p, long tokens, int n_seqs, int G,
+                           int n_kv) {
+  return (p.least > 0 ? p.units : paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G)) *
+         n_kv;
 }
 
 // Prompt rows and the merge of their parts
@@ -548,23 +675,25 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
                        int max_blocks, long q_stride, long out_stride,
                        const PagedRows& plan, const PagedMore& x,
                        const PagedAhead& ahead, hipStream_t stream) {
-  const int n_part = plan.parts;
   const int G = n_qheads / n_kv;
   if (tokens == 0 || n_seqs <= 0) return;
-  float* ws_ml = ws_o + tokens * n_qheads * n_part * D;
-  const dim3 grid(
-      (unsigned)(paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv * n_part +
-                 ahead.wgs));
-#define PF_GO(KG)                                                              \
-  hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG>), grid,       \
-                     dim3(KG * 256), 0, stream, out, ws_o, ws_ml, q, k_cache,  \
-                     v_cache, block_tables, cu_q, seq_lens, n_seqs, scale, G,  \
-                     n_kv, max_blocks, q_stride, out_stride, n_part, x, ahead)
-  if (plan.groups == 2) PF_GO(2);
-  else PF_GO(1);
+  const long wgs = paged_rows_wgs(plan, tokens, n_seqs, G, n_kv);
+  float* ws_ml = ws_o + wgs * PF_ROWS * D;
+  int2* ws_at = reinterpret_cast<int2*>(ws_ml + wgs * PF_ROWS * 2);
+#define PF_GO(KG, SPLIT)                                                       \
+  hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG, SPLIT>),      \
+                     dim3((unsigned)(wgs + ahead.wgs)), dim3(KG * 256), 0,     \
+                     stream, out, ws_o, ws_ml, ws_at, q, k_cache, v_cache,     \
+                     block_tables, cu_q, seq_lens, n_seqs, scale, G, n_kv,     \
+                     max_blocks, q_stride, out_stride, plan.least, plan.most, x,  \
+                     ahead)
+  if (plan.groups == 2 && plan.least > 0) PF_GO(2, true);
+  else if (plan.groups == 2) PF_GO(2, false);
+  else if (plan.least > 0) PF_GO(1, true);
+  else PF_GO(1, false);
 #undef PF_GO
-  if (n_part > 1)
-    paged_merge<D, MORE>(out, ws_o, ws_ml, n_qheads, n_part, out_stride,
+  if (plan.least > 0)
+    paged_merge<D, MORE>(out, ws_o, ws_ml, ws_at, n_qheads, out_stride,
                          tokens * n_qheads, x, stream, cu_q, n_seqs);
 }
 

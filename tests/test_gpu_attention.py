@@ -595,6 +595,42 @@ def test_prefill_parts_by_length(kv_heads, per, dim, lens, ctx, sign):
     test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign)
 
 
+@pytest.mark.parametrize("kv_heads,per,dim,lens,ctx", [
+    (2, 4, 128, [50, 60, 9], [3900, 100, 700]),      # six parts of two groups: two rounds
+    (8, 4, 128, [300], [2000]),                      # three of one sequence
+    (12, 1, 64, [420], [900]),                       # one group
+])
+def test_prefill_parts_meet(kv_heads, per, dim, lens, ctx):
+    """Parts that the last one merges: over scratch that held anything before, and
+    in replays of a captured call whose lengths change, to the same bits."""
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(ctx))
+    heads, scale = kv_heads * per, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim)).contiguous()
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0))).int().cuda()
+    dev = [t.cuda() for t in (q, k, v, table)]
+    sl = torch.tensor([n + c for n, c in zip(lens, ctx)]).int().cuda()
+    out = torch.empty_like(dev[0])
+
+    def step():
+        for fill in (0, -1, 0x7f7f7f7f7f7f7f01):
+            torch.full((1 << 22,), fill, dtype=torch.int64, device="cuda")
+        ops.paged_attn_prefill(*dev, cu, sl, scale, out=out)
+    step()
+    check(out, *want(q, k, v, table, lens, ctx, scale))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for behind in (ctx, ctx, [c // 3 for c in ctx], ctx):
+        sl.copy_(torch.tensor([n + c for n, c in zip(lens, behind)]))
+        out.fill_(3.0)
+        graph.replay()
+        got = out.clone()
+        ops.paged_attn_prefill(*dev, cu, sl, scale, out=out)
+        assert torch.equal(got, out)
+        check(got, *want(q, k, v, table, lens, behind, scale))
+
+
 @pytest.mark.parametrize("opts", ["cap", "window", "sink"])
 def test_prefill_parts_with_options(opts):
     test_prefill_options_of_forms([40, 3, 200], [1700, 5, 600], 2, 4, 900, opts)

@@ -29,7 +29,8 @@
 //
 // Few row tiles over a long context leave most of the chip idle: then the
 // keys of a tile are split over workgroups, by the length of its own sequence
-// (pf_parts), and a second kernel merges the fp32 partial results.
+// (pf_parts). Of a few parts the last one to finish merges the fp32 partial results
+// of all (PagedMeet), of many a second kernel does, which all CUs share.
 //
 // Bound by the matrix pipe and the vector unit in turn: a tile costs a wave
 // 32 products (about 1000 cycles) and about as many cycles of exponentials,
@@ -121,12 +122,13 @@ XLLM_DEV int pf_scan(int v) {
 // WIDTH tiles of a sequence to a level, which share its keys and stay together. The level
 // of tile b is found by halves, a lane counting its sequence's tiles above one. Up to 64
 // sequences; of more, one sequence after the other (pf_locate).
-//   Tiles past the first `turn` come in the reverse order if they are no more than another
-// `turn`: two workgroups share a CU then, and the longest chains meet the shortest. By
-// sequences, the tiles of two equal prompts met their likes: 2 x 1.8-2.3 k in a window of
-// 1024 59.5 -> 54.8 us, 4 x 512 of 32/8 heads 28.3 -> 22.8, 3 x 500 capped 51.5 -> 40.2.
-// WIDTH 1, 2 and 4: 40 x 60 behind 500, whose two tiles read the same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500 and
-// 300 of 64-wide heads 26.6, 26.6, 27.6.
+//   Tiles past the first `turn` come in the reverse order if they are no more than
+// another `turn`: two workgroups share a CU then, and the longest chains meet the
+// shortest. By sequences, the tiles of two equal prompts met their likes: 2 x 1.8-2.3 k
+// in a window of 1024 59.5 -> 54.8 us, 4 x 512 of 32/8 heads 28.3 -> 22.8, 3 x 500
+// capped 51.5 -> 40.2. WIDTH 1, 2 and 4: 40 x 60 behind 500, whose two tiles read the
+// same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500 and 300 of 64-wide heads 26.6,
+// 26.6, 27.6.
 template <int ROWS, int WIDTH>
 XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
                          int n_seqs, int G, int lane, PfPlace* place) {
@@ -272,9 +274,10 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& 
 template <int D, int TERMS, bool MORE, int KG, bool SPLIT>
 __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     void* __restrict__ out,                  // [total_q, n_qheads, D]
-    float* __restrict__ ws_o,                // [slots][D] (least > 0)
-    float* __restrict__ ws_ml,               // [slots][2]
+    float* __restrict__ ws_o,                // [blocks][PF_ROWS * D], a block for a part
+    float* __restrict__ ws_ml,               // [blocks][PF_ROWS][2]
     int2* __restrict__ ws_at,                // [total_q*n_qheads]: first slot, parts
+    const PagedMeet meet,                    // [2][blocks]: by fours, by sixteens
     const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
     const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
     const unsigned short* __restrict__ v_cache,
@@ -330,6 +333,14 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   const PagedTiles list = paged_tiles<MORE>(x, ctx + row0 / G + 1, kmax,
                                             n_tiles, PF_KT);
   const int tpp = (max(list.n, 0) + parts - 1) / parts;
+  // its parts' place: their blocks lie together
+  const long block = SPLIT ? (long)first * n_kv + kvh * parts : 0;
+  u64 seen[2] = {0, 0};
+  const bool meets = SPLIT && parts > 1 && meet.count != nullptr;
+  if (meets && threadIdx.x == 0) {
+    seen[0] = paged_seen(meet.count + block + (part & ~3));
+    if (parts > 4) seen[1] = paged_seen(meet.count + meet.units + block);
+  }
   const int p_begin = part * tpp;
   const int i_end = min(list.n, p_begin + tpp);
   const int i_begin = p_begin + kg;              // every KG-th of a group's
@@ -517,8 +528,21 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   // ---- epilogue: o_acc[dt][r] = O[row][dt*32 + 8*(r>>2) + 4h + (r&3)] --------
   l = pair_sum(l);
   m = m == -INFINITY ? m : m * sc.c;
+  if (meets && threadIdx.x == 0) {
+    paged_open(meet.count + block + (part & ~3), seen[0], meet.tag);
+    if (parts > 4) paged_open(meet.count + meet.units + block, seen[1], meet.tag);
+  }
   constexpr int OWN = DT / KG;                   // column tiles a group finishes
   const int dt0 = kg * OWN;
+  constexpr unsigned GONE = 0x7ffffff0;          // out of the bounds: no store, zeros
+  const int row = wid * 32 + c32;
+  const unsigned size_o = SPLIT && parts > 1 ? parts * (PF_ROWS * D * 4) : 0;
+  const auto unit_o = mr_buffer(SPLIT ? ws_o + block * (PF_ROWS * D) : nullptr, size_o);
+  const auto unit_ml =
+      mr_buffer(SPLIT ? ws_ml + block * (PF_ROWS * 2) : nullptr, size_o / D * 2);
+  auto piece = [&](int b, int j, int r) {        // of part b: 1 KB of a wave's
+    return (unsigned)(((((b * 4 + wid) * DT + dt0 + j) * 4 + r) * 64 + lane) * 16);
+  };
   if constexpr (KG > 1) {
     // the groups swap halves of their sums
     __syncthreads();
@@ -557,14 +581,97 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
         }
       }
   }
+  if (meets) {
+    // ---- the last of four parts merges them, the last of four fours those -------
+    // A wave writes and reads its sums as its lanes hold them, 1 KB at a time. Where a
+    // row has up to four parts this takes 3-4 us less than the kernel of merges: its start,
+    // its rows' places, and one part less to read (rule: PagedRows).
+    u64* count = meet.count + block;
+    int n = parts, pos = part, step = 1;
+    for (; n > 1; n = (n + 3) / 4, pos /= 4, step *= 4) {
+      const int k0 = pos & ~3, size = min(4, n - k0), own = pos & 3;
+      if (size > 1) {
+        mr_store_far2(unit_ml, h == 0 && kg == 0 ? (pos * step * PF_ROWS + row) * 8 : GONE,
+                      make_float2(m, l));
+#pragma unroll
+        for (int j = 0; j < OWN; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            mr_store_far(unit_o, piece(pos * step, j, r),
+                         make_float4(o_acc[j][4 * r], o_acc[j][4 * r + 1],
+                                     o_acc[j][4 * r + 2], o_acc[j][4 * r + 3]));
+        if (!paged_last(count + k0 * step, size, reinterpret_cast<int*>(kv_lds)))
+          return;
+        float2 z[4];
+        bool on[4];                              // without keys: no part in the row
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          on[k] = k < size && (k0 + k) * step * tpp < list.n;
+          z[k] = mr_load_far2(unit_ml, on[k] ? ((k0 + k) * step * PF_ROWS + row) * 8
+                                             : GONE);
+        }
+        float top = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          if (k == own) z[k] = make_float2(m, l);
+          if (on[k]) top = fmaxf(top, z[k].x);
+        }
+        m = top;
+        if (top == -INFINITY) top = 0.0f;
+        l = 0.0f;
+        float w[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          w[k] = on[k] ? __builtin_amdgcn_exp2f(z[k].x - top) : 0.0f;
+          l += on[k] ? z[k].y * w[k] : 0.0f;
+        }
+        // in the order of the parts, whichever is the last
+        constexpr int JB = OWN < 2 ? OWN : 2;
+#pragma unroll
+        for (int j0 = 0; j0 < OWN; j0 += JB) {
+          float4 y[4][JB][4];
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int j = 0; j < JB; j++)
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                y[k][j][r] = mr_load_far(
+                    unit_o, on[k] && k != own ? piece((k0 + k) * step, j0 + j, r)
+                                              : GONE);
+#pragma unroll
+          for (int j = 0; j < JB; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const float4 mine =
+                  make_float4(o_acc[j0 + j][4 * r], o_acc[j0 + j][4 * r + 1],
+                              o_acc[j0 + j][4 * r + 2], o_acc[j0 + j][4 * r + 3]);
+              float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+              for (int k = 0; k < 4; k++) {
+                const float4 v = k == own ? mine : y[k][j][r];
+                a.x += on[k] ? v.x * w[k] : 0.0f;
+                a.y += on[k] ? v.y * w[k] : 0.0f;
+                a.z += on[k] ? v.z * w[k] : 0.0f;
+                a.w += on[k] ? v.w * w[k] : 0.0f;
+              }
+              o_acc[j0 + j][4 * r] = a.x;
+              o_acc[j0 + j][4 * r + 1] = a.y;
+              o_acc[j0 + j][4 * r + 2] = a.z;
+              o_acc[j0 + j][4 * r + 3] = a.w;
+            }
+        }
+      }
+      count += meet.units;
+    }
+  }
   if (!row_ok) return;
   const long grow = (long)(q_start + qi) * n_qheads + head;
-  // the parts of a row lie together (strided, the merge took up to 9 us more)
-  const int slot = (first * n_kv + kvh * parts) * PF_ROWS +
-                   (wid * 32 + c32) * parts + part;
-  if (SPLIT && part == 0 && h == 0 && kg == 0)
-    ws_at[grow] = make_int2(slot, parts);
-  if (!SPLIT || parts == 1) {
+  // for the merge, the parts of a row lie together (strided, it took up to 9 us more)
+  const long slot = block * PF_ROWS + row * parts + part;
+  if (SPLIT && meet.count == nullptr && part == 0 && h == 0 && kg == 0)
+    ws_at[grow] = make_int2((int)slot, parts);
+  if (!SPLIT || meets || parts == 1) {
     if (MORE && x.sink != nullptr)
       l += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f - m);
     const float inv = l != 0.0f ? 1.0f / l : 0.0f;
@@ -579,11 +686,11 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     return;
   }
   if (h == 0 && kg == 0) {
-    ws_ml[slot * 2L] = m;
-    ws_ml[slot * 2L + 1] = p_begin < i_end ? l : PAGED_ABSENT;
+    ws_ml[slot * 2] = m;
+    ws_ml[slot * 2 + 1] = p_begin < i_end ? l : PAGED_ABSENT;
   }
   if (p_begin >= i_end) return;
-  float* o = ws_o + (long)slot * D + 4 * h;
+  float* o = ws_o + slot * D + 4 * h;
 #pragma unroll
   for (int j = 0; j < OWN; j++)
 #pragma unroll
@@ -598,36 +705,47 @@ template <int ROWS>
 inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
   return (tokens * G + n_seqs * (ROWS - 1L)) / ROWS;
 }
-// Groups of waves, and parts of the keys. Parts (pf_parts): about two groups of waves per
-// CU are wanted, and parts of at least eight tiles of keys (four with 32-bit weights, whose
-// tiles take twice as long): the merge costs more than smaller ones save. At least six: 3
-// chunks of 93-261 tokens 36.5 us (eight: 31.8); up to 16 parts, not 8: 29.7 (34.9) for 50-300
-// tokens behind up to 9000. Measured (us, by parts 1 | 2 | 4 | 8), 32-bit weights: 2 x 64 rows
-// of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of 16 over 600 37 | 26 | 24 | 28; 1024
-// of 32 over 8000 (264 row tiles) 374 | 298 | 302 | 325; 4096 of 16 in a window (520 row
-// tiles) 69 | 87 | 111 | 182.
-//   Parts of two groups of waves, which leave half the partial results in memory (24 MB of
-// the 3 chunks'), where their larger units still fill the CUs, one turn of them and no more:
-// one sequence in 200-256 of at least three parts, several in up to 144 before they are
-// split; us, one | two groups: the 3 chunks 31.4 | 29.6, 2 x 200 behind 3000 43.7 | 41.1, 300 behind 2000 of 32/8
-// 37.2 | 31.5, 300 behind 12000 of 16/4 64.8 | 48.7, of 28/4 (204 units) 91 | 78, capped 1900
-// and 32/8 47.1 | 44; but 272 units of the last but one 110, two parts (256 units) of 1000
-// behind 500 of 16/4 capped 38.6 | 42.8, 31, 322 and 416 tokens of 32 heads (288) 30.5 | 35.7.
+// Groups of waves, and parts of the keys. Parts (pf_parts): about two groups of waves
+// per CU are wanted, and parts of at least eight tiles of keys (four with 32-bit
+// weights, whose tiles take twice as long): the merge costs more than smaller ones save.
+// At least six: 3 chunks of 93-261 tokens 36.5 us (eight: 31.8); up to 16 parts, not 8:
+// 29.7 (34.9) for 50-300 tokens behind up to 9000. Measured (us, by parts 1 | 2 | 4 |
+// 8), 32-bit weights: 2 x 64 rows of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of
+// 16 over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles) 374 | 298 | 302 |
+// 325; 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
+//   Parts of two groups of waves, which leave half the partial results in memory (24 MB
+// of the 3 chunks'), where their larger units still fill the CUs, one turn of them and
+// no more: one sequence in 200-256 of at least three parts, several in up to 144 before
+// they are split; us, one | two groups: the 3 chunks 31.4 | 29.6, 2 x 200 behind 3000
+// 43.7 | 41.1, 300 behind 2000 of 32/8 37.2 | 31.5, 300 behind 12000 of 16/4 64.8 |
+// 48.7, of 28/4 (204 units) 91 | 78, capped 1900 and 32/8 47.1 | 44; but 272 units of
+// the last but one 110, two parts (256 units) of 1000 behind 500 of 16/4 capped 38.6 |
+// 42.8, 31, 322 and 416 tokens of 32 heads (288) 30.5 | 35.7.
 //   Two groups of waves and one part where these fill one turn of the CUs: 128-wide
-// heads, up to 24 tiles, or for a single sequence that fills most of the CUs; us, as before
-// (parts) | two groups: 1024 tokens of 32/8 heads 34.5 (2) | 25.5, 28/4 32.5 (2) | 24.8, 3 x
-// 300 behind 1000 44 (2) | 33, 1000 behind 1000 49.5 (2) | 42.2, 700 20.9 (1) | 20.0, but 300
-// 13.2 (1) | 14.1; 300 behind 1000, 28/4 (66 workgroups) 27.3 | 28.5, 16/4 1000 behind 1000
-// (125) 34.9 (4) | 37.5; and one prompt in up to 448 workgroups, whose chains differ: 1200 of
-// 32/32 (19 tiles) 44 | 30, 1400
-// of 32/8 39 | 32.8, 2048 of 28/4 (448) 54.2 | 50, 32/8 (512) 55.5 | 56.4, 850 of 64/8 (14 tiles)
-// 29 | 31.4. 32-bit weights, 2 x 400 behind 500 of 32/8 in a window 46.3 (2) | 33, in
-// one of 512 41 (2) | 29.5, capped 51.8 |
-// 40, but 300 behind 1000 (75) 37 (4) | 42, 2000 of 16/4 capped 71 (2) | 73.7. 64-wide, two
-// workgroups to a CU: 8 prompts of 64-448 13.3 (1) | 12.4, 1700 (168) 27.8 (3) | 32.7.
+// heads, up to 24 tiles, or for a single sequence that fills most of the CUs; us, as
+// before (parts) | two groups: 1024 tokens of 32/8 heads 34.5 (2) | 25.5, 28/4 32.5 (2)
+// | 24.8, 3 x 300 behind 1000 44 (2) | 33, 1000 behind 1000 49.5 (2) | 42.2, 700 20.9
+// (1) | 20.0, but 300 13.2 (1) | 14.1; 300 behind 1000, 28/4 (66 workgroups) 27.3 |
+// 28.5, 16/4 1000 behind 1000 (125) 34.9 (4) | 37.5; and one prompt in up to 448
+// workgroups, whose chains differ: 1200 of 32/32 (19 tiles) 44 | 30, 1400 of 32/8 39 |
+// 32.8, 2048 of 28/4 (448) 54.2 | 50, 32/8 (512) 55.5 | 56.4, 850 of 64/8 (14 tiles) 29
+// | 31.4. 32-bit weights, 2 x 400 behind 500 of 32/8 in a window 46.3 (2) | 33, in one
+// of 512 41 (2) | 29.5, capped 51.8 | 40, but 300 behind 1000 (75) 37 (4) | 42, 2000 of
+// 16/4 capped 71 (2) | 73.7. 64-wide, two workgroups to a CU: 8 prompts of 64-448 13.3
+// (1) | 12.4, 1700 (168) 27.8 (3) | 32.7.
+//   The last part merges (meet), or a kernel of its own; us, kernel | last: the 3 chunks
+// 31 | 27, 90 and 200 behind 2300 and 900 of 32/8 29 | 23.4, 1700 of 64-wide heads 28.8
+// | 23.3, 300 behind 2000 of 32/8 31.3 | 26.4, 700 in a window 32.2 | 26.4; four parts
+// of few tiles, whose merge is short, 60 behind 2000 (64 units) 20.6 | 22.4, of 32 heads
+// (128) 21.3 | 23.5; up to eight 60 behind 4000 23.4 | 28.2, 31, 322 and 416 behind
+// 4052, 20 and 27 30.5 | 35.6, sixteen 50-300 behind up to 9000 28.6 | 30.4.
 // groups: KG; least: tiles of a part, 0 without parts; most: parts of a tile; units: tiles
 // and parts a grid holds; scratch: floats
-struct PagedRows { int groups = 1, least = 0, most = 1; long units = 0, scratch = 0; };
+struct PagedRows {
+  int groups = 1, least = 0, most = 1;
+  bool meet = false;
+  long units = 0, scratch = 0;
+};
 inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D,
                                  long max_blocks, int terms) {
   PagedRows x;
@@ -654,7 +772,10 @@ inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D
     x.least = x.groups == 2 ? 12 : D == 64 ? 4 : least;
     x.units = n_seqs > 1 ? row_tiles + PF_UNITS / x.groups / n_kv + 1
                          : row_tiles * x.most;
-    x.scratch = x.units * n_kv * PF_ROWS * (D + 2) + tokens * G * n_kv * 2;
+    x.meet = n_seqs > 1 ? tiles <= (x.groups == 2 ? 64 : 4 * x.least)
+                        : x.most <= 2 || (x.most <= 4 && wgs * x.most >= 160);
+    x.scratch = x.units * n_kv * (PF_ROWS * (D + 2) + (x.meet ? 4 : 0)) +
+                (x.meet ? 0 : tokens * G * n_kv * 2);
   }
   return x;
 }
@@ -678,12 +799,17 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
   const int G = n_qheads / n_kv;
   if (tokens == 0 || n_seqs <= 0) return;
   const long wgs = paged_rows_wgs(plan, tokens, n_seqs, G, n_kv);
+  PagedMeet meet;
   float* ws_ml = ws_o + wgs * PF_ROWS * D;
+  if (plan.least > 0) {
+    if (plan.meet) meet = paged_meet(ws_ml, wgs * PF_ROWS, 1);
+    meet.units = wgs;
+  }
   int2* ws_at = reinterpret_cast<int2*>(ws_ml + wgs * PF_ROWS * 2);
 #define PF_GO(KG, SPLIT)                                                       \
   hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG, SPLIT>),      \
                      dim3((unsigned)(wgs + ahead.wgs)), dim3(KG * 256), 0,     \
-                     stream, out, ws_o, ws_ml, ws_at, q, k_cache, v_cache,     \
+                     stream, out, ws_o, ws_ml, ws_at, meet, q, k_cache, v_cache, \
                      block_tables, cu_q, seq_lens, n_seqs, scale, G, n_kv,     \
                      max_blocks, q_stride, out_stride, plan.least, plan.most, x,  \
                      ahead)
@@ -692,7 +818,7 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
   else if (plan.least > 0) PF_GO(1, true);
   else PF_GO(1, false);
 #undef PF_GO
-  if (plan.least > 0)
+  if (plan.least > 0 && !plan.meet)
     paged_merge<D, MORE>(out, ws_o, ws_ml, ws_at, n_qheads, out_stride,
                          tokens * n_qheads, x, stream, cu_q, n_seqs);
 }

@@ -3,6 +3,7 @@
 #pragma once
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <random>
 
 #include "mfma_rows.h"
@@ -31,9 +32,10 @@ struct PagedMore {
 // again. Decoded rows stream their weights at the rate of memory, and gained nothing.)
 struct PagedAhead {
   static constexpr int N = 4;
+  int from = INT_MAX;                 // the first that does so (a kernel that asks for the
+  int wgs = 0;                        // size of its grid waits for it), how many do
   const unsigned short* at[N] = {};
   unsigned bytes[N] = {};
-  int wgs = 0;                        // that do so
 };
 // by workgroup `mine` of them, through LDS that it does not look at: 1 KB a wave
 XLLM_DEV void paged_fetch(const PagedAhead& a, int mine, unsigned short* lds) {
@@ -55,6 +57,7 @@ inline PagedAhead paged_ahead(long wgs, const void* const* at,
                               const long* bytes) {
   PagedAhead a;
   if (at == nullptr || wgs > 256 - 32) return a;
+  a.from = (int)wgs;
   a.wgs = (int)(256 - wgs);
   long room = std::min<long>(48 << 20, a.wgs * (450L << 10));
   for (int i = 0; i < PagedAhead::N; i++) {

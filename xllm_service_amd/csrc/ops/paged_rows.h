@@ -302,9 +302,8 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   const int wid = wave & 3, kg = KG > 1 ? wave >> 2 : 0;
   const int h = lane >> 5, c32 = lane & 31;
 
-  const int beyond = (int)blockIdx.x - (int)(gridDim.x - ahead.wgs);
-  if (!MORE && beyond >= 0) {
-    paged_fetch(ahead, beyond, kv_lds);
+  if (!MORE && (int)blockIdx.x >= ahead.from) {
+    paged_fetch(ahead, blockIdx.x - ahead.from, kv_lds);
     return;
   }
   const int kvh = blockIdx.x % n_kv;

@@ -18,9 +18,12 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 OPS = os.path.join(ROOT, "xllm_service_amd", "csrc", "ops")
 HYB = os.path.join(ROOT, "xllm_service_amd", "csrc", "hybrid")
 
-# hipcc only: fp32 math compiles to scalar-lane ops (no packed fp32 forms)
+# hipcc only: fp32 math compiles to scalar-lane ops (no packed fp32 forms); products
+# keep their sums in registers that other instructions read. A kernel that has a SIMD
+# for one wave got them in the other half of its registers, and its loops copied them
+# back and forth: 290 of 850 instructions of a tile in paged_short.h.
 HIP_FLAGS = ["-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-             "-packed-fp32-ops"]
+             "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 ext_modules = [
     CUDAExtension(

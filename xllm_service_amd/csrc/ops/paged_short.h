@@ -14,6 +14,9 @@
 // heads of 64 19.8 | 14.6, 300 of 16/4 in a window 17.3 | 13.7, capped 22.2 | 16.1. What a CU
 // pulls (61 KB/us: each wave has tiles of its own) bounds longer chains: 64 rows a wave,
 // half as much to pull, were slower (300 tokens 17, 100 behind 4000 60 | 40 for 32 rows).
+// A SIMD has one wave, whose products' sums would lie in the half of its registers that
+// only products read: with them in the other half (a flag of the build) 60 behind 500 of
+// 32/8 heads 13.1 -> 12.4, 100 behind 1000 18.0 -> 17.3, 2 x 500 of 12/12 of 64 14 -> 13.3.
 #pragma once
 #include "paged_rows.h"
 

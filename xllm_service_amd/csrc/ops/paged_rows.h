@@ -116,16 +116,24 @@ XLLM_DEV int pf_scan(int v) {
   return v;
 }
 
+// Which of `total` units, the longest first, workgroup b takes where a CU holds two and
+// `turn` come one to a CU: what is left over joins the shortest of those, the very shortest
+// the longest of them, so that the longest have a CU to themselves. (Joined to the longest
+// of all, 500 and 695 tokens of 28/4 heads, 268 workgroups, took 24.1 us, 22.7 so.)
+XLLM_DEV int pf_fold(int b, int total, int turn) {
+  const int over = total - turn;
+  if (over <= 0 || over > turn) return b;
+  return b >= turn ? turn + total - 1 - b : b < over ? turn - over + b : b - over;
+}
+
 // Row tile `b` of the batch, the longest chains of keys first whatever their
 // sequences: a tile of a sequence has ROWS rows (of query and head) fewer before it
 // than the next one, so all tiles sort into levels of WIDTH of those with at most
 // WIDTH tiles of a sequence to a level, which share its keys and stay together. The level
 // of tile b is found by halves, a lane counting its sequence's tiles above one. Up to 64
 // sequences; of more, one sequence after the other (pf_locate).
-//   Tiles past the first `turn` come in the reverse order if they are no more than
-// another `turn`: two workgroups share a CU then, and the longest chains meet the
-// shortest. By sequences, the tiles of two equal prompts met their likes: 2 x 1.8-2.3 k
-// in a window of 1024 59.5 -> 54.8 us, 4 x 512 of 32/8 heads 28.3 -> 22.8, 3 x 500
+//   Two turns of workgroups come folded (pf_fold). By sequences, the tiles of two equal
+// prompts met their likes: 2 x 1.8-2.3 k in a window of 1024 59.5 -> 54.8 us, 4 x 512 of 32/8 heads 28.3 -> 22.8, 3 x 500
 // capped 51.5 -> 40.2. WIDTH 1, 2 and 4: 40 x 60 behind 500, whose two tiles read the
 // same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500 and 300 of 64-wide heads 26.6,
 // 26.6, 27.6.
@@ -137,7 +145,7 @@ XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
   if (n_seqs == 1) {                             // without scans: 0.4 us of a small call
     const int q0 = cu_q[0], n = cu_q[1] - q0, all = (n * G + ROWS - 1) / ROWS;
     if (b >= all) return false;
-    if (b >= turn && all <= 2 * turn) b = turn + all - 1 - b;
+    b = pf_fold(b, all, turn);
     *place = {0, all - 1 - b, q0, n, seq_lens[0]};
     return true;
   }
@@ -152,7 +160,7 @@ XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
       pf_scan<false>(nt > 0 ? top : INT_MIN), 63);
   const int total = __builtin_amdgcn_readlane(pf_scan<true>(nt), 63);
   if (b >= total) return false;
-  if (b >= turn && total <= 2 * turn) b = turn + total - 1 - b;
+  b = pf_fold(b, total, turn);
   // its tiles from the top: [first, first + nt)
   const int first = nt > 0 ? (most - top) / ROWS : 0;
   const int depth = __builtin_amdgcn_readlane(pf_scan<false>(first + nt), 63);
@@ -209,8 +217,7 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& 
     const int p = max(min((tiles_of(keys) + 3) / 4, most), 1);
     const int all = (len * G + ROWS - 1) / ROWS * p;
     if (b >= all) return false;
-    const int turn = 256 / n_kv;                 // as in pf_longest
-    if (b >= turn && all <= 2 * turn) b = turn + all - 1 - b;
+    b = pf_fold(b, all, 256 / n_kv);
     *part = b % p;
     *parts = p;
     *first = b - b % p;
@@ -235,12 +242,16 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& 
   }
   const int some = PF_UNITS / groups;
   int per = max(least, (work * n_kv + some - 1) / some);
-  // a few workgroups left for another turn cost up to a third
+  // a few workgroups left for another turn cost up to a third, much longer parts more:
+  // 1100 and 1000 tokens of 16/4 heads, capped, 71 us in parts of 16 tiles, 56 of 11
   if (n_seqs <= 64)
-    for (int i = 0; i < 8; i++, per++) {
-      const int p = max(min((n + per - 1) / per, most), 1);
-      if (__builtin_amdgcn_readlane(pf_scan<true>(nt * p), 63) * n_kv <= PF_TURN / groups)
+    for (int q = per; q <= per + per / 4; q++) {
+      const int p = max(min((n + q - 1) / q, most), 1);
+      if (__builtin_amdgcn_readlane(pf_scan<true>(nt * p), 63) * n_kv <=
+          PF_TURN / groups) {
+        per = q;
         break;
+      }
     }
   int acc = 0;
   for (int base = 0; base < n_seqs; base += 64) {

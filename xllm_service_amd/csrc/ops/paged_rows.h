@@ -133,10 +133,10 @@ XLLM_DEV int pf_fold(int b, int total, int turn) {
 // of tile b is found by halves, a lane counting its sequence's tiles above one. Up to 64
 // sequences; of more, one sequence after the other (pf_locate).
 //   Two turns of workgroups come folded (pf_fold). By sequences, the tiles of two equal
-// prompts met their likes: 2 x 1.8-2.3 k in a window of 1024 59.5 -> 54.8 us, 4 x 512 of 32/8 heads 28.3 -> 22.8, 3 x 500
-// capped 51.5 -> 40.2. WIDTH 1, 2 and 4: 40 x 60 behind 500, whose two tiles read the
-// same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500 and 300 of 64-wide heads 26.6,
-// 26.6, 27.6.
+// prompts met their likes: 2 x 1.8-2.3 k in a window of 1024 59.5 -> 54.8 us, 4 x 512 of
+// 32/8 heads 28.3 -> 22.8, 3 x 500 capped 51.5 -> 40.2. WIDTH 1, 2 and 4: 40 x 60 behind
+// 500, whose two tiles read the same keys, 48.6, 46.0, 46.5 (46.7 by sequences), 1500
+// and 300 of 64-wide heads 26.6, 26.6, 27.6.
 template <int ROWS, int WIDTH>
 XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
                          int n_seqs, int G, int lane, PfPlace* place) {

@@ -631,6 +631,33 @@ def test_prefill_parts_meet(kv_heads, per, dim, lens, ctx):
         check(got, *want(q, k, v, table, lens, behind, scale))
 
 
+@pytest.mark.parametrize("kv_heads,per,lens,keys", [
+    (4, 4, [20, 33, 40, 31, 9], [3840, 3785, 3900, 3780, 100]),   # five and six parts
+    (2, 7, [70, 30, 18, 1], [3264, 3901, 3584, 3905]),            # the last ends early
+    (1, 1, [1, 128, 129, 5, 40, 64], [4096, 3840, 4090, 3901, 3111, 64]),
+    (8, 4, [60, 40], [4096, 3841]),
+])
+def test_prefill_parts_meet_twice(kv_heads, per, lens, keys):
+    """Five and six parts of two groups of waves: what is merged first is stored where
+    its first part was, which both groups read. Calls alone and among others end their
+    parts in different orders, and all of them have the same bits."""
+    dim, ctx = 128, [n - m for n, m in zip(keys, lens)]
+    rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(keys))
+    heads, scale = kv_heads * per, dim ** -0.5
+    q = rows[:, :heads * dim].unflatten(-1, (heads, dim)).contiguous()
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0))).int().cuda()
+    dev = [t.cuda() for t in (q, k, v, table)]
+    sl = torch.tensor(keys).int().cuda()
+    outs = [torch.empty_like(dev[0]) for _ in range(64)]
+    for i, out in enumerate(outs):
+        if i % 8 == 0:
+            torch.cuda.synchronize()
+        ops.paged_attn_prefill(*dev, cu, sl, scale, out=out)
+    check(outs[0], *want(q, k, v, table, lens, ctx, scale))
+    for out in outs[1:]:
+        assert torch.equal(out, outs[0])
+
+
 @pytest.mark.parametrize("opts", ["cap", "window", "sink"])
 def test_prefill_parts_with_options(opts):
     test_prefill_options_of_forms([40, 3, 200], [1700, 5, 600], 2, 4, 900, opts)

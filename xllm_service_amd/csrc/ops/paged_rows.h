@@ -671,6 +671,12 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
               o_acc[j0 + j][4 * r + 3] = a.w;
             }
         }
+        // the next round's store of (m, l) goes to the first of these parts, which
+        // the waves of the other group may not have read yet
+        if (KG > 1 && n > 4) {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();
+        }
       }
       count += meet.units;
     }

@@ -504,6 +504,20 @@ def test_decode_without_keys(dim, width):
         assert (out == 0).all()
 
 
+@pytest.mark.parametrize("dim,seqs,kv_heads,per", [
+    (128, 12, 8, 4), (64, 12, 8, 4), (64, 32, 6, 4), (128, 32, 4, 1),
+    (64, 16, 12, 1), (128, 100, 8, 2)])
+def test_decode_without_keys_of_many(dim, seqs, kv_heads, per):
+    """Tables without columns, pairs of sequence and key head by tens: zeros."""
+    k = torch.randn(3, kv_heads, PAGE, dim, device="cuda").to(torch.bfloat16)
+    q = torch.randn(seqs, kv_heads * per, dim, device="cuda").to(torch.bfloat16)
+    table = torch.zeros(seqs, 0, dtype=torch.int32, device="cuda")
+    sl = torch.zeros(seqs, dtype=torch.int32, device="cuda")
+    out = torch.full_like(q, 7.0)
+    ops.paged_attn_decode(q, k, k, table, sl, 0.1, out=out)
+    assert (out == 0).all()
+
+
 OPTIONS = {
     "plain": {},
     "window": dict(window=50),

@@ -150,7 +150,7 @@ static PagedSplit decode_split(long num_seqs, int n_kv_heads, int D,
     if (units > 192) return x;
     x.per = 16;
     x.least = units <= 128 ? 24 : 48;
-    x.parts = (int)std::min<long>(4, (max_blocks + 31) / 32);
+    x.parts = (int)std::min<long>(4, std::max<long>(1, (max_blocks + 31) / 32));
     return x;
   }
   x = paged_stream_split(num_seqs, n_kv_heads, max_blocks);

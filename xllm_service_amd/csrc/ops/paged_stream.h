@@ -455,7 +455,8 @@ inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
                                      long max_blocks, bool options = false,
                                      bool capped = false) {
   const long units = num_seqs * n_kv_heads;
-  const long table = (max_blocks * PA_BS + PA_KT - 1) / PA_KT;
+  // a table without columns, of sequences without keys, is one part like any other
+  const long table = std::max<long>(1, (max_blocks * PA_BS + PA_KT - 1) / PA_KT);
   PagedSplit x;
   if (units == 0) return x;
   if (units < 86) {

@@ -518,6 +518,33 @@ def test_decode_without_keys_of_many(dim, seqs, kv_heads, per):
     assert (out == 0).all()
 
 
+@pytest.mark.parametrize("tokens,keys,width,decode", [
+    (40, 30, 64, False), (40, 0, 64, False),         # parts that meet
+    (60, 20, 256, False),                            # parts of a kernel of merges
+    (40, 30, 10, False), (300, 250, 40, False),      # few rows, a group of waves,
+    (900, 700, 56, False),                           # two of them
+    (1, 0, 64, True)])
+def test_sinks_of_no_weight(tokens, keys, width, decode):
+    """A sink of -inf: rows without keys are zero, the others as without it."""
+    heads, kv_heads, dim, none = 32, 8, 128, min(keys, tokens) - tokens
+    g = torch.Generator().manual_seed(tokens)
+    k, v = (torch.randn(max(width, 1), kv_heads, PAGE, dim, generator=g)
+            .to(torch.bfloat16).cuda() for _ in range(2))
+    q = torch.randn(tokens, heads * dim, generator=g).to(torch.bfloat16).cuda()
+    table = torch.arange(width, dtype=torch.int32, device="cuda")[None]
+    cu = torch.tensor([0, tokens], dtype=torch.int32, device="cuda")
+    sl = torch.tensor([keys], dtype=torch.int32, device="cuda")
+    outs = []
+    for value in (-math.inf, -1e30):
+        sink = torch.full((heads,), value, device="cuda")
+        out = torch.full((tokens, heads, dim), 7.0, device="cuda")
+        H.capped_attn(q, k, v, table, None if decode else cu, sl, heads, 0.1, 0.0,
+                      out, sink=sink)
+        assert (out[:-none] == 0).all() and torch.isfinite(out).all()
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
 OPTIONS = {
     "plain": {},
     "window": dict(window=50),

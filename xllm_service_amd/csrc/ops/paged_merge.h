@@ -188,6 +188,14 @@ struct PagedSplit {
   }
 };
 
+// What the sink of a head adds to the sum of a row whose maximum is `top` (with the
+// factor of its scores). Rows without keys have no maximum, and a sink of -inf has no
+// weight for them either.
+XLLM_DEV float paged_sink(const PagedMore& x, int head, float top) {
+  return __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f -
+                                (top == -INFINITY ? 0.0f : top));
+}
+
 // four neighbouring results
 template <bool MORE>
 XLLM_DEV void paged_put(const PagedMore& x, void* out, long at, float a,

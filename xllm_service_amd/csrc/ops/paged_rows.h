@@ -688,8 +688,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   if (SPLIT && meet.count == nullptr && part == 0 && h == 0 && kg == 0)
     ws_at[grow] = make_int2((int)slot, parts);
   if (!SPLIT || meets || parts == 1) {
-    if (MORE && x.sink != nullptr)
-      l += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f - m);
+    if (MORE && x.sink != nullptr) l += paged_sink(x, head, m);
     const float inv = l != 0.0f ? 1.0f / l : 0.0f;
     const long to = (long)(q_start + qi) * out_stride + (long)head * D + 4 * h;
 #pragma unroll

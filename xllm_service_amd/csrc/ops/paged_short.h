@@ -263,8 +263,7 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
                  : 0.0f;
     if (w < n) sum += z.y * f[w];
   }
-  if (MORE && x.sink != nullptr)
-    sum += __builtin_amdgcn_exp2f(x.sink[head] * 1.4426950408889634f - top);
+  if (MORE && x.sink != nullptr) sum += paged_sink(x, head, top);
   const float inv = sum != 0.0f ? 1.0f / sum : 0.0f;
   // a wave writes one (two) of every four pieces of its rows
   const long to = (long)(q_start + qi) * out_stride + (long)head * D + 4 * h;

@@ -385,9 +385,7 @@ paged_attn_stream_kernel(
       a[0] += y.x * f; a[1] += y.y * f; a[2] += y.z * f; a[3] += y.w * f;
     }
     if (!SPLIT || parts == 1) {
-      if (MORE && x.sink != nullptr)
-        L += __builtin_amdgcn_exp2f(
-            x.sink[kvh * G + row] * 1.4426950408889634f - M);
+      if (MORE && x.sink != nullptr) L += paged_sink(x, kvh * G + row, M);
       const float inv = L != 0.0f ? 1.0f / L : 0.0f;
       paged_put<MORE>(x, out, (long)seq * out_stride +
                       (long)(kvh * G + row) * D + at,

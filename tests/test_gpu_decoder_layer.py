@@ -304,3 +304,18 @@ def test_layers_against_64_bits(hidden, inter, heads, kv_heads, bias, gate_bias,
 def test_layers_of_small_weights(prompts):
     """Weights of no whole kilobytes, which CUs that attention leaves idle fetch."""
     test_layers_against_64_bits(136, 40, 2, 1, False, False, False, prompts, [])
+
+
+@pytest.mark.parametrize("prompts", [[90], [40, 70]])
+def test_layers_of_weights_off_16_bytes(prompts, monkeypatch):
+    """Weights that begin within 16 bytes, which nothing fetches by as many."""
+    def layer_of(*args, make=LlamaDecoderLayer):
+        layer = make(*args)
+        for m in (layer.attn.qkv_proj, layer.attn.o_proj, layer.mlp.gate_up,
+                  layer.mlp.down):
+            room = torch.empty(m.weight.numel() + 4, dtype=torch.bfloat16)
+            m.weight = torch.nn.Parameter(room[4:].view_as(m.weight))
+            assert m.weight.is_contiguous() and m.weight.data_ptr() % 16 == 8
+        return layer
+    monkeypatch.setitem(globals(), "LlamaDecoderLayer", layer_of)
+    test_layers_against_64_bits(256, 512, 2, 1, False, False, False, prompts, [])

@@ -266,7 +266,9 @@ struct Ahead {
   const void* at[4] = {};
   long bytes[4] = {};
   void add(int i, const torch::Tensor& w) {
-    if (!w.is_contiguous()) return;
+    // read by 16 bytes
+    if (!w.is_contiguous() || reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 != 0)
+      return;
     at[i] = w.data_ptr();
     bytes[i] = w.numel() * w.element_size();
   }

@@ -434,6 +434,50 @@ def test_narrow_decode_forms(keys, kv_heads, per):
     check(got, *want(q, k, v, table, [1] * len(keys), ctx, 0.125))
 
 
+def on_litter(call, size, fill):
+    """call(), which asks for `size` bytes, on memory that holds `fill`, and that
+    memory: the allocator gives a freed block between two that stay to the next one
+    who asks for as much."""
+    held = [torch.full((size // 8,), fill, dtype=torch.int64, device="cuda")
+            for _ in range(8)]
+    for i in range(len(held)):
+        at, held[i] = held[i].data_ptr(), None
+        call()
+        held[i] = torch.empty(size // 8, dtype=torch.int64, device="cuda")
+        if held[i].data_ptr() == at:
+            return held[i]
+    assert False, "scratch lies elsewhere"
+
+
+def over_litter(call, out, sl, lengths, ref):
+    """call() into out, for `lengths` in sl, over scratch of several values: alone,
+    and in replays of a graph, to the same bits. The first lengths are split."""
+    call()
+    was = torch.cuda.memory_stats()["requested_bytes.all.allocated"]
+    call()
+    size = torch.cuda.memory_stats()["requested_bytes.all.allocated"] - was
+    assert size > 0
+    refs = {tuple(n): ref(n) for n in lengths}
+    for fill in (0, -1, 0x7f7f7f7f7f7f7f01):
+        out.fill_(3.0)
+        scratch = on_litter(call, size, fill)
+        assert (scratch != fill).any()             # parts were in it
+        check(out, *refs[tuple(lengths[0])])
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            scratch = on_litter(call, size, fill)
+        for now in lengths:
+            sl.copy_(torch.tensor(now))
+            out.fill_(3.0)
+            graph.replay()
+            got = out.clone()
+            assert now != lengths[0] or (scratch != fill).any()
+            call()
+            assert torch.equal(got, out)
+            check(got, *refs[tuple(now)])
+
+
 @pytest.mark.parametrize("dim,keys,kv_heads,per", [
     (128, [12 * 32, 12 * 32 + 1, 17 * 32], 8, 4),     # where parts begin
     (128, [32 * 32 + 1, 65 * 32, 8 * 65 * 32 + 5], 1, 7),   # eight of them, more
@@ -451,29 +495,11 @@ def test_decode_parts_meet(dim, keys, kv_heads, per):
     dev = [t.cuda() for t in (q, k, v, table)]
     sl = torch.tensor(keys, dtype=torch.int32, device="cuda")
     out = torch.empty_like(dev[0])
-
-    def litter():              # where scratch will be: any values
-        for fill in (0, -1, 0x7f7f7f7f7f7f7f01):
-            torch.full((1 << 18,), fill, dtype=torch.int64, device="cuda")
-
-    def step():
-        litter()
-        ops.paged_attn_decode(*dev, sl, scale, out=out)
-    step()
-    check(out, *want(q, k, v, table, [1] * len(keys), ctx, scale))
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        step()
-    for lens in (keys, keys, [max(1, n // 2) for n in keys], keys):
-        sl.copy_(torch.tensor(lens))
-        out.fill_(3.0)
-        graph.replay()
-        got = out.clone()
-        ops.paged_attn_decode(*dev, sl, scale, out=out)
-        assert torch.equal(got, out)
-        check(got, *want(q, k, v, table, [1] * len(lens),
-                         [n - 1 for n in lens], scale))
+    over_litter(
+        lambda: ops.paged_attn_decode(*dev, sl, scale, out=out), out, sl,
+        [keys, keys, [max(1, n // 2) for n in keys], keys],
+        lambda lens: want(q, k, v, table, [1] * len(lens), [n - 1 for n in lens],
+                          scale))
 
 
 def test_decode_standout_scores():
@@ -649,27 +675,14 @@ def test_prefill_parts_meet(kv_heads, per, dim, lens, ctx):
     q = rows[:, :heads * dim].unflatten(-1, (heads, dim)).contiguous()
     cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0))).int().cuda()
     dev = [t.cuda() for t in (q, k, v, table)]
-    sl = torch.tensor([n + c for n, c in zip(lens, ctx)]).int().cuda()
+    keys = [[n + c // by for n, c in zip(lens, ctx)] for by in (1, 3)]
+    sl = torch.tensor(keys[0]).int().cuda()
     out = torch.empty_like(dev[0])
-
-    def step():
-        for fill in (0, -1, 0x7f7f7f7f7f7f7f01):
-            torch.full((1 << 22,), fill, dtype=torch.int64, device="cuda")
-        ops.paged_attn_prefill(*dev, cu, sl, scale, out=out)
-    step()
-    check(out, *want(q, k, v, table, lens, ctx, scale))
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        step()
-    for behind in (ctx, ctx, [c // 3 for c in ctx], ctx):
-        sl.copy_(torch.tensor([n + c for n, c in zip(lens, behind)]))
-        out.fill_(3.0)
-        graph.replay()
-        got = out.clone()
-        ops.paged_attn_prefill(*dev, cu, sl, scale, out=out)
-        assert torch.equal(got, out)
-        check(got, *want(q, k, v, table, lens, behind, scale))
+    over_litter(
+        lambda: ops.paged_attn_prefill(*dev, cu, sl, scale, out=out), out, sl,
+        [keys[0], keys[0], keys[1], keys[0]],
+        lambda now: want(q, k, v, table, lens, [m - n for m, n in zip(now, lens)],
+                         scale))
 
 
 @pytest.mark.parametrize("kv_heads,per,lens,keys", [

@@ -50,7 +50,7 @@ void launch_paged_attn_prefill(unsigned short*, float*, const unsigned short*,
                                const unsigned short*, const unsigned short*,
                                const int*, const int*, const int*, long, int,
                                float, int, int, int, int, long, long,
-                               const void* const*, const long*, hipStream_t);
+                               const void* const*, const long*, long, hipStream_t);
 void launch_greedy_sample(long*, const unsigned short*, int, int, hipStream_t);
 void launch_mfma_gemm(unsigned short*, const unsigned short*,
                       const unsigned short*, const unsigned short*, int, int,
@@ -265,6 +265,7 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
 struct Ahead {
   const void* at[4] = {};
   long bytes[4] = {};
+  long streamed = 0;             // of the caches of decoded rows, before them
   void add(int i, const torch::Tensor& w) {
     // read by 16 bytes
     if (!w.is_contiguous() || reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 != 0)
@@ -322,7 +323,7 @@ static void prefill_attn(torch::Tensor out, torch::Tensor q,
       cu_q.data_ptr<int>(), seq_lens.data_ptr<int>(), tokens, n_seqs,
       (float)scale, n_qheads, n_kv, D, block_tables.size(1), q.stride(0),
       out.stride(0), ahead ? ahead->at : nullptr,
-      ahead ? ahead->bytes : nullptr, cur_stream());
+      ahead ? ahead->bytes : nullptr, ahead ? ahead->streamed : 0, cur_stream());
 }
 void paged_attn_prefill(torch::Tensor out, torch::Tensor q,
                         torch::Tensor k_cache, torch::Tensor v_cache,
@@ -666,6 +667,9 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor>> decoder_layers(
       ahead.add(1, p.gate_up_w);
       ahead.add(2, p.down_w);
       if (i + 1 < layers.size()) ahead.add(3, layers[i + 1].qkv_w);
+      if (n_decode > 0)
+        ahead.streamed = decode_tables.value().numel() * 4 *
+                         p.k_cache.size(1) * p.k_cache.size(2) * D;
       prefill_attn(out3.slice(0, 0, n_prefill), q.slice(0, 0, n_prefill),
                    p.k_cache, p.v_cache, prefill_tables.value(), cu_q.value(),
                    prefill_lens.value(), scale, &ahead);

@@ -20,7 +20,8 @@ long paged_attn_prefill_scratch(long tokens, int n_seqs, int G, int n_kv, int D,
   return prompts(tokens, n_seqs, G, n_kv, D, max_blocks).scratch;
 }
 
-// ahead: four pieces of memory that is read next, or null
+// ahead: four pieces of memory that is read next, or null; streamed: bytes that are
+// read before them
 void launch_paged_attn_prefill(unsigned short* out, float* ws,
                                const unsigned short* q,
                                const unsigned short* k_cache,
@@ -30,15 +31,15 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws,
                                float scale, int n_qheads, int n_kv, int D,
                                int max_blocks, long q_stride, long out_stride,
                                const void* const* ahead, const long* ahead_bytes,
-                               hipStream_t stream) {
+                               long streamed, hipStream_t stream) {
   if (tokens == 0 || n_seqs <= 0) return;
   const int G = n_qheads / n_kv;
   const PagedPrompts p = prompts(tokens, n_seqs, G, n_kv, D, max_blocks);
   if (p.few) {
     auto go = D == 128 ? paged_short<128, 1, false> : paged_short<64, 3, false>;
     const PagedAhead a =
-        paged_ahead(paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv, ahead,
-                    ahead_bytes);
+        paged_ahead(paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv,
+                    max_blocks * (long)PF_BS, ahead, ahead_bytes, streamed);
     go(out, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
        scale, n_qheads, n_kv, max_blocks, q_stride, out_stride, PagedMore{}, a,
        stream);
@@ -51,8 +52,9 @@ void launch_paged_attn_prefill(unsigned short* out, float* ws,
                stream);
     return;
   }
-  const PagedAhead a = paged_ahead(
-      paged_rows_wgs(p, tokens, n_seqs, G, n_kv), ahead, ahead_bytes);
+  const PagedAhead a =
+      paged_ahead(paged_rows_wgs(p, tokens, n_seqs, G, n_kv),
+                  max_blocks * (long)PF_BS, ahead, ahead_bytes, streamed);
   auto go = D == 128 ? paged_rows<128, 1, false> : paged_rows<64, 3, false>;
   go(out, ws, q, k_cache, v_cache, block_tables, cu_q, seq_lens, tokens, n_seqs,
      scale, n_qheads, n_kv, max_blocks, q_stride, out_stride, p, PagedMore{},

@@ -51,15 +51,28 @@ XLLM_DEV void paged_fetch(const PagedAhead& a, int mine, unsigned short* lds) {
 }
 
 // What the CUs that `wgs` workgroups leave can fetch of N pieces while those run: a CU
-// pulls 60 KB/us, memory 5 MB/us. 300 rows of 2048, 46 MB a layer: up to 24 MB 509 us, 32
-// 508, 41 (400 KB a CU) 502, all 490; 150 of 4096, 184 MB: 41 MB 821, 52 835.
-inline PagedAhead paged_ahead(long wgs, const void* const* at,
-                              const long* bytes) {
+// pulls 60 KB/us, memory 5 MB/us. Rows that see few keys are done sooner. Us a layer,
+// nothing fetched | 300 | 450 KB a CU: 40 rows of 4096 71.8 | 69.8 | 70.2, 200 (keys) 107.8
+// | 106.9 | 109.0, 300 137.2 | 134.9 | 134.7; of 2048 100 49.6 | 47.1 | 47.0, 300 61.5 | 58.9 |
+// 56.8, 600 93.8 | 89.8 | 89.5. 60 and 120 KB gain nothing: the first product reads most of
+// its weights from memory all the same.
+//   streamed: what decoded rows of the same step read of their caches before the first
+// weight is used, through the same cache in front of memory. Us a layer, nothing | 300 KB a
+// CU beside rows of 600-1400 keys, MB of their pages: 100 rows of 2048 and 16 (46 MB) 64.4 |
+// 59.4, 64 (180) 79.7 | 77.6, 96 (270) 95.3 | 97.6, 128 106.5 | 108.9; of 4096 16 (90) 110.9 |
+// 106.5, 32 (180) 127.9 | 124.1, 48 (270) 143 | 144, 64 154.8 | 158.1; 300 rows, which fetch
+// 48 MB, and 16 157.1 | 154.9, 32 174.2 | 176.6.
+inline PagedAhead paged_ahead(long wgs, long keys, const void* const* at,
+                              const long* bytes, long streamed) {
   PagedAhead a;
   if (at == nullptr || wgs > 256 - 32) return a;
+  const long cus = 256 - wgs;
+  const long most =
+      std::min<long>(48 << 20, cus * ((keys <= 256 ? 300L : 450L) << 10));
+  if (most + streamed > 224L << 20) return a;
   a.from = (int)wgs;
-  a.wgs = (int)(256 - wgs);
-  long room = std::min<long>(48 << 20, a.wgs * (450L << 10));
+  a.wgs = (int)cus;
+  long room = most;
   for (int i = 0; i < PagedAhead::N; i++) {
     const long n = std::min(bytes[i], room) / 1024 * 1024;
     if (n <= 0) continue;

@@ -663,7 +663,8 @@ def test_prefill_parts_by_length(kv_heads, per, dim, lens, ctx, sign):
 
 
 @pytest.mark.parametrize("kv_heads,per,dim,lens,ctx", [
-    (2, 4, 128, [50, 60, 9], [3900, 100, 700]),      # six parts of two groups: two rounds
+    (2, 4, 128, [50, 60, 9], [3900, 100, 700]),      # parts of a kernel of merges
+    (8, 4, 128, [60, 200, 40], [4000, 100, 700]),    # six of two groups
     (8, 4, 128, [300], [2000]),                      # three of one sequence
     (12, 1, 64, [420], [900]),                       # one group
 ])
@@ -685,17 +686,29 @@ def test_prefill_parts_meet(kv_heads, per, dim, lens, ctx):
                          scale))
 
 
-@pytest.mark.parametrize("kv_heads,per,lens,keys", [
-    (4, 4, [20, 33, 40, 31, 9], [3840, 3785, 3900, 3780, 100]),   # five and six parts
-    (2, 7, [70, 30, 18, 1], [3264, 3901, 3584, 3905]),            # the last ends early
-    (1, 1, [1, 128, 129, 5, 40, 64], [4096, 3840, 4090, 3901, 3111, 64]),
-    (8, 4, [60, 40], [4096, 3841]),
+@pytest.mark.parametrize("kv_heads,per,dim,lens,keys", [
+    (4, 4, 128, [20, 33, 40, 31, 9], [3840, 3785, 3900, 3780, 100]),
+    (2, 7, 128, [70, 30, 18, 1], [3264, 3901, 3584, 3905]),
+    (1, 1, 128, [1, 128, 129, 5, 40, 64], [4096, 3840, 4090, 3901, 3111, 64]),
+    (8, 4, 128, [60, 40], [4096, 3841]),
+    # two groups of waves, the last part merges: four parts, six, eight, and one of 13 tiles
+    (8, 4, 128, [60, 200, 40], [2113, 700, 90]),
+    (8, 4, 128, [60, 200, 40], [4060, 300, 4033]),
+    (8, 4, 128, [60, 200, 40, 1], [7100, 8190, 40, 6145]),
+    (4, 7, 128, [40, 33, 120, 9], [832, 833, 400, 9]),
+    # one group, up to four; in a turn by longer parts, or none
+    (8, 4, 128, [500, 60, 90], [1800, 2049, 90]),
+    (8, 4, 128, [618, 647], [1212, 1288]),
+    (4, 4, 128, [1000, 1100], [1000, 1100]),
+    (12, 1, 64, [300, 200, 129], [1800, 1537, 300]),
+    # few rows of many key heads
+    (32, 1, 128, [10, 12, 9], [2000, 700, 3454]),
 ])
-def test_prefill_parts_meet_twice(kv_heads, per, lens, keys):
-    """Five and six parts of two groups of waves: what is merged first is stored where
-    its first part was, which both groups read. Calls alone and among others end their
-    parts in different orders, and all of them have the same bits."""
-    dim, ctx = 128, [n - m for n, m in zip(keys, lens)]
+def test_prefill_parts_of_several(kv_heads, per, dim, lens, keys):
+    """Parts by each sequence's length, which the last one merges where row tiles are
+    many. Calls alone and among others end their parts in different orders, and all of
+    them have the same bits."""
+    ctx = [n - m for n, m in zip(keys, lens)]
     rows, k, v, table = make(lens, ctx, kv_heads, per, dim, sum(keys))
     heads, scale = kv_heads * per, dim ** -0.5
     q = rows[:, :heads * dim].unflatten(-1, (heads, dim)).contiguous()

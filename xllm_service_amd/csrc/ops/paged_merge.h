@@ -287,7 +287,6 @@ XLLM_DEV void paged_add_parts(const Ml& ml, const O& o, int parts, float& M,
 struct PagedMeet {
   unsigned long long* count = nullptr;   // [units]
   unsigned long long tag = 0;            // low 8 bits: none
-  long units = 0;                        // counters, where there are two for each
 };
 typedef unsigned long long u64;
 // by one thread of a workgroup, early: at, its unit's counter

@@ -29,8 +29,8 @@
 //
 // Few row tiles over a long context leave most of the chip idle: then the
 // keys of a tile are split over workgroups, by the length of its own sequence
-// (pf_parts). Of a few parts the last one to finish merges the fp32 partial results
-// of all (PagedMeet), of many a second kernel does, which all CUs share.
+// (pf_parts). Of up to eight parts the last one to finish merges the fp32 partial results
+// of all (PagedMeet), of more a second kernel does, which all CUs share.
 //
 // Bound by the matrix pipe and the vector unit in turn: a tile costs a wave
 // 32 products (about 1000 cycles) and about as many cycles of exponentials,
@@ -189,14 +189,16 @@ XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
 
 #define PF_UNITS 448       // groups of waves that a batch's keys are split over,
 #define PF_TURN 512        // and that the CUs hold at once
+// parts that the last one merges, at most, by groups of waves
+#define PF_MEET(KG) ((KG) > 1 ? 8 : 4)
 
 // Unit `b` of a batch whose keys are split: a row tile and one of its parts, b - part the
 // tile's first. One sequence: up to `most` equal parts, of at least four tiles of keys.
 // Several: parts of `per` tiles, so that all of the batch walk about as many, whatever its
-// sequences' lengths. Never more parts than ceil(n / per), or than `most` for one sequence:
-// the grid and the scratch hold that many units (PagedRows), and a row whose unit was not
-// in the grid would leave the merge without its place. PF_UNITS: just under two groups of
-// waves to a CU.
+// sequences' lengths; if the last part merges, four of them and more only of twelve tiles.
+// Never more parts than ceil(n / per), or than `most`: the grid and the scratch hold that
+// many units (PagedRows), and a row whose unit was not in the grid would leave the merge
+// without its place. PF_UNITS: just under two groups of waves to a CU.
 //   The same number of parts for all, as many as the longest's table asks for, left one
 // sequence's chain to be waited for: 50, 60, 300 and 20 tokens behind 9000, 100, 0 and 700
 // of 32/8 heads 59.4 -> 34.4 us, of 28/4 51.4 -> 29, 31, 322 and 416 behind 4052, 20 and
@@ -242,21 +244,44 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& 
   }
   const int some = PF_UNITS / groups;
   int per = max(least, (work * n_kv + some - 1) / some);
-  // a few workgroups left for another turn cost up to a third, much longer parts more:
-  // 1100 and 1000 tokens of 16/4 heads, capped, 71 us in parts of 16 tiles, 56 of 11
-  if (n_seqs <= 64)
-    for (int q = per; q <= per + per / 4; q++) {
-      const int p = max(min((n + q - 1) / q, most), 1);
-      if (__builtin_amdgcn_readlane(pf_scan<true>(nt * p), 63) * n_kv <=
-          PF_TURN / groups) {
-        per = q;
-        break;
-      }
+  const bool few = most <= 8;
+  auto parts_of = [&](int q) {
+    const int p = max(min((n + q - 1) / q, most), 1);
+    return few ? min(p, max(4, (n + 11) / 12)) : p;
+  };
+  if (n_seqs <= 64) {
+    auto fits = [&](int p) {
+      return __builtin_amdgcn_readlane(pf_scan<true>(nt * p), 63) * n_kv <=
+             PF_TURN / groups;
+    };
+    auto chain = [&](int p) {
+      return __builtin_amdgcn_readlane(
+          pf_scan<false>(nt > 0 ? (n + p - 1) / p : 0), 63);
+    };
+    // Units left for another turn are waited for: parts are lengthened until there are
+    // none, unless that takes longer than the turn. 2 x 600 behind 500 of 28/4 in a window
+    // 53.9 us in two parts of 6 tiles, 39.1 in one of 11, 2 x 420 behind 3600-6900 of 32/8,
+    // capped, 232 and 194; but 1000 and 1100 of 16/4, capped, 50.4 in two of up to 9, 65.9 in
+    // one. Two groups of waves, 6 x 337 behind 230 of 8/1 in a window 34.9 and 24.8.
+    if (!fits(parts_of(per))) {
+      // of a causal prompt the row tiles are half as long on average as the last of them
+      const int seen = min(n, (max(keys - len / 2, 0) + PF_KT - 1) / PF_KT);
+      const int mean = __builtin_amdgcn_readlane(pf_scan<true>(nt * seen), 63);
+      const int now = chain(parts_of(per)), step = max(per / 8, 1);
+      const int turns = groups > 1 ? 2 * now
+                                   : now + (int)((float)now * mean / max(work, 1)) +
+                                         (MORE ? 2 : 4);
+      for (int q = per + step; q <= 2 * per; q += step)
+        if (fits(parts_of(q))) {
+          if (chain(parts_of(q)) <= turns) per = q;
+          break;
+        }
     }
+  }
   int acc = 0;
   for (int base = 0; base < n_seqs; base += 64) {
     if (n_seqs > 64) look(base + lane);
-    const int p = max(min((n + per - 1) / per, most), 1);
+    const int p = parts_of(per);
     const int upto = acc + pf_scan<true>(nt * p);
     const unsigned long long hit = __ballot(b < upto);
     if (hit != 0) {
@@ -288,7 +313,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     float* __restrict__ ws_o,                // [blocks][PF_ROWS * D], a block for a part
     float* __restrict__ ws_ml,               // [blocks][PF_ROWS][2]
     int2* __restrict__ ws_at,                // [total_q*n_qheads]: first slot, parts
-    const PagedMeet meet,                    // [2][blocks]: by fours, by sixteens
+    const PagedMeet meet,                    // [blocks]: its first part's counts
     const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
     const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
     const unsigned short* __restrict__ v_cache,
@@ -345,12 +370,9 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   const int tpp = (max(list.n, 0) + parts - 1) / parts;
   // its parts' place: their blocks lie together
   const long block = SPLIT ? (long)first * n_kv + kvh * parts : 0;
-  u64 seen[2] = {0, 0};
+  u64 seen = 0;
   const bool meets = SPLIT && parts > 1 && meet.count != nullptr;
-  if (meets && threadIdx.x == 0) {
-    seen[0] = paged_seen(meet.count + block + (part & ~3));
-    if (parts > 4) seen[1] = paged_seen(meet.count + meet.units + block);
-  }
+  if (meets && threadIdx.x == 0) seen = paged_seen(meet.count + block);
   const int p_begin = part * tpp;
   const int i_end = min(list.n, p_begin + tpp);
   const int i_begin = p_begin + kg;              // every KG-th of a group's
@@ -538,10 +560,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   // ---- epilogue: o_acc[dt][r] = O[row][dt*32 + 8*(r>>2) + 4h + (r&3)] --------
   l = pair_sum(l);
   m = m == -INFINITY ? m : m * sc.c;
-  if (meets && threadIdx.x == 0) {
-    paged_open(meet.count + block + (part & ~3), seen[0], meet.tag);
-    if (parts > 4) paged_open(meet.count + meet.units + block, seen[1], meet.tag);
-  }
+  if (meets && threadIdx.x == 0) paged_open(meet.count + block, seen, meet.tag);
   constexpr int OWN = DT / KG;                   // column tiles a group finishes
   const int dt0 = kg * OWN;
   constexpr unsigned GONE = 0x7ffffff0;          // out of the bounds: no store, zeros
@@ -592,93 +611,91 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
       }
   }
   if (meets) {
-    // ---- the last of four parts merges them, the last of four fours those -------
-    // A wave writes and reads its sums as its lanes hold them, 1 KB at a time. Where a
-    // row has up to four parts this takes 3-4 us less than the kernel of merges: its start,
-    // its rows' places, and one part less to read (rule: PagedRows).
-    u64* count = meet.count + block;
-    int n = parts, pos = part, step = 1;
-    for (; n > 1; n = (n + 3) / 4, pos /= 4, step *= 4) {
-      const int k0 = pos & ~3, size = min(4, n - k0), own = pos & 3;
-      if (size > 1) {
-        mr_store_far2(unit_ml, h == 0 && kg == 0 ? (pos * step * PF_ROWS + row) * 8 : GONE,
-                      make_float2(m, l));
+    // ---- the last of a few parts merges them -------------------------------
+    // A wave writes and reads its sums as its lanes hold them, 1 KB at a time: 3-4 us
+    // less than the kernel of merges takes, with its start, its rows' places, and one part
+    // more to read. More parts by fours, and those again, took longer than that kernel
+    // (7 to 25% of calls of 20 to 50 us).
+    constexpr int MEET = PF_MEET(KG);
+    mr_store_far2(unit_ml, h == 0 && kg == 0 ? (part * PF_ROWS + row) * 8 : GONE,
+                  make_float2(m, l));
 #pragma unroll
-        for (int j = 0; j < OWN; j++)
+    for (int j = 0; j < OWN; j++)
 #pragma unroll
-          for (int r = 0; r < 4; r++)
-            mr_store_far(unit_o, piece(pos * step, j, r),
-                         make_float4(o_acc[j][4 * r], o_acc[j][4 * r + 1],
-                                     o_acc[j][4 * r + 2], o_acc[j][4 * r + 3]));
-        if (!paged_last(count + k0 * step, size, reinterpret_cast<int*>(kv_lds)))
-          return;
-        float2 z[4];
-        bool on[4];                              // without keys: no part in the row
+      for (int r = 0; r < 4; r++)
+        mr_store_far(unit_o, piece(part, j, r),
+                     make_float4(o_acc[j][4 * r], o_acc[j][4 * r + 1],
+                                 o_acc[j][4 * r + 2], o_acc[j][4 * r + 3]));
+    if (!paged_last(meet.count + block, parts, reinterpret_cast<int*>(kv_lds)))
+      return;
+    float2 z[MEET];
+    bool on[MEET];                            // without keys: no part in the row
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          on[k] = k < size && (k0 + k) * step * tpp < list.n;
-          z[k] = mr_load_far2(unit_ml, on[k] ? ((k0 + k) * step * PF_ROWS + row) * 8
-                                             : GONE);
-        }
-        float top = -INFINITY;
+    for (int k = 0; k < MEET; k++) {
+      on[k] = k < parts && k * tpp < list.n;
+      z[k] = mr_load_far2(unit_ml, on[k] ? (k * PF_ROWS + row) * 8 : GONE);
+    }
+    float top = -INFINITY;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          if (k == own) z[k] = make_float2(m, l);
-          if (on[k]) top = fmaxf(top, z[k].x);
-        }
-        m = top;
-        if (top == -INFINITY) top = 0.0f;
-        l = 0.0f;
-        float w[4];
+    for (int k = 0; k < MEET; k++) {
+      if (k == part) z[k] = make_float2(m, l);
+      if (on[k]) top = fmaxf(top, z[k].x);
+    }
+    m = top;
+    if (top == -INFINITY) top = 0.0f;
+    l = 0.0f;
+    float w[MEET];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          w[k] = on[k] ? __builtin_amdgcn_exp2f(z[k].x - top) : 0.0f;
-          l += on[k] ? z[k].y * w[k] : 0.0f;
-        }
-        // in the order of the parts, whichever is the last
-        constexpr int JB = OWN < 2 ? OWN : 2;
+    for (int k = 0; k < MEET; k++) {
+      w[k] = on[k] ? __builtin_amdgcn_exp2f(z[k].x - top) : 0.0f;
+      l += on[k] ? z[k].y * w[k] : 0.0f;
+    }
+    // in the order of the parts, whichever is the last
+    constexpr int JB = OWN < 2 ? OWN : 2, KB = 4;
 #pragma unroll
-        for (int j0 = 0; j0 < OWN; j0 += JB) {
-          float4 y[4][JB][4];
+    for (int j0 = 0; j0 < OWN; j0 += JB) {
+      float4 sum[JB][4];
 #pragma unroll
-          for (int k = 0; k < 4; k++)
+      for (int k0 = 0; k0 < MEET; k0 += KB) {
+        if (k0 >= parts) break;                  // uniform
+        float4 y[KB][JB][4];
 #pragma unroll
-            for (int j = 0; j < JB; j++)
-#pragma unroll
-              for (int r = 0; r < 4; r++)
-                y[k][j][r] = mr_load_far(
-                    unit_o, on[k] && k != own ? piece((k0 + k) * step, j0 + j, r)
-                                              : GONE);
+        for (int k = 0; k < KB; k++)
 #pragma unroll
           for (int j = 0; j < JB; j++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-              const float4 mine =
-                  make_float4(o_acc[j0 + j][4 * r], o_acc[j0 + j][4 * r + 1],
-                              o_acc[j0 + j][4 * r + 2], o_acc[j0 + j][4 * r + 3]);
-              float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            for (int r = 0; r < 4; r++)
+              y[k][j][r] = mr_load_far(
+                  unit_o, on[k0 + k] && k0 + k != part ? piece(k0 + k, j0 + j, r)
+                                                       : GONE);
 #pragma unroll
-              for (int k = 0; k < 4; k++) {
-                const float4 v = k == own ? mine : y[k][j][r];
-                a.x += on[k] ? v.x * w[k] : 0.0f;
-                a.y += on[k] ? v.y * w[k] : 0.0f;
-                a.z += on[k] ? v.z * w[k] : 0.0f;
-                a.w += on[k] ? v.w * w[k] : 0.0f;
-              }
-              o_acc[j0 + j][4 * r] = a.x;
-              o_acc[j0 + j][4 * r + 1] = a.y;
-              o_acc[j0 + j][4 * r + 2] = a.z;
-              o_acc[j0 + j][4 * r + 3] = a.w;
+        for (int j = 0; j < JB; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float4 mine =
+                make_float4(o_acc[j0 + j][4 * r], o_acc[j0 + j][4 * r + 1],
+                            o_acc[j0 + j][4 * r + 2], o_acc[j0 + j][4 * r + 3]);
+            float4 a = k0 > 0 ? sum[j][r] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+            for (int k = k0; k < k0 + KB; k++) {
+              const float4 v = k == part ? mine : y[k - k0][j][r];
+              a.x += on[k] ? v.x * w[k] : 0.0f;
+              a.y += on[k] ? v.y * w[k] : 0.0f;
+              a.z += on[k] ? v.z * w[k] : 0.0f;
+              a.w += on[k] ? v.w * w[k] : 0.0f;
             }
-        }
-        // the next round's store of (m, l) goes to the first of these parts, which
-        // the waves of the other group may not have read yet
-        if (KG > 1 && n > 4) {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __syncthreads();
-        }
+            sum[j][r] = a;
+          }
       }
-      count += meet.units;
+#pragma unroll
+      for (int j = 0; j < JB; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          o_acc[j0 + j][4 * r] = sum[j][r].x;
+          o_acc[j0 + j][4 * r + 1] = sum[j][r].y;
+          o_acc[j0 + j][4 * r + 2] = sum[j][r].z;
+          o_acc[j0 + j][4 * r + 3] = sum[j][r].w;
+        }
     }
   }
   if (!row_ok) return;
@@ -720,22 +737,12 @@ template <int ROWS>
 inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
   return (tokens * G + n_seqs * (ROWS - 1L)) / ROWS;
 }
-// Groups of waves, and parts of the keys. Parts (pf_parts): about two groups of waves
-// per CU are wanted, and parts of at least eight tiles of keys (four with 32-bit
-// weights, whose tiles take twice as long): the merge costs more than smaller ones save.
-// At least six: 3 chunks of 93-261 tokens 36.5 us (eight: 31.8); up to 16 parts, not 8:
-// 29.7 (34.9) for 50-300 tokens behind up to 9000. Measured (us, by parts 1 | 2 | 4 |
-// 8), 32-bit weights: 2 x 64 rows of 32 heads over 4000 keys 191 | 104 | 60 | 40; 300 of
-// 16 over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles) 374 | 298 | 302 |
-// 325; 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
-//   Parts of two groups of waves, which leave half the partial results in memory (24 MB
-// of the 3 chunks'), where their larger units still fill the CUs, one turn of them and
-// no more: one sequence in 200-256 of at least three parts, several in up to 144 before
-// they are split; us, one | two groups: the 3 chunks 31.4 | 29.6, 2 x 200 behind 3000
-// 43.7 | 41.1, 300 behind 2000 of 32/8 37.2 | 31.5, 300 behind 12000 of 16/4 64.8 |
-// 48.7, of 28/4 (204 units) 91 | 78, capped 1900 and 32/8 47.1 | 44; but 272 units of
-// the last but one 110, two parts (256 units) of 1000 behind 500 of 16/4 capped 38.6 |
-// 42.8, 31, 322 and 416 tokens of 32 heads (288) 30.5 | 35.7.
+// Groups of waves, and parts of the keys (pf_parts): about two groups of waves per CU are
+// wanted, and parts of at least eight tiles of keys (four with 32-bit weights, whose
+// tiles take twice as long): the merge costs more than smaller ones save. Measured (us,
+// by parts 1 | 2 | 4 | 8), 32-bit weights: 2 x 64 rows of 32 heads over 4000 keys 191 |
+// 104 | 60 | 40; 300 of 16 over 600 37 | 26 | 24 | 28; 1024 of 32 over 8000 (264 row tiles)
+// 374 | 298 | 302 | 325; 4096 of 16 in a window (520 row tiles) 69 | 87 | 111 | 182.
 //   Two groups of waves and one part where these fill one turn of the CUs: 128-wide
 // heads, up to 24 tiles, or for a single sequence that fills most of the CUs; us, as
 // before (parts) | two groups: 1024 tokens of 32/8 heads 34.5 (2) | 25.5, 28/4 32.5 (2)
@@ -748,12 +755,6 @@ inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
 // of 512 41 (2) | 29.5, capped 51.8 | 40, but 300 behind 1000 (75) 37 (4) | 42, 2000 of
 // 16/4 capped 71 (2) | 73.7. 64-wide, two workgroups to a CU: 8 prompts of 64-448 13.3
 // (1) | 12.4, 1700 (168) 27.8 (3) | 32.7.
-//   The last part merges (meet), or a kernel of its own; us, kernel | last: the 3 chunks
-// 31 | 27, 90 and 200 behind 2300 and 900 of 32/8 29 | 23.4, 1700 of 64-wide heads 28.8
-// | 23.3, 300 behind 2000 of 32/8 31.3 | 26.4, 700 in a window 32.2 | 26.4; four parts
-// of few tiles, whose merge is short, 60 behind 2000 (64 units) 20.6 | 22.4, of 32 heads
-// (128) 21.3 | 23.5; up to eight 60 behind 4000 23.4 | 28.2, 31, 322 and 416 behind
-// 4052, 20 and 27 30.5 | 35.6, sixteen 50-300 behind up to 9000 28.6 | 30.4.
 // groups: KG; least: tiles of a part, 0 without parts; most: parts of a tile; units: tiles
 // and parts a grid holds; scratch: floats
 struct PagedRows {
@@ -761,37 +762,96 @@ struct PagedRows {
   bool meet = false;
   long units = 0, scratch = 0;
 };
+// Parts of a single sequence: of two groups of waves, which leave half the partial
+// results in memory, where at least three of them make 200 to 256 units; us, one | two
+// groups: 300 behind 2000 of 32/8 37.2 | 31.5, 300 behind 12000 of 16/4 64.8 | 48.7, of
+// 28/4 (204 units) 91 | 78, capped 1900 and 32/8 47.1 | 44; two parts (256 units) of 1000
+// behind 500 of 16/4 capped 38.6 | 42.8. The last part merges (meet) or a kernel of its
+// own; us, kernel | last: 1700 of 64-wide heads 28.8 | 23.3, 300 behind 2000 of 32/8 31.3 |
+// 26.4, 700 in a window 32.2 | 26.4; four parts of few tiles, whose merge is short, 60
+// behind 2000 (64 units) 20.6 | 22.4, of 32 heads (128) 21.3 | 23.5; up to eight 60 behind
+// 4000 23.4 | 28.2.
+inline void paged_rows_one(PagedRows& x, long wgs, long tiles, int D, int terms) {
+  const int least = terms == 1 ? 8 : 4;
+  if (x.groups > 1 || wgs > 340 || tiles < 2 * least) return;
+  const long twos = std::min<long>({256 / wgs, tiles / (terms == 1 ? 8 : 5), 16});
+  if (D == 128 && twos > 2 && wgs * twos >= 200) x.groups = 2;
+  x.most = x.groups == 2
+               ? (int)twos
+               : (int)std::min<long>({(512 + wgs / 2) / wgs, tiles / least, 16});
+  x.least = x.groups == 2 ? 12 : least;
+  x.meet = x.most <= 2 || (x.most <= 4 && wgs * x.most >= 160);
+}
+// Parts of several sequences, whose lengths only the kernel knows. Where their row tiles
+// are many, parts are few: the last one merges. Where they are few a long sequence has
+// many, which a kernel of its own merges sooner, and which are shorter. thin: so few rows
+// that what the last part reads would be mostly padding.
+//   712 drawn batches of 2 to 70 sequences, time over that of as many parts for all and a
+// kernel for the merge, by workgroups before keys are split; one group of waves and a
+// kernel | two and a kernel | one and the last | two and the last part. bf16 weights: up
+// to 19 0.90 | 0.96 | 1.17 | 1.12, 39 0.85 | 0.87 | 0.98 | 0.93, 63 0.92 | 0.88 | 0.99 |
+// 0.91, 95 0.93 | 0.88 | 0.90 | 0.82, 144 0.88 | 0.88 | 0.87 | 0.82, 199 0.92 | 0.99 | 0.85 |
+// 0.88, 259 0.90 | 0.94 | 0.83 | 0.87, 340 0.97 | 1.01 | 0.89 | 0.95; thin ones from 64 on
+// 0.90 | 0.99 | 0.95 | 0.97. 128-wide, 32-bit weights: 39 0.94 | 0.92 | 1.20 | 1.09, 63
+// 0.96 | 0.96 | 0.94 | 0.93, 144 0.97 | 0.92 | 0.91 | 0.84, 256 0.96 | 0.99 | 0.87 | 0.92, 340
+// 0.95 | 0.91 | 0.87 | 0.85. 64-wide from 64 on 0.97 | - | 0.82 | 0.85.
+//   By two groups in 13 to 24 tiles too, below 145 workgroups (one part of two groups | by
+// parts): 16 x 17-27 behind up to 1500 of 28/4 31.0 | 20.8, 3 x 19-127 of 32/32 27.1 | 20.2, 2
+// x 168-385 behind 400-1100 of 16/4 29.3 | 21.5.
+inline void paged_rows_several(PagedRows& x, long wgs, long tiles, int D, int terms,
+                               bool thin) {
+  if (wgs > 340) return;
+  if (terms == 1) {
+    if (x.groups > 1 ? wgs >= 145 || tiles < 13 : tiles < 16) return;
+    x.meet = !thin && wgs >= 64 && (wgs >= 145 || tiles <= 128);
+    if (x.meet) {
+      x.groups = wgs < 145 ? 2 : 1;
+      x.least = x.groups == 1 || tiles < 17 ? 12 : 8;
+    } else {
+      x.groups = thin || wgs < 20 || (wgs < 40 && tiles > 64) ? 1 : 2;
+      x.least = wgs < 20 ? 4 : 6;
+    }
+  } else if (D == 128) {
+    if (x.groups > 1 || tiles < 8) return;
+    x.meet = !thin && wgs >= 40 && (wgs >= 64 || tiles <= 16) &&
+             (wgs >= 96 || tiles <= 64);
+    if (x.meet) {
+      x.groups = wgs >= 64 && wgs < 145 ? 2 : 1;
+      x.least = wgs < 64 ? 4 : wgs < 257 ? 6 : 8;
+    } else {
+      x.groups = tiles > 16 && !thin ? 2 : 1;
+      x.least = 4;
+    }
+  } else {
+    if (x.groups > 1 || tiles < 8) return;
+    x.meet = !thin && wgs >= 64;
+    x.least = x.meet ? 6 : 4;
+  }
+  x.most = x.meet ? PF_MEET(x.groups) : 16;
+}
 inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D,
                                  long max_blocks, int terms) {
   PagedRows x;
-  const long wgs = paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G) * n_kv;
+  const long row_tiles = paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G);
+  const long wgs = row_tiles * n_kv;
   const long keys = max_blocks * PF_BS, tiles = keys / PF_KT;
   const bool alone = n_seqs == 1 && 2 * keys < 3 * tokens;
+  if (wgs == 0) return x;
   if (D == 64)
-    x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 ? 2 : 1;
+    x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 &&
+               (n_seqs == 1 || tiles <= 24 || wgs > 340) ? 2 : 1;
   else if (terms > 1)
     x.groups = keys >= 512 && tiles <= 20 && wgs >= 200 && wgs <= 256 ? 2 : 1;
   else if (keys >= 640 && wgs >= 72)
     x.groups = wgs <= 256 ? (tiles <= 24 || (n_seqs == 1 && wgs >= 200) ? 2 : 1)
                           : (wgs <= 448 && alone && tiles >= 18 ? 2 : 1);
-  const int least = terms == 1 ? 8 : 4;
-  if (x.groups == 1 && wgs > 0 && wgs <= 340 && tiles >= 2 * least) {
-    const long row_tiles = paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G);
-    const long twos = std::min<long>({256 / wgs, tiles / (terms == 1 ? 8 : 5), 16});
-    if (D == 128 && (n_seqs > 1 ? terms == 1 && wgs <= 144
-                                : twos > 2 && wgs * twos >= 200))
-      x.groups = 2;
-    x.most = n_seqs > 1 ? 16
-             : x.groups == 2 ? (int)twos
-                 : (int)std::min<long>({(512 + wgs / 2) / wgs, tiles / least, 16});
-    x.least = x.groups == 2 ? 12 : D == 64 ? 4 : least;
-    x.units = n_seqs > 1 ? row_tiles + PF_UNITS / x.groups / n_kv + 1
-                         : row_tiles * x.most;
-    x.meet = n_seqs > 1 ? tiles <= (x.groups == 2 ? 64 : 4 * x.least)
-                        : x.most <= 2 || (x.most <= 4 && wgs * x.most >= 160);
-    x.scratch = x.units * n_kv * (PF_ROWS * (D + 2) + (x.meet ? 4 : 0)) +
-                (x.meet ? 0 : tokens * G * n_kv * 2);
-  }
+  if (n_seqs == 1) paged_rows_one(x, wgs, tiles, D, terms);
+  else paged_rows_several(x, wgs, tiles, D, terms, tokens * G <= 64L * n_seqs);
+  if (x.least == 0) return x;
+  x.units = n_seqs > 1 ? row_tiles + PF_UNITS / x.groups / n_kv + 1
+                       : row_tiles * x.most;
+  x.scratch = x.units * n_kv * (PF_ROWS * (D + 2) + (x.meet ? 2 : 0)) +
+              (x.meet ? 0 : tokens * G * n_kv * 2);
   return x;
 }
 
@@ -816,10 +876,7 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
   const long wgs = paged_rows_wgs(plan, tokens, n_seqs, G, n_kv);
   PagedMeet meet;
   float* ws_ml = ws_o + wgs * PF_ROWS * D;
-  if (plan.least > 0) {
-    if (plan.meet) meet = paged_meet(ws_ml, wgs * PF_ROWS, 1);
-    meet.units = wgs;
-  }
+  if (plan.meet) meet = paged_meet(ws_ml, wgs * PF_ROWS, 1);
   int2* ws_at = reinterpret_cast<int2*>(ws_ml + wgs * PF_ROWS * 2);
 #define PF_GO(KG, SPLIT)                                                       \
   hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG, SPLIT>),      \

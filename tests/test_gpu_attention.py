@@ -647,6 +647,17 @@ def test_prefill_orders_and_groups(kv_heads, per, dim, lens, ctx, sign):
 
 
 @pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [
+    (8, 4, 128, [200, 90, 333, 1, 150, 0, 257] * 3, [7, 60, 5] * 7, 1.0),   # over three
+    (8, 4, 128, [200, 90, 333, 1, 150, 0, 257] * 2, [7, 60, 5, 9] * 3 + [3, 0], -1.0),
+    (8, 4, 128, [260, 301, 330, 280, 270, 289], [0, 100, 3, 0, 0, 20], -1.0),   # under two
+    (8, 4, 128, [64, 1, 0, 65, 33], [0, 9, 5, 0, 3], 1.0),                  # less than one
+])
+def test_prefill_order_of_turns(kv_heads, per, dim, lens, ctx, sign):
+    """Row tiles of one turn of the CUs as they are, of more than two folded."""
+    test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign)
+
+
+@pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [
     (2, 4, 128, [50, 60, 0, 130, 20], [2500, 100, 30, 0, 700], 1.0),
     (4, 4, 128, [3] * 68 + [64, 1], [0, 90] * 34 + [1300, 1100], -1.0),
     (3, 5, 128, [9, 77], [1015, 1016], 1.0),         # parts of eight tiles, and nine

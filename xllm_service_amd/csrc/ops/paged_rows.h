@@ -211,25 +211,22 @@ XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
 // 27 of 32/32 56 -> 30.5, 2 x 200 behind 3000 52.3 -> 41.1; equal ones (8 x 100 behind 500,
 // 20.1) gain nothing.
 template <int ROWS, bool MORE>
-XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& x,
+XLLM_DEV bool pf_parts(int b, int least, int most, int groups, int turn,
+                       const PagedMore& x,
                        const int* cu_q, const int* seq_lens, int n_seqs, int G,
                        int n_kv, int lane, PfPlace* at, int* part, int* parts,
                        int* first) {
-  auto tiles_of = [&](int keys) {
-    const int n = (max(keys, 0) + PF_KT - 1) / PF_KT;
-    return MORE && x.window > 0
-               ? min(n, (x.window + x.keep_first) / PF_KT + 3) : n;
-  };
   if (n_seqs == 1) {
     const int q0 = cu_q[0], len = cu_q[1] - q0, keys = seq_lens[0];
-    const int p = max(min((tiles_of(keys) + 3) / 4, most), 1);
-    const int all = (len * G + ROWS - 1) / ROWS * p;
+    const int p = paged_equal<MORE>(x, keys, PF_KT, most);
+    const int nt = (len * G + ROWS - 1) / ROWS, all = nt * p;
     if (b >= all) return false;
-    b = pf_fold(b, all, 256 / n_kv);
-    *part = b % p;
+    b = pf_fold(b, all, turn);
+    const int t = b / p;                         // a division takes 0.05 us
+    *part = b - t * p;
     *parts = p;
-    *first = b - b % p;
-    *at = {0, (all - 1 - b) / p, q0, len, keys};
+    *first = t * p;
+    *at = {0, nt - 1 - t, q0, len, keys};
     return true;
   }
   int start = 0, len = 0, keys = 0, nt = 0, n = 0;
@@ -241,7 +238,7 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& 
       keys = seq_lens[i];
     }
     nt = (len * G + ROWS - 1) / ROWS;
-    n = tiles_of(keys);
+    n = paged_walk<MORE>(x, keys, PF_KT);
   };
   int work = 0;
   for (int base = 0; base < n_seqs; base += 64) {
@@ -294,10 +291,11 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, const PagedMore& 
       const int l = __builtin_amdgcn_readfirstlane(__ffsll(hit) - 1);
       const int pl = __builtin_amdgcn_readlane(p, l);
       const int r = b - __builtin_amdgcn_readlane(upto - nt * p, l);
-      *part = r % pl;
+      const int t = r / pl;
+      *part = r - t * pl;
       *parts = pl;
-      *first = b - r % pl;
-      *at = {base + l, __builtin_amdgcn_readlane(nt, l) - 1 - r / pl,
+      *first = b - *part;
+      *at = {base + l, __builtin_amdgcn_readlane(nt, l) - 1 - t,
              __builtin_amdgcn_readlane(start, l),
              __builtin_amdgcn_readlane(len, l),
              __builtin_amdgcn_readlane(keys, l)};
@@ -318,7 +316,8 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     void* __restrict__ out,                  // [total_q, n_qheads, D]
     float* __restrict__ ws_o,                // [blocks][PF_ROWS * D], a block for a part
     float* __restrict__ ws_ml,               // [blocks][PF_ROWS][2]
-    int2* __restrict__ ws_at,                // [total_q*n_qheads]: first slot, parts
+    int2* __restrict__ ws_at,                // [total_q*n_qheads]: first slot, parts;
+                                             // of several prompts, for the merge
     const PagedMeet meet,                    // [blocks]: its first part's counts
     const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
     const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
@@ -353,7 +352,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   int part = 0, parts = 1, first = 0;
   PfPlace at;
   if constexpr (SPLIT) {
-    if (!pf_parts<PF_ROWS, MORE>(blockIdx.x / n_kv, least, most, KG, x, cu_q,
+    if (!pf_parts<PF_ROWS, MORE>(blockIdx.x / n_kv, least, most, KG, turn, x, cu_q,
                                  seq_lens, n_seqs, G, n_kv, lane, &at, &part,
                                  &parts, &first))
       return;
@@ -708,7 +707,7 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
   const long grow = (long)(q_start + qi) * n_qheads + head;
   // for the merge, the parts of a row lie together (strided, it took up to 9 us more)
   const long slot = block * PF_ROWS + row * parts + part;
-  if (SPLIT && meet.count == nullptr && part == 0 && h == 0 && kg == 0)
+  if (SPLIT && ws_at != nullptr && part == 0 && h == 0 && kg == 0)
     ws_at[grow] = make_int2((int)slot, parts);
   if (!SPLIT || meets || parts == 1) {
     if (MORE && x.sink != nullptr) l += paged_sink(x, head, m);
@@ -843,21 +842,21 @@ inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D
   const long keys = max_blocks * PF_BS, tiles = keys / PF_KT;
   const bool alone = n_seqs == 1 && 2 * keys < 3 * tokens;
   if (wgs == 0) return x;
-  if (D == 64)
-    x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 &&
-               (n_seqs == 1 || tiles <= 24 || wgs > 340) ? 2 : 1;
-  else if (terms > 1)
+  if (D == 64) {
+    x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 ? 2 : 1;
+  } else if (terms > 1) {
     x.groups = keys >= 512 && tiles <= 20 && wgs >= 200 && wgs <= 256 ? 2 : 1;
-  else if (keys >= 640 && wgs >= 72)
+  } else if (keys >= 640 && wgs >= 72) {
     x.groups = wgs <= 256 ? (tiles <= 24 || (n_seqs == 1 && wgs >= 200) ? 2 : 1)
                           : (wgs <= 448 && alone && tiles >= 18 ? 2 : 1);
+  }
   if (n_seqs == 1) paged_rows_one(x, wgs, tiles, D, terms);
   else paged_rows_several(x, wgs, tiles, D, terms, tokens * G <= 64L * n_seqs);
   if (x.least == 0) return x;
   x.units = n_seqs > 1 ? row_tiles + PF_UNITS / x.groups / n_kv + 1
                        : row_tiles * x.most;
   x.scratch = x.units * n_kv * (PF_ROWS * (D + 2) + (x.meet ? 2 : 0)) +
-              (x.meet ? 0 : tokens * G * n_kv * 2);
+              (x.meet || n_seqs == 1 ? 0 : tokens * G * n_kv * 2);
   return x;
 }
 
@@ -883,7 +882,8 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
   PagedMeet meet;
   float* ws_ml = ws_o + wgs * PF_ROWS * D;
   if (plan.meet) meet = paged_meet(ws_ml, wgs * PF_ROWS, 1);
-  int2* ws_at = reinterpret_cast<int2*>(ws_ml + wgs * PF_ROWS * 2);
+  int2* ws_at = plan.least > 0 && !plan.meet && n_seqs > 1
+                    ? reinterpret_cast<int2*>(ws_ml + wgs * PF_ROWS * 2) : nullptr;
   // Batches that the CUs hold one to each come as they are, without a search: 8 x 38-140 of
   // 28/4 9.62 -> 9.46 us, 60 drawn ones 1.00 -> 0.985 of the time before the search.
   const int turn = n_seqs > 1 && wgs <= 256 ? 0 : 256 / n_kv;
@@ -900,8 +900,9 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
   else PF_GO(1, false);
 #undef PF_GO
   if (plan.least > 0 && !plan.meet)
-    paged_merge<D, MORE>(out, ws_o, ws_ml, ws_at, n_qheads, out_stride,
-                         tokens * n_qheads, x, stream, cu_q, n_seqs);
+    paged_merge<D, MORE, PF_ROWS, PF_KT>(out, ws_o, ws_ml, ws_at, n_qheads, out_stride,
+                                         tokens * n_qheads, x, stream, cu_q, seq_lens,
+                                         n_seqs, n_kv, plan.most);
 }
 
 }  // namespace xllm

@@ -651,6 +651,8 @@ def test_prefill_orders_and_groups(kv_heads, per, dim, lens, ctx, sign):
     (8, 4, 128, [200, 90, 333, 1, 150, 0, 257] * 2, [7, 60, 5, 9] * 3 + [3, 0], -1.0),
     (8, 4, 128, [260, 301, 330, 280, 270, 289], [0, 100, 3, 0, 0, 20], -1.0),   # under two
     (8, 4, 128, [64, 1, 0, 65, 33], [0, 9, 5, 0, 3], 1.0),                  # less than one
+    (12, 1, 64, [406, 300, 430] * 2 + [33, 64] * 4, [0, 18] * 7, 1.0),      # of 64-wide heads
+    (12, 1, 64, [58, 115, 97, 31, 64, 0, 60] * 2, [3, 1] * 7, -1.0),
 ])
 def test_prefill_order_of_turns(kv_heads, per, dim, lens, ctx, sign):
     """Row tiles of one turn of the CUs as they are, of more than two folded."""

@@ -759,7 +759,10 @@ inline long paged_rows_tiles(long tokens, int n_seqs, int G) {
 // | 31.4. 32-bit weights, 2 x 400 behind 500 of 32/8 in a window 46.3 (2) | 33, in one
 // of 512 41 (2) | 29.5, capped 51.8 | 40, but 300 behind 1000 (75) 37 (4) | 42, 2000 of
 // 16/4 capped 71 (2) | 73.7. 64-wide, two workgroups to a CU: 8 prompts of 64-448 13.3
-// (1) | 12.4, 1700 (168) 27.8 (3) | 32.7.
+// (1) | 12.4, 1700 (168) 27.8 (3) | 32.7; but two turns of short chains start and end
+// together: several in 300 workgroups and more, up to 7 tiles 0.94 to 0.98 of the time before | 1.02 to
+// 1.21, from 350 on up to 11 tiles 0.92 to 0.98 | 1.04, 12 and more 0.82 to 0.94 | 0.80 to 0.88,
+// capped 0.91 | 0.76.
 // groups: KG; least: tiles of a part, 0 without parts; most: parts of a tile; units: tiles
 // and parts a grid holds; scratch: floats
 struct PagedRows {
@@ -835,7 +838,7 @@ inline void paged_rows_several(PagedRows& x, long wgs, long tiles, int D, int te
   x.most = x.meet ? PF_MEET(x.groups) : 16;
 }
 inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D,
-                                 long max_blocks, int terms) {
+                                 long max_blocks, int terms, bool options) {
   PagedRows x;
   const long row_tiles = paged_rows_tiles<PF_ROWS>(tokens, n_seqs, G);
   const long wgs = row_tiles * n_kv;
@@ -843,7 +846,9 @@ inline PagedRows paged_rows_plan(long tokens, int n_seqs, int G, int n_kv, int D
   const bool alone = n_seqs == 1 && 2 * keys < 3 * tokens;
   if (wgs == 0) return x;
   if (D == 64) {
-    x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 ? 2 : 1;
+    const bool brief = !options && n_seqs > 1 && wgs >= 300 &&
+                       tiles <= (wgs < 350 ? 7 : 11);
+    x.groups = keys >= 384 && wgs >= 200 && wgs <= 448 && !brief ? 2 : 1;
   } else if (terms > 1) {
     x.groups = keys >= 512 && tiles <= 20 && wgs >= 200 && wgs <= 256 ? 2 : 1;
   } else if (keys >= 640 && wgs >= 72) {

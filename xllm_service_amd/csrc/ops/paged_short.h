@@ -284,7 +284,9 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
 // long. More workgroups take a second turn for what fewer waves do over the same keys
 // (us, paged_rows.h | here): 300 tokens of 32/8 heads (304 workgroups) 12.3 | 13.3, in a
 // window 17.5 | 19.2, 8 prompts of 64-448 of 12/12 of 64 (764) 12.4 | 17.4, 594 behind up to
-// 3000 keys (616) 50 | 68; but 2 x 600 behind 200 (456) 22.3 | 16.5. In one or two tiles of keys
+// 3000 keys (616) 50 | 68; but 2 x 600 behind 200 (456) 22.3 | 16.5; over up to 192
+// keys 12 x 58-115 (504) 0.96 | 1.10 of the time of the kernel before, 20 x 17-49 behind 43-84
+// (480) 0.97 | 1.17, but 8 x 27-231 0.99 | 0.85. In one or two tiles of keys
 // there is nothing to share: 20 tokens 6.3 | 7.0, 64 of 64-wide heads 5.4 | 6.1. Longer
 // tables go to more workgroups there: 32 tokens of 28/4 heads behind 1000 keys 18.5 | 15.9,
 // 100 of 32/8 behind 1600 22.0 | 20.5, but 32 behind 3000 21.9 | 29.4; 16 of 64-wide heads
@@ -297,7 +299,7 @@ inline bool paged_short_takes(long tokens, int n_seqs, int G, int n_kv, int D,
                               long max_blocks, bool options) {
   const long keys = max_blocks * PF_BS;
   return paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv <=
-             (D == 64 ? 512 : 256) &&
+             (D == 64 ? keys >= 192 || options ? 512 : 400 : 256) &&
          keys >= 128 &&
          keys <= (options ? 768 : D == 64 ? PS_KEYS / 2 : PS_KEYS) &&
          (keys < 1536 || tokens * G >= (long)PF_ROWS * n_seqs);
@@ -333,7 +335,7 @@ inline PagedPrompts paged_prompts(long tokens, int n_seqs, int G, int n_kv, int 
   p.few = paged_short_takes(tokens, n_seqs, G, n_kv, D, max_blocks, options);
   if (!p.few)
     static_cast<PagedRows&>(p) =
-        paged_rows_plan(tokens, n_seqs, G, n_kv, D, max_blocks, terms);
+        paged_rows_plan(tokens, n_seqs, G, n_kv, D, max_blocks, terms, options);
   return p;
 }
 

@@ -483,6 +483,9 @@ def over_litter(call, out, sl, lengths, ref):
     (128, [32 * 32 + 1, 65 * 32, 8 * 65 * 32 + 5], 1, 7),   # eight of them, more
     (64, [16 * 32, 16 * 32 + 1, 21 * 32, 31, 2000], 16, 1),
     (128, [23 * 32, 23 * 32 + 1, 3000, 40] * 3, 8, 3),      # 96 pairs
+    (128, [24 * 32, 24 * 32 + 1, 3000, 40] * 3, 8, 1),
+    (128, [40 * 32, 40 * 32 + 1, 4000, 9, 700] * 3, 8, 2),  # 120
+    (128, [32 * 32 + 1, 4200, 900, 40] * 3, 8, 4),          # in a longer table
     (64, [19 * 32, 19 * 32 + 1, 2000, 700] * 2, 12, 1),
     (64, [39 * 32, 39 * 32 + 1, 2000, 9] * 4, 12, 2)])      # 192
 def test_decode_parts_meet(dim, keys, kv_heads, per):

@@ -190,14 +190,12 @@ struct PagedSplit {
   int parts = 1, per = 1;
   int near = 1 << 20;        // tiles
   int least = 0;             // tiles of the shortest list that is split
-  bool twos = false;         // 2, 4 or 8 of them
   int waves = 4;             // of a workgroup
   __host__ __device__ int of(int n) const {
     const int far = paged_parts(n, parts, per);
     const int most = paged_parts(n, parts < 8 ? parts : 8, near);
     if (n < least) return 1;
-    return twos ? far < 2 ? 1 : far < 5 ? 2 : far < 8 ? 4 : 8
-                : far > most ? far : most;
+    return far > most ? far : most;
   }
 };
 

@@ -429,10 +429,13 @@ paged_attn_stream_kernel(
 //   With options (a window, a cap, a sink) weights have 32 bits and a tile is longer: four
 // tiles a part however many, from nine on (4 key heads, 1 x 300 keys, capped 10.5 whole,
 // 8.3 in three, 1 x 1000 19.7, 8.5 in eight; a window of 512 12.0, 8.2 in five).
-//   Up to 128 pairs, whole | by 16 tiles, 2, 4 or 8 parts: 11 x 1000 16.8 | 14.3, 16 x 1000
-// 17.7 | 17.6, 11 x 0.5-4 k 31.0 | 21.6, 16 x 0.2-2 k 25.3 | 20.5. Not 3: 264 workgroups for 256
-// CUs, 11 x 1500 20.4 | 23.2 and 19.0 in two; 11 x 2000 21.6 in two, 23.8 in four. Long
-// tables, up to 32 tiles a part: 22 x 1-20 k, 4 key heads, 84.0 | 86.9 by 16, 83.5 by 32.
+//   Up to 128 pairs in tables of up to 4096 keys, two parts, whose 256 workgroups fill one
+// turn, of sequences over 24 tiles (40 from 118 pairs on, which lose by it when they are
+// equal); us, whole | two: 13 x 1.9-2.6 k 31.8 | 26.8, 11 x 0.5-4 k 31.0 | 21.6, 4 key heads, 29 x
+// 0.9-2.5 k 29.7 | 24.8, 24 x 0.4-1.25 k 14.9 | 13.0, 31 x 1.1-1.4 k 16.1 | 18.2. Three or four fill
+// it and a bit: 11 x 2000 23.8, 21.6 in two. Longer tables by 32 tiles, as those of more pairs,
+// so that none of a batch outlasts the rest: by 16 | at most two | by 32, 11 x 0.9-8 k 51.6 |
+// 52.3 | 44.5, 4 key heads, 26 x 0.3-4.9 k in tables of 8192 42.0 | 37.9 | 35.3.
 //   More pairs fill the chip, and equal ones lose by a split what the merge costs (24 x
 // 0.6-1.4 k 22.8 | 26.4; 32 x 1-2 k 38.2 | 41.3), but a long sequence among short ones is a
 // chain of tiles that outlasts the rest. By parts of 32 tiles, at most 8: 8 key heads, 16 x
@@ -465,11 +468,9 @@ inline PagedSplit paged_stream_split(long num_seqs, int n_kv_heads,
     x.parts = x.of((int)std::min<long>(table, 1 << 20));
     return x;
   }
-  if (units <= 128 && !options) {
-    x.per = (int)std::min<long>(32, std::max<long>(16, table / 8));
-    x.least = 24;
-    x.twos = true;
-    x.parts = (int)std::min<long>(8, (table + x.per - 1) / x.per);
+  if (units <= 128 && !options && table <= 128) {
+    x.per = units < 118 ? 24 : 40;
+    x.parts = table > x.per ? 2 : 1;
     return x;
   }
   const long f = capped ? 2 : 1, tiles = f * table;

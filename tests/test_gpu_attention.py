@@ -635,6 +635,21 @@ def test_options(dim, bf16_out, lens, ctx, kv_heads, per, decode, opts):
         assert (wide[:, heads * dim:] == 7.0).all()
 
 
+@pytest.mark.parametrize("opts", ["window", "cap", "sink", "chunks", "window + kept"])
+@pytest.mark.parametrize("dim,lens,ctx,kv_heads,per,decode", [
+    (128, [1] * 6, [0, 14, 15, 16, 31, 47], 4, 4, True),
+    (128, [1] * 4, [15, 63, 64, 100], 1, 32, True),
+    (64, [1] * 5, [0, 15, 16, 31, 63], 2, 16, True),
+    (128, [16, 1, 40], [0, 30, 7], 2, 8, False),
+    (128, [48, 49, 33] * 5, [0, 0, 15] * 5, 8, 1, False),
+    (64, [16, 1, 40], [0, 30, 7], 3, 2, False),
+])
+def test_options_over_few_keys(dim, lens, ctx, kv_heads, per, decode, opts):
+    """Where one tile or two hold all keys, on both sides of what the kernels of 16
+    rows a wave are left."""
+    test_options(dim, False, lens, ctx, kv_heads, per, decode, opts)
+
+
 @pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [
     (8, 4, 128, [650], [0], 1.0),                    # waves in two groups
     (8, 4, 128, [60, 700, 1], [900, 0, 130], -1.0),  # tiles for one group only

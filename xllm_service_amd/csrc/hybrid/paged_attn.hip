@@ -38,49 +38,37 @@ long paged_attn_scratch(bool decode, long tokens, int n_seqs, int heads, int n_k
   return parts > 1 ? tokens * heads * parts * (D + 2) + 2L * n_seqs * n_kv : 0;
 }
 
-// Whether the kernels of capped_attn_mfma.hip are faster: they have 16 rows a wave
-// and 32 keys a tile, so that one tile is done in half the time, but move four times
-// as much through LDS, do not split the keys of prompts and look for a row tile's
-// sequence one by one.
-//   Decode, by the keys a row sees, us there | here: 16 or 32 5.6 | 6.3 (4 query heads
-// a key head), 5.7 | 7.5 (16), 6.0 | 9.0 (32); 64 7.4 | 5.8, 7.2 | 6.8, 7.8 | 8.6; 300
-// 11.4 | 8.5. The merge of the waves' results grows with the heads: above 16 a key
-// head, for 2 pairs, 300 keys in tables of 4096 9.7 | 11.1, windows of 512 11.1 |
-// 12.9 (16 heads 10.6 | 11.3), for 16 pairs 21.6 | 13.6.
-//   Prompts, by the keys from the first to the last one of a row tile and by the
-// number of row tiles: window 16, 64-wide heads, 256 tokens 7.2 | 9.9, 64 sequences of
-// 128 56 | 39; window 512, 256 tokens 36 | 19; 128-wide, window 16 9.2 | 12.7, 64 of one
-// head 16.8 | 17.8, 128 26 | 19, window 16 over 260 x 4 row tiles 24.6 | 22.1. In between
-// a fit to 1370 timed calls of each kind decides, of which 70 to 130 take over 5 %
-// longer than by the other kernels, one a third.
+// Whether the kernels of capped_attn_mfma.hip are faster: they have 16 rows a wave and 32
+// keys a tile, so that one tile is done in half the time, but move four times as much
+// through LDS, do not split the keys of prompts and look for a row tile's sequence one by
+// one. They are where one tile holds all keys. Time there over that here, 1270 drawn calls:
+//   Prompts, by the keys from the first to the last one of a row tile and by the workgroups
+// here: up to 32 keys 0.91 (up to 99 workgroups), 1.07 (255), capped 0.85, 0.96; 33 to 48 1.06,
+// 1.17, capped 0.97, 1.08; then 1.16 to 2.4. (A fit to calls of both before few rows' keys were shared by waves sent 179 of 600
+// there, of which 77 took over 5% longer.)
+//   Decode, 128 wide, by the keys a row sees: tables of up to 32 keys 0.97, 0.87 (9 to 16
+// heads a key head), 0.72 (more); windows as small in longer ones lie in two tiles, 1.31, 1.17,
+// 0.96; 33 to 64 keys 1.27, 1.19, 0.97; 65 to 128 1.89, 1.78, 1.50; more 1.6, 1.3, and 0.90 for
+// up to eight pairs of sequence and key head (their merge of waves' results is longest
+// here), 1.36 for many. 64 wide 1.1 to 2.2.
 bool paged_attn_small(bool decode, long tokens, int n_seqs, int heads, int n_kv,
                       int D, long max_blocks, int window, int keep_first,
                       bool capped) {
   const long keys = max_blocks * 16, G = heads / n_kv;
+  if (keys == 0) return true;          // tables without columns: not read there
   if (decode) {
     const long walk = window > 0 ? std::min<long>(keys, window) : keys;
     const long pairs = (long)n_seqs * n_kv;
-    return walk <= 32 || (G > 16 && (walk <= 64 || (pairs <= 8 && walk <= 4096))) ||
-           (G > 8 && pairs <= 16 && window > 256 && walk <= 1024);
+    return D == 128 &&
+           (keys <= 32 || (G > 16 && (walk <= 64 || (pairs <= 8 && walk > 128 &&
+                                                     walk <= 4096))));
   }
-  // us: a + b * tiles of a walk, more where row tiles wait for others
-  struct Fit { double a, b, wgs; };
-  static const Fit there[2][2] = {{{4.8, 1.56, 350}, {5.1, 1.85, 340}},
-                                  {{5.7, 2.45, 300}, {5.9, 2.73, 300}}};
-  static const Fit here[2][2] = {{{7.1, 1.50, 190}, {8.1, 2.41, 240}},
-                                 {{8.6, 2.10, 150}, {9.6, 3.01, 180}}};
-  auto walk = [&](long rows) {
-    const long span = std::max<long>(1, std::min<long>(tokens, rows / G));
-    return (double)(window > 0 ? std::min<long>(keys, window + span + keep_first)
-                               : keys);
-  };
-  auto time = [&](const Fit& f, int rows, int tile) {
-    const double wgs = ((double)tokens * G / rows + n_seqs) * n_kv;
-    return f.a + f.b * walk(rows) / tile * std::max(1.0, wgs / f.wgs);
-  };
-  return walk(64) <= 400 &&
-         time(there[D == 128][capped], 64, 32) + 0.15 * n_seqs <
-             time(here[D == 128][capped], 128, 64);
+  const long span = std::max<long>(1, std::min<long>(tokens, 64 / G));
+  const long walk = window > 0 ? std::min<long>(keys, window + span + keep_first)
+                               : keys;
+  const long wgs = (tokens * G / 128 + n_seqs) * n_kv;
+  return capped ? wgs < 256 && walk <= (D == 128 && wgs < 100 ? 63 : 32)
+                : wgs < 100 && walk <= 32;
 }
 
 // out [tokens, heads * D] rows of out_stride, fp32 or bf16; q rows, caches and

@@ -44,8 +44,8 @@ long paged_attn_scratch(bool decode, long tokens, int n_seqs, int heads, int n_k
 // one. They are where one tile holds all keys. Time there over that here, 1270 drawn calls:
 //   Prompts, by the keys from the first to the last one of a row tile and by the workgroups
 // here: up to 32 keys 0.91 (up to 99 workgroups), 1.07 (255), capped 0.85, 0.96; 33 to 48 1.06,
-// 1.17, capped 0.97, 1.08; then 1.16 to 2.4. (A fit to calls of both before few rows' keys were shared by waves sent 179 of 600
-// there, of which 77 took over 5% longer.)
+// 1.17, capped 0.97, 1.08; then 1.16 to 2.4. (A fit to calls of both before few rows' keys
+// were shared by waves sent 179 of 600 there, of which 77 took over 5% longer.)
 //   Decode, 128 wide, by the keys a row sees: tables of up to 32 keys 0.97, 0.87 (9 to 16
 // heads a key head), 0.72 (more); windows as small in longer ones lie in two tiles, 1.31, 1.17,
 // 0.96; 33 to 64 keys 1.27, 1.19, 0.97; 65 to 128 1.89, 1.78, 1.50; more 1.6, 1.3, and 0.90 for

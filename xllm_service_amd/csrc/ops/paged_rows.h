@@ -268,15 +268,19 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, int turn,
     // one. Two groups of waves, 6 x 337 behind 230 of 8/1 in a window 34.9 and 24.8.
     if (!fits(parts_of(per))) {
       // of a causal prompt the row tiles are half as long on average as the last of them
-      const int seen = min(n, (max(keys - len / 2, 0) + PF_KT - 1) / PF_KT);
-      const int mean = __builtin_amdgcn_readlane(pf_scan<true>(nt * seen), 63);
-      const int now = chain(parts_of(per)), step = max(per / 8, 1);
-      const int turns = groups > 1 ? 2 * now
-                                   : now + (int)((float)now * mean / max(work, 1)) +
-                                         (MORE ? 2 : 4);
+      auto turns = [&]() {
+        const int now = chain(parts_of(per));
+        if (groups > 1) return 2 * now;
+        const int seen = min(n, (max(keys - len / 2, 0) + PF_KT - 1) / PF_KT);
+        const int mean = __builtin_amdgcn_readlane(pf_scan<true>(nt * seen), 63);
+        return now + (int)((float)now * mean / max(work, 1)) + (MORE ? 2 : 4);
+      };
+      const int step = max(per / 8, 1);
       for (int q = per + step; q <= 2 * per; q += step)
         if (fits(parts_of(q))) {
-          if (chain(parts_of(q)) <= turns) per = q;
+          // two groups of waves: a quarter more is no turn
+          if ((groups > 1 && q <= per + per / 4) || chain(parts_of(q)) <= turns())
+            per = q;
           break;
         }
     }
@@ -638,7 +642,8 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
 #pragma unroll
     for (int k = 0; k < MEET; k++) {
       on[k] = k < parts && k * tpp < list.n;
-      z[k] = mr_load_far2(unit_ml, on[k] ? (k * PF_ROWS + row) * 8 : GONE);
+      if (k < 4 || parts > 4)
+        z[k] = mr_load_far2(unit_ml, on[k] ? (k * PF_ROWS + row) * 8 : GONE);
     }
     float top = -INFINITY;
 #pragma unroll

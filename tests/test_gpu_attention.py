@@ -673,7 +673,7 @@ def test_prefill_orders_and_groups(kv_heads, per, dim, lens, ctx, sign):
     (12, 1, 64, [58, 115, 97, 31, 64, 0, 60] * 2, [3, 1] * 7, -1.0),
 ])
 def test_prefill_order_of_turns(kv_heads, per, dim, lens, ctx, sign):
-    """Row tiles of one turn of the CUs as they are, of more than two folded."""
+    """Row tiles of one turn of the CUs as they are, of up to two folded, of more."""
     test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign)
 
 

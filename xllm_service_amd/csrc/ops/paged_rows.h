@@ -119,15 +119,11 @@ XLLM_DEV int pf_scan(int v) {
 // Which of `total` units, the longest first, workgroup b takes where a CU holds two and
 // `turn` come one to a CU: what is left over joins the shortest of those, the very shortest
 // the longest of them, so that the longest have a CU to themselves. (Joined to the longest
-// of all, 500 and 695 tokens of 28/4 heads, 268 workgroups, took 24.1 us, 22.7 so.) Of more
-// than two turns the second comes the shortest first, what is left after it: 369 drawn
-// batches in up to four turns 0.956 -> 0.949 of the time by sequences, 6 x 559-1273 behind
-// 400-760 of 16/4 71.5 -> 67.5 us, but 3 x 508-845 behind 300 of 32/8 (536) 39.1 -> 42.2. (The
-// longest and the shortest as neighbours 0.987, the fourth turn reversed too 0.948.)
+// of all, 500 and 695 tokens of 28/4 heads, 268 workgroups, took 24.1 us, 22.7 so.) (More
+// than two turns with the second reversed: 1318 drawn batches, no faster.)
 XLLM_DEV int pf_fold(int b, int total, int turn) {
   const int over = total - turn;
-  if (over > turn) return b >= turn && b < 2 * turn ? 3 * turn - 1 - b : b;
-  if (over <= 0) return b;
+  if (over <= 0 || over > turn) return b;
   return b >= turn ? turn + total - 1 - b : b < over ? turn - over + b : b - over;
 }
 
@@ -136,8 +132,7 @@ XLLM_DEV int pf_fold(int b, int total, int turn) {
 // than the next one, so all tiles sort into levels of WIDTH of those with at most
 // WIDTH tiles of a sequence to a level, which share its keys and stay together. The level
 // of tile b is found by halves, a lane counting its sequence's tiles above one. Up to 64
-// sequences; of more, and where no order is asked for (turn 0), one sequence after the
-// other (pf_locate).
+// sequences; of more, one sequence after the other (pf_locate).
 //   Two turns of workgroups come folded (pf_fold). By sequences, the tiles of two equal
 // prompts met their likes: 2 x 1.8-2.3 k in a window of 1024 59.5 -> 54.8 us, 4 x 512 of
 // 32/8 heads 28.3 -> 22.8, 3 x 500 capped 51.5 -> 40.2. WIDTH 1, 2 and 4: 40 x 60 behind
@@ -146,7 +141,7 @@ XLLM_DEV int pf_fold(int b, int total, int turn) {
 template <int ROWS, int WIDTH>
 XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
                          int n_seqs, int G, int lane, PfPlace* place) {
-  if (n_seqs > 64 || turn == 0)
+  if (n_seqs > 64)
     return pf_locate<ROWS>(b, cu_q, seq_lens, n_seqs, G, lane, place);
   if (n_seqs == 1) {                             // without scans: 0.4 us of a small call
     const int q0 = cu_q[0], n = cu_q[1] - q0, all = (n * G + ROWS - 1) / ROWS;
@@ -315,7 +310,8 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, int turn,
 // product of its own into the same fp32 sums. MORE: the options of PagedMore.
 // KG: groups of four waves, each with the same rows and its share of the tiles: what
 // splitting keys over workgroups does, without partial results in memory.
-template <int D, int TERMS, bool MORE, int KG, bool SPLIT>
+// SORT: the longest chains first, where keys are not split.
+template <int D, int TERMS, bool MORE, int KG, bool SPLIT, bool SORT = true>
 __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
     void* __restrict__ out,                  // [total_q, n_qheads, D]
     float* __restrict__ ws_o,                // [blocks][PF_ROWS * D], a block for a part
@@ -360,9 +356,13 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
                                  seq_lens, n_seqs, G, n_kv, lane, &at, &part,
                                  &parts, &first))
       return;
+  } else if constexpr (SORT) {
+    if (!pf_longest<PF_ROWS, 2>(blockIdx.x / n_kv,
+                                KG > 1 ? INT_MAX / 2 : 256 / n_kv, cu_q, seq_lens,
+                                n_seqs, G, lane, &at))
+      return;
   } else {
-    if (!pf_longest<PF_ROWS, 2>(blockIdx.x / n_kv, KG > 1 ? INT_MAX / 2 : turn, cu_q,
-                                seq_lens, n_seqs, G, lane, &at))
+    if (!pf_locate<PF_ROWS>(blockIdx.x / n_kv, cu_q, seq_lens, n_seqs, G, lane, &at))
       return;
   }
   const int seq = at.seq, lt = at.lt, q_start = at.q_start, q_len = at.q_len,
@@ -894,20 +894,22 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
   if (plan.meet) meet = paged_meet(ws_ml, wgs * PF_ROWS, 1);
   int2* ws_at = plan.least > 0 && !plan.meet && n_seqs > 1
                     ? reinterpret_cast<int2*>(ws_ml + wgs * PF_ROWS * 2) : nullptr;
+  const int turn = 256 / n_kv;
   // Batches that the CUs hold one to each come as they are, without a search: 8 x 38-140 of
-  // 28/4 9.62 -> 9.46 us, 60 drawn ones 1.00 -> 0.985 of the time before the search.
-  const int turn = n_seqs > 1 && wgs <= 256 ? 0 : 256 / n_kv;
-#define PF_GO(KG, SPLIT)                                                       \
-  hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG, SPLIT>),      \
+  // 28/4 9.62 -> 9.46 us, 325 drawn ones 0.941 -> 0.934 of the time before there was one.
+  const bool as_is = n_seqs > 1 && wgs <= 256;
+#define PF_GO(KG, SPLIT, SORT)                                                 \
+  hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG, SPLIT, SORT>),\
                      dim3((unsigned)(wgs + ahead.wgs)), dim3(KG * 256), 0,     \
                      stream, out, ws_o, ws_ml, ws_at, meet, q, k_cache, v_cache, \
                      block_tables, cu_q, seq_lens, n_seqs, scale, G, n_kv,     \
                      max_blocks, q_stride, out_stride, plan.least, plan.most,  \
                      turn, x, ahead)
-  if (plan.groups == 2 && plan.least > 0) PF_GO(2, true);
-  else if (plan.groups == 2) PF_GO(2, false);
-  else if (plan.least > 0) PF_GO(1, true);
-  else PF_GO(1, false);
+  if (plan.groups == 2 && plan.least > 0) PF_GO(2, true, true);
+  else if (plan.groups == 2) PF_GO(2, false, true);
+  else if (plan.least > 0) PF_GO(1, true, true);
+  else if (as_is) PF_GO(1, false, false);
+  else PF_GO(1, false, true);
 #undef PF_GO
   if (plan.least > 0 && !plan.meet)
     paged_merge<D, MORE, PF_ROWS, PF_KT>(out, ws_o, ws_ml, ws_at, n_qheads, out_stride,

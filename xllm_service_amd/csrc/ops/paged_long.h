@@ -1,5 +1,5 @@
-// Paged attention of long prompts, 128-wide heads, bf16 in and out, causal: the
-// matrix pipe and the vector unit at once.
+// Paged attention of long prompts, 128-wide heads, bf16 in and out, causal: waves that
+// multiply and weigh in turn.
 //
 // Rows, tiles, products and LDS images are those of paged_rows.h. There each wave
 // does a tile's products and then its weights, and what the two waves of a SIMD overlap
@@ -14,7 +14,8 @@
 // v_readlane fetch from a table of 64 tiles made at once: by scalar arithmetic on the way
 // a step's loads cost 700 cycles.
 //
-// Bound by both in turn: 2210 cycles, the pipe 1024, the vector unit 1240 of them. 4
+// Bound by both, one after the other: 2210 cycles, the pipe 1024, the vector unit 1240 of
+// them, nearly their sum; whether barriers or reads from LDS keep them apart is not known. 4
 // prompts of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads of 128: 353 -> 335
 // us. What it costs is one workgroup per CU: nothing covers its start and its end, so it
 // is taken for whole turns of workgroups with long chains only (paged_long_takes).

@@ -287,7 +287,7 @@ struct PagedMeet {
   unsigned long long tag = 0;            // low 8 bits: none
 };
 typedef unsigned long long u64;
-// by one thread of a workgroup, early: at, its unit's counter
+// by one thread of a workgroup, before it counts its part: at, its unit's counter
 XLLM_DEV void paged_open(u64* at, u64 seen, u64 tag) {
   if (((seen ^ tag) >> 8) != 0)
     __hip_atomic_compare_exchange_strong(at, &seen, tag, __ATOMIC_RELAXED,

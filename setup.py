@@ -60,7 +60,8 @@ ext_modules = [
         sources=[
             os.path.join(HYB, f)
             for f in ("bindings.cpp", "norms.hip", "latent_attn.hip",
-                      "latent_attn_mfma.hip", "latent_stream.hip",
+                      "latent_attn_mfma.hip", "latent_rows.hip",
+                      "latent_stream.hip",
                       "decay_attn.hip",
                       "decay_attn_mfma.hip", "moe.hip",
                       "streams.hip", "short_conv.hip",

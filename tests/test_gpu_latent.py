@@ -1,5 +1,5 @@
-"""Decoded rows of latent attention at rank 512, at the edges of pages, tiles,
-windows and key parts, against fp64. The weights have 32 bits: an output may
+"""Decoded and prompt rows of latent attention at rank 512, at the edges of pages,
+tiles, windows and key parts, against fp64. The weights have 32 bits: an output may
 be off by 2^-17 of the weighted sum of absolute values (exponents are rounded
 products of up to 2^5)."""
 import math
@@ -90,3 +90,81 @@ def test_fixed_parts(op, monkeypatch):
         used[parts] = torch.cuda.max_memory_allocated() - before
         assert (out - free).abs().max() <= 1e-5
     assert used[1] == 0 and used[16] > 0, used
+
+
+@pytest.mark.parametrize("tail", [0, 64])
+@pytest.mark.parametrize("heads,new,old,window", [
+    (16, [1, 8, 9, 40], [0, 31, 64, 15], 0),     # edges of row and key tiles
+    (21, [7, 1, 30], [90, 33, 0], 40),           # heads that divide no row tile
+    (32, [5], [1500], 0),                        # parts of one sequence
+    (16, [3, 20, 2], [1100, 0, 400], 0),         # ... of several, and one without
+    (32, [9, 4], [700, 1300], 500),              # ... in a window
+    (1, [300, 2], [10, 5], 1),
+    (16, [3] * 70, [40] * 70, 0),                # more sequences than lanes
+    (32, [500, 300, 60], [0, 70, 800], 0)])      # a turn of the CUs and more
+def test_prompt_edges(tail, heads, new, old, window):
+    g = torch.Generator().manual_seed(tail + heads + window + len(new))
+    W, r, scale = 512 + tail, 512, 192 ** -0.5
+    keys = [n + o for n, o in zip(new, old)]
+    need = [-(-n // 16) for n in keys]
+    cache = torch.randn(sum(need) + 3, 16, W, generator=g).to(torch.bfloat16)
+    order = torch.randperm(sum(need) + 3, generator=g).to(torch.int32)
+    table = torch.zeros(len(keys), max(need) + 1, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        table[i, :n] = order[at:at + n]
+        at += n
+    q = torch.randn(sum(new), heads, W, generator=g).to(torch.bfloat16)
+    cache[table[0, 0], 0] *= 20.0                # one key far above the others
+    cu = [0]
+    for n in new:
+        cu.append(cu[-1] + n)
+    for sign in (1.0, -1.0):
+        out = torch.full((sum(new), heads, r), 9.0, device="cuda")
+        H.latent_attn(q.cuda(), cache.cuda(), table.cuda(),
+                      torch.tensor(cu, dtype=torch.int32, device="cuda"),
+                      torch.tensor(keys, dtype=torch.int32, device="cuda"),
+                      sign * scale, r, out, window)
+        for s, n in enumerate(new):
+            k = cache[table[s, :need[s]].long()].reshape(-1, W)[:keys[s]].cuda()
+            k = k.double()
+            z = q[cu[s]:cu[s + 1]].cuda().double() @ k.t() * (sign * scale)
+            pos = old[s] + torch.arange(n, device="cuda")[:, None, None]
+            at = torch.arange(keys[s], device="cuda")
+            z = z.masked_fill((at > pos) | (window > 0) & (at <= pos - window),
+                              -math.inf)
+            p = torch.softmax(z, -1)
+            off = (out[cu[s]:cu[s + 1]].double() - p @ k[:, :r]).abs()
+            # A score is a sum of 36 products in a row, each rounded to 2^-24 of what
+            # is summed, at most |q| |k|: errors of 6 such steps, as they add up at
+            # random, are more than 2^-17 where the standout key is seen.
+            most = (q[cu[s]:cu[s + 1]].cuda().double().abs() @ k.abs().t()).masked_fill(
+                z == -math.inf, 0.0).amax(-1, keepdim=True) * scale
+            bound = (6 * 2.0 ** -24 * most).clamp(min=2.0 ** -17)
+            over = off - bound * (p @ k[:, :r].abs())
+            assert over.max() <= 1e-7, f"sequence {s}: off by {off.max():.3g}"
+
+
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("heads,old", [(16, 0), (32, 70), (16, 1500)])
+def test_prompt_nonfinite(heads, old, bad):
+    """A new token's latent that is not finite is lost to the rows that see it, and to
+    no token in front of its 64 rows; so is a NaN factor to all."""
+    g = torch.Generator().manual_seed(heads + old)
+    n, W, at = 24, 576, 9
+    need = -(-(n + old) // 16)
+    cache = torch.randn(need, 16, W, generator=g).to(torch.bfloat16)
+    cache.view(-1, W)[old + at, 40] = bad
+    table = torch.arange(need, dtype=torch.int32)[None].cuda()
+    q = torch.randn(n, heads, W, generator=g).to(torch.bfloat16).cuda()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    out = torch.zeros(n, heads, 512, device="cuda")
+
+    def run(scale):
+        H.latent_attn(q, cache.cuda(), table, torch.tensor([0, n], **i32),
+                      torch.tensor([n + old], **i32), scale, 512, out, 0)
+        return torch.isfinite(out)
+    fine = run(0.07)
+    assert not fine[at:, :, 40].any()
+    assert fine[:at * heads // 64 * 64 // heads].all()
+    assert not run(math.nan).any()

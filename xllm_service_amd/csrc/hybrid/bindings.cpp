@@ -65,6 +65,12 @@ void launch_latent_attn(float*, const T*, const T*, const int*, const int*,
                         const int*, int, int, int, int, int, int, int, float,
                         long, int, hipStream_t);
 int latent_attn_mfma_class(int W, int r);
+bool latent_rows_takes(int, int, int);
+long latent_rows_scratch(long, int, int, long, int);
+void launch_latent_rows(float*, float*, const unsigned short*,
+                        const unsigned short*, const int*, const int*,
+                        const int*, long, int, int, int, int, float, int,
+                        hipStream_t);
 bool latent_stream_takes(int, int, int, int);
 int latent_stream_parts(int, int, long, int);
 void launch_latent_stream(float*, float*, float*, const unsigned short*,
@@ -596,6 +602,20 @@ void latent_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables,
                              ptr<bf>(cache), ptr<int>(block_tables),
                              ptr<int>(seq_lens), n_seqs, H, W,
                              block_tables.size(1), scale, n_part, window, cur());
+    return;
+  }
+  // prompt rows of these sizes
+  if (is_bf16(q) && cu != nullptr &&
+      hy::latent_rows_takes(W, r, cache.size(1)) && aligned(q) &&
+      aligned(cache) && aligned(out) && block_tables.size(1) > 0) {
+    const long n =
+        hy::latent_rows_scratch(T, n_seqs, H, block_tables.size(1), window);
+    Tensor ws;
+    if (n > 0) ws = torch::empty({n}, out.options());
+    hy::launch_latent_rows(ptr<float>(out), n > 0 ? ptr<float>(ws) : nullptr,
+                           ptr<bf>(q), ptr<bf>(cache), ptr<int>(block_tables),
+                           cu, ptr<int>(seq_lens), T, n_seqs, H, W,
+                           block_tables.size(1), scale, window, cur());
     return;
   }
   // bf16: MFMA kernel when the sizes fit one of its instantiations

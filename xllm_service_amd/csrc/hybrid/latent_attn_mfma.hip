@@ -1,4 +1,5 @@
-// MFMA latent attention (bf16 activations/cache) for gfx950.
+// MFMA latent attention (bf16 activations/cache) for gfx950. Rank 512 with 16-token
+// pages: latent_stream.hip (decoded rows, up to 32 heads) and latent_rows.hip (prompts).
 //
 // All heads of a token attend to the SAME cached rows [latent | rotated key],
 // so (query, head) pairs are just rows of one big query matrix: row

@@ -1,6 +1,6 @@
 // Latent attention of decoded rows (bf16) for gfx950: rank 512 with a rotated
-// tail of 0 or 64 entries, 16-token pages, at most 32 heads. Other sizes and
-// prompt rows: latent_attn_mfma.hip.
+// tail of 0 or 64 entries, 16-token pages, at most 32 heads. Prompt rows:
+// latent_rows.hip, other sizes: latent_attn_mfma.hip.
 //
 // One new token per sequence; its heads attend to the SAME cached rows of W =
 // 512 + tail entries, values are the first 512 of a row. The step is a stream

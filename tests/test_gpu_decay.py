@@ -82,6 +82,19 @@ def test_prompt_rows(D, V, lens, bound):
         sum(lens) + D + V)
 
 
+@pytest.mark.parametrize("D,V", [(128, 128), (64, 128), (128, 64), (64, 64)])
+@pytest.mark.parametrize("lens,bound", [
+    ([100, 40, 128, 3] * 23, 128),      # more workgroups than CUs: one chunk each
+    ([130, 64, 257, 2, 65] * 20, 257),  # ... and sequences that are walked
+    ([1500, 1, 3], 1500),               # few long ones: sums and a scan
+    ([128, 256, 192], 256)])            # walked, by few
+def test_prompt_routes(D, V, lens, bound):
+    """Each way from chunk to chunk, and outputs by four waves and by sixteen."""
+    n = len(lens)
+    run(D, V, lens, [5 * (i % 3) for i in range(n)],
+        [i if i % 7 else -1 for i in range(n)], [0.999, 0.75, 1.0], bound, n + D + V)
+
+
 def test_many_chunks_and_hard_decays():
     """More chunks than the scan holds in flight; decays whose powers leave
     fp32's normal range within a chunk, and none at all."""

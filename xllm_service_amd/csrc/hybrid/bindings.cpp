@@ -87,7 +87,7 @@ void launch_decay_attn_mfma(float*, const unsigned short*,
                             const unsigned short*, const unsigned short*,
                             const float*, float*, const int*, const int*,
                             const int*, long, int, int, int, int, long, long,
-                            long, float*, hipStream_t);
+                            long, float*, long, hipStream_t);
 template <typename T>
 void launch_decay_attn(float*, const T*, const T*, const T*, const float*,
                        float*, const int*, const int*, const int*, int, int,
@@ -708,7 +708,7 @@ void decay_attn(Tensor out, Tensor q, Tensor k, Tensor v, Tensor decay,
           ptr<float>(out), ptr<bf>(q), ptr<bf>(k), ptr<bf>(v),
           ptr<float>(decay), ptr<float>(state), ptr<int>(slots), cu,
           ptr<int>(ctx_lens), T, n_seqs, H, D, Dv, q.stride(0), k.stride(0),
-          v.stride(0), one ? nullptr : ptr<float>(ws), cur());
+          v.stride(0), one ? nullptr : ptr<float>(ws), longest, cur());
       return;
     }
   }

@@ -13,9 +13,10 @@
 //
 //   sum   what every (chunk, head) adds to the state, all chunks at once
 //   scan  chunk after chunk per state element (recurrent_chunks.h)
-//   out   the outputs of every (chunk, head)
+//   walk  both, by workgroups that follow a sequence: many sequences of few chunks
+//   out   the outputs of every (chunk, head), by four waves or by sixteen
 // Batches whose sequences all fit one chunk need no scratch and no scan: out
-// reads the slots, then sum moves them.
+// reads the slots, then sum or walk moves them.
 //
 // Chunks of 128 tokens halve the scratch traffic of 64 (a record is a whole
 // state per head), and the products within a chunk they add are cheap.
@@ -25,7 +26,9 @@
 // the vector unit, two passes and a scan. out and sum run one round of workgroups whose
 // phases (activate, split, multiply) follow each other, two to a CU, and are bound by
 // the vector unit: activations and splits. What a phase reads is fetched during the one
-// before it: 68.0 -> 61.9 us in all.
+// before it: 68.0 -> 61.9 us in all. One wave issues a vector instruction in 6 cycles, two
+// of a SIMD in 3 each: a workgroup alone on a CU takes as long as two, 19 us of out for
+// 160 of them, hence the kernels of 8 and 16 waves for small batches.
 #include "../ops/mfma_rows.h"
 #include "recurrent_chunks.h"
 
@@ -218,14 +221,177 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
 #pragma unroll
   for (int i = 0; i < DT; ++i)
 #pragma unroll
-    for (int j = 0; j < VT; ++j)
+    for (int j = 0; j < VT; ++j) {
+      float* p = dst + ((d0 + i) * 32 + 4 * h) * V + (e0 + j) * 32 + n;
+      // all of it on the way before the first is stored, which might be another's place
+      float x[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) x[r] = add ? p[(8 * (r >> 2) + (r & 3)) * V] : 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int d = (d0 + i) * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-        float* p = dst + d * V + (e0 + j) * 32 + n;
         const float u = acc[0][i][j][r] + acc[1][i][j][r];
-        *p = add ? keep * *p + u : u;
+        p[(8 * (r >> 2) + (r & 3)) * V] = add ? keep * x[r] + u : u;
       }
+    }
+}
+
+// ---- walk: a state from chunk to chunk --------------------------------------------
+// A workgroup (8 waves) owns 64 x 64 entries of one (sequence, head)'s state and walks its
+// chunks: the state before each goes to the chunk's record, the last one to the slot. A
+// wave makes 32 x 32 of what a chunk adds from half of its tokens; two waves swap halves
+// of their sums and keep half of the state each. 64 tokens are staged at a time, a 16 B
+// piece of both a thread, into one of two buffers while the other one is multiplied.
+//   A chunk takes 2.9 us, most of it activations and splits (each key and value is
+// activated for two slices), whatever the number of sequences up to two workgroups a CU;
+// in return records go out once and never come back to be summed. Us in all, sum and scan
+// | walk: 2 prompts of 164-341 tokens, 32 heads 39.1 | 25.6, 8 of 197-471 114 | 90, 6 of
+// 449-912 154 | 126, 30 of 200-300 353 | 229; but 3 of 700-2000, 16 heads 65 | 76.
+template <int D, int V>
+__global__ void __launch_bounds__(512, 4) decay_walk_mfma_kernel(DMArgs P) {
+  constexpr int ST = 64, IMG = ST * 64, BUF = 4 * IMG;     // three of keys, one of values
+  constexpr int SL = (D / 64) * (V / 64);
+  // one object: its end swaps the sums
+  __shared__ __attribute__((aligned(1024))) unsigned short
+      lds[2 * BUF + 8 * 2 * 64 * 8];
+  typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f4;
+  f4* swap = reinterpret_cast<f4*>(lds + 2 * BUF);         // [wave][2][lane]
+  // slices of a state on one XCD: they read the same rows
+  const int sl = blockIdx.x / 8 % SL;
+  const int sh = blockIdx.x / (8 * SL) * 8 + blockIdx.x % 8;
+  if (sh >= P.n_seqs * P.heads) return;
+  const int s = sh / P.heads, hd = sh - s * P.heads;
+  const int d0 = sl % (D / 64) * 64, e0 = sl / (D / 64) * 64;
+  const int t0 = P.cu_q[s], len = P.cu_q[s + 1] - t0;
+  const int slot = P.slots[s];
+  const bool carried = slot >= 0 && P.ctx_lens[s] > 0;
+  const int chunks = (len + DM_C - 1) / DM_C;
+  const int last = len - (chunks - 1) * DM_C;              // tokens of the last one
+  long rec = 0;                                            // its first record
+  if (P.ws != nullptr)
+    for (int i = 0; i < s; ++i)
+      rec += (P.cu_q[i + 1] - P.cu_q[i] + DM_C - 1) / DM_C;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, n = lane & 31;
+  const int dt = w & 1, et = w >> 1 & 1, half = w >> 2;
+  const int r = tid >> 3, ch = tid & 7;                    // of its pieces
+
+  // pieces of two chunks on their way
+  ushort8_t kr[2][2], vr[2][2];
+  auto fetch = [&](int c, int p, ushort8_t& k, ushort8_t& v) {
+    const long t = t0 + min(c * DM_C + p * ST + r, len - 1);
+    k = dm_row(P.k + t * P.k_stride + hd * D + d0 + ch * 8);
+    v = dm_row(P.v + t * P.v_stride + hd * V + e0 + ch * 8);
+  };
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      if (c < chunks) fetch(c, p, kr[c][p], vr[c][p]);
+  // this wave's half of the 32 x 32: registers 8 half .. of a product's
+  long at[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    at[i] = (long)(d0 + dt * 32 + 16 * half + 8 * i + 4 * h) * V + e0 + et * 32 + n;
+  float S[8];
+  float* st = P.state + ((long)max(slot, 0) * P.heads + hd) * (D * V);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) S[i] = carried ? st[at[i >> 2] + (i & 3) * V] : 0.f;
+  // weights of this thread's token in either half of a whole chunk, and of the last
+  const float a = P.decay[hd];
+  float whole[2] = {0.f, 0.f}, keep = 0.f;
+  if (chunks > 1) {
+    whole[0] = dm_pow(a, DM_C - 1 - r);
+    whole[1] = dm_pow(a, ST - 1 - r);
+    keep = dm_pow(a, DM_C);
+  }
+  const float rest[2] = {dm_pow(a, max(last - 1 - r, 0)),
+                         dm_pow(a, max(last - ST - 1 - r, 0))};
+  const float keep_last = dm_pow(a, max(last, 0));
+  auto stage = [&](int c, int p, const ushort8_t& k, const ushort8_t& v) {
+    const bool end = c == chunks - 1;
+    const bool in = !end || p * ST + r < last;
+    unsigned short* ks = lds + p * BUF;
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    dm_u4 y = {{0u, 0u, 0u, 0u}};
+    if (in) {
+      const dm_u4 z = dm_act(k);
+      const float wgt = end ? rest[p] : whole[p];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[2 * j] = __uint_as_float(z.x[j] << 16) * wgt;
+        x[2 * j + 1] = __uint_as_float(z.x[j] & 0xffff0000u) * wgt;
+      }
+      y = dm_act(v);
+    }
+    const int to = r * 64 + ((ch ^ mr_swz_cols<64>(r)) << 3);
+    dm_split(x, ks + to, IMG);
+    *reinterpret_cast<dm_u4*>(ks + 3 * IMG + to) = y;
+  };
+  const int base = mr_col_base<64>(lane) + half * 32 * 64;
+  // leading and other terms apart, as in sum
+  f32x16 acc[2];
+  auto multiply = [&](int p) {
+    const lds_u16* ks = (const lds_u16*)lds + p * BUF;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const bf16x8 b = mr_cols<64>(ks + 3 * IMG + (base ^ (et << 5)) + k * 16 * 64);
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        acc[t > 0] = mr_mma(
+            mr_cols<64>(ks + t * IMG + (base ^ (dt << 5)) + k * 16 * 64), b,
+            acc[t > 0]);
+    }
+  };
+  auto chunk = [&](int c, ushort8_t (&k)[2], ushort8_t (&v)[2], ushort8_t& k_next,
+                   ushort8_t& v_next) {
+    acc[0] = acc[1] = mr_zero();
+    multiply(0);
+    const bool two = c < chunks - 1 || last > ST;  // halves of the chunk, uniform
+    if (two) stage(c, 1, k[1], v[1]);
+    if (c + 2 < chunks) {
+      fetch(c + 2, 0, k[0], v[0]);
+      fetch(c + 2, 1, k[1], v[1]);
+    }
+    __syncthreads();
+    if (two) multiply(1);
+    if (c + 1 < chunks) stage(c + 1, 0, k_next, v_next);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      f4 z;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int x = 4 * i + j;
+        z[j] = half ? acc[0][x] + acc[1][x] : acc[0][8 + x] + acc[1][8 + x];
+      }
+      swap[(w * 2 + i) * 64 + lane] = z;
+    }
+    __syncthreads();
+    float* to = P.ws + ((rec + c) * P.heads + hd) * (D * V);
+    const bool store = P.ws != nullptr && (c > 0 || carried);
+    const float by = c == chunks - 1 ? keep_last : keep;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f4 z = swap[((w ^ 4) * 2 + i) * 64 + lane];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int x = 4 * i + j;
+        const float u =
+            (half ? acc[0][8 + x] + acc[1][8 + x] : acc[0][x] + acc[1][x]) + z[j];
+        if (store) to[at[i] + j * V] = S[x];
+        S[x] = fmaf(by, S[x], u);
+      }
+    }
+  };
+  if (chunks > 0) stage(0, 0, kr[0][0], vr[0][0]);
+  __syncthreads();
+  for (int c = 0; c < chunks; c += 2) {
+    chunk(c, kr[0], vr[0], kr[1][0], vr[1][0]);
+    if (c + 1 < chunks) chunk(c + 1, kr[1], vr[1], kr[0][0], vr[0][0]);
+  }
+  if (slot < 0 || (len <= 0 && carried)) return;           // nothing to keep, or as it is
+#pragma unroll
+  for (int i = 0; i < 8; ++i) st[at[i >> 2] + (i & 3) * V] = S[i];
 }
 
 // ---- out ------------------------------------------------------------------------
@@ -455,6 +621,237 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
           acc[0][j][r + 3] + acc[1][j][r + 3]);
 }
 
+// ---- out, few workgroups ---------------------------------------------------------
+// A workgroup (16 waves, 8 of 64 values, a CU to itself) owns a (chunk, head); a wave 32
+// queries by 32 values, sums in 32 registers. All that it reads is asked for at once;
+// then the state's three images and the queries go to LDS and meet there, keys and values
+// are activated in registers meanwhile and take the images' place. Each weighted tile of
+// scores is made once, by one of the waves that want it, and passed on through LDS: 16 B a
+// lane, as the products take it.
+//   Up to a workgroup for each CU it takes 14 us for 19 of the four waves' kernel (2
+// prompts of 164-341 tokens, 32 heads, 30.3 -> 25.6 in all): all it reads comes at the rate
+// of a CU (160 KB, 2 us), then a SIMD has four waves to issue from. Beyond that nothing
+// is read while it computes, and two workgroups a CU are faster: 528 of them 31 | 36.
+template <int D, int V>
+__global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
+  constexpr int NV = V / 32, NT = 256 * NV;       // column tiles, threads
+  constexpr int KS = D / 16;
+  constexpr int QP = DM_C * D / 8 / NT, VP = DM_C * V / 8 / NT;   // pieces of a thread
+  constexpr int SP = D * V / 8 / NT;
+  // queries | state, then keys, values, weights | powers, first lost token of a column
+  constexpr int IMG = D * V, KEYS = DM_C * D, VALS = KEYS + DM_C * D,
+                WGTS = VALS + DM_C * V, TILE = 3 * 2 * 64 * 8;
+  constexpr int END = (KEYS + 3 * IMG > WGTS + 10 * TILE ? KEYS + 3 * IMG
+                                                         : WGTS + 10 * TILE);
+  __shared__ __attribute__((aligned(1024))) unsigned short
+      lds[END + 2 * (DM_C + 4) + 2 * V];
+  float* pw = reinterpret_cast<float*>(lds + END);
+  int* lost = reinterpret_cast<int*>(lds + END + 2 * (DM_C + 4));
+  int s, c, t0, len;
+  if (!dm_locate(P, &s, &c, &t0, &len) || len <= 0) return;
+  const int hd = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a SIMD's waves have different queries: later ones meet more keys
+  const int vt = w >> 2, qt = (w + vt) & 3;
+  const int h = lane >> 5, n = lane & 31;
+  const int slot = P.slots[s];
+  const bool carried = slot >= 0 && P.ctx_lens[s] > 0;
+  const bool before = c > 0 || carried;           // uniform
+  const float* S =
+      (P.ws != nullptr
+           ? P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V)
+           : P.state + ((long)max(slot, 0) * P.heads + hd) * (D * V));
+  auto row_of = [&](int idx, int W) { return min(idx / (W / 8), len - 1); };
+  ushort8_t qr[QP], kr[QP], vr[VP];
+  float sr[SP][8];
+#pragma unroll
+  for (int i = 0; i < QP; ++i) {
+    const int idx = tid + i * NT;
+    qr[i] = dm_row(P.q + (long)(t0 + row_of(idx, D)) * P.q_stride + hd * D +
+                   idx % (D / 8) * 8);
+  }
+  if (before) {
+#pragma unroll
+    for (int i = 0; i < SP; ++i) {
+      const float* p = S + (tid + i * NT) * 8;
+      Quad<float>::ld(p, sr[i]);
+      Quad<float>::ld(p + 4, sr[i] + 4);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < QP; ++i) {
+    const int idx = tid + i * NT;
+    kr[i] = dm_row(P.k + (long)(t0 + row_of(idx, D)) * P.k_stride + hd * D +
+                   idx % (D / 8) * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < VP; ++i) {
+    const int idx = tid + i * NT;
+    vr[i] = dm_row(P.v + (long)(t0 + row_of(idx, V)) * P.v_stride + hd * V +
+                   idx % (V / 8) * 8);
+  }
+  if (tid <= DM_C) pw[tid] = dm_pow(P.decay[hd], tid);
+#pragma unroll
+  for (int i = 0; i < QP; ++i) {
+    const int idx = tid + i * NT, r = idx / (D / 8), ch = idx % (D / 8);
+    dm_u4 y = {{0u, 0u, 0u, 0u}};
+    if (r < len) y = dm_act(qr[i]);
+    *reinterpret_cast<dm_u4*>(lds + r * D + ((ch ^ mr_swz_rows<D>(r)) << 3)) = y;
+  }
+  if (before) {
+#pragma unroll
+    for (int i = 0; i < SP; ++i) {
+      const int idx = tid + i * NT, r = idx / (V / 8), ch = idx % (V / 8);
+      dm_split(sr[i], lds + KEYS + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3), IMG);
+    }
+  }
+  __syncthreads();
+  const bool on = qt * 32 < len;                  // uniform in a wave
+  const int qi = qt * 32 + n;
+  const int rbase = mr_row_base<D>(lane), vbase = mr_col_base<V>(lane) ^ (vt << 5);
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    qf[ks] = *reinterpret_cast<const lds_bf16x8*>(
+        (const lds_u16*)lds + qi * D + (((2 * ks + h) ^ mr_swz_rows<D>(qi)) << 3));
+  // Products of the leading terms and those of the other two are summed apart, and the
+  // leading ones of four steps (of two within the chunk) before they meet the large sum,
+  // which then is rounded 6 times instead of 16. Error against 64 bits, 3 prompts of
+  // 853-1657 tokens: 8.2e-8 -> 6.7e-8 (the recurrence: 7.1e-8).
+  f32x16 acc[2] = {mr_zero(), mr_zero()};
+
+  // ---- through the state before the chunk ------------------------------------
+  if (before && on) {
+#pragma unroll
+    for (int d0 = 0; d0 < D; d0 += 64) {
+      f32x16 z = mr_zero();
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          const bf16x8 x = mr_cols<V>((const lds_u16*)lds + KEYS + t * IMG +
+                                      (d0 + st * 16) * V + vbase);
+          if (t == 0) z = mr_mma(x, qf[d0 / 16 + st], z);
+          else acc[1] = mr_mma(x, qf[d0 / 16 + st], acc[1]);
+        }
+      acc[0] += z;
+    }
+    const float fade = pw[min(qi, DM_C - 1) + 1];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      acc[0][r] *= fade;
+      acc[1][r] *= fade;
+    }
+  }
+  // ---- within the chunk --------------------------------------------------------
+  unsigned odd = 0u;
+  dm_u4 ka[QP], va[VP];
+#pragma unroll
+  for (int i = 0; i < QP; ++i) {
+    ka[i] = dm_u4{{0u, 0u, 0u, 0u}};
+    if ((tid + i * NT) / (D / 8) < len) ka[i] = dm_act(kr[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < VP; ++i) {
+    va[i] = dm_u4{{0u, 0u, 0u, 0u}};
+    if ((tid + i * NT) / (V / 8) < len) va[i] = dm_act(vr[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) odd |= dm_odd(va[i].x[j]);
+  }
+  if (before) __syncthreads();                    // the images are read
+  unsigned short* vs = lds + VALS;
+#pragma unroll
+  for (int i = 0; i < QP; ++i) {
+    const int idx = tid + i * NT, r = idx / (D / 8), ch = idx % (D / 8);
+    *reinterpret_cast<dm_u4*>(lds + KEYS + r * D +
+                              ((ch ^ mr_swz_rows<D>(r)) << 3)) = ka[i];
+  }
+#pragma unroll
+  for (int i = 0; i < VP; ++i) {
+    const int idx = tid + i * NT, r = idx / (V / 8), ch = idx % (V / 8);
+    *reinterpret_cast<dm_u4*>(vs + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3)) = va[i];
+  }
+  // A weight of zero keeps a key out of a row unless its value is not finite: the
+  // products see zero instead, and rows from that token on are NaN at the end.
+  const bool any_lost = __syncthreads_or(odd != 0u);
+  if (any_lost) {
+    for (int i = tid; i < V; i += NT) lost[i] = DM_C;
+    __syncthreads();
+    for (int i = tid; i < DM_C * V; i += NT) {
+      const int r = i / V, e = i % V;
+      unsigned short* x = vs + r * V + (((e >> 3) ^ mr_swz_cols<V>(r)) << 3) +
+                          (e & 7);
+      if (dm_odd(*x) == 0u) continue;
+      *x = 0;
+      atomicMin(lost + e, r);
+    }
+    __syncthreads();
+  }
+  // the weights of keys 32 kt .. for queries 32 qt ..: tile qt (qt + 1) / 2 + kt
+  typedef __attribute__((address_space(3))) bf16x8 lds_frag;
+  lds_frag* wt = (lds_frag*)((lds_u16*)lds + WGTS) + qt * (qt + 1) / 2 * 6 * 64 + lane;
+  if (on) {
+    for (int kt = vt; kt <= qt; kt += NV) {
+      f32x16 z = mr_zero();
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        z = mr_mma(*reinterpret_cast<const lds_bf16x8*>(
+                       (const lds_u16*)lds + KEYS + (rbase ^ (ks << 4)) + kt * 32 * D),
+                   qf[ks], z);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int back = qi - kt * 32 - mr_key_of(r, h);
+        z[r] = back >= 0 ? z[r] * pw[max(back, 0)] : 0.f;
+      }
+      bf16x8 p[3][2];
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        float x = z[r], y = z[r + 1];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          const unsigned u = pack_bf16(x, y);
+          reinterpret_cast<unsigned*>(&p[t][r >> 3])[(r & 7) >> 1] = u;
+          drop_bf16(x, y, u);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int st = 0; st < 2; ++st) wt[(kt * 6 + t * 2 + st) * 64] = p[t][st];
+    }
+  }
+  __syncthreads();
+  if (!on) return;
+  for (int kt = 0; kt <= qt; ++kt) {
+    f32x16 y = mr_zero();
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      const bf16x8 x =
+          mr_cols<V>((const lds_u16*)vs + vbase + (kt * 32 + st * 16) * V);
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const bf16x8 p = wt[(kt * 6 + t * 2 + st) * 64];
+        if (t == 0) y = mr_mma(x, p, y);
+        else acc[1] = mr_mma(x, p, acc[1]);
+      }
+    }
+    acc[0] += y;
+  }
+  if (qi >= len) return;
+  if (any_lost) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (lost[vt * 32 + 8 * (r >> 2) + 4 * h + (r & 3)] <= qi) acc[0][r] = NAN;
+  }
+  float* o = P.out + ((long)(t0 + qi) * P.heads + hd) * V + vt * 32 + 4 * h;
+#pragma unroll
+  for (int r = 0; r < 16; r += 4)
+    *reinterpret_cast<float4*>(o + 2 * r) =
+        make_float4(acc[0][r] + acc[1][r], acc[0][r + 1] + acc[1][r + 1],
+                    acc[0][r + 2] + acc[1][r + 2], acc[0][r + 3] + acc[1][r + 3]);
+}
+
 // records of scratch for a batch of prompt rows
 long decay_attn_mfma_chunks(long tokens, long n_seqs) {
   return tokens / DM_C + n_seqs;
@@ -478,24 +875,55 @@ bool decay_attn_short(long longest, long states, int D, int V) {
   return longest * 10 <= most * tenths;
 }
 
+// Whether walk takes the place of sum and scan: its time, 3 us and 2.9 a chunk of the
+// longest sequence, against theirs, a start and so much for each (chunk, head). Measured
+// (us, both kernels' | chunks of the longest, units), 128 x 128: 15 | 3, 48; 17 | 4, 128;
+// 27 | 5, 480; 30 | 13, 528; 38 | 8, 1024; 45 | 13, 1056; 51 | 7, 1150. 64 x 128 and back:
+// 12 | 4, 68; 15 | 5, 144; 17 | 3, 192; 22 | 4, 368; 27 | 3, 496. 64 x 64: 10 | 3, 48; 12 |
+// 3, 176; 18 | 5, 448; 22 | 6, 928. One chunk each, without scan: us in all, sum | walk, 32
+// (sequence, head)s of 128 tokens 20.6 | 16.8, 64 21.9 | 19.3, 128 15.6 | 16.6, 2048 147 |
+// 188; of 64 keys 48 13.0 | 13.3.
+static bool decay_walks(long longest, long tokens, int n_seqs, int heads, int D, int V) {
+  const long chunks = (longest + DM_C - 1) / DM_C;
+  if (chunks <= 1) return D == 128 && (long)n_seqs * heads <= 96;
+  const long units = (2 * tokens / DM_C + n_seqs) * heads / 2;
+  const long there = D + V == 256 ? 14000 + 30 * units
+                     : D + V == 192 ? 9000 + 40 * units : 8500 + 18 * units;   // ns
+  return 3000 + 2900 * chunks < there;
+}
+
 // D, V in {64, 128}; rows 16 B aligned. ws null: no sequence has more than
-// DM_C tokens.
+// DM_C tokens. longest: tokens of a sequence at most
 void launch_decay_attn_mfma(float* out, const unsigned short* q,
                             const unsigned short* k, const unsigned short* v,
                             const float* decay, float* state, const int* slots,
                             const int* cu_q, const int* ctx_lens, long tokens,
                             int n_seqs, int heads, int D, int V, long q_stride,
                             long k_stride, long v_stride, float* ws,
-                            hipStream_t st) {
+                            long longest, hipStream_t st) {
   if (n_seqs == 0) return;
   const DMArgs P = {out, q, k, v, q_stride, k_stride, v_stride, decay, state,
                     ws, slots, cu_q, ctx_lens, n_seqs, heads};
   const dim3 grid(
       (unsigned)(ws ? decay_attn_mfma_chunks(tokens, n_seqs) : n_seqs), heads);
+  const bool wide = (long)grid.x * heads <= 256;
+  const bool walk = decay_walks(longest, tokens, n_seqs, heads, D, V);
 #define DM_SUM(DD, VV)                                                        \
   hipLaunchKernelGGL((decay_sum_mfma_kernel<DD, VV>), grid, dim3(256), 0, st, P)
+#define DM_WALK(DD, VV)                                                       \
+  hipLaunchKernelGGL((decay_walk_mfma_kernel<DD, VV>),                        \
+                     dim3((unsigned)(((long)n_seqs * heads + 7) / 8 * 8 *     \
+                                     (DD / 64) * (VV / 64))),                 \
+                     dim3(512), 0, st, P)
 #define DM_OUT(DD, VV)                                                        \
-  hipLaunchKernelGGL((decay_out_mfma_kernel<DD, VV>), grid, dim3(256), 0, st, P)
+  do {                                                                        \
+    if (wide)                                                                 \
+      hipLaunchKernelGGL((decay_out_wide_kernel<DD, VV>), grid, dim3(8 * VV), \
+                         0, st, P);                                           \
+    else                                                                      \
+      hipLaunchKernelGGL((decay_out_mfma_kernel<DD, VV>), grid, dim3(256), 0, \
+                         st, P);                                              \
+  } while (0)
 #define DM_BY_SIZE(CALL)                                                      \
   do {                                                                        \
     if (D == 128) { if (V == 128) CALL(128, 128); else CALL(128, 64); }       \
@@ -503,18 +931,23 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
   } while (0)
   if (ws == nullptr) {
     DM_BY_SIZE(DM_OUT);
-    DM_BY_SIZE(DM_SUM);
+    if (walk) DM_BY_SIZE(DM_WALK); else DM_BY_SIZE(DM_SUM);
     return;
   }
-  DM_BY_SIZE(DM_SUM);
-  const long per_head = (long)D * V, per_seq = per_head * heads;
-  hipLaunchKernelGGL((chunk_scan_kernel<DM_C>),
-                     dim3((unsigned)((per_seq + 255) / 256), n_seqs),
-                     dim3(256), 0, st, ws, state, decay, slots, cu_q, ctx_lens,
-                     heads, per_head, true);
+  if (walk) {
+    DM_BY_SIZE(DM_WALK);
+  } else {
+    DM_BY_SIZE(DM_SUM);
+    const long per_head = (long)D * V, per_seq = per_head * heads;
+    hipLaunchKernelGGL((chunk_scan_kernel<DM_C>),
+                       dim3((unsigned)((per_seq + 255) / 256), n_seqs),
+                       dim3(256), 0, st, ws, state, decay, slots, cu_q, ctx_lens,
+                       heads, per_head, true);
+  }
   DM_BY_SIZE(DM_OUT);
 #undef DM_BY_SIZE
 #undef DM_OUT
+#undef DM_WALK
 #undef DM_SUM
 }
 

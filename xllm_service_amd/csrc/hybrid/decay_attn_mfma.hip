@@ -793,12 +793,16 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
   lds_frag* wt = (lds_frag*)((lds_u16*)lds + WGTS) + qt * (qt + 1) / 2 * 6 * 64 + lane;
   if (on) {
     for (int kt = vt; kt <= qt; kt += NV) {
-      f32x16 z = mr_zero();
+      // in two chains: a chunk of 16 tokens is no less precise than the recurrence
+      f32x16 z = mr_zero(), z1 = mr_zero();
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        z = mr_mma(*reinterpret_cast<const lds_bf16x8*>(
-                       (const lds_u16*)lds + KEYS + (rbase ^ (ks << 4)) + kt * 32 * D),
-                   qf[ks], z);
+      for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8 x = *reinterpret_cast<const lds_bf16x8*>(
+            (const lds_u16*)lds + KEYS + (rbase ^ (ks << 4)) + kt * 32 * D);
+        if (ks % 2 == 0) z = mr_mma(x, qf[ks], z);
+        else z1 = mr_mma(x, qf[ks], z1);
+      }
+      z += z1;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int back = qi - kt * 32 - mr_key_of(r, h);
@@ -862,17 +866,17 @@ int decay_attn_mfma_chunk() { return DM_C; }
 // nearly as much as one of 32 (both passes move the whole state through LDS), where
 // the recurrence of decay_attn.hip walks token by token, one workgroup per 16
 // columns of a state, whose rate falls once they fill the chip. Measured (us, the
-// recurrence | here), 128 x 128, 8 states: 2 tokens 5.8 | 24, 16 16.8 | 24.6, 24 23.3 |
-// 25.6, 32 29.6 | 25.9; 256 states: 8 22.6 | 26.7, 12 28.7 | 26.7; 1024: 8 68 | 82, 12
-// 88 | 82. 64 x 64, 8 states: 8 8.6 | 12.0, 14 12.2 | 12.1; 512: 4 13.4 | 14.0, 6 16.3 |
-// 13.9. 64 x 128, 64: 16 14.2 | 16.6, 20 17.1 | 17.2; 128 x 64, 256: 10 16.3 | 18.4, 14
-// 20.2 | 18.4.
+// recurrence | here, tokens), fresh sequences; continued ones meet one or two tokens later.
+// 128 x 128, 16 states: 8 9.7 | 10.8, 10 11.3 | 10.9, 16 16.2 | 11.0, 24 22.7 | 11.3; 64: 8
+// 10.6 | 11.4, 10 12.3 | 11.5; 256: 4 14.4 | 14.0; 1024: 2 27.3 | 34.2, 4 37.2 | 34.3. 64 x
+// 64, 64 states: 8 8.0 | 8.8, 10 9.4 | 8.9; 256: 4 7.5 | 9.4, 6 9.3 | 9.3; 1024: 2 14.8 | 16.1,
+// 4 18.7 | 16.2. 64 x 128, 256: 2 9.4 | 11.1, 4 11.8 | 11.2; 128 x 64, 256: 6 11.2 | 11.5, 8
+// 13.2 | 11.6; 1024: 4 22.9 | 25.6, 6 28.9 | 25.6.
 bool decay_attn_short(long longest, long states, int D, int V) {
-  const int most = D != V ? 16 : D == 128 ? 24 : 12;   // tokens, few workgroups
   const long wgs = states * (V / 16);
-  const int tenths = wgs <= 512 ? 10 : wgs <= 1024 ? 8 : wgs <= 1536 ? 6
-                     : wgs <= 2048 ? 4 : D == 64 ? 3 : V == 64 ? 6 : 4;
-  return longest * 10 <= most * tenths;
+  const int most = wgs <= 512 ? 9 : wgs <= 1024 ? 5 : wgs <= 2048 ? (D == 128 ? 4 : 3)
+                   : D == 128 ? 3 : 2;             // tokens
+  return longest <= most;
 }
 
 // Whether walk takes the place of sum and scan: its time, 3 us and 2.9 a chunk of the

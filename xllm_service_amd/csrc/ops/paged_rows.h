@@ -526,7 +526,11 @@ __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
 #pragma unroll
       for (int r = 0; r < 16; r++) mt = fmaxf(mt, s[i][r]);
     mt = pair_max(mt);
-    if (__any(mt > m)) {
+    // Some row of 32 has a new maximum in most tiles. Weights of 32 bits and sums round the
+    // same whatever they are scaled by, so there sums are scaled only where one has grown
+    // by more than 2^8: 2 of 1.5-2.6 k in a window of 1024 53.4 -> 51.4 us, 911 and 1317
+    // capped 64.5 -> 61.8, errors 1-2% smaller. (One rounded to bf16 is exact where it is 1.)
+    if (TERMS > 1 ? __any((mt - m) * c > 8.0f) : __any(mt > m)) {
       const float m_new = fmaxf(m, mt);
       const float alpha =
           __builtin_amdgcn_exp2f((m - (m_new == -INFINITY ? 0.f : m_new)) * c);

@@ -95,6 +95,18 @@ def test_prompt_routes(D, V, lens, bound):
         [i if i % 7 else -1 for i in range(n)], [0.999, 0.75, 1.0], bound, n + D + V)
 
 
+@pytest.mark.parametrize("lens,heads", [
+    ([700, 3, 129, 384], 3), ([513, 1, 640, 385], 3),   # outputs by sixteen waves
+    ([900, 640, 1100, 515, 700], 8)])                   # by four
+def test_groups_of_chunks(lens, heads):
+    """Sequences walked in up to four groups: whole and ragged last ones, fewer
+    chunks than groups, states carried or not, one without a slot."""
+    n = len(lens)
+    run(128, 128, lens, [7 * (i % 3 != 1) for i in range(n)],
+        [i if i != 2 else -1 for i in range(n)],
+        [0.999, 0.75, 1.0, 0.9999, 0.0, 0.3, 0.99, 0.996][:heads], max(lens), n)
+
+
 def test_many_chunks_and_hard_decays():
     """More chunks than the scan holds in flight; decays whose powers leave
     fp32's normal range within a chunk, and none at all."""

@@ -82,6 +82,7 @@ void launch_latent_attn_mfma(float*, float*, float*, const unsigned short*,
                              float, int, int, hipStream_t);
 long decay_attn_mfma_chunks(long, long);
 int decay_attn_mfma_chunk();
+int decay_attn_mfma_groups(long, long, int, int, int, int);
 bool decay_attn_short(long, long, int, int);
 void launch_decay_attn_mfma(float*, const unsigned short*,
                             const unsigned short*, const unsigned short*,
@@ -703,7 +704,12 @@ void decay_attn(Tensor out, Tensor q, Tensor k, Tensor v, Tensor decay,
     if (!hy::decay_attn_short(longest, (long)n_seqs * H, D, Dv) &&
         (one || n * 4 <= (1L << 31))) {
       Tensor ws;
-      if (!one) ws = torch::empty({n}, state.options());
+      if (!one) {
+        const bool groups =
+            hy::decay_attn_mfma_groups(longest, T, n_seqs, H, D, Dv) > 1;
+        ws = torch::empty({n + (groups ? (long)n_seqs * H * D * Dv : 0)},
+                          state.options());
+      }
       hy::launch_decay_attn_mfma(
           ptr<float>(out), ptr<bf>(q), ptr<bf>(k), ptr<bf>(v),
           ptr<float>(decay), ptr<float>(state), ptr<int>(slots), cu,

@@ -13,7 +13,8 @@
 //
 //   sum   what every (chunk, head) adds to the state, all chunks at once
 //   scan  chunk after chunk per state element (recurrent_chunks.h)
-//   walk  both, by workgroups that follow a sequence: many sequences of few chunks
+//   walk  both, by workgroups that follow a sequence, or one of up to four groups of its
+//         chunks: many sequences, or few chunks
 //   out   the outputs of every (chunk, head), by four waves or by sixteen
 // Batches whose sequences all fit one chunk need no scratch and no scan: out
 // reads the slots, then sum or walk moves them.
@@ -46,6 +47,21 @@ struct DMArgs {
   float* ws;                   // [chunks, heads, D, V]; null: one chunk each
   const int *slots, *cu_q, *ctx_lens;
   int n_seqs, heads;
+  int groups;                  // that walk cuts a sequence's chunks into (DMGroups)
+  long tail;                   // records of ws before the last groups' sums
+};
+
+// Where walk has more than one group to a sequence, of `size` chunks each, all but the
+// first start from nothing: what group i adds by its end lies in the record of the chunk
+// after it, which needs none of its own, the last one's in the tail. Chunk c's state
+// before it is then its record's, of its own group, and the start of that faded.
+struct DMGroups {
+  int chunks, size, count;
+  XLLM_DEV DMGroups(const DMArgs& P, int len) {
+    chunks = (len + DM_C - 1) / DM_C;
+    size = max((chunks + P.groups - 1) / P.groups, 1);
+    count = max((chunks + size - 1) / size, 1);
+  }
 };
 
 // the workgroup's sequence and tokens
@@ -110,6 +126,16 @@ XLLM_DEV float dm_pow(float a, int n) {
     b *= b;
   }
   return (float)r;
+}
+
+// a^n, rounded once, and finite: a state's zeros stay zero
+XLLM_DEV float dm_pow_far(float a, int n) {
+  double r = 1.0, b = (double)a;
+  for (; n > 0; n >>= 1) {
+    if (n & 1) r *= b;
+    b *= b;
+  }
+  return fminf((float)r, 3.4028235e38f);
 }
 
 // ---- sum: U[d][e] = sum_j a^(len-1-j) k_j[d] v_j[e] ---------------------------
@@ -246,6 +272,10 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
 // in return records go out once and never come back to be summed. Us in all, sum and scan
 // | walk: 2 prompts of 164-341 tokens, 32 heads 39.1 | 25.6, 8 of 197-471 114 | 90, 6 of
 // 449-912 154 | 126, 30 of 200-300 353 | 229; but 3 of 700-2000, 16 heads 65 | 76.
+//   Few sequences leave CUs idle and are long chains, so their chunks are cut into groups
+// that are walked side by side (DMGroups; figures at decay_attn_mfma_groups): 800 tokens of
+// 16 heads 34.7 -> 29.5 in all. Errors against 64 bits of seven such batches: 6.1e-8 -> 6.0e-8,
+// states 5.9e-8 -> 5.2e-8.
 template <int D, int V>
 __global__ void __launch_bounds__(512, 4) decay_walk_mfma_kernel(DMArgs P) {
   constexpr int ST = 64, IMG = ST * 64, BUF = 4 * IMG;     // three of keys, one of values
@@ -256,17 +286,25 @@ __global__ void __launch_bounds__(512, 4) decay_walk_mfma_kernel(DMArgs P) {
   typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f4;
   f4* swap = reinterpret_cast<f4*>(lds + 2 * BUF);         // [wave][2][lane]
   // slices of a state on one XCD: they read the same rows
-  const int sl = blockIdx.x / 8 % SL;
-  const int sh = blockIdx.x / (8 * SL) * 8 + blockIdx.x % 8;
+  const int in_group = gridDim.x / P.groups;
+  const int group = blockIdx.x / in_group, b = blockIdx.x - group * in_group;
+  const int sl = b / 8 % SL;
+  const int sh = b / (8 * SL) * 8 + b % 8;
   if (sh >= P.n_seqs * P.heads) return;
   const int s = sh / P.heads, hd = sh - s * P.heads;
   const int d0 = sl % (D / 64) * 64, e0 = sl / (D / 64) * 64;
-  const int t0 = P.cu_q[s], len = P.cu_q[s + 1] - t0;
+  const int all = P.cu_q[s + 1] - P.cu_q[s];
+  const DMGroups of(P, all);
+  if (group >= of.count) return;
+  const bool final = group == of.count - 1;
+  const int c0 = group * of.size;                          // its first chunk
+  const int t0 = P.cu_q[s] + c0 * DM_C;
+  const int len = final ? all - c0 * DM_C : of.size * DM_C;
   const int slot = P.slots[s];
-  const bool carried = slot >= 0 && P.ctx_lens[s] > 0;
+  const bool carried = group == 0 && slot >= 0 && P.ctx_lens[s] > 0;
   const int chunks = (len + DM_C - 1) / DM_C;
   const int last = len - (chunks - 1) * DM_C;              // tokens of the last one
-  long rec = 0;                                            // its first record
+  long rec = c0;                                           // its first record
   if (P.ws != nullptr)
     for (int i = 0; i < s; ++i)
       rec += (P.cu_q[i + 1] - P.cu_q[i] + DM_C - 1) / DM_C;
@@ -389,15 +427,98 @@ __global__ void __launch_bounds__(512, 4) decay_walk_mfma_kernel(DMArgs P) {
     chunk(c, kr[0], vr[0], kr[1][0], vr[1][0]);
     if (c + 1 < chunks) chunk(c + 1, kr[1], vr[1], kr[0][0], vr[0][0]);
   }
-  if (slot < 0 || (len <= 0 && carried)) return;           // nothing to keep, or as it is
+  if (!final) {
+    st = P.ws + ((rec + chunks) * P.heads + hd) * (D * V);
+  } else {
+    if (slot < 0 || (len <= 0 && carried)) return;         // nothing to keep, or as it is
+    if (group > 0) st = P.ws + ((P.tail + s) * P.heads + hd) * (D * V);
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i) st[at[i >> 2] + (i & 3) * V] = S[i];
 }
 
+// A sequence's last state, where walk had groups of it: by workgroups of `out` past its
+// heads, which nothing there waits for
+template <int D, int V, int NT>
+XLLM_DEV void dm_last_state(const DMArgs& P) {
+  const long unit = (long)(blockIdx.y - P.heads) * gridDim.x + blockIdx.x;
+  if (unit >= (long)P.n_seqs * P.heads) return;
+  const int s = (int)(unit / P.heads), hd = (int)(unit - (long)s * P.heads);
+  const int len = P.cu_q[s + 1] - P.cu_q[s], slot = P.slots[s];
+  const DMGroups of(P, len);
+  if (of.count < 2 || slot < 0) return;           // it is there
+  long rec = 0;
+  for (int i = 0; i < s; ++i)
+    rec += (P.cu_q[i + 1] - P.cu_q[i] + DM_C - 1) / DM_C;
+  const float a = P.decay[hd], by = dm_pow_far(a, of.size * DM_C);
+  const float by_last = dm_pow_far(a, len - (of.count - 1) * of.size * DM_C);
+  const long step = (long)of.size * P.heads * (D * V);
+  const float* first = P.ws + ((rec + of.size) * P.heads + hd) * (D * V);
+  const float* tail = P.ws + ((P.tail + s) * P.heads + hd) * (D * V);
+  float* to = P.state + ((long)slot * P.heads + hd) * (D * V);
+#pragma unroll 4
+  for (int i = threadIdx.x * 4; i < D * V; i += NT * 4) {
+    float S[4], x[4], y[4];
+    Quad<float>::ld(first + i, S);
+    Quad<float>::ld(tail + i, y);
+    for (int g = 1; g + 1 < of.count; ++g) {
+      Quad<float>::ld(first + g * step + i, x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[e] = fmaf(by, S[e], x[e]);
+    }
+    *reinterpret_cast<float4*>(to + i) =
+        make_float4(fmaf(by_last, S[0], y[0]), fmaf(by_last, S[1], y[1]),
+                    fmaf(by_last, S[2], y[2]), fmaf(by_last, S[3], y[3]));
+  }
+}
+// What a chunk's state before it is made of
+struct DMStart {
+  const float *own, *first;    // its record or slot, null: nothing; the first group's end
+  long step;                   // from one group's end to the next one's
+  int more;                    // groups between the first one and its own
+  float by, fade;              // over a group, and since its own began
+  template <int DV>
+  XLLM_DEV void init(const DMArgs& P, int s, int c, int hd, const float* S) {
+    const DMGroups of(P, P.cu_q[s + 1] - P.cu_q[s]);
+    const int g = c / of.size, in = c - g * of.size;
+    if (g == 0) return;
+    const float a = P.decay[hd];
+    more = g - 1;
+    step = (long)of.size * P.heads * DV;
+    first = S - (long)(c - of.size) * P.heads * DV;
+    if (in == 0) own = nullptr;
+    by = more > 0 ? dm_pow_far(a, of.size * DM_C) : 0.f;
+    fade = dm_pow_far(a, in * DM_C);
+  }
+  // x: its own 8 entries from `at` on, y: the first group's end
+  XLLM_DEV void ask(long at, float (&x)[8]) const {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = 0.f;
+    if (own == nullptr) return;                   // uniform
+    Quad<float>::ld(own + at, x);
+    Quad<float>::ld(own + at + 4, x + 4);
+  }
+  XLLM_DEV void ask_first(long at, float (&y)[8]) const {
+    Quad<float>::ld(first + at, y);
+    Quad<float>::ld(first + at + 4, y + 4);
+  }
+  XLLM_DEV void join(long at, float (&x)[8], float (&y)[8]) const {
+    for (int g = 1; g <= more; ++g) {
+      float z[8];
+      Quad<float>::ld(first + g * step + at, z);
+      Quad<float>::ld(first + g * step + at + 4, z + 4);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = fmaf(by, y[e], z[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = fmaf(fade, y[e], x[e]);
+  }
+};
+
 // ---- out ------------------------------------------------------------------------
 // A wave owns 32 queries. O^T = S^T Q^T with the state staged as three images of
 // 64 rows at a time, faded, then the tiles of 32 keys up to its own.
-template <int D, int V>
+template <int D, int V, bool GROUPS>
 __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
   constexpr int KS = D / 16, VT = V / 32;
   constexpr int KV = DM_C * (D + V), SI = 3 * 64 * V;
@@ -406,6 +527,7 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
   __shared__ float pw[DM_C + 1];
   __shared__ int lost[V];      // first token with a non-finite value, if any has
   int s, c, t0, len;
+  if (GROUPS && (int)blockIdx.y >= P.heads) return dm_last_state<D, V, 256>(P);
   if (!dm_locate(P, &s, &c, &t0, &len)) return;
   const int hd = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -424,14 +546,12 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
            ? P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V)
            : P.state + ((long)max(slot, 0) * P.heads + hd) * (D * V));
   constexpr int SN = 64 * (V / 8) / 256;
+  DMStart start = {S, nullptr, 0, 0, 0.f, 0.f};
+  if constexpr (GROUPS) start.init<D * V>(P, s, c, hd, S);
   float sr[SN][8];
   auto fetch_state = [&](int d0) {
 #pragma unroll
-    for (int i = 0; i < SN; ++i) {
-      const float* p = S + d0 * V + (tid + i * 256) * 8;
-      Quad<float>::ld(p, sr[i]);
-      Quad<float>::ld(p + 4, sr[i] + 4);
-    }
+    for (int i = 0; i < SN; ++i) start.ask(d0 * V + (tid + i * 256) * 8, sr[i]);
   };
   bf16x8 qf[KS];
   {
@@ -480,6 +600,15 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
   if (before) {
 #pragma unroll
     for (int d0 = 0; d0 < D; d0 += 64) {
+      if (start.first != nullptr) {
+        float y[SN][8];
+#pragma unroll
+        for (int i = 0; i < SN; ++i)
+          start.ask_first(d0 * V + (tid + i * 256) * 8, y[i]);
+#pragma unroll
+        for (int i = 0; i < SN; ++i)
+          start.join(d0 * V + (tid + i * 256) * 8, sr[i], y[i]);
+      }
       if (d0) __syncthreads();
 #pragma unroll
       for (int i = 0; i < SN; ++i) {
@@ -632,7 +761,7 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
 // prompts of 164-341 tokens, 32 heads, 30.3 -> 25.6 in all): all it reads comes at the rate
 // of a CU (160 KB, 2 us), then a SIMD has four waves to issue from. Beyond that nothing
 // is read while it computes, and two workgroups a CU are faster: 528 of them 31 | 36.
-template <int D, int V>
+template <int D, int V, bool GROUPS>
 __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
   constexpr int NV = V / 32, NT = 256 * NV;       // column tiles, threads
   constexpr int KS = D / 16;
@@ -648,6 +777,7 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
   float* pw = reinterpret_cast<float*>(lds + END);
   int* lost = reinterpret_cast<int*>(lds + END + 2 * (DM_C + 4));
   int s, c, t0, len;
+  if (GROUPS && (int)blockIdx.y >= P.heads) return dm_last_state<D, V, NT>(P);
   if (!dm_locate(P, &s, &c, &t0, &len) || len <= 0) return;
   const int hd = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -663,8 +793,10 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
            ? P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V)
            : P.state + ((long)max(slot, 0) * P.heads + hd) * (D * V));
   auto row_of = [&](int idx, int W) { return min(idx / (W / 8), len - 1); };
+  DMStart start = {S, nullptr, 0, 0, 0.f, 0.f};
+  if constexpr (GROUPS) start.init<D * V>(P, s, c, hd, S);
   ushort8_t qr[QP], kr[QP], vr[VP];
-  float sr[SP][8];
+  float sr[SP][8], sy[SP][8];
 #pragma unroll
   for (int i = 0; i < QP; ++i) {
     const int idx = tid + i * NT;
@@ -673,11 +805,11 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
   }
   if (before) {
 #pragma unroll
-    for (int i = 0; i < SP; ++i) {
-      const float* p = S + (tid + i * NT) * 8;
-      Quad<float>::ld(p, sr[i]);
-      Quad<float>::ld(p + 4, sr[i] + 4);
-    }
+    for (int i = 0; i < SP; ++i) start.ask((tid + i * NT) * 8, sr[i]);
+  }
+  if (start.first != nullptr) {
+#pragma unroll
+    for (int i = 0; i < SP; ++i) start.ask_first((tid + i * NT) * 8, sy[i]);
   }
 #pragma unroll
   for (int i = 0; i < QP; ++i) {
@@ -703,6 +835,7 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
 #pragma unroll
     for (int i = 0; i < SP; ++i) {
       const int idx = tid + i * NT, r = idx / (V / 8), ch = idx % (V / 8);
+      if (start.first != nullptr) start.join(idx * 8, sr[i], sy[i]);
       dm_split(sr[i], lds + KEYS + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3), IMG);
     }
   }
@@ -879,21 +1012,45 @@ bool decay_attn_short(long longest, long states, int D, int V) {
   return longest <= most;
 }
 
-// Whether walk takes the place of sum and scan: its time, 3 us and 2.9 a chunk of the
-// longest sequence, against theirs, a start and so much for each (chunk, head). Measured
+// Groups of chunks that walk, in the place of sum and scan, cuts a sequence into; 0: sum
+// and scan. Walk's time is 3 us and 2.9 a chunk of the longest sequence's groups, more with
+// two workgroups on a CU; theirs a start and so much for each (chunk, head). Measured
 // (us, both kernels' | chunks of the longest, units), 128 x 128: 15 | 3, 48; 17 | 4, 128;
 // 27 | 5, 480; 30 | 13, 528; 38 | 8, 1024; 45 | 13, 1056; 51 | 7, 1150. 64 x 128 and back:
 // 12 | 4, 68; 15 | 5, 144; 17 | 3, 192; 22 | 4, 368; 27 | 3, 496. 64 x 64: 10 | 3, 48; 12 |
 // 3, 176; 18 | 5, 448; 22 | 6, 928. One chunk each, without scan: us in all, sum | walk, 32
 // (sequence, head)s of 128 tokens 20.6 | 16.8, 64 21.9 | 19.3, 128 15.6 | 16.6, 2048 147 |
 // 188; of 64 keys 48 13.0 | 13.3.
-static bool decay_walks(long longest, long tokens, int n_seqs, int heads, int D, int V) {
-  const long chunks = (longest + DM_C - 1) / DM_C;
-  if (chunks <= 1) return D == 128 && (long)n_seqs * heads <= 96;
+//   More than one group leaves `out` more to read, a record for each group before a
+// chunk's, and the last states to make: 0.6 us and 4.5 ns a unit for each. 4 more where
+// workgroups of 16 waves, one to a CU, leave none free for those. Us in all, 128 x 128, sum
+// and scan | one group | two | three | four: 16 heads, 300 tokens 29.6 | 25.4 | 23.4 | 21.2 |
+// 21.2, 500 30.3 | 29.7 | 24.7 | 24.8 | 23.7, 800 34.7 | 39.4 | 33.3 | 31.2 | 29.5, 1200 37.0 |
+// 50.1 | 38.8 | 36.0 | 34.8, but 2000 40.5 | 72.2 | 53.6 | 48.9 | 45.7; 2 x 500-900 39.0 | 39.7 |
+// 34.7 | 34.6 | 34.5, 4 x 500-1200 60.0 | 59.2 | 56.8 | 57.7 | 60.8; 32 heads, 400 35.1 | 30.5 |
+// 27.2 | 27.3 | 28.7, but 1000 40.5 | 48.8 | 42.1 | 43.6 | 43.3.
+int decay_attn_mfma_groups(long longest, long tokens, int n_seqs, int heads, int D,
+                           int V) {
+  const long chunks = (longest + DM_C - 1) / DM_C, chains = (long)n_seqs * heads;
+  if (chunks <= 1) return D == 128 && chains <= 96;
   const long units = (2 * tokens / DM_C + n_seqs) * heads / 2;
   const long there = D + V == 256 ? 14000 + 30 * units
                      : D + V == 192 ? 9000 + 40 * units : 8500 + 18 * units;   // ns
-  return 3000 + 2900 * chunks < there;
+  const bool one = 3000 + 2900 * chunks < there;
+  if (D + V < 256) return one;
+  const long grid = decay_attn_mfma_chunks(tokens, n_seqs) * heads;
+  const long crowd = grid <= 256 && grid + chains > 256 ? 4000 : 0;
+  auto cost = [&](long g) {
+    const long wgs = 4 * chains * g;
+    const long chunk = wgs <= 256 ? 2900 : wgs <= 512 ? 2200 + wgs * 3 : wgs * 7;
+    return 3000 + (chunks + g - 1) / g * chunk +
+           (g > 1 ? crowd + (g - 1) * (600 + units * 9 / 2) : 0);
+  };
+  long best = one ? std::min(cost(1), there) : there, at = one;
+  best -= best / 8;                               // not for a little
+  for (int g = 2; g <= 4 && g <= chunks; ++g)
+    if (cost(g) < best) best = cost(g), at = g;
+  return (int)at;
 }
 
 // D, V in {64, 128}; rows 16 B aligned. ws null: no sequence has more than
@@ -906,28 +1063,35 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
                             long k_stride, long v_stride, float* ws,
                             long longest, hipStream_t st) {
   if (n_seqs == 0) return;
+  const int groups = decay_attn_mfma_groups(longest, tokens, n_seqs, heads, D, V);
+  const bool walk = groups > 0;
   const DMArgs P = {out, q, k, v, q_stride, k_stride, v_stride, decay, state,
-                    ws, slots, cu_q, ctx_lens, n_seqs, heads};
+                    ws, slots, cu_q, ctx_lens, n_seqs, heads,
+                    std::max(groups, 1),
+                    decay_attn_mfma_chunks(tokens, n_seqs)};
   const dim3 grid(
       (unsigned)(ws ? decay_attn_mfma_chunks(tokens, n_seqs) : n_seqs), heads);
+  // with those that make the last states (dm_last_state)
+  const dim3 grid_out(
+      grid.x, heads + (groups > 1 ? (n_seqs * heads + grid.x - 1) / grid.x : 0));
   const bool wide = (long)grid.x * heads <= 256;
-  const bool walk = decay_walks(longest, tokens, n_seqs, heads, D, V);
 #define DM_SUM(DD, VV)                                                        \
   hipLaunchKernelGGL((decay_sum_mfma_kernel<DD, VV>), grid, dim3(256), 0, st, P)
 #define DM_WALK(DD, VV)                                                       \
   hipLaunchKernelGGL((decay_walk_mfma_kernel<DD, VV>),                        \
                      dim3((unsigned)(((long)n_seqs * heads + 7) / 8 * 8 *     \
-                                     (DD / 64) * (VV / 64))),                 \
+                                     (DD / 64) * (VV / 64) * P.groups)),       \
                      dim3(512), 0, st, P)
-#define DM_OUT(DD, VV)                                                        \
+#define DM_OUT_(DD, VV, GROUPS)                                               \
   do {                                                                        \
     if (wide)                                                                 \
-      hipLaunchKernelGGL((decay_out_wide_kernel<DD, VV>), grid, dim3(8 * VV), \
-                         0, st, P);                                           \
+      hipLaunchKernelGGL((decay_out_wide_kernel<DD, VV, GROUPS>), grid_out,   \
+                         dim3(8 * VV), 0, st, P);                             \
     else                                                                      \
-      hipLaunchKernelGGL((decay_out_mfma_kernel<DD, VV>), grid, dim3(256), 0, \
-                         st, P);                                              \
+      hipLaunchKernelGGL((decay_out_mfma_kernel<DD, VV, GROUPS>), grid_out,   \
+                         dim3(256), 0, st, P);                                \
   } while (0)
+#define DM_OUT(DD, VV) DM_OUT_(DD, VV, false)
 #define DM_BY_SIZE(CALL)                                                      \
   do {                                                                        \
     if (D == 128) { if (V == 128) CALL(128, 128); else CALL(128, 64); }       \
@@ -948,9 +1112,11 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
                        dim3(256), 0, st, ws, state, decay, slots, cu_q, ctx_lens,
                        heads, per_head, true);
   }
-  DM_BY_SIZE(DM_OUT);
+  if (groups > 1) DM_OUT_(128, 128, true);       // the only ones with groups
+  else DM_BY_SIZE(DM_OUT);
 #undef DM_BY_SIZE
 #undef DM_OUT
+#undef DM_OUT_
 #undef DM_WALK
 #undef DM_SUM
 }

@@ -145,6 +145,15 @@ def test_prompt_edges(tail, heads, new, old, window):
             assert over.max() <= 1e-7, f"sequence {s}: off by {off.max():.3g}"
 
 
+@pytest.mark.parametrize("tail", [0, 64])
+@pytest.mark.parametrize("heads,new,old", [
+    (16, [301], [2900]), (32, [40, 6, 130], [3000, 2500, 2800]),   # parts
+    (32, [300, 221, 400, 475, 250], [200, 39, 257, 100, 0])])
+def test_prompt_tiles_of_128_rows(tail, heads, new, old):
+    """Calls that row tiles of 64 would take longer for."""
+    test_prompt_edges(tail, heads, new, old, 0)
+
+
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
 @pytest.mark.parametrize("heads,old", [(16, 0), (32, 70), (16, 1500)])
 def test_prompt_nonfinite(heads, old, bad):

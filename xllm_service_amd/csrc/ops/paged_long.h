@@ -14,10 +14,14 @@
 // v_readlane fetch from a table of 64 tiles made at once: by scalar arithmetic on the way
 // a step's loads cost 700 cycles.
 //
-// Bound by both, one after the other: 2210 cycles, the pipe 1024, the vector unit 1240 of
-// them, nearly their sum; whether barriers or reads from LDS keep them apart is not known. 4
-// prompts of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads of 128: 353 -> 335
-// us. What it costs is one workgroup per CU: nothing covers its start and its end, so it
+// Bound by the card's power: the clock falls to 1.64 GHz while calls follow each other
+// (1.84 for a single one, 2.2 to 2.4 with zeros for data), a step of two tiles a SIMD takes
+// 3430 cycles there, and schedules that take fewer run at a lower clock still or the same
+// time (all operands in registers before their products: 1660 -> 1380 cycles for a tile's 32,
+// 328 -> 333 us). What is left out counts: without exponentials 313, without three
+// quarters of the operands' reads 308, without the scaling of sums 321, and scaling them
+// only in the lanes whose maximum has grown 328 -> 325. 4 prompts of 1.6-2.3 k tokens over
+// up to 3.1 k cached ones, 32 heads of 128: 353 -> 335 -> 325 us. What it costs is one workgroup per CU: nothing covers its start and its end, so it
 // is taken for whole turns of workgroups with long chains only (paged_long_takes).
 #pragma once
 #include "paged_rows.h"
@@ -222,11 +226,9 @@ __global__ __launch_bounds__(512) void paged_attn_long_kernel(
 #pragma unroll
       for (int r = 0; r < 16; r++) mt = fmaxf(mt, s[i][r]);
     mt = pair_max(mt);
-    if (__any(mt > m)) {
-      const float m_new = fmaxf(m, mt);
-      const float alpha =
-          __builtin_amdgcn_exp2f((m - (m_new == -INFINITY ? 0.f : m_new)) * c);
-      m = m_new;
+    if (mt > m) {                                // lanes without a new one rest
+      const float alpha = __builtin_amdgcn_exp2f((m - mt) * c);
+      m = mt;
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < DT; i++)

@@ -21,9 +21,12 @@ HYB = os.path.join(ROOT, "xllm_service_amd", "csrc", "hybrid")
 # hipcc only: fp32 math compiles to scalar-lane ops (no packed fp32 forms); products
 # keep their sums in registers that other instructions read. A kernel that has a SIMD
 # for one wave got them in the other half of its registers, and its loops copied them
-# back and forth: 290 of 850 instructions of a tile in paged_short.h.
+# back and forth: 290 of 850 instructions of a tile in paged_short.h. The first 14 words of
+# a kernel's arguments come in registers: 0.2 us of a chain that begins with loads that
+# need them (prompts 12.7 -> 12.4, 10.0 -> 9.6, decode of few sequences 9.0 -> 8.8).
 HIP_FLAGS = ["-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-             "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+             "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form=1",
+             "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 ext_modules = [
     CUDAExtension(

@@ -62,6 +62,40 @@ namespace xllm {
 // Where a workgroup's rows are: tile lt of sequence seq
 struct PfPlace { int seq, lt, q_start, q_len, seq_len; };
 
+// Which of `total` units, the longest first, workgroup b takes where a CU holds two and
+// `turn` come one to a CU: what is left over joins the shortest of those, the very shortest
+// the longest of them, so that the longest have a CU to themselves. (Joined to the longest
+// of all, 500 and 695 tokens of 28/4 heads, 268 workgroups, took 24.1 us, 22.7 so.) (More
+// than two turns with the second reversed: 1318 drawn batches, no faster.)
+XLLM_DEV int pf_fold(int b, int total, int turn) {
+  const int over = total - turn;
+  if (over <= 0 || over > turn) return b;
+  return b >= turn ? turn + total - 1 - b : b < over ? turn - over + b : b - over;
+}
+
+// What there is to know of a single sequence, fetched together
+struct PfOnly {
+  int start, len, keys;
+  XLLM_DEV PfOnly(const int* cu_q, const int* seq_lens) {
+    const int end = cu_q[1];
+    start = cu_q[0];
+    keys = seq_lens[0];
+    asm volatile("" ::"s"(start), "s"(end), "s"(keys));
+    len = end - start;
+  }
+};
+// Row tile `b` of a single sequence, without scans: 0.4 us of a small call
+template <int ROWS>
+XLLM_DEV bool pf_only(int b, int turn, const int* cu_q, const int* seq_lens, int G,
+                      PfPlace* place) {
+  const PfOnly s(cu_q, seq_lens);
+  const int all = (s.len * G + ROWS - 1) / ROWS;
+  if (b >= all) return false;
+  b = pf_fold(b, all, turn);
+  *place = {0, all - 1 - b, s.start, s.len, s.keys};
+  return true;
+}
+
 // Row tile `b` of the batch; later tiles of a sequence (more keys) come first. False:
 // past the last one. One wave looks 64 sequences over at a time, and what it
 // found of the one it wants is taken from its lane: fetched again by a scalar load it
@@ -116,17 +150,6 @@ XLLM_DEV int pf_scan(int v) {
   return v;
 }
 
-// Which of `total` units, the longest first, workgroup b takes where a CU holds two and
-// `turn` come one to a CU: what is left over joins the shortest of those, the very shortest
-// the longest of them, so that the longest have a CU to themselves. (Joined to the longest
-// of all, 500 and 695 tokens of 28/4 heads, 268 workgroups, took 24.1 us, 22.7 so.) (More
-// than two turns with the second reversed: 1318 drawn batches, no faster.)
-XLLM_DEV int pf_fold(int b, int total, int turn) {
-  const int over = total - turn;
-  if (over <= 0 || over > turn) return b;
-  return b >= turn ? turn + total - 1 - b : b < over ? turn - over + b : b - over;
-}
-
 // Row tile `b` of the batch, the longest chains of keys first whatever their
 // sequences: a tile of a sequence has ROWS rows (of query and head) fewer before it
 // than the next one, so all tiles sort into levels of WIDTH of those with at most
@@ -143,13 +166,7 @@ XLLM_DEV bool pf_longest(int b, int turn, const int* cu_q, const int* seq_lens,
                          int n_seqs, int G, int lane, PfPlace* place) {
   if (n_seqs > 64)
     return pf_locate<ROWS>(b, cu_q, seq_lens, n_seqs, G, lane, place);
-  if (n_seqs == 1) {                             // without scans: 0.4 us of a small call
-    const int q0 = cu_q[0], n = cu_q[1] - q0, all = (n * G + ROWS - 1) / ROWS;
-    if (b >= all) return false;
-    b = pf_fold(b, all, turn);
-    *place = {0, all - 1 - b, q0, n, seq_lens[0]};
-    return true;
-  }
+  if (n_seqs == 1) return pf_only<ROWS>(b, turn, cu_q, seq_lens, G, place);
   int start = 0, len = 0, keys = 0;              // of sequence `lane`
   if (lane < n_seqs) {
     start = cu_q[lane];
@@ -212,16 +229,16 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, int turn,
                        int n_kv, int lane, PfPlace* at, int* part, int* parts,
                        int* first) {
   if (n_seqs == 1) {
-    const int q0 = cu_q[0], len = cu_q[1] - q0, keys = seq_lens[0];
-    const int p = paged_equal<MORE>(x, keys, PF_KT, most);
-    const int nt = (len * G + ROWS - 1) / ROWS, all = nt * p;
+    const PfOnly s(cu_q, seq_lens);
+    const int p = paged_equal<MORE>(x, s.keys, PF_KT, most);
+    const int nt = (s.len * G + ROWS - 1) / ROWS, all = nt * p;
     if (b >= all) return false;
     b = pf_fold(b, all, turn);
     const int t = b / p;                         // a division takes 0.05 us
     *part = b - t * p;
     *parts = p;
     *first = t * p;
-    *at = {0, nt - 1 - t, q0, len, keys};
+    *at = {0, nt - 1 - t, s.start, s.len, s.keys};
     return true;
   }
   int start = 0, len = 0, keys = 0, nt = 0, n = 0;
@@ -313,20 +330,21 @@ XLLM_DEV bool pf_parts(int b, int least, int most, int groups, int turn,
 // SORT: the longest chains first, where keys are not split.
 template <int D, int TERMS, bool MORE, int KG, bool SPLIT, bool SORT = true>
 __global__ __launch_bounds__(KG * 256, 2) void paged_attn_rows_kernel(
+    // (what the first loads need comes first: these are in registers)
+    const int* __restrict__ block_tables,    // [num_seqs, max_blocks]
+    const int* __restrict__ cu_q,            // [num_seqs+1] query offsets
+    const int* __restrict__ seq_lens,        // [num_seqs] total key len
+    const int n_seqs, const int G, const int n_kv, const int max_blocks,
+    const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
+    const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
+    const unsigned short* __restrict__ v_cache,
     void* __restrict__ out,                  // [total_q, n_qheads, D]
     float* __restrict__ ws_o,                // [blocks][PF_ROWS * D], a block for a part
     float* __restrict__ ws_ml,               // [blocks][PF_ROWS][2]
     int2* __restrict__ ws_at,                // [total_q*n_qheads]: first slot, parts;
                                              // of several prompts, for the merge
     const PagedMeet meet,                    // [blocks]: its first part's counts
-    const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
-    const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
-    const unsigned short* __restrict__ v_cache,
-    const int* __restrict__ block_tables,    // [num_seqs, max_blocks]
-    const int* __restrict__ cu_q,            // [num_seqs+1] query offsets
-    const int* __restrict__ seq_lens,        // [num_seqs] total key len
-    const int n_seqs, const float scale, const int G, const int n_kv,
-    const int max_blocks, const long q_stride, const long out_stride,
+    const float scale, const long q_stride, const long out_stride,
     const int least, const int most, const int turn, const PagedMore x,
     const PagedAhead ahead) {
   constexpr int KS = D / 16;                 // k steps of a score product
@@ -905,9 +923,9 @@ inline void paged_rows(void* out, float* ws_o, const unsigned short* q,
 #define PF_GO(KG, SPLIT, SORT)                                                 \
   hipLaunchKernelGGL((paged_attn_rows_kernel<D, TERMS, MORE, KG, SPLIT, SORT>),\
                      dim3((unsigned)(wgs + ahead.wgs)), dim3(KG * 256), 0,     \
-                     stream, out, ws_o, ws_ml, ws_at, meet, q, k_cache, v_cache, \
-                     block_tables, cu_q, seq_lens, n_seqs, scale, G, n_kv,     \
-                     max_blocks, q_stride, out_stride, plan.least, plan.most,  \
+                     stream, block_tables, cu_q, seq_lens, n_seqs, G, n_kv,    \
+                     max_blocks, k_cache, q, v_cache, out, ws_o, ws_ml, ws_at, \
+                     meet, scale, q_stride, out_stride, plan.least, plan.most, \
                      turn, x, ahead)
   if (plan.groups == 2 && plan.least > 0) PF_GO(2, true, true);
   else if (plan.groups == 2) PF_GO(2, false, true);

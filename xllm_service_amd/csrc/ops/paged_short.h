@@ -14,6 +14,9 @@
 // heads of 64 19.8 | 14.6, 300 of 16/4 in a window 17.3 | 13.7, capped 22.2 | 16.1. What a CU
 // pulls (61 KB/us: each wave has tiles of its own) bounds longer chains: 64 rows a wave,
 // half as much to pull, were slower (300 tokens 17, 100 behind 4000 60 | 40 for 32 rows).
+// A single sequence's chain begins with its pages and arguments at once (a kernel of its
+// own: a branch costs the others what it saves here): 300 tokens of 16/4 heads 9.9 -> 9.0,
+// 100 behind 800 of 32/8 13.8 -> 12.4, 60 behind 1000 of 28/4 15.4 -> 14.1.
 // A SIMD has one wave, whose products' sums would lie in the half of its registers that
 // only products read: with them in the other half (a flag of the build) 60 behind 500 of
 // 32/8 heads 13.1 -> 12.4, 100 behind 1000 18.0 -> 17.3, 2 x 500 of 12/12 of 64 14 -> 13.3.
@@ -26,17 +29,18 @@ namespace xllm {
 #define PS_WAVES 4
 #define PS_KEYS 2048       // that a row sees, at most
 
-template <int D, int TERMS, bool MORE>
+// ONE: there is a single sequence
+template <int D, int TERMS, bool MORE, bool ONE>
 __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
-    void* __restrict__ out,                  // [total_q, n_qheads, D]
-    const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
-    const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
-    const unsigned short* __restrict__ v_cache,
     const int* __restrict__ block_tables,    // [num_seqs, max_blocks]
     const int* __restrict__ cu_q,            // [num_seqs+1] query offsets
     const int* __restrict__ seq_lens,        // [num_seqs] total key len
-    const int n_seqs, const float scale, const int G, const int n_kv,
-    const int max_blocks, const long q_stride, const long out_stride,
+    const int n_seqs, const int G, const int n_kv, const int max_blocks,
+    const unsigned short* __restrict__ k_cache,  // [blocks, n_kv, 16, D]
+    const unsigned short* __restrict__ q,    // [total_q, n_qheads, D] bf16
+    const unsigned short* __restrict__ v_cache,
+    void* __restrict__ out,                  // [total_q, n_qheads, D]
+    const float scale, const long q_stride, const long out_stride,
     const PagedMore x, const PagedAhead ahead) {
   constexpr int KS = D / 16;                 // k steps of a score product
   constexpr int DT = D / 32;                 // 32-wide tiles of the head
@@ -54,14 +58,26 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, c32 = lane & 31;
 
+  // Of a single sequence the pages of the wave's 16 tiles are asked for before its length
+  // is known: what lies past the last one is not used. The arguments come together, as the
+  // compiler would not ask for them: each wait for some of them is 0.2 us. (Several
+  // sequences' first pages, a sequence to a lane, delay the search: 3 x 40-120 behind
+  // 100-500 of 16/4 heads 10.0 -> 10.2.)
+  const int tile = wid + PS_WAVES * (lane / PAGES);   // of this lane's page
+  const bool early = ONE && (!MORE || x.window <= 0);
+  int id = 0;
+  if (early) id = block_tables[min(tile * PAGES + lane % PAGES, max_blocks - 1)];
   if (!MORE && (int)blockIdx.x >= ahead.from) {
     paged_fetch(ahead, blockIdx.x - ahead.from, kv_lds);
     return;
   }
+  if constexpr (ONE)
+    asm volatile("" ::"s"(q), "s"(k_cache), "s"(v_cache), "s"(q_stride), "s"(scale));
   const int kvh = blockIdx.x % n_kv;
   PfPlace place;
-  if (!pf_locate<PS_ROWS>(blockIdx.x / n_kv, cu_q, seq_lens, n_seqs, G, lane,
-                          &place))
+  if (ONE ? !pf_only<PS_ROWS>(blockIdx.x / n_kv, INT_MAX / 2, cu_q, seq_lens, G, &place)
+          : !pf_locate<PS_ROWS>(blockIdx.x / n_kv, cu_q, seq_lens, n_seqs, G, lane,
+                                &place))
     return;
   const int q_start = place.q_start, q_len = place.q_len,
             seq_len = place.seq_len;
@@ -117,13 +133,12 @@ __global__ __launch_bounds__(PS_WAVES * 64) void paged_attn_short_kernel(
   static_assert((PS_KEYS / PF_KT / PS_WAVES + 2) * PAGES <= 64, "pages per lane");
   unsigned at_lo = 0, at_hi = 0, bytes = 0;
   auto look_up = [&]() {
-    const int i = wid + PS_WAVES * (lane / PAGES);
-    const int pg = list.at(min(i, n - 1)) * PAGES + lane % PAGES;
-    const long at =
-        ((long)btab[min(pg, last_blk)] * n_kv + kvh) * (PF_BS * D * 2);
+    const int pg = list.at(min(tile, n - 1)) * PAGES + lane % PAGES;
+    if (!early) id = btab[min(pg, last_blk)];
+    const long at = ((long)id * n_kv + kvh) * (PF_BS * D * 2);
     at_lo = (unsigned)at;
     at_hi = (unsigned)(at >> 32);
-    bytes = i < n ? min(max(seq_len - pg * PF_BS, 0), PF_BS) * (D * 2) : 0;
+    bytes = tile < n ? min(max(seq_len - pg * PF_BS, 0), PF_BS) * (D * 2) : 0;
     asm volatile("" : "+v"(at_lo), "+v"(at_hi), "+v"(bytes));   // waited for here
   };
   unsigned short* kv = kv_lds + wid * (2 * TILE);
@@ -315,13 +330,14 @@ inline void paged_short(void* out, const unsigned short* q,
                         const PagedMore& x, const PagedAhead& ahead,
                         hipStream_t stream) {
   const int G = n_qheads / n_kv;
+  auto go = n_seqs == 1 ? paged_attn_short_kernel<D, TERMS, MORE, true>
+                        : paged_attn_short_kernel<D, TERMS, MORE, false>;
   hipLaunchKernelGGL(
-      (paged_attn_short_kernel<D, TERMS, MORE>),
+      go,
       dim3((unsigned)(paged_rows_tiles<PS_ROWS>(tokens, n_seqs, G) * n_kv +
                       ahead.wgs)),
-      dim3(PS_WAVES * 64), 0, stream, out, q, k_cache, v_cache, block_tables,
-      cu_q, seq_lens, n_seqs, scale, G, n_kv, max_blocks, q_stride, out_stride, x,
-      ahead);
+      dim3(PS_WAVES * 64), 0, stream, block_tables, cu_q, seq_lens, n_seqs, G, n_kv,
+      max_blocks, k_cache, q, v_cache, out, scale, q_stride, out_stride, x, ahead);
 }
 
 // How a batch of prompts is run: by this kernel, or by paged_rows.h. max_blocks: pages

@@ -664,6 +664,14 @@ def test_prefill_orders_and_groups(kv_heads, per, dim, lens, ctx, sign):
     test_prefill_few_rows(kv_heads, per, dim, lens, ctx, sign)
 
 
+@pytest.mark.parametrize("kv_heads,per,dim", [(3, 3, 128), (5, 5, 64), (7, 6, 128),
+                                               (1, 11, 64), (2, 25, 128), (1, 71, 64)])
+def test_prefill_heads_of_no_power_of_two(kv_heads, per, dim):
+    """Rows and workgroups are divided by head counts with a multiplication."""
+    test_prefill_few_rows(kv_heads, per, dim, [257, 1, 0, 130, 333], [40, 700, 5, 0, 90],
+                          1.0)
+
+
 @pytest.mark.parametrize("kv_heads,per,dim,lens,ctx,sign", [
     (8, 4, 128, [200, 90, 333, 1, 150, 0, 257] * 3, [7, 60, 5] * 7, 1.0),   # over three
     (8, 4, 128, [200, 90, 333, 1, 150, 0, 257] * 2, [7, 60, 5, 9] * 3 + [3, 0], -1.0),

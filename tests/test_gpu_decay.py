@@ -210,3 +210,37 @@ def test_short_batches(heads, D, V):
     for n in (1, 3, 9, 12, 13, 16, 17, 24, 25):
         run(D, V, [n, max(1, n // 2), n], [0, 5, 3], [1, -1, 0],
             [0.75 + 0.24 * h / heads for h in range(heads)], n, n)
+
+
+@pytest.mark.parametrize("heads,D,V,lens", [
+    (16, 128, 128, [128, 1, 15, 16, 17, 33, 127]),    # tiles of 16 and 32 tokens
+    (24, 128, 128, [63, 64, 65, 96, 97, 8] * 2),      # beyond a workgroup for each CU
+    (40, 64, 64, [128, 31, 5, 112, 2, 64]), (43, 64, 64, [128, 31, 5, 112, 2, 64]),
+    (60, 64, 128, [32, 3, 20, 7, 16] * 2), (60, 64, 128, [33, 3, 20, 7, 128] * 2),
+    (64, 128, 64, [33, 128, 9, 50, 16, 100, 65]), (65, 128, 64, [33, 128, 9, 50, 16, 100, 65]),
+])
+def test_one_chunk_each(heads, D, V, lens):
+    """States moved by the workgroups of the outputs, or after them, on both sides of the
+    lines between; some states not kept, some carried."""
+    n = len(lens)
+    run(D, V, lens, [i % 3 * 4 for i in range(n)],
+        [-1 if i % 5 == 3 else i for i in range(n)],
+        [0.75 + 0.249 * h / heads for h in range(heads)], max(lens), n + heads)
+
+
+@pytest.mark.parametrize("tokens", [100, 200])        # a chunk; two
+def test_states_of_values_that_are_not_finite(tokens):
+    """One chunk or more: a value that is not finite ends up in its column alone."""
+    g = torch.Generator().manual_seed(5)
+    rows = torch.randn(tokens, 3 * 128, generator=g).to(torch.bfloat16)
+    rows[7, 256 + 40] = float("inf")
+    rows[90, 256 + 41] = float("nan")
+    rows = rows.cuda()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    state = torch.zeros(1, 1, 128, 128, device="cuda")
+    out = torch.zeros(tokens, 1, 128, device="cuda")
+    H.decay_attn(*rows.chunk(3, 1), torch.full((1,), 0.97, device="cuda"), state,
+                 torch.zeros(1, **i32), torch.tensor([0, tokens], **i32),
+                 torch.zeros(1, **i32), out, max_q_len=tokens)
+    odd = ~torch.isfinite(state[0, 0]).cpu()
+    assert odd[:, 40:42].all() and not odd[:, :40].any() and not odd[:, 42:].any()

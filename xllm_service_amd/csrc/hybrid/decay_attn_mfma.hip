@@ -17,7 +17,7 @@
 //         chunks: many sequences, or few chunks
 //   out   the outputs of every (chunk, head), by four waves or by sixteen
 // Batches whose sequences all fit one chunk need no scratch and no scan: out
-// reads the slots, then sum or walk moves them.
+// reads the slots and moves them too, or sum does afterwards.
 //
 // Chunks of 128 tokens halve the scratch traffic of 64 (a record is a whole
 // state per head), and the products within a chunk they add are cheap.
@@ -305,9 +305,8 @@ __global__ void __launch_bounds__(512, 4) decay_walk_mfma_kernel(DMArgs P) {
   const int chunks = (len + DM_C - 1) / DM_C;
   const int last = len - (chunks - 1) * DM_C;              // tokens of the last one
   long rec = c0;                                           // its first record
-  if (P.ws != nullptr)
-    for (int i = 0; i < s; ++i)
-      rec += (P.cu_q[i + 1] - P.cu_q[i] + DM_C - 1) / DM_C;
+  for (int i = 0; i < s; ++i)
+    rec += (P.cu_q[i + 1] - P.cu_q[i] + DM_C - 1) / DM_C;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, n = lane & 31;
@@ -406,7 +405,7 @@ __global__ void __launch_bounds__(512, 4) decay_walk_mfma_kernel(DMArgs P) {
     }
     __syncthreads();
     float* to = P.ws + ((rec + c) * P.heads + hd) * (D * V);
-    const bool store = P.ws != nullptr && (c > 0 || carried);
+    const bool store = c > 0 || carried;
     const float by = c == chunks - 1 ? keep_last : keep;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -761,37 +760,46 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
 // prompts of 164-341 tokens, 32 heads, 30.3 -> 25.6 in all): all it reads comes at the rate
 // of a CU (160 KB, 2 us), then a SIMD has four waves to issue from. Beyond that nothing
 // is read while it computes, and two workgroups a CU are faster: 528 of them 31 | 36.
-template <int D, int V, bool GROUPS>
+//   LAST: each sequence is one chunk, whose workgroup then moves its state too: the keys lie
+// in LDS, are weighted and split in place of queries, keys and weights, and a wave has 32 x
+// 32 of the state. A kernel of its own would start over, fetch and activate again; figures
+// at decay_attn_one.
+template <int D, int V, bool GROUPS, bool LAST>
 __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
   constexpr int NV = V / 32, NT = 256 * NV;       // column tiles, threads
   constexpr int KS = D / 16;
   constexpr int QP = DM_C * D / 8 / NT, VP = DM_C * V / 8 / NT;   // pieces of a thread
   constexpr int SP = D * V / 8 / NT;
-  // queries | state, then keys, values, weights | powers, first lost token of a column
-  constexpr int IMG = D * V, KEYS = DM_C * D, VALS = KEYS + DM_C * D,
-                WGTS = VALS + DM_C * V, TILE = 3 * 2 * 64 * 8;
-  constexpr int END = (KEYS + 3 * IMG > WGTS + 10 * TILE ? KEYS + 3 * IMG
-                                                         : WGTS + 10 * TILE);
+  // queries | state, then keys, weights, values | powers, first lost token of a column
+  constexpr int IMG = D * V, KEYS = DM_C * D, WGTS = KEYS + DM_C * D,
+                TILE = 3 * 2 * 64 * 8, VALS = WGTS + 10 * TILE;
+  constexpr int END = (KEYS + 3 * IMG > VALS + DM_C * V ? KEYS + 3 * IMG
+                                                        : VALS + DM_C * V);
   __shared__ __attribute__((aligned(1024))) unsigned short
       lds[END + 2 * (DM_C + 4) + 2 * V];
   float* pw = reinterpret_cast<float*>(lds + END);
   int* lost = reinterpret_cast<int*>(lds + END + 2 * (DM_C + 4));
   int s, c, t0, len;
   if (GROUPS && (int)blockIdx.y >= P.heads) return dm_last_state<D, V, NT>(P);
-  if (!dm_locate(P, &s, &c, &t0, &len) || len <= 0) return;
+  if (!dm_locate(P, &s, &c, &t0, &len)) return;
   const int hd = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63;
+  const int slot = P.slots[s];
+  const bool carried = slot >= 0 && P.ctx_lens[s] > 0;
+  float* kept = P.state + ((long)max(slot, 0) * P.heads + hd) * (D * V);
+  if (len <= 0) {
+    if (LAST && slot >= 0 && !carried)            // a new state, of no tokens
+      for (int i = tid * 4; i < D * V; i += NT * 4)
+        *reinterpret_cast<float4*>(kept + i) = make_float4(0.f, 0.f, 0.f, 0.f);
+    return;
+  }
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   // a SIMD's waves have different queries: later ones meet more keys
   const int vt = w >> 2, qt = (w + vt) & 3;
   const int h = lane >> 5, n = lane & 31;
-  const int slot = P.slots[s];
-  const bool carried = slot >= 0 && P.ctx_lens[s] > 0;
   const bool before = c > 0 || carried;           // uniform
-  const float* S =
-      (P.ws != nullptr
-           ? P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V)
-           : P.state + ((long)max(slot, 0) * P.heads + hd) * (D * V));
+  const float* S = (P.ws != nullptr
+                        ? P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V) : kept);
   auto row_of = [&](int idx, int W) { return min(idx / (W / 8), len - 1); };
   DMStart start = {S, nullptr, 0, 0, 0.f, 0.f};
   if constexpr (GROUPS) start.init<D * V>(P, s, c, hd, S);
@@ -959,34 +967,94 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
     }
   }
   __syncthreads();
-  if (!on) return;
-  for (int kt = 0; kt <= qt; ++kt) {
-    f32x16 y = mr_zero();
+  auto outputs = [&] {
+    for (int kt = 0; kt <= qt; ++kt) {
+      f32x16 y = mr_zero();
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      const bf16x8 x =
-          mr_cols<V>((const lds_u16*)vs + vbase + (kt * 32 + st * 16) * V);
+      for (int st = 0; st < 2; ++st) {
+        const bf16x8 x =
+            mr_cols<V>((const lds_u16*)vs + vbase + (kt * 32 + st * 16) * V);
 #pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        const bf16x8 p = wt[(kt * 6 + t * 2 + st) * 64];
-        if (t == 0) y = mr_mma(x, p, y);
-        else acc[1] = mr_mma(x, p, acc[1]);
+        for (int t = 0; t < 3; ++t) {
+          const bf16x8 p = wt[(kt * 6 + t * 2 + st) * 64];
+          if (t == 0) y = mr_mma(x, p, y);
+          else acc[1] = mr_mma(x, p, acc[1]);
+        }
       }
+      acc[0] += y;
     }
-    acc[0] += y;
-  }
-  if (qi >= len) return;
-  if (any_lost) {
+    if (qi >= len) return;
+    if (any_lost) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (lost[vt * 32 + 8 * (r >> 2) + 4 * h + (r & 3)] <= qi) acc[0][r] = NAN;
+    }
+    float* o = P.out + ((long)(t0 + qi) * P.heads + hd) * V + vt * 32 + 4 * h;
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *reinterpret_cast<float4*>(o + 2 * r) =
+          make_float4(acc[0][r] + acc[1][r], acc[0][r + 1] + acc[1][r + 1],
+                      acc[0][r + 2] + acc[1][r + 2], acc[0][r + 3] + acc[1][r + 3]);
+  };
+  if (on) outputs();
+  if constexpr (LAST) {
+    if (slot < 0) return;                         // uniform
+    // ---- the state: this wave's 32 keys' columns (dt) by 32 values' -------------
+    const int dt = w & 3;
+    const bool mine = dt < D / 32;
+    float* st = kept + (long)(dt * 32 + 4 * h) * V + vt * 32 + n;
+    float x0[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-      if (lost[vt * 32 + 8 * (r >> 2) + 4 * h + (r & 3)] <= qi) acc[0][r] = NAN;
-  }
-  float* o = P.out + ((long)(t0 + qi) * P.heads + hd) * V + vt * 32 + 4 * h;
+      x0[r] = carried && mine ? st[(8 * (r >> 2) + (r & 3)) * V] : 0.f;
+    __syncthreads();                              // weights and values are read
+    // a row's pieces are a wave's, which has read them all when it writes the first
 #pragma unroll
-  for (int r = 0; r < 16; r += 4)
-    *reinterpret_cast<float4*>(o + 2 * r) =
-        make_float4(acc[0][r] + acc[1][r], acc[0][r + 1] + acc[1][r + 1],
-                    acc[0][r + 2] + acc[1][r + 2], acc[0][r + 3] + acc[1][r + 3]);
+    for (int i = 0; i < QP; ++i) {
+      const int idx = tid + i * NT, r = idx / (D / 8), ch = idx % (D / 8);
+      const dm_u4 z = *reinterpret_cast<const dm_u4*>(
+          lds + KEYS + r * D + ((ch ^ mr_swz_rows<D>(r)) << 3));
+      float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (r < len) {
+        const float wgt = pw[len - 1 - r];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          x[2 * j] = __uint_as_float(z.x[j] << 16) * wgt;
+          x[2 * j + 1] = __uint_as_float(z.x[j] & 0xffff0000u) * wgt;
+        }
+      }
+      dm_split(x, lds + r * D + ((ch ^ mr_swz_cols<D>(r)) << 3), DM_C * D);
+    }
+    if (any_lost) {                               // values as they were
+      for (int i = tid; i < DM_C * V / 8; i += NT) {
+        const int r = i / (V / 8), ch = i % (V / 8);
+        dm_u4 y = {{0u, 0u, 0u, 0u}};
+        if (r < len)
+          y = dm_act(dm_row(P.v + (long)(t0 + r) * P.v_stride + hd * V + ch * 8));
+        *reinterpret_cast<dm_u4*>(vs + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3)) = y;
+      }
+    }
+    __syncthreads();
+    if (!mine) return;
+    const int cbase = mr_col_base<D>(lane) ^ (dt << 5);
+    acc[0] = acc[1] = mr_zero();
+    // leading and other terms apart. The last tokens weigh most and come last: one chain
+    // of leading products is no less precise than sums of some of them.
+#pragma unroll 4
+    for (int k = 0; k < len; k += 16) {
+      const bf16x8 y = mr_cols<V>((const lds_u16*)vs + vbase + k * V);
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        acc[t > 0] = mr_mma(mr_cols<D>((const lds_u16*)lds + t * DM_C * D + k * D + cbase),
+                            y, acc[t > 0]);
+    }
+    const float by = pw[len];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float u = acc[0][r] + acc[1][r];
+      st[(8 * (r >> 2) + (r & 3)) * V] = carried ? fmaf(by, x0[r], u) : u;
+    }
+  }
 }
 
 // records of scratch for a batch of prompt rows
@@ -999,16 +1067,20 @@ int decay_attn_mfma_chunk() { return DM_C; }
 // nearly as much as one of 32 (both passes move the whole state through LDS), where
 // the recurrence of decay_attn.hip walks token by token, one workgroup per 16
 // columns of a state, whose rate falls once they fill the chip. Measured (us, the
-// recurrence | here, tokens), fresh sequences; continued ones meet one or two tokens later.
-// 128 x 128, 16 states: 8 9.7 | 10.8, 10 11.3 | 10.9, 16 16.2 | 11.0, 24 22.7 | 11.3; 64: 8
-// 10.6 | 11.4, 10 12.3 | 11.5; 256: 4 14.4 | 14.0; 1024: 2 27.3 | 34.2, 4 37.2 | 34.3. 64 x
-// 64, 64 states: 8 8.0 | 8.8, 10 9.4 | 8.9; 256: 4 7.5 | 9.4, 6 9.3 | 9.3; 1024: 2 14.8 | 16.1,
-// 4 18.7 | 16.2. 64 x 128, 256: 2 9.4 | 11.1, 4 11.8 | 11.2; 128 x 64, 256: 6 11.2 | 11.5, 8
-// 13.2 | 11.6; 1024: 4 22.9 | 25.6, 6 28.9 | 25.6.
+// recurrence | here, tokens), fresh, continued: 128 x 128, 16 states: 6 8.1 9.0 | 7.9 10.3, 8
+// 9.7 10.6 | 8.6 10.2; 64: 5 8.8 9.5 | 8.5 10.8, 7 10.2 11.1 | 8.6 10.7; 128: 5 10.4 12.4 |
+// 9.4 11.6; 256: 4 14.8 19.0 | 10.7 14.7; fresh ones, 1024: 2 27.3 | 34.2, 4 37.2 | 34.3. 64 x
+// 64, 64 states: 6 7.5 7.7 | 7.3 7.5; 256: 4 7.6 9.1 | 7.4 8.1, 5 8.8 10.0 | 7.6 8.0; 1024: 2
+// 15.3 | 16.7, 3 17.2 | 16.8. 64 x 128, 256: 4 11.9 14.8 | 8.4 9.5; 128 x 64, 256: 4 9.2 10.9 |
+// 9.0 10.9, 6 11.3 13.1 | 9.0 11.0; 1024: 4 22.9 | 25.6, 6 28.9 | 25.6. Two to four tokens of
+// a fresh state stay with the recurrence where it was the faster one before out moved the
+// states itself: they are 2.5-3.5e-8 off 64 bits there, 3.0-3.7e-8 here; of 5 tokens 3.9 |
+// 3.8e-8, of 7 4.4 | 4.0e-8.
 bool decay_attn_short(long longest, long states, int D, int V) {
   const long wgs = states * (V / 16);
-  const int most = wgs <= 512 ? 9 : wgs <= 1024 ? 5 : wgs <= 2048 ? (D == 128 ? 4 : 3)
-                   : D == 128 ? 3 : 2;             // tokens
+  const int most = wgs <= 128 ? 7 : wgs <= 512 ? 6                    // tokens
+                   : wgs <= 2048 ? (D == 128 || wgs <= 1024 ? 4 : 3)
+                   : D == 128 ? 3 : 2;
   return longest <= most;
 }
 
@@ -1018,9 +1090,7 @@ bool decay_attn_short(long longest, long states, int D, int V) {
 // (us, both kernels' | chunks of the longest, units), 128 x 128: 15 | 3, 48; 17 | 4, 128;
 // 27 | 5, 480; 30 | 13, 528; 38 | 8, 1024; 45 | 13, 1056; 51 | 7, 1150. 64 x 128 and back:
 // 12 | 4, 68; 15 | 5, 144; 17 | 3, 192; 22 | 4, 368; 27 | 3, 496. 64 x 64: 10 | 3, 48; 12 |
-// 3, 176; 18 | 5, 448; 22 | 6, 928. One chunk each, without scan: us in all, sum | walk, 32
-// (sequence, head)s of 128 tokens 20.6 | 16.8, 64 21.9 | 19.3, 128 15.6 | 16.6, 2048 147 |
-// 188; of 64 keys 48 13.0 | 13.3.
+// 3, 176; 18 | 5, 448; 22 | 6, 928.
 //   More than one group leaves `out` more to read, a record for each group before a
 // chunk's, and the last states to make: 0.6 us and 4.5 ns a unit for each. 4 more where
 // workgroups of 16 waves, one to a CU, leave none free for those. Us in all, 128 x 128, sum
@@ -1032,7 +1102,7 @@ bool decay_attn_short(long longest, long states, int D, int V) {
 int decay_attn_mfma_groups(long longest, long tokens, int n_seqs, int heads, int D,
                            int V) {
   const long chunks = (longest + DM_C - 1) / DM_C, chains = (long)n_seqs * heads;
-  if (chunks <= 1) return D == 128 && chains <= 96;
+  if (chunks <= 1) return 0;
   const long units = (2 * tokens / DM_C + n_seqs) * heads / 2;
   const long there = D + V == 256 ? 14000 + 30 * units
                      : D + V == 192 ? 9000 + 40 * units : 8500 + 18 * units;   // ns
@@ -1051,6 +1121,21 @@ int decay_attn_mfma_groups(long longest, long tokens, int n_seqs, int heads, int
   for (int g = 2; g <= 4 && g <= chunks; ++g)
     if (cost(g) < best) best = cost(g), at = g;
   return (int)at;
+}
+
+// Whether out moves the states of sequences of a chunk each, in workgroups of 16 or 8
+// waves. Instead: out by four waves (beyond 256 states) and sum. Measured (us, two kernels |
+// one; fresh, continued; states), 128 x 128: 64 tokens 64 17.8 28.1 | 11.0 13.8, 272 26.5
+// 33.8 | 23.2 29.7, 1024 59.4 81.2 | 53.4 76.8, 4096 207 293 | 184 255, 20 tokens 272 19.2
+// 24.8 | 17.9 24.1, 4096 142 230 | 141 191. 64 x 128: 128 tokens 280 29.4 33.6 | 27.8 31.9,
+// 4096 241 292 | 223 268, 40 tokens 800 32.7 42.3 | 31.9 39.5, 20 tokens 1024 27.4 38.0 | 28.0
+// 35.2, 4096 93 136 | 104 131. 128 x 64: 128 tokens 280 30.7 34.1 | 27.8 33.1, 448 33.5 38.4 |
+// 30.3 36.7, 520 42.8 49.7 | 41.3 49.7, 20 tokens 320 15.8 18.5 | 16.0 19.6. 64 x 64: 128
+// tokens 256 18.0 20.7 | 13.1 15.6, 320 22.2 24.4 | 22.0 24.8, 768 32.4 36.9 | 34.3 39.4.
+static bool decay_attn_one(long longest, long states, int D, int V) {
+  if (states <= 256 || (D == 128 && V == 128)) return true;
+  if (V == 128) return states <= 512 || longest > 32;
+  return D == 128 && states <= 448 && longest > 32;
 }
 
 // D, V in {64, 128}; rows 16 B aligned. ws null: no sequence has more than
@@ -1082,11 +1167,13 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
                      dim3((unsigned)(((long)n_seqs * heads + 7) / 8 * 8 *     \
                                      (DD / 64) * (VV / 64) * P.groups)),       \
                      dim3(512), 0, st, P)
+#define DM_WIDE(DD, VV, GROUPS, LAST)                                         \
+  hipLaunchKernelGGL((decay_out_wide_kernel<DD, VV, GROUPS, LAST>), grid_out, \
+                     dim3(8 * VV), 0, st, P)
 #define DM_OUT_(DD, VV, GROUPS)                                               \
   do {                                                                        \
     if (wide)                                                                 \
-      hipLaunchKernelGGL((decay_out_wide_kernel<DD, VV, GROUPS>), grid_out,   \
-                         dim3(8 * VV), 0, st, P);                             \
+      DM_WIDE(DD, VV, GROUPS, false);                                         \
     else                                                                      \
       hipLaunchKernelGGL((decay_out_mfma_kernel<DD, VV, GROUPS>), grid_out,   \
                          dim3(256), 0, st, P);                                \
@@ -1097,9 +1184,14 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
     if (D == 128) { if (V == 128) CALL(128, 128); else CALL(128, 64); }       \
     else { if (V == 128) CALL(64, 128); else CALL(64, 64); }                  \
   } while (0)
-  if (ws == nullptr) {
-    DM_BY_SIZE(DM_OUT);
-    if (walk) DM_BY_SIZE(DM_WALK); else DM_BY_SIZE(DM_SUM);
+#define DM_ALL(DD, VV) DM_WIDE(DD, VV, false, true)
+  if (ws == nullptr) {                            // a chunk each
+    if (decay_attn_one(longest, (long)n_seqs * heads, D, V)) {
+      DM_BY_SIZE(DM_ALL);
+    } else {
+      DM_BY_SIZE(DM_OUT);
+      DM_BY_SIZE(DM_SUM);
+    }
     return;
   }
   if (walk) {
@@ -1116,6 +1208,8 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
   else DM_BY_SIZE(DM_OUT);
 #undef DM_BY_SIZE
 #undef DM_OUT
+#undef DM_ALL
+#undef DM_WIDE
 #undef DM_OUT_
 #undef DM_WALK
 #undef DM_SUM

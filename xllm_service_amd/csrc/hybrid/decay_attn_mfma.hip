@@ -1092,7 +1092,9 @@ bool decay_attn_short(long longest, long states, int D, int V) {
 // 12 | 4, 68; 15 | 5, 144; 17 | 3, 192; 22 | 4, 368; 27 | 3, 496. 64 x 64: 10 | 3, 48; 12 |
 // 3, 176; 18 | 5, 448; 22 | 6, 928.
 //   More than one group leaves `out` more to read, a record for each group before a
-// chunk's, and the last states to make: 0.6 us and 4.5 ns a unit for each. 4 more where
+// chunk's, and the last states to make: 0.6 us and 4.5 ns a unit for each, 9 ns by four
+// waves, which have no registers left for it (1200, 1300 and 1323 tokens of 16 heads: 66.0
+// by sum and scan, 71.8 | 72.1 | 73.3 by groups; 2 of 1000, 32 heads, 69.9 | 71.1). 4 more where
 // workgroups of 16 waves, one to a CU, leave none free for those. Us in all, 128 x 128, sum
 // and scan | one group | two | three | four: 16 heads, 300 tokens 29.6 | 25.4 | 23.4 | 21.2 |
 // 21.2, 500 30.3 | 29.7 | 24.7 | 24.8 | 23.7, 800 34.7 | 39.4 | 33.3 | 31.2 | 29.5, 1200 37.0 |
@@ -1106,18 +1108,18 @@ int decay_attn_mfma_groups(long longest, long tokens, int n_seqs, int heads, int
   const long units = (2 * tokens / DM_C + n_seqs) * heads / 2;
   const long there = D + V == 256 ? 14000 + 30 * units
                      : D + V == 192 ? 9000 + 40 * units : 8500 + 18 * units;   // ns
-  const bool one = 3000 + 2900 * chunks < there;
-  if (D + V < 256) return one;
+  if (D + V < 256) return 3000 + 2900 * chunks < there;
   const long grid = decay_attn_mfma_chunks(tokens, n_seqs) * heads;
   const long crowd = grid <= 256 && grid + chains > 256 ? 4000 : 0;
   auto cost = [&](long g) {
     const long wgs = 4 * chains * g;
     const long chunk = wgs <= 256 ? 2900 : wgs <= 512 ? 2200 + wgs * 3 : wgs * 7;
     return 3000 + (chunks + g - 1) / g * chunk +
-           (g > 1 ? crowd + (g - 1) * (600 + units * 9 / 2) : 0);
+           (g > 1 ? crowd + (g - 1) * (600 + units * (grid <= 256 ? 9 : 18) / 2) : 0);
   };
-  long best = one ? std::min(cost(1), there) : there, at = one;
-  best -= best / 8;                               // not for a little
+  // not for a little: 5 of 365 to 850 tokens 60.7 by sum and scan, 63.2 by one group
+  long at = cost(1) < there - there / 16, best = at ? cost(1) : there;
+  best -= best / 8;
   for (int g = 2; g <= 4 && g <= chunks; ++g)
     if (cost(g) < best) best = cost(g), at = g;
   return (int)at;

@@ -29,9 +29,10 @@
 // Measured, us, before | here: 16 heads, rows of 576, 1800 and 2200 tokens 1002 | 229 (1090
 // TFLOP/s executed), 1000 tokens 247 | 75, 434 and 45 behind 5000 1244 | 128 (parts), by
 // four waves 256 tokens 68 | 24, 16 25 | 9.2 (two waves 33 and 13.6); 32 heads, rows of 512 in
-// a window of 1024, 3077 and 63 560 | 161. A tile takes about 7000 cycles of a CU for products of 4750. Of a wave's, steps of K asked for as they
-// were needed took 900 more, and loads at the start of a tile 1000: their instructions
-// queue. Error against 64 bits, the first three: 3.6e-7 | 3.0e-7, 3.3 | 2.1, 7.0 | 2.5.
+// a window of 1024, 3077 and 63 560 | 161. A tile takes about 7000 cycles of a CU for
+// products of 4750. Of a wave's, steps of K asked for as they were needed took 900 more, and
+// loads at the start of a tile 1000: their instructions queue. Error against 64 bits,
+// the first three: 3.6e-7 | 3.0e-7, 3.3 | 2.1, 7.0 | 2.5.
 //
 // LDS image: rows 1152 B apart (those of 512 entries too), 16 B chunk c of row k at
 // c ^ lr_swz(k). Rows alternate between the halves of the banks; with that the 16 rows of

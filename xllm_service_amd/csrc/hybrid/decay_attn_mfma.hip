@@ -37,6 +37,7 @@ namespace xllm {
 namespace hyb {
 
 constexpr int DM_C = 128;      // tokens per chunk
+constexpr int DM_LATE = 4;     // ... at most that join the state one by one
 
 struct DMArgs {
   float* out;                  // [T, heads, V]
@@ -138,15 +139,69 @@ XLLM_DEV float dm_pow_far(float a, int n) {
   return fminf((float)r, 3.4028235e38f);
 }
 
+// A state's last tokens. They weigh most, and the matrix pipe cuts off what the products
+// of 16 tokens have below the last bit of the largest. So some of them are left out of its
+// sums (their weights are zero) and join one by one with a rounding each, as in the
+// recurrence: all of up to four, else two below a decay of 3/4 and one below 0.9. Errors
+// of states against 64 bits, 1e-8, fresh ones, without that | with it | the recurrence:
+// heads of 0.75 to 0.996, 3 tokens 3.3 | 3.1 | 3.1, 6 3.8 | 3.8 | 4.4; of 0.3 to 0.7, 6
+// tokens 3.8 | 3.0 | 3.0, 16 4.8 | 3.2 | 3.0. It takes 0.3 to 0.5 us of 6 to 11.
+struct DMLate {
+  float a;
+  int from, end, len;          // the first one; the token as of which the others weigh
+  XLLM_DEV DMLate(float decay, int n) {
+    a = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(decay)));
+    len = n;
+    from = n <= DM_LATE ? 0 : n - (a < 0.75f ? 2 : a < 0.9f ? 1 : 0);
+    end = min(from, n - 1);
+  }
+  XLLM_DEV int place(int r) const { return r - len + DM_LATE; }
+  // acc: what the pipe has summed, leading and other terms; x: the state before, faded by
+  // `fade`; k, v: of the last tokens, of this lane's key and value column
+  XLLM_DEV void join(f32x16 (&acc)[2], const float (&x)[16], float fade,
+                     const unsigned short (&k)[DM_LATE], const unsigned short (&v)[DM_LATE],
+                     int h) const {
+    const float by =
+        __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(fade)));
+    const bool alone = from == 0;                  // uniform, as all below
+    if (alone) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][r] = x[r];
+    } else if (by < 0.5f) {                        // a state that has faded meets the
+#pragma unroll
+      for (int r = 0; r < 16; ++r)                 // small terms, another one their sum
+        acc[0][r] = fmaf(by, x[r], acc[1][r]) + acc[0][r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[0][r] = fmaf(by, x[r], acc[0][r] + acc[1][r]);
+    }
+#pragma unroll
+    for (int i = 0; i < DM_LATE; ++i) {
+      if (i < place(from)) continue;               // uniform
+      // one product an entry, exact: the step's other 15 tokens are zeros
+      bf16x8 a16 = {0, 0, 0, 0, 0, 0, 0, 0}, b16 = a16;
+      a16[0] = h ? (short)0 : (short)k[i];
+      b16[0] = h ? (short)0 : (short)v[i];
+      const f32x16 z = mr_mma(a16, b16, mr_zero());
+      const float keep = alone || i > place(from) ? a : 1.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][r] = fmaf(keep, acc[0][r], z[r]);
+    }
+  }
+};
+
 // ---- sum: U[d][e] = sum_j a^(len-1-j) k_j[d] v_j[e] ---------------------------
 // A wave owns a quarter of the D x V sums; 64 tokens are staged at a time, the
 // weighted keys as three images.
-template <int D, int V>
+//   ONE: each sequence is one chunk, whose sum goes to its slot (DMLate).
+template <int D, int V, bool ONE>
 __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
   constexpr int ST = 64;
   constexpr int DT = D / 64, VT = V / 64;         // 32-wide tiles of a wave
   __shared__ __attribute__((aligned(1024))) unsigned short
-      lds[3 * ST * D + ST * V];
+      lds[3 * ST * D + ST * V + (ONE ? DM_LATE * (D + V) : 0)];
+  unsigned short* newest = lds + 3 * ST * D + ST * V;     // keys, values, with ONE
   __shared__ float pw[DM_C + 1];
   int s, c, t0, len;
   if (!dm_locate(P, &s, &c, &t0, &len)) return;
@@ -154,6 +209,8 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = lane >> 5, n = lane & 31;
   const float a = P.decay[hd];
+  const DMLate late(a, len);
+  const int sum_to = ONE ? late.from : len;      // tokens that the pipe sums
   if (tid <= DM_C) pw[tid] = dm_pow(a, tid);
   unsigned short* ks = lds;
   unsigned short* vs = lds + 3 * ST * D;
@@ -190,9 +247,11 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
     for (int i = 0; i < KI; ++i) {
       const int idx = tid + i * 256, r = idx / (D / 8), ch = idx % (D / 8);
       float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (b0 + r < len) {
+      if (ONE && b0 + r >= sum_to && b0 + r < len)
+        *reinterpret_cast<dm_u4*>(newest + late.place(b0 + r) * D + ch * 8) = dm_act(kr[i]);
+      if (b0 + r < sum_to) {
         const dm_u4 y = dm_act(kr[i]);
-        const float wgt = pw[len - 1 - b0 - r];
+        const float wgt = pw[(ONE ? late.end : len - 1) - b0 - r];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           x[2 * j] = __uint_as_float(y.x[j] << 16) * wgt;
@@ -206,6 +265,8 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
       const int idx = tid + i * 256, r = idx / (V / 8), ch = idx % (V / 8);
       dm_u4 y = {{0u, 0u, 0u, 0u}};
       if (b0 + r < len) y = dm_act(vr[i]);
+      if (ONE && b0 + r >= sum_to && b0 + r < len)
+        *reinterpret_cast<dm_u4*>(newest + DM_LATE * D + late.place(b0 + r) * V + ch * 8) = y;
       *reinterpret_cast<dm_u4*>(vs + r * V + ((ch ^ mr_swz_cols<V>(r)) << 3)) =
           y;
     }
@@ -231,33 +292,43 @@ __global__ void __launch_bounds__(256, 2) decay_sum_mfma_kernel(DMArgs P) {
     }
   }
   float* dst;
-  bool add = false;                               // to what is there,
-  float keep = 0.f;                               // by this factor
-  if (P.ws != nullptr) {
+  bool carried = false;
+  if constexpr (!ONE) {
     dst = P.ws + ((long)blockIdx.x * P.heads + hd) * (D * V);
   } else {
     const int slot = P.slots[s];
     if (slot < 0) return;
     dst = P.state + ((long)slot * P.heads + hd) * (D * V);
-    add = P.ctx_lens[s] > 0;
+    carried = P.ctx_lens[s] > 0;
     // no new tokens: a carried state stays (and no barrier has made pw visible)
-    if (add && len <= 0) return;
-    if (add) keep = pw[len];
+    if (carried && len <= 0) return;
   }
 #pragma unroll
   for (int i = 0; i < DT; ++i)
 #pragma unroll
     for (int j = 0; j < VT; ++j) {
       float* p = dst + ((d0 + i) * 32 + 4 * h) * V + (e0 + j) * 32 + n;
-      // all of it on the way before the first is stored, which might be another's place
-      float x[16];
+      f32x16 u[2] = {acc[0][i][j], acc[1][i][j]};
+      if constexpr (ONE) {
+        // all of it on the way before the first is stored, which might be another's place
+        float x[16];
+        unsigned short late_k[DM_LATE], late_v[DM_LATE];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) x[r] = add ? p[(8 * (r >> 2) + (r & 3)) * V] : 0.f;
+        for (int r = 0; r < 16; ++r)
+          x[r] = carried ? p[(8 * (r >> 2) + (r & 3)) * V] : 0.f;
+        if (len > 0) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float u = acc[0][i][j][r] + acc[1][i][j][r];
-        p[(8 * (r >> 2) + (r & 3)) * V] = add ? keep * x[r] + u : u;
+          for (int t = 0; t < DM_LATE; ++t) {
+            late_k[t] = newest[t * D + (d0 + i) * 32 + n];
+            late_v[t] = newest[DM_LATE * D + t * V + (e0 + j) * 32 + n];
+          }
+          late.join(u, x, carried ? pw[late.end + 1] : 0.f, late_k, late_v, h);
+        }
+      } else {
+        u[0] += u[1];
       }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[(8 * (r >> 2) + (r & 3)) * V] = u[0][r];
     }
 }
 
@@ -693,12 +764,21 @@ __global__ void __launch_bounds__(256, 2) decay_out_mfma_kernel(DMArgs P) {
   if (!on) return;
   const int kbase = mr_row_base<D>(lane);
   for (int kt = 0; kt <= w; ++kt) {
-    f32x16 z = mr_zero();
+    // 128 wide keys in two chains, as in the kernel of 8 and 16 waves, where there are
+    // registers for both: scores of one, over 64-wide values, made outputs of 4 to 9
+    // tokens 6.4e-8 off, 5.7e-8 by the recurrence
+    constexpr int CHAINS = D == 128 && V == 64 ? 2 : 1;
+    f32x16 zs[CHAINS];
+#pragma unroll
+    for (int i = 0; i < CHAINS; ++i) zs[i] = mr_zero();
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
-      z = mr_mma(*reinterpret_cast<const lds_bf16x8*>(
-                     (const lds_u16*)ks_ + (kbase ^ (ks << 4)) + kt * 32 * D),
-                 qf[ks], z);
+      zs[ks % CHAINS] = mr_mma(
+          *reinterpret_cast<const lds_bf16x8*>(
+              (const lds_u16*)ks_ + (kbase ^ (ks << 4)) + kt * 32 * D),
+          qf[ks], zs[ks % CHAINS]);
+    f32x16 z = zs[0];
+    if constexpr (CHAINS > 1) z += zs[CHAINS - 1];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int back = qi - kt * 32 - mr_key_of(r, h);
@@ -796,6 +876,7 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   // a SIMD's waves have different queries: later ones meet more keys
   const int vt = w >> 2, qt = (w + vt) & 3;
+  const DMLate late(LAST ? P.decay[hd] : 0.f, len);
   const int h = lane >> 5, n = lane & 31;
   const bool before = c > 0 || carried;           // uniform
   const float* S = (P.ws != nullptr
@@ -981,6 +1062,8 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
           else acc[1] = mr_mma(x, p, acc[1]);
         }
       }
+      // the nearest keys weigh most: what is small meets what they do not add to
+      if (kt == qt) acc[0] += acc[1];
       acc[0] += y;
     }
     if (qi >= len) return;
@@ -993,8 +1076,7 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
 #pragma unroll
     for (int r = 0; r < 16; r += 4)
       *reinterpret_cast<float4*>(o + 2 * r) =
-          make_float4(acc[0][r] + acc[1][r], acc[0][r + 1] + acc[1][r + 1],
-                      acc[0][r + 2] + acc[1][r + 2], acc[0][r + 3] + acc[1][r + 3]);
+          make_float4(acc[0][r], acc[0][r + 1], acc[0][r + 2], acc[0][r + 3]);
   };
   if (on) outputs();
   if constexpr (LAST) {
@@ -1007,6 +1089,13 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       x0[r] = carried && mine ? st[(8 * (r >> 2) + (r & 3)) * V] : 0.f;
+    const float by = carried ? pw[late.end + 1] : 0.f;
+    unsigned short late_k[DM_LATE], late_v[DM_LATE];
+#pragma unroll
+    for (int i = 0; i < DM_LATE; ++i) {
+      const int t = max(len - DM_LATE + i, 0), d = (dt & (D / 32 - 1)) * 32 + n;
+      late_k[i] = lds[KEYS + t * D + (((d >> 3) ^ mr_swz_rows<D>(t)) << 3) + (d & 7)];
+    }
     __syncthreads();                              // weights and values are read
     // a row's pieces are a wave's, which has read them all when it writes the first
 #pragma unroll
@@ -1015,8 +1104,8 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
       const dm_u4 z = *reinterpret_cast<const dm_u4*>(
           lds + KEYS + r * D + ((ch ^ mr_swz_rows<D>(r)) << 3));
       float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (r < len) {
-        const float wgt = pw[len - 1 - r];
+      if (r < late.from) {
+        const float wgt = pw[late.end - r];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           x[2 * j] = __uint_as_float(z.x[j] << 16) * wgt;
@@ -1037,9 +1126,13 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
     __syncthreads();
     if (!mine) return;
     const int cbase = mr_col_base<D>(lane) ^ (dt << 5);
+#pragma unroll
+    for (int i = 0; i < DM_LATE; ++i) {
+      const int t = max(len - DM_LATE + i, 0), e = vt * 32 + n;
+      late_v[i] = vs[t * V + (((e >> 3) ^ mr_swz_cols<V>(t)) << 3) + (e & 7)];
+    }
     acc[0] = acc[1] = mr_zero();
-    // leading and other terms apart. The last tokens weigh most and come last: one chain
-    // of leading products is no less precise than sums of some of them.
+    // leading and other terms apart, without the late tokens
 #pragma unroll 4
     for (int k = 0; k < len; k += 16) {
       const bf16x8 y = mr_cols<V>((const lds_u16*)vs + vbase + k * V);
@@ -1048,12 +1141,9 @@ __global__ void __launch_bounds__(32 * V / 4) decay_out_wide_kernel(DMArgs P) {
         acc[t > 0] = mr_mma(mr_cols<D>((const lds_u16*)lds + t * DM_C * D + k * D + cbase),
                             y, acc[t > 0]);
     }
-    const float by = pw[len];
+    late.join(acc, x0, by, late_k, late_v, h);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float u = acc[0][r] + acc[1][r];
-      st[(8 * (r >> 2) + (r & 3)) * V] = carried ? fmaf(by, x0[r], u) : u;
-    }
+    for (int r = 0; r < 16; ++r) st[(8 * (r >> 2) + (r & 3)) * V] = acc[0][r];
   }
 }
 
@@ -1072,10 +1162,8 @@ int decay_attn_mfma_chunk() { return DM_C; }
 // 9.4 11.6; 256: 4 14.8 19.0 | 10.7 14.7; fresh ones, 1024: 2 27.3 | 34.2, 4 37.2 | 34.3. 64 x
 // 64, 64 states: 6 7.5 7.7 | 7.3 7.5; 256: 4 7.6 9.1 | 7.4 8.1, 5 8.8 10.0 | 7.6 8.0; 1024: 2
 // 15.3 | 16.7, 3 17.2 | 16.8. 64 x 128, 256: 4 11.9 14.8 | 8.4 9.5; 128 x 64, 256: 4 9.2 10.9 |
-// 9.0 10.9, 6 11.3 13.1 | 9.0 11.0; 1024: 4 22.9 | 25.6, 6 28.9 | 25.6. Two to four tokens of
-// a fresh state stay with the recurrence where it was the faster one before out moved the
-// states itself: they are 2.5-3.5e-8 off 64 bits there, 3.0-3.7e-8 here; of 5 tokens 3.9 |
-// 3.8e-8, of 7 4.4 | 4.0e-8.
+// 9.0 10.9, 6 11.3 13.1 | 9.0 11.0; 1024: 4 22.9 | 25.6, 6 28.9 | 25.6. Whatever the
+// length, outputs and states are no further off 64 bits here (DMLate).
 bool decay_attn_short(long longest, long states, int D, int V) {
   const long wgs = states * (V / 16);
   const int most = wgs <= 128 ? 7 : wgs <= 512 ? 6                    // tokens
@@ -1162,8 +1250,14 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
   const dim3 grid_out(
       grid.x, heads + (groups > 1 ? (n_seqs * heads + grid.x - 1) / grid.x : 0));
   const bool wide = (long)grid.x * heads <= 256;
-#define DM_SUM(DD, VV)                                                        \
-  hipLaunchKernelGGL((decay_sum_mfma_kernel<DD, VV>), grid, dim3(256), 0, st, P)
+#define DM_SUM_(DD, VV, ONE)                                                  \
+  hipLaunchKernelGGL((decay_sum_mfma_kernel<DD, VV, ONE>), grid, dim3(256), 0, st, P)
+#define DM_SUM(DD, VV) DM_SUM_(DD, VV, false)
+// (128 x 128: decay_attn_one)
+#define DM_SUM_ONE(DD, VV)                                                    \
+  do {                                                                        \
+    if constexpr (DD + VV < 256) DM_SUM_(DD, VV, true);                       \
+  } while (0)
 #define DM_WALK(DD, VV)                                                       \
   hipLaunchKernelGGL((decay_walk_mfma_kernel<DD, VV>),                        \
                      dim3((unsigned)(((long)n_seqs * heads + 7) / 8 * 8 *     \
@@ -1192,7 +1286,7 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
       DM_BY_SIZE(DM_ALL);
     } else {
       DM_BY_SIZE(DM_OUT);
-      DM_BY_SIZE(DM_SUM);
+      DM_BY_SIZE(DM_SUM_ONE);
     }
     return;
   }
@@ -1215,6 +1309,8 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
 #undef DM_OUT_
 #undef DM_WALK
 #undef DM_SUM
+#undef DM_SUM_ONE
+#undef DM_SUM_
 }
 
 }  // namespace hyb

@@ -478,18 +478,35 @@ __global__ void __launch_bounds__(512, 4) decay_walk_mfma_kernel(DMArgs P) {
     float* to = P.ws + ((rec + c) * P.heads + hd) * (D * V);
     const bool store = c > 0 || carried;
     const float by = c == chunks - 1 ? keep_last : keep;
+    // z: the other half's. What weighs little comes first, so that most sums are not
+    // rounded against what is large: small terms, a state that has faded, earlier tokens.
+    // A state that has not is what is large. (Error of states of 130-1000 tokens against
+    // 64 bits, by sum and scan | here before | now: decays of 0.3 to 0.97 5.03e-8 | 5.25 |
+    // 4.95, of 0.3 to 0.7 4.73 | 5.12 | 4.91, of 0.75 to 0.996 5.9 | 5.6 | 5.6.)
+    const bool faded = __builtin_amdgcn_readfirstlane(by < 0.5f);
+    // whether the chunk's last 32 tokens are this wave's
+    const bool latest = half == (c == chunks - 1 ? (last - 1) >> 5 & 1 : 1);
+    auto join = [&](auto second) {
+      constexpr int o = second.value ? 8 : 0;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const f4 z = swap[((w ^ 4) * 2 + i) * 64 + lane];
+      for (int i = 0; i < 2; ++i) {
+        const f4 z = swap[((w ^ 4) * 2 + i) * 64 + lane];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int x = 4 * i + j;
-        const float u =
-            (half ? acc[0][8 + x] + acc[1][8 + x] : acc[0][x] + acc[1][x]) + z[j];
-        if (store) to[at[i] + j * V] = S[x];
-        S[x] = fmaf(by, S[x], u);
+        for (int j = 0; j < 4; ++j) {
+          const int x = 4 * i + j;
+          const float lead = acc[0][o + x], u = acc[1][o + x];
+          if (store) to[at[i] + j * V] = S[x];
+          if (faded) {
+            const float y = fmaf(by, S[x], u);
+            S[x] = latest ? (y + z[j]) + lead : (y + lead) + z[j];
+          } else {
+            S[x] = fmaf(by, S[x], (lead + u) + z[j]);
+          }
+        }
       }
-    }
+    };
+    if (half) join(std::true_type{});              // uniform
+    else join(std::false_type{});
   };
   if (chunks > 0) stage(0, 0, kr[0][0], vr[0][0]);
   __syncthreads();

@@ -33,6 +33,12 @@ def recur(q, k, v, a, S):
     return torch.stack(out), S
 
 
+def way(heads, D, V, lens):
+    """How a batch goes: the way, groups of chunks that are walked, waves of outputs."""
+    return "%s %d %d" % H._hyb().decay_attn_way(max(lens), sum(lens), len(lens), heads,
+                                                D, V)
+
+
 def run(D, V, lens, ctx, slots, decay, bound, seed):
     g = torch.Generator().manual_seed(seed)
     heads, T = len(decay), sum(lens)
@@ -51,13 +57,12 @@ def run(D, V, lens, ctx, slots, decay, bound, seed):
     H.decay_attn(*(rd[:, x:y] for x, y in zip(cut, cut[1:])), a.cuda(), sd,
                  torch.tensor(slots, **i32), torch.tensor(starts, **i32),
                  torch.tensor(ctx, **i32), out, max_q_len=bound)
-    out, sd, used = out.cpu().to(F64), sd.cpu(), set()
+    out, used, f, a64 = out.to(F64), set(), f.cuda(), a.cuda().to(F64)
     for s, (n, c, slot) in enumerate(zip(lens, ctx, slots)):
         x = [f[starts[s]:starts[s + 1], p:e].reshape(n, heads, -1)
              for p, e in zip(cut, cut[1:])]
-        S = state[slot].to(F64) if slot >= 0 and c > 0 else torch.zeros(
-            heads, D, V, dtype=F64)
-        a64 = a.to(F64)
+        S = (state[slot] if slot >= 0 and c > 0 else torch.zeros(heads, D, V)).to(
+            "cuda", F64)
         want, after = recur(*x, a64, S)
         big, top = recur(*(z.abs() for z in x), a64.abs(), S.abs())
         off = (out[starts[s]:starts[s + 1]] - want).abs() - 2.0 ** -20 * big
@@ -68,7 +73,7 @@ def run(D, V, lens, ctx, slots, decay, bound, seed):
             assert off.max() <= 1e-30, f"state {s}: over by {off.max():.3g}"
     for slot in range(state.shape[0]):
         if slot not in used:
-            assert torch.equal(sd[slot], state[slot])
+            assert torch.equal(sd[slot].cpu(), state[slot])
 
 
 @pytest.mark.parametrize("D,V", [(128, 128), (64, 128), (128, 64), (64, 64)])
@@ -83,28 +88,36 @@ def test_prompt_rows(D, V, lens, bound):
 
 
 @pytest.mark.parametrize("D,V", [(128, 128), (64, 128), (128, 64), (64, 64)])
-@pytest.mark.parametrize("lens,bound", [
-    ([100, 40, 128, 3] * 23, 128),      # more workgroups than CUs: one chunk each
-    ([130, 64, 257, 2, 65] * 20, 257),  # ... and sequences that are walked
-    ([1500, 1, 3], 1500),               # few long ones: sums and a scan
-    ([128, 256, 192], 256)])            # walked, by few
-def test_prompt_routes(D, V, lens, bound):
-    """Each way from chunk to chunk, and outputs by four waves and by sixteen."""
+@pytest.mark.parametrize("lens,heads,ways", [
+    # 128 x 128 | 64 x 128 | 128 x 64 | 64 x 64
+    ([100, 40, 128, 3] * 23, 3, "one 0 16|one 0 16|one 0 8|two 0 4"),
+    ([150, 3, 200], 32, "walk 1 16|walk 1 16|walk 1 8|walk 1 8"),
+    ([300, 164, 250, 130], 32, "walk 1 4|walk 1 4|walk 1 4|walk 1 4"),
+    ([130, 64, 257, 2, 65] * 20, 3, "scan 0 4|walk 1 4|walk 1 4|walk 1 4"),
+    ([1500, 1, 3], 3, "scan 0 16|scan 0 16|scan 0 8|scan 0 8"),
+    ([128, 256, 192], 3, "walk 2 16|walk 1 16|walk 1 8|walk 1 8")])
+def test_prompt_routes(D, V, lens, heads, ways):
+    """Each way from chunk to chunk, with outputs by four waves and by more; states
+    carried, fresh and not kept."""
+    assert way(heads, D, V, lens) == ways.split("|")[(D == 64) + 2 * (V == 64)]
     n = len(lens)
-    run(D, V, lens, [5 * (i % 3) for i in range(n)],
-        [i if i % 7 else -1 for i in range(n)], [0.999, 0.75, 1.0], bound, n + D + V)
+    run(D, V, lens, [5 * (i % 3 > 0) for i in range(n)],
+        [i if (i + 5) % 7 else -1 for i in range(n)],
+        ([0.999, 0.75, 1.0, 0.97, 0.3] * 7)[:heads], max(lens), n + D + V)
 
 
-@pytest.mark.parametrize("lens,heads", [
-    ([700, 3, 129, 384], 3), ([513, 1, 640, 385], 3),   # outputs by sixteen waves
-    ([900, 640, 1100, 515, 700], 8)])                   # by four
-def test_groups_of_chunks(lens, heads):
+@pytest.mark.parametrize("lens,heads,groups,waves", [
+    ([700, 3, 129, 384], 3, 3, 16), ([513, 1, 640, 385], 3, 3, 16),
+    ([430, 130], 8, 4, 16), ([880, 881, 515], 3, 4, 16), ([880, 881, 515], 16, 2, 4),
+    ([1030, 900], 16, 3, 4), ([1030], 32, 3, 4)])
+def test_groups_of_chunks(lens, heads, groups, waves):
     """Sequences walked in up to four groups: whole and ragged last ones, fewer
     chunks than groups, states carried or not, one without a slot."""
+    assert way(heads, 128, 128, lens) == f"walk {groups} {waves}"
     n = len(lens)
     run(128, 128, lens, [7 * (i % 3 != 1) for i in range(n)],
         [i if i != 2 else -1 for i in range(n)],
-        [0.999, 0.75, 1.0, 0.9999, 0.0, 0.3, 0.99, 0.996][:heads], max(lens), n)
+        ([0.999, 0.75, 1.0, 0.9999, 0.0, 0.3, 0.99, 0.996] * 4)[:heads], max(lens), n)
 
 
 def test_many_chunks_and_hard_decays():
@@ -252,16 +265,21 @@ def test_short_prompts_no_less_precise(heads, D, V, n, longest):
                 ctx, lo, here, there)
 
 
-@pytest.mark.parametrize("D,V", [(128, 128), (64, 128), (128, 64), (64, 64)])
-@pytest.mark.parametrize("lens", [[300, 256], [210, 130], [384, 200, 129]])
-def test_walk_no_less_precise_than_scan(D, V, lens):
+@pytest.mark.parametrize("heads,D,V,lens", [
+    (16, 128, 128, [300, 256]), (16, 128, 128, [210, 130]), (16, 128, 128, [384, 200, 129]),
+    (32, 128, 128, [300, 256]), (16, 64, 128, [300, 256]), (16, 64, 128, [384, 200, 129]),
+    (16, 128, 64, [300, 256]), (16, 128, 64, [210, 130]), (16, 64, 64, [210, 130]),
+    (32, 64, 64, [384, 200, 129])])
+def test_walk_no_less_precise_than_scan(heads, D, V, lens):
     """Sequences that are walked and the same ones beside a long one, which makes the batch
     go by sums and a scan: states are no further off 64 bits (1% for what 10^5 entries
     scatter). Where all heads decay to a half within a token, half of the entries of a
     walked state are rounded twice, by sums all of them once: up to 5%."""
+    assert way(heads, D, V, lens)[:4] == "walk"
+    assert way(heads, D, V, lens + [4000])[:4] == "scan"
     g = torch.Generator(device="cuda").manual_seed(sum(lens))
     for lo, hi, most in ((0.3, 0.7, 1.05), (0.75, 0.996, 1.01), (0.996, 0.999, 1.01)):
-        heads, off = 16, []
+        off = []
         a = torch.linspace(lo, hi, heads, device="cuda")
         x, f = features(torch.randn(sum(lens) + 4000, heads * (2 * D + V), generator=g,
                                     device="cuda").to(torch.bfloat16))
@@ -287,26 +305,31 @@ def test_walk_no_less_precise_than_scan(D, V, lens):
         assert off[0] <= most * off[1], (lo, off)
 
 
-@pytest.mark.parametrize("heads,D,V", [(1, 128, 128), (48, 64, 64),
-                                       (40, 128, 64), (20, 64, 128)])
-def test_short_batches(heads, D, V):
+@pytest.mark.parametrize("heads,D,V,most", [
+    (1, 128, 128, 7), (48, 64, 64, 4), (40, 128, 64, 6), (20, 64, 128, 6),
+    (86, 128, 128, 3), (86, 128, 64, 4), (100, 64, 64, 3), (172, 64, 64, 2)])
+def test_short_batches(heads, D, V, most):
     """Lengths on both sides of the line between the recurrence and the
     matrix-pipe form, for few and for many states."""
-    for n in (1, 3, 9, 12, 13, 16, 17, 24, 25):
+    for n in (1, 2, 3, 4, 5, 6, 7, 8, 9, 17, 25):
+        assert (way(heads, D, V, [n] * 3)[:3] == "rec") == (n <= most)
         run(D, V, [n, max(1, n // 2), n], [0, 5, 3], [1, -1, 0],
             [0.75 + 0.24 * h / heads for h in range(heads)], n, n)
 
 
-@pytest.mark.parametrize("heads,D,V,lens", [
-    (16, 128, 128, [128, 1, 15, 16, 17, 33, 127]),    # tiles of 16 and 32 tokens
-    (24, 128, 128, [63, 64, 65, 96, 97, 8] * 2),      # beyond a workgroup for each CU
-    (40, 64, 64, [128, 31, 5, 112, 2, 64]), (43, 64, 64, [128, 31, 5, 112, 2, 64]),
-    (60, 64, 128, [32, 3, 20, 7, 16] * 2), (60, 64, 128, [33, 3, 20, 7, 128] * 2),
-    (64, 128, 64, [33, 128, 9, 50, 16, 100, 65]), (65, 128, 64, [33, 128, 9, 50, 16, 100, 65]),
-])
-def test_one_chunk_each(heads, D, V, lens):
+@pytest.mark.parametrize("heads,D,V,lens,kind", [
+    (16, 128, 128, [128, 1, 15, 16, 17, 33, 127], "one"),    # tiles of 16 and 32 tokens
+    (24, 128, 128, [63, 64, 65, 96, 97, 8] * 2, "one"),      # more than one for each CU
+    (40, 64, 64, [128, 31, 5, 112, 2, 64], "one"),
+    (43, 64, 64, [128, 31, 5, 112, 2, 64], "two"),
+    (60, 64, 128, [32, 3, 20, 7, 16] * 2, "two"),
+    (60, 64, 128, [33, 3, 20, 7, 128] * 2, "one"),
+    (64, 128, 64, [33, 128, 9, 50, 16, 100, 65], "one"),
+    (65, 128, 64, [33, 128, 9, 50, 16, 100, 65], "two")])
+def test_one_chunk_each(heads, D, V, lens, kind):
     """States moved by the workgroups of the outputs, or after them, on both sides of the
     lines between; some states not kept, some carried."""
+    assert way(heads, D, V, lens)[:3] == kind
     n = len(lens)
     run(D, V, lens, [i % 3 * 4 for i in range(n)],
         [-1 if i % 5 == 3 else i for i in range(n)],

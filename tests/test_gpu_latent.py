@@ -101,6 +101,11 @@ def test_fixed_parts(op, monkeypatch):
     (32, [9, 4], [700, 1300], 500),              # ... in a window
     (1, [300, 2], [10, 5], 1),
     (16, [3] * 70, [40] * 70, 0),                # more sequences than lanes
+    (16, [3] * 70, ([0, 40, 600] * 24)[:70], 0),     # ... and parts of them
+    (16, [0, 5, 0, 33, 0], [40, 90, 0, 0, 7], 0),    # sequences of no new tokens
+    (16, [5, 0, 33, 0], [900, 1300, 0, 40], 0),      # ... beside parts
+    (40, [9, 1, 40], [100, 700, 0], 0),          # many heads
+    (64, [20], [1500], 0),
     (32, [500, 300, 60], [0, 70, 800], 0)])      # a turn of the CUs and more
 def test_prompt_edges(tail, heads, new, old, window):
     g = torch.Generator().manual_seed(tail + heads + window + len(new))
@@ -126,6 +131,8 @@ def test_prompt_edges(tail, heads, new, old, window):
                       torch.tensor(keys, dtype=torch.int32, device="cuda"),
                       sign * scale, r, out, window)
         for s, n in enumerate(new):
+            if n == 0:
+                continue
             k = cache[table[s, :need[s]].long()].reshape(-1, W)[:keys[s]].cuda()
             k = k.double()
             z = q[cu[s]:cu[s + 1]].cuda().double() @ k.t() * (sign * scale)
@@ -151,7 +158,72 @@ def test_prompt_edges(tail, heads, new, old, window):
     (32, [300, 221, 400, 475, 250], [200, 39, 257, 100, 0])])
 def test_prompt_tiles_of_128_rows(tail, heads, new, old):
     """Calls that row tiles of 64 would take longer for."""
+    assert prompt_way(heads, new, old)[0] == 128
     test_prompt_edges(tail, heads, new, old, 0)
+
+
+def prompt_way(heads, new, old, window=0):
+    """Rows of a tile, 64-key tiles of a part at least (0: no parts), parts at most of
+    what test_prompt_edges makes of these."""
+    width = max(-(-(n + o) // 16) for n, o in zip(new, old)) + 1
+    return H._hyb().latent_rows_way(sum(new), len(new), heads, width, window)
+
+
+@pytest.mark.parametrize("tail", [0, 64])
+@pytest.mark.parametrize("rows,heads,new,old", [
+    (64, 16, [1100], [0]), (64, 16, [1300, 200], [0, 0]),
+    (128, 32, [533], [2600]), (128, 32, [400, 30, 500], [1500, 3000, 600])])
+def test_prompt_long_chains(tail, rows, heads, new, old):
+    """Keys in one piece, more than the 1024 whose pages a wave asks for at a time."""
+    assert prompt_way(heads, new, old)[:2] == (rows, 0)
+    test_prompt_edges(tail, heads, new, old, 0)
+
+
+@pytest.mark.parametrize("heads,new,old,window", [
+    (32, [5], [1500], 0), (16, [3, 20, 2], [1100, 0, 400], 0),
+    (32, [9, 4], [700, 1300], 500), (16, [3] * 70, ([0, 40, 600] * 24)[:70], 0),
+    (16, [5, 0, 33, 0], [900, 1300, 0, 40], 0), (64, [20], [1500], 0),
+    (16, [301], [2900], 0), (32, [40, 6, 130], [3000, 2500, 2800], 0)])
+def test_prompts_in_parts(heads, new, old, window):
+    """The calls above that are meant to have parts have them."""
+    _, least, most = prompt_way(heads, new, old, window)
+    assert least > 0 and most > 1
+
+
+@pytest.mark.parametrize("r,tail,page", [(512, 64, 32), (512, 0, 8), (480, 64, 16),
+                                         (272, 32, 16)])
+@pytest.mark.parametrize("heads,window", [(16, 0), (17, 40), (64, 0)])
+def test_prompts_of_other_sizes(r, tail, page, heads, window):
+    """Wide rows of another rank, or in pages of another size."""
+    g = torch.Generator().manual_seed(r + page + heads)
+    W, new, old, scale = r + tail, [5, 40, 1, 16], [70, 0, 300, 33], 0.07
+    keys = [n + o for n, o in zip(new, old)]
+    need = [-(-n // page) for n in keys]
+    cache = torch.randn(sum(need) + 2, page, W, generator=g).to(torch.bfloat16)
+    order = torch.randperm(sum(need) + 2, generator=g).to(torch.int32)
+    table = torch.zeros(len(keys), max(need), dtype=torch.int32)
+    cu = [0]
+    for i, n in enumerate(need):
+        table[i, :n] = order[sum(need[:i]):sum(need[:i]) + n]
+        cu.append(cu[-1] + new[i])
+    q = torch.randn(sum(new), heads, W, generator=g).to(torch.bfloat16)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    out = torch.full((sum(new), heads, r), 9.0, device="cuda")
+    H.latent_attn(q.cuda(), cache.cuda(), table.cuda(), torch.tensor(cu, **i32),
+                  torch.tensor(keys, **i32), scale, r, out, window)
+    for s, n in enumerate(new):
+        k = cache[table[s, :need[s]].long()].reshape(-1, W)[:keys[s]].double()
+        z = q[cu[s]:cu[s + 1]].double() @ k.t() * scale
+        pos = old[s] + torch.arange(n)[:, None, None]
+        at = torch.arange(keys[s])
+        z = z.masked_fill((at > pos) | (window > 0) & (at <= pos - window), -math.inf)
+        p = torch.softmax(z, -1)
+        off = (out[cu[s]:cu[s + 1]].double().cpu() - p @ k[:, :r]).abs()
+        most = (q[cu[s]:cu[s + 1]].double().abs() @ k.abs().t()).masked_fill(
+            z == -math.inf, 0.0).amax(-1, keepdim=True) * scale
+        bound = (6 * 2.0 ** -24 * most).clamp(min=2.0 ** -17)   # as above
+        over = off - bound * (p @ k[:, :r].abs())
+        assert over.max() <= 1e-7, f"sequence {s}: off by {over.max():.3g}"
 
 
 @pytest.mark.parametrize("bad", [math.nan, math.inf])

@@ -67,6 +67,7 @@ void launch_latent_attn(float*, const T*, const T*, const int*, const int*,
 int latent_attn_mfma_class(int W, int r);
 bool latent_rows_takes(int, int, int);
 long latent_rows_scratch(long, int, int, long, int);
+void latent_rows_way(long, int, int, long, int, int*, int*, int*);
 void launch_latent_rows(float*, float*, const unsigned short*,
                         const unsigned short*, const int*, const int*,
                         const int*, long, int, int, int, int, float, int,
@@ -82,6 +83,7 @@ void launch_latent_attn_mfma(float*, float*, float*, const unsigned short*,
                              float, int, int, hipStream_t);
 long decay_attn_mfma_chunks(long, long);
 int decay_attn_mfma_chunk();
+void decay_attn_mfma_way(long, long, int, int, int, int, int*, bool*, bool*);
 int decay_attn_mfma_groups(long, long, int, int, int, int);
 bool decay_attn_short(long, long, int, int);
 void launch_decay_attn_mfma(float*, const unsigned short*,
@@ -659,6 +661,15 @@ void latent_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables,
     hy::launch_latent_attn<bf>(ptr<float>(out), ptr<bf>(q), ptr<bf>(cache), ptr<int>(block_tables), cu, ptr<int>(seq_lens), T, n_seqs, H, r, W - r, cache.size(1), block_tables.size(1), scale, q.stride(0), window, cur());
 }
 
+// What latent_attn does with prompt rows of rank 512: rows of a tile, 64-key tiles of a
+// part at least (0: keys are not split), parts of a row tile at most
+std::tuple<int, int, int> latent_rows_way(long tokens, int n_seqs, int heads,
+                                          long table_width, int window) {
+  int rows, least, most;
+  hy::latent_rows_way(tokens, n_seqs, heads, table_width, window, &rows, &least, &most);
+  return {rows, least, most};
+}
+
 // out fp32 [T, H, Dv]; q,k [T, H*D] / v [T, H*Dv] row views (pre-activation)
 // state fp32 [slots, H, D, Dv]; cu_q None => one token per sequence
 // max_q_len: host-side bound on the longest sequence chunk (0 = unknown);
@@ -736,6 +747,21 @@ void decay_attn(Tensor out, Tensor q, Tensor k, Tensor v, Tensor decay,
     hy::launch_decay_attn<float>(ptr<float>(out), ptr<float>(q), ptr<float>(k), ptr<float>(v), ptr<float>(decay), ptr<float>(state), ptr<int>(slots), cu, ptr<int>(ctx_lens), n_seqs, H, D, Dv, q.stride(0), k.stride(0), v.stride(0), chunk, max_chunks, wsp, cur());
   else
     hy::launch_decay_attn<bf>(ptr<float>(out), ptr<bf>(q), ptr<bf>(k), ptr<bf>(v), ptr<float>(decay), ptr<float>(state), ptr<int>(slots), cu, ptr<int>(ctx_lens), n_seqs, H, D, Dv, q.stride(0), k.stride(0), v.stride(0), chunk, max_chunks, wsp, cur());
+}
+
+// What decay_attn does with aligned bf16 prompt rows whose scratch fits: "recurrence"; a
+// chunk each by "one" kernel or "two"; "scan"; "walk". Groups of chunks that are walked,
+// waves of a workgroup of outputs.
+std::tuple<std::string, int, int> decay_attn_way(long longest, long tokens, int n_seqs,
+                                                 int heads, int D, int V) {
+  if (hy::decay_attn_short(longest, (long)n_seqs * heads, D, V))
+    return {"recurrence", 0, 0};
+  int groups;
+  bool one, wide;
+  hy::decay_attn_mfma_way(longest, tokens, n_seqs, heads, D, V, &groups, &one, &wide);
+  const char* way = longest <= hy::decay_attn_mfma_chunk() ? (one ? "one" : "two")
+                    : groups > 0 ? "walk" : "scan";
+  return {way, groups, wide ? V / 8 : 4};
 }
 
 // z fp32 [T, E] router logits -> ids int32 [T, top], wts fp32 [T, top]
@@ -1483,7 +1509,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rope_interleaved", &rope_interleaved);
   m.def("latent_kv_store", &latent_kv_store);
   m.def("latent_attn", &latent_attn);
+  m.def("latent_rows_way", &latent_rows_way);
   m.def("decay_attn", &decay_attn);
+  m.def("decay_attn_way", &decay_attn_way);
   m.def("moe_route", &moe_route);
   m.def("moe_combine", &moe_combine);
   m.def("streams_mix_norm", &streams_mix_norm);

@@ -1180,7 +1180,9 @@ int decay_attn_mfma_chunk() { return DM_C; }
 // 64, 64 states: 6 7.5 7.7 | 7.3 7.5; 256: 4 7.6 9.1 | 7.4 8.1, 5 8.8 10.0 | 7.6 8.0; 1024: 2
 // 15.3 | 16.7, 3 17.2 | 16.8. 64 x 128, 256: 4 11.9 14.8 | 8.4 9.5; 128 x 64, 256: 4 9.2 10.9 |
 // 9.0 10.9, 6 11.3 13.1 | 9.0 11.0; 1024: 4 22.9 | 25.6, 6 28.9 | 25.6. Whatever the
-// length, outputs and states are no further off 64 bits here (DMLate).
+// length, outputs and states are no further off 64 bits here (DMLate), heads of 0.75 to
+// 0.996 or of 0.5 to 0.996 (184 sizes, parts of the recurrence's: 0.88 and 0.82, at most
+// 1.00); where all of them decay to 0.7 or less within a token, states 1.03, at most 1.09.
 bool decay_attn_short(long longest, long states, int D, int V) {
   const long wgs = states * (V / 16);
   const int most = wgs <= 128 ? 7 : wgs <= 512 ? 6                    // tokens
@@ -1245,6 +1247,18 @@ static bool decay_attn_one(long longest, long states, int D, int V) {
   return D == 128 && states <= 448 && longest > 32;
 }
 
+// How a batch of prompt rows goes: groups of chunks that are walked (0: sum and scan, if
+// any has more than a chunk); whether out moves the states of a chunk each; whether its
+// workgroups have 8 or 16 waves.
+void decay_attn_mfma_way(long longest, long tokens, int n_seqs, int heads, int D, int V,
+                         int* groups, bool* one, bool* wide) {
+  *groups = decay_attn_mfma_groups(longest, tokens, n_seqs, heads, D, V);
+  *one = longest <= DM_C && decay_attn_one(longest, (long)n_seqs * heads, D, V);
+  const long units =
+      (longest > DM_C ? decay_attn_mfma_chunks(tokens, n_seqs) : n_seqs) * heads;
+  *wide = *one || units <= 256;
+}
+
 // D, V in {64, 128}; rows 16 B aligned. ws null: no sequence has more than
 // DM_C tokens. longest: tokens of a sequence at most
 void launch_decay_attn_mfma(float* out, const unsigned short* q,
@@ -1255,8 +1269,9 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
                             long k_stride, long v_stride, float* ws,
                             long longest, hipStream_t st) {
   if (n_seqs == 0) return;
-  const int groups = decay_attn_mfma_groups(longest, tokens, n_seqs, heads, D, V);
-  const bool walk = groups > 0;
+  int groups;
+  bool one, wide;
+  decay_attn_mfma_way(longest, tokens, n_seqs, heads, D, V, &groups, &one, &wide);
   const DMArgs P = {out, q, k, v, q_stride, k_stride, v_stride, decay, state,
                     ws, slots, cu_q, ctx_lens, n_seqs, heads,
                     std::max(groups, 1),
@@ -1266,7 +1281,6 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
   // with those that make the last states (dm_last_state)
   const dim3 grid_out(
       grid.x, heads + (groups > 1 ? (n_seqs * heads + grid.x - 1) / grid.x : 0));
-  const bool wide = (long)grid.x * heads <= 256;
 #define DM_SUM_(DD, VV, ONE)                                                  \
   hipLaunchKernelGGL((decay_sum_mfma_kernel<DD, VV, ONE>), grid, dim3(256), 0, st, P)
 #define DM_SUM(DD, VV) DM_SUM_(DD, VV, false)
@@ -1299,7 +1313,7 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
   } while (0)
 #define DM_ALL(DD, VV) DM_WIDE(DD, VV, false, true)
   if (ws == nullptr) {                            // a chunk each
-    if (decay_attn_one(longest, (long)n_seqs * heads, D, V)) {
+    if (one) {
       DM_BY_SIZE(DM_ALL);
     } else {
       DM_BY_SIZE(DM_OUT);
@@ -1307,7 +1321,7 @@ void launch_decay_attn_mfma(float* out, const unsigned short* q,
     }
     return;
   }
-  if (walk) {
+  if (groups > 0) {
     DM_BY_SIZE(DM_WALK);
   } else {
     DM_BY_SIZE(DM_SUM);

@@ -14,9 +14,9 @@
 //                                reads of the same image, P split exactly into three
 //                                bf16 terms, a product each
 // So a wave keeps its queries (64 registers; two steps of 18 are in LDS) and sums (128)
-// where they are, and a CU reads 340 KB of LDS per tile, 0.63 of the time that its products
-// take. (16 rows a wave, 16x16x32 products and a tile at a time read as long as they
-// multiplied, and waited for each tile.)
+// where they are, and a CU reads 320 KB of LDS per tile, 2560 cycles beside the 4224 of its
+// products (66 of 32 cycles a wave, two waves a SIMD). (16 rows a wave, 16x16x32 products
+// and a tile at a time read as long as they multiplied, and waited for each tile.)
 //
 // The two waves of a SIMD belong to different rows, and one's exponentials meet the
 // other's products: half of the waves pass the barrier of the next tile between the
@@ -29,8 +29,8 @@
 // Measured, us, before | here: 16 heads, rows of 576, 1800 and 2200 tokens 1002 | 229 (1090
 // TFLOP/s executed), 1000 tokens 247 | 75, 434 and 45 behind 5000 1244 | 128 (parts), by
 // four waves 256 tokens 68 | 24, 16 25 | 9.2 (two waves 33 and 13.6); 32 heads, rows of 512 in
-// a window of 1024, 3077 and 63 560 | 161. A tile takes about 7000 cycles of a CU for
-// products of 4750. Of a wave's, steps of K asked for as they were needed took 900 more, and
+// a window of 1024, 3077 and 63 560 | 161. A tile takes about 7000 cycles of a CU (2.9 us),
+// its products 4224. Of a wave's, steps of K asked for as they were needed took 900 more, and
 // loads at the start of a tile 1000: their instructions queue. Error against 64 bits,
 // the first three: 3.6e-7 | 3.0e-7, 3.3 | 2.1, 7.0 | 2.5.
 //
@@ -522,6 +522,14 @@ static LrPlan lr_plan(long tokens, int n_seqs, int heads, long table_width,
 long latent_rows_scratch(long tokens, int n_seqs, int heads, long table_width,
                          int window) {
   return lr_plan(tokens, n_seqs, heads, table_width, window).scratch;
+}
+
+void latent_rows_way(long tokens, int n_seqs, int heads, long table_width, int window,
+                     int* rows, int* least, int* most) {
+  const LrPlan p = lr_plan(tokens, n_seqs, heads, table_width, window);
+  *rows = p.rows;
+  *least = p.least;
+  *most = p.most;
 }
 
 // q, cache and out 16 B aligned

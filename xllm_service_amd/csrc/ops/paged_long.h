@@ -21,8 +21,9 @@
 // 328 -> 333 us). What is left out counts: without exponentials 313, without three
 // quarters of the operands' reads 308, without the scaling of sums 321, and scaling them
 // only in the lanes whose maximum has grown 328 -> 325. 4 prompts of 1.6-2.3 k tokens over
-// up to 3.1 k cached ones, 32 heads of 128: 353 -> 335 -> 325 us. What it costs is one workgroup per CU: nothing covers its start and its end, so it
-// is taken for whole turns of workgroups with long chains only (paged_long_takes).
+// up to 3.1 k cached ones, 32 heads of 128: 353 -> 335 -> 325 us. What it costs is one
+// workgroup per CU: nothing covers its start and its end, so it is taken for whole turns of
+// workgroups with long chains only (paged_long_takes).
 #pragma once
 #include "paged_rows.h"
 

@@ -1182,7 +1182,7 @@ int decay_attn_mfma_chunk() { return DM_C; }
 // 9.0 10.9, 6 11.3 13.1 | 9.0 11.0; 1024: 4 22.9 | 25.6, 6 28.9 | 25.6. Whatever the
 // length, outputs and states are no further off 64 bits here (DMLate), heads of 0.75 to
 // 0.996 or of 0.5 to 0.996 (184 sizes, parts of the recurrence's: 0.88 and 0.82, at most
-// 1.00); where all of them decay to 0.7 or less within a token, states 1.03, at most 1.09.
+// 1.01); where all of them decay to 0.7 or less within a token, states 1.03, at most 1.09.
 bool decay_attn_short(long longest, long states, int D, int V) {
   const long wgs = states * (V / 16);
   const int most = wgs <= 128 ? 7 : wgs <= 512 ? 6                    // tokens

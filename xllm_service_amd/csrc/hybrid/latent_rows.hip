@@ -30,7 +30,8 @@
 // TFLOP/s executed), 1000 tokens 247 | 75, 434 and 45 behind 5000 1244 | 128 (parts), by
 // four waves 256 tokens 68 | 24, 16 25 | 9.2 (two waves 33 and 13.6); 32 heads, rows of 512 in
 // a window of 1024, 3077 and 63 560 | 161. A tile takes about 7000 cycles of a CU (2.9 us),
-// its products 4224. Of a wave's, steps of K asked for as they were needed took 900 more, and
+// its products 4224; the clock is 1.9 GHz meanwhile (2.39 with zeros for data, in as many
+// cycles). Of a wave's, steps of K asked for as they were needed took 900 more, and
 // loads at the start of a tile 1000: their instructions queue. Error against 64 bits,
 // the first three: 3.6e-7 | 3.0e-7, 3.3 | 2.1, 7.0 | 2.5.
 //
@@ -447,6 +448,8 @@ bool latent_rows_takes(int W, int r, int block_size) {
 // | 42 (least 4 46, 8 60), 45 and 434 behind 5000 416 | 132, 34-309 behind 1000 93 | 54,
 // 1000 alone 90 | 74. Between 128 and 200 row tiles short tables gain nothing: 44 and 1024
 // of 32 heads 55 | 61, 389 and 1250 85 | 91; long ones do: 210-828 behind 150-4000 206 | 154.
+// Parts take scratch: at most 67 MB for one sequence (256 units of 128 rows), 112 MB for
+// several (425).
 struct LrPlan { int rows = LR_ROWS, least = 0, most = 1; long units = 0, scratch = 0; };
 static LrPlan lr_split(int rows, long wgs, int n_seqs, long tiles) {
   LrPlan x;

@@ -14,16 +14,15 @@
 // v_readlane fetch from a table of 64 tiles made at once: by scalar arithmetic on the way
 // a step's loads cost 700 cycles.
 //
-// Bound by the card's power: the clock falls to 1.64 GHz while calls follow each other
-// (1.84 for a single one, 2.2 to 2.4 with zeros for data), a step of two tiles a SIMD takes
-// 3430 cycles there, and schedules that take fewer run at a lower clock still or the same
-// time (all operands in registers before their products: 1660 -> 1380 cycles for a tile's 32,
-// 328 -> 333 us). What is left out counts: without exponentials 313, without three
-// quarters of the operands' reads 308, without the scaling of sums 321, and scaling them
-// only in the lanes whose maximum has grown 328 -> 325. 4 prompts of 1.6-2.3 k tokens over
-// up to 3.1 k cached ones, 32 heads of 128: 353 -> 335 -> 325 us. What it costs is one
-// workgroup per CU: nothing covers its start and its end, so it is taken for whole turns of
-// workgroups with long chains only (paged_long_takes).
+// Bound by the card's power: 640 k cycles at 1.8 GHz while calls follow each other, 623 k at
+// 2.35 with zeros for data (350 | 265 us). So what takes fewer cycles and as much energy gains
+// nothing (all operands in registers before their products: 1660 -> 1380 cycles for a tile's
+// 32, 328 -> 333 us), and what is left out counts: without exponentials 328 -> 313, without
+// three quarters of the operands' reads 308, without the scaling of sums 321. Scaling them
+// only in the lanes whose maximum has grown: 353.5 -> 348.0 (runs of one side differ by 0.7%;
+// cards differ by 8%). 4 prompts of 1.6-2.3 k tokens over up to 3.1 k cached ones, 32 heads
+// of 128. What it costs is one workgroup per CU: nothing covers its start and its end, so it
+// is taken for whole turns of workgroups with long chains only (paged_long_takes).
 #pragma once
 #include "paged_rows.h"
 
